@@ -16,7 +16,8 @@ extern "C" __global__ void store_kv_fp8_kernel(const bf16_t*, const bf16_t*, uns
 extern "C" void launch_attn_decode_partial(float*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, float, int, int, int, int, int, int, int, int, int, hipStream_t);
 extern "C" __global__ void attn_decode_reduce_kernel(bf16_t*, const float*, const int*, int, int, int, int);
 extern "C" __global__ void attn_prefill_kernel(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, float, int, int, int, int);  // grouped: [G], [G], [G*8]
-extern "C" __global__ void sample_kernel(int64_t*, float*, const float*, const float*, const float*, const int*, const int64_t*, const int64_t*, const uint32_t*, int, float*);
+extern "C" int sample_slices(int B, int V);
+extern "C" void launch_sample(int64_t*, float*, void*, const float*, const float*, const float*, const int*, const int64_t*, const int64_t*, const uint32_t*, int, int, float*, hipStream_t);
 extern "C" __global__ void mfma_selftest_kernel(float*, const bf16_t*, const bf16_t*);
 
 #define CHECK_BF16_CONTIG(t) \
@@ -172,13 +173,14 @@ void sample(torch::Tensor tokens, torch::Tensor logprobs, torch::Tensor logits,
   const int B = logits.size(0), V = logits.size(1);
   const uint32_t* mptr = mask.numel() > 0
       ? reinterpret_cast<const uint32_t*>(mask.data_ptr<int>()) : nullptr;
-  const size_t lds = 16 * 256 * (sizeof(float) + sizeof(unsigned int));  // per-wave histograms
-  hipLaunchKernelGGL(sample_kernel, dim3(B), dim3(1024), lds, cur_stream(),
-                     tokens.data_ptr<int64_t>(), logprobs.data_ptr<float>(),
-                     logits.data_ptr<float>(), temperatures.data_ptr<float>(),
-                     top_ps.data_ptr<float>(), top_ks.data_ptr<int>(),
-                     seeds.data_ptr<int64_t>(), steps.data_ptr<int64_t>(), mptr, V,
-                     dbg.numel() ? dbg.data_ptr<float>() : nullptr);
+  if (B == 0 || V == 0) return;
+  // per-slice results: 6 words each (SlicePart)
+  auto parts = torch::empty({(int64_t)B * sample_slices(B, V) * 3},
+                            torch::dtype(torch::kLong).device(logits.device()));
+  launch_sample(tokens.data_ptr<int64_t>(), logprobs.data_ptr<float>(), parts.data_ptr(),
+                logits.data_ptr<float>(), temperatures.data_ptr<float>(), top_ps.data_ptr<float>(),
+                top_ks.data_ptr<int>(), seeds.data_ptr<int64_t>(), steps.data_ptr<int64_t>(), mptr,
+                B, V, dbg.numel() ? dbg.data_ptr<float>() : nullptr, cur_stream());
 }
 
 torch::Tensor mfma_selftest(torch::Tensor A, torch::Tensor B) {

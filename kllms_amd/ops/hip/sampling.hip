@@ -1,28 +1,39 @@
-// Fused sampling + logprob kernel for gfx950.
+// Sampling + logprob for gfx950, in two launches.
 //
-// One 1024-thread block per sequence row over the full vocab (grid-stride):
-//   pass A: masked max (constrained-decode bitmask applied here) + argmax
-//   pass B: unscaled sum-exp (for the OpenAI-style model logprob); when top-p
-//           or top-k truncation is requested, also a 256-bin PER-WAVE
-//           histogram of temperature-scaled probability mass + count
-//           (per-wave copies kill the LDS same-bin atomic serialization that
-//           made a single shared histogram ~50x slower)
-//   pass C: admission threshold from the histogram suffix (top-p by mass,
-//           top-k by count), then up to 3 REFINEMENT sweeps that re-histogram
-//           only the boundary bin at 256x finer resolution each time —
-//           threshold resolution 20/256^4 ~ 5e-9 in scaled-logit space, i.e.
-//           exact top-k/top-p up to fp32 rounding of the logits themselves
+//   sample_part   every row cut into slices, one 256-thread workgroup each: the
+//                 slice's max and argmax, its sum of exp, and - for rows
+//                 without top-p / top-k - the Gumbel-max draw over the slice
+//   sample_final  one workgroup per row: folds the slices; rows with top-p /
+//                 top-k find their threshold and draw here
 //
-//   pass D: Gumbel-max draw over admitted tokens — counter-based RNG
-//           hash(seed, step, token): deterministic, stream-ordered, and
-//           identical regardless of batch composition.
+// Why split: one workgroup per row leaves a 120-row batch on 120 of 256 compute
+// units and a 16-row one on 16, and walks the row three times. The draw, not
+// memory, bounds the split form: per 64 tokens the two 64-bit products of the
+// hash, three transcendentals and the compare take about 280 issue cycles, 27 us
+// for 120 x 128256 tokens on 1024 SIMDs (the logits alone: 61.6 MB, 13 us at the
+// 4.7 TB/s a copy reaches).
 //
-// temperature == 0 -> greedy (argmax + logprob only).
+// Rows with top-p / top-k (sample_final): a 256-bin histogram of the scaled mass
+// and count (per-wave copies: a single one serialises on same-bin LDS atomics)
+// names the boundary bin, up to 3 refinements at 256x finer resolution each
+// (20/256^4 ~ 5e-9 in scaled-logit space: exact up to fp32 rounding of the
+// logits) the threshold in it. Atomics and exponentials are what a sweep costs,
+// so the bins near the max are counted first, with their tokens listed in LDS; a
+// peaked row needs no more. Flat rows take further sweeps, and a boundary bin that
+// outgrows the list is refined by rescans of the row.
+//
+// Measured, 128256 tokens a row, beside one workgroup per row walking it three to
+// six times: 120 rows, half of them with top-p 0.95 and top-k 50, 79 us (346);
+// 16 masked rows 12.2 us (136). sample_part is 29 us of the former, at its bound;
+// sample_final 52, the slowest truncated row's sweeps.
+//
+// The draw is counter-based: hash(seed, step, token), identical regardless of
+// batch composition and of the slicing. temperature == 0 -> greedy.
 
 #include "common.h"
 
-// sx(x) must be BIT-IDENTICAL across pass B (histogram), pass C's
-// refinement rescans and pass D (admission). hipcc contracts even
+// sx(x) must be BIT-IDENTICAL across the histogram, the refinements and the
+// admission. hipcc contracts even
 // __fmul_rn/__fsub_rn pairs into an fma, and may do so at one site but not
 // another — the recomputed sx of the MAX token then comes out as the
 // product's rounding residual (~1e-10, either sign) instead of 0 and falls
@@ -38,10 +49,164 @@ __device__ __forceinline__ float sx_of(float x, float inv_t, float smax) {
 #define NW (NT / WAVE)     // 16 waves
 #define SBINS 256
 #define SRANGE 20.0f       // scaled-logit window below max covered by the histogram
+// bins counted by the first, second and third sweep: scaled logits within 5 of
+// the max, within 10, the rest. A sweep that counts every token is bound by its
+// two LDS atomics (about one lane a cycle: 100 us for 128k tokens), one that counts
+// a few hundred by its loads (8 us); most rows' cut lies within 10
+#define SNEAR 64
+#define SMID 128
+#define SLIST 3072         // tokens listed in LDS (a flat row of 128k tokens has up to ~2500 in its boundary bin)
+#define PT 256             // threads of a slice's workgroup
+#define PU 8               // logits in flight per thread
 
-extern "C" __global__ void __launch_bounds__(NT) sample_kernel(
+// what a slice hands to sample_final: 6 words
+struct SlicePart {
+  float max;
+  float sum;                 // sum of exp(x - max)
+  int arg;                   // lowest token at the max, -1: none above -inf
+  float ssum;                // rows with top-p / top-k: sum of exp((x - max) / temperature)
+  unsigned long long best;   // ordered key bits << 32 | token
+};
+
+__device__ __forceinline__ unsigned long long pack_key(float key, int tok) {
+  uint32_t k = __float_as_uint(key);
+  k = (k & 0x80000000u) ? ~k : (k | 0x80000000u);
+  return ((unsigned long long)k << 32) | (uint32_t)tok;
+}
+
+// key bits of -inf: nothing was drawn
+#define NO_KEY 0x007fffffu
+
+__device__ __forceinline__ uint64_t draw_base(int64_t seed, int64_t step) {
+  return splitmix64((uint64_t)seed * 0x9E3779B97F4A7C15ULL + (uint64_t)step * 0xBF58476D1CE4E5B9ULL);
+}
+
+__device__ __forceinline__ float draw_key(uint64_t base, int tok, float x, float inv_t) {
+  const float u = u64_to_uniform(splitmix64(base ^ (uint64_t)tok));
+  const float gumbel = -__logf(-__logf(u));
+  return x * inv_t + gumbel;
+}
+
+__device__ __forceinline__ bool truncates(float top_p, int top_k, int V) {
+  return (top_p < 1.0f) || (top_k > 0 && top_k < V);
+}
+
+// exp(a - m) with exp(-inf - -inf) taken as an empty sum
+__device__ __forceinline__ float exp_from(float a, float m) {
+  return a == -INFINITY ? 0.0f : __expf(a - m);
+}
+
+__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned long long o = __shfl_xor(v, off);
+    v = o > v ? o : v;
+  }
+  return v;
+}
+
+extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
+    SlicePart* __restrict__ parts,        // [B, slices]
+    const float* __restrict__ logits,     // [B, V]
+    const float* __restrict__ temperatures, const float* __restrict__ top_ps,
+    const int* __restrict__ top_ks, const int64_t* __restrict__ seeds,
+    const int64_t* __restrict__ steps,
+    const uint32_t* __restrict__ mask,    // [B, ceil(V/32)] or nullptr
+    int V, int slice) {
+  const int b = blockIdx.y;
+  const int tid = threadIdx.x;
+  const int lo = blockIdx.x * slice;
+  const int hi = min(V, lo + slice);
+  const float* row = logits + (int64_t)b * V;
+  const uint32_t* mrow = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
+  const float temp = temperatures[b];
+  const bool cuts = temp != 0.0f && truncates(top_ps[b], top_ks[b], V);
+  const bool draw = temp != 0.0f && !cuts;
+  const float inv_t = (temp > 0.0f) ? 1.0f / temp : 0.0f;
+  const uint64_t base = draw_base(seeds[b], steps[b]);
+
+  float m = -INFINITY, sum = 0.0f, ssum = 0.0f, best = -INFINITY;
+  int arg = -1, btok = 0;
+  for (int i0 = lo + tid; i0 < hi; i0 += PT * PU) {
+    float x[PU];
+    bool ok[PU];
+#pragma unroll
+    for (int j = 0; j < PU; ++j) {
+      const int i = i0 + j * PT;
+      ok[j] = i < hi;
+      x[j] = ok[j] ? row[i] : -INFINITY;
+    }
+    if (mrow) {
+#pragma unroll
+      for (int j = 0; j < PU; ++j) {
+        const int i = i0 + j * PT;
+        if (ok[j]) ok[j] = (mrow[i >> 5] >> (i & 31)) & 1;
+        if (!ok[j]) x[j] = -INFINITY;
+      }
+    }
+    float cm = x[0];
+#pragma unroll
+    for (int j = 1; j < PU; ++j) cm = fmaxf(cm, x[j]);
+    if (cm > m) {
+      sum *= exp_from(m, cm);
+      ssum *= m == -INFINITY ? 0.0f : __expf((m - cm) * inv_t);
+      m = cm;
+#pragma unroll
+      for (int j = PU - 1; j >= 0; --j)
+        if (x[j] == cm) arg = i0 + j * PT;
+    }
+#pragma unroll
+    for (int j = 0; j < PU; ++j) sum += exp_from(x[j], m);
+    if (cuts) {
+#pragma unroll
+      for (int j = 0; j < PU; ++j)
+        if (ok[j]) ssum += __expf((x[j] - m) * inv_t);
+    }
+    if (draw) {
+#pragma unroll
+      for (int j = 0; j < PU; ++j) {
+        if (!ok[j]) continue;
+        const float key = draw_key(base, i0 + j * PT, x[j], inv_t);
+        if (key > best) { best = key; btok = i0 + j * PT; }
+      }
+    }
+  }
+
+  // fold the threads: max, lowest token at it, rescaled sums, best key
+  __shared__ float red[16];
+  __shared__ unsigned long long sh_best[PT / WAVE];
+  __shared__ int sh_arg[PT / WAVE];
+  const float M = block_reduce_max<PT / WAVE>(m, red);
+  const float S = block_reduce_sum<PT / WAVE>(sum * (m == M ? 1.0f : exp_from(m, M)), red);
+  const float SS = cuts ? block_reduce_sum<PT / WAVE>(ssum * (m == M ? 1.0f : __expf((m - M) * inv_t)), red) : 0.0f;
+  int a = (m == M && arg >= 0) ? arg : 0x7fffffff;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) a = min(a, __shfl_xor(a, off));
+  const unsigned long long w = wave_max_u64(pack_key(best, btok));
+  if ((tid & 63) == 0) { sh_best[tid >> 6] = w; sh_arg[tid >> 6] = a; }
+  __syncthreads();
+  if (tid == 0) {
+    SlicePart p;
+    p.max = M;
+    p.sum = S;
+    p.best = sh_best[0];
+    p.arg = sh_arg[0];
+#pragma unroll
+    for (int k = 1; k < PT / WAVE; ++k) {
+      p.best = sh_best[k] > p.best ? sh_best[k] : p.best;
+      p.arg = min(p.arg, sh_arg[k]);
+    }
+    if (p.arg == 0x7fffffff) p.arg = -1;
+    p.ssum = SS;
+    parts[(int64_t)b * gridDim.x + blockIdx.x] = p;
+  }
+}
+
+extern "C" __global__ void __launch_bounds__(NT) sample_final_kernel(
     int64_t* __restrict__ out_tokens,     // [B]
     float* __restrict__ out_logprobs,     // [B]
+    const SlicePart* __restrict__ parts,  // [B, slices], slices <= 64
+    int slices,
     const float* __restrict__ logits,     // [B, V]
     const float* __restrict__ temperatures,
     const float* __restrict__ top_ps,
@@ -59,75 +224,62 @@ extern "C" __global__ void __launch_bounds__(NT) sample_kernel(
   const float temp = temperatures[b];
   const float top_p = top_ps[b];
   const int top_k = top_ks[b];
-  const bool truncate = (top_p < 1.0f) || (top_k > 0 && top_k < V);
+  const float inv_t = (temp > 0.0f) ? 1.0f / temp : 0.0f;
 
-  __shared__ float red[16];
-  __shared__ float sh_thresh;
+  __shared__ float sh_max, sh_sum, sh_ssum;
   __shared__ int sh_argmax;
   __shared__ unsigned long long sh_best;
-  extern __shared__ __attribute__((aligned(16))) char hist_smem[];
-  float* hist_mass = reinterpret_cast<float*>(hist_smem);              // [NW][SBINS]
-  unsigned int* hist_cnt = reinterpret_cast<unsigned int*>(hist_mass + NW * SBINS);
-
-  if (truncate) {
-    for (int i = tid; i < NW * SBINS; i += NT) {
-      hist_mass[i] = 0.0f;
-      hist_cnt[i] = 0;
+  if (wid == 0) {
+    SlicePart p{-INFINITY, 0.0f, -1, 0.0f, (unsigned long long)NO_KEY << 32};
+    if (lane < slices) p = parts[(int64_t)b * slices + lane];
+    const float M = wave_reduce_max(p.max);
+    const float S = wave_reduce_sum(p.sum * (p.max == M ? 1.0f : exp_from(p.max, M)));
+    // a slice without an allowed token has nothing to add
+    const float SS = wave_reduce_sum(p.arg < 0 ? 0.0f : p.ssum * (p.max == M ? 1.0f : __expf((p.max - M) * inv_t)));
+    int a = (p.max == M && p.arg >= 0) ? p.arg : 0x7fffffff;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) a = min(a, __shfl_xor(a, off));
+    const unsigned long long w = wave_max_u64(p.best);
+    if (lane == 0) {
+      sh_max = M;
+      sh_sum = S;
+      sh_ssum = SS;
+      sh_argmax = a == 0x7fffffff ? 0 : a;
+      sh_best = w;
     }
   }
-  if (tid == 0) { sh_argmax = 0; sh_best = 0; }
   __syncthreads();
-
-  // ---- pass A: masked max + argmax ---------------------------------------
-  float lmax = -INFINITY;
-  int larg = -1;
-  for (int i = tid; i < V; i += NT) {
-    if (mrow && !((mrow[i >> 5] >> (i & 31)) & 1)) continue;
-    const float x = row[i];
-    if (x > lmax) { lmax = x; larg = i; }
-  }
-  const float gmax = block_reduce_max<16>(lmax, red);
-  if (lmax == gmax && larg >= 0) sh_argmax = larg;
-  __syncthreads();
+  const float gmax = sh_max;
+  const float gsum_unscaled = sh_sum;
   const int argmax_tok = sh_argmax;
-
-  // ---- pass B: unscaled sumexp (+ optional scaled-mass histogram) ---------
-  const float inv_t = (temp > 0.0f) ? 1.0f / temp : 0.0f;
-  const float smax = gmax * inv_t;
-  float lsum_unscaled = 0.0f;
-  float lsum_scaled = 0.0f;
-  float* my_mass = hist_mass + wid * SBINS;
-  unsigned int* my_cnt = hist_cnt + wid * SBINS;
-  for (int i = tid; i < V; i += NT) {
-    if (mrow && !((mrow[i >> 5] >> (i & 31)) & 1)) continue;
-    const float x = row[i];
-    lsum_unscaled += __expf(x - gmax);
-    if (truncate) {
-      const float sx = sx_of(x, inv_t, smax);
-      const float w = __expf(sx);
-      lsum_scaled += w;
-      int bin = (int)(-sx * (SBINS / SRANGE));
-      bin = min(bin, SBINS - 1);
-      atomicAdd(&my_mass[bin], w);
-      atomicAdd(&my_cnt[bin], 1u);
-    }
-  }
-  const float gsum_unscaled = block_reduce_sum<16>(lsum_unscaled, red);
-
-  if (temp == 0.0f) {
+  if (temp == 0.0f || !truncates(top_p, top_k, V)) {
     if (tid == 0) {
-      out_tokens[b] = argmax_tok;
-      out_logprobs[b] = row[argmax_tok] - gmax - __logf(gsum_unscaled);
+      const int tok = (temp == 0.0f || (uint32_t)(sh_best >> 32) == NO_KEY) ? argmax_tok
+                                                                           : (int)(sh_best & 0xffffffffu);
+      out_tokens[b] = tok;
+      out_logprobs[b] = row[tok] - gmax - __logf(gsum_unscaled);
     }
     return;
   }
 
-  // ---- pass C: admission threshold ----------------------------------------
-  float x_thresh = -INFINITY;
-  if (truncate) {
-    const float gsum_scaled = block_reduce_sum<16>(lsum_scaled, red);
-    // fold the per-wave histograms: thread j < SBINS owns bin j
-    if (tid < SBINS) {
+  __shared__ float hist_mass[NW * SBINS];
+  __shared__ unsigned int hist_cnt[NW * SBINS];
+  __shared__ float list_sx[SLIST];
+  __shared__ int list_tok[SLIST];
+  __shared__ int sh_listed;
+  const float smax = gmax * inv_t;
+  float* my_mass = hist_mass + wid * SBINS;
+  unsigned int* my_cnt = hist_cnt + wid * SBINS;
+  auto clear_hist = [&]() {
+    for (int i = tid; i < NW * SBINS; i += NT) {
+      hist_mass[i] = 0.0f;
+      hist_cnt[i] = 0;
+    }
+  };
+  // fold the per-wave histograms over bins [from, to): thread j owns bin j; the
+  // copy of wave 0 becomes the whole
+  auto fold_hist = [&](int from, int to) {
+    if (tid >= from && tid < to) {
       float m = 0.0f;
       unsigned int c = 0;
 #pragma unroll 4
@@ -138,111 +290,253 @@ extern "C" __global__ void __launch_bounds__(NT) sample_kernel(
       hist_mass[tid] = m;
       hist_cnt[tid] = c;
     }
-    __syncthreads();
-    // boundary-interval state (sx space: 0 at the max, negative below);
-    // need_* is the admission still OWED by the boundary interval after
-    // everything strictly above it is admitted. MEMBERSHIP in the boundary
-    // interval is tested by re-evaluating the PREVIOUS level's exact binning
-    // expression (sel_*) — never by interval comparisons, which disagree
-    // with the truncating multiply by an ulp at bin edges (and at sx ~ 0).
-    __shared__ float sh_lo, sh_hi, sh_need_mass;
-    __shared__ float sh_sel_hi, sh_sel_invw;
-    __shared__ int sh_sel_cut, sh_sel_coarse;
-    __shared__ unsigned int sh_need_cnt;
-    __shared__ int sh_state;  // 0 = threshold at sh_lo, 1 = refine, 2 = admit all
-    if (tid == 0) {
-      const float need_mass = top_p < 1.0f ? top_p * gsum_scaled : INFINITY;
-      const unsigned int need_cnt =
-          (top_k > 0 && top_k < V) ? (unsigned)top_k : 0xffffffffu;
-      float acc_mass = 0.0f;
-      unsigned int acc_cnt = 0;
-      int cut_bin = -1;
-      for (int bn = 0; bn < SBINS; ++bn) {
-        acc_mass += hist_mass[bn];
-        acc_cnt += hist_cnt[bn];
-        if (acc_mass >= need_mass || acc_cnt >= need_cnt) { cut_bin = bn; break; }
+  };
+  // f(token, x, sx) over the row's allowed tokens whose sx is not at or below
+  // ``from`` (NaN: all of them). One workgroup hides a sweep's latency by bytes
+  // in flight alone: 128 a thread, as 16-byte loads from the row's first aligned
+  // token on.
+  auto sweep = [&](float from, auto f) {
+    auto one = [&](int i, float x) {
+      const float sx = sx_of(x, inv_t, smax);
+      if (!(sx <= from) && (!mrow || ((mrow[i >> 5] >> (i & 31)) & 1))) f(i, x, sx);
+    };
+    const int head = min((int)((4 - (((int64_t)b * V) & 3)) & 3), V);
+    const int nvec = (V - head) / 4;
+    const f32x4* rv = reinterpret_cast<const f32x4*>(row + head);
+    for (int i0 = tid; i0 < nvec; i0 += NT * 8) {
+      f32x4 x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = rv[min(i0 + j * NT, nvec - 1)];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int v = i0 + j * NT;
+        bool any = false;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) any |= !(sx_of(x[j][k], inv_t, smax) <= from);
+        if (v < nvec && any) {
+          const int i = head + v * 4;
+          for (int k = 0; k < 4; ++k) one(i + k, k == 0 ? x[j][0] : k == 1 ? x[j][1] : k == 2 ? x[j][2] : x[j][3]);
+        }
       }
-      if (cut_bin < 0) {
-        sh_state = 2;  // window never met the need: admit everything
-      } else {
-        const float binw = SRANGE / SBINS;
-        const float before_mass = acc_mass - hist_mass[cut_bin];
-        const unsigned int before_cnt = acc_cnt - hist_cnt[cut_bin];
-        sh_lo = -(cut_bin + 1) * binw;
-        sh_hi = -cut_bin * binw;
-        sh_need_mass = need_mass - before_mass;
-        sh_need_cnt = (need_cnt == 0xffffffffu) ? 0xffffffffu : need_cnt - before_cnt;
-        sh_sel_coarse = 1;
-        sh_sel_cut = cut_bin;
-        // the whole bin is exactly owed -> no refinement needed
-        sh_state = (hist_cnt[cut_bin] == sh_need_cnt) ? 0 : 1;
-        if (dbg) {
-          dbg[b * 16 + 0] = (float)cut_bin;
-          dbg[b * 16 + 1] = (float)hist_cnt[cut_bin];
-          dbg[b * 16 + 2] = (float)sh_need_cnt;
-          dbg[b * 16 + 3] = (float)sh_state;
+    }
+    if (tid < head) one(tid, row[tid]);
+    const int tail = head + nvec * 4 + tid;
+    if (tail < V) one(tail, row[tail]);
+  };
+  auto coarse_bin = [](float sx) { return min((int)(-sx * (SBINS / SRANGE)), SBINS - 1); };
+
+  // boundary-interval state (sx space: 0 at the max, negative below);
+  // need_* is the admission still OWED by the boundary interval after
+  // everything strictly above it is admitted. MEMBERSHIP in the boundary
+  // interval is tested by re-evaluating the PREVIOUS level's exact binning
+  // expression (sel_*) — never by interval comparisons, which disagree
+  // with the truncating multiply by an ulp at bin edges (and at sx ~ 0).
+  __shared__ float sh_lo, sh_hi, sh_need_mass;
+  __shared__ float sh_sel_hi, sh_sel_invw;
+  __shared__ int sh_sel_cut, sh_sel_coarse, sh_cut;
+  __shared__ unsigned int sh_need_cnt;
+  __shared__ int sh_state;  // 0 = threshold at sh_lo, 1 = refine, 2 = admit all
+  // first of the folded bins [0, n) where the running mass or count meets the
+  // need, with what lies before it; -1: none. Wave 0 only, four bins a lane (one
+  // thread's walk over 256 bins in LDS takes 14 us)
+  auto find_cut = [&](int n, float need_mass, unsigned int need_cnt, float& before_mass, unsigned int& before_cnt) {
+    float m[4];
+    unsigned int c[4];
+    float ms = 0.0f;
+    unsigned int cs = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      m[k] = hist_mass[lane * 4 + k];
+      c[k] = hist_cnt[lane * 4 + k];
+      ms += m[k];
+      cs += c[k];
+    }
+    float mi = ms;
+    unsigned int ci = cs;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const float mo = __shfl_up(mi, off);
+      const unsigned int co = __shfl_up(ci, off);
+      if (lane >= off) { mi += mo; ci += co; }
+    }
+    float mb = __shfl_up(mi, 1);
+    unsigned int cb = __shfl_up(ci, 1);
+    if (lane == 0) { mb = 0.0f; cb = 0; }
+    int hit = -1;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (hit < 0) {
+        if (lane * 4 + k < n && (mb + m[k] >= need_mass || cb + c[k] >= need_cnt)) {
+          hit = lane * 4 + k;
+        } else {
+          mb += m[k];
+          cb += c[k];
+        }
+      }
+    }
+    const unsigned long long any = __ballot(hit >= 0);
+    if (!any) return -1;
+    const int src = __ffsll(any) - 1;
+    before_mass = __shfl(mb, src);
+    before_cnt = __shfl(cb, src);
+    return __shfl(hit, src);
+  };
+
+  // ---- histogram of the scaled mass, boundary bin --------------------------
+  // The bins near the max first, their tokens listed: a peaked row's cut lies
+  // there, and the list then stands in for the row.
+  const float need_mass = top_p < 1.0f ? top_p * sh_ssum : INFINITY;
+  const unsigned int need_cnt = (top_k > 0 && top_k < V) ? (unsigned)top_k : 0xffffffffu;
+  const uint64_t base = draw_base(seeds[b], steps[b]);
+  clear_hist();
+  if (tid == 0) { sh_listed = 0; sh_best = (unsigned long long)NO_KEY << 32; }
+  __syncthreads();
+  for (int part = 0; part < 3; ++part) {
+    const int from = part == 0 ? 0 : part == 1 ? SNEAR : SMID;
+    const int to = part == 0 ? SNEAR : part == 1 ? SMID : SBINS;
+    sweep(part < 2 ? -to * (SRANGE / SBINS) - 1e-3f : NAN, [&](int i, float x, float sx) {
+      const int bin = coarse_bin(sx);
+      if (bin < from || bin >= to) return;
+      atomicAdd(&my_mass[bin], __expf(sx));
+      atomicAdd(&my_cnt[bin], 1u);
+      if (part < 2) {
+        const int at = atomicAdd(&sh_listed, 1);
+        if (at < SLIST) {
+          list_sx[at] = sx;
+          list_tok[at] = i;
+        }
+      }
+    });
+    __syncthreads();
+    fold_hist(from, to);
+    __syncthreads();
+    if (wid == 0) {
+      float before_mass = 0.0f;
+      unsigned int before_cnt = 0;
+      const int cut_bin = find_cut(to, need_mass, need_cnt, before_mass, before_cnt);
+      if (lane == 0) {
+        if (cut_bin < 0) {
+          sh_state = 2;  // window never met the need: admit everything
+          sh_cut = SBINS;
+          sh_lo = -INFINITY;
+        } else {
+          const float binw = SRANGE / SBINS;
+          sh_lo = -(cut_bin + 1) * binw;
+          sh_hi = -cut_bin * binw;
+          sh_need_mass = need_mass - before_mass;
+          sh_need_cnt = (need_cnt == 0xffffffffu) ? 0xffffffffu : need_cnt - before_cnt;
+          sh_sel_coarse = 1;
+          sh_sel_cut = cut_bin;
+          sh_cut = cut_bin;
+          // the whole bin is exactly owed -> no refinement needed
+          sh_state = (hist_cnt[cut_bin] == sh_need_cnt) ? 0 : 1;
+          if (dbg) {
+            dbg[b * 16 + 0] = (float)cut_bin;
+            dbg[b * 16 + 1] = (float)hist_cnt[cut_bin];
+            dbg[b * 16 + 2] = (float)sh_need_cnt;
+            dbg[b * 16 + 3] = (float)sh_state;
+          }
         }
       }
     }
     __syncthreads();
+    if (sh_cut < SBINS) break;
+  }
 
-    // refinement: re-histogram ONLY the boundary interval at 256x finer
-    // resolution; each sweep divides the threshold uncertainty by SBINS
-    for (int it = 0; it < 3; ++it) {
-      if (sh_state != 1) break;
-      const float lo = sh_lo, hi = sh_hi;
-      const float inv_w = SBINS / (hi - lo);
-      for (int i = tid; i < NW * SBINS; i += NT) {
-        hist_mass[i] = 0.0f;
-        hist_cnt[i] = 0;
-      }
-      __syncthreads();
-      const int sel_coarse = sh_sel_coarse;
-      const int sel_cut = sh_sel_cut;
-      const float sel_hi = sh_sel_hi;
-      const float sel_invw = sh_sel_invw;
-      for (int i = tid; i < V; i += NT) {
-        if (mrow && !((mrow[i >> 5] >> (i & 31)) & 1)) continue;
-        const float sx = sx_of(row[i], inv_t, smax);
-        // membership = the EXACT bin the previous level counted this token
-        // into equals its boundary bin (bit-identical re-evaluation)
-        int pb;
-        if (sel_coarse) {
-          pb = min((int)(-sx * (SBINS / SRANGE)), SBINS - 1);
-        } else {
-          pb = min(max((int)((sel_hi - sx) * sel_invw), 0), SBINS - 1);
+  // ---- draw over the bins above the boundary --------------------------------
+  // afterwards the list holds the boundary bin's tokens, among others, unless
+  // they outgrow it
+  const int cut = sh_cut;
+  const bool near = cut < SMID && sh_listed <= SLIST;
+  const bool fits = near || (cut < SBINS && hist_cnt[cut] <= SLIST);
+  float best = -INFINITY;
+  int btok = argmax_tok;
+  auto consider = [&](int i, float x) {
+    const float key = draw_key(base, i, x, inv_t);
+    if (key > best) { best = key; btok = i; }
+  };
+  if (near) {
+    const int n = sh_listed;
+    for (int e = tid; e < n; e += NT)
+      if (coarse_bin(list_sx[e]) < cut) consider(list_tok[e], row[list_tok[e]]);
+  } else {
+    __syncthreads();
+    if (tid == 0) sh_listed = 0;
+    __syncthreads();
+    sweep(cut == SBINS ? NAN : -(cut + 1) * (SRANGE / SBINS) - 1e-3f, [&](int i, float x, float sx) {
+      const int bin = coarse_bin(sx);
+      if (cut == SBINS || bin < cut) {
+        consider(i, x);
+      } else if (fits && bin == cut) {
+        const int at = atomicAdd(&sh_listed, 1);
+        if (at < SLIST) {
+          list_sx[at] = sx;
+          list_tok[at] = i;
         }
-        if (pb != sel_cut) continue;
-        int bn = (int)((hi - sx) * inv_w);
-        bn = min(max(bn, 0), SBINS - 1);
-        atomicAdd(&my_mass[bn], __expf(sx));
-        atomicAdd(&my_cnt[bn], 1u);
       }
-      __syncthreads();
-      if (tid < SBINS) {
-        float m = 0.0f;
-        unsigned int c = 0;
-#pragma unroll 4
-        for (int w = 0; w < NW; ++w) {
-          m += hist_mass[w * SBINS + tid];
-          c += hist_cnt[w * SBINS + tid];
+    });
+  }
+  __syncthreads();
+  const int listed = min(sh_listed, SLIST);
+  // f(token, sx) over the boundary bin's tokens
+  auto boundary = [&](auto f) {
+    if (fits) {
+      for (int e = tid; e < listed; e += NT)
+        if (coarse_bin(list_sx[e]) == cut) f(list_tok[e], list_sx[e]);
+    } else {
+      sweep(NAN, [&](int i, float x, float sx) {
+        if (coarse_bin(sx) == cut) f(i, sx);
+      });
+    }
+  };
+
+  // refinement: re-histogram ONLY the boundary interval at 256x finer
+  // resolution; each level divides the threshold uncertainty by SBINS
+  for (int it = 0; it < 3; ++it) {
+    if (sh_state != 1) break;
+    const float lo = sh_lo, hi = sh_hi;
+    const float inv_w = SBINS / (hi - lo);
+    const int sel_coarse = sh_sel_coarse;
+    const int sel_cut = sh_sel_cut;
+    const float sel_hi = sh_sel_hi;
+    const float sel_invw = sh_sel_invw;
+    clear_hist();
+    __syncthreads();
+    boundary([&](int, float sx) {
+      // membership = the EXACT bin the previous level counted this token
+      // into equals its boundary bin (bit-identical re-evaluation)
+      if (!sel_coarse && min(max((int)((sel_hi - sx) * sel_invw), 0), SBINS - 1) != sel_cut) return;
+      int bn = (int)((hi - sx) * inv_w);
+      bn = min(max(bn, 0), SBINS - 1);
+      atomicAdd(&my_mass[bn], __expf(sx));
+      atomicAdd(&my_cnt[bn], 1u);
+    });
+    __syncthreads();
+    fold_hist(0, SBINS);
+    __syncthreads();
+    if (wid == 0) {
+      float before_mass = 0.0f;
+      unsigned int before_cnt = 0;
+      int cut_bin = find_cut(SBINS, sh_need_mass, sh_need_cnt, before_mass, before_cnt);
+      if (cut_bin < 0) {
+        // the need is met inside [lo, hi) up to the rounding of the sums: the
+        // last bin, with all the others before it
+        cut_bin = SBINS - 1;
+        before_mass = 0.0f;
+        before_cnt = 0;
+        for (int k = 0; k < 4; ++k) {
+          const int bn = lane * 4 + k;
+          before_mass += bn < SBINS - 1 ? hist_mass[bn] : 0.0f;
+          before_cnt += bn < SBINS - 1 ? hist_cnt[bn] : 0u;
         }
-        hist_mass[tid] = m;
-        hist_cnt[tid] = c;
+        before_mass = wave_reduce_sum(before_mass);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) before_cnt += __shfl_xor(before_cnt, off);
       }
-      __syncthreads();
-      if (tid == 0) {
-        float acc_mass = 0.0f;
-        unsigned int acc_cnt = 0;
-        int cut_bin = SBINS - 1;  // need is guaranteed met inside [lo, hi)
-        for (int bn = 0; bn < SBINS; ++bn) {
-          acc_mass += hist_mass[bn];
-          acc_cnt += hist_cnt[bn];
-          if (acc_mass >= sh_need_mass || acc_cnt >= sh_need_cnt) { cut_bin = bn; break; }
-        }
+      if (lane == 0) {
         const float subw = (hi - lo) / SBINS;
-        sh_need_mass -= acc_mass - hist_mass[cut_bin];
-        if (sh_need_cnt != 0xffffffffu) sh_need_cnt -= acc_cnt - hist_cnt[cut_bin];
+        sh_need_mass -= before_mass;
+        if (sh_need_cnt != 0xffffffffu) sh_need_cnt -= before_cnt;
         sh_lo = hi - (cut_bin + 1) * subw;
         sh_hi = hi - cut_bin * subw;
         sh_sel_coarse = 0;
@@ -263,45 +557,47 @@ extern "C" __global__ void __launch_bounds__(NT) sample_kernel(
           }
         }
       }
-      __syncthreads();
     }
-    if (sh_state != 2) {
-      // threshold stays in SX space: pass D recomputes each token's sx with
-      // the IDENTICAL f32 expression and compares sx > lo, so the decision
-      // is bit-consistent with the refinement that chose lo (converting
-      // back to x-space loses the ~1e-9 refined margin to fp32 rounding)
-      if (tid == 0) sh_thresh = sh_lo;
-      __syncthreads();
-      x_thresh = sh_thresh;
-    }
+    __syncthreads();
   }
 
-  // ---- pass D: Gumbel-max over admitted tokens ----------------------------
-  const uint64_t base = splitmix64((uint64_t)seeds[b] * 0x9E3779B97F4A7C15ULL +
-                                   (uint64_t)steps[b] * 0xBF58476D1CE4E5B9ULL);
-  float best_key = -INFINITY;
-  int best_tok = argmax_tok;
-  for (int i = tid; i < V; i += NT) {
-    if (mrow && !((mrow[i >> 5] >> (i & 31)) & 1)) continue;
-    const float x = row[i];
-    // sx-space admission, exclusive lower edge (matches the (lo, hi] bin
-    // convention of passes B/C); x_thresh = -inf admits everything
-    if (sx_of(x, inv_t, smax) <= x_thresh) continue;
-    const float u = u64_to_uniform(splitmix64(base ^ (uint64_t)i));
-    const float gumbel = -__logf(-__logf(u));
-    const float key = x * inv_t + gumbel;
-    if (key > best_key) { best_key = key; best_tok = i; }
+  // ---- draw over what the boundary bin admits ------------------------------
+  if (cut < SBINS) {
+    // the threshold stays in sx space (converting it back to x loses the
+    // refined margin to fp32 rounding), exclusive at its lower edge as the bins
+    const float thresh = sh_lo;
+    boundary([&](int i, float sx) {
+      if (sx > thresh) consider(i, row[i]);
+    });
   }
-  {
-    uint32_t kbits = __float_as_uint(best_key);
-    kbits = (kbits & 0x80000000u) ? ~kbits : (kbits | 0x80000000u);
-    const unsigned long long packed = ((unsigned long long)kbits << 32) | (uint32_t)best_tok;
-    atomicMax(&sh_best, packed);
-  }
+  const unsigned long long w = wave_max_u64(pack_key(best, btok));
+  if (lane == 0) atomicMax(&sh_best, w);
   __syncthreads();
   if (tid == 0) {
     const int tok = (int)(sh_best & 0xffffffffu);
     out_tokens[b] = tok;
     out_logprobs[b] = row[tok] - gmax - __logf(gsum_unscaled);
   }
+}
+
+// rows -> slices: about eight 256-thread workgroups per compute unit, no slice
+// under 2048 tokens (one load round per thread) and at most 64 slices a row (one
+// per lane of sample_final's fold)
+extern "C" int sample_slices(int B, int V) {
+  const int most = (V + PT * PU - 1) / (PT * PU);
+  const int want = (2048 + B - 1) / B;
+  const int n = want < most ? want : most;
+  return n < 1 ? 1 : n > 64 ? 64 : n;
+}
+
+extern "C" void launch_sample(int64_t* tokens, float* logprobs, void* parts, const float* logits,
+                              const float* temps, const float* top_ps, const int* top_ks,
+                              const int64_t* seeds, const int64_t* steps, const uint32_t* mask, int B,
+                              int V, float* dbg, hipStream_t stream) {
+  const int n = sample_slices(B, V);
+  const int slice = (V + n - 1) / n;
+  hipLaunchKernelGGL(sample_part_kernel, dim3(n, B), dim3(PT), 0, stream, (SlicePart*)parts, logits,
+                     temps, top_ps, top_ks, seeds, steps, mask, V, slice);
+  hipLaunchKernelGGL(sample_final_kernel, dim3(B), dim3(NT), 0, stream, tokens, logprobs,
+                     (const SlicePart*)parts, n, logits, temps, top_ps, top_ks, seeds, steps, mask, V, dbg);
 }

@@ -1,0 +1,80 @@
+"""The sliced sampler against the same draw in float64: slice edges, short
+rows, ragged vocabularies, masks, boundary bins that outgrow the LDS list."""
+
+import numpy as np
+import pytest
+import torch
+
+from kllms_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def splitmix(x):
+    with np.errstate(over="ignore"):
+        x = x + np.uint64(0x9E3779B97F4A7C15)
+        x = (x ^ (x >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        x = (x ^ (x >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        return x ^ (x >> np.uint64(31))
+
+
+def gumbel(seed, step, V):
+    """float64 Gumbel values of one row's counter-based draw (the uniform is formed in float32, as the kernel's)."""
+    with np.errstate(over="ignore"):
+        base = splitmix(np.uint64(seed) * np.uint64(0x9E3779B97F4A7C15) + np.uint64(step) * np.uint64(0xBF58476D1CE4E5B9))
+    h = splitmix(base ^ np.arange(V, dtype=np.uint64)) >> np.uint64(40)
+    u = (h + np.uint64(1)).astype(np.float32) * np.float32(1.0 / 16777217.0)
+    return -np.log(-np.log(u.astype(np.float64)))
+
+
+@pytest.mark.parametrize("mode", ["plain", "greedy", "masked", "top_k", "top_p", "both", "crowded"])
+@pytest.mark.parametrize("B,V", [(1, 1), (2, 5), (3, 63), (1, 2047), (1, 2048), (2, 2049), (5, 8193), (33, 32000),
+                                 (250, 4099), (3, 131071)])
+def test_draw_matches_float64(B, V, mode):
+    g = torch.Generator().manual_seed(V * 7 + B)
+    logits = torch.randn(B, V, generator=g) * (0.01 if mode == "crowded" else 3.0)
+    temp = torch.zeros(B) if mode == "greedy" else torch.rand(B, generator=g) * 0.8 + 0.4
+    top_p = torch.full((B,), 0.8 if mode in ("top_p", "both") else 1.0)
+    top_k = torch.full((B,), 9 if mode in ("top_k", "both", "crowded") else 0, dtype=torch.int32)
+    if mode == "both" and B > 1:
+        top_p[0], top_k[0] = 1.0, 0          # a row without truncation among the others
+    seeds = torch.randint(0, 2**40, (B,), generator=g)
+    steps = torch.randint(0, 99, (B,), generator=g)
+    mask = None
+    x = logits.double().numpy()
+    if mode == "masked":
+        bits = torch.rand(B, (V + 31) // 32 * 32, generator=g) < 0.2
+        bits[:, 0] = True
+        w = (bits.view(B, -1, 32).long() << torch.arange(32)).sum(-1)
+        mask = torch.where(w >= 2**31, w - 2**32, w).to(torch.int32)
+        x = np.where(bits[:, :V].numpy(), x, -np.inf)
+    dev = lambda t: t.to(DEV)  # noqa: E731
+    toks, lps = ops.sample(dev(logits), dev(temp.float()), dev(top_p.float()), dev(top_k), dev(seeds), dev(steps),
+                           None if mask is None else dev(mask))
+    toks, lps = toks.cpu().numpy(), lps.cpu().numpy()
+    for b in range(B):
+        t = int(toks[b])
+        assert 0 <= t < V
+        m = x[b].max()
+        ref = x[b, t] - m - np.log(np.exp(x[b] - m).sum())
+        # fp32: the logits' own rounding (1e-6 at 16) and a tree sum of V terms
+        assert abs(lps[b] - ref) < 2e-5
+        if mode == "greedy":
+            assert t == int(x[b].argmax())
+            continue
+        s = x[b] / float(np.float32(temp[b]))
+        order = np.argsort(-s, kind="stable")
+        p = np.exp(s[order] - s.max())
+        p /= p.sum()
+        before = np.cumsum(p) - p
+        k = int(top_k[b]) if int(top_k[b]) > 0 else V
+        # the last member is decided by fp32 mass sums and a threshold rounded to fp32 just below it: the draw may
+        # count it in or out
+        may, must = before < float(top_p[b]) + 1e-5, before + p < float(top_p[b]) - 1e-5
+        may[k:] = must[k:] = False
+        must[0] = True
+        assert t in set(order[may].tolist())
+        key = s + gumbel(int(seeds[b]), int(steps[b]), V)
+        # two fast logarithms in fp32: 1e-7 absolute in the inner one, over a winner's 1 - u of about 1 / V
+        assert key[t] >= key[order[must]].max() - max(1e-3, 4e-7 * V)
