@@ -1,40 +1,69 @@
 // Paged decode attention (single new token per stream) for gfx950.
 //
-// Flash-decoding structure: the context is partitioned into key chunks and
-// each (sequence, kv_head, chunk) is one 256-thread workgroup — with B x KVH
-// blocks alone (e.g. 20 x 8 = 160) the 256-CU chip sits idle, so the chunk
-// split is what fills it. Each block emits a partial (m, l, o[gqa][128]);
-// a small reduce kernel merges chunks with the standard log-sum-exp combine.
+// Flash decoding over 32-key tiles, one tile per WAVE: a wave takes every
+// (Z*4)-th tile of its (stream, kv head), keeps its own running max and sum, and
+// the four waves of a workgroup fold once at the end. Z workgroups share a
+// context; their partials are merged by a second launch (none with Z = 1).
 //
-// Memory behavior: each block streams its chunk of K/V exactly ONCE:
-//   - scores: 8-lane thread groups per key, 16-byte K loads, in-wave reduce;
-//   - online softmax: one wave per head (in-wave shuffles, single barrier);
-//   - V accumulation: threads partition the KEYS (4 partitions x 64 dim-pair
-//     lanes), each thread accumulating ALL q-heads for its dim pair, so a V
-//     row is loaded once per block (a head-partitioned layout re-fetches the
-//     64 KB V tile per head-group wave — it exceeds the 32 KB L1);
-//   - per-key cache-row offsets staged in LDS once per tile.
+// What bounds it is bytes in flight: a wave issues the K and V loads of a whole
+// tile (16 KB in bf16, 64 registers a lane) before it uses any, so twelve waves
+// keep 192 KB in flight per compute unit, and no barrier stands between a wave's
+// scores, softmax and weighted sum. (64-key tiles leave two waves per SIMD, and
+// loading the next tile ahead spills: 43 and 126 us where this takes 36.)
 //
-// The kernel is TEMPLATED on the GQA group size: the per-head accumulator
-// array must be statically indexed (a runtime-gqa loop sends it to scratch —
-// cdna guide §5.4 rule 20) and the head loops fully unrolled.
+//   scores   S[key][head] on the matrix cores (16x16x32): K rows go from memory to
+//            fragments as they lie - lane group g takes dims 32g..32g+31 of its
+//            row, 64 contiguous bytes in four loads, and Q is read in the same
+//            order (a dot product does not care which order its terms have)
+//   softmax  fp32, head per lane column, exchanges over the four lane groups only
+//   P V      fp32 on the vector unit: 16 lanes x 8 dims span a V row, four keys at
+//            a time; P crosses lanes through a wave-private LDS strip
+//
+// Workgroups are laid out kv head fastest: with 8 kv heads each XCD serves one of
+// them, and the streams of a request, neighbours in the batch, find their shared
+// prompt's rows in that XCD's L2.
 //
 // Layouts: q [B, H, D=128]; caches [NB, KVH, BS, D]; block_tables [B, MAXB];
 // context_lens INCLUDE the current token. GQA in {1, 2, 4, 8}.
+//
+// Measured with the merge, 32 heads / 8 kv heads, beside 256-key workgroups with
+// block-wide passes: 120 streams of 560 keys 36.5 us (68), 5 streams 8.5 us (23), 16
+// fp8 streams of 5850 keys 49 us (109, 198 MB: 4 TB/s); 16 / 4 heads, one stream of
+// 170 keys 7.8 us (21).
 
 #include "common.h"
 
-#define TKV ATTN_DECODE_TKV
-#define NTHREADS 256
-#define KLANES 4           // lanes cooperating on one key's dot product
-// chunk size is a runtime arg (adaptive split-K: big batches need no split)
+typedef __bf16 bf16x8_mfma __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// partials layout: [B, KVH, max_chunks, gqa, 130]: 128 o values + m + l
+#define NTHREADS 256
+#define TKEYS 32           // keys of a wave's tile
+// partials layout: [B, KVH, Z, GQA, 130]: 128 o values + m + l
 #define PART_STRIDE 130
 
+union Frag {
+  u32x4 u;
+  bf16x8_mfma m;
+};
+
+// 8 fp8 -> 8 bf16 (every e4m3 value is a bf16 value)
+__device__ __forceinline__ Frag fp8x8_to_bf16(u32x2 v) {
+  Frag f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i], false);
+    const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i], true);
+    f.u[2 * i] = __builtin_amdgcn_perm(__float_as_uint(lo[1]), __float_as_uint(lo[0]), 0x07060302u);
+    f.u[2 * i + 1] = __builtin_amdgcn_perm(__float_as_uint(hi[1]), __float_as_uint(hi[0]), 0x07060302u);
+  }
+  return f;
+}
+
 template <int GQA, bool FP8>
-__global__ __launch_bounds__(NTHREADS) void attn_decode_partial_t(
-    float* __restrict__ partials,
+__global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
+    float* __restrict__ partials, bf16_t* __restrict__ out,  // out: written when gridDim.z == 1
     const bf16_t* __restrict__ q,        // [B, H, 128], row stride q_tstride
     const char* __restrict__ k_cache,    // [NB, KVH, BS, 128], bf16 or fp8
     const char* __restrict__ v_cache,
@@ -42,280 +71,285 @@ __global__ __launch_bounds__(NTHREADS) void attn_decode_partial_t(
     const float* __restrict__ v_scale,
     const int* __restrict__ block_tables,  // [B, max_blocks]
     const int* __restrict__ context_lens,  // [B]
-    float scale, int num_kv_heads,
-    int block_size, int max_blocks, int max_chunks, int q_tstride, int chunk_keys) {
-  const int b = blockIdx.x;
-  const int g_kv = blockIdx.y;
-  const int chunk = blockIdx.z;
+    float scale, int block_size, int max_blocks, int q_tstride) {
+  const int g_kv = blockIdx.x, num_kv_heads = gridDim.x;
+  const int b = blockIdx.y;
+  const int z = blockIdx.z, Z = gridDim.z;
   const int L = context_lens[b];
-  const int c0 = chunk * chunk_keys;
-  if (c0 >= L && chunk > 0) return;     // no keys for this chunk
-  const int c1 = min(L, c0 + chunk_keys);
-  const int tid = threadIdx.x;
+  const int tiles = (L + TKEYS - 1) / TKEYS;
+  if (z * 4 >= tiles && Z > 1) return;   // no keys here: the merge skips this partial
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int col = lane & 15, grp = lane >> 4;
 
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* q_lds = reinterpret_cast<float*>(smem);          // [GQA][128]
-  float* s_lds = q_lds + GQA * 128;                       // [GQA][TKV]
-  float* mstate = s_lds + GQA * TKV;                      // [GQA]
-  float* lstate = mstate + 8;                              // [GQA]
-  float* alpha_lds = lstate + 8;                           // [GQA]
-  float* o_scratch = alpha_lds + 8;                        // [4][GQA][128]
-  int64_t* rowoff = reinterpret_cast<int64_t*>(o_scratch + 4 * GQA * 128);  // [TKV]
-  float* ks_lds = reinterpret_cast<float*>(rowoff + TKV);                   // [TKV] (FP8)
-  float* vs_lds = ks_lds + TKV;                                             // [TKV] (FP8)
+  __shared__ __attribute__((aligned(16))) float p_lds[4][TKEYS * GQA];
+  __shared__ float o_lds[4][GQA * 128];
+  __shared__ float m_lds[4][GQA], l_lds[4][GQA];
+  float* p_me = p_lds[wave];
 
-  for (int i = tid; i < GQA * 128; i += NTHREADS) {
-    const int g = i >> 7, d = i & 127;
-    const bf16_t* qp = q + (int64_t)b * q_tstride + (g_kv * GQA + g) * 128;
-    q_lds[i] = bf16_to_f32(((const short*)qp)[d]) * scale;
-  }
-  if (tid < 8) { mstate[tid] = -INFINITY; lstate[tid] = 0.0f; }
-  __syncthreads();
-
-  float o_part[GQA][2];
+  Frag qf[4];
+  {
+    const short* qp = (const short*)q + (int64_t)b * q_tstride + (g_kv * GQA + min(col, GQA - 1)) * 128 + grp * 32;
 #pragma unroll
-  for (int g = 0; g < GQA; ++g) { o_part[g][0] = 0.f; o_part[g][1] = 0.f; }
-
+    for (int s = 0; s < 4; ++s)
+      qf[s].u = col < GQA ? *reinterpret_cast<const u32x4*>(qp + s * 8) : u32x4{0, 0, 0, 0};
+  }
   const int* bt = block_tables + (int64_t)b * max_blocks;
 
-  for (int tile = c0; tile < c1; tile += TKV) {
-    const int nkeys = min(TKV, c1 - tile);
-    // stage per-key cache-row element offsets (shared by K and V) and, for
-    // fp8 caches, the per-row dequant scales (scale row index = rowoff/128)
-    for (int i = tid; i < nkeys; i += NTHREADS) {
-      const int gk = tile + i;
-      const int64_t off = (((int64_t)bt[gk / block_size] * num_kv_heads + g_kv) * block_size +
-                           (gk % block_size)) * 128;
-      rowoff[i] = off;
+  float m_run = -INFINITY, l_run = 0.0f;   // of head ``col``; l_run: this lane's keys only
+  float o[GQA][8];
+#pragma unroll
+  for (int h = 0; h < GQA; ++h)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[h][j] = 0.0f;
+
+  // cache row of key tile * 32 + (lane & 31); keys behind the context repeat its
+  // last row
+  auto row_of = [&](int tile) {
+    const int kc = min(tile * TKEYS + (lane & (TKEYS - 1)), L - 1);
+    return (bt[kc / block_size] * num_kv_heads + g_kv) * block_size + kc % block_size;
+  };
+  const int t0 = z * 4 + wave;
+  int row_next = t0 < tiles ? row_of(t0) : 0;
+#pragma unroll 1
+  for (int t = t0; t < tiles; t += Z * 4) {
+    const int base = t * TKEYS;
+    const int rowi = row_next;
+    float ks = 1.0f, vs = 1.0f;
+    if constexpr (FP8) { ks = k_scale[rowi]; vs = v_scale[rowi]; }
+    u32x4 kraw[TKEYS / 16][FP8 ? 2 : 4];
+#pragma unroll
+    for (int tt = 0; tt < TKEYS / 16; ++tt) {
+      const int64_t r = __shfl(rowi, tt * 16 + col);
+      const u32x4* kp = reinterpret_cast<const u32x4*>(k_cache + r * (FP8 ? 128 : 256) + grp * (FP8 ? 32 : 64));
+#pragma unroll
+      for (int s = 0; s < (FP8 ? 2 : 4); ++s) kraw[tt][s] = kp[s];
+    }
+    u32x4 vraw[TKEYS / 4];
+#pragma unroll
+    for (int i = 0; i < TKEYS / 4; ++i) {
+      const int64_t r = __shfl(rowi, i * 4 + grp);
       if constexpr (FP8) {
-        ks_lds[i] = k_scale[off >> 7];
-        vs_lds[i] = v_scale[off >> 7];
+        const u32x2 v = *reinterpret_cast<const u32x2*>(v_cache + r * 128 + col * 8);
+        vraw[i][0] = v[0];
+        vraw[i][1] = v[1];
+      } else {
+        vraw[i] = *reinterpret_cast<const u32x4*>(v_cache + r * 256 + col * 16);
       }
     }
-    __syncthreads();
+    row_next = row_of(min(t + Z * 4, tiles - 1));
 
-    // ---- scores: KLANES lanes per key, 128/KLANES bf16 per lane -----------
-    {
-      constexpr int ELEMS = 128 / KLANES;     // per-lane K elements
-      constexpr int VECS = ELEMS / 8;         // 16-byte pieces per lane
-      const int kg = tid / KLANES;
-      const int kl = tid % KLANES;
-      for (int key0 = 0; key0 < nkeys; key0 += NTHREADS / KLANES) {
-        const int key = key0 + kg;
-        if (key < nkeys) {
-          float af[ELEMS];
-          if constexpr (FP8) {
-            const u8x8_vec* kv8 = reinterpret_cast<const u8x8_vec*>(k_cache + rowoff[key]) + kl * VECS;
+    // ---- scores: lane (col, grp) holds keys tt*16 + grp*4 + r of head col ----
+    float sc[TKEYS / 16][4];
+    float tmax = -INFINITY;
 #pragma unroll
-            for (int c = 0; c < VECS; ++c) {
-              u8x8_vec kv = kv8[c];
+    for (int tt = 0; tt < TKEYS / 16; ++tt) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-              for (int j = 0; j < 8; ++j) af[c * 8 + j] = fp8_to_f32(kv[j]);
-            }
-          } else {
-            const bf16x8_vec* kv8 =
-                reinterpret_cast<const bf16x8_vec*>(k_cache + 2 * rowoff[key]) + kl * VECS;
-#pragma unroll
-            for (int c = 0; c < VECS; ++c) {
-              bf16x8_vec kv = kv8[c];
-#pragma unroll
-              for (int j = 0; j < 8; ++j) af[c * 8 + j] = bf16_to_f32(kv[j]);
-            }
-          }
-#pragma unroll
-          for (int g = 0; g < GQA; ++g) {
-            const float* qg = q_lds + g * 128 + kl * ELEMS;
-            float acc = 0.f;
-#pragma unroll
-            for (int j = 0; j < ELEMS; ++j) acc += af[j] * qg[j];
-#pragma unroll
-            for (int off = KLANES / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-            // fp8: fold the key row's dequant scale into the score (q already
-            // carries the softmax scale; s_k is per-key, shared across g)
-            if (kl == 0) s_lds[g * TKV + key] = FP8 ? acc * ks_lds[key] : acc;
-          }
-        }
-      }
-    }
-    __syncthreads();
-
-    // ---- online softmax: one WAVE per head, in-wave reductions only -------
-    {
-      const int wave = tid >> 6;
-      const int wlane = tid & 63;
-      for (int g = wave; g < GQA; g += NTHREADS / 64) {
-        float lm = -INFINITY;
-        for (int i = wlane; i < nkeys; i += 64) lm = fmaxf(lm, s_lds[g * TKV + i]);
-        const float tile_max = wave_reduce_max(lm);
-        const float m_old = mstate[g];
-        const float m_new = fmaxf(m_old, tile_max);
-        const float alpha = (m_old == -INFINITY) ? 0.0f : __expf(m_old - m_new);
-        float ls = 0.f;
-        for (int i = wlane; i < nkeys; i += 64) {
-          const float p = __expf(s_lds[g * TKV + i] - m_new);
-          s_lds[g * TKV + i] = p;
-          ls += p;
-        }
-        const float tile_sum = wave_reduce_sum(ls);
-        if (wlane == 0) {
-          alpha_lds[g] = alpha;
-          mstate[g] = m_new;
-          lstate[g] = lstate[g] * alpha + tile_sum;
-        }
-      }
-    }
-    __syncthreads();
-
-    // ---- V accumulation (key-partitioned, V read once) --------------------
-    {
-      const int kpart = tid >> 6;        // wave id = key partition
-      const int d0 = (tid & 63) * 2;     // this thread's dim pair
-#pragma unroll
-      for (int g = 0; g < GQA; ++g) {
-        const float alpha = alpha_lds[g];
-        o_part[g][0] *= alpha;
-        o_part[g][1] *= alpha;
-      }
-      const int nk4 = (nkeys + 3) >> 2;
-      const int kbeg = kpart * nk4;
-      const int kend = min(nkeys, kbeg + nk4);
-      int key = kbeg;
-      // 4 keys in flight: loads issued before use (hides the per-key chain)
-      for (; key + 4 <= kend; key += 4) {
-        uint32_t pairs[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          if constexpr (FP8)
-            pairs[u] = *reinterpret_cast<const unsigned short*>(v_cache + rowoff[key + u] + d0);
-          else
-            pairs[u] = *reinterpret_cast<const uint32_t*>(v_cache + 2 * (rowoff[key + u] + d0));
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const float vs = FP8 ? vs_lds[key + u] : 1.0f;  // per-row V dequant
-          const float v0 = vs * (FP8 ? fp8_to_f32((unsigned char)(pairs[u] & 0xff))
-                                     : bf16_to_f32((short)(pairs[u] & 0xffff)));
-          const float v1 = vs * (FP8 ? fp8_to_f32((unsigned char)((pairs[u] >> 8) & 0xff))
-                                     : bf16_to_f32((short)(pairs[u] >> 16)));
-#pragma unroll
-          for (int g = 0; g < GQA; ++g) {
-            const float p = s_lds[g * TKV + key + u];  // wave-uniform: LDS broadcast
-            o_part[g][0] += p * v0;
-            o_part[g][1] += p * v1;
-          }
-        }
-      }
-      for (; key < kend; ++key) {
-        uint32_t pair;
+      for (int s = 0; s < 4; ++s) {
+        Frag kf;
         if constexpr (FP8)
-          pair = *reinterpret_cast<const unsigned short*>(v_cache + rowoff[key] + d0);
+          kf = fp8x8_to_bf16(u32x2{kraw[tt][s >> 1][(s & 1) * 2], kraw[tt][s >> 1][(s & 1) * 2 + 1]});
         else
-          pair = *reinterpret_cast<const uint32_t*>(v_cache + 2 * (rowoff[key] + d0));
-        const float vs = FP8 ? vs_lds[key] : 1.0f;
-        const float v0 = vs * (FP8 ? fp8_to_f32((unsigned char)(pair & 0xff))
-                                   : bf16_to_f32((short)(pair & 0xffff)));
-        const float v1 = vs * (FP8 ? fp8_to_f32((unsigned char)((pair >> 8) & 0xff))
-                                   : bf16_to_f32((short)(pair >> 16)));
+          kf.u = kraw[tt][s];
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.m, qf[s].m, acc, 0, 0, 0);
+      }
 #pragma unroll
-        for (int g = 0; g < GQA; ++g) {
-          const float p = s_lds[g * TKV + key];
-          o_part[g][0] += p * v0;
-          o_part[g][1] += p * v1;
-        }
+      for (int r = 0; r < 4; ++r) {
+        const int key = tt * 16 + grp * 4 + r;
+        float x = acc[r] * scale;
+        if constexpr (FP8) x *= __shfl(ks, key);
+        sc[tt][r] = base + key < L ? x : -INFINITY;
+        tmax = fmaxf(tmax, sc[tt][r]);
       }
     }
-    __syncthreads();
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+    const float m_new = fmaxf(m_run, tmax);
+    const float alpha = (m_run == -INFINITY) ? 0.0f : __expf(m_run - m_new);
+    m_run = m_new;
+    l_run *= alpha;
+#pragma unroll
+    for (int tt = 0; tt < TKEYS / 16; ++tt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float p = (sc[tt][r] == -INFINITY) ? 0.0f : __expf(sc[tt][r] - m_new);
+        l_run += p;
+        if (col < GQA) p_me[(tt * 16 + grp * 4 + r) * GQA + col] = p;
+      }
+    // the strip is this wave's own: in-order LDS, only the compiler is held
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int h = 0; h < GQA; ++h) {
+      const float a = __shfl(alpha, h);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[h][j] *= a;
+    }
+
+    // ---- P V: lane (col, grp) adds dims col*8.. of keys i*4 + grp ------------
+#pragma unroll
+    for (int i = 0; i < TKEYS / 4; ++i) {
+      float p[GQA];
+#pragma unroll
+      for (int h = 0; h < GQA; ++h) p[h] = p_me[(i * 4 + grp) * GQA + h];
+      if constexpr (FP8) {
+        const float s = __shfl(vs, i * 4 + grp);
+#pragma unroll
+        for (int h = 0; h < GQA; ++h) p[h] *= s;
+      }
+      float v[8];
+#pragma unroll
+      for (int w = 0; w < (FP8 ? 2 : 4); ++w) {
+        if constexpr (FP8) {
+          const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)vraw[i][w], false);
+          const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)vraw[i][w], true);
+          v[4 * w] = lo[0];
+          v[4 * w + 1] = lo[1];
+          v[4 * w + 2] = hi[0];
+          v[4 * w + 3] = hi[1];
+        } else {
+          v[2 * w] = __uint_as_float(vraw[i][w] << 16);
+          v[2 * w + 1] = __uint_as_float(vraw[i][w] & 0xffff0000u);
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < GQA; ++h)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[h][j] += p[h] * v[j];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 
-  // ---- combine the 4 key partitions, write partial (m, l, o) --------------
-  {
-    const int kpart = tid >> 6;
-    const int d0 = (tid & 63) * 2;
+  // ---- fold the lane groups' keys, then the waves ---------------------------
+  l_run += __shfl_xor(l_run, 16);
+  l_run += __shfl_xor(l_run, 32);
+  // halves, then odd and even rows of 16 lanes: each exchange sums two values and
+  // leaves one in either part, so a lane ends with dims 2*grp' and 2*grp'+1 of its
+  // eight, grp' = the part it landed in
 #pragma unroll
-    for (int g = 0; g < GQA; ++g) {
-      o_scratch[((kpart * GQA + g) * 128) + d0] = o_part[g][0];
-      o_scratch[((kpart * GQA + g) * 128) + d0 + 1] = o_part[g][1];
+  for (int h = 0; h < GQA; ++h) {
+    float half[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[h][j]), __float_as_uint(o[h][j + 4]), false, false);
+      half[j] = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);   // lanes 0-31: dim j, 32-63: dim j + 4
     }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(half[j]), __float_as_uint(half[j + 2]), false, false);
+      const float v = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);  // even rows: dim j, odd rows: dim j + 2
+      o_lds[wave][h * 128 + col * 8 + (lane >> 5) * 4 + (grp & 1) * 2 + j] = v;
+    }
+  }
+  if (lane < GQA) {
+    m_lds[wave][lane] = m_run;
+    l_lds[wave][lane] = l_run;
   }
   __syncthreads();
-  float* base = partials +
-      ((((int64_t)b * num_kv_heads + g_kv) * max_chunks + chunk) * GQA) * PART_STRIDE;
+  float* base = partials + (((int64_t)b * num_kv_heads + g_kv) * Z + z) * GQA * PART_STRIDE;
   for (int i = tid; i < GQA * 128; i += NTHREADS) {
-    const int g = i >> 7, d = i & 127;
-    float acc = 0.f;
+    const int h = i >> 7, d = i & 127;
+    float M = m_lds[0][h];
 #pragma unroll
-    for (int kp = 0; kp < 4; ++kp) acc += o_scratch[((kp * GQA + g) * 128) + d];
-    base[g * PART_STRIDE + d] = acc;
-  }
-  if (tid < 8 && tid < GQA) {
-    float* pg = base + tid * PART_STRIDE;
-    pg[128] = mstate[tid];
-    pg[129] = lstate[tid];
+    for (int w = 1; w < 4; ++w) M = fmaxf(M, m_lds[w][h]);
+    float acc = 0.0f, l = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float e = m_lds[w][h] == -INFINITY ? 0.0f : __expf(m_lds[w][h] - M);   // a wave without a tile
+      acc += o_lds[w][i] * e;
+      l += l_lds[w][h] * e;
+    }
+    if (Z == 1) {
+      const float v = l > 0.0f ? acc / l : 0.0f;
+      ((short*)out)[((int64_t)b * num_kv_heads * GQA + g_kv * GQA + h) * 128 + d] = f32_to_bf16(v);
+    } else {
+      base[h * PART_STRIDE + d] = acc;
+      if (d == 0) {
+        base[h * PART_STRIDE + 128] = M;
+        base[h * PART_STRIDE + 129] = l;
+      }
+    }
   }
 }
 
-// host-side dispatcher: picks the GQA template instantiation
-extern "C" void launch_attn_decode_partial(
-    float* partials, const bf16_t* q, const void* k_cache, const void* v_cache,
-    const float* k_scale, const float* v_scale,
-    const int* block_tables, const int* context_lens, float scale,
-    int num_q_heads, int num_kv_heads, int block_size, int max_blocks,
-    int max_chunks, int q_tstride, int chunk_keys, int B, int cache_fp8,
-    hipStream_t stream) {
+// Workgroups per context: about 640 in all, and never more than the longest
+// context has groups of four tiles. Below that the chip is not full, above it the
+// merge and the workgroups' fixed part (lengths, table, fold: 4 us) cost more than
+// the shorter loops give. With the merge, bf16, 960 (stream, kv head) pairs of 560
+// keys: 36.5 us with 1, 42 with 2, 47 with 8; fp8, 128 pairs of 5850 keys: 114 with
+// 1, 58 with 3, 49 with 4 to 6, 54 with 24.
+extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx) {
+  const int most = (max_ctx + 4 * TKEYS - 1) / (4 * TKEYS);
+  const int want = (640 + B * num_kv_heads / 2) / (B * num_kv_heads);
+  const int z = want < most ? want : most;
+  return z < 1 ? 1 : z;
+}
+
+// merge the partials of a (stream, q head): two dims per lane, the partials dealt
+// to four waves
+__global__ void __launch_bounds__(256) attn_decode_merge_kernel(
+    bf16_t* __restrict__ out,            // [B, H, 128]
+    const float* __restrict__ partials,  // [B, KVH, Z, gqa, 130]
+    const int* __restrict__ context_lens, int gqa, int Z) {
+  const int b = blockIdx.y, h = blockIdx.x, num_q_heads = gridDim.x;
+  const int g_kv = h / gqa, g = h % gqa;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tiles = (context_lens[b] + TKEYS - 1) / TKEYS;
+  const int n = min(Z, (tiles + 3) / 4);
+  const float* base = partials + (((int64_t)b * (num_q_heads / gqa) + g_kv) * Z * gqa + g) * PART_STRIDE;
+  const int64_t step = (int64_t)gqa * PART_STRIDE;
+  float m = -INFINITY;
+  for (int c = lane; c < n; c += 64) m = fmaxf(m, base[c * step + 128]);
+  m = wave_reduce_max(m);
+  float a0 = 0.0f, a1 = 0.0f, l = 0.0f;
+#pragma unroll 4
+  for (int c = wave; c < n; c += 4) {
+    const float* p = base + c * step;
+    const float w = __expf(p[128] - m);
+    const f32x2 v = *reinterpret_cast<const f32x2*>(p + lane * 2);
+    l += p[129] * w;
+    a0 += v[0] * w;
+    a1 += v[1] * w;
+  }
+  __shared__ float sh_o[4][128], sh_l[4];
+  sh_o[wave][lane * 2] = a0;
+  sh_o[wave][lane * 2 + 1] = a1;
+  if (lane == 0) sh_l[wave] = l;
+  __syncthreads();
+  const int d = threadIdx.x;
+  if (d < 128) {
+    const float acc = sh_o[0][d] + sh_o[1][d] + sh_o[2][d] + sh_o[3][d];
+    const float lt = sh_l[0] + sh_l[1] + sh_l[2] + sh_l[3];
+    ((short*)out)[((int64_t)b * num_q_heads + h) * 128 + d] = f32_to_bf16(lt > 0.0f ? acc / lt : 0.0f);
+  }
+}
+
+// picks the GQA instantiation (the binding admits 1, 2, 4, 8); partials: room for
+// B * KVH * splits * gqa * 130 floats when splits > 1
+extern "C" void launch_attn_decode(
+    bf16_t* out, float* partials, const bf16_t* q, const void* k_cache, const void* v_cache,
+    const float* k_scale, const float* v_scale, const int* block_tables, const int* context_lens,
+    float scale, int num_q_heads, int num_kv_heads, int block_size, int max_blocks, int splits,
+    int q_tstride, int B, int cache_fp8, hipStream_t stream) {
   const int gqa = num_q_heads / num_kv_heads;
-  const dim3 grid(B, num_kv_heads, max_chunks);
-  const size_t lds = (gqa * 128 + gqa * TKV + 24 + 4 * gqa * 128) * sizeof(float) +
-                     TKV * sizeof(int64_t) + 2 * TKV * sizeof(float);
-#define LAUNCH(G, F)                                                                  \
-  hipLaunchKernelGGL((attn_decode_partial_t<G, F>), grid, dim3(NTHREADS), lds, stream, \
-                     partials, q, (const char*)k_cache, (const char*)v_cache,          \
-                     k_scale, v_scale,                                                 \
-                     block_tables, context_lens, scale, num_kv_heads, block_size,      \
-                     max_blocks, max_chunks, q_tstride, chunk_keys)
+  const dim3 grid(num_kv_heads, B, splits);
+#define LAUNCH(G, F)                                                                            \
+  hipLaunchKernelGGL((attn_decode_tiles<G, F>), grid, dim3(NTHREADS), 0, stream, partials, out, q, \
+                     (const char*)k_cache, (const char*)v_cache, k_scale, v_scale, block_tables,   \
+                     context_lens, scale, block_size, max_blocks, q_tstride)
 #define DISPATCH(G) do { if (cache_fp8) LAUNCH(G, true); else LAUNCH(G, false); } while (0)
   switch (gqa) {
     case 1: DISPATCH(1); break;
     case 2: DISPATCH(2); break;
     case 4: DISPATCH(4); break;
-    case 8: DISPATCH(8); break;
-    default: DISPATCH(8); break;  // guarded by the binding's gqa<=8 check
+    default: DISPATCH(8); break;
   }
 #undef DISPATCH
 #undef LAUNCH
-}
-
-// merge the per-chunk partials: one 64-lane wave per (b, q_head)
-extern "C" __global__ void __launch_bounds__(64) attn_decode_reduce_kernel(
-    bf16_t* __restrict__ out,            // [B, H, 128]
-    const float* __restrict__ partials,  // [B, KVH, max_chunks, gqa, 130]
-    const int* __restrict__ context_lens,
-    int num_q_heads, int num_kv_heads, int max_chunks, int chunk_keys) {
-  const int b = blockIdx.x;
-  const int h = blockIdx.y;
-  const int gqa = num_q_heads / num_kv_heads;
-  const int g_kv = h / gqa;
-  const int g = h % gqa;
-  const int lane = threadIdx.x;
-  const int nchunks = min(max_chunks, (context_lens[b] + chunk_keys - 1) / chunk_keys);
-
-  const float* base = partials +
-      ((((int64_t)b * num_kv_heads + g_kv) * max_chunks) * gqa + g) * PART_STRIDE;
-
-  // global max over chunks
-  float m = -INFINITY;
-  for (int c = 0; c < nchunks; ++c) m = fmaxf(m, base[(int64_t)c * gqa * PART_STRIDE + 128]);
-  float l_tot = 0.0f;
-  float acc0 = 0.0f, acc1 = 0.0f;   // two dims per lane (d = lane*2)
-  for (int c = 0; c < nchunks; ++c) {
-    const float* pc = base + (int64_t)c * gqa * PART_STRIDE;
-    const float w = __expf(pc[128] - m);
-    l_tot += pc[129] * w;
-    acc0 += pc[lane * 2] * w;
-    acc1 += pc[lane * 2 + 1] * w;
-  }
-  const float inv_l = (l_tot > 0.f) ? 1.0f / l_tot : 0.0f;
-  bf16_t* op = out + (((int64_t)b * num_q_heads) + h) * 128;
-  const uint32_t pair = ((uint32_t)(uint16_t)f32_to_bf16(acc1 * inv_l) << 16) |
-                        (uint16_t)f32_to_bf16(acc0 * inv_l);
-  *reinterpret_cast<uint32_t*>((short*)op + lane * 2) = pair;
+  if (splits > 1)
+    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(num_q_heads, B), dim3(256), 0, stream, out,
+                       partials, context_lens, gqa, splits);
 }

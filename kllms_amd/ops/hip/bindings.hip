@@ -13,8 +13,8 @@ extern "C" __global__ void silu_mul_kernel(bf16_t*, const bf16_t*, const bf16_t*
 extern "C" __global__ void rope_kernel(bf16_t*, bf16_t*, const int64_t*, const float*, int, int, int, int, int);
 extern "C" __global__ void store_kv_kernel(const bf16_t*, const bf16_t*, bf16_t*, bf16_t*, const int64_t*, int, int, int, int, int);
 extern "C" __global__ void store_kv_fp8_kernel(const bf16_t*, const bf16_t*, unsigned char*, unsigned char*, float*, float*, const int64_t*, int, int, int, int, int);
-extern "C" void launch_attn_decode_partial(float*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, float, int, int, int, int, int, int, int, int, int, hipStream_t);
-extern "C" __global__ void attn_decode_reduce_kernel(bf16_t*, const float*, const int*, int, int, int, int);
+extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx);
+extern "C" void launch_attn_decode(bf16_t*, float*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, float, int, int, int, int, int, int, int, int, hipStream_t);
 extern "C" __global__ void attn_prefill_kernel(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, float, int, int, int, int);  // grouped: [G], [G], [G*8]
 extern "C" int sample_slices(int B, int V);
 extern "C" void launch_sample(int64_t*, float*, void*, const float*, const float*, const float*, const int*, const int64_t*, const int64_t*, const uint32_t*, int, int, float*, hipStream_t);
@@ -123,13 +123,12 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
               "attn_decode: GQA group must be 1, 2, 4 or 8");
   const int gqa = H / KVH;
   const int max_blocks = block_tables.size(1);
-  // split-K granule: fixed 256 keys measured best across B=40..240 and
-  // ctx 576..2048 (adaptive coarser chunks trade combine traffic for lost
-  // block-level parallelism and net 0..-5%; chunk size stays a runtime arg)
-  const int max_ctx = max_blocks * BS;
-  const int CHUNK_KEYS = ATTN_DECODE_TKV;  // 256
-  const int max_chunks = std::max(1, (max_ctx + CHUNK_KEYS - 1) / CHUNK_KEYS);
-  auto partials = torch::empty({(int64_t)B * KVH * max_chunks * gqa * 130},
+  TORCH_CHECK((int64_t)k_cache.size(0) * KVH * BS < (1LL << 31), "attn_decode: cache rows exceed 32-bit indexing");
+  if (B == 0) return;
+  // 16-byte query loads
+  if (q.stride(0) % 8 != 0 || reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 != 0) q = q.contiguous();
+  const int splits = attn_decode_splits(B, KVH, max_blocks * BS);
+  auto partials = torch::empty({splits > 1 ? (int64_t)B * KVH * splits * gqa * 130 : 0},
                                torch::dtype(torch::kFloat).device(q.device()));
   const int cache_fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn ? 1 : 0;
   if (cache_fp8) {
@@ -137,16 +136,12 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
                     k_scale.scalar_type() == at::kFloat && v_scale.numel() == k_scale.numel(),
                 "fp8 attn_decode requires [NB, KVH, BS] fp32 k_scale/v_scale");
   }
-  launch_attn_decode_partial(
-      partials.data_ptr<float>(), cbf(q), k_cache.data_ptr(), v_cache.data_ptr(),
+  launch_attn_decode(
+      bf(out), partials.data_ptr<float>(), cbf(q), k_cache.data_ptr(), v_cache.data_ptr(),
       cache_fp8 ? k_scale.data_ptr<float>() : nullptr,
       cache_fp8 ? v_scale.data_ptr<float>() : nullptr,
       block_tables.data_ptr<int>(), context_lens.data_ptr<int>(),
-      (float)scale, H, KVH, BS, max_blocks, max_chunks, (int)q.stride(0), CHUNK_KEYS, B,
-      cache_fp8, cur_stream());
-  hipLaunchKernelGGL(attn_decode_reduce_kernel, dim3(B, H), dim3(64), 0, cur_stream(),
-                     bf(out), partials.data_ptr<float>(), context_lens.data_ptr<int>(),
-                     H, KVH, max_chunks, CHUNK_KEYS);
+      (float)scale, H, KVH, BS, max_blocks, splits, (int)q.stride(0), B, cache_fp8, cur_stream());
 }
 
 void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k, torch::Tensor v,

@@ -113,7 +113,3 @@ __device__ __forceinline__ float u64_to_uniform(uint64_t h) {
       printf("kernel launch failed: %s\n", hipGetErrorString(e_));             \
     }                                                                          \
   } while (0)
-
-// decode-attention split-K geometry (shared by attn_decode.hip and bindings)
-#define ATTN_DECODE_CHUNK 256   // keys per workgroup
-#define ATTN_DECODE_TKV 256     // keys per LDS tile (one tile per chunk)
