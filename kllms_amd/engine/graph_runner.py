@@ -20,6 +20,7 @@ from typing import Dict, List, Optional
 
 import torch
 
+from .. import ops
 from ..models.llama import ForwardBatch
 
 
@@ -130,19 +131,20 @@ class DecodeGraphRunner:
                 self._recover_generator_state()
                 return self.engine.model.forward_decode(ids, batch)
         buf = self.buffers[bs]
-        scratch_slot = self._scratch_block * self.engine.config.kv_block_size
-        buf["ids"][:B].copy_(ids)
-        buf["ids"][B:].fill_(0)
-        buf["positions"][:B].copy_(batch.positions)
-        buf["positions"][B:].fill_(0)
-        buf["slots"][:B].copy_(batch.slot_mapping)
-        buf["slots"][B:].fill_(scratch_slot)
-        nb = batch.block_tables.shape[1]
-        buf["block_tables"][:B, :nb].copy_(batch.block_tables)
-        buf["block_tables"][:B, nb:].fill_(self._scratch_block)
-        buf["block_tables"][B:].fill_(self._scratch_block)
-        buf["context_lens"][:B].copy_(batch.context_lens)
-        buf["context_lens"][B:].fill_(1)
+        if not ops.decode_inputs(buf, ids, batch, self._scratch_block, self.engine.config.kv_block_size):
+            scratch_slot = self._scratch_block * self.engine.config.kv_block_size
+            buf["ids"][:B].copy_(ids)
+            buf["ids"][B:].fill_(0)
+            buf["positions"][:B].copy_(batch.positions)
+            buf["positions"][B:].fill_(0)
+            buf["slots"][:B].copy_(batch.slot_mapping)
+            buf["slots"][B:].fill_(scratch_slot)
+            nb = batch.block_tables.shape[1]
+            buf["block_tables"][:B, :nb].copy_(batch.block_tables)
+            buf["block_tables"][:B, nb:].fill_(self._scratch_block)
+            buf["block_tables"][B:].fill_(self._scratch_block)
+            buf["context_lens"][:B].copy_(batch.context_lens)
+            buf["context_lens"][B:].fill_(1)
         if self.engine.stateful:
             buf["seg_start"][:B].copy_(batch.seg_start)
             buf["seg_start"][B:].fill_(0)

@@ -156,6 +156,68 @@ def attn_decode_paged(
                                        k_scale, v_scale)
 
 
+# --- products of a few rows (decode steps) ----------------------------------------
+# GPU-only: callers ask linear_rows_ok first and keep F.linear for everything else.
+
+LINEAR_ROWS_MAX = 128
+
+
+def linear_rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the few-row kernel takes x [M, K] @ w [N, K]^T: bf16 on the GPU, rows and sizes that its 16-byte loads
+    and 128-deep chunks divide."""
+    return (x.is_cuda and not _force_torch() and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
+            and 1 <= x.shape[0] <= LINEAR_ROWS_MAX and x.shape[1] % 128 == 0 and w.shape[0] % 16 == 0
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and x.requires_grad))
+
+
+def linear_part(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """fp32 sums [S, M, N] of x @ w^T over S shares of K; the consumer adds them up."""
+    return _hip_or_raise().linear_rows(x, w, _none(x), 0, 0)
+
+
+def linear_silu_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up of a fused [gate; up] matrix, bf16."""
+    return _hip_or_raise().linear_rows(x, w, _none(x), 3, 1)
+
+
+def linear_f32_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """fp32 x @ w^T without a rounding to bf16 (logits)."""
+    return _hip_or_raise().linear_rows(x, w, _none(x), 2, 1)
+
+
+def embed_norm_rows(ids, table, weight, eps):
+    """(rms(table[ids]) * weight, table[ids])."""
+    return _hip_or_raise().embed_norm_rows(ids, table, weight, eps)
+
+
+def add_norm_rows(part, residual, weight, eps):
+    """residual += the sums of ``part`` (in place); returns rms(residual) * weight."""
+    return _hip_or_raise().add_norm_rows(part, residual, weight, eps)
+
+
+def rope_store_rows(part, bias, num_heads, positions, cos_sin, k_cache, v_cache, slot_mapping, k_scale=None, v_scale=None):
+    """Rotates q and k of the fused qkv sums, stores k and v into the paged cache; returns q [M, H, 128]."""
+    f = torch.empty(0, dtype=torch.float32, device=part.device)
+    return _hip_or_raise().rope_store_rows(
+        part, bias if bias is not None else torch.empty(0, dtype=torch.bfloat16, device=part.device), num_heads,
+        positions, cos_sin, k_cache, v_cache, slot_mapping, k_scale if k_scale is not None else f,
+        v_scale if v_scale is not None else f)
+
+
+def decode_inputs(buf: dict, ids, batch, scratch_block: int, block_size: int) -> bool:
+    """Fills a captured decode step's fixed buffers in one launch; False where the caller's tensors are not plain
+    int64 / int32 rows on the GPU (nothing is written then)."""
+    src = (ids, batch.positions, batch.slot_mapping, batch.context_lens, batch.block_tables)
+    kinds = (torch.long, torch.long, torch.long, torch.int32, torch.int32)
+    if _force_torch() or not all(t.device == buf["ids"].device and t.is_cuda and t.is_contiguous() and t.dtype == d
+                                 for t, d in zip(src, kinds)):
+        return False
+    _hip_or_raise().decode_inputs(buf["ids"], buf["positions"], buf["slots"], buf["context_lens"], buf["block_tables"],
+                                  *src, scratch_block, block_size)
+    return True
+
+
 def sample(
     logits: torch.Tensor,
     temperatures: torch.Tensor,

@@ -250,6 +250,125 @@ void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor
                   pad_offsets.data_ptr<int>(), E, H, IN, cur_stream());
 }
 
+// --- products of a few rows (linear_rows.hip) ---------------------------------
+extern "C" void launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
+                                   int K, int x_stride, int form, int splits, hipStream_t stream);
+extern "C" int linear_rows_splits(int M, int N, int K);
+
+// form 0: fp32 sums [S, M, N]; 1: bf16 [M, N] (+ bias); 2: fp32 [M, N]; 3: silu(gate) * up of a fused
+// [gate; up] matrix, bf16 [M, N / 2]
+torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, torch::Tensor bias, int64_t form, int64_t splits) {
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 &&
+                  x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
+              "x must be a bf16 [M, K] row view, 16-byte aligned");
+  CHECK_BF16_CONTIG(w);
+  const int M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == K && M >= 1 && M <= 128 && K % 128 == 0 && N % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
+              "linear_rows: M in 1..128, K a multiple of 128, N of 16");
+  TORCH_CHECK(form >= 0 && form <= 3 && (form != 3 || N % 64 == 0));
+  TORCH_CHECK(bias.numel() == 0 || (form == 1 && bias.numel() == N && bias.is_contiguous() &&
+                                    bias.scalar_type() == at::kBFloat16), "bias: bf16 [N], bf16 form only");
+  int S = 1;
+  if (form == 0) S = splits > 0 ? (int)splits : linear_rows_splits(M, N, K);
+  auto out = form == 0 ? torch::empty({S, M, N}, x.options().dtype(torch::kFloat))
+           : form == 2 ? torch::empty({M, N}, x.options().dtype(torch::kFloat))
+                       : torch::empty({M, form == 3 ? N / 2 : N}, x.options());
+  launch_linear_rows(out.data_ptr(), cbf(x), cbf(w), bias.numel() ? cbf(bias) : nullptr, M, N, K,
+                     (int)x.stride(0), (int)form, S, cur_stream());
+  return out;
+}
+
+// --- row-wise steps of a decode step (decode_rows.hip) -------------------------
+extern "C" void launch_add_norm_rows(bf16_t* out, bf16_t* residual, const float* part, const int64_t* ids,
+                                     const bf16_t* table, const bf16_t* w, int S, int M, int n, int64_t vocab,
+                                     float eps, hipStream_t stream);
+extern "C" void launch_rope_store_rows(bf16_t* q_out, const float* part, const bf16_t* bias, const int64_t* positions,
+                                       const float* cos_sin, void* k_cache, void* v_cache, float* k_scale,
+                                       float* v_scale, const int64_t* slots, int S, int M, int H, int G,
+                                       int block_size, int fp8, hipStream_t stream);
+extern "C" void launch_decode_inputs(int64_t* ids, int64_t* positions, int64_t* slots, int* ctx, int* tables,
+                                     const int64_t* ids_in, const int64_t* positions_in, const int64_t* slots_in,
+                                     const int* ctx_in, const int* tables_in, int B, int bs, int nb, int mb,
+                                     int scratch_block, int block_size, hipStream_t stream);
+
+// residual += split sums [S, M, n]; returns rms(residual) * weight
+torch::Tensor add_norm_rows(torch::Tensor part, torch::Tensor residual, torch::Tensor weight, double eps) {
+  CHECK_BF16_CONTIG(residual); CHECK_BF16_CONTIG(weight);
+  TORCH_CHECK(part.is_cuda() && part.is_contiguous() && part.scalar_type() == at::kFloat && part.dim() == 3);
+  const int S = part.size(0), M = part.size(1), n = part.size(2);
+  TORCH_CHECK(residual.dim() == 2 && residual.size(0) == M && residual.size(1) == n && weight.numel() == n &&
+                  n % 4 == 0 && n <= 16384 && S >= 1 && M >= 1, "add_norm_rows: sizes");
+  auto out = torch::empty_like(residual);
+  launch_add_norm_rows(bf(out), bf(residual), part.data_ptr<float>(), nullptr, nullptr, cbf(weight), S, M, n, 0,
+                       (float)eps, cur_stream());
+  return out;
+}
+
+// (rms(table[ids]) * weight, table[ids])
+std::vector<torch::Tensor> embed_norm_rows(torch::Tensor ids, torch::Tensor table, torch::Tensor weight, double eps) {
+  CHECK_BF16_CONTIG(table); CHECK_BF16_CONTIG(weight);
+  TORCH_CHECK(ids.is_cuda() && ids.is_contiguous() && ids.scalar_type() == at::kLong && ids.dim() == 1);
+  const int M = ids.size(0), n = table.size(1);
+  TORCH_CHECK(weight.numel() == n && n % 4 == 0 && n <= 16384 && M >= 1, "embed_norm_rows: sizes");
+  auto residual = torch::empty({M, n}, table.options());
+  auto out = torch::empty_like(residual);
+  launch_add_norm_rows(bf(out), bf(residual), nullptr, ids.data_ptr<int64_t>(), cbf(table), cbf(weight), 0, M, n,
+                       table.size(0), (float)eps, cur_stream());
+  return {out, residual};
+}
+
+// rotates q and k of the fused projection's split sums, stores k and v; returns q [M, H, 128]
+torch::Tensor rope_store_rows(torch::Tensor part, torch::Tensor bias, int64_t H, torch::Tensor positions,
+                              torch::Tensor cos_sin, torch::Tensor k_cache, torch::Tensor v_cache,
+                              torch::Tensor slots, torch::Tensor k_scale, torch::Tensor v_scale) {
+  CHECK_KV_CACHE(k_cache); CHECK_KV_CACHE(v_cache);
+  TORCH_CHECK(part.is_cuda() && part.is_contiguous() && part.scalar_type() == at::kFloat && part.dim() == 3);
+  const int S = part.size(0), M = part.size(1), G = k_cache.size(1), BS = k_cache.size(2);
+  TORCH_CHECK(k_cache.size(3) == 128 && v_cache.sizes() == k_cache.sizes() &&
+                  v_cache.scalar_type() == k_cache.scalar_type() && part.size(2) == (H + 2 * G) * 128 && S >= 1 &&
+                  M >= 1, "rope_store_rows: sizes");
+  TORCH_CHECK(positions.scalar_type() == at::kLong && positions.is_contiguous() && positions.numel() == M &&
+                  slots.scalar_type() == at::kLong && slots.is_contiguous() && slots.numel() == M &&
+                  cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() && cos_sin.size(-1) == 128,
+              "rope_store_rows: positions, slots or angles");
+  TORCH_CHECK(bias.numel() == 0 || (bias.scalar_type() == at::kBFloat16 && bias.is_contiguous() &&
+                                    bias.numel() == part.size(2)), "rope_store_rows: bias");
+  const int fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn ? 1 : 0;
+  if (fp8)
+    TORCH_CHECK(k_scale.numel() == k_cache.size(0) * G * BS && k_scale.is_contiguous() &&
+                    k_scale.scalar_type() == at::kFloat && v_scale.numel() == k_scale.numel() &&
+                    v_scale.is_contiguous() && v_scale.scalar_type() == at::kFloat,
+                "fp8 rope_store_rows requires [NB, KVH, BS] fp32 k_scale/v_scale");
+  auto q = torch::empty({M, H, 128}, part.options().dtype(torch::kBFloat16));
+  launch_rope_store_rows(bf(q), part.data_ptr<float>(), bias.numel() ? cbf(bias) : nullptr,
+                         positions.data_ptr<int64_t>(), cos_sin.data_ptr<float>(), k_cache.data_ptr(),
+                         v_cache.data_ptr(), fp8 ? k_scale.data_ptr<float>() : nullptr,
+                         fp8 ? v_scale.data_ptr<float>() : nullptr, slots.data_ptr<int64_t>(), S, M, (int)H, G, BS,
+                         fp8, cur_stream());
+  return q;
+}
+
+// fills the fixed buffers of a captured step of bs rows from B <= bs rows
+void decode_inputs(torch::Tensor ids, torch::Tensor positions, torch::Tensor slots, torch::Tensor ctx,
+                   torch::Tensor tables, torch::Tensor ids_in, torch::Tensor positions_in, torch::Tensor slots_in,
+                   torch::Tensor ctx_in, torch::Tensor tables_in, int64_t scratch_block, int64_t block_size) {
+  const int64_t bs = ids.numel(), B = ids_in.numel();
+  for (const auto& t : {ids, positions, slots, ids_in, positions_in, slots_in})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.scalar_type() == at::kLong, "decode_inputs: int64 rows");
+  for (const auto& t : {ctx, ctx_in, tables, tables_in})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.scalar_type() == at::kInt, "decode_inputs: int32 rows");
+  TORCH_CHECK(B <= bs && bs >= 1 && positions.numel() == bs && slots.numel() == bs && ctx.numel() == bs &&
+                  positions_in.numel() == B && slots_in.numel() == B && ctx_in.numel() == B && tables.dim() == 2 &&
+                  tables.size(0) == bs && tables_in.dim() == 2 && tables_in.size(0) == B &&
+                  tables_in.size(1) <= tables.size(1), "decode_inputs: sizes");
+  launch_decode_inputs(ids.data_ptr<int64_t>(), positions.data_ptr<int64_t>(), slots.data_ptr<int64_t>(),
+                       ctx.data_ptr<int>(), tables.data_ptr<int>(), ids_in.data_ptr<int64_t>(),
+                       positions_in.data_ptr<int64_t>(), slots_in.data_ptr<int64_t>(), ctx_in.data_ptr<int>(),
+                       tables_in.data_ptr<int>(), (int)B, (int)bs, (int)tables_in.size(1), (int)tables.size(1),
+                       (int)scratch_block, (int)block_size, cur_stream());
+}
+
 // --- batched Levenshtein (levenshtein.hip) -----------------------------------
 extern "C" void launch_levenshtein(int* out, const unsigned char* chars, const int* lens,
                                    const int* pi, const int* pj, long n_pairs,
@@ -305,6 +424,11 @@ void ipc_allreduce_destroy(int64_t ctx) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("levenshtein_pairs", &levenshtein_pairs);
+  m.def("linear_rows", &linear_rows);
+  m.def("add_norm_rows", &add_norm_rows);
+  m.def("embed_norm_rows", &embed_norm_rows);
+  m.def("rope_store_rows", &rope_store_rows);
+  m.def("decode_inputs", &decode_inputs);
   m.def("moe_gateup", &moe_gateup);
   m.def("moe_down", &moe_down);
   m.def("ipc_allreduce_create", &ipc_allreduce_create);

@@ -1,0 +1,195 @@
+// The row-wise steps between the products of a decode step, for gfx950: what a step
+// of up to 128 rows does there is launch latency (4.7 us a kernel in a replayed
+// graph) and little else, so each of these kernels does all the work that lies
+// between two products, and takes the previous product's fp32 split sums as they are
+// (linear_rows.hip), which saves the reduction's launch. The sums are rounded to bf16
+// where a whole product's result would be: a step of few rows and one of many then
+// agree to the last bits of their sums.
+//
+// Per layer: residual + norm (twice) and rope + cache store, beside attention and
+// four products: 8 launches, where separate reductions, rope, store and activation
+// took 11. A step of 5 rows (32 heads, width 4096, 6 layers, contexts of 560) went
+// from 948 to 774 us with these and linear_rows.hip, one of 120 rows from 1516 to 1237,
+// one of a single row at width 2048 from 492 to 391.
+
+#include "common.h"
+
+#define DR_THREADS 1024
+
+// sum of the splits of part [S, M, n4 * 4] at (m, vector i)
+__device__ __forceinline__ f32x4 split_sum(const float* __restrict__ part, int S, int64_t MN, int64_t at) {
+  f32x4 a = *reinterpret_cast<const f32x4*>(part + at);
+#pragma unroll 4
+  for (int s = 1; s < S; ++s) {
+    const f32x4 b = *reinterpret_cast<const f32x4*>(part + s * MN + at);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j] += b[j];
+  }
+  return a;
+}
+
+// residual[m] += sum of splits (written back, bf16), or residual[m] = table[ids[m]]
+// (EMBED); out[m] = rms(residual[m]) * w. One workgroup per row, the row in registers:
+// rows of up to 4 * DR_THREADS * DR_VECS elements.
+#define DR_VECS 4
+template <bool EMBED>
+__global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
+    bf16_t* __restrict__ out, bf16_t* __restrict__ residual, const float* __restrict__ part,
+    const int64_t* __restrict__ ids, const bf16_t* __restrict__ table, const bf16_t* __restrict__ w, int S, int M,
+    int n, int64_t vocab, float eps) {
+  __shared__ float red[16];
+  const int m = blockIdx.x, tid = threadIdx.x;
+  const int nvec = n / 4;
+  bf16x4_vec* rv = reinterpret_cast<bf16x4_vec*>(residual + (int64_t)m * n);
+  bf16x4_vec* ov = reinterpret_cast<bf16x4_vec*>(out + (int64_t)m * n);
+  const bf16x4_vec* wv = reinterpret_cast<const bf16x4_vec*>(w);
+  const int64_t id = EMBED ? ids[m] : 0;
+  const bool known = id >= 0 && id < vocab;   // an id without a row: NaN, never another's memory
+  f32x4 x[DR_VECS];
+  float ss = 0.0f;
+#pragma unroll
+  for (int k = 0; k < DR_VECS; ++k) {
+    const int i = tid + k * DR_THREADS;
+    if (i >= nvec) break;
+    bf16x4_vec r;
+    if constexpr (EMBED) {
+      r = known ? reinterpret_cast<const bf16x4_vec*>(table + id * n)[i] : bf16x4_vec{0x7fc0, 0x7fc0, 0x7fc0, 0x7fc0};
+    } else {
+      r = rv[i];
+      const f32x4 a = split_sum(part, S, (int64_t)M * n, (int64_t)m * n + i * 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[j] = f32_to_bf16(bf16_to_f32(r[j]) + bf16_to_f32(f32_to_bf16(a[j])));
+    }
+    rv[i] = r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      x[k][j] = bf16_to_f32(r[j]);
+      ss += x[k][j] * x[k][j];
+    }
+  }
+  ss = block_reduce_sum<16>(ss, red);
+  const float inv = rsqrtf(ss / n + eps);
+#pragma unroll
+  for (int k = 0; k < DR_VECS; ++k) {
+    const int i = tid + k * DR_THREADS;
+    if (i >= nvec) break;
+    const bf16x4_vec g = wv[i];
+    bf16x4_vec o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = f32_to_bf16(x[k][j] * inv * bf16_to_f32(g[j]));
+    ov[i] = o;
+  }
+}
+
+extern "C" void launch_add_norm_rows(bf16_t* out, bf16_t* residual, const float* part, const int64_t* ids,
+                                     const bf16_t* table, const bf16_t* w, int S, int M, int n, int64_t vocab,
+                                     float eps, hipStream_t stream) {
+  if (ids)
+    hipLaunchKernelGGL(add_norm_rows_kernel<true>, dim3(M), dim3(DR_THREADS), 0, stream, out, residual, part, ids,
+                       table, w, S, M, n, vocab, eps);
+  else
+    hipLaunchKernelGGL(add_norm_rows_kernel<false>, dim3(M), dim3(DR_THREADS), 0, stream, out, residual, part, ids,
+                       table, w, S, M, n, vocab, eps);
+}
+
+// qkv sums [S, M, (H + 2G) * 128] (+ bias): q and k rotated (entry i with i + 64), q
+// out as bf16 rows, k and v into the paged cache - as bf16, or as e4m3 with a scale
+// per row (amax / 448 of the bf16 row). A wave per (row, head), two dims a lane.
+template <bool FP8>
+__global__ void __launch_bounds__(256) rope_store_rows_kernel(
+    bf16_t* __restrict__ q_out, const float* __restrict__ part, const bf16_t* __restrict__ bias,
+    const int64_t* __restrict__ positions, const float* __restrict__ cos_sin, void* __restrict__ k_cache,
+    void* __restrict__ v_cache, float* __restrict__ k_scale, float* __restrict__ v_scale,
+    const int64_t* __restrict__ slots, int S, int M, int H, int G, int block_size) {
+  const int m = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int head = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (head >= H + 2 * G) return;
+  const int N = (H + 2 * G) * 128;
+  const int64_t MN = (int64_t)M * N;
+  const float* p = part + (int64_t)m * N + head * 128 + lane;
+  float a = 0.0f, b = 0.0f;
+#pragma unroll 4
+  for (int s = 0; s < S; ++s) {
+    a += p[s * MN];
+    b += p[s * MN + 64];
+  }
+  if (bias) {
+    a += bf16_to_f32(((const short*)bias)[head * 128 + lane]);
+    b += bf16_to_f32(((const short*)bias)[head * 128 + lane + 64]);
+  }
+  a = bf16_to_f32(f32_to_bf16(a));
+  b = bf16_to_f32(f32_to_bf16(b));
+  if (head < H + G) {
+    const float* cs = cos_sin + positions[m] * 128;
+    const float c = cs[lane], sn = cs[64 + lane];
+    const float x = a, y = b;
+    a = x * c - y * sn;
+    b = y * c + x * sn;
+  }
+  const short lo = f32_to_bf16(a), hi = f32_to_bf16(b);
+  if (head < H) {
+    short* o = (short*)q_out + ((int64_t)m * H + head) * 128;
+    o[lane] = lo;
+    o[lane + 64] = hi;
+    return;
+  }
+  const bool is_k = head < H + G;
+  const int g = head - H - (is_k ? 0 : G);
+  const int64_t slot = slots[m];
+  const int64_t row = ((slot / block_size) * G + g) * block_size + slot % block_size;
+  if constexpr (FP8) {
+    const float x = bf16_to_f32(lo), y = bf16_to_f32(hi);
+    const float sc = fmaxf(wave_reduce_max(fmaxf(fabsf(x), fabsf(y))) * (1.0f / 448.0f), 1e-8f);
+    const float inv = 1.0f / sc;
+    unsigned char* o = (unsigned char*)(is_k ? k_cache : v_cache) + row * 128;
+    o[lane] = f32_to_fp8(x * inv);
+    o[lane + 64] = f32_to_fp8(y * inv);
+    if (lane == 0) (is_k ? k_scale : v_scale)[row] = sc;
+  } else {
+    short* o = (short*)(is_k ? k_cache : v_cache) + row * 128;
+    o[lane] = lo;
+    o[lane + 64] = hi;
+  }
+}
+
+extern "C" void launch_rope_store_rows(bf16_t* q_out, const float* part, const bf16_t* bias, const int64_t* positions,
+                                       const float* cos_sin, void* k_cache, void* v_cache, float* k_scale,
+                                       float* v_scale, const int64_t* slots, int S, int M, int H, int G,
+                                       int block_size, int fp8, hipStream_t stream) {
+  const dim3 grid((H + 2 * G + 3) / 4, M);
+  if (fp8)
+    hipLaunchKernelGGL(rope_store_rows_kernel<true>, grid, dim3(256), 0, stream, q_out, part, bias, positions,
+                       cos_sin, k_cache, v_cache, k_scale, v_scale, slots, S, M, H, G, block_size);
+  else
+    hipLaunchKernelGGL(rope_store_rows_kernel<false>, grid, dim3(256), 0, stream, q_out, part, bias, positions,
+                       cos_sin, k_cache, v_cache, k_scale, v_scale, slots, S, M, H, G, block_size);
+}
+
+// Inputs of a captured decode step, in one launch (twelve copies and fills otherwise):
+// rows [0, B) from the caller's tensors, [B, bs) padding on the scratch block, block
+// tables widened from nb to mb columns with it.
+__global__ void __launch_bounds__(256) decode_inputs_kernel(
+    int64_t* __restrict__ ids, int64_t* __restrict__ positions, int64_t* __restrict__ slots, int* __restrict__ ctx,
+    int* __restrict__ tables, const int64_t* __restrict__ ids_in, const int64_t* __restrict__ positions_in,
+    const int64_t* __restrict__ slots_in, const int* __restrict__ ctx_in, const int* __restrict__ tables_in,
+    int B, int nb, int mb, int scratch_block, int block_size) {
+  const int b = blockIdx.x;
+  const bool real = b < B;
+  for (int i = threadIdx.x; i < mb; i += 256)
+    tables[(int64_t)b * mb + i] = real && i < nb ? tables_in[(int64_t)b * nb + i] : scratch_block;
+  if (threadIdx.x == 0) {
+    ids[b] = real ? ids_in[b] : 0;
+    positions[b] = real ? positions_in[b] : 0;
+    slots[b] = real ? slots_in[b] : (int64_t)scratch_block * block_size;
+    ctx[b] = real ? ctx_in[b] : 1;
+  }
+}
+
+extern "C" void launch_decode_inputs(int64_t* ids, int64_t* positions, int64_t* slots, int* ctx, int* tables,
+                                     const int64_t* ids_in, const int64_t* positions_in, const int64_t* slots_in,
+                                     const int* ctx_in, const int* tables_in, int B, int bs, int nb, int mb,
+                                     int scratch_block, int block_size, hipStream_t stream) {
+  hipLaunchKernelGGL(decode_inputs_kernel, dim3(bs), dim3(256), 0, stream, ids, positions, slots, ctx, tables, ids_in,
+                     positions_in, slots_in, ctx_in, tables_in, B, nb, mb, scratch_block, block_size);
+}

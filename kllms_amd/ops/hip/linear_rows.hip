@@ -1,0 +1,190 @@
+// Products of a few rows with a weight matrix, y[M, N] = x[M, K] W[N, K]^T, M <= 128
+// (the projections of a decode step), for gfx950.
+//
+// The weights' stream is the bound: 64 weight rows per 256-thread workgroup, 16 per
+// wave, each read once and straight from memory to matrix fragments (16x16x32) - a
+// lane group takes 32 contiguous bytes of its row in two loads, so every 128-byte line
+// is used whole, and x is read in the same order of k. x goes through LDS in 128-deep
+// chunks, double-buffered, shared by the four waves; its 16-byte units are XORed with
+// the row, which keeps the 16-row fragment reads free of bank conflicts. The weights of
+// the next two chunks are in flight while one is multiplied (8 KB a wave).
+//
+// A matrix of few rows is also split over k (linear_rows_splits); the splits' fp32 sums are left to the consumer, which reads them anyway (rope + store,
+// residual + norm). Forms of the result:
+//   PART  fp32 sums [S, M, N]          BF16  rounded once, bias added before it
+//   F32   fp32, S = 1 (logits)         SILU  silu(gate) * up of a fused [gate; up] matrix
+//
+// Measured with the weights out of cache (the library's kernel in brackets), us:
+//   4096 x 4096   5 rows 9 (15.6), 128 rows 16.3 (24.8)
+//   4096 x 14336  5 rows 23.4 (26.7: 5 TB/s either way), 64 rows 30 (42), 128 rows 39.5 (75.6)
+//   2048 x 8192   1 row 9.2 (12.8), 64 rows 11.9 (22.6)
+//   28672 x 4096  with silu 50 (64 + 5) for 5 rows, 60 (54 + 5) for 64, 74 (57 + 5) for 128
+// Above 64 rows every wave reads all of x from LDS for 16 weight rows, and LDS is the
+// bound where K is not split far.
+
+#include "common.h"
+
+typedef __bf16 bf16x8_mfma __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+#define LR_KC 128          // k depth of a chunk
+#define LR_STEPS 4         // matrix steps (32 k) of a chunk
+
+enum LinearForm { LR_PART = 0, LR_BF16 = 1, LR_F32 = 2, LR_SILU = 3 };
+
+union LrFrag {
+  u32x4 u;
+  bf16x8_mfma m;
+};
+
+template <int MT, int FORM>
+__global__ __launch_bounds__(256) void linear_rows_kernel(
+    void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+    const bf16_t* __restrict__ bias, int M, int N, int K, int x_stride, int chunks_per_split) {
+  __shared__ __attribute__((aligned(16))) u32x4 xs[2][MT * 256];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int nchunks = K / LR_KC;
+  const int c_begin = blockIdx.y * chunks_per_split;
+  const int c_end = min(nchunks, c_begin + chunks_per_split);
+  // weight row of this wave's tile; SILU: waves 0, 1 hold gate rows, 2, 3 the up rows of the same columns
+  const int n0 = FORM == LR_SILU ? (wave >> 1) * (N / 2) + blockIdx.x * 32 + (wave & 1) * 16
+                                 : blockIdx.x * 64 + wave * 16;
+  const char* wrow = (const char*)(w + (int64_t)min(n0 + col, N - 1) * K) + grp * 32;
+
+  f32x4 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  u32x4 wr[2][LR_STEPS];
+  u32x4 xr[MT];
+  auto load_w = [&](int c, int slot, int st) {
+    wr[slot][st] = *reinterpret_cast<const u32x4*>(wrow + (int64_t)c * (LR_KC * 2) + (st >> 1) * 128 + (st & 1) * 16);
+  };
+  // unit tid of each 16-row group: row tid / 16, 16-byte unit tid % 16
+  const int xrow = tid >> 4, xunit = tid & 15;
+  auto load_x = [&](int c) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+      xr[i] = *reinterpret_cast<const u32x4*>((const char*)(x + (int64_t)min(i * 16 + xrow, M - 1) * x_stride) +
+                                              (int64_t)c * (LR_KC * 2) + xunit * 16);
+  };
+  auto store_x = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) xs[buf][i * 256 + xrow * 16 + (xunit ^ xrow)] = xr[i];
+  };
+
+  if (c_begin < c_end) {
+    load_x(c_begin);
+#pragma unroll
+    for (int st = 0; st < LR_STEPS; ++st) load_w(c_begin, 0, st);
+    if (c_begin + 1 < c_end) {
+#pragma unroll
+      for (int st = 0; st < LR_STEPS; ++st) load_w(c_begin + 1, 1, st);
+    }
+    store_x(0);
+    __syncthreads();
+    for (int c = c_begin; c < c_end; c += 2) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (c + u < c_end) {
+          const bool next = c + u + 1 < c_end;
+          if (next) load_x(c + u + 1);
+#pragma unroll
+          for (int st = 0; st < LR_STEPS; ++st) {
+            LrFrag a;
+            a.u = wr[u][st];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+              LrFrag b;
+              b.u = xs[u][i * 256 + col * 16 + (((st >> 1) * 8 + grp * 2 + (st & 1)) ^ col)];
+              acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, b.m, acc[i], 0, 0, 0);
+            }
+          }
+          if (c + u + 2 < c_end) {
+#pragma unroll
+            for (int st = 0; st < LR_STEPS; ++st) load_w(c + u + 2, u, st);
+          }
+          if (next) store_x(1 - u);
+          __syncthreads();
+        }
+      }
+    }
+  }
+
+  // lane (col, grp): rows n0 + grp*4 .. +3 of the weights, row i*16 + col of x
+  const int n = n0 + grp * 4;
+  if constexpr (FORM == LR_SILU) {
+    float* up = reinterpret_cast<float*>(&xs[0][0]);   // [2 waves][MT*16 rows][16]
+    if (wave >= 2) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        *reinterpret_cast<f32x4*>(up + (((wave - 2) * MT + i) * 16 + col) * 16 + grp * 4) = acc[i];
+    }
+    __syncthreads();
+    if (wave < 2) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const int m = i * 16 + col;
+        const f32x4 u = *reinterpret_cast<const f32x4*>(up + ((wave * MT + i) * 16 + col) * 16 + grp * 4);
+        bf16x4_vec o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          // rounded as the separate product's result is
+          const float g = bf16_to_f32(f32_to_bf16(acc[i][r])), v = bf16_to_f32(f32_to_bf16(u[r]));
+          o[r] = f32_to_bf16(g / (1.0f + __expf(-g)) * v);
+        }
+        if (m < M) *reinterpret_cast<bf16x4_vec*>((short*)out + (int64_t)m * (N / 2) + n) = o;
+      }
+    }
+  } else {
+    if (n >= N) return;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = i * 16 + col;
+      if (m >= M) continue;
+      if constexpr (FORM == LR_PART) {
+        *reinterpret_cast<f32x4*>((float*)out + ((int64_t)blockIdx.y * M + m) * N + n) = acc[i];
+      } else if constexpr (FORM == LR_F32) {
+        *reinterpret_cast<f32x4*>((float*)out + (int64_t)m * N + n) = acc[i];
+      } else {
+        bf16x4_vec o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          o[r] = f32_to_bf16(acc[i][r] + (bias ? bf16_to_f32(((const short*)bias)[n + r]) : 0.0f));
+        *reinterpret_cast<bf16x4_vec*>((short*)out + (int64_t)m * N + n) = o;
+      }
+    }
+  }
+}
+
+extern "C" void launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
+                                   int K, int x_stride, int form, int splits, hipStream_t stream) {
+  const int per = (K / LR_KC + splits - 1) / splits;
+  const dim3 grid(form == LR_SILU ? N / 64 : (N + 63) / 64, splits);
+#define LR_GO(MT, F) \
+  hipLaunchKernelGGL((linear_rows_kernel<MT, F>), grid, dim3(256), 0, stream, out, x, w, bias, M, N, K, x_stride, per)
+#define LR_FORM(MT)                       \
+  switch (form) {                         \
+    case LR_PART: LR_GO(MT, LR_PART); break; \
+    case LR_BF16: LR_GO(MT, LR_BF16); break; \
+    case LR_F32: LR_GO(MT, LR_F32); break;   \
+    default: LR_GO(MT, LR_SILU); break;      \
+  }
+  if (M <= 16) { LR_FORM(1); }
+  else if (M <= 32) { LR_FORM(2); }
+  else if (M <= 64) { LR_FORM(4); }
+  else { LR_FORM(8); }
+#undef LR_FORM
+#undef LR_GO
+}
+
+// splits of k for the PART form: about 800 workgroups, 512 where the rows' sums weigh
+// more (M > 32), none below two chunks
+extern "C" int linear_rows_splits(int M, int N, int K) {
+  const int tiles = (N + 63) / 64, chunks = K / LR_KC;
+  int s = ((M <= 32 ? 800 : 512) + tiles / 2) / tiles;
+  s = s < chunks / 2 ? s : chunks / 2;
+  return s < 1 ? 1 : s;
+}

@@ -29,6 +29,8 @@ SOURCES = [
         "mfma_selftest.hip",
         "allreduce.hip",
         "moe.hip",
+        "linear_rows.hip",
+        "decode_rows.hip",
         "levenshtein.hip",
     )
 ]

@@ -68,3 +68,124 @@ def test_paged_decode_tiles(gqa, KVH, BS, ctx, width, fp8):
     err = (out.double().cpu() - ref).abs()
     # one bf16 rounding of the result (2^-9), fp32 sums before it
     assert (err <= 2 ** -8 * ref.abs() + 2e-5).all(), err.max()
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 64, 65, 128])
+@pytest.mark.parametrize("N,K", [(16, 128), (48, 256), (64, 384), (192, 1280), (2048, 2048)])
+def test_linear_rows(M, N, K):
+    g = torch.Generator().manual_seed(M * 13 + N + K)
+    x = torch.randn(M, K + 8, generator=g).bfloat16().to(DEV)[:, :K]      # a row view
+    w = (torch.randn(N, K, generator=g) * 0.05).bfloat16().to(DEV)
+    assert ops.linear_rows_ok(x, w)
+    ref = x.double() @ w.double().t()
+    # fp32 sums of K products: K * 2^-24 of the terms' size
+    tol = K * 2 ** -24 * (x.double().abs() @ w.double().abs().t())
+    for s in (0, 1, 2, 5):
+        got = ops._hip_or_raise().linear_rows(x, w, ops._none(x), 0, min(s, K // 128)).double().sum(0)
+        assert ((got - ref).abs() <= tol).all()
+    assert ((ops.linear_f32_rows(x, w).double() - ref).abs() <= tol).all()
+    b = torch.randn(N, generator=g).bfloat16().to(DEV)
+    got = ops._hip_or_raise().linear_rows(x, w, b, 1, 1).double()
+    full = ref + b.double()
+    assert ((got - full).abs() <= tol + 2 ** -8 * full.abs()).all()
+    if N % 64 == 0:
+        gate, up = ref.chunk(2, -1)
+        full = torch.nn.functional.silu(gate) * up
+        got = ops.linear_silu_rows(x, w).double()
+        # the sums' and their bf16 rounding's error through silu(g) * u (slope below 1.1 in g), a fast exponential, the
+        # result's rounding
+        tg, tu = (tol + 2 ** -9 * ref.abs()).chunk(2, -1)
+        assert ((got - full).abs() <= 1.1 * tg * (up.abs() + tu) + tu * gate.abs() + 2 ** -8 * full.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("S,M,n", [(1, 1, 128), (3, 5, 4096), (8, 128, 512), (2, 2, 16384), (5, 7, 4100)])
+def test_add_and_embed_norm_rows(S, M, n):
+    g = torch.Generator().manual_seed(S + M + n)
+    part = torch.randn(S, M, n, generator=g).to(DEV)
+    res = torch.randn(M, n, generator=g).bfloat16().to(DEV)
+    w = torch.rand(n, generator=g).bfloat16().to(DEV)
+    want = (res.double() + part.double().sum(0))
+    out = ops.add_norm_rows(part, res, w, 1e-5)
+    # the sum's rounding to bf16, then the residual's
+    assert ((res.double() - want).abs() <= 2 ** -8 * (want.abs() + part.double().sum(0).abs()) + 1e-5).all()
+    r = res.double()
+    ref = r / torch.sqrt((r * r).mean(-1, keepdim=True) + 1e-5) * w.double()
+    assert ((out.double() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5).all()
+    table = torch.randn(11, n, generator=g).bfloat16().to(DEV)
+    ids = torch.randint(0, 11, (M,), generator=g).to(DEV)
+    out, row = ops.embed_norm_rows(ids, table, w, 1e-5)
+    assert torch.equal(row, table[ids])
+    r = row.double()
+    ref = r / torch.sqrt((r * r).mean(-1, keepdim=True) + 1e-5) * w.double()
+    assert ((out.double() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("S,M,H,G,BS,bias", [(1, 1, 4, 4, 16, False), (3, 5, 8, 2, 16, True), (8, 128, 32, 8, 8, False)])
+def test_rope_store_rows(S, M, H, G, BS, bias, fp8):
+    g = torch.Generator().manual_seed(S * M + H)
+    N = (H + 2 * G) * D
+    # sums that are bf16 values already, so that the separate kernels start from the same numbers
+    part = torch.zeros(S, M, N)
+    part[-1] = torch.randn(M, N, generator=g).bfloat16().float()
+    part = part.to(DEV)
+    b = torch.randn(N, generator=g).bfloat16().to(DEV) if bias else None
+    NB = (M + BS - 1) // BS + 1
+    slots = torch.randperm(NB * BS, generator=g)[:M].to(DEV)
+    pos = torch.randint(0, 500, (M,), generator=g).to(DEV)
+    ang = torch.arange(512).unsqueeze(1) * 10000.0 ** (-torch.arange(0, D, 2) / D)
+    cs = torch.cat([ang.cos(), ang.sin()], 1).to(DEV)
+    kind = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    new = lambda: (torch.zeros(NB, G, BS, D, device=DEV, dtype=kind), torch.zeros(NB, G, BS, D, device=DEV, dtype=kind),  # noqa: E731
+                   torch.ones(NB, G, BS, device=DEV) if fp8 else None, torch.ones(NB, G, BS, device=DEV) if fp8 else None)
+    kc, vc, ks, vs = new()
+    q = ops.rope_store_rows(part, b, H, pos, cs, kc, vc, slots, ks, vs)
+    full = (part[-1].double() + (b.double() if bias else 0)).bfloat16().double()
+    c, s = cs[pos].double()[:, None, :64], cs[pos].double()[:, None, 64:]
+    rows = full.view(M, H + 2 * G, D)
+    lo, hi = rows[..., :64], rows[..., 64:]
+    rot = torch.cat([lo * c - hi * s, hi * c + lo * s], -1)
+    want = torch.cat([rot[:, :H + G], rows[:, H + G:]], 1)
+    size = 2 ** -8 * torch.maximum(want.abs(), want.roll(64, -1).abs()) + 1e-6
+    assert ((q.double() - want[:, :H]).abs() <= size[:, :H]).all()
+    for cache, sc, part64, tol in ((kc, ks, want[:, H:H + G], size[:, H:H + G]), (vc, vs, want[:, H + G:], size[:, H + G:])):
+        got = cache[slots // BS, :, slots % BS].float().double()
+        if fp8:
+            sc = sc[slots // BS, :, slots % BS].double().unsqueeze(-1)
+            assert torch.allclose(sc.squeeze(-1), part64.abs().amax(-1) / 448, rtol=2 ** -7)
+            got, tol = got * sc, tol + part64.abs() * 2 ** -4 + sc * 2 ** -9    # e4m3: 3 bits, subnormals of 2^-9
+        assert ((got - part64).abs() <= tol).all()
+    assert int((kc.view(torch.uint8) != 0).any(-1).sum()) <= M * G      # nothing beside the slots
+
+
+@pytest.mark.parametrize("preset", ["mid-llama", "mid-qwen", "mid-mixtral"])
+@pytest.mark.parametrize("rows", [1, 16, 65, 128, 129])
+def test_decode_rows_match_general_path(preset, rows):
+    """A whole decode step through the few-row kernels against the same model's general kernels (the path of any other
+    row count), both within bf16 rounding of each other."""
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+    from kllms_amd.models.llama import ForwardBatch
+
+    eng = LLMEngine(EngineConfig(model=preset, max_kv_blocks=1024, use_hip_graphs=False, seed=3))
+    g = torch.Generator().manual_seed(rows)
+    ctx = torch.randint(1, 60, (rows,), generator=g)
+    seqs = [eng.kv.alloc_sequence(int(c)) for c in ctx]
+    bt = torch.zeros(rows, 4, dtype=torch.int32)
+    for i, s in enumerate(seqs):
+        bt[i, :len(s.blocks)] = torch.tensor(s.blocks, dtype=torch.int32)
+    eng.kv.k_all.normal_()
+    eng.kv.v_all.normal_()
+    slots = torch.tensor([s.blocks[(int(c) - 1) // 16] * 16 + (int(c) - 1) % 16 for s, c in zip(seqs, ctx)])
+    batch = ForwardBatch(mode="decode", positions=(ctx - 1).to(DEV), slot_mapping=slots.to(DEV),
+                         kv_caches=eng.kv.layer_caches(), block_tables=bt.to(DEV),
+                         context_lens=ctx.to(torch.int32).to(DEV))
+    ids = torch.randint(0, 2000, (rows,), generator=g).to(DEV)
+    with torch.inference_mode():
+        assert eng.model._takes_rows(ids, batch) == (rows <= 128)
+        got = eng.model.forward_decode(ids, batch)
+        eng.model._takes_rows = lambda *a: False
+        want = eng.model.forward_decode(ids, batch)
+    # bf16 activations through two layers; a routed row may change its experts
+    off = (got - want).norm(dim=-1) / want.norm(dim=-1)
+    assert float(off.median()) < 0.02 and (preset == "mid-mixtral" or float(off.max()) < 0.05)
