@@ -493,35 +493,43 @@ class LLMEngine:
         cached head included). Returns last-token logits per sequence
         [len(seqs), V]."""
         dev = self.device
+        bs = self.kv.block_size
         all_ids: List[int] = []
-        all_pos: List[int] = []
         all_slots: List[int] = []
-        ctx_lens: List[int] = []
-        bt_blocks: List[List[int]] = []
         last_rows: List[int] = []
         for seq, ids, start in zip(seqs, ids_list, starts):
-            slots_all = self.kv.prefill_slot_mapping(seq)
-            for p in range(start, len(ids)):
-                all_ids.append(ids[p])
-                all_pos.append(p)
-                all_slots.append(slots_all[p])
-                ctx_lens.append(p + 1)
-                bt_blocks.append(seq.blocks)
+            all_ids.extend(ids[start:])
+            all_slots.extend(seq.blocks[p // bs] * bs + p % bs for p in range(start, len(ids)))
             last_rows.append(len(all_ids) - 1)
-        max_nb = max(len(b) for b in bt_blocks)
-        bt = torch.zeros((len(bt_blocks), max_nb), dtype=torch.int32)
-        for r, blocks in enumerate(bt_blocks):
-            bt[r, : len(blocks)] = torch.tensor(blocks, dtype=torch.int32)
-        batch = ForwardBatch(
-            mode="decode",
-            positions=torch.tensor(all_pos, dtype=torch.long, device=dev),
-            slot_mapping=torch.tensor(all_slots, dtype=torch.long, device=dev),
-            kv_caches=self.kv.layer_caches(),
-            block_tables=bt.to(dev),
-            context_lens=torch.tensor(ctx_lens, dtype=torch.int32, device=dev),
-        )
+        batch = self._rows_batch([(seq, start, len(ids) - start) for seq, ids, start in zip(seqs, ids_list, starts)],
+                                 all_slots)
         hidden = self.model.forward_hidden(torch.tensor(all_ids, dtype=torch.long, device=dev), batch)
         return self.model.compute_logits(hidden[torch.tensor(last_rows, device=dev)])
+
+    def _rows_batch(self, segs: List[Tuple[SequenceKV, int, int]], slots: List[int]) -> ForwardBatch:
+        """Decode-mode ForwardBatch of an attention-only model: one row per new
+        token of segs (sequence, first position, row count), packed in that
+        order; slots: the flat cache slot of every row."""
+        dev = self.device
+        pos = [p for _, start, n in segs for p in range(start, start + n)]
+        width = max(len(seq.blocks) for seq, _, _ in segs)
+        bt = torch.zeros((len(segs), width), dtype=torch.int32)
+        for b, (seq, _, _) in enumerate(segs):
+            bt[b, : len(seq.blocks)] = torch.tensor(seq.blocks, dtype=torch.int32)
+        bt = bt.to(dev)
+        positions = torch.tensor(pos, dtype=torch.long, device=dev)
+        row_seg = torch.tensor([b for b, (_, _, n) in enumerate(segs) for _ in range(n)], dtype=torch.long, device=dev)
+        return ForwardBatch(
+            mode="decode",
+            positions=positions,
+            slot_mapping=torch.tensor(slots, dtype=torch.long, device=dev),
+            kv_caches=self.kv.layer_caches(),
+            block_tables=bt[row_seg],
+            context_lens=(positions + 1).to(torch.int32),
+            seg_start=torch.tensor([start for _, start, _ in segs], dtype=torch.int32, device=dev),
+            host_segs=[(start, n) for _, start, n in segs],
+            seg_tables=bt,
+        )
 
     def _alloc_with_prefix(self, ids: List[int], prefix_blocks: List[int]) -> SequenceKV:
         """Sequence backed by cached prefix blocks (increfed) + freshly
@@ -600,23 +608,9 @@ class LLMEngine:
             batch = self._segment_batch([(seq, start, end - start)], slots_all[start:end])
             hidden = self.model.forward_hidden(ids, batch)
             return self.model.compute_logits(hidden[-1:]) if want_logits else None
-        pos = torch.arange(start, end, dtype=torch.long, device=dev)
-        slots_all = self.kv.prefill_slot_mapping(seq)
-        slots = torch.tensor(slots_all[start:end], dtype=torch.long, device=dev)
-        nb = len(seq.blocks)
-        bt = (
-            torch.tensor(seq.blocks, dtype=torch.int32, device=dev)
-            .unsqueeze(0).expand(end - start, nb).contiguous()
-        )
-        ctx = torch.arange(start + 1, end + 1, dtype=torch.int32, device=dev)
-        batch = ForwardBatch(
-            mode="decode",
-            positions=pos,
-            slot_mapping=slots,
-            kv_caches=self.kv.layer_caches(),
-            block_tables=bt,
-            context_lens=ctx,
-        )
+        bs = self.kv.block_size
+        batch = self._rows_batch([(seq, start, end - start)],
+                                 [seq.blocks[p // bs] * bs + p % bs for p in range(start, end)])
         hidden = self.model.forward_hidden(ids, batch)
         if want_logits:
             return self.model.compute_logits(hidden[-1:])
@@ -692,22 +686,7 @@ class LLMEngine:
         else:
             # attention-only models: one decode-mode row per token, each row
             # attending to its own sequence's cache up to its position
-            width = max(len(seq.blocks) for seq, _, _ in segs)
-            rows_bt = torch.zeros((len(ids), width), dtype=torch.int32)
-            pos: List[int] = []
-            r = 0
-            for seq, start, n in segs:
-                rows_bt[r : r + n, : len(seq.blocks)] = torch.tensor(seq.blocks, dtype=torch.int32)
-                pos.extend(range(start, start + n))
-                r += n
-            batch = ForwardBatch(
-                mode="decode",
-                positions=torch.tensor(pos, dtype=torch.long, device=dev),
-                slot_mapping=torch.tensor(slots, dtype=torch.long, device=dev),
-                kv_caches=self.kv.layer_caches(),
-                block_tables=rows_bt.to(dev),
-                context_lens=torch.tensor([p + 1 for p in pos], dtype=torch.int32, device=dev),
-            )
+            batch = self._rows_batch(segs, slots)
         hidden = self.model.forward_hidden(input_ids, batch)
         if not want_rows:
             return None

@@ -17,7 +17,7 @@ Two forward modes driven by ForwardBatch:
 from __future__ import annotations
 
 import math
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import List, Literal, Optional, Tuple
 
 import torch
@@ -51,6 +51,10 @@ class ForwardBatch:
     # layer plan per-piece kernels without a device sync; plans are cached here
     host_segs: Optional[list] = None
     plans: Optional[dict] = None
+    # decode-mode batches built from segments of an attention-only model (with
+    # host_segs and seg_start): one block table per segment, so that the rows of
+    # a long segment can attend together
+    seg_tables: Optional[torch.Tensor] = None    # [B, max_blocks] int32
 
 
 class LlamaAttention(nn.Module):
@@ -91,13 +95,23 @@ class LlamaAttention(nn.Module):
         ops.store_kv(k, v, k_cache, v_cache, batch.slot_mapping, k_scale, v_scale)
 
         if batch.mode == "prefill":
-            out = ops.attn_prefill_varlen(q, k, v, batch.cu_seqlens, self.scale)
+            out = ops.attn_prefill_varlen(q, k, v, batch.cu_seqlens, self.scale, (batch.plans or {}).get("prefill"))
         else:
-            out = ops.attn_decode_paged(
-                q, k_cache, v_cache, batch.block_tables, batch.context_lens, self.scale,
-                k_scale, v_scale,
-            )
+            out = self.attend_cache(q, batch)
         return self.o_proj(out.reshape(T, -1))
+
+    def attend_cache(self, q: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
+        """Attention of decode-mode rows q [T, H, D] against the paged cache."""
+        k_cache, v_cache, k_scale, v_scale = batch.kv_caches[self.layer_idx]
+        paged = (batch.plans or {}).get("paged")
+        if paged is not None and k_scale is None:
+            plan, short = paged
+            return ops.attn_segments_paged(q, k_cache, v_cache, batch.block_tables, batch.context_lens, self.scale,
+                                           plan, short, batch.seg_tables, batch.seg_start)
+        return ops.attn_decode_paged(
+            q, k_cache, v_cache, batch.block_tables, batch.context_lens, self.scale,
+            k_scale, v_scale,
+        )
 
 
 class LlamaMLP(nn.Module):
@@ -277,8 +291,7 @@ class LlamaForCausalLM(nn.Module):
             k_cache, v_cache, k_scale, v_scale = batch.kv_caches[at.layer_idx]
             q = ops.rope_store_rows(ops.linear_part(x, at.qkv_proj.weight), at.qkv_proj.bias, at.num_heads,
                                     batch.positions, self.cos_sin, k_cache, v_cache, batch.slot_mapping, k_scale, v_scale)
-            att = ops.attn_decode_paged(q, k_cache, v_cache, batch.block_tables, batch.context_lens, at.scale,
-                                        k_scale, v_scale)
+            att = at.attend_cache(q, batch)
             x = ops.add_norm_rows(ops.linear_part(att.view(T, -1), at.o_proj.weight), residual, norm.weight, norm.eps)
             norm = layers[i + 1].input_layernorm if i + 1 < len(layers) else self.norm
             mlp = layer.mlp
@@ -293,7 +306,23 @@ class LlamaForCausalLM(nn.Module):
                 x, residual = ops.fused_add_rmsnorm(mlp(x), residual, norm.weight, norm.eps)
         return x
 
+    def _planned(self, input_ids: torch.Tensor, batch: ForwardBatch) -> ForwardBatch:
+        """The batch with this pass's attention plans, made once for all layers."""
+        if not input_ids.is_cuda or ops._force_torch():
+            return batch
+        if batch.mode == "prefill":
+            plan = ops.prefill_plan(batch.cu_seqlens.to(device=input_ids.device, dtype=torch.int32).contiguous(),
+                                    input_ids.shape[0])
+            return replace(batch, plans={**(batch.plans or {}), "prefill": plan})
+        if (batch.host_segs is not None and batch.seg_tables is not None and self.dtype == torch.bfloat16
+                and self.layers and self.layers[0].self_attn.head_dim == 128):
+            plan, short = ops.paged_prefill_plan(batch.host_segs, input_ids.device)
+            if plan is not None:
+                return replace(batch, plans={**(batch.plans or {}), "paged": (plan, short)})
+        return batch
+
     def forward_hidden(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
+        batch = self._planned(input_ids, batch)
         if self._takes_rows(input_ids, batch):
             return self._forward_rows(input_ids, batch)
         hidden = self.embed_tokens(input_ids)

@@ -102,36 +102,58 @@ def store_kv(
     torch_ref.store_kv(k, v, k_cache, v_cache, slot_mapping, k_scale, v_scale)
 
 
-def _prefill_tiles(cu_seqlens: torch.Tensor, device) -> tuple:
-    """Grouped q-tile metadata for the MFMA prefill kernel: 32-row q-tiles of
-    each sequence packed 8 per workgroup (the 8 waves share the K/V LDS
-    staging); idle wave slots padded with -1. One host round-trip per prefill
-    batch (once per generate() call)."""
-    NW = 8
-    cu = cu_seqlens.cpu().tolist()
-    grp_start, grp_len, grp_qpos0 = [], [], []
-    for i in range(len(cu) - 1):
-        s, e = cu[i], cu[i + 1]
-        L = e - s
-        tiles = list(range(0, L, 32))
-        for g0 in range(0, len(tiles), NW):
-            grp_start.append(s)
-            grp_len.append(L)
-            grp = tiles[g0 : g0 + NW]
-            grp_qpos0.extend(grp + [-1] * (NW - len(grp)))
-    t = lambda x: torch.tensor(x, dtype=torch.int32, device=device)
-    return t(grp_start), t(grp_qpos0), t(grp_len)
+def prefill_plan(cu_seqlens: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
+    """Row groups of packed sequences for attn_prefill_varlen, made on the GPU (None on the CPU): one launch serves
+    every layer of a forward pass."""
+    if cu_seqlens.is_cuda and not _force_torch():
+        return _hip_or_raise().attn_prefill_plan(cu_seqlens, rows)
+    return None
 
 
 def attn_prefill_varlen(
-    q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlens: torch.Tensor, scale: float
+    q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlens: torch.Tensor, scale: float,
+    plan: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     if q.is_cuda and not _force_torch():
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        gs, gq, gl = _prefill_tiles(cu_seqlens, q.device)
-        _hip_or_raise().attn_prefill(out, q, k, v, gs, gq, gl, scale)
+        if plan is None:
+            plan = prefill_plan(cu_seqlens.to(device=q.device, dtype=torch.int32).contiguous(), q.shape[0])
+        _hip_or_raise().attn_prefill(out, q, k, v, plan, scale)
         return out
     return torch_ref.attn_prefill_varlen(q, k, v, cu_seqlens, scale)
+
+
+# segments shorter than this attend row by row: a workgroup of the paged prefill kernel has eight 32-row tiles
+PAGED_PREFILL_ROWS = 32
+
+
+def paged_prefill_plan(segs, device) -> tuple:
+    """(groups [4, G] on the device, [(first row, rows)] left to row-by-row attention) for segments
+    [(start position, rows)] packed in that order; groups None when every segment is short."""
+    groups, short, row = [], [], 0
+    for i, (_, n) in enumerate(segs):
+        if n >= PAGED_PREFILL_ROWS:
+            groups.extend((row, n, r, i) for r in range(0, n, 256))
+        elif n and short and short[-1][0] + short[-1][1] == row:
+            short[-1] = (short[-1][0], short[-1][1] + n)
+        elif n:
+            short.append((row, n))
+        row += n
+    # the groups that see most first
+    groups.sort(key=lambda g: -(segs[g[3]][0] + g[2]))
+    plan = torch.tensor(groups, dtype=torch.int32).t().contiguous().to(device) if groups else None
+    return plan, short
+
+
+def attn_segments_paged(q, k_cache, v_cache, block_tables, context_lens, scale, plan, short, seg_tables, seg_start):
+    """Rows of long segments on the matrix cores against the paged bf16 cache, the others row by row (GPU only)."""
+    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    _hip_or_raise().attn_prefill_paged(out, q, k_cache, v_cache, plan, seg_tables, seg_start, scale)
+    f = torch.empty(0, dtype=torch.float32, device=q.device)
+    for r, n in short:
+        _hip_or_raise().attn_decode_paged(out[r:r + n], q[r:r + n], k_cache, v_cache, block_tables[r:r + n],
+                                          context_lens[r:r + n], scale, f, f)
+    return out
 
 
 def attn_decode_paged(
@@ -395,7 +417,7 @@ def attn_varlen_mfma(out, q, k, v, grp_start, grp_qpos0, grp_len, scale) -> None
 
 def dense_tile_groups(pieces, device):
     """Host metadata for attn_varlen_mfma: pieces = [(first row, length)];
-    32-row q-tiles of each piece, 8 per workgroup (idle wave slots = -1)."""
+    32-row q-tiles of each piece, 8 in a row per workgroup (idle wave slots = -1)."""
     NW = 8
     gs, gl, gq = [], [], []
     for row0, L in pieces:

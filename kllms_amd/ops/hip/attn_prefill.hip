@@ -1,230 +1,256 @@
-// Varlen causal prefill attention for gfx950 — flash-style MFMA kernel.
+// Causal prefill attention for gfx950 - flash-style MFMA kernel over rows of packed
+// sequences, keys either from the same packed rows or from the paged cache.
 //
-// Structure:
-//   - an 8-WAVE workgroup serves 8 consecutive 32-row q-tiles of ONE
-//     (sequence, q-head): the K/V LDS staging is shared by the 8 waves, so
-//     its cost is amortized 8x over the 1-wave-per-block version;
-//   - KV tiles of 32 keys staged in LDS; K XOR-swizzled (G4: row-major tiles
-//     at D=128 are an up-to-16-way ds_read_b128 conflict; byte ^= (row&15)<<4
-//     makes the 16-lane group conflict-free); V staged TRANSPOSED
-//     ([128][32+pad]) so the PV A-fragment reads are contiguous 16B;
-//   - SWAPPED QK^T: S = mfma(A=K_tile, B=Q) so each lane's accumulators hold
-//     one q-row's scores -> softmax is in-register (fmax chain + one
-//     permlane32_swap half-merge), no cross-lane LDS traffic;
-//   - P repacked to bf16 MFMA B-fragments with pack + permlane32_swap half
-//     exchanges (T12/T21 pattern);
-//   - PV as O^T = mfma(A=V^T, B=P) over 4 d-tiles;
-//   - online softmax with per-lane running max/sum (rows are lane-local).
+//   - an 8-wave workgroup serves 8 consecutive 32-row q-tiles of ONE (sequence,
+//     q-head); 64 keys at a time are staged in LDS for all waves, double-buffered:
+//     the next 64 are on their way to registers while these are multiplied
+//   - SWAPPED QK^T: S = mfma(A=K_tile, B=Q), so a lane's accumulators hold one q-row's
+//     scores and the softmax is in registers (one permlane32_swap merges the halves)
+//   - P goes to bf16 MFMA B-fragments with pack + half swaps; O^T = mfma(A=V^T, B=P).
+//     V lies in LDS as it lies in memory; ds_read_b64_tr_b16 turns it on the way to
+//     the fragment (staging it transposed took 16 two-byte LDS writes a thread)
+//   - K's 16-byte units are XORed with the row, V's 32-byte slots too: both fragment
+//     reads are free of bank conflicts
+//
+// What bounds it: per 32 x 32 scores 16 matrix instructions (512 cycles of a SIMD)
+// stand beside about 500 vector cycles of softmax - half of them the exponentials at a
+// quarter of the rate - and two waves per SIMD overlap the two. So the softmax is kept
+// lean: base-2 exponentials of one fma each, the mask only where a tile crosses the
+// diagonal or the end, the packed conversion instruction, and a running max that is
+// renewed only when it grows by more than 8 (P stays below e^8, fine in fp32 and bf16).
+//
+// Grid: q-heads fastest, the heads of a kv head 8 apart, so that with 8 kv heads an
+// XCD's L2 serves one of them; groups of rows longest first, since causal groups
+// differ in length.
+//
+// Measured, 32 heads / 8 kv heads: one sequence of 7777 rows 612 us (810 TFLOP/s; 2019
+// with V staged transposed, synchronous staging and the mask in every tile), 24 of about
+// 512 rows 157 us (345); 8 segments of 150 rows behind 1536 cached keys 65 us (1017 as
+// single rows).
 //
 // MFMA fragment maps (v_mfma_f32_32x32x16_bf16, verified on-device by the
 // mfma_selftest binding):
 //   A[i][k]: lane l holds i = l&31, k = (l>>5)*8 + j   (j = 0..7)
 //   B[k][j]: lane l holds j = l&31, k = (l>>5)*8 + jj
 //   C/D[i][j]: lane l holds j = l&31, i = (r&3) + 8*(r>>2) + 4*(l>>5)  (r = 0..15)
-//
-// Host metadata (built in ops/__init__._prefill_tiles): q-tiles grouped 4 per
-// block PER SEQUENCE; grp_qpos0 = -1 pads idle waves.
+// ds_read_b64_tr_b16, per 16 lanes: lane 4r + c addresses row r, elements 4c..4c+3 of
+// 16; lane i receives element i of rows 0..3.
 
 #include "common.h"
 
 typedef __bf16 bf16x8_mfma __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 #define QBLK 32
-#define KVBLK 64                   // staged keys per barrier round (2 MFMA sub-tiles)
+#define KVBLK 64                   // staged keys per barrier round
 #define DHEAD 128
 #define NWAVES 8
-#define K_ROW_BYTES 256            // 128 bf16
-#define VT_ROW_SHORTS 72           // 64 keys + 8 pad (conflict-free b128 reads)
+#define TILE_BYTES (KVBLK * 256)   // K or V of a round
 
 __device__ __forceinline__ int acc_row(int r, int half) {
   return (r & 3) + 8 * (r >> 2) + 4 * half;   // C/D row map
 }
 
-extern "C" __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
+template <bool PAGED>
+__global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
     bf16_t* __restrict__ out,       // [T, H, D] contiguous
     const bf16_t* __restrict__ q,   // [T, H, D], token stride q_tstride
-    const bf16_t* __restrict__ k,   // [T, KVH, D], token stride kv_tstride
+    const bf16_t* __restrict__ k,   // [T, KVH, D], token stride kv_tstride; PAGED: cache [NB, KVH, BS, D]
     const bf16_t* __restrict__ v,
-    const int* __restrict__ grp_seq_start,   // [G] first token of the group's seq
-    const int* __restrict__ grp_seqlen,      // [G]
-    const int* __restrict__ grp_qpos0,       // [G*NWAVES], -1 = idle wave
-    float scale, int num_q_heads, int num_kv_heads, int q_tstride, int kv_tstride) {
-  const int grp = blockIdx.x;
-  const int h = blockIdx.y;
-  const int g_kv = h / (num_q_heads / num_kv_heads);
+    const int* __restrict__ grp_start,   // [G] first row of the group's sequence
+    const int* __restrict__ grp_len,     // [G] rows of the sequence, 0: idle group
+    const int* __restrict__ grp_q0,      // [G * q0_stride] group's first row within the sequence
+    const int* __restrict__ grp_seg,     // PAGED: [G] row of block_tables / seg_pos
+    const int* __restrict__ block_tables, const int* __restrict__ seg_pos,  // PAGED: position of a segment's row 0
+    float scale, int num_kv_heads, int q_tstride, int kv_tstride, int q0_stride, int block_size, int max_blocks) {
+  const int grp = blockIdx.y;
+  const int num_q_heads = gridDim.x;
+  const int g_kv = blockIdx.x % num_kv_heads;
+  const int h = g_kv * (num_q_heads / num_kv_heads) + blockIdx.x / num_kv_heads;
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int half = lane >> 5;
-  const int col = lane & 31;       // q-row (B/C col) or K/VT row (A row)
+  const int col = lane & 31;       // q-row (B/C col) or K row / V^T row (A row)
 
-  const int seq_start = grp_seq_start[grp];
-  const int seqlen = grp_seqlen[grp];
-  const int qpos0 = grp_qpos0[grp * NWAVES + wave];   // -1: idle wave
-  const bool active = qpos0 >= 0;
-  const int my_qpos = active ? qpos0 + col : 0;
+  const int seqlen = grp_len[grp];
+  const int q0 = grp_q0[grp * q0_stride];
+  if (seqlen <= 0 || q0 >= seqlen) return;
+  const int seq_start = grp_start[grp];
+  const int seg = PAGED ? grp_seg[grp] : 0;
+  const int pos0 = PAGED ? seg_pos[seg] : 0;          // keys before the sequence's first row
+  const int qrow0 = q0 + wave * QBLK;
+  const bool active = qrow0 < seqlen;
+  const int my_pos = pos0 + qrow0 + col;
+  // keys visible to the group's last row, and to this wave's
+  const int kv_end_grp = pos0 + min(seqlen, q0 + NWAVES * QBLK);
+  const int kv_end_me = active ? pos0 + min(seqlen, qrow0 + QBLK) : 0;
 
-  __shared__ __attribute__((aligned(16))) char smem[KVBLK * K_ROW_BYTES +
-                                                    DHEAD * VT_ROW_SHORTS * 2];
-  char* k_lds = smem;                                   // [64][256B], XOR-swizzled
-  short* vt_lds = reinterpret_cast<short*>(smem + KVBLK * K_ROW_BYTES);  // [128][72]
+  __shared__ __attribute__((aligned(16))) char smem[2][2 * TILE_BYTES];  // [buffer][K | V]
 
   // ---- Q fragments (B-operand): 8 d-slices of 16 --------------------------
-  bf16x8_mfma q_frag[8];
+  union QFrag { u32x4 u; bf16x8_mfma m; };
+  QFrag q_frag[8];
   {
-    const int qrow_c = active ? min(my_qpos, seqlen - 1) : 0;
-    const bf16_t* qp = q + (int64_t)(seq_start + qrow_c) * q_tstride + h * DHEAD;
+    const int row = min(qrow0 + col, seqlen - 1);
+    const short* qp = (const short*)q + (int64_t)(seq_start + row) * q_tstride + h * DHEAD + half * 8;
+    // a negative scale goes into Q's signs: the max below is taken before scaling
+    const uint32_t sign = scale < 0.0f ? 0x80008000u : 0u;
 #pragma unroll
-    for (int s = 0; s < 8; ++s)
-      q_frag[s] = *reinterpret_cast<const bf16x8_mfma*>((const short*)qp + s * 16 + half * 8);
+    for (int s = 0; s < 8; ++s) {
+      q_frag[s].u = *reinterpret_cast<const u32x4*>(qp + s * 16);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) q_frag[s].u[j] ^= sign;
+    }
   }
+  // scores to base-2 exponents; above zero, so that a masked score stays -inf
+  const float c2 = fmaxf(fabsf(scale) * 1.44269504088896340736f, 1e-30f);
+  const float THR2 = 8.0f * 1.44269504088896340736f;
+
+  // ---- staging: one key per 8 threads, 32 bytes of K and of V each ---------
+  const int st_key = tid >> 3, st_piece = tid & 7;
+  u32x4 rk[2], rv[2];
+  const int* bt = PAGED ? block_tables + (int64_t)seg * max_blocks : nullptr;
+  auto row_of = [&](int kt) -> int64_t {              // element offset of this thread's key
+    const int key = min(kt + st_key, kv_end_grp - 1);
+    if constexpr (PAGED)
+      return (((int64_t)bt[key / block_size] * num_kv_heads + g_kv) * block_size + key % block_size) * DHEAD;
+    else
+      return (int64_t)(seq_start + key) * kv_tstride + g_kv * DHEAD;
+  };
+  auto load_kv = [&](int64_t row) {
+    const u32x4* kp = reinterpret_cast<const u32x4*>((const short*)k + row) + st_piece * 2;
+    const u32x4* vp = reinterpret_cast<const u32x4*>((const short*)v + row) + st_piece * 2;
+    rk[0] = kp[0];
+    rk[1] = kp[1];
+    rv[0] = vp[0];
+    rv[1] = vp[1];
+  };
+  auto store_kv = [&](int buf) {
+    char* kb = smem[buf] + st_key * 256;
+    *reinterpret_cast<u32x4*>(kb + (((st_piece * 2) ^ (st_key & 15)) << 4)) = rk[0];
+    *reinterpret_cast<u32x4*>(kb + (((st_piece * 2 + 1) ^ (st_key & 15)) << 4)) = rk[1];
+    u32x4* vb = reinterpret_cast<u32x4*>(smem[buf] + TILE_BYTES + st_key * 256 + ((st_piece ^ (st_key & 7)) << 5));
+    vb[0] = rv[0];
+    vb[1] = rv[1];
+  };
 
   f32x16 o_acc[4] = {};
   float m_run = -INFINITY;
   float l_run = 0.0f;
 
-  // group-wide kv bound: the group's last active wave reaches furthest
-  int kv_end_grp = 0;
-#pragma unroll
-  for (int w = 0; w < NWAVES; ++w) {
-    const int qp0 = grp_qpos0[grp * NWAVES + w];
-    if (qp0 >= 0) kv_end_grp = max(kv_end_grp, min(seqlen, qp0 + QBLK));
-  }
-  const int kv_end_me = active ? min(seqlen, qpos0 + QBLK) : 0;
-
-  for (int kt00 = 0; kt00 < kv_end_grp; kt00 += KVBLK) {
-    const int nkeys_blk = min(KVBLK, kv_end_grp - kt00);
-
-    // ---- stage K (swizzled) + V^T, all 512 threads cooperatively ----------
-    {
-      const int key = tid >> 3;               // one key per 8 threads
-      const int piece = tid & 7;              // 16-dim sliver of that key
-      const bool valid = key < nkeys_blk;
-      const bf16_t* kp = k + (int64_t)(seq_start + kt00 + min(key, nkeys_blk - 1)) * kv_tstride + g_kv * DHEAD;
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const int byte_off = piece * 32 + c * 16;
-        bf16x8_vec val = valid
-            ? reinterpret_cast<const bf16x8_vec*>((const short*)kp)[byte_off / 16]
-            : bf16x8_vec{0, 0, 0, 0, 0, 0, 0, 0};
-        *reinterpret_cast<bf16x8_vec*>(
-            k_lds + key * K_ROW_BYTES + (byte_off ^ ((key & 15) << 4))) = val;
-      }
-      // V^T: this thread transposes its [16 dims x 1 key] sliver
-      const bf16_t* vp = v + (int64_t)(seq_start + kt00 + min(key, nkeys_blk - 1)) * kv_tstride + g_kv * DHEAD;
-      bf16x8_vec va = valid ? reinterpret_cast<const bf16x8_vec*>((const short*)vp)[piece * 2]
-                            : bf16x8_vec{0, 0, 0, 0, 0, 0, 0, 0};
-      bf16x8_vec vb = valid ? reinterpret_cast<const bf16x8_vec*>((const short*)vp)[piece * 2 + 1]
-                            : bf16x8_vec{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        vt_lds[(piece * 16 + j) * VT_ROW_SHORTS + key] = va[j];
-        vt_lds[(piece * 16 + 8 + j) * VT_ROW_SHORTS + key] = vb[j];
-      }
+  load_kv(row_of(0));
+  int64_t row_next = row_of(KVBLK);
+  store_kv(0);
+  __syncthreads();
+  int buf = 0;
+  for (int kt = 0; kt < kv_end_grp; kt += KVBLK, buf ^= 1) {
+    const bool more = kt + KVBLK < kv_end_grp;
+    if (more) {
+      load_kv(row_next);
+      row_next = row_of(kt + 2 * KVBLK);
     }
-    __syncthreads();
-
-#pragma unroll
-    for (int sub = 0; sub < 2; ++sub) {
-    const int kt0 = kt00 + sub * 32;
-    const int nkeys = min(32, nkeys_blk - sub * 32);
-    if (active && kt0 < kv_end_me && nkeys > 0) {
-      // ---- QK^T: S[key][qrow] over 8 d-slices -----------------------------
-      f32x16 s_acc = {};
+    if (kt < kv_end_me) {
+      const char* k_lds = smem[buf];
+      // ---- QK^T: S[key][qrow], two 32-key halves ----------------------------
+      f32x16 s_acc[2] = {};
 #pragma unroll
       for (int s = 0; s < 8; ++s) {
-        const int byte_off = (s * 2 + half) * 16;
-        const int krow = col + sub * 32;
-        bf16x8_mfma a_frag = *reinterpret_cast<const bf16x8_mfma*>(
-            k_lds + krow * K_ROW_BYTES + (byte_off ^ ((krow & 15) << 4)));
-        s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a_frag, q_frag[s], s_acc, 0, 0, 0);
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+          const int krow = col + sub * 32;
+          const bf16x8_mfma a = *reinterpret_cast<const bf16x8_mfma*>(
+              k_lds + krow * 256 + (((s * 2 + half) ^ (krow & 15)) << 4));
+          s_acc[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, q_frag[s].m, s_acc[sub], 0, 0, 0);
+        }
+      }
+      if (kt + KVBLK > pos0 + qrow0 || kt + KVBLK > kv_end_grp) {
+        // rows see keys up to their own position, which also ends the sequence
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = kt + sub * 32 + acc_row(r, half);
+            if (key > my_pos || key >= kv_end_grp) s_acc[sub][r] = -INFINITY;
+          }
       }
 
-      // ---- mask + scale ----------------------------------------------------
-      float sv[16];
+      // ---- online softmax (row = lane-local) --------------------------------
+      float tmax = s_acc[0][0];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = kt0 + acc_row(r, half);
-        const bool ok = (key <= my_qpos) && (acc_row(r, half) < nkeys) && (key < seqlen);
-        sv[r] = ok ? s_acc[r] * scale : -INFINITY;
-      }
-
-      // ---- online softmax (row = lane-local) -------------------------------
-      float tmax = sv[0];
+      for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
-      for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, sv[r]);
+        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s_acc[sub][r]);
       {
         auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
-        tmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+        tmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * c2;
       }
-      // defer-max (T13): rows are lane-local, so the defer decision is
-      // per-lane — keep the old running max while the tile max grew < THR
-      // (P then bounded by e^THR, fine for f32 p / bf16 pack). Decision
-      // happens BEFORE this tile's P is exponentiated (the safe order).
-      const float DEFER_THR = 8.0f;
-      float m_new, alpha;
-      if (tmax <= m_run + DEFER_THR) {       // first tile: m_run=-inf fails this
-        m_new = m_run;
-        alpha = 1.0f;
-      } else {
-        m_new = fmaxf(m_run, tmax);
-        alpha = (m_run == -INFINITY) ? 0.0f : __expf(m_run - m_new);
+      // the running max is renewed per row (lane) and only when it grows by more
+      // than THR2; the first tile always renews it, a tile without a visible key never
+      float alpha = 1.0f;
+      if (!(tmax <= m_run + THR2)) {
+        const float m_new = fmaxf(m_run, tmax);
+        alpha = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
       }
-      m_run = m_new;
       if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
           for (int r = 0; r < 16; ++r) o_acc[dt][r] *= alpha;
+        l_run *= alpha;
       }
-
-      float p[16];
-      float psum = 0.0f;
+      // masked scores: fma(-inf, c2, -m) = -inf, whose exponential is 0
+      const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+      uint32_t packs[2][8];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        p[r] = (sv[r] == -INFINITY) ? 0.0f : __expf(sv[r] - m_new);
-        psum += p[r];
-      }
-      l_run = l_run * alpha + psum;
-
-      // ---- repack P -> bf16 B-fragments (T12/T21 half swaps) ---------------
-      uint32_t packs[8];
+      for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
-      for (int pr = 0; pr < 8; ++pr) {
-        const short lo = f32_to_bf16(p[2 * pr]);
-        const short hi = f32_to_bf16(p[2 * pr + 1]);
-        packs[pr] = ((uint32_t)(uint16_t)hi << 16) | (uint16_t)lo;
-      }
-      uint32_t bfrag[2][4];
+        for (int pr = 0; pr < 8; ++pr) {
+          f32x2 p;
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        auto r0 = __builtin_amdgcn_permlane32_swap(packs[4 * kt + 0], packs[4 * kt + 2], false, false);
-        auto r1 = __builtin_amdgcn_permlane32_swap(packs[4 * kt + 1], packs[4 * kt + 3], false, false);
-        bfrag[kt][0] = r0[0];
-        bfrag[kt][1] = r1[0];
-        bfrag[kt][2] = r0[1];
-        bfrag[kt][3] = r1[1];
-      }
-
-      // ---- PV: O^T += V^T x P ----------------------------------------------
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        const int d_row = dt * 32 + col;
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-          bf16x8_mfma vfrag = *reinterpret_cast<const bf16x8_mfma*>(
-              vt_lds + d_row * VT_ROW_SHORTS + sub * 32 + kt * 16 + half * 8);
-          bf16x8_mfma pfrag;
-          {
-            uint32_t* pf = reinterpret_cast<uint32_t*>(&pfrag);
-#pragma unroll
-            for (int w = 0; w < 4; ++w) pf[w] = bfrag[kt][w];
+          for (int e = 0; e < 2; ++e) {
+            p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[sub][2 * pr + e], c2, -m_use));
+            l_run += p[e];
           }
-          o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfrag, pfrag, o_acc[dt], 0, 0, 0);
+          packs[sub][pr] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
         }
-      }
+
+      // ---- PV: O^T += V^T x P, 16 keys at a time ------------------------------
+      const char* v_lds = smem[buf] + TILE_BYTES;
+      // this lane's share of a transposed read: row (lane & 15) / 4, 4 elements
+      const int tr_row = half * 8 + ((lane & 15) >> 2);
+      const int tr_byte = (lane & 3) * 8;
+      const int tr_slot = (lane >> 4) & 1;
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int kw = 0; kw < 2; ++kw) {
+          union { uint32_t w[4]; bf16x8_mfma m; } pf;
+          auto r0 = __builtin_amdgcn_permlane32_swap(packs[sub][4 * kw + 0], packs[sub][4 * kw + 2], false, false);
+          auto r1 = __builtin_amdgcn_permlane32_swap(packs[sub][4 * kw + 1], packs[sub][4 * kw + 3], false, false);
+          pf.w[0] = r0[0];
+          pf.w[1] = r1[0];
+          pf.w[2] = r0[1];
+          pf.w[3] = r1[1];
+          const int key = sub * 32 + kw * 16 + tr_row;
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt) {
+            union { s16x4 t[2]; bf16x8_mfma m; } vf;
+#pragma unroll
+            for (int rd = 0; rd < 2; ++rd) {
+              const int kr = key + rd * 4;
+              const char* p = v_lds + kr * 256 + (((dt * 2 + tr_slot) ^ (kr & 7)) << 5) + tr_byte;
+              vf.t[rd] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+            }
+            o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.m, pf.m, o_acc[dt], 0, 0, 0);
+          }
+        }
     }
-    }  // sub
+    if (more) store_kv(buf ^ 1);
     __syncthreads();
   }
 
@@ -233,22 +259,81 @@ extern "C" __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
     l_run = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
-  if (active && my_qpos < seqlen) {
+  if (active && qrow0 + col < seqlen) {
     const float inv_l = (l_run > 0.0f) ? 1.0f / l_run : 0.0f;
-    bf16_t* op = out + (((int64_t)(seq_start + my_qpos)) * num_q_heads + h) * DHEAD;
+    bf16_t* op = out + (((int64_t)(seq_start + qrow0 + col)) * num_q_heads + h) * DHEAD;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
 #pragma unroll
       for (int g2 = 0; g2 < 4; ++g2) {   // regs 4*g2..+3 = d consecutive
         const int d0 = dt * 32 + 8 * g2 + 4 * half;
-        uint64_t word = 0;
+        bf16x4_vec o;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float val = o_acc[dt][4 * g2 + j] * inv_l;
-          word |= ((uint64_t)(uint16_t)f32_to_bf16(val)) << (16 * j);
-        }
-        *reinterpret_cast<uint64_t*>((short*)op + d0) = word;
+        for (int j = 0; j < 4; ++j) o[j] = f32_to_bf16(o_acc[dt][4 * g2 + j] * inv_l);
+        *reinterpret_cast<bf16x4_vec*>((short*)op + d0) = o;
       }
     }
   }
+}
+
+extern "C" void launch_attn_prefill(bf16_t* out, const bf16_t* q, const bf16_t* k, const bf16_t* v,
+                                    const int* grp_start, const int* grp_len, const int* grp_q0, int q0_stride,
+                                    int ngroups, float scale, int num_q_heads, int num_kv_heads, int q_tstride,
+                                    int kv_tstride, hipStream_t stream) {
+  hipLaunchKernelGGL(attn_prefill_kernel<false>, dim3(num_q_heads, ngroups), dim3(64 * NWAVES), 0, stream, out, q, k,
+                     v, grp_start, grp_len, grp_q0, nullptr, nullptr, nullptr, scale, num_kv_heads, q_tstride,
+                     kv_tstride, q0_stride, 1, 0);
+}
+
+extern "C" void launch_attn_prefill_paged(bf16_t* out, const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache,
+                                          const int* grp_start, const int* grp_len, const int* grp_q0,
+                                          const int* grp_seg, const int* block_tables, const int* seg_pos, int ngroups,
+                                          float scale, int num_q_heads, int num_kv_heads, int q_tstride,
+                                          int block_size, int max_blocks, hipStream_t stream) {
+  hipLaunchKernelGGL(attn_prefill_kernel<true>, dim3(num_q_heads, ngroups), dim3(64 * NWAVES), 0, stream, out, q,
+                     k_cache, v_cache, grp_start, grp_len, grp_q0, grp_seg, block_tables, seg_pos, scale,
+                     num_kv_heads, q_tstride, 0, 1, block_size, max_blocks);
+}
+
+// Groups of 256 rows of each sequence cu[i]..cu[i+1], into plan [3, G] (start, length,
+// first row), written back to front - a sequence's last rows see the most keys - and
+// idle in front. One workgroup, no host round trip.
+__global__ void __launch_bounds__(1024) attn_prefill_plan_kernel(int* __restrict__ plan, const int* __restrict__ cu,
+                                                                 int n, int G) {
+  __shared__ int sums[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int before = 0;                       // groups of the sequences handled so far
+  for (int s0 = 0; s0 < n; s0 += 1024) {
+    const int s = s0 + tid;
+    const int start = s < n ? cu[s] : 0;
+    const int len = s < n ? max(0, cu[s + 1] - start) : 0;
+    const int mine = (len + NWAVES * QBLK - 1) / (NWAVES * QBLK);
+    int incl = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(incl, off);
+      if (lane >= off) incl += o;
+    }
+    __syncthreads();
+    if (lane == 63) sums[wave] = incl;
+    __syncthreads();
+    int at = before + incl - mine, all = 0;
+    for (int w = 0; w < 16; ++w) {
+      if (w < wave) at += sums[w];
+      all += sums[w];
+    }
+    for (int j = 0; j < mine; ++j) {
+      const int g = G - 1 - (at + j);
+      if (g < 0) break;                 // more groups than rows allow: cu is not what the caller said
+      plan[g] = start;
+      plan[G + g] = len;
+      plan[2 * G + g] = j * NWAVES * QBLK;
+    }
+    before += all;
+  }
+  for (int g = tid; g < G - before; g += 1024) plan[G + g] = 0;
+}
+
+extern "C" void launch_attn_prefill_plan(int* plan, const int* cu, int n, int G, hipStream_t stream) {
+  hipLaunchKernelGGL(attn_prefill_plan_kernel, dim3(1), dim3(1024), 0, stream, plan, cu, n, G);
 }

@@ -15,7 +15,9 @@ extern "C" __global__ void store_kv_kernel(const bf16_t*, const bf16_t*, bf16_t*
 extern "C" __global__ void store_kv_fp8_kernel(const bf16_t*, const bf16_t*, unsigned char*, unsigned char*, float*, float*, const int64_t*, int, int, int, int, int);
 extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx);
 extern "C" void launch_attn_decode(bf16_t*, float*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, float, int, int, int, int, int, int, int, int, hipStream_t);
-extern "C" __global__ void attn_prefill_kernel(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, float, int, int, int, int);  // grouped: [G], [G], [G*8]
+extern "C" void launch_attn_prefill(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, int, int, float, int, int, int, int, hipStream_t);
+extern "C" void launch_attn_prefill_paged(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, const int*, const int*, const int*, int, float, int, int, int, int, int, hipStream_t);
+extern "C" void launch_attn_prefill_plan(int*, const int*, int, int, hipStream_t);
 extern "C" int sample_slices(int B, int V);
 extern "C" void launch_sample(int64_t*, float*, void*, const float*, const float*, const float*, const int*, const int64_t*, const int64_t*, const uint32_t*, int, int, float*, hipStream_t);
 extern "C" __global__ void mfma_selftest_kernel(float*, const bf16_t*, const bf16_t*);
@@ -144,20 +146,58 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
       (float)scale, H, KVH, BS, max_blocks, splits, (int)q.stride(0), B, cache_fp8, cur_stream());
 }
 
+static bool rows_aligned(const torch::Tensor& t) {  // 16-byte row loads
+  return t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
+// groups of 256 rows of the packed sequences cu [n + 1] over T rows: [3, G] (start, length, first row)
+torch::Tensor attn_prefill_plan(torch::Tensor cu, int64_t T) {
+  TORCH_CHECK(cu.is_cuda() && cu.is_contiguous() && cu.scalar_type() == at::kInt && cu.numel() >= 1);
+  const int n = cu.numel() - 1;
+  const int G = (int)(T / 256) + n;
+  auto plan = torch::empty({3, G}, cu.options());
+  if (G > 0) launch_attn_prefill_plan(plan.data_ptr<int>(), cu.data_ptr<int>(), n, G, cur_stream());
+  return plan;
+}
+
 void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k, torch::Tensor v,
-                  torch::Tensor grp_seq_start, torch::Tensor grp_qpos0,
-                  torch::Tensor grp_seqlen, double scale) {
+                  torch::Tensor plan, double scale) {
   CHECK_BF16_CONTIG(out); CHECK_BF16_ROWS(q); CHECK_BF16_ROWS(k); CHECK_BF16_ROWS(v);
   const int H = q.size(1), D = q.size(2), KVH = k.size(1);
   TORCH_CHECK(D == 128, "attn_prefill: head_dim must be 128");
+  TORCH_CHECK(H % KVH == 0, "attn_prefill: H must be a multiple of KVH");
   TORCH_CHECK(k.stride(0) == v.stride(0), "k/v must share the token stride");
-  const int ngroups = grp_seq_start.size(0);
-  TORCH_CHECK(grp_qpos0.size(0) == ngroups * 8, "grp_qpos0 must be [G*8]");
-  hipLaunchKernelGGL(attn_prefill_kernel, dim3(ngroups, H), dim3(512), 0, cur_stream(),
-                     bf(out), cbf(q), cbf(k), cbf(v),
-                     grp_seq_start.data_ptr<int>(), grp_seqlen.data_ptr<int>(),
-                     grp_qpos0.data_ptr<int>(), (float)scale, H, KVH,
-                     (int)q.stride(0), (int)k.stride(0));
+  TORCH_CHECK(plan.is_cuda() && plan.is_contiguous() && plan.scalar_type() == at::kInt && plan.dim() == 2 &&
+                  plan.size(0) == 3, "plan must come from attn_prefill_plan");
+  const int G = plan.size(1);
+  if (G == 0) return;
+  if (!rows_aligned(q)) q = q.contiguous();
+  if (!rows_aligned(k) || !rows_aligned(v)) { k = k.contiguous(); v = v.contiguous(); }
+  const int* p = plan.data_ptr<int>();
+  launch_attn_prefill(bf(out), cbf(q), cbf(k), cbf(v), p, p + G, p + 2 * G, 1, G, (float)scale, H, KVH,
+                      (int)q.stride(0), (int)k.stride(0), cur_stream());
+}
+
+// rows of segments against the paged cache (bf16): plan [4, G] int32 (first row, rows, first row within the
+// segment, segment), tables [n, MAXB], pos [n] = position of each segment's first row. The segments' own keys and
+// values are in the cache already.
+void attn_prefill_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache, torch::Tensor v_cache,
+                        torch::Tensor plan, torch::Tensor tables, torch::Tensor pos, double scale) {
+  CHECK_BF16_CONTIG(out); CHECK_BF16_ROWS(q); CHECK_BF16_CONTIG(k_cache); CHECK_BF16_CONTIG(v_cache);
+  const int H = q.size(1), KVH = k_cache.size(1), BS = k_cache.size(2);
+  TORCH_CHECK(q.size(2) == 128 && k_cache.size(3) == 128 && v_cache.sizes() == k_cache.sizes() && H % KVH == 0,
+              "attn_prefill_paged: head size 128, whole groups");
+  TORCH_CHECK(plan.is_cuda() && plan.is_contiguous() && plan.scalar_type() == at::kInt && plan.dim() == 2 &&
+                  plan.size(0) == 4 && tables.is_cuda() && tables.is_contiguous() && tables.scalar_type() == at::kInt &&
+                  tables.dim() == 2 && pos.is_cuda() && pos.is_contiguous() && pos.scalar_type() == at::kInt &&
+                  pos.numel() == tables.size(0), "attn_prefill_paged: plan, tables or positions");
+  const int G = plan.size(1);
+  if (G == 0) return;
+  if (!rows_aligned(q)) q = q.contiguous();
+  const int* p = plan.data_ptr<int>();
+  launch_attn_prefill_paged(bf(out), cbf(q), cbf(k_cache), cbf(v_cache), p, p + G, p + 2 * G, p + 3 * G,
+                            tables.data_ptr<int>(), pos.data_ptr<int>(), G, (float)scale, H, KVH, (int)q.stride(0),
+                            BS, (int)tables.size(1), cur_stream());
 }
 
 void sample(torch::Tensor tokens, torch::Tensor logprobs, torch::Tensor logits,
@@ -442,6 +482,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("store_kv", &store_kv);
   m.def("attn_decode_paged", &attn_decode_paged);
   m.def("attn_prefill", &attn_prefill);
+  m.def("attn_prefill_plan", &attn_prefill_plan);
+  m.def("attn_prefill_paged", &attn_prefill_paged);
   m.def("sample", &sample);
   m.def("mfma_selftest", &mfma_selftest);
   m.def("one_shot_allreduce", &one_shot_allreduce);

@@ -1,0 +1,115 @@
+"""Causal prefill attention, packed and against the paged cache, against float64 at the edges of its tiles."""
+
+import pytest
+import torch
+
+from kllms_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+D = 128
+
+
+def causal64(q, k, v, scale, first):
+    """Rows first.. of one sequence; also the bound sum p |v| of what rounding P to bf16 can move."""
+    T, H, _ = q.shape
+    rep = H // k.shape[1]
+    k, v, q = (t.double().to(DEV) for t in (k, v, q))
+    hide = torch.arange(k.shape[0], device=DEV) > torch.arange(first, first + T, device=DEV).unsqueeze(1)
+    out, size = [], []
+    for h in range(H):
+        p = torch.softmax((q[:, h] @ k[:, h // rep].t() * scale).masked_fill(hide, -torch.inf), -1)
+        out.append(p @ v[:, h // rep])
+        size.append(p @ v[:, h // rep].abs())
+    return torch.stack(out, 1), torch.stack(size, 1)
+
+
+def check(got, ref, size):
+    # P in bf16 (2^-9 of each term) with a fast exponential, the result rounded to bf16
+    err = (got.double() - ref).abs()
+    assert (err <= 2 ** -8 * size + 2 ** -8 * ref.abs() + 1e-6).all(), float((err - 2 ** -8 * size).max())
+
+
+@pytest.mark.parametrize("H,G", [(4, 4), (8, 2), (32, 8), (7, 1)])
+@pytest.mark.parametrize("lens", [[1], [31, 32, 33], [63, 64, 65, 0, 1], [255, 256, 257], [700, 5, 513]])
+@pytest.mark.parametrize("scale", [D ** -0.5, -0.3])
+def test_packed(H, G, lens, scale):
+    g = torch.Generator().manual_seed(sum(lens) + H)
+    T = sum(lens)
+    qkv = torch.randn(T, H + 2 * G, D, generator=g).bfloat16().to(DEV)      # the fused projection's layout
+    q, k, v = qkv.split([H, G, G], 1)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).to(DEV)
+    out = ops.attn_prefill_varlen(q, k, v, cu, scale)
+    plan = ops.prefill_plan(cu, T)
+    assert torch.equal(out, ops.attn_prefill_varlen(q, k, v, cu, scale, plan))
+    r = 0
+    for n in lens:
+        if n:
+            check(out[r:r + n], *causal64(q[r:r + n].cpu(), k[r:r + n].cpu(), v[r:r + n].cpu(), scale, 0))
+        r += n
+
+
+def test_plan_covers_many_sequences():
+    g = torch.Generator().manual_seed(1)
+    lens = torch.randint(0, 700, (1500,), generator=g)
+    cu = torch.cat([torch.zeros(1, dtype=torch.long), lens.cumsum(0)]).to(torch.int32).to(DEV)
+    start, length, first = ops.prefill_plan(cu, int(lens.sum())).cpu().long()
+    live = length > 0
+    got = sorted(zip(start[live].tolist(), length[live].tolist(), first[live].tolist()))
+    want = sorted((int(s), int(n), f) for s, n in zip(cu.cpu()[:-1], lens) for f in range(0, int(n), 256))
+    assert got == want
+
+
+@pytest.mark.parametrize("H,G,BS", [(8, 2, 16), (32, 8, 16), (4, 4, 5)])
+@pytest.mark.parametrize("segs", [[(0, 40)], [(17, 32), (1000, 300), (3, 1), (5, 2)], [(255, 1), (64, 257), (0, 31), (700, 33)]])
+def test_segments_against_cache(H, G, BS, segs):
+    g = torch.Generator().manual_seed(sum(n for _, n in segs) + H)
+    NB = sum((s + n + BS - 1) // BS for s, n in segs) + 2
+    perm = torch.randperm(NB, generator=g).tolist()
+    kc, vc = (torch.randn(NB, G, BS, D, generator=g).bfloat16() for _ in range(2))
+    width = max((s + n + BS - 1) // BS for s, n in segs)
+    bt = torch.zeros(len(segs), width, dtype=torch.int32)
+    for i, (s, n) in enumerate(segs):
+        m = (s + n + BS - 1) // BS
+        bt[i, :m] = torch.tensor([perm.pop() for _ in range(m)], dtype=torch.int32)
+    T = sum(n for _, n in segs)
+    q = torch.randn(T, H + 1, D, generator=g).bfloat16().to(DEV)[:, :H]
+    plan, short = ops.paged_prefill_plan(segs, DEV)
+    row_seg = torch.tensor([i for i, (_, n) in enumerate(segs) for _ in range(n)])
+    ctx = torch.tensor([s + j + 1 for s, n in segs for j in range(n)], dtype=torch.int32)
+    if plan is None:
+        return
+    out = ops.attn_segments_paged(q, kc.to(DEV), vc.to(DEV), bt[row_seg].to(DEV), ctx.to(DEV), D ** -0.5, plan, short,
+                                  bt.to(DEV), torch.tensor([s for s, _ in segs], dtype=torch.int32).to(DEV))
+    r = 0
+    for i, (s, n) in enumerate(segs):
+        at = torch.arange(s + n)
+        blk = bt[i].long()[at // BS]
+        check(out[r:r + n], *causal64(q[r:r + n].cpu(), kc[blk, :, at % BS], vc[blk, :, at % BS], D ** -0.5, s))
+        r += n
+
+
+@pytest.mark.parametrize("rows", [[40, 20], [150, 1, 33], [300]])
+def test_step_segments_matches_row_by_row(rows):
+    """Portions behind a cached head through LLMEngine.step_segments, every row's logits, against the same step with
+    each row attending alone."""
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+
+    eng = LLMEngine(EngineConfig(model="mid-llama", max_kv_blocks=512, use_hip_graphs=False, seed=3))
+    g = torch.Generator().manual_seed(sum(rows))
+
+    def step(alone):
+        eng.model._planned = (lambda ids, batch: batch) if alone else type(eng.model)._planned.__get__(eng.model)
+        seqs = [eng.open_sequence() for _ in rows]
+        heads = [torch.randint(0, 2000, (37 + 11 * i,), generator=torch.Generator().manual_seed(i)).tolist()
+                 for i in range(len(rows))]
+        eng.step_segments([(s, h, []) for s, h in zip(seqs, heads)])
+        out = eng.step_segments([(s, t, list(range(len(t)))) for s, t in zip(seqs, toks)])
+        for s in seqs:
+            eng.kv.free_sequence(s)
+        return out
+
+    toks = [torch.randint(0, 2000, (n,), generator=g).tolist() for n in rows]
+    a, b = step(False), step(True)
+    assert float(((a - b).norm(dim=-1) / b.norm(dim=-1)).max()) < 0.03     # bf16 through two layers
