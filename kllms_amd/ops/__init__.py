@@ -268,23 +268,34 @@ def moe_gateup(
     x: torch.Tensor,
     w_gate_up: torch.Tensor,
     sorted_ids: torch.Tensor,
-    pad_offsets: torch.Tensor,
+    offsets: torch.Tensor,
     zeros: torch.Tensor,
 ) -> None:
     """Grouped MoE gate/up GEMM + fused silu*mul into `act` (sorted-by-expert
-    row space). GPU-only (Mixtral prefill hot path); the CPU path keeps the
+    row space, expert e at offsets[e]..offsets[e+1]; a sorted id of -1 reads
+    `zeros`). GPU-only (Mixtral prefill hot path); the CPU path keeps the
     per-expert torch loop in models/mixtral.py."""
-    _hip_or_raise().moe_gateup(act, x, w_gate_up, sorted_ids, pad_offsets, zeros)
+    _hip_or_raise().moe_gateup(act, x, w_gate_up, sorted_ids, offsets, zeros)
 
 
 def moe_down(
     y: torch.Tensor,
     act: torch.Tensor,
     w_down: torch.Tensor,
-    pad_offsets: torch.Tensor,
+    offsets: torch.Tensor,
 ) -> None:
     """Grouped MoE down GEMM in sorted-row space (see moe_gateup)."""
-    _hip_or_raise().moe_down(y, act, w_down, pad_offsets)
+    _hip_or_raise().moe_down(y, act, w_down, offsets)
+
+
+def moe_sort(topi: torch.Tensor, experts: int):
+    """(token of each sorted place, place of each (token, choice), expert offsets), without a host round trip."""
+    return _hip_or_raise().moe_sort(topi.long().contiguous(), experts)
+
+
+def moe_combine_rows(y: torch.Tensor, weights: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
+    """sum over choices of weights[t, j] * y[pos[t, j]], fp32 sums, bf16 result."""
+    return _hip_or_raise().moe_combine(y, weights.float().contiguous(), pos)
 
 
 def levenshtein_pairs(

@@ -253,41 +253,69 @@ void one_shot_allreduce(std::vector<torch::Tensor> bufs) {
 }
 
 // --- grouped MoE expert GEMMs (moe.hip) --------------------------------------
-extern "C" void launch_moe_gateup(void* act, const void* x, const void* w,
-                                  const int* sorted_ids, const int* pad_offsets,
-                                  const void* zeros, int E, int IN, int K,
-                                  hipStream_t stream);
-extern "C" void launch_moe_down(void* y, const void* act, const void* w,
-                                const int* pad_offsets, int E, int H, int IN,
+extern "C" int launch_moe_gateup(void* act, const void* x, const void* w, const int* sorted_ids, const int* offsets,
+                                 const void* zeros, int S, int E, int IN, int K, hipStream_t stream);
+extern "C" int launch_moe_down(void* y, const void* act, const void* w, const int* offsets, int S, int E, int H,
+                               int IN, hipStream_t stream);
+extern "C" void launch_moe_sort(int* ids, int* pos, int* offsets, const int64_t* topi, int P, int k, int E,
                                 hipStream_t stream);
+extern "C" void launch_moe_combine(void* out, const void* y, const float* weights, const int* pos, int T, int k,
+                                   int H, hipStream_t stream);
 
 void moe_gateup(torch::Tensor act, torch::Tensor x, torch::Tensor w,
-                torch::Tensor sorted_ids, torch::Tensor pad_offsets, torch::Tensor zeros) {
+                torch::Tensor sorted_ids, torch::Tensor offsets, torch::Tensor zeros) {
   CHECK_BF16_CONTIG(act); CHECK_BF16_CONTIG(x); CHECK_BF16_CONTIG(w); CHECK_BF16_CONTIG(zeros);
-  TORCH_CHECK(sorted_ids.scalar_type() == at::kInt && pad_offsets.scalar_type() == at::kInt,
-              "routing tensors must be int32");
+  TORCH_CHECK(sorted_ids.scalar_type() == at::kInt && offsets.scalar_type() == at::kInt &&
+                  sorted_ids.is_contiguous() && offsets.is_contiguous(), "routing tensors must be int32");
   const int E = w.size(0);
   const int IN = w.size(1) / 2;
   const int K = w.size(2);
   TORCH_CHECK(IN % 64 == 0 && K % 64 == 0, "IN % 64, K % 64 required");
   TORCH_CHECK(act.size(1) == IN && x.size(1) == K && zeros.numel() >= K);
-  TORCH_CHECK(act.size(0) % 128 == 0, "sorted rows must be padded to 128");
-  TORCH_CHECK(pad_offsets.numel() == E + 1);
-  launch_moe_gateup(act.data_ptr(), x.data_ptr(), w.data_ptr(),
-                    sorted_ids.data_ptr<int>(), pad_offsets.data_ptr<int>(),
-                    zeros.data_ptr(), E, IN, K, cur_stream());
+  TORCH_CHECK(sorted_ids.numel() >= act.size(0), "one id per sorted row");
+  TORCH_CHECK(offsets.numel() == E + 1);
+  if (act.size(0) == 0) return;
+  TORCH_CHECK(launch_moe_gateup(act.data_ptr(), x.data_ptr(), w.data_ptr(), sorted_ids.data_ptr<int>(),
+                                offsets.data_ptr<int>(), zeros.data_ptr(), (int)act.size(0), E, IN, K,
+                                cur_stream()) == 0, "moe_gateup: 128 KB of LDS are not available");
 }
 
-void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor pad_offsets) {
+void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor offsets) {
   CHECK_BF16_CONTIG(y); CHECK_BF16_CONTIG(act); CHECK_BF16_CONTIG(w);
   const int E = w.size(0);
   const int H = w.size(1);
   const int IN = w.size(2);
   TORCH_CHECK(H % 64 == 0 && IN % 64 == 0, "H % 64, IN % 64 required");
-  TORCH_CHECK(y.size(1) == H && act.size(1) == IN);
-  TORCH_CHECK(pad_offsets.numel() == E + 1);
-  launch_moe_down(y.data_ptr(), act.data_ptr(), w.data_ptr(),
-                  pad_offsets.data_ptr<int>(), E, H, IN, cur_stream());
+  TORCH_CHECK(y.size(1) == H && act.size(1) == IN && y.size(0) >= act.size(0));
+  TORCH_CHECK(offsets.numel() == E + 1 && offsets.scalar_type() == at::kInt && offsets.is_contiguous());
+  if (act.size(0) == 0) return;
+  TORCH_CHECK(launch_moe_down(y.data_ptr(), act.data_ptr(), w.data_ptr(), offsets.data_ptr<int>(), (int)act.size(0), E,
+                              H, IN, cur_stream()) == 0, "moe_down: 128 KB of LDS are not available");
+}
+
+// topi [T, k] int64 -> (ids [T * k] token of each sorted place, pos [T, k] sorted place of each pair,
+// offsets [E + 1]); a pair without an expert of 0..E-1 gets pos -1
+std::vector<torch::Tensor> moe_sort(torch::Tensor topi, int64_t E) {
+  TORCH_CHECK(topi.is_cuda() && topi.is_contiguous() && topi.scalar_type() == at::kLong && topi.dim() == 2);
+  TORCH_CHECK(E >= 1 && E <= 4096 && topi.numel() < (1LL << 31), "moe_sort: sizes");
+  const int P = topi.numel(), k = topi.size(1);
+  auto i32 = topi.options().dtype(torch::kInt);
+  auto ids = torch::empty({P}, i32), pos = torch::empty({topi.size(0), k}, i32), offsets = torch::empty({E + 1}, i32);
+  launch_moe_sort(ids.data_ptr<int>(), pos.data_ptr<int>(), offsets.data_ptr<int>(), topi.data_ptr<int64_t>(), P,
+                  k > 0 ? k : 1, (int)E, cur_stream());
+  return {ids, pos, offsets};
+}
+
+torch::Tensor moe_combine(torch::Tensor y, torch::Tensor weights, torch::Tensor pos) {
+  CHECK_BF16_CONTIG(y);
+  TORCH_CHECK(weights.is_cuda() && weights.is_contiguous() && weights.scalar_type() == at::kFloat &&
+                  pos.is_cuda() && pos.is_contiguous() && pos.scalar_type() == at::kInt && pos.dim() == 2 &&
+                  weights.sizes() == pos.sizes() && y.dim() == 2 && y.size(1) % 8 == 0 && pos.size(0) <= 65535);
+  auto out = torch::empty({pos.size(0), y.size(1)}, y.options());
+  if (out.numel() == 0) return out;
+  launch_moe_combine(out.data_ptr(), y.data_ptr(), weights.data_ptr<float>(), pos.data_ptr<int>(), (int)pos.size(0),
+                     (int)pos.size(1), (int)y.size(1), cur_stream());
+  return out;
 }
 
 // --- products of a few rows (linear_rows.hip) ---------------------------------
@@ -471,6 +499,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_inputs", &decode_inputs);
   m.def("moe_gateup", &moe_gateup);
   m.def("moe_down", &moe_down);
+  m.def("moe_sort", &moe_sort);
+  m.def("moe_combine", &moe_combine);
   m.def("ipc_allreduce_create", &ipc_allreduce_create);
   m.def("ipc_allreduce_connect", &ipc_allreduce_connect);
   m.def("ipc_allreduce_run", &ipc_allreduce_run);

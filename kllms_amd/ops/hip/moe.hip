@@ -1,278 +1,281 @@
-// Grouped MoE expert GEMMs for gfx950 (Mixtral prefill path).
+// Grouped mixture-of-experts products for gfx950 (prefill shapes):
 //
-// replace the per-expert Python loop (8 experts x
-// mask/gather/2 GEMM/index_add per layer) with TWO MFMA kernel launches:
+//   moe_sort      (token, choice) pairs grouped by expert, without the host
+//   moe_gateup    act[s, :] = silu(x[tok(s)] Wg[e]^T) * (x[tok(s)] Wu[e]^T)
+//   moe_down      y[s, :]   = act[s] Wd[e]^T
+//   moe_combine   out[t, :] = sum over choices j of w[t, j] y[pos(t, j)], in fp32
 //
-//   moe_gateup_kernel: act[s, :] = silu(x[tok(s)] @ Wg[e]^T) * (x[tok(s)] @ Wu[e]^T)
-//   moe_down_kernel:   y[s, :]   = act[s] @ Wd[e]^T
+// The products: a 512-thread workgroup (8 waves, 2 x 4) computes 256 rows of one
+// expert by 256 columns (gate/up: 128 gate and the same 128 up columns), 128 x 64 a
+// wave with v_mfma_f32_32x32x16_bf16 (fragment maps verified by mfma_selftest.hip).
+// K goes by 64 through double-buffered LDS (128 KB, one workgroup per compute unit):
+// the next 64 are fetched to registers under the matrix work of these (32 matrix
+// instructions a wave and stage, 2048 cycles for the two waves of a SIMD), written to
+// the other buffer at the stage's end, one barrier per stage. Rows of 128 bytes, their
+// 16-byte units XORed with the row: staging and fragment reads are conflict-free.
 //
-// over tokens SORTED by expert (host side: argsort + per-expert padding to
-// BM rows; models/mixtral.py). The routing-weight multiply + scatter back to
-// token order is one torch index_add afterwards.
+// Why this tile: 128 x 64 a wave reads 6 KB of LDS for 8 matrix instructions, which
+// with the staging keeps LDS just below the matrix units; 32 x (64 + 64), the tile this
+// replaces, read 5 KB for 4, had one stage of 512 cycles to hide a fetch under, and
+// looped over an expert's rows. 256 rows leave padding (about 512 rows an expert at
+// 2048 tokens are two or three tiles), so the upper four waves of a tile with at most
+// 128 rows only help staging: such a tile takes half the matrix time.
 //
-// Kernel geometry (both kernels): one block = 256 threads = 4 waves computes
-// a [BM=128, BN=64] output tile with v_mfma_f32_32x32x16_bf16 (fragment maps
-// verified by mfma_selftest.hip). Wave w owns rows [32w, 32w+32). The block
-// LOOPS the m-tiles of its (expert, n-tile) so each W panel streams from
-// HBM once and re-reads from its XCD's L2.
+// Workgroups are numbered (expert, column tile, row tile), rows fastest, and dealt to
+// the 8 XCDs in equal runs: an XCD's L2 sees each weight panel once, for its two or
+// three row tiles, and mostly one expert's rows.
 //
-// Operands go THROUGH LDS in full 128-byte lines (the guide's M=256 GEMM
-// recipe): fragment-shaped direct loads put each 16-lane group on 32
-// DIFFERENT cache lines per instruction (TA-path bound — measured 198 TF/s);
-// cooperative row staging + XOR-swizzled ds_read_b128 fragment reads fix the
-// access pattern. Double-buffered BK=64 stages, ONE barrier per stage, with
-// the next stage's global loads issued before the current stage's MFMAs
-// (T14: HBM/L2 latency hides under the matrix work).
+// MEASURED_HERE
 
 #include "common.h"
 
-#define MOE_BM 128
-#define MOE_BN 64
+#define MOE_BM 256
 #define MOE_BK 64                      // k-depth per stage (128 B per row)
-#define ROW_B 128                      // bytes per staged row (64 bf16)
+#define MOE_LDS (2 * 2 * MOE_BM * 128) // two buffers of 256 A rows and 256 B rows
 
 typedef __bf16 bf16x8_mfma __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ bf16x8_mfma load16(const bf16_t* p) {
-  return *reinterpret_cast<const bf16x8_mfma*>(p);
+// byte offset inside a staged tile of 128-byte rows, with the bank-conflict XOR
+__device__ __forceinline__ int tile_off(int row, int unit) {
+  return row * 128 + ((unit ^ (row & 7)) << 4);
 }
 
-__device__ __forceinline__ float silu(float x) {
-  return x / (1.0f + __expf(-x));
-}
+// GATEUP: a = x [T, K] gathered by ids, w [E, 2 * N, K] (gate at [0, N), up behind),
+// out [S, N]. Down: a = act [S, K], w [E, N, K], out [S, N]. offsets [E + 1]: row range
+// of each expert in sorted space.
+template <bool GATEUP>
+__global__ void __launch_bounds__(512) moe_product_kernel(
+    bf16_t* __restrict__ out, const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
+    const int* __restrict__ ids,         // GATEUP: [S] token index, or -1 (a zero row)
+    const bf16_t* __restrict__ zeros,    // GATEUP: [K]
+    const int* __restrict__ offsets, int E, int N, int K) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;   // waves w and w + 4 share a SIMD
+  const int half = lane >> 5, col = lane & 31;
+  constexpr int BN = GATEUP ? 128 : 256;     // output columns of a workgroup
+  const int n_tiles = (N + BN - 1) / BN;
 
-// byte offset inside a staged tile, with the bank-conflict XOR swizzle
-__device__ __forceinline__ int tile_off(int row, int byte_in_row) {
-  return row * ROW_B + (byte_in_row ^ ((row & 7) << 4));
-}
+  // ---- which (expert, column tile, row tile): equal runs per XCD -----------
+  int total = 0;
+  for (int e = 0; e < E; ++e) total += (offsets[e + 1] - offsets[e] + MOE_BM - 1) / MOE_BM;
+  total *= n_tiles;
+  const int run = (total + 7) / 8;
+  int id = (blockIdx.x & 7) * run + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= run || id >= total) return;
+  int e = 0, m_begin = 0, m_end = 0, m_tiles = 0;
+  for (; e < E; ++e) {
+    m_begin = offsets[e];
+    m_end = offsets[e + 1];
+    m_tiles = (m_end - m_begin + MOE_BM - 1) / MOE_BM;
+    if (id < m_tiles * n_tiles) break;
+    id -= m_tiles * n_tiles;
+  }
+  if (e >= E) return;
+  const int n0 = (id / m_tiles) * BN;
+  const int m0 = m_begin + (id % m_tiles) * MOE_BM;
 
-// gate_up: x [T, K] gathered by sorted_ids; w [E, 2*IN, K] fused rows
-// (gate at [0, IN), up at [IN, 2*IN)); act out [S, IN] bf16 in sorted space.
-// pad_offsets [E+1]: sorted-space row range of expert e (multiples of BM).
-extern "C" __global__ void __launch_bounds__(256) moe_gateup_kernel(
-    bf16_t* __restrict__ act,            // [S, IN]
-    const bf16_t* __restrict__ x,        // [T, K]
-    const bf16_t* __restrict__ w,        // [E, 2*IN, K]
-    const int* __restrict__ sorted_ids,  // [S] token index or -1 (pad)
-    const int* __restrict__ pad_offsets, // [E+1]
-    const bf16_t* __restrict__ zeros,    // [K] zero page for pad rows
-    int IN, int K, int n_tiles) {
-  const int e = blockIdx.x / n_tiles;
-  const int n0 = (blockIdx.x % n_tiles) * MOE_BN;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wv = tid >> 6;
-  const int half = lane >> 5;
-  const int jc = lane & 31;
-
-  const int m_begin = pad_offsets[e];
-  const int m_end = pad_offsets[e + 1];
-  const bf16_t* we = w + (long)e * (2 * (long)IN) * K;
-
-  // staging assignment: thread t stages 64 B (4 x 16 B) of one row
-  const int st_arow = tid >> 1;                 // A: 128 rows x 2 threads
-  const int st_aoff = (tid & 1) * 32;           // element offset in the row
-  const int st_brow = (tid & 127) >> 1;         // B: 64 rows x 2 threads
-  const int st_boff = (tid & 1) * 32;
-  const bool st_up = tid >= 128;                // low half: gate, high: up
-  const bf16_t* st_bsrc =
-      we + ((long)((st_up ? IN : 0) + n0 + st_brow)) * K + st_boff;
-
-  // [2 buffers][A 16 KB + gate 8 KB + up 8 KB] (offset selection — pointer
-  // arrays into LDS fail to compile as static initializers)
-  __shared__ __attribute__((aligned(16))) char smem[2 * (MOE_BM + 2 * MOE_BN) * ROW_B];
-  const int BUF_STRIDE = (MOE_BM + 2 * MOE_BN) * ROW_B;
-  auto a_lds = [&](int b) -> char* { return smem + b * BUF_STRIDE; };
-  auto g_lds = [&](int b) -> char* { return smem + b * BUF_STRIDE + MOE_BM * ROW_B; };
-  auto u_lds = [&](int b) -> char* { return smem + b * BUF_STRIDE + (MOE_BM + MOE_BN) * ROW_B; };
-
-  const int n_stages = K / MOE_BK;
-
-  for (int m0 = m_begin; m0 < m_end; m0 += MOE_BM) {
-    const int tok = sorted_ids[m0 + st_arow];
-    const bf16_t* st_asrc = ((tok >= 0) ? x + (long)tok * K : zeros) + st_aoff;
-
-    f32x16 accg[2] = {{}, {}};
-    f32x16 accu[2] = {{}, {}};
-
-    bf16x8_vec ra[4], rb[4];
-    auto ld = [&](int stage) {
-      const bf16_t* ap = st_asrc + stage * MOE_BK;
-      const bf16_t* bp = st_bsrc + stage * MOE_BK;
+  // ---- staging: 4 rows of A and of B per thread, 16 bytes each --------------
+  const int st_row = tid >> 3, st_unit = tid & 7;   // rows st_row + 64 i
+  const char* a_src[4];
+  const char* b_src[4];
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        ra[p] = reinterpret_cast<const bf16x8_vec*>(ap)[p];
-        rb[p] = reinterpret_cast<const bf16x8_vec*>(bp)[p];
-      }
-    };
-    auto st = [&](int buf) {
-      char* bt = st_up ? u_lds(buf) : g_lds(buf);
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        *reinterpret_cast<bf16x8_vec*>(
-            a_lds(buf) + tile_off(st_arow, st_aoff * 2 + p * 16)) = ra[p];
-        *reinterpret_cast<bf16x8_vec*>(
-            bt + tile_off(st_brow, st_boff * 2 + p * 16)) = rb[p];
-      }
-    };
-
-    ld(0);
-    st(0);
-    __syncthreads();
-    for (int stage = 0; stage < n_stages; ++stage) {
-      if (stage + 1 < n_stages) ld(stage + 1);
-      const int buf = stage & 1;
-      const int arow = wv * 32 + jc;
-#pragma unroll
-      for (int wdw = 0; wdw < 4; ++wdw) {            // 4 k-windows of 16
-        const int bib = wdw * 32 + half * 16;
-        const bf16x8_mfma af = *reinterpret_cast<const bf16x8_mfma*>(
-            a_lds(buf) + tile_off(arow, bib));
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) {
-          const int brow = ct * 32 + jc;
-          const bf16x8_mfma gf = *reinterpret_cast<const bf16x8_mfma*>(
-              g_lds(buf) + tile_off(brow, bib));
-          const bf16x8_mfma uf = *reinterpret_cast<const bf16x8_mfma*>(
-              u_lds(buf) + tile_off(brow, bib));
-          accg[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, gf, accg[ct], 0, 0, 0);
-          accu[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, uf, accu[ct], 0, 0, 0);
-        }
-      }
-      if (stage + 1 < n_stages) st(1 - buf);
-      __syncthreads();
+  for (int i = 0; i < 4; ++i) {
+    const int r = min(m0 + st_row + 64 * i, m_end - 1);
+    if constexpr (GATEUP) {
+      const int tok = ids[r];
+      a_src[i] = (const char*)(tok >= 0 ? a + (int64_t)tok * K : zeros) + st_unit * 16;
+      // B rows 0..127 gate, 128..255 up of the same columns
+      const int n = min(n0 + ((st_row + 64 * i) & 127), N - 1) + (i >= 2 ? N : 0);
+      b_src[i] = (const char*)(w + ((int64_t)e * 2 * N + n) * K) + st_unit * 16;
+    } else {
+      a_src[i] = (const char*)(a + (int64_t)r * K) + st_unit * 16;
+      b_src[i] = (const char*)(w + ((int64_t)e * N + min(n0 + st_row + 64 * i, N - 1)) * K) + st_unit * 16;
     }
+  }
+  u32x4 ra[4], rb[4];
+  auto load = [&](int stage) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ra[i] = *reinterpret_cast<const u32x4*>(a_src[i] + (int64_t)stage * 128);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rb[i] = *reinterpret_cast<const u32x4*>(b_src[i] + (int64_t)stage * 128);
+  };
+  auto store = [&](int buf) {
+    char* base = smem + buf * (2 * MOE_BM * 128);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(base + tile_off(st_row + 64 * i, st_unit)) = ra[i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u32x4*>(base + MOE_BM * 128 + tile_off(st_row + 64 * i, st_unit)) = rb[i];
+  };
 
-    // epilogue: silu(gate) * up -> act rows (sorted space; pad rows land in
-    // pad slots that the down kernel's own pad handling discards)
+  f32x16 acc[4][2] = {};
+  const bool busy = m0 + wm * 128 < m_end;
+  // B rows of this wave's two column sets
+  const int b0 = GATEUP ? wn * 32 + col : wn * 64 + col;
+  const int b1 = GATEUP ? 128 + wn * 32 + col : wn * 64 + 32 + col;
+  const int stages = K / MOE_BK;
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int s = 0; s < stages; ++s) {
+    const bool more = s + 1 < stages;
+    if (more) load(s + 1);
+    if (busy) {
+      const char* at = smem + (s & 1) * (2 * MOE_BM * 128);
+      const char* bt = at + MOE_BM * 128;
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
+      for (int kw = 0; kw < 4; ++kw) {            // 4 k-windows of 16
+        const int unit = kw * 2 + half;
+        bf16x8_mfma bf[2], af[4];
+        bf[0] = *reinterpret_cast<const bf16x8_mfma*>(bt + tile_off(b0, unit));
+        bf[1] = *reinterpret_cast<const bf16x8_mfma*>(bt + tile_off(b1, unit));
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = (r & 3) + 8 * (r >> 2) + 4 * half;   // D-row map
-        const long out_row = m0 + wv * 32 + i;
-        act[out_row * IN + n0 + ct * 32 + jc] =
-            __float2bfloat16(silu(accg[ct][r]) * accu[ct][r]);
+        for (int mt = 0; mt < 4; ++mt)
+          af[mt] = *reinterpret_cast<const bf16x8_mfma*>(at + tile_off(wm * 128 + mt * 32 + col, unit));
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[mt][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mt], bf[j], acc[mt][j], 0, 0, 0);
+      }
+    }
+    if (more) store((s + 1) & 1);
+    __syncthreads();
+  }
+
+  // lane: column col of the set, rows (r & 3) + 8 (r >> 2) + 4 half of each 32
+  if (!busy) return;
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = m0 + wm * 128 + mt * 32 + (r & 3) + 8 * (r >> 2) + 4 * half;
+      if (row >= m_end) continue;
+      if constexpr (GATEUP) {
+        const int n = n0 + wn * 32 + col;
+        const float g = acc[mt][0][r];
+        if (n < N) ((short*)out)[(int64_t)row * N + n] = f32_to_bf16(g / (1.0f + __expf(-g)) * acc[mt][1][r]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int n = n0 + wn * 64 + j * 32 + col;
+          if (n < N) ((short*)out)[(int64_t)row * N + n] = f32_to_bf16(acc[mt][j][r]);
+        }
       }
     }
   }
 }
 
-// down: y[s, :] = act[s] @ Wd[e]^T ; Wd [E, H, IN]; y [S, H] bf16 (sorted
-// space, pad rows garbage-but-confined — rows are independent in MFMA).
-extern "C" __global__ void __launch_bounds__(256) moe_down_kernel(
-    bf16_t* __restrict__ y,              // [S, H]
-    const bf16_t* __restrict__ act,      // [S, IN]
-    const bf16_t* __restrict__ w,        // [E, H, IN]
-    const int* __restrict__ pad_offsets, // [E+1]
-    int H, int IN, int n_tiles) {
-  const int e = blockIdx.x / n_tiles;
-  const int n0 = (blockIdx.x % n_tiles) * MOE_BN;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wv = tid >> 6;
-  const int half = lane >> 5;
-  const int jc = lane & 31;
-
-  const int m_begin = pad_offsets[e];
-  const int m_end = pad_offsets[e + 1];
-  const bf16_t* we = w + (long)e * (long)H * IN;
-
-  const int st_arow = tid >> 1;
-  const int st_aoff = (tid & 1) * 32;
-  const int st_brow = (tid & 127) >> 1;
-  const int st_boff = (tid & 1) * 32;
-  const bool st_b = tid < 128;                  // low half stages B
-  const bf16_t* st_bsrc = we + ((long)(n0 + st_brow)) * IN + st_boff;
-
-  __shared__ __attribute__((aligned(16))) char smem[2 * (MOE_BM + MOE_BN) * ROW_B];
-  const int BUF_STRIDE = (MOE_BM + MOE_BN) * ROW_B;
-  auto a_lds = [&](int b) -> char* { return smem + b * BUF_STRIDE; };
-  auto b_lds = [&](int b) -> char* { return smem + b * BUF_STRIDE + MOE_BM * ROW_B; };
-
-  const int n_stages = IN / MOE_BK;
-
-  for (int m0 = m_begin; m0 < m_end; m0 += MOE_BM) {
-    const bf16_t* st_asrc = act + (long)(m0 + st_arow) * IN + st_aoff;
-
-    f32x16 acc[2] = {{}, {}};
-    bf16x8_vec ra[4], rb[4];
-    auto ld = [&](int stage) {
-      const bf16_t* ap = st_asrc + stage * MOE_BK;
-#pragma unroll
-      for (int p = 0; p < 4; ++p) ra[p] = reinterpret_cast<const bf16x8_vec*>(ap)[p];
-      if (st_b) {
-        const bf16_t* bp = st_bsrc + stage * MOE_BK;
-#pragma unroll
-        for (int p = 0; p < 4; ++p) rb[p] = reinterpret_cast<const bf16x8_vec*>(bp)[p];
-      }
-    };
-    auto st = [&](int buf) {
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        *reinterpret_cast<bf16x8_vec*>(
-            a_lds(buf) + tile_off(st_arow, st_aoff * 2 + p * 16)) = ra[p];
-      }
-      if (st_b) {
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-          *reinterpret_cast<bf16x8_vec*>(
-              b_lds(buf) + tile_off(st_brow, st_boff * 2 + p * 16)) = rb[p];
-        }
-      }
-    };
-
-    ld(0);
-    st(0);
-    __syncthreads();
-    for (int stage = 0; stage < n_stages; ++stage) {
-      if (stage + 1 < n_stages) ld(stage + 1);
-      const int buf = stage & 1;
-      const int arow = wv * 32 + jc;
-#pragma unroll
-      for (int wdw = 0; wdw < 4; ++wdw) {
-        const int bib = wdw * 32 + half * 16;
-        const bf16x8_mfma af = *reinterpret_cast<const bf16x8_mfma*>(
-            a_lds(buf) + tile_off(arow, bib));
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) {
-          const int brow = ct * 32 + jc;
-          const bf16x8_mfma bf = *reinterpret_cast<const bf16x8_mfma*>(
-              b_lds(buf) + tile_off(brow, bib));
-          acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bf, acc[ct], 0, 0, 0);
-        }
-      }
-      if (stage + 1 < n_stages) st(1 - buf);
-      __syncthreads();
+// topi [P] (P = tokens x choices) -> offsets [E + 1], pos [P] = sorted place of each
+// pair, ids [P] = token of each sorted place. One workgroup: counts by wave ballots,
+// which also give the places (same order as the pairs' within a wave's 64; the order
+// inside an expert matters to nobody).
+__global__ void __launch_bounds__(1024) moe_sort_kernel(int* __restrict__ ids, int* __restrict__ pos,
+                                                        int* __restrict__ offsets, const int64_t* __restrict__ topi,
+                                                        int P, int k, int E) {
+  extern __shared__ int cnt[];           // [E] counts, then cursors
+  const int tid = threadIdx.x, lane = tid & 63;
+  for (int e = tid; e < E; e += 1024) cnt[e] = 0;
+  __syncthreads();
+  for (int p0 = 0; p0 < P; p0 += 1024) {
+    const int p = p0 + tid;
+    const int e = p < P ? (int)topi[p] : -1;
+    for (int c = 0; c < E; ++c) {
+      const unsigned long long m = __ballot(e == c);
+      if (m && lane == 0) atomicAdd(&cnt[c], (int)__popcll(m));
     }
-
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = (r & 3) + 8 * (r >> 2) + 4 * half;
-        const long out_row = m0 + wv * 32 + i;
-        y[out_row * H + n0 + ct * 32 + jc] = __float2bfloat16(acc[ct][r]);
-      }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int at = 0;
+    for (int e = 0; e < E; ++e) {
+      const int n = cnt[e];
+      offsets[e] = at;
+      cnt[e] = at;
+      at += n;
+    }
+    offsets[E] = at;
+  }
+  __syncthreads();
+  for (int p0 = 0; p0 < P; p0 += 1024) {
+    const int p = p0 + tid;
+    const int e = p < P ? (int)topi[p] : -1;
+    int place = -1;
+    for (int c = 0; c < E; ++c) {
+      const unsigned long long m = __ballot(e == c);
+      if (!m) continue;
+      int first = 0;
+      if (lane == 0) first = atomicAdd(&cnt[c], (int)__popcll(m));
+      first = __shfl(first, 0);
+      if (e == c) place = first + (int)__popcll(m & ((1ULL << lane) - 1));
+    }
+    if (p < P) {
+      pos[p] = place;
+      if (place >= 0) ids[place] = p / k;
     }
   }
 }
 
-extern "C" void launch_moe_gateup(void* act, const void* x, const void* w,
-                                  const int* sorted_ids, const int* pad_offsets,
-                                  const void* zeros, int E, int IN, int K,
-                                  hipStream_t stream) {
-  const int n_tiles = IN / MOE_BN;
-  hipLaunchKernelGGL(moe_gateup_kernel, dim3(E * n_tiles), dim3(256), 0, stream,
-                     (bf16_t*)act, (const bf16_t*)x, (const bf16_t*)w,
-                     sorted_ids, pad_offsets, (const bf16_t*)zeros, IN, K, n_tiles);
+__global__ void __launch_bounds__(256) moe_combine_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ y,
+                                                          const float* __restrict__ weights,
+                                                          const int* __restrict__ pos, int k, int nvec) {
+  const int t = blockIdx.y;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= nvec) return;
+  float s[8] = {};
+  for (int j = 0; j < k; ++j) {
+    const int p = pos[t * k + j];
+    if (p < 0) continue;
+    const float w = weights[t * k + j];
+    const bf16x8_vec v = reinterpret_cast<const bf16x8_vec*>(y)[(int64_t)p * nvec + i];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) s[c] += w * bf16_to_f32(v[c]);
+  }
+  bf16x8_vec o;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) o[c] = f32_to_bf16(s[c]);
+  reinterpret_cast<bf16x8_vec*>(out)[(int64_t)t * nvec + i] = o;
 }
 
-extern "C" void launch_moe_down(void* y, const void* act, const void* w,
-                                const int* pad_offsets, int E, int H, int IN,
+// room for 128 KB of LDS; once per process and kernel is enough, a repeat harmless
+template <bool GATEUP>
+static bool lds_ready() {
+  static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_product_kernel<GATEUP>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, MOE_LDS) == hipSuccess;
+  return ok;
+}
+
+// rows S in sorted space; the grid holds the most tiles that S rows of E experts can
+// make. Returns 0, or -1 where the LDS cannot be had
+extern "C" int launch_moe_gateup(void* act, const void* x, const void* w, const int* sorted_ids, const int* offsets,
+                                 const void* zeros, int S, int E, int IN, int K, hipStream_t stream) {
+  if (!lds_ready<true>()) return -1;
+  const int64_t blocks = (int64_t)(S / MOE_BM + E) * ((IN + 127) / 128);
+  hipLaunchKernelGGL(moe_product_kernel<true>, dim3((blocks + 7) / 8 * 8), dim3(512), MOE_LDS, stream, (bf16_t*)act,
+                     (const bf16_t*)x, (const bf16_t*)w, sorted_ids, (const bf16_t*)zeros, offsets, E, IN, K);
+  return 0;
+}
+
+extern "C" int launch_moe_down(void* y, const void* act, const void* w, const int* offsets, int S, int E, int H,
+                               int IN, hipStream_t stream) {
+  if (!lds_ready<false>()) return -1;
+  const int64_t blocks = (int64_t)(S / MOE_BM + E) * ((H + 255) / 256);
+  hipLaunchKernelGGL(moe_product_kernel<false>, dim3((blocks + 7) / 8 * 8), dim3(512), MOE_LDS, stream, (bf16_t*)y,
+                     (const bf16_t*)act, (const bf16_t*)w, nullptr, nullptr, offsets, E, H, IN);
+  return 0;
+}
+
+extern "C" void launch_moe_sort(int* ids, int* pos, int* offsets, const int64_t* topi, int P, int k, int E,
                                 hipStream_t stream) {
-  const int n_tiles = H / MOE_BN;
-  hipLaunchKernelGGL(moe_down_kernel, dim3(E * n_tiles), dim3(256), 0, stream,
-                     (bf16_t*)y, (const bf16_t*)act, (const bf16_t*)w,
-                     pad_offsets, H, IN, n_tiles);
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), E * sizeof(int), stream, ids, pos, offsets, topi, P, k, E);
+}
+
+extern "C" void launch_moe_combine(void* out, const void* y, const float* weights, const int* pos, int T, int k,
+                                   int H, hipStream_t stream) {
+  const int nvec = H / 8;
+  hipLaunchKernelGGL(moe_combine_kernel, dim3((nvec + 255) / 256, T), dim3(256), 0, stream, (bf16_t*)out,
+                     (const bf16_t*)y, weights, pos, k, nvec);
 }
