@@ -10,9 +10,12 @@
 // wave with v_mfma_f32_32x32x16_bf16 (fragment maps verified by mfma_selftest.hip).
 // K goes by 64 through double-buffered LDS (128 KB, one workgroup per compute unit):
 // the next 64 are fetched to registers under the matrix work of these (32 matrix
-// instructions a wave and stage, 2048 cycles for the two waves of a SIMD), written to
-// the other buffer at the stage's end, one barrier per stage. Rows of 128 bytes, their
-// 16-byte units XORed with the row: staging and fragment reads are conflict-free.
+// instructions a wave and stage, 2048 cycles for the two waves of a SIMD) and written
+// to the other buffer between the last ones, one barrier per stage. A stage is one
+// branch-free scheduling region whose issue order is fixed: the next k-window's LDS
+// reads between this one's matrix instructions (left to itself the compiler reads,
+// waits and multiplies in turn: 15% slower). Rows of 128 bytes, their 16-byte units
+// XORed with the row: staging and fragment reads are conflict-free.
 //
 // Why this tile: 128 x 64 a wave reads 6 KB of LDS for 8 matrix instructions, which
 // with the staging keeps LDS just below the matrix units; 32 x (64 + 64), the tile this
@@ -25,7 +28,9 @@
 // the 8 XCDs in equal runs: an XCD's L2 sees each weight panel once, for its two or
 // three row tiles, and mostly one expert's rows.
 //
-// MEASURED_HERE
+// Measured at 2048 rows, 8 experts of 14336, top 2, width 4096: gate/up 1174 us (820
+// TFLOP/s; 2714 before), down 791 (608: 320 tiles are a round and a quarter; 1347
+// before); with routing around them 1903 us (4358).
 
 #include "common.h"
 
@@ -113,36 +118,64 @@ __global__ void __launch_bounds__(512) moe_product_kernel(
 
   f32x16 acc[4][2] = {};
   const bool busy = m0 + wm * 128 < m_end;
-  // B rows of this wave's two column sets
-  const int b0 = GATEUP ? wn * 32 + col : wn * 64 + col;
-  const int b1 = GATEUP ? 128 + wn * 32 + col : wn * 64 + 32 + col;
+  // Fragment addresses: rows of a wave's sets differ by multiples of 32, so one XORed
+  // offset per k-window serves them all and the rows are immediate offsets.
+  int at_kw[4];
+#pragma unroll
+  for (int kw = 0; kw < 4; ++kw) at_kw[kw] = col * 128 + (((kw * 2 + half) ^ (col & 7)) << 4);
+  const int a_off = wm * 128 * 128;
+  const int b_off = MOE_BM * 128 + (GATEUP ? wn * 32 : wn * 64) * 128;
+  constexpr int B_SET = (GATEUP ? 128 : 32) * 128;   // from a wave's first column set to its second
   const int stages = K / MOE_BK;
   load(0);
   store(0);
   __syncthreads();
+  // the last stage fetches and stores itself again: one scheduling region, no branches
   for (int s = 0; s < stages; ++s) {
-    const bool more = s + 1 < stages;
-    if (more) load(s + 1);
+    load(min(s + 1, stages - 1));
     if (busy) {
-      const char* at = smem + (s & 1) * (2 * MOE_BM * 128);
-      const char* bt = at + MOE_BM * 128;
+      const char* base = smem + (s & 1) * (2 * MOE_BM * 128);
+      bf16x8_mfma af[2][4], bf[2][2];
+      auto fetch = [&](int kw) {
+        const char* p = base + at_kw[kw];
 #pragma unroll
-      for (int kw = 0; kw < 4; ++kw) {            // 4 k-windows of 16
-        const int unit = kw * 2 + half;
-        bf16x8_mfma bf[2], af[4];
-        bf[0] = *reinterpret_cast<const bf16x8_mfma*>(bt + tile_off(b0, unit));
-        bf[1] = *reinterpret_cast<const bf16x8_mfma*>(bt + tile_off(b1, unit));
+        for (int j = 0; j < 2; ++j)
+          bf[kw & 1][j] = *reinterpret_cast<const bf16x8_mfma*>(p + b_off + j * B_SET);
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
-          af[mt] = *reinterpret_cast<const bf16x8_mfma*>(at + tile_off(wm * 128 + mt * 32 + col, unit));
+          af[kw & 1][mt] = *reinterpret_cast<const bf16x8_mfma*>(p + a_off + mt * 32 * 128);
+      };
+      // the next window's fragments are read under this one's matrix work
+      fetch(0);
+#pragma unroll
+      for (int kw = 0; kw < 4; ++kw) {            // 4 k-windows of 16
+        if (kw < 3) fetch(kw + 1);
+        else store((s + 1) & 1);
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
           for (int j = 0; j < 2; ++j)
-            acc[mt][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mt], bf[j], acc[mt][j], 0, 0, 0);
+            acc[mt][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kw & 1][mt], bf[kw & 1][j], acc[mt][j], 0, 0, 0);
       }
+      // order of issue: six reads, then per window the next one's reads between matrix instructions
+      __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+      for (int kw = 0; kw < 3; ++kw) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+      }
+    } else {
+      store((s + 1) & 1);
     }
-    if (more) store((s + 1) & 1);
     __syncthreads();
   }
 
