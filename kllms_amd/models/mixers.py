@@ -64,6 +64,24 @@ def single_rows(batch) -> bool:
     return batch.mode == "decode" or (batch.host_segs is not None and all(n == 1 for _, n in batch.host_segs))
 
 
+# steps whose longest segment is shorter than this run their fixed-decay recurrences token by token
+MIN_CHUNK_ROWS = 16
+
+
+def step_chunks(batch, dim: int):
+    """The step's rows cut into chunks for the chunk-parallel form of a
+    fixed-decay recurrence of key size ``dim`` (built once per step), or None
+    for the token-by-token form."""
+    if (batch.host_segs is None or batch.plans is None or not batch.positions.is_cuda
+            or dim > ops.RETENTION_MAX_DIM):
+        return None
+    key = "retention_chunks"
+    if key not in batch.plans:
+        long = max((n for _, n in batch.host_segs), default=0) >= MIN_CHUNK_ROWS
+        batch.plans[key] = ops.retention_chunks(batch.host_segs, batch.positions.device) if long else None
+    return batch.plans[key]
+
+
 class FusedInput(nn.Module):
     """Several projections of the same input as ONE GEMM: the checkpoint's
     separate [out_i, in] matrices are stacked along the output dim (optionally
@@ -175,8 +193,14 @@ class BlockLocalAttention(nn.Module):
         plan = self._dense_plan(q, batch)
         if plan is None:
             ops.rope_pairs_store(q, k, v, batch.positions, self.inv_freq, st.k, st.v, batch.slot_mapping)
-            att = ops.attn_blocklocal_paged(q, st.k, st.v, batch.block_tables, batch.token_seg,
-                                            batch.positions, sp.scale, sp.mask_size, gate)
+            if (single_rows(batch) and batch.context_lens is not None and batch.block_tables.shape[0] == T
+                    and ops.blocklocal_rows_ok(q, st.k, st.v, gate)):
+                # row i is segment i: the decode kernel, whose heads of a group share their keys
+                att = ops.attn_blocklocal_rows(q, st.k, st.v, batch.block_tables, batch.context_lens, sp.scale,
+                                               sp.mask_size, gate)
+            else:
+                att = ops.attn_blocklocal_paged(q, st.k, st.v, batch.block_tables, batch.token_seg,
+                                                batch.positions, sp.scale, sp.mask_size, gate)
         else:
             (gs, gq, gl), row_map = plan
             fresh = torch.empty((T, 2, sp.kv_heads, sp.dim), dtype=q.dtype, device=q.device)
@@ -213,7 +237,7 @@ class DecayLinearAttention(nn.Module):
         sp = self.spec
         o = ops.linear_attn_decay(q.unflatten(1, (sp.heads, sp.dim)), k.unflatten(1, (sp.heads, sp.dim)),
                                   v.unflatten(1, (sp.heads, sp.vdim)), self.decay, st.rec,
-                                  batch.state_slots, batch.cu_seqlens, batch.seg_start)
+                                  batch.state_slots, batch.cu_seqlens, batch.seg_start, step_chunks(batch, sp.dim))
         y = ops.gated_rmsnorm(o.view(o.shape[0], 1, -1), self.norm, gate, self.eps, self.o_proj.dtype)
         return F.linear(y, self.o_proj)
 
@@ -493,21 +517,6 @@ class Retention(nn.Module):
         sp = self.spec
         return LayerCacheSpec(rec=(sp.heads, sp.dim, sp.vdim))
 
-    # steps whose longest segment is shorter than this run token by token
-    MIN_CHUNK_ROWS = 16
-
-    def _chunks(self, batch):
-        """The step's rows cut into chunks for the chunk-parallel form (built
-        once per step), or None for the token-by-token form."""
-        if (batch.host_segs is None or batch.plans is None or not batch.positions.is_cuda
-                or self.spec.dim > ops.RETENTION_MAX_DIM):
-            return None
-        key = "retention_chunks"
-        if key not in batch.plans:
-            long = max((n for _, n in batch.host_segs), default=0) >= self.MIN_CHUNK_ROWS
-            batch.plans[key] = ops.retention_chunks(batch.host_segs, batch.positions.device) if long else None
-        return batch.plans[key]
-
     def forward(self, h: torch.Tensor, batch, st: LayerState) -> torch.Tensor:
         sp = self.spec
         y = self.inp(h)
@@ -515,7 +524,7 @@ class Retention(nn.Module):
         r = ops.retention_mix_out(s(y, "q").unflatten(1, (sp.heads, sp.dim)), s(y, "k").unflatten(1, (sp.heads, sp.dim)),
                                   s(y, "v").unflatten(1, (sp.heads, sp.vdim)), s(y, "g"), self.decay, batch.positions,
                                   self.inv_freq, st.rec, batch.state_slots, batch.cu_seqlens, batch.seg_start,
-                                  self.eps, self.o_proj.dtype, self._chunks(batch), single_rows(batch))
+                                  self.eps, self.o_proj.dtype, step_chunks(batch, sp.dim), single_rows(batch))
         return F.linear(r, self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:

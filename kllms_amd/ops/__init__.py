@@ -93,7 +93,7 @@ def store_kv(
     """k_scale/v_scale: [NB, KVH, BS] fp32 per-row dequant scales, REQUIRED
     when the caches are fp8 (written here: s = amax(|row|)/448), None for bf16."""
     if k.is_cuda and not _force_torch():
-        none = torch.empty(0, dtype=torch.float32, device=k.device)
+        none = _none(k, torch.float32)
         _hip_or_raise().store_kv(
             k, v, k_cache, v_cache, slot_mapping,
             k_scale if k_scale is not None else none,
@@ -149,10 +149,27 @@ def attn_segments_paged(q, k_cache, v_cache, block_tables, context_lens, scale, 
     """Rows of long segments on the matrix cores against the paged bf16 cache, the others row by row (GPU only)."""
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     _hip_or_raise().attn_prefill_paged(out, q, k_cache, v_cache, plan, seg_tables, seg_start, scale)
-    f = torch.empty(0, dtype=torch.float32, device=q.device)
+    f = _none(q, torch.float32)
     for r, n in short:
         _hip_or_raise().attn_decode_paged(out[r:r + n], q[r:r + n], k_cache, v_cache, block_tables[r:r + n],
-                                          context_lens[r:r + n], scale, f, f)
+                                          context_lens[r:r + n], scale, f, f, f)
+    return out
+
+
+def blocklocal_rows_ok(q, k_cache, v_cache, gate) -> bool:
+    """Whether attn_blocklocal_rows takes a step: bf16, head sizes of 128, a group size the decode kernel has."""
+    return (_gpu(q) and q.dtype == torch.bfloat16 and k_cache.dtype == torch.bfloat16 and q.shape[2] == 128
+            and k_cache.shape[3] == 128 and v_cache.shape[3] == 128 and q.shape[1] // k_cache.shape[1] in (1, 2, 4, 8)
+            and q.shape[1] % k_cache.shape[1] == 0 and (gate is None or gate.dtype == torch.bfloat16)
+            and q.stride(2) == 1 and q.stride(1) == 128)
+
+
+def attn_blocklocal_rows(q, k_cache, v_cache, block_tables, context_lens, scale, mask_size, gate=None):
+    """Single decoded rows of the block-local mask (0: plain causal), per-head gate: row i against table row i."""
+    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    f = _none(q, torch.float32)
+    _hip_or_raise().attn_decode_paged(out, q, k_cache, v_cache, block_tables, context_lens, scale, f, f,
+                                      gate if gate is not None else f, int(mask_size))
     return out
 
 
@@ -168,11 +185,11 @@ def attn_decode_paged(
 ) -> torch.Tensor:
     if q.is_cuda and not _force_torch():
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        none = torch.empty(0, dtype=torch.float32, device=q.device)
+        none = _none(q, torch.float32)
         _hip_or_raise().attn_decode_paged(
             out, q, k_cache, v_cache, block_tables, context_lens, scale,
             k_scale if k_scale is not None else none,
-            v_scale if v_scale is not None else none)
+            v_scale if v_scale is not None else none, none)
         return out
     return torch_ref.attn_decode_paged(q, k_cache, v_cache, block_tables, context_lens, scale,
                                        k_scale, v_scale)
@@ -220,9 +237,9 @@ def add_norm_rows(part, residual, weight, eps):
 
 def rope_store_rows(part, bias, num_heads, positions, cos_sin, k_cache, v_cache, slot_mapping, k_scale=None, v_scale=None):
     """Rotates q and k of the fused qkv sums, stores k and v into the paged cache; returns q [M, H, 128]."""
-    f = torch.empty(0, dtype=torch.float32, device=part.device)
+    f = _none(part, torch.float32)
     return _hip_or_raise().rope_store_rows(
-        part, bias if bias is not None else torch.empty(0, dtype=torch.bfloat16, device=part.device), num_heads,
+        part, bias if bias is not None else _none(part, torch.bfloat16), num_heads,
         positions, cos_sin, k_cache, v_cache, slot_mapping, k_scale if k_scale is not None else f,
         v_scale if v_scale is not None else f)
 
@@ -256,8 +273,8 @@ def sample(
         logprobs = torch.empty(B, dtype=torch.float32, device=logits.device)
         _hip_or_raise().sample(
             tokens, logprobs, logits, temperatures, top_ps, top_ks, seeds, steps,
-            mask if mask is not None else torch.empty(0, dtype=torch.int32, device=logits.device),
-            dbg if dbg is not None else torch.empty(0, dtype=torch.float32, device=logits.device),
+            mask if mask is not None else _none(logits, torch.int32),
+            dbg if dbg is not None else _none(logits, torch.float32),
         )
         return tokens, logprobs
     return torch_ref.sample(logits, temperatures, top_ps, top_ks, seeds, steps, mask)
@@ -335,8 +352,16 @@ def _gpu(t: torch.Tensor) -> bool:
     return t.is_cuda and not _force_torch()
 
 
+_NONE: dict = {}   # (dtype, device) -> an empty tensor standing for "not given"; it holds nothing, so sharing is safe
+
+
 def _none(ref: torch.Tensor, dtype=None) -> torch.Tensor:
-    return torch.empty(0, dtype=dtype or ref.dtype, device=ref.device)
+    key = (dtype or ref.dtype, ref.device)
+    t = _NONE.get(key)
+    if t is None:
+        with torch.inference_mode(False):
+            t = _NONE[key] = torch.empty(0, dtype=key[0], device=key[1])
+    return t
 
 
 def embed_rmsnorm(ids, table, weight, eps, pos_table=None, positions=None):
@@ -450,10 +475,15 @@ def head_gate(out, gate) -> None:
     out.mul_(torch.sigmoid(gate.float()).unsqueeze(-1).to(out.dtype))
 
 
-def linear_attn_decay(q, k, v, decay, state, state_slots, cu_seqlens, seg_start):
+def linear_attn_decay(q, k, v, decay, state, state_slots, cu_seqlens, seg_start, chunks=None):
+    """S <- decay_h S + silu(k) silu(v)^T, o = S^T silu(q) over segments; o [T,
+    H, V] fp32. ``chunks`` (GPU, from retention_chunks): the chunk-parallel form;
+    None: token by token."""
     if _gpu(q):
         o = torch.empty((q.shape[0], q.shape[1], v.shape[2]), dtype=torch.float32, device=q.device)
-        _seq().linear_attn_decay(o, q, k, v, decay, state, state_slots, cu_seqlens, seg_start)
+        e = _none(q, torch.int32)
+        ch, c0 = chunks if chunks is not None else (e, e)
+        _seq().linear_attn_decay(o, q, k, v, decay, state, state_slots, cu_seqlens, seg_start, ch, c0)
         return o
     return torch_ref.linear_attn_decay(q, k, v, decay, state, state_slots, cu_seqlens, seg_start)
 

@@ -24,12 +24,15 @@
 // prompt's rows in that XCD's L2.
 //
 // Layouts: q [B, H, D=128]; caches [NB, KVH, BS, D]; block_tables [B, MAXB];
-// context_lens INCLUDE the current token. GQA in {1, 2, 4, 8}.
+// context_lens INCLUDE the current token. GQA in {1, 2, 4, 8}. Optionally a context sees
+// only its last token's aligned block of mask_size positions, and each head's result
+// passes a sigmoid gate (the block-local layers of the hybrid family).
 //
 // Measured with the merge, 32 heads / 8 kv heads, beside 256-key workgroups with
 // block-wide passes: 120 streams of 560 keys 36.5 us (68), 5 streams 8.5 us (23), 16
 // fp8 streams of 5850 keys 49 us (109, 198 MB: 4 TB/s); 16 / 4 heads, one stream of
-// 170 keys 7.8 us (21).
+// 170 keys 7.8 us (21); block-local, 40 rows of 600 keys, 16 / 4 heads,
+// 20.5 us (81 with a workgroup per row and q-head).
 
 #include "common.h"
 
@@ -61,6 +64,17 @@ __device__ __forceinline__ Frag fp8x8_to_bf16(u32x2 v) {
   return f;
 }
 
+// first key that a context of L keys sees: 0, or the start of its last token's aligned
+// block of mask_size positions
+__device__ __forceinline__ int first_key(int L, int mask_size) {
+  return mask_size > 0 ? max(L - 1, 0) / mask_size * mask_size : 0;
+}
+
+__device__ __forceinline__ float head_gate(const bf16_t* __restrict__ gate, int stride, int b, int h) {
+  if (!gate) return 1.0f;
+  return 1.0f / (1.0f + __expf(-bf16_to_f32(((const short*)gate)[(int64_t)b * stride + h])));
+}
+
 template <int GQA, bool FP8>
 __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
     float* __restrict__ partials, bf16_t* __restrict__ out,  // out: written when gridDim.z == 1
@@ -71,12 +85,14 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
     const float* __restrict__ v_scale,
     const int* __restrict__ block_tables,  // [B, max_blocks]
     const int* __restrict__ context_lens,  // [B]
-    float scale, int block_size, int max_blocks, int q_tstride) {
+    const bf16_t* __restrict__ gate, int gate_stride,  // [B, H] logits of the heads' sigmoid gates, or nullptr
+    float scale, int block_size, int max_blocks, int q_tstride, int mask_size) {
   const int g_kv = blockIdx.x, num_kv_heads = gridDim.x;
   const int b = blockIdx.y;
   const int z = blockIdx.z, Z = gridDim.z;
   const int L = context_lens[b];
-  const int tiles = (L + TKEYS - 1) / TKEYS;
+  const int first = first_key(L, mask_size);
+  const int tiles = (L - first + TKEYS - 1) / TKEYS;
   if (z * 4 >= tiles && Z > 1) return;   // no keys here: the merge skips this partial
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 15, grp = lane >> 4;
@@ -102,17 +118,17 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
 #pragma unroll
     for (int j = 0; j < 8; ++j) o[h][j] = 0.0f;
 
-  // cache row of key tile * 32 + (lane & 31); keys behind the context repeat its
+  // cache row of key first + tile * 32 + (lane & 31); keys behind the context repeat its
   // last row
   auto row_of = [&](int tile) {
-    const int kc = min(tile * TKEYS + (lane & (TKEYS - 1)), L - 1);
+    const int kc = min(first + tile * TKEYS + (lane & (TKEYS - 1)), L - 1);
     return (bt[kc / block_size] * num_kv_heads + g_kv) * block_size + kc % block_size;
   };
   const int t0 = z * 4 + wave;
   int row_next = t0 < tiles ? row_of(t0) : 0;
 #pragma unroll 1
   for (int t = t0; t < tiles; t += Z * 4) {
-    const int base = t * TKEYS;
+    const int base = first + t * TKEYS;
     const int rowi = row_next;
     float ks = 1.0f, vs = 1.0f;
     if constexpr (FP8) { ks = k_scale[rowi]; vs = v_scale[rowi]; }
@@ -263,7 +279,7 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
       l += l_lds[w][h] * e;
     }
     if (Z == 1) {
-      const float v = l > 0.0f ? acc / l : 0.0f;
+      const float v = (l > 0.0f ? acc / l : 0.0f) * head_gate(gate, gate_stride, b, g_kv * GQA + h);
       ((short*)out)[((int64_t)b * num_kv_heads * GQA + g_kv * GQA + h) * 128 + d] = f32_to_bf16(v);
     } else {
       base[h * PART_STRIDE + d] = acc;
@@ -293,11 +309,13 @@ extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx) {
 __global__ void __launch_bounds__(256) attn_decode_merge_kernel(
     bf16_t* __restrict__ out,            // [B, H, 128]
     const float* __restrict__ partials,  // [B, KVH, Z, gqa, 130]
-    const int* __restrict__ context_lens, int gqa, int Z) {
+    const int* __restrict__ context_lens, const bf16_t* __restrict__ gate, int gate_stride, int gqa, int Z,
+    int mask_size) {
   const int b = blockIdx.y, h = blockIdx.x, num_q_heads = gridDim.x;
   const int g_kv = h / gqa, g = h % gqa;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tiles = (context_lens[b] + TKEYS - 1) / TKEYS;
+  const int L = context_lens[b];
+  const int tiles = (L - first_key(L, mask_size) + TKEYS - 1) / TKEYS;
   const int n = min(Z, (tiles + 3) / 4);
   const float* base = partials + (((int64_t)b * (num_q_heads / gqa) + g_kv) * Z * gqa + g) * PART_STRIDE;
   const int64_t step = (int64_t)gqa * PART_STRIDE;
@@ -323,7 +341,7 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(
   if (d < 128) {
     const float acc = sh_o[0][d] + sh_o[1][d] + sh_o[2][d] + sh_o[3][d];
     const float lt = sh_l[0] + sh_l[1] + sh_l[2] + sh_l[3];
-    ((short*)out)[((int64_t)b * num_q_heads + h) * 128 + d] = f32_to_bf16(lt > 0.0f ? acc / lt : 0.0f);
+    ((short*)out)[((int64_t)b * num_q_heads + h) * 128 + d] = f32_to_bf16((lt > 0.0f ? acc / lt : 0.0f) * head_gate(gate, gate_stride, b, h));
   }
 }
 
@@ -332,14 +350,14 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(
 extern "C" void launch_attn_decode(
     bf16_t* out, float* partials, const bf16_t* q, const void* k_cache, const void* v_cache,
     const float* k_scale, const float* v_scale, const int* block_tables, const int* context_lens,
-    float scale, int num_q_heads, int num_kv_heads, int block_size, int max_blocks, int splits,
-    int q_tstride, int B, int cache_fp8, hipStream_t stream) {
+    const bf16_t* gate, int gate_stride, float scale, int num_q_heads, int num_kv_heads, int block_size,
+    int max_blocks, int splits, int q_tstride, int B, int cache_fp8, int mask_size, hipStream_t stream) {
   const int gqa = num_q_heads / num_kv_heads;
   const dim3 grid(num_kv_heads, B, splits);
 #define LAUNCH(G, F)                                                                            \
   hipLaunchKernelGGL((attn_decode_tiles<G, F>), grid, dim3(NTHREADS), 0, stream, partials, out, q, \
                      (const char*)k_cache, (const char*)v_cache, k_scale, v_scale, block_tables,   \
-                     context_lens, scale, block_size, max_blocks, q_tstride)
+                     context_lens, gate, gate_stride, scale, block_size, max_blocks, q_tstride, mask_size)
 #define DISPATCH(G) do { if (cache_fp8) LAUNCH(G, true); else LAUNCH(G, false); } while (0)
   switch (gqa) {
     case 1: DISPATCH(1); break;
@@ -351,5 +369,5 @@ extern "C" void launch_attn_decode(
 #undef LAUNCH
   if (splits > 1)
     hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(num_q_heads, B), dim3(256), 0, stream, out,
-                       partials, context_lens, gqa, splits);
+                       partials, context_lens, gate, gate_stride, gqa, splits, mask_size);
 }

@@ -14,7 +14,7 @@ extern "C" __global__ void rope_kernel(bf16_t*, bf16_t*, const int64_t*, const f
 extern "C" __global__ void store_kv_kernel(const bf16_t*, const bf16_t*, bf16_t*, bf16_t*, const int64_t*, int, int, int, int, int);
 extern "C" __global__ void store_kv_fp8_kernel(const bf16_t*, const bf16_t*, unsigned char*, unsigned char*, float*, float*, const int64_t*, int, int, int, int, int);
 extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx);
-extern "C" void launch_attn_decode(bf16_t*, float*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, float, int, int, int, int, int, int, int, int, hipStream_t);
+extern "C" void launch_attn_decode(bf16_t*, float*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, const bf16_t*, int, float, int, int, int, int, int, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, int, int, float, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill_paged(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, const int*, const int*, const int*, int, float, int, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill_plan(int*, const int*, int, int, hipStream_t);
@@ -115,7 +115,7 @@ void store_kv(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache, torch::Te
 void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                        torch::Tensor v_cache, torch::Tensor block_tables,
                        torch::Tensor context_lens, double scale,
-                       torch::Tensor k_scale, torch::Tensor v_scale) {
+                       torch::Tensor k_scale, torch::Tensor v_scale, torch::Tensor gate, int64_t mask_size) {
   CHECK_BF16_CONTIG(out); CHECK_BF16_ROWS(q); CHECK_KV_CACHE(k_cache); CHECK_KV_CACHE(v_cache);
   const int B = q.size(0), H = q.size(1), D = q.size(2);
   const int KVH = k_cache.size(1), BS = k_cache.size(2);
@@ -129,7 +129,11 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
   if (B == 0) return;
   // 16-byte query loads
   if (q.stride(0) % 8 != 0 || reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 != 0) q = q.contiguous();
-  const int splits = attn_decode_splits(B, KVH, max_blocks * BS);
+  if (gate.numel() > 0)
+    TORCH_CHECK(gate.is_cuda() && gate.scalar_type() == at::kBFloat16 && gate.dim() == 2 && gate.size(0) == B &&
+                    gate.size(1) == H && gate.stride(1) == 1, "gate must be a bf16 [B, H] row view");
+  const int64_t longest = mask_size > 0 ? std::min<int64_t>(mask_size, (int64_t)max_blocks * BS) : (int64_t)max_blocks * BS;
+  const int splits = attn_decode_splits(B, KVH, (int)longest);
   auto partials = torch::empty({splits > 1 ? (int64_t)B * KVH * splits * gqa * 130 : 0},
                                torch::dtype(torch::kFloat).device(q.device()));
   const int cache_fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn ? 1 : 0;
@@ -142,8 +146,9 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
       bf(out), partials.data_ptr<float>(), cbf(q), k_cache.data_ptr(), v_cache.data_ptr(),
       cache_fp8 ? k_scale.data_ptr<float>() : nullptr,
       cache_fp8 ? v_scale.data_ptr<float>() : nullptr,
-      block_tables.data_ptr<int>(), context_lens.data_ptr<int>(),
-      (float)scale, H, KVH, BS, max_blocks, splits, (int)q.stride(0), B, cache_fp8, cur_stream());
+      block_tables.data_ptr<int>(), context_lens.data_ptr<int>(), gate.numel() ? cbf(gate) : nullptr,
+      gate.numel() ? (int)gate.stride(0) : 0, (float)scale, H, KVH, BS, max_blocks, splits, (int)q.stride(0), B,
+      cache_fp8, (int)mask_size, cur_stream());
 }
 
 static bool rows_aligned(const torch::Tensor& t) {  // 16-byte row loads
@@ -510,7 +515,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_mul", &silu_mul);
   m.def("rope_inplace", &rope_inplace);
   m.def("store_kv", &store_kv);
-  m.def("attn_decode_paged", &attn_decode_paged);
+  m.def("attn_decode_paged", &attn_decode_paged, py::arg("out"), py::arg("q"), py::arg("k_cache"),
+        py::arg("v_cache"), py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"), py::arg("k_scale"),
+        py::arg("v_scale"), py::arg("gate"), py::arg("mask_size") = 0);
   m.def("attn_prefill", &attn_prefill);
   m.def("attn_prefill_plan", &attn_prefill_plan);
   m.def("attn_prefill_paged", &attn_prefill_paged);

@@ -84,6 +84,9 @@ void seq_launch_head_gate(void*, const void*, int, int, int, int, int, hipStream
 void seq_launch_linear_attn_decay(float*, const void*, const void*, const void*, const float*, float*, float*,
                                   const int*, const int*, const int*, int, int, int, int, int, int, int, int,
                                   int, hipStream_t);
+void seq_launch_linear_attn_chunks(float*, const void*, const void*, const void*, const float*, float*, float*,
+                                   const int*, const int*, const int*, const int*, int, int, int, int, int, int, int,
+                                   int, int, hipStream_t);
 void seq_launch_causal_conv_silu(void*, const void*, const float*, void*, const int*, const int*, const int*,
                                  const int*, const float*, int, int, int, int, int, int, hipStream_t);
 void seq_launch_gated_delta_rule(float*, const void*, const void*, const void*, const void*, const void*,
@@ -514,8 +517,10 @@ static void check_segments(const torch::Tensor& slots, const torch::Tensor& cu, 
   TORCH_CHECK(state.is_cuda() && state.is_contiguous());
 }
 
+// chunks empty: token by token. Else as for retention below
 void linear_attn_decay(torch::Tensor o, torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor decay,
-                       torch::Tensor state, torch::Tensor slots, torch::Tensor cu, torch::Tensor seg_start) {
+                       torch::Tensor state, torch::Tensor slots, torch::Tensor cu, torch::Tensor seg_start,
+                       torch::Tensor chunks, torch::Tensor seg_c0) {
   CHECK_F32C(o); CHECK_ACT(q); CHECK_ROWS3(q); CHECK_ROWS3(k); CHECK_ROWS3(v); CHECK_SAME(k, q); CHECK_SAME(v, q);
   CHECK_F32C(decay); CHECK_F32C(state);
   check_segments(slots, cu, seg_start, state);
@@ -526,6 +531,20 @@ void linear_attn_decay(torch::Tensor o, torch::Tensor q, torch::Tensor k, torch:
   TORCH_CHECK(state.dim() == 4 && state.size(1) == H && state.size(2) == D && state.size(3) == V);
   TORCH_CHECK(decay.numel() == H && o.numel() == (int64_t)T * H * V);
   if (T == 0 || B == 0) return;
+  if (chunks.numel() > 0) {
+    CHECK_I32C(chunks); CHECK_I32C(seg_c0);
+    TORCH_CHECK(chunks.dim() == 2 && chunks.size(1) == 4 && seg_c0.numel() == B + 1);
+    TORCH_CHECK(D <= 128, "the chunk kernels serve key sizes up to 128");
+    const int NC = chunks.size(0);
+    auto U = torch::empty({(int64_t)NC, (int64_t)H, (int64_t)D, (int64_t)V},
+                          torch::dtype(torch::kFloat).device(q.device()));
+    seq_launch_linear_attn_chunks(o.data_ptr<float>(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                  decay.data_ptr<float>(), U.data_ptr<float>(), state.data_ptr<float>(),
+                                  slots.data_ptr<int>(), seg_start.data_ptr<int>(), chunks.data_ptr<int>(),
+                                  seg_c0.data_ptr<int>(), B, NC, H, D, V, (int)q.stride(0), (int)k.stride(0),
+                                  (int)v.stride(0), f32flag(q), cur_stream());
+    return;
+  }
   // silu(q) | silu(k) | silu(v) per (token, head), fp32, from the parallel pre-pass
   auto packed = torch::empty({(int64_t)T, (int64_t)H * (2 * D + V)}, torch::dtype(torch::kFloat).device(q.device()));
   seq_launch_linear_attn_decay(o.data_ptr<float>(), q.data_ptr(), k.data_ptr(), v.data_ptr(),

@@ -17,6 +17,11 @@
 //   retention_chunk_out  o of every (chunk, head), in parallel
 // A step whose segments are all single rows (decode) is one kernel:
 //   retention_step       rotation, update, read-out, RMS norm per head, silu gate
+//
+// Decayed linear attention is the same recurrence on silu(q), silu(k), silu(v) without
+// rotation and scale; its prompt portions take the chunk kernels too (SILU). 7800 rows
+// of 16 heads, 64 x 128: 55 + 28 + 84 us, where the pre-pass and the token-by-token
+// kernel took 38 + 562.
 
 #include "seq_common.h"
 
@@ -80,7 +85,7 @@ __device__ __forceinline__ void ret_load_rotated(const T* __restrict__ row, cons
 // Rotated rows of one head -> LDS [RET_L][DM + 1], zeros past n rows and D
 // columns. The odd row stride puts both a row's and a column's 32 neighbours on
 // 32 banks. pw != nullptr: row r is scaled by pw[n-1-r].
-template <typename T, int DM, int VEC>
+template <typename T, int DM, int VEC, bool SILU>
 __device__ __forceinline__ void ret_stage(float* __restrict__ dst, const T* __restrict__ src, int64_t stride,
                                           const float* __restrict__ cs, int n, int D, int R2, float scale,
                                           const float* pw) {
@@ -91,7 +96,13 @@ __device__ __forceinline__ void ret_stage(float* __restrict__ dst, const T* __re
 #pragma unroll
     for (int e = 0; e < VEC; ++e) x[e] = 0.f;
     if (r < n && c < D) {
-      ret_load_rotated<T, VEC>(src + r * stride, cs + (int64_t)r * 2 * R2, c, R2, x);
+      if constexpr (SILU) {
+        if constexpr (VEC == 8) ld8(src + r * stride + c, x); else x[0] = ldf(src + r * stride + c);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) x[e] = silu_exact(x[e]);
+      } else {
+        ret_load_rotated<T, VEC>(src + r * stride, cs + (int64_t)r * 2 * R2, c, R2, x);
+      }
       const float f = pw != nullptr ? scale * pw[n - 1 - r] : scale;
 #pragma unroll
       for (int e = 0; e < VEC; ++e) x[e] *= f;
@@ -101,9 +112,15 @@ __device__ __forceinline__ void ret_stage(float* __restrict__ dst, const T* __re
   }
 }
 
+template <typename T, bool SILU>
+__device__ __forceinline__ float ret_value(const T* __restrict__ v, uint32_t at) {
+  const float x = ldf(v + at);
+  return SILU ? silu_exact(x) : x;
+}
+
 // chunks [NC, 4] int32: first row, rows, segment, -
 // grid (NC, H): U [NC, H, D, V]
-template <typename T, int DM, int VEC>
+template <typename T, int DM, int VEC, bool SILU>
 __global__ void __launch_bounds__(RET_THREADS, DM > 64 ? 2 : 4) retention_chunk_u_kernel(
     float* __restrict__ U, const T* __restrict__ k, const T* __restrict__ v, const float* __restrict__ cs,
     const float* __restrict__ decay, const int* __restrict__ chunks, float kscale, int H, int D, int V, int R2,
@@ -115,7 +132,7 @@ __global__ void __launch_bounds__(RET_THREADS, DM > 64 ? 2 : 4) retention_chunk_
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, half = lane >> 5, lr = lane & 31;
   ret_powers(pw, decay[h]);
   __syncthreads();
-  ret_stage<T, DM, VEC>(ks, k + (int64_t)row0 * k_stride + (int64_t)h * D, k_stride, cs + (int64_t)row0 * 2 * R2, n,
+  ret_stage<T, DM, VEC, SILU>(ks, k + (int64_t)row0 * k_stride + (int64_t)h * D, k_stride, cs + (int64_t)row0 * 2 * R2, n,
                         D, R2, kscale, pw);
   __syncthreads();
   constexpr int DT = DM / 32;
@@ -132,7 +149,7 @@ __global__ void __launch_bounds__(RET_THREADS, DM > 64 ? 2 : 4) retention_chunk_
     for (int t = 0; t < n; t += 2 * RET_KU, kp += 2 * RET_KU * (DM + 1)) {
       float b[RET_KU];             // rows past n: the keys there are zero
 #pragma unroll
-      for (int u = 0; u < RET_KU; ++u) b[u] = ldf(vp + (uint32_t)(min(t + 2 * u + half, n - 1) * v_stride + jc));
+      for (int u = 0; u < RET_KU; ++u) b[u] = ret_value<T, SILU>(vp, (uint32_t)(min(t + 2 * u + half, n - 1) * v_stride + jc));
 #pragma unroll
       for (int u = 0; u < RET_KU; ++u)
 #pragma unroll
@@ -196,7 +213,7 @@ __global__ void __launch_bounds__(RET_THREADS) retention_scan_kernel(
 }
 
 // grid (NC, H): o [T, H, V]. S0: the state before each chunk [NC, H, D, V]
-template <typename T, int DM, int VEC>
+template <typename T, int DM, int VEC, bool SILU>
 __global__ void __launch_bounds__(RET_THREADS, DM > 64 ? 2 : 3) retention_chunk_out_kernel(
     float* __restrict__ o, const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const float* __restrict__ S0, const float* __restrict__ cs, const float* __restrict__ decay,
@@ -212,8 +229,8 @@ __global__ void __launch_bounds__(RET_THREADS, DM > 64 ? 2 : 3) retention_chunk_
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, half = lane >> 5, lr = lane & 31;
   const float* csr = cs + (int64_t)row0 * 2 * R2;
   ret_powers(pw, decay[h]);
-  ret_stage<T, DM, VEC>(qs, q + (int64_t)row0 * q_stride + (int64_t)h * D, q_stride, csr, n, D, R2, 1.0f, nullptr);
-  ret_stage<T, DM, VEC>(ks, k + (int64_t)row0 * k_stride + (int64_t)h * D, k_stride, csr, n, D, R2, kscale, nullptr);
+  ret_stage<T, DM, VEC, SILU>(qs, q + (int64_t)row0 * q_stride + (int64_t)h * D, q_stride, csr, n, D, R2, 1.0f, nullptr);
+  ret_stage<T, DM, VEC, SILU>(ks, k + (int64_t)row0 * k_stride + (int64_t)h * D, k_stride, csr, n, D, R2, kscale, nullptr);
   __syncthreads();
   // scores q_i . k_j, one 32 x 32 tile per wave (the tile above the diagonal is never read)
   const int it = wave >> 1, jt = wave & 1;
@@ -269,7 +286,7 @@ __global__ void __launch_bounds__(RET_THREADS, DM > 64 ? 2 : 3) retention_chunk_
     for (int t = 0; t < n; t += 2 * RET_KU, pp += 2 * RET_KU) {
       float b[RET_KU];
 #pragma unroll
-      for (int u = 0; u < RET_KU; ++u) b[u] = ldf(vp + (uint32_t)(min(t + 2 * u + half, n - 1) * v_stride + jc));
+      for (int u = 0; u < RET_KU; ++u) b[u] = ret_value<T, SILU>(vp, (uint32_t)(min(t + 2 * u + half, n - 1) * v_stride + jc));
       if (t < 32) {                            // tokens 32.. lie after rows 0..31
 #pragma unroll
         for (int u = 0; u < RET_KU; ++u) a0 = __builtin_amdgcn_mfma_f32_32x32x2f32(pp[2 * u], b[u], a0, 0, 0, 0);
@@ -379,6 +396,24 @@ __global__ void __launch_bounds__(RET_THREADS) retention_step_kernel(
   else if (D <= 64) { constexpr int DM = 64; __VA_ARGS__ }          \
   else { constexpr int DM = 128; __VA_ARGS__ }
 
+template <typename T, int DM, int VEC, bool SILU>
+static void ret_chunks(float* o, const T* q, const T* k, const T* v, const float* decay, const float* cs, float* U,
+                       float* state, const int* slots, const int* seg_start, const int* chunks, const int* seg_c0,
+                       float kscale, int B, int NC, int H, int D, int V, int R2, int q_stride, int k_stride,
+                       int v_stride, hipStream_t st) {
+  hipLaunchKernelGGL((retention_chunk_u_kernel<T, DM, VEC, SILU>), dim3(NC, H), dim3(RET_THREADS), 0, st, U, k, v, cs,
+                     decay, chunks, kscale, H, D, V, R2, k_stride, v_stride);
+  const int64_t DV = (int64_t)D * V;
+  if (DV % 4 == 0 && aligned16(U) && aligned16(state))
+    hipLaunchKernelGGL(retention_scan_kernel<4>, dim3(B, H, (unsigned)((DV / 4 + RET_THREADS - 1) / RET_THREADS)),
+                       dim3(RET_THREADS), 0, st, U, state, decay, chunks, seg_c0, slots, seg_start, H, DV);
+  else
+    hipLaunchKernelGGL(retention_scan_kernel<1>, dim3(B, H, (unsigned)((DV + RET_THREADS - 1) / RET_THREADS)),
+                       dim3(RET_THREADS), 0, st, U, state, decay, chunks, seg_c0, slots, seg_start, H, DV);
+  hipLaunchKernelGGL((retention_chunk_out_kernel<T, DM, VEC, SILU>), dim3(NC, H), dim3(RET_THREADS), 0, st, o, q, k, v,
+                     U, cs, decay, chunks, kscale, H, D, V, R2, q_stride, k_stride, v_stride);
+}
+
 // cs [T, 2 R2], U [NC, H, D, V]: fp32 scratch; chunks [NC, 4], seg_c0 [B + 1]: the step's chunks. D <= 128
 extern "C" void seq_launch_retention_chunks(float* o, const void* q, const void* k, const void* v, const float* decay,
                                             const int64_t* positions, const float* inv_freq, float* cs, float* U,
@@ -393,26 +428,22 @@ extern "C" void seq_launch_retention_chunks(float* o, const void* q, const void*
   const bool v8 = D % 8 == 0 && R2 % 8 == 0 && q_stride % 8 == 0 && k_stride % 8 == 0 && aligned16(q) &&
                   aligned16(k) && aligned16(cs);
   DISPATCH_T(is_f32, DISPATCH_D(D,
-             if (v8) hipLaunchKernelGGL((retention_chunk_u_kernel<T, DM, 8>), dim3(NC, H), dim3(RET_THREADS), 0, st, U,
-                                        (const T*)k, (const T*)v, cs, decay, chunks, kscale, H, D, V, R2, k_stride,
-                                        v_stride);
-             else hipLaunchKernelGGL((retention_chunk_u_kernel<T, DM, 1>), dim3(NC, H), dim3(RET_THREADS), 0, st, U,
-                                     (const T*)k, (const T*)v, cs, decay, chunks, kscale, H, D, V, R2, k_stride,
-                                     v_stride);))
-  const int64_t DV = (int64_t)D * V;
-  if (DV % 4 == 0 && aligned16(U) && aligned16(state))
-    hipLaunchKernelGGL(retention_scan_kernel<4>, dim3(B, H, (unsigned)((DV / 4 + RET_THREADS - 1) / RET_THREADS)),
-                       dim3(RET_THREADS), 0, st, U, state, decay, chunks, seg_c0, slots, seg_start, H, DV);
-  else
-    hipLaunchKernelGGL(retention_scan_kernel<1>, dim3(B, H, (unsigned)((DV + RET_THREADS - 1) / RET_THREADS)),
-                       dim3(RET_THREADS), 0, st, U, state, decay, chunks, seg_c0, slots, seg_start, H, DV);
+             auto run = v8 ? ret_chunks<T, DM, 8, false> : ret_chunks<T, DM, 1, false>;
+             run(o, (const T*)q, (const T*)k, (const T*)v, decay, cs, U, state, slots, seg_start, chunks, seg_c0,
+                 kscale, B, NC, H, D, V, R2, q_stride, k_stride, v_stride, st);))
+}
+
+// decayed linear attention of prompt portions; U [NC, H, D, V] fp32 scratch. D <= 128
+extern "C" void seq_launch_linear_attn_chunks(float* o, const void* q, const void* k, const void* v,
+                                              const float* decay, float* U, float* state, const int* slots,
+                                              const int* seg_start, const int* chunks, const int* seg_c0, int B, int NC,
+                                              int H, int D, int V, int q_stride, int k_stride, int v_stride, int is_f32,
+                                              hipStream_t st) {
+  const bool v8 = D % 8 == 0 && q_stride % 8 == 0 && k_stride % 8 == 0 && aligned16(q) && aligned16(k);
   DISPATCH_T(is_f32, DISPATCH_D(D,
-             if (v8) hipLaunchKernelGGL((retention_chunk_out_kernel<T, DM, 8>), dim3(NC, H), dim3(RET_THREADS), 0, st,
-                                        o, (const T*)q, (const T*)k, (const T*)v, U, cs, decay, chunks, kscale, H, D,
-                                        V, R2, q_stride, k_stride, v_stride);
-             else hipLaunchKernelGGL((retention_chunk_out_kernel<T, DM, 1>), dim3(NC, H), dim3(RET_THREADS), 0, st, o,
-                                     (const T*)q, (const T*)k, (const T*)v, U, cs, decay, chunks, kscale, H, D, V, R2,
-                                     q_stride, k_stride, v_stride);))
+             auto run = v8 ? ret_chunks<T, DM, 8, true> : ret_chunks<T, DM, 1, true>;
+             run(o, (const T*)q, (const T*)k, (const T*)v, decay, nullptr, U, state, slots, seg_start, chunks, seg_c0,
+                 1.0f, B, NC, H, D, V, 0, q_stride, k_stride, v_stride, st);))
 }
 
 // V <= RET_THREADS, or V % 4 == 0 and V <= 4 RET_THREADS; D <= 1024

@@ -189,3 +189,62 @@ def test_decode_rows_match_general_path(preset, rows):
     # bf16 activations through two layers; a routed row may change its experts
     off = (got - want).norm(dim=-1) / want.norm(dim=-1)
     assert float(off.median()) < 0.02 and (preset == "mid-mixtral" or float(off.max()) < 0.05)
+
+
+@pytest.mark.parametrize("gqa,KVH,BS", [(4, 4, 16), (1, 2, 8), (8, 1, 16)])
+@pytest.mark.parametrize("mask", [24, 256, 1024])
+def test_blocklocal_rows(gqa, KVH, BS, mask):
+    ctx = [1, 23, 24, 25, 48, 256, 257, 1000, 1024, 1025]
+    q, k, v, _, _, bt, n = paged_case(len(ctx), KVH, gqa, BS, ctx, False, seed=mask)
+    gate = torch.randn(len(ctx), KVH * gqa + 8, generator=torch.Generator().manual_seed(1)).bfloat16().to(DEV)[:, :KVH * gqa]
+    scale = D ** -0.5
+    out = ops.attn_blocklocal_rows(q.to(DEV), k.to(DEV), v.to(DEV), bt.to(DEV), n.to(DEV), scale, mask, gate)
+    for b, L in enumerate(ctx):
+        lo = (L - 1) // mask * mask
+        at = torch.arange(lo, L)
+        blk = bt[b].long()[at // BS]
+        kk, vv = k[blk, :, at % BS].double(), v[blk, :, at % BS].double()
+        for h in range(KVH * gqa):
+            ref = torch.softmax(kk[:, h // gqa] @ q[b, h].double() * scale, 0) @ vv[:, h // gqa]
+            ref = ref * torch.sigmoid(gate[b, h].double().cpu())
+            assert ((out[b, h].double().cpu() - ref).abs() <= 2 ** -8 * ref.abs() + 2e-5).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,Dk,V", [(2, 64, 128), (3, 128, 96), (2, 24, 40), (1, 5, 7)])
+def test_linear_attention_chunks(H, Dk, V, dtype):
+    """Chunk-parallel decayed linear attention against the recurrence in float64; segments fresh and continued, with
+    lengths around the chunk size and single rows among them."""
+    segs = [(0, 64), (5, 1), (0, 200), (9, 65), (3, 17)]
+    T = sum(n for _, n in segs)
+    g = torch.Generator().manual_seed(H + Dk)
+    wide = torch.randn(T, H * (2 * Dk + V) + 8, generator=g).to(dtype)
+    q, k, v = (wide[:, a:b].unflatten(1, (H, -1)) for a, b in
+               ((0, H * Dk), (H * Dk, 2 * H * Dk), (2 * H * Dk, H * (2 * Dk + V))))
+    decay = torch.exp(-1.0 / 2.0 ** (1 + 3 * torch.arange(H))).float()
+    state = torch.randn(7, H, Dk, V, generator=g)
+    slots = torch.tensor([4, 0, 6, 2, 3], dtype=torch.int32)
+    cu = torch.tensor([0] + [n for _, n in segs]).cumsum(0).to(torch.int32)
+    start = torch.tensor([s for s, _ in segs], dtype=torch.int32)
+    dev = wide.to(DEV)
+    qd, kd, vd = (dev[:, a:b].unflatten(1, (H, -1)) for a, b in
+                  ((0, H * Dk), (H * Dk, 2 * H * Dk), (2 * H * Dk, H * (2 * Dk + V))))
+    got_state = state.to(DEV)
+    o = ops.linear_attn_decay(qd, kd, vd, decay.to(DEV), got_state, slots.to(DEV), cu.to(DEV), start.to(DEV),
+                              ops.retention_chunks(segs, DEV))
+    silu = torch.nn.functional.silu
+    r = 0
+    for b, (s, n) in enumerate(segs):
+        S = torch.zeros(H, Dk, V, dtype=torch.float64) if s == 0 else state[slots[b]].double()
+        size = S.abs()
+        for t in range(r, r + n):
+            kk, vv, qq = silu(k[t].double()), silu(v[t].double()), silu(q[t].double())
+            S = S * decay.double().view(H, 1, 1) + kk.unsqueeze(-1) * vv.unsqueeze(-2)
+            size = size * decay.double().view(H, 1, 1) + (kk.unsqueeze(-1) * vv.unsqueeze(-2)).abs()
+            ref = (qq.unsqueeze(-2) @ S).squeeze(-2)
+            bound = (qq.abs().unsqueeze(-2) @ size).squeeze(-2)
+            # fp32 sums of at most Dk + 64 products of the terms' size, a few roundings each (fast silu included)
+            assert ((o[t].double().cpu() - ref).abs() <= (Dk + 64) * 2 ** -23 * bound + 1e-6).all()
+        assert ((got_state[slots[b]].double().cpu() - S).abs() <= 300 * 2 ** -23 * size + 1e-6).all()
+        r += n
+    assert torch.equal(got_state[1].cpu(), state[1])
