@@ -17,6 +17,7 @@ import time
 from dataclasses import dataclass, field
 from typing import Any, List, Optional, Tuple
 
+import numpy as np
 import torch
 
 from ..models.llama import ForwardBatch
@@ -506,30 +507,26 @@ class LLMEngine:
         hidden = self.model.forward_hidden(torch.tensor(all_ids, dtype=torch.long, device=dev), batch)
         return self.model.compute_logits(hidden[torch.tensor(last_rows, device=dev)])
 
-    def _rows_batch(self, segs: List[Tuple[SequenceKV, int, int]], slots: List[int]) -> ForwardBatch:
+    def _rows_batch(self, segs: List[Tuple[SequenceKV, int, int]], slots: List[int], extra=()):
         """Decode-mode ForwardBatch of an attention-only model: one row per new
         token of segs (sequence, first position, row count), packed in that
-        order; slots: the flat cache slot of every row."""
-        dev = self.device
-        pos = [p for _, start, n in segs for p in range(start, start + n)]
-        width = max(len(seq.blocks) for seq, _, _ in segs)
-        bt = torch.zeros((len(segs), width), dtype=torch.int32)
-        for b, (seq, _, _) in enumerate(segs):
-            bt[b, : len(seq.blocks)] = torch.tensor(seq.blocks, dtype=torch.int32)
-        bt = bt.to(dev)
-        positions = torch.tensor(pos, dtype=torch.long, device=dev)
-        row_seg = torch.tensor([b for b, (_, _, n) in enumerate(segs) for _ in range(n)], dtype=torch.long, device=dev)
-        return ForwardBatch(
+        order; slots: the flat cache slot of every row; extra: as for
+        _segment_batch."""
+        pos, row_seg, tables = self._host_rows(segs)
+        (positions, slot_map, rows, *rest), (bt, ctx, first) = self._upload(
+            [pos, slots, row_seg, *extra], [tables, pos + 1, [start for _, start, _ in segs]])
+        batch = ForwardBatch(
             mode="decode",
             positions=positions,
-            slot_mapping=torch.tensor(slots, dtype=torch.long, device=dev),
+            slot_mapping=slot_map,
             kv_caches=self.kv.layer_caches(),
-            block_tables=bt[row_seg],
-            context_lens=(positions + 1).to(torch.int32),
-            seg_start=torch.tensor([start for _, start, _ in segs], dtype=torch.int32, device=dev),
+            block_tables=bt[rows],
+            context_lens=ctx,
+            seg_start=first,
             host_segs=[(start, n) for _, start, n in segs],
             seg_tables=bt,
         )
+        return (batch, *rest) if extra else batch
 
     def _alloc_with_prefix(self, ids: List[int], prefix_blocks: List[int]) -> SequenceKV:
         """Sequence backed by cached prefix blocks (increfed) + freshly
@@ -617,39 +614,56 @@ class LLMEngine:
         return None
 
     # --- segment steps -------------------------------------------------------
-    def _segment_batch(self, segs: List[Tuple[SequenceKV, int, int]], slots: List[int]) -> ForwardBatch:
+    def _segment_batch(self, segs: List[Tuple[SequenceKV, int, int]], slots: List[int], extra=()):
         """ForwardBatch in segment form. segs: (sequence, first position,
         row count) per segment, rows packed in that order; slots: the flat
         cache slot of every row. The sequences' block lists must already
-        cover the new rows."""
-        dev = self.device
-        pos: List[int] = []
-        tseg: List[int] = []
-        cu = [0]
-        for b, (_seq, start, n) in enumerate(segs):
-            pos.extend(range(start, start + n))
-            tseg.extend([b] * n)
-            cu.append(cu[-1] + n)
-        width = max(1, max(len(seq.blocks) for seq, _, _ in segs))
-        bt = torch.zeros((len(segs), width), dtype=torch.int32)
-        for b, (seq, _, _) in enumerate(segs):
-            if seq.blocks:
-                bt[b, : len(seq.blocks)] = torch.tensor(seq.blocks, dtype=torch.int32)
-        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
-        return ForwardBatch(
+        cover the new rows. extra: further int64 lists to bring along; with
+        them (batch, *their tensors) is returned."""
+        pos, token_seg, tables = self._host_rows(segs)
+        counts = [n for _, _, n in segs]
+        (positions, slot_map, *rest), (cu, bt, ctx, first, state, tseg) = self._upload(
+            [pos, slots, *extra],
+            [np.cumsum([0] + counts), tables, [start + n for _, start, n in segs], [start for _, start, _ in segs],
+             [seq.state_slot for seq, _, _ in segs], token_seg])
+        batch = ForwardBatch(
             mode="segments",
-            positions=torch.tensor(pos, dtype=torch.long, device=dev),
-            slot_mapping=torch.tensor(slots, dtype=torch.long, device=dev),
+            positions=positions,
+            slot_mapping=slot_map,
             kv_caches=self.kv.layer_caches(),
-            cu_seqlens=i32(cu),
-            block_tables=bt.to(dev),
-            context_lens=i32([start + n for _, start, n in segs]),
-            seg_start=i32([start for _, start, _ in segs]),
-            state_slots=i32([seq.state_slot for seq, _, _ in segs]),
-            token_seg=i32(tseg),
+            cu_seqlens=cu,
+            block_tables=bt,
+            context_lens=ctx,
+            seg_start=first,
+            state_slots=state,
+            token_seg=tseg,
             host_segs=[(start, n) for _, start, n in segs],
             plans={},
         )
+        return (batch, *rest) if extra else batch
+
+    def _host_rows(self, segs: List[Tuple[SequenceKV, int, int]]):
+        """(position, segment index) of every row of segs, and the segments' block tables padded with zeros."""
+        counts = np.array([n for _, _, n in segs], dtype=np.int64)
+        starts = np.array([start for _, start, _ in segs], dtype=np.int64)
+        ends = np.cumsum(counts)
+        seg = np.repeat(np.arange(len(segs)), counts)
+        pos = np.arange(int(ends[-1]) if len(segs) else 0) - (ends - counts)[seg] + starts[seg]
+        tables = np.zeros((len(segs), max(1, max(len(seq.blocks) for seq, _, _ in segs))), dtype=np.int32)
+        for b, (seq, _, _) in enumerate(segs):
+            tables[b, : len(seq.blocks)] = seq.blocks
+        return pos, seg, tables
+
+    def _upload(self, longs, ints):
+        """Host rows as int64 / int32 device tensors, one copy for each type
+        (a copy of a few hundred bytes costs the host as much as a launch)."""
+        out = []
+        for rows, kind in ((longs, np.int64), (ints, np.int32)):
+            rows = [np.asarray(r, dtype=kind) for r in rows]
+            flat = torch.from_numpy(np.concatenate([r.reshape(-1) for r in rows])).to(self.device)
+            parts = flat.split([r.size for r in rows])
+            out.append([p if r.ndim == 1 else p.view(r.shape) for p, r in zip(parts, rows)])
+        return out
 
     def open_sequence(self) -> SequenceKV:
         """An empty sequence to be fed step by step through step_segments()."""
@@ -666,7 +680,6 @@ class LLMEngine:
         needed. Returns fp32 logits [n_wanted, V] in entry order (None when
         nothing is wanted). The step function under generation's prefill
         slices and decode steps, exposed for replaying recorded schedules."""
-        dev = self.device
         entries = [e for e in entries if len(e[1]) > 0]
         if not entries:
             return None
@@ -680,17 +693,14 @@ class LLMEngine:
             want_rows.extend(len(ids) + w for w in want)
             ids.extend(toks)
             segs.append((seq, start, len(toks)))
-        input_ids = torch.tensor(ids, dtype=torch.long, device=dev)
-        if self.stateful:
-            batch = self._segment_batch(segs, slots)
-        else:
-            # attention-only models: one decode-mode row per token, each row
-            # attending to its own sequence's cache up to its position
-            batch = self._rows_batch(segs, slots)
+        # attention-only models: one decode-mode row per token, each row
+        # attending to its own sequence's cache up to its position
+        make = self._segment_batch if self.stateful else self._rows_batch
+        batch, input_ids, wanted = make(segs, slots, (ids, want_rows))
         hidden = self.model.forward_hidden(input_ids, batch)
         if not want_rows:
             return None
-        return self.model.compute_logits(hidden[torch.tensor(want_rows, dtype=torch.long, device=dev)])
+        return self.model.compute_logits(hidden if want_rows == list(range(len(ids))) else hidden[wanted])
 
     def finish_stream(self, s: _Stream) -> StreamOutput:
         """Phase 3: detokenize (unless a stop-string already trimmed the
