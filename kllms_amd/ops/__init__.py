@@ -102,6 +102,22 @@ def store_kv(
     torch_ref.store_kv(k, v, k_cache, v_cache, slot_mapping, k_scale, v_scale)
 
 
+def rope_store(q, k, v, positions, cos_sin, k_cache, v_cache, slot_mapping, k_scale=None, v_scale=None) -> None:
+    """rope_inplace(q, k) and store_kv(k, v): one launch for aligned rows of head size 128, else the two."""
+    if (q.is_cuda and not _force_torch() and q.dtype == k.dtype == v.dtype == torch.bfloat16
+            and q.shape[2] == 128 and k.stride(0) == v.stride(0)
+            and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 and t.stride(2) == 1 and t.stride(1) == 128
+                    for t in (q, k, v))
+            and all(t.dtype == torch.long and t.is_contiguous() for t in (positions, slot_mapping))
+            and cos_sin.is_contiguous() and k_cache.dtype == v_cache.dtype):
+        none = _none(k, torch.float32)
+        _hip_or_raise().rope_store(q, k, v, positions, cos_sin, k_cache, v_cache, slot_mapping,
+                                   k_scale if k_scale is not None else none, v_scale if v_scale is not None else none)
+        return
+    rope_inplace(q, k, positions, cos_sin)
+    store_kv(k, v, k_cache, v_cache, slot_mapping, k_scale, v_scale)
+
+
 def prefill_plan(cu_seqlens: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
     """Row groups of packed sequences for attn_prefill_varlen, made on the GPU (None on the CPU): one launch serves
     every layer of a forward pass."""

@@ -112,6 +112,40 @@ void store_kv(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache, torch::Te
   }
 }
 
+extern "C" void launch_rope_store(bf16_t* q, bf16_t* k, const bf16_t* v, const int64_t* positions,
+                                  const float* cos_sin, void* k_cache, void* v_cache, float* k_scale, float* v_scale,
+                                  const int64_t* slots, int T, int H, int G, int q_stride, int kv_stride,
+                                  int block_size, int fp8, hipStream_t stream);
+
+// rope_inplace and store_kv of rows of head size 128 in one launch; views of 16-byte aligned rows
+void rope_store(torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor positions, torch::Tensor cos_sin,
+                torch::Tensor k_cache, torch::Tensor v_cache, torch::Tensor slots, torch::Tensor k_scale,
+                torch::Tensor v_scale) {
+  CHECK_BF16_ROWS(q); CHECK_BF16_ROWS(k); CHECK_BF16_ROWS(v); CHECK_KV_CACHE(k_cache); CHECK_KV_CACHE(v_cache);
+  const int T = q.size(0), H = q.size(1), G = k.size(1), BS = k_cache.size(2);
+  TORCH_CHECK(q.size(2) == 128 && k.size(2) == 128 && v.sizes() == k.sizes() && k.size(0) == T &&
+                  k.stride(0) == v.stride(0) && k_cache.size(1) == G && k_cache.size(3) == 128 &&
+                  v_cache.sizes() == k_cache.sizes() && v_cache.scalar_type() == k_cache.scalar_type(),
+              "rope_store: sizes");
+  for (const auto& t : {q, k, v})
+    TORCH_CHECK(t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "rope_store: alignment");
+  TORCH_CHECK(positions.scalar_type() == at::kLong && positions.is_contiguous() && positions.numel() == T &&
+                  slots.scalar_type() == at::kLong && slots.is_contiguous() && slots.numel() == T &&
+                  cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() && cos_sin.size(-1) == 128,
+              "rope_store: positions, slots or angles");
+  const int fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn ? 1 : 0;
+  if (fp8)
+    TORCH_CHECK(k_scale.numel() == k_cache.size(0) * G * BS && k_scale.is_contiguous() &&
+                    k_scale.scalar_type() == at::kFloat && v_scale.numel() == k_scale.numel() &&
+                    v_scale.is_contiguous() && v_scale.scalar_type() == at::kFloat,
+                "fp8 rope_store requires [NB, KVH, BS] fp32 k_scale/v_scale");
+  if (T == 0) return;
+  launch_rope_store(bf(q), bf(k), cbf(v), positions.data_ptr<int64_t>(), cos_sin.data_ptr<float>(), k_cache.data_ptr(),
+                    v_cache.data_ptr(), fp8 ? k_scale.data_ptr<float>() : nullptr,
+                    fp8 ? v_scale.data_ptr<float>() : nullptr, slots.data_ptr<int64_t>(), T, H, G, (int)q.stride(0),
+                    (int)k.stride(0), BS, fp8, cur_stream());
+}
+
 void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                        torch::Tensor v_cache, torch::Tensor block_tables,
                        torch::Tensor context_lens, double scale,
@@ -515,6 +549,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_mul", &silu_mul);
   m.def("rope_inplace", &rope_inplace);
   m.def("store_kv", &store_kv);
+  m.def("rope_store", &rope_store);
   m.def("attn_decode_paged", &attn_decode_paged, py::arg("out"), py::arg("q"), py::arg("k_cache"),
         py::arg("v_cache"), py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"), py::arg("k_scale"),
         py::arg("v_scale"), py::arg("gate"), py::arg("mask_size") = 0);

@@ -113,3 +113,38 @@ def test_step_segments_matches_row_by_row(rows):
     toks = [torch.randint(0, 2000, (n,), generator=g).tolist() for n in rows]
     a, b = step(False), step(True)
     assert float(((a - b).norm(dim=-1) / b.norm(dim=-1)).max()) < 0.03     # bf16 through two layers
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("T,H,G,BS", [(1, 4, 2, 16), (33, 7, 1, 5), (257, 32, 8, 16)])
+def test_rope_store_matches_the_two_kernels(T, H, G, BS, fp8):
+    g = torch.Generator().manual_seed(T)
+    qkv = torch.randn(T, H + 2 * G, D, generator=g).bfloat16().to(DEV)
+    NB = (T + BS - 1) // BS + 1
+    slots = torch.randperm(NB * BS, generator=g)[:T].to(DEV)
+    pos = torch.randint(0, 300, (T,), generator=g).to(DEV)
+    ang = torch.arange(300).unsqueeze(1) * 10000.0 ** (-torch.arange(0, D, 2) / D)
+    cs = torch.cat([ang.cos(), ang.sin()], 1).to(DEV)
+    kind = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    got = []
+    for fused in (True, False):
+        rows = qkv.clone()
+        q, k, v = rows.split([H, G, G], 1)
+        kc, vc = (torch.zeros(NB, G, BS, D, device=DEV, dtype=kind) for _ in range(2))
+        ks, vs = (torch.ones(NB, G, BS, device=DEV) for _ in range(2)) if fp8 else (None, None)
+        if fused:
+            ops.rope_store(q, k, v, pos, cs, kc, vc, slots, ks, vs)
+        else:
+            ops.rope_inplace(q, k, pos, cs)
+            ops.store_kv(k, v, kc, vc, slots, ks, vs)
+        got.append((rows, kc.view(torch.uint8), vc.view(torch.uint8), ks, vs))
+    a, b = got
+    # the same products, which one of the two may contract into a fused multiply-add: a last place of bf16 in the rows
+    # (2^-8 of the larger term), the same bytes of V
+    big = torch.maximum(qkv.float().abs(), qkv.float().abs().roll(64, -1))
+    assert ((a[0].float() - b[0].float()).abs() <= 2 ** -7 * big).all()
+    assert float((a[0] != b[0]).float().mean()) < 0.01
+    assert torch.equal(a[2], b[2])
+    assert float((a[1] != b[1]).float().mean()) < 0.02
+    if fp8:
+        assert torch.equal(a[4], b[4]) and torch.allclose(a[3], b[3], rtol=2 ** -7)
