@@ -262,7 +262,7 @@ class LlamaForCausalLM(nn.Module):
 
     # --- forward ------------------------------------------------------------
     # the fused [gate; up] product of more rows than this is the library's: at 128 rows of 28672 x 4096 it takes 57 us
-    # and the few-row kernel 74 (its x fragments saturate LDS), at 64 rows 54 + 5 for the activation against 60
+    # and 5 for the activation, the few-row kernel 68 (its reads of x grow with the rows), at 64 rows 54 + 5 against 57
     SILU_ROWS_MAX = 64
 
     def _takes_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> bool:

@@ -1,11 +1,11 @@
 // Products of a few rows with a weight matrix, y[M, N] = x[M, K] W[N, K]^T, M <= 128
 // (the projections of a decode step), for gfx950.
 //
-// The weights' stream is the bound: 64 weight rows per 256-thread workgroup, 16 per
-// wave, each read once and straight from memory to matrix fragments (16x16x32) - a
+// The weights' stream is the bound: 64 weight rows per 256-thread workgroup (128 per 512
+// for many rows of x), 16 per wave, each read once and straight from memory to matrix fragments (16x16x32) - a
 // lane group takes 32 contiguous bytes of its row in two loads, so every 128-byte line
 // is used whole, and x is read in the same order of k. x goes through LDS in 128-deep
-// chunks, double-buffered, shared by the four waves; its 16-byte units are XORed with
+// chunks, double-buffered, shared by the waves; its 16-byte units are XORed with
 // the row, which keeps the 16-row fragment reads free of bank conflicts. The weights of
 // the next two chunks are in flight while one is multiplied (8 KB a wave).
 //
@@ -15,10 +15,10 @@
 //   F32   fp32, S = 1 (logits)         SILU  silu(gate) * up of a fused [gate; up] matrix
 //
 // Measured with the weights out of cache (the library's kernel in brackets), us:
-//   4096 x 4096   5 rows 9 (15.6), 128 rows 16.3 (24.8)
-//   4096 x 14336  5 rows 23.4 (26.7: 5 TB/s either way), 64 rows 30 (42), 128 rows 39.5 (75.6)
+//   4096 x 4096   5 rows 9 (15.6), 128 rows 15.6 (24.5)
+//   4096 x 14336  5 rows 23.4 (26.7: 5 TB/s either way), 64 rows 30 (42), 128 rows 36 (75.5)
 //   2048 x 8192   1 row 9.2 (12.8), 64 rows 11.9 (22.6)
-//   28672 x 4096  with silu 50 (64 + 5) for 5 rows, 60 (54 + 5) for 64, 74 (57 + 5) for 128
+//   28672 x 4096  with silu 50 (64 + 5) for 5 rows, 57 (54 + 5) for 64, 68 (57 + 5) for 128
 // Above 64 rows every wave reads all of x from LDS for 16 weight rows, and LDS is the
 // bound where K is not split far.
 
@@ -37,8 +37,8 @@ union LrFrag {
   bf16x8_mfma m;
 };
 
-template <int MT, int FORM>
-__global__ __launch_bounds__(256) void linear_rows_kernel(
+template <int MT, int FORM, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
     void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
     const bf16_t* __restrict__ bias, int M, int N, int K, int x_stride, int chunks_per_split) {
   __shared__ __attribute__((aligned(16))) u32x4 xs[2][MT * 256];
@@ -48,9 +48,11 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(
   const int nchunks = K / LR_KC;
   const int c_begin = blockIdx.y * chunks_per_split;
   const int c_end = min(nchunks, c_begin + chunks_per_split);
-  // weight row of this wave's tile; SILU: waves 0, 1 hold gate rows, 2, 3 the up rows of the same columns
-  const int n0 = FORM == LR_SILU ? (wave >> 1) * (N / 2) + blockIdx.x * 32 + (wave & 1) * 16
-                                 : blockIdx.x * 64 + wave * 16;
+  // weight row of this wave's tile; SILU: the first half of the waves hold gate rows, the others the up rows of
+  // the same columns
+  constexpr int HW = WAVES / 2;
+  const int n0 = FORM == LR_SILU ? (wave / HW) * (N / 2) + blockIdx.x * (16 * HW) + (wave % HW) * 16
+                                 : blockIdx.x * (16 * WAVES) + wave * 16;
   const char* wrow = (const char*)(w + (int64_t)min(n0 + col, N - 1) * K) + grp * 32;
 
   f32x4 acc[MT];
@@ -58,21 +60,23 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(
   for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   u32x4 wr[2][LR_STEPS];
-  u32x4 xr[MT];
+  constexpr int XP = MT * 4 / WAVES;      // passes of a chunk's x over the threads
+  static_assert(XP >= 1, "as many 16-byte units as threads");
+  u32x4 xr[XP];
   auto load_w = [&](int c, int slot, int st) {
     wr[slot][st] = *reinterpret_cast<const u32x4*>(wrow + (int64_t)c * (LR_KC * 2) + (st >> 1) * 128 + (st & 1) * 16);
   };
-  // unit tid of each 16-row group: row tid / 16, 16-byte unit tid % 16
+  // row tid / 16 of each pass, 16-byte unit tid % 16
   const int xrow = tid >> 4, xunit = tid & 15;
   auto load_x = [&](int c) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-      xr[i] = *reinterpret_cast<const u32x4*>((const char*)(x + (int64_t)min(i * 16 + xrow, M - 1) * x_stride) +
+    for (int i = 0; i < XP; ++i)
+      xr[i] = *reinterpret_cast<const u32x4*>((const char*)(x + (int64_t)min(i * 4 * WAVES + xrow, M - 1) * x_stride) +
                                               (int64_t)c * (LR_KC * 2) + xunit * 16);
   };
   auto store_x = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) xs[buf][i * 256 + xrow * 16 + (xunit ^ xrow)] = xr[i];
+    for (int i = 0; i < XP; ++i) xs[buf][(i * 4 * WAVES + xrow) * 16 + (xunit ^ (xrow & 15))] = xr[i];
   };
 
   if (c_begin < c_end) {
@@ -116,14 +120,15 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(
   // lane (col, grp): rows n0 + grp*4 .. +3 of the weights, row i*16 + col of x
   const int n = n0 + grp * 4;
   if constexpr (FORM == LR_SILU) {
-    float* up = reinterpret_cast<float*>(&xs[0][0]);   // [2 waves][MT*16 rows][16]
-    if (wave >= 2) {
+    float* up = reinterpret_cast<float*>(&xs[0][0]);   // [HW waves][MT*16 rows][16]
+    static_assert(HW * MT * 16 * 16 * 4 <= sizeof(xs), "the up halves fit the staging buffers");
+    if (wave >= HW) {
 #pragma unroll
       for (int i = 0; i < MT; ++i)
-        *reinterpret_cast<f32x4*>(up + (((wave - 2) * MT + i) * 16 + col) * 16 + grp * 4) = acc[i];
+        *reinterpret_cast<f32x4*>(up + (((wave - HW) * MT + i) * 16 + col) * 16 + grp * 4) = acc[i];
     }
     __syncthreads();
-    if (wave < 2) {
+    if (wave < HW) {
 #pragma unroll
       for (int i = 0; i < MT; ++i) {
         const int m = i * 16 + col;
@@ -159,32 +164,47 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(
   }
 }
 
+// Waves of a workgroup. Eight halve the reads of x, which at 128 rows and 64 weight rows
+// a workgroup are twice the weights' bytes; they pay where the weights still make enough
+// workgroups: 128 rows, 4096 x 14336 36 us (39.5 with four), 6144 x 4096 21.7 (23.9), but
+// 2048 x 2048 8.5 (6.9); unsplit, 28672 x 4096 with silu at 64 rows 57.4 (59.6), but
+// 16384 x 2048 27.5 (23.0).
+static int linear_rows_waves(int M, int N, int form) {
+  if (N % 128 != 0) return 4;
+  return (form == LR_PART ? M > 64 && N >= 4096 : M > 32 && N >= 200 * 128) ? 8 : 4;
+}
+
 extern "C" void launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
                                    int K, int x_stride, int form, int splits, hipStream_t stream) {
   const int per = (K / LR_KC + splits - 1) / splits;
-  const dim3 grid(form == LR_SILU ? N / 64 : (N + 63) / 64, splits);
-#define LR_GO(MT, F) \
-  hipLaunchKernelGGL((linear_rows_kernel<MT, F>), grid, dim3(256), 0, stream, out, x, w, bias, M, N, K, x_stride, per)
-#define LR_FORM(MT)                       \
-  switch (form) {                         \
-    case LR_PART: LR_GO(MT, LR_PART); break; \
-    case LR_BF16: LR_GO(MT, LR_BF16); break; \
-    case LR_F32: LR_GO(MT, LR_F32); break;   \
-    default: LR_GO(MT, LR_SILU); break;      \
+  const int waves = linear_rows_waves(M, N, form);
+  const dim3 grid((N + 16 * waves - 1) / (16 * waves), splits);
+#define LR_GO(MT, F, WV)                                                                                          \
+  hipLaunchKernelGGL((linear_rows_kernel<MT, F, WV>), grid, dim3(64 * WV), 0, stream, out, x, w, bias, M, N, K, \
+                     x_stride, per)
+#define LR_FORM(MT, WV)                          \
+  switch (form) {                                \
+    case LR_PART: LR_GO(MT, LR_PART, WV); break; \
+    case LR_BF16: LR_GO(MT, LR_BF16, WV); break; \
+    case LR_F32: LR_GO(MT, LR_F32, WV); break;   \
+    default: LR_GO(MT, LR_SILU, WV); break;      \
   }
-  if (M <= 16) { LR_FORM(1); }
-  else if (M <= 32) { LR_FORM(2); }
-  else if (M <= 64) { LR_FORM(4); }
-  else { LR_FORM(8); }
+  if (M <= 16) { LR_FORM(1, 4); }
+  else if (M <= 32) { LR_FORM(2, 4); }
+  else if (waves == 8 && M <= 64) { LR_FORM(4, 8); }
+  else if (waves == 8) { LR_FORM(8, 8); }
+  else if (M <= 64) { LR_FORM(4, 4); }
+  else { LR_FORM(8, 4); }
 #undef LR_FORM
 #undef LR_GO
 }
 
-// splits of k for the PART form: about 800 workgroups, 512 where the rows' sums weigh
-// more (M > 32), none below two chunks
+// splits of k for the PART form: about 800 workgroups, 512 (256 of eight waves) where
+// the rows' sums weigh more (M > 32), and two chunks at least
 extern "C" int linear_rows_splits(int M, int N, int K) {
-  const int tiles = (N + 63) / 64, chunks = K / LR_KC;
-  int s = ((M <= 32 ? 800 : 512) + tiles / 2) / tiles;
+  const int waves = linear_rows_waves(M, N, LR_PART);
+  const int tiles = (N + 16 * waves - 1) / (16 * waves), chunks = K / LR_KC;
+  int s = ((M <= 32 ? 800 : 2048 / waves) + tiles / 2) / tiles;
   s = s < chunks / 2 ? s : chunks / 2;
   return s < 1 ? 1 : s;
 }
