@@ -106,8 +106,7 @@ __global__ void __launch_bounds__(WAVE) linear_attn_decay_kernel(
       S[d] = dc * S[d] + buf[DMAX + d0 + d] * vj;
       acc += S[d] * buf[d0 + d];
     }
-#pragma unroll
-    for (int off = COLS; off < WAVE; off <<= 1) acc += __shfl_xor(acc, off);
+    acc = group_sum<COLS>(acc);
     if (live) {
       if (grp == 0) o[((int64_t)t0 * H + h) * V + j] = acc + skp * vj;
 #pragma unroll
@@ -164,8 +163,7 @@ __global__ void __launch_bounds__(WAVE) linear_attn_decay_kernel(
           S[d] = dc[u] * S[d] + buf[DMAX + d0 + d] * vj[u];
           acc += S[d] * buf[d0 + d];
         }
-#pragma unroll
-        for (int off = COLS; off < WAVE; off <<= 1) acc += __shfl_xor(acc, off);
+        acc = group_sum<COLS>(acc);
         if (live && grp == 0) o[((int64_t)(tg + u) * H + h) * V + j] = acc + skp * vj[u];
       }
     }
@@ -399,8 +397,7 @@ __global__ void __launch_bounds__(WAVE) gated_delta_rule_kernel(
       S[d] *= buf[2 * DMAX + d0 + d];
       pred += S[d] * buf[DMAX + d0 + d];
     }
-#pragma unroll
-    for (int off = COLS; off < WAVE; off <<= 1) pred += __shfl_xor(pred, off);
+    pred = group_sum<COLS>(pred);
     const float uu = beta * (vj - pred);
     float acc = 0.f;
 #pragma unroll
@@ -408,8 +405,7 @@ __global__ void __launch_bounds__(WAVE) gated_delta_rule_kernel(
       S[d] += buf[DMAX + d0 + d] * uu;
       acc += S[d] * buf[d0 + d];
     }
-#pragma unroll
-    for (int off = COLS; off < WAVE; off <<= 1) acc += __shfl_xor(acc, off);
+    acc = group_sum<COLS>(acc);
     if (live) {
       if (grp == 0) o[((int64_t)t0 * H + h) * V + j] = acc;
 #pragma unroll
@@ -467,8 +463,7 @@ __global__ void __launch_bounds__(WAVE) gated_delta_rule_kernel(
           S[d] *= buf[2 * DMAX + d0 + d];
           pred += S[d] * buf[DMAX + d0 + d];
         }
-#pragma unroll
-        for (int off = COLS; off < WAVE; off <<= 1) pred += __shfl_xor(pred, off);
+        pred = group_sum<COLS>(pred);
         const float uu = beta[u] * (vj[u] - pred);
         float acc = 0.f;
 #pragma unroll
@@ -476,8 +471,7 @@ __global__ void __launch_bounds__(WAVE) gated_delta_rule_kernel(
           S[d] += buf[DMAX + d0 + d] * uu;
           acc += S[d] * buf[d0 + d];
         }
-#pragma unroll
-        for (int off = COLS; off < WAVE; off <<= 1) acc += __shfl_xor(acc, off);
+        acc = group_sum<COLS>(acc);
         if (live && grp == 0) o[((int64_t)(tg + u) * H + h) * V + j] = acc;
       }
     }
