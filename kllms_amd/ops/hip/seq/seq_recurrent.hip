@@ -356,8 +356,9 @@ __global__ void delta_prep_kernel(float* __restrict__ qn, float* __restrict__ kn
 }
 
 // The recurrence proper, on the pre-pass's fp32 operands; wave layout and
-// pipeline as in linear_attn_decay_kernel.
-template <int DMAX, int NS>
+// pipeline as in linear_attn_decay_kernel. RUN tokens are one block of straight
+// code: the next token's LDS reads go out while this one's chain runs.
+template <int DMAX, int NS, int RUN>
 __global__ void __launch_bounds__(WAVE) gated_delta_rule_kernel(
     float* __restrict__ o, const float* __restrict__ qn, const float* __restrict__ kn,
     const float* __restrict__ gd, const float* __restrict__ vf, const float* __restrict__ bt,
@@ -415,29 +416,50 @@ __global__ void __launch_bounds__(WAVE) gated_delta_rule_kernel(
   }
   for (int i = lane; i < 2 * TB * 3 * DMAX; i += WAVE) (&buf_[0][0][0])[i] = 0.f;   // pad rows stay zero
   __syncthreads();
+  const int jc = live ? j : V - 1;
   float pre[TB][PER], vpre[TB], bpre[TB];
   // where each staged element comes from and goes to, fixed per lane: element
-  // i = lane + r*64 of q|k|g (no index division inside the token loop)
+  // i = lane + r*64 of q|k|g (no index division inside the token loop). Lanes
+  // without an element, columns past V and tokens past the end read a valid
+  // neighbour and drop it, so that a group's loads carry no branch
   const float* src[PER];
   int src_step[PER], dst[PER];
 #pragma unroll
   for (int r = 0; r < PER; ++r) {
-    const int i = lane + r * WAVE;
+    const bool has = lane + r * WAVE < 3 * D;
+    const int i = has ? lane + r * WAVE : 0;
     const int which = i / D, d = i - which * D;
-    dst[r] = which < 3 ? which * DMAX + d : -1;
+    dst[r] = has ? which * DMAX + d : -1;
     src[r] = which == 0 ? qn + (int64_t)g * D + d : which == 1 ? kn + (int64_t)g * D + d : gd + (int64_t)h * D + d;
     src_step[r] = which == 2 ? H * D : G * D;
   }
   auto fetch = [&](int tg) {
 #pragma unroll
     for (int u = 0; u < TB; ++u) {
-      const int t = tg + u;
-      const bool on = t < t1;
+      const int t = min(tg + u, t1 - 1);
 #pragma unroll
-      for (int r = 0; r < PER; ++r) pre[u][r] = (on && dst[r] >= 0) ? src[r][(int64_t)t * src_step[r]] : 0.f;
-      vpre[u] = (on && live) ? vf[((int64_t)t * H + h) * V + j] : 0.f;
-      bpre[u] = on ? bt[(int64_t)t * H + h] : 0.f;
+      for (int r = 0; r < PER; ++r) pre[u][r] = src[r][(int64_t)t * src_step[r]];
+      vpre[u] = vf[((int64_t)t * H + h) * V + jc];
+      bpre[u] = bt[(int64_t)t * H + h];
     }
+  };
+  auto token = [&](const float* buf, int t, float v, float beta) {
+    float pred = 0.f;
+#pragma unroll
+    for (int d = 0; d < DR; ++d) {
+      S[d] *= buf[2 * DMAX + d0 + d];
+      pred += S[d] * buf[DMAX + d0 + d];
+    }
+    pred = group_sum<COLS>(pred);
+    const float uu = beta * (v - pred);
+    float acc = 0.f;
+#pragma unroll
+    for (int d = 0; d < DR; ++d) {
+      S[d] += buf[DMAX + d0 + d] * uu;
+      acc += S[d] * buf[d0 + d];
+    }
+    acc = group_sum<COLS>(acc);
+    if (live && grp == 0) o[((int64_t)t * H + h) * V + j] = acc;
   };
   if (t0 < t1) fetch(t0);
   int flip = 0;
@@ -454,25 +476,14 @@ __global__ void __launch_bounds__(WAVE) gated_delta_rule_kernel(
     __syncthreads();
     if (tg + TB < t1) fetch(tg + TB);
 #pragma unroll
-    for (int u = 0; u < TB; ++u) {
-      if (tg + u < t1) {
-        const float* buf = buf_[flip][u];
-        float pred = 0.f;
+    for (int u = 0; u < TB; u += RUN) {
+      if (tg + u + RUN <= t1) {
 #pragma unroll
-        for (int d = 0; d < DR; ++d) {
-          S[d] *= buf[2 * DMAX + d0 + d];
-          pred += S[d] * buf[DMAX + d0 + d];
-        }
-        pred = group_sum<COLS>(pred);
-        const float uu = beta[u] * (vj[u] - pred);
-        float acc = 0.f;
+        for (int w = 0; w < RUN; ++w) token(buf_[flip][u + w], tg + u + w, vj[u + w], beta[u + w]);
+      } else {
 #pragma unroll
-        for (int d = 0; d < DR; ++d) {
-          S[d] += buf[DMAX + d0 + d] * uu;
-          acc += S[d] * buf[d0 + d];
-        }
-        acc = group_sum<COLS>(acc);
-        if (live && grp == 0) o[((int64_t)(tg + u) * H + h) * V + j] = acc;
+        for (int w = 0; w < RUN - 1; ++w)
+          if (tg + u + w < t1) token(buf_[flip][u + w], tg + u + w, vj[u + w], beta[u + w]);
       }
     }
   }
@@ -627,10 +638,22 @@ extern "C" void seq_launch_gated_delta_rule(float* o, const void* q, const void*
                                         (const T*)a, dt_bias, a_log, H, G, D, V, q_stride, k_stride, v_stride,
                                         beta_stride, a_stride);)
   const int ns = pick_split(B, H, V);
-  DISPATCH_NS(ns, DISPATCH_D(D, hipLaunchKernelGGL((gated_delta_rule_kernel<DMAX, NS>),
-                                                   dim3(B, H, (V + WAVE / NS - 1) / (WAVE / NS)), dim3(WAVE), 0,
-                                                   st, o, qn, kn, gd, vf, bt, state, slots, cu, seg_start, H, G,
-                                                   D, V);))
+  const dim3 grid(B, H, (V + WAVE / ns - 1) / (WAVE / ns));
+  // Four tokens of straight code where they can pay: at the finest split a SIMD has
+  // few waves and a token's chain takes the time, while coarser splits come with many
+  // waves and lose more to the registers; one row a segment has no next token. 8
+  // prompts of 1000 tokens, 16 heads: D = V = 64 478 us (a token at a time and LDS
+  // shuffles: 643), D = V = 128 705 (904). 64 x 250 tokens, 32 heads of 128 (split
+  // into 4): 3558 us as straight code and 111 us for one row each, 2118 and 82 with a
+  // token at a time.
+  if (ns == 8 && T_ > B) {
+    DISPATCH_D(D, hipLaunchKernelGGL((gated_delta_rule_kernel<DMAX, 8, 4>), grid, dim3(WAVE), 0, st, o, qn, kn, gd,
+                                     vf, bt, state, slots, cu, seg_start, H, G, D, V);)
+  } else {
+    DISPATCH_NS(ns, DISPATCH_D(D, hipLaunchKernelGGL((gated_delta_rule_kernel<DMAX, NS, 1>), grid, dim3(WAVE), 0,
+                                                     st, o, qn, kn, gd, vf, bt, state, slots, cu, seg_start, H, G,
+                                                     D, V);))
+  }
 }
 
 // the carried history alone, for kernels of other files that convolve by themselves

@@ -182,3 +182,26 @@ def test_gated_delta_rule(dtype, H, G, D, V):
     o2 = torch_ref.gated_delta_rule(q, k, v, beta, a, dt, alog, s2, slots, cu, st)
     close(o1, o2, torch.float32, scale=10)
     close(s1, s2, torch.float32, scale=10)
+
+
+# the two forms of the recurrence (several tokens of straight code, and one at a time) at their remainders: the same
+# sums in the same order, so one long prompt and the same tokens one by one give the same bits
+@pytest.mark.parametrize("D,V", [(24, 5), (32, 8), (64, 72), (128, 16), (256, 9)])
+def test_gated_delta_rule_runs_match_single_tokens(D, V):
+    lens, H, G = [1, 2, 3, 4, 5, 7, 8, 9], 2, 1
+    T, B = sum(lens), len(lens)
+    slots = torch.randperm(B).to(torch.int32).to(DEV)
+    x = [rnd(T, G, D, seed=1), rnd(T, G, D, seed=2), rnd(T, H, V, seed=3), rnd(T, H, seed=4), rnd(T, H * D, seed=5)]
+    dt, alog = rnd(H * D, seed=6) * 0.5, rnd(H, seed=7) * 0.5
+    s1 = rnd(B, H, D, V, seed=8)
+    s2 = s1.clone()
+    cu, st, _ = segments(lens, [0, 3] * (B // 2))
+    o1 = ops.gated_delta_rule(*x, dt, alog, s1, slots, cu, st)
+    o2 = torch.empty_like(o1)
+    for step in range(max(lens)):
+        live = [b for b in range(B) if step < lens[b]]
+        rows = [int(cu[b]) + step for b in live]
+        c1, t1, _ = segments([1] * len(live), [step + 3 * (b % 2) for b in live])
+        o2[rows] = ops.gated_delta_rule(*(t[rows].contiguous() for t in x), dt, alog, s2, slots[live].contiguous(),
+                                        c1, t1)
+    assert torch.equal(o1, o2) and torch.equal(s1, s2)
