@@ -7,6 +7,8 @@
 //   - SWAPPED QK^T: S = mfma(A=K_tile, B=Q), so a lane's accumulators hold one q-row's
 //     scores and the softmax is in registers (one permlane32_swap merges the halves)
 //   - P goes to bf16 MFMA B-fragments with pack + half swaps; O^T = mfma(A=V^T, B=P).
+//     The paged form multiplies P as two bf16 parts (16 bits of it and more), since
+//     rows behind a cache otherwise take the decode kernel, whose P is fp32
 //     V lies in LDS as it lies in memory; ds_read_b64_tr_b16 turns it on the way to
 //     the fragment (staging it transposed took 16 two-byte LDS writes a thread)
 //   - K's 16-byte units are XORed with the row, V's 32-byte slots too: both fragment
@@ -25,8 +27,8 @@
 //
 // Measured, 32 heads / 8 kv heads: one sequence of 7777 rows 612 us (810 TFLOP/s; 2019
 // with V staged transposed, synchronous staging and the mask in every tile), 24 of about
-// 512 rows 157 us (345); 8 segments of 150 rows behind 1536 cached keys 65 us (1017 as
-// single rows).
+// 512 rows 157 us (345); 8 segments of 150 rows behind 1536 cached keys 82 us (65 with
+// one part of P; 1017 as single rows).
 //
 // MFMA fragment maps (v_mfma_f32_32x32x16_bf16, verified on-device by the
 // mfma_selftest binding):
@@ -205,9 +207,8 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
       }
       // masked scores: fma(-inf, c2, -m) = -inf, whose exponential is 0
       const float m_use = m_run == -INFINITY ? 0.0f : m_run;
-      uint32_t packs[2][8];
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
+      // 32 keys of P to B-fragment words; paged: also what bf16 leaves of it
+      auto expo = [&](int sub, uint32_t (&hi)[8], uint32_t (&lo)[8]) {
 #pragma unroll
         for (int pr = 0; pr < 8; ++pr) {
           f32x2 p;
@@ -216,8 +217,14 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
             p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[sub][2 * pr + e], c2, -m_use));
             l_run += p[e];
           }
-          packs[sub][pr] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
+          hi[pr] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
+          if constexpr (PAGED) {
+            p[0] -= __uint_as_float(hi[pr] << 16);
+            p[1] -= __uint_as_float(hi[pr] & 0xffff0000u);
+            lo[pr] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
+          }
         }
+      };
 
       // ---- PV: O^T += V^T x P, 16 keys at a time ------------------------------
       const char* v_lds = smem[buf] + TILE_BYTES;
@@ -225,17 +232,23 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
       const int tr_row = half * 8 + ((lane & 15) >> 2);
       const int tr_byte = (lane & 3) * 8;
       const int tr_slot = (lane >> 4) & 1;
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
+      union PFrag { uint32_t w[4]; bf16x8_mfma m; };
+      auto fragment = [&](const uint32_t (&packs)[8], int kw) {
+        PFrag pf;
+        auto r0 = __builtin_amdgcn_permlane32_swap(packs[4 * kw + 0], packs[4 * kw + 2], false, false);
+        auto r1 = __builtin_amdgcn_permlane32_swap(packs[4 * kw + 1], packs[4 * kw + 3], false, false);
+        pf.w[0] = r0[0];
+        pf.w[1] = r1[0];
+        pf.w[2] = r0[1];
+        pf.w[3] = r1[1];
+        return pf;
+      };
+      auto weighted = [&](int sub, const uint32_t (&hi)[8], const uint32_t (&lo)[8]) {
 #pragma unroll
         for (int kw = 0; kw < 2; ++kw) {
-          union { uint32_t w[4]; bf16x8_mfma m; } pf;
-          auto r0 = __builtin_amdgcn_permlane32_swap(packs[sub][4 * kw + 0], packs[sub][4 * kw + 2], false, false);
-          auto r1 = __builtin_amdgcn_permlane32_swap(packs[sub][4 * kw + 1], packs[sub][4 * kw + 3], false, false);
-          pf.w[0] = r0[0];
-          pf.w[1] = r1[0];
-          pf.w[2] = r0[1];
-          pf.w[3] = r1[1];
+          const PFrag ph = fragment(hi, kw);
+          PFrag pl;
+          if constexpr (PAGED) pl = fragment(lo, kw);
           const int key = sub * 32 + kw * 16 + tr_row;
 #pragma unroll
           for (int dt = 0; dt < 4; ++dt) {
@@ -246,9 +259,24 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
               const char* p = v_lds + kr * 256 + (((dt * 2 + tr_slot) ^ (kr & 7)) << 5) + tr_byte;
               vf.t[rd] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
             }
-            o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.m, pf.m, o_acc[dt], 0, 0, 0);
+            o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.m, ph.m, o_acc[dt], 0, 0, 0);
+            if constexpr (PAGED) o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.m, pl.m, o_acc[dt], 0, 0, 0);
           }
         }
+      };
+      uint32_t hi[2][8], lo[2][8];
+      if constexpr (PAGED) {       // one half after the other: the registers of all four parts are not there
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+          expo(sub, hi[sub], lo[sub]);
+          weighted(sub, hi[sub], lo[sub]);
+        }
+      } else {
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) expo(sub, hi[sub], lo[sub]);
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) weighted(sub, hi[sub], lo[sub]);
+      }
     }
     if (more) store_kv(buf ^ 1);
     __syncthreads();
