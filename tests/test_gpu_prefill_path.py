@@ -149,3 +149,36 @@ def test_rope_store_matches_the_two_kernels(T, H, G, BS, fp8):
     assert float((a[1] != b[1]).float().mean()) < 0.02
     if fp8:
         assert torch.equal(a[4], b[4]) and torch.allclose(a[3], b[3], rtol=2 ** -7)
+
+
+@pytest.mark.parametrize("H,I,counts", [(64, 64, [1, 0, 2]), (320, 192, [0, 255, 256, 257, 1]), (512, 448, [31, 512, 0, 0, 33])])
+def test_mixture_products_against_float64(H, I, counts):
+    E, k = len(counts), 2
+    g = torch.Generator().manual_seed(H)
+    T = sum(counts)
+    first = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])[torch.randperm(T, generator=g)]
+    topi = torch.stack([first, (first + 1) % E], 1).to(DEV)
+    topw = torch.rand(T, k, generator=g).to(DEV)
+    x = torch.randn(T, H, generator=g).bfloat16().to(DEV)
+    wg = (torch.randn(E, 2 * I, H, generator=g) * H ** -0.5).bfloat16().to(DEV)
+    wd = (torch.randn(E, H, I, generator=g) * I ** -0.5).bfloat16().to(DEV)
+    ids, pos, offsets = ops.moe_sort(topi, E)
+    assert offsets.tolist() == [0] + torch.bincount(topi.flatten(), minlength=E).cumsum(0).tolist()
+    assert torch.equal(ids[pos.view(T, k).long()], torch.arange(T, device=DEV, dtype=ids.dtype).unsqueeze(1).expand(T, k))
+    act = torch.empty(T * k, I, device=DEV, dtype=x.dtype)
+    y = torch.empty(T * k, H, device=DEV, dtype=x.dtype)
+    ops.moe_gateup(act, x, wg, ids, offsets, x)
+    ops.moe_down(y, act, wd, offsets)
+    got = ops.moe_combine_rows(y, topw, pos)
+    # act, y and the result are each rounded to bf16 (2^-9); the sums and silu in 32 bits stay far below that
+    ref, lim = torch.zeros(T, H, device=DEV, dtype=torch.float64), torch.zeros(T, H, device=DEV, dtype=torch.float64)
+    for j in range(k):
+        for e in range(E):
+            rows = (topi[:, j] == e).nonzero()[:, 0]
+            gate, up = (x[rows].double() @ wg[e].double().t().contiguous()).split([I, I], 1)
+            a = torch.nn.functional.silu(gate) * up
+            ye = a @ wd[e].double().t().contiguous()
+            w = topw[rows, j].double().unsqueeze(1)
+            ref[rows] += w * ye
+            lim[rows] += w * 2 ** -8 * (a.abs() @ wd[e].double().abs().t().contiguous() + ye.abs())
+    assert ((got.double() - ref).abs() <= lim + 2 ** -8 * ref.abs() + 1e-5).all()
