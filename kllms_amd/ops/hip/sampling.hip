@@ -159,8 +159,8 @@ extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
     for (int j = 0; j < PU; ++j) sum += exp_from(x[j], m);
     if (cuts) {
 #pragma unroll
-      for (int j = 0; j < PU; ++j)
-        if (ok[j]) ssum += __expf((x[j] - m) * inv_t);
+      for (int j = 0; j < PU; ++j)   // as exp_from: -inf adds nothing, also before the thread has seen a finite token
+        if (x[j] != -INFINITY) ssum += __expf((x[j] - m) * inv_t);
     }
     if (draw) {
 #pragma unroll

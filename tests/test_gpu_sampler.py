@@ -78,3 +78,46 @@ def test_draw_matches_float64(B, V, mode):
         key = s + gumbel(int(seeds[b]), int(steps[b]), V)
         # two fast logarithms in fp32: 1e-7 absolute in the inner one, over a winner's 1 - u of about 1 / V
         assert key[t] >= key[order[must]].max() - max(1e-3, 4e-7 * V)
+
+
+@pytest.mark.parametrize("mode", ["top_p", "top_k", "both"])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("B,V", [(3, 63), (2, 2049), (33, 4099), (2, 131071)])
+def test_truncated_rows_with_minus_infinity_logits(B, V, masked, mode):
+    """Rows whose logits are -inf for all but a few tokens, for a padded tail, for every token of some threads'
+    strides: a thread that sees none before its first finite token adds nothing to the row's mass."""
+    g = torch.Generator().manual_seed(V + B)
+    logits = torch.randn(B, V, generator=g) * 2.0
+    at, kind = torch.arange(V), torch.arange(B).unsqueeze(1) % 3
+    logits[(kind == 0) & (torch.rand(B, V, generator=g) > max(20 / V, 0.004))] = -torch.inf
+    logits[(kind == 1) & (at >= V * 2 // 3)] = -torch.inf
+    logits[(kind == 2) & (at % 256 < 200)] = -torch.inf
+    logits[:, V // 2] = 1.0
+    mask, x = None, logits.double().numpy()
+    if masked:
+        bits = torch.rand(B, (V + 31) // 32, 32, generator=g) < 0.5
+        bits.view(B, -1)[:, V // 2] = True
+        w = (bits.long() << torch.arange(32)).sum(-1)
+        mask = torch.where(w >= 2**31, w - 2**32, w).to(torch.int32).to(DEV)
+        x = np.where(bits.view(B, -1)[:, :V].numpy(), x, -np.inf)
+    top_p, top_k = 1.0 if mode == "top_k" else 0.5, 0 if mode == "top_p" else 7
+    temp = torch.rand(B, generator=g) * 0.8 + 0.4
+    seeds, steps = torch.randint(0, 2**40, (B,), generator=g), torch.randint(0, 99, (B,), generator=g)
+    toks, lps = ops.sample(logits.to(DEV), temp.to(DEV), torch.full((B,), top_p, device=DEV),
+                           torch.full((B,), top_k, device=DEV, dtype=torch.int32), seeds.to(DEV), steps.to(DEV), mask)
+    for b, t in enumerate(toks.tolist()):
+        assert np.isfinite(x[b, t])
+        ref = x[b, t] - x[b].max() - np.log(np.exp(x[b] - x[b].max()).sum())
+        assert abs(float(lps[b]) - ref) < 2e-5      # as above
+        s = x[b] / float(temp[b])
+        order = np.argsort(-s, kind="stable")
+        p = np.exp(s[order] - s.max())
+        p /= p.sum()
+        before = np.cumsum(p) - p
+        may, must = before < top_p + 1e-5, before + p < top_p - 1e-5
+        if top_k:
+            may[top_k:] = must[top_k:] = False
+        must[0] = True
+        assert t in order[may]
+        key = s + gumbel(int(seeds[b]), int(steps[b]), V)
+        assert key[t] >= key[order[must]].max() - max(1e-3, 4e-7 * V)
