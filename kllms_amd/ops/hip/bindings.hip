@@ -349,7 +349,7 @@ torch::Tensor moe_combine(torch::Tensor y, torch::Tensor weights, torch::Tensor 
   CHECK_BF16_CONTIG(y);
   TORCH_CHECK(weights.is_cuda() && weights.is_contiguous() && weights.scalar_type() == at::kFloat &&
                   pos.is_cuda() && pos.is_contiguous() && pos.scalar_type() == at::kInt && pos.dim() == 2 &&
-                  weights.sizes() == pos.sizes() && y.dim() == 2 && y.size(1) % 8 == 0 && pos.size(0) <= 65535);
+                  weights.sizes() == pos.sizes() && y.dim() == 2 && y.size(1) % 8 == 0);
   auto out = torch::empty({pos.size(0), y.size(1)}, y.options());
   if (out.numel() == 0) return out;
   launch_moe_combine(out.data_ptr(), y.data_ptr(), weights.data_ptr<float>(), pos.data_ptr<int>(), (int)pos.size(0),

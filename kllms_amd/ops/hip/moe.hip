@@ -252,17 +252,18 @@ __global__ void __launch_bounds__(1024) moe_sort_kernel(int* __restrict__ ids, i
   }
 }
 
+// tokens on the grid's x: y and z stop at 65535, a packed prompt batch does not
 __global__ void __launch_bounds__(256) moe_combine_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ y,
                                                           const float* __restrict__ weights,
                                                           const int* __restrict__ pos, int k, int nvec) {
-  const int t = blockIdx.y;
-  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int t = blockIdx.x;
+  const int i = blockIdx.y * 256 + threadIdx.x;
   if (i >= nvec) return;
   float s[8] = {};
   for (int j = 0; j < k; ++j) {
-    const int p = pos[t * k + j];
+    const int p = pos[(int64_t)t * k + j];
     if (p < 0) continue;
-    const float w = weights[t * k + j];
+    const float w = weights[(int64_t)t * k + j];
     const bf16x8_vec v = reinterpret_cast<const bf16x8_vec*>(y)[(int64_t)p * nvec + i];
 #pragma unroll
     for (int c = 0; c < 8; ++c) s[c] += w * bf16_to_f32(v[c]);
@@ -309,6 +310,6 @@ extern "C" void launch_moe_sort(int* ids, int* pos, int* offsets, const int64_t*
 extern "C" void launch_moe_combine(void* out, const void* y, const float* weights, const int* pos, int T, int k,
                                    int H, hipStream_t stream) {
   const int nvec = H / 8;
-  hipLaunchKernelGGL(moe_combine_kernel, dim3((nvec + 255) / 256, T), dim3(256), 0, stream, (bf16_t*)out,
+  hipLaunchKernelGGL(moe_combine_kernel, dim3(T, (nvec + 255) / 256), dim3(256), 0, stream, (bf16_t*)out,
                      (const bf16_t*)y, weights, pos, k, nvec);
 }

@@ -182,3 +182,20 @@ def test_mixture_products_against_float64(H, I, counts):
             ref[rows] += w * ye
             lim[rows] += w * 2 ** -8 * (a.abs() @ wd[e].double().abs().t().contiguous() + ye.abs())
     assert ((got.double() - ref).abs() <= lim + 2 ** -8 * ref.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("T,H", [(65535, 8), (65536, 64), (70001, 2056)])
+def test_mixture_of_more_rows_than_a_grid_has_in_y(T, H):
+    g = torch.Generator(device=DEV).manual_seed(T)
+    E, k = 8, 2
+    topi = torch.rand(T, E, generator=g, device=DEV).topk(k, -1).indices
+    topw = torch.rand(T, k, generator=g, device=DEV)
+    ids, pos, offsets = ops.moe_sort(topi, E)
+    assert torch.equal(ids[pos.long()], torch.arange(T, device=DEV, dtype=ids.dtype).unsqueeze(1).expand(T, k))
+    y = torch.randn(T * k, H, generator=g, device=DEV).bfloat16()
+    got = ops.moe_combine_rows(y, topw, pos)
+    rows = y[pos.long()].float()
+    ref = (rows * topw.unsqueeze(-1)).sum(1)
+    # two products and a sum in fp32, one rounding to bf16 (2^-9)
+    lim = 2 ** -8 * ref.abs() + 2 ** -22 * (rows.abs() * topw.unsqueeze(-1)).sum(1)
+    assert ((got.float() - ref).abs() <= lim).all()
