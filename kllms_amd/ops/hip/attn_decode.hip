@@ -345,29 +345,41 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(
   }
 }
 
+// Rows of one launch: they lie on the grid's y, which ends at 65535. Steps with a row
+// per token (prompt portions on the fp8 cache, short segments) can have more and go out
+// in several launches; on x, beside the kv heads, every workgroup would divide.
+#define MAX_ROWS 65535
+
 // picks the GQA instantiation (the binding admits 1, 2, 4, 8); partials: room for
-// B * KVH * splits * gqa * 130 floats when splits > 1
+// min(B, MAX_ROWS) * KVH * splits * gqa * 130 floats when splits > 1
 extern "C" void launch_attn_decode(
     bf16_t* out, float* partials, const bf16_t* q, const void* k_cache, const void* v_cache,
     const float* k_scale, const float* v_scale, const int* block_tables, const int* context_lens,
     const bf16_t* gate, int gate_stride, float scale, int num_q_heads, int num_kv_heads, int block_size,
     int max_blocks, int splits, int q_tstride, int B, int cache_fp8, int mask_size, hipStream_t stream) {
   const int gqa = num_q_heads / num_kv_heads;
-  const dim3 grid(num_kv_heads, B, splits);
+  for (int b0 = 0; b0 < B; b0 += MAX_ROWS) {
+    const int rows = B - b0 < MAX_ROWS ? B - b0 : MAX_ROWS;
+    const dim3 grid(num_kv_heads, rows, splits);
+    bf16_t* o = out + (int64_t)b0 * num_q_heads * 128;
+    const bf16_t* q0 = q + (int64_t)b0 * q_tstride;
+    const int* bt = block_tables + (int64_t)b0 * max_blocks;
+    const bf16_t* g0 = gate ? gate + (int64_t)b0 * gate_stride : nullptr;
 #define LAUNCH(G, F)                                                                            \
-  hipLaunchKernelGGL((attn_decode_tiles<G, F>), grid, dim3(NTHREADS), 0, stream, partials, out, q, \
-                     (const char*)k_cache, (const char*)v_cache, k_scale, v_scale, block_tables,   \
-                     context_lens, gate, gate_stride, scale, block_size, max_blocks, q_tstride, mask_size)
+  hipLaunchKernelGGL((attn_decode_tiles<G, F>), grid, dim3(NTHREADS), 0, stream, partials, o, q0, \
+                     (const char*)k_cache, (const char*)v_cache, k_scale, v_scale, bt,             \
+                     context_lens + b0, g0, gate_stride, scale, block_size, max_blocks, q_tstride, mask_size)
 #define DISPATCH(G) do { if (cache_fp8) LAUNCH(G, true); else LAUNCH(G, false); } while (0)
-  switch (gqa) {
-    case 1: DISPATCH(1); break;
-    case 2: DISPATCH(2); break;
-    case 4: DISPATCH(4); break;
-    default: DISPATCH(8); break;
-  }
+    switch (gqa) {
+      case 1: DISPATCH(1); break;
+      case 2: DISPATCH(2); break;
+      case 4: DISPATCH(4); break;
+      default: DISPATCH(8); break;
+    }
 #undef DISPATCH
 #undef LAUNCH
-  if (splits > 1)
-    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(num_q_heads, B), dim3(256), 0, stream, out,
-                       partials, context_lens, gate, gate_stride, gqa, splits, mask_size);
+    if (splits > 1)
+      hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(num_q_heads, rows), dim3(256), 0, stream, o,
+                         partials, context_lens + b0, g0, gate_stride, gqa, splits, mask_size);
+  }
 }

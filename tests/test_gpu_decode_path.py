@@ -248,3 +248,26 @@ def test_linear_attention_chunks(H, Dk, V, dtype):
         assert ((got_state[slots[b]].double().cpu() - S).abs() <= 300 * 2 ** -23 * size + 1e-6).all()
         r += n
     assert torch.equal(got_state[1].cpu(), state[1])
+
+
+@pytest.mark.parametrize("gated,fp8", [(False, False), (False, True), (True, False)])
+def test_more_decode_rows_than_a_grid_has_in_y(gated, fp8):
+    """65536 rows and more (a row per token of long prompt portions), against the same rows in two calls."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    B, H, KVH, BS, NB = 65539, 2, 1, 16, 64
+    q = torch.randn(B, H, D, generator=g, device=DEV).bfloat16()
+    k, v = (torch.randn(NB, KVH, BS, D, generator=g, device=DEV).bfloat16() for _ in range(2))
+    sc = [None, None]
+    if fp8:
+        sc = [torch.rand(NB, KVH, BS, generator=g, device=DEV) + 0.5 for _ in range(2)]
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+    bt = torch.randint(0, NB, (B, 2), generator=g, device=DEV, dtype=torch.int32)
+    ctx = torch.randint(1, 33, (B,), generator=g, device=DEV, dtype=torch.int32)
+    gate = torch.randn(B, H, generator=g, device=DEV).bfloat16()
+
+    def rows(a, b):
+        if gated:
+            return ops.attn_blocklocal_rows(q[a:b], k, v, bt[a:b], ctx[a:b], 0.1, 24, gate[a:b])
+        return ops.attn_decode_paged(q[a:b], k, v, bt[a:b], ctx[a:b], 0.1, *sc)
+
+    assert torch.equal(rows(0, B), torch.cat([rows(0, 40000), rows(40000, B)]))
