@@ -304,13 +304,19 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
   }
 }
 
+// groups of a launch: they lie on the grid's y, which ends at 65535 (a sequence has one at
+// least, so many short prompts have as many)
+#define MAX_GROUPS 65535
+
 extern "C" void launch_attn_prefill(bf16_t* out, const bf16_t* q, const bf16_t* k, const bf16_t* v,
                                     const int* grp_start, const int* grp_len, const int* grp_q0, int q0_stride,
                                     int ngroups, float scale, int num_q_heads, int num_kv_heads, int q_tstride,
                                     int kv_tstride, hipStream_t stream) {
-  hipLaunchKernelGGL(attn_prefill_kernel<false>, dim3(num_q_heads, ngroups), dim3(64 * NWAVES), 0, stream, out, q, k,
-                     v, grp_start, grp_len, grp_q0, nullptr, nullptr, nullptr, scale, num_kv_heads, q_tstride,
-                     kv_tstride, q0_stride, 1, 0);
+  for (int g = 0; g < ngroups; g += MAX_GROUPS)
+    hipLaunchKernelGGL(attn_prefill_kernel<false>, dim3(num_q_heads, ngroups - g < MAX_GROUPS ? ngroups - g : MAX_GROUPS),
+                       dim3(64 * NWAVES), 0, stream, out, q, k, v, grp_start + g, grp_len + g,
+                       grp_q0 + (int64_t)g * q0_stride, nullptr, nullptr, nullptr, scale, num_kv_heads, q_tstride,
+                       kv_tstride, q0_stride, 1, 0);
 }
 
 extern "C" void launch_attn_prefill_paged(bf16_t* out, const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache,
@@ -318,9 +324,11 @@ extern "C" void launch_attn_prefill_paged(bf16_t* out, const bf16_t* q, const bf
                                           const int* grp_seg, const int* block_tables, const int* seg_pos, int ngroups,
                                           float scale, int num_q_heads, int num_kv_heads, int q_tstride,
                                           int block_size, int max_blocks, hipStream_t stream) {
-  hipLaunchKernelGGL(attn_prefill_kernel<true>, dim3(num_q_heads, ngroups), dim3(64 * NWAVES), 0, stream, out, q,
-                     k_cache, v_cache, grp_start, grp_len, grp_q0, grp_seg, block_tables, seg_pos, scale,
-                     num_kv_heads, q_tstride, 0, 1, block_size, max_blocks);
+  for (int g = 0; g < ngroups; g += MAX_GROUPS)
+    hipLaunchKernelGGL(attn_prefill_kernel<true>, dim3(num_q_heads, ngroups - g < MAX_GROUPS ? ngroups - g : MAX_GROUPS),
+                       dim3(64 * NWAVES), 0, stream, out, q, k_cache, v_cache, grp_start + g, grp_len + g, grp_q0 + g,
+                       grp_seg + g, block_tables, seg_pos, scale, num_kv_heads, q_tstride, 0, 1, block_size,
+                       max_blocks);
 }
 
 // Groups of 256 rows of each sequence cu[i]..cu[i+1], into plan [3, G] (start, length,

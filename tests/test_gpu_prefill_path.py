@@ -199,3 +199,35 @@ def test_mixture_of_more_rows_than_a_grid_has_in_y(T, H):
     # two products and a sum in fp32, one rounding to bf16 (2^-9)
     lim = 2 ** -8 * ref.abs() + 2 ** -22 * (rows.abs() * topw.unsqueeze(-1)).sum(1)
     assert ((got.float() - ref).abs() <= lim).all()
+
+
+@pytest.mark.parametrize("n", [65535, 66000])
+def test_more_prompts_than_a_grid_has_in_y(n):
+    """As many groups as sequences: the same rows attended in two calls."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    lens = torch.randint(1, 4, (n,), generator=g, device=DEV)
+    cu = torch.cat([lens.new_zeros(1), lens.cumsum(0)]).to(torch.int32)
+    T, cut = int(cu[-1]), int(cu[30000])
+    qkv = torch.randn(T, 3, D, generator=g, device=DEV).bfloat16()
+    q, k, v = qkv.split([1, 1, 1], 1)
+    out = ops.attn_prefill_varlen(q, k, v, cu, 0.1)
+    halves = [ops.attn_prefill_varlen(q[a:b], k[a:b], v[a:b], c, 0.1)
+              for a, b, c in ((0, cut, cu[:30001]), (cut, T, cu[30000:] - cut))]
+    assert torch.equal(out, torch.cat(halves))
+
+
+def test_more_segments_than_a_grid_has_in_y():
+    g = torch.Generator(device=DEV).manual_seed(3)
+    n, rows, NB = 65600, 32, 8
+    kc, vc = (torch.randn(NB, 1, 32, D, generator=g, device=DEV).bfloat16() for _ in range(2))
+    tables = torch.randint(0, NB, (n, 1), generator=g, device=DEV, dtype=torch.int32)
+    pos = torch.zeros(n, dtype=torch.int32, device=DEV)
+    q = torch.randn(n * rows, 1, D, generator=g, device=DEV).bfloat16()
+    plan, short = ops.paged_prefill_plan([(0, rows)] * n, DEV)
+    assert plan.shape[1] == n and not short
+    out = ops.attn_segments_paged(q, kc, vc, None, None, 0.1, plan, short, tables, pos)
+    for lo, hi in ((0, 200), (n - 200, n)):
+        part, _ = ops.paged_prefill_plan([(0, rows)] * (hi - lo), DEV)
+        want = ops.attn_segments_paged(q[lo * rows:hi * rows], kc, vc, None, None, 0.1, part, [], tables[lo:hi].contiguous(),
+                                       pos[lo:hi])
+        assert torch.equal(out[lo * rows:hi * rows], want)
