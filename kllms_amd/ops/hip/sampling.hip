@@ -596,8 +596,16 @@ extern "C" void launch_sample(int64_t* tokens, float* logprobs, void* parts, con
                               int V, float* dbg, hipStream_t stream) {
   const int n = sample_slices(B, V);
   const int slice = (V + n - 1) / n;
-  hipLaunchKernelGGL(sample_part_kernel, dim3(n, B), dim3(PT), 0, stream, (SlicePart*)parts, logits,
-                     temps, top_ps, top_ks, seeds, steps, mask, V, slice);
-  hipLaunchKernelGGL(sample_final_kernel, dim3(B), dim3(NT), 0, stream, tokens, logprobs,
-                     (const SlicePart*)parts, n, logits, temps, top_ps, top_ks, seeds, steps, mask, V, dbg);
+  // rows of a launch lie on the grid's y, which ends at 65535
+  for (int b = 0; b < B; b += 65535) {
+    const int rows = B - b < 65535 ? B - b : 65535;
+    SlicePart* p = (SlicePart*)parts + (int64_t)b * n;
+    const float* x = logits + (int64_t)b * V;
+    const uint32_t* m = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
+    hipLaunchKernelGGL(sample_part_kernel, dim3(n, rows), dim3(PT), 0, stream, p, x, temps + b, top_ps + b,
+                       top_ks + b, seeds + b, steps + b, m, V, slice);
+    hipLaunchKernelGGL(sample_final_kernel, dim3(rows), dim3(NT), 0, stream, tokens + b, logprobs + b,
+                       (const SlicePart*)p, n, x, temps + b, top_ps + b, top_ks + b, seeds + b, steps + b, m, V,
+                       dbg ? dbg + (int64_t)b * 16 : nullptr);
+  }
 }

@@ -121,3 +121,19 @@ def test_truncated_rows_with_minus_infinity_logits(B, V, masked, mode):
         assert t in order[may]
         key = s + gumbel(int(seeds[b]), int(steps[b]), V)
         assert key[t] >= key[order[must]].max() - max(1e-3, 4e-7 * V)
+
+
+@pytest.mark.parametrize("V", [1, 70])
+def test_more_rows_than_a_grid_has_in_y(V):
+    g = torch.Generator(device=DEV).manual_seed(V)
+    B = 65600
+    logits = torch.randn(B, V, generator=g, device=DEV)
+    temp = torch.rand(B, generator=g, device=DEV) + 0.3
+    top_p = torch.where(torch.arange(B, device=DEV) % 2 == 0, 0.7, 1.0)
+    top_k = torch.randint(0, 5, (B,), generator=g, device=DEV, dtype=torch.int32)
+    seeds, steps = torch.randint(0, 2**40, (B,), generator=g, device=DEV), torch.arange(B, device=DEV)
+    mask = torch.randint(-2**31, 2**31, (B, (V + 31) // 32), generator=g, device=DEV).to(torch.int32) | 1
+    whole = ops.sample(logits, temp, top_p, top_k, seeds, steps, mask)
+    for a, b in ((0, 300), (B - 300, B)):
+        part = ops.sample(*(t[a:b] for t in (logits, temp, top_p, top_k, seeds, steps, mask)))
+        assert torch.equal(whole[0][a:b], part[0]) and torch.equal(whole[1][a:b], part[1])
