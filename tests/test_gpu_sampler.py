@@ -137,3 +137,35 @@ def test_more_rows_than_a_grid_has_in_y(V):
     for a, b in ((0, 300), (B - 300, B)):
         part = ops.sample(*(t[a:b] for t in (logits, temp, top_p, top_k, seeds, steps, mask)))
         assert torch.equal(whole[0][a:b], part[0]) and torch.equal(whole[1][a:b], part[1])
+
+
+@pytest.mark.parametrize("V", [9000, 128256])
+@pytest.mark.parametrize("temp", [0.01, 0.7])
+def test_top_p_cut_does_not_move(V, temp):
+    """The cut of a row with a scaled maximum in the thousands (rounded by 1e-4 there) whose outer tokens hold about
+    that much, against float64; tokens and log-probabilities of the same rows at other batch sizes."""
+    g = torch.Generator().manual_seed(V)
+    R = 250
+    s = -torch.rand(R, V, generator=g) * 4.0 - (np.log(V) + 4.5)        # outer tokens: 0.003 of the mass
+    s[:, 5] = 0.0
+    x = (30.0 + 0.1 * torch.rand(R, 1, generator=g) + s * temp).float()
+    x64 = (x.double() - x.double().max(-1, keepdim=True).values) / float(np.float32(temp))
+    order = x64.sort(-1, descending=True).values.numpy()
+    share = np.exp(order).cumsum(-1) / np.exp(order).sum(-1, keepdims=True)
+    top_p = np.float32(1 - 0.4 * (1 - share[:, 0]))                     # inside the outer tokens
+    dev = lambda t: torch.as_tensor(t, device=DEV)  # noqa: E731
+    args = [dev(x), torch.full((R,), temp, device=DEV), dev(top_p), torch.zeros(R, dtype=torch.int32, device=DEV),
+            torch.randint(0, 2**40, (R,), generator=g).to(DEV), torch.zeros(R, dtype=torch.long, device=DEV)]
+    dbg = torch.zeros(R, 16, device=DEV)
+    toks, lps = ops.sample(*args, None, dbg)
+    low = torch.where(dbg[:, 9] > 0, dbg[:, 11], dbg[:, 7]).cpu().numpy()       # the last refinement's lower edge
+    for b in range(R):
+        # one fp32 rounding of a mass of 1 is 6e-8, of the outer tokens' 0.003 2e-5 for each sum it went through; and of
+        # x itself at 30, 2e-6 / temp in scaled logits
+        kept = int((order[b] > low[b]).sum()) - 1
+        want = int((share[b] < float(top_p[b])).sum())
+        assert abs(kept - want) <= 0.01 * V, (b, kept, want)
+    for n in (1, 7, 100):
+        t, p = ops.sample(*(a[:n] for a in args))
+        # the slices' sums in another order: a few fp32 roundings of each level of their tree
+        assert torch.equal(t, toks[:n]) and torch.allclose(p, lps[:n], rtol=0, atol=2e-6)
