@@ -146,6 +146,7 @@ void rope_store(torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor
                     (int)k.stride(0), BS, fp8, cur_stream());
 }
 
+// mask_size: -1 for plain decode rows, from 0 (plain causal) on for those of a block-local layer
 void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                        torch::Tensor v_cache, torch::Tensor block_tables,
                        torch::Tensor context_lens, double scale,
@@ -552,7 +553,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_store", &rope_store);
   m.def("attn_decode_paged", &attn_decode_paged, py::arg("out"), py::arg("q"), py::arg("k_cache"),
         py::arg("v_cache"), py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"), py::arg("k_scale"),
-        py::arg("v_scale"), py::arg("gate"), py::arg("mask_size") = 0);
+        py::arg("v_scale"), py::arg("gate"), py::arg("mask_size") = -1);
   m.def("attn_prefill", &attn_prefill);
   m.def("attn_prefill_plan", &attn_prefill_plan);
   m.def("attn_prefill_paged", &attn_prefill_paged);

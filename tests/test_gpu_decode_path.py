@@ -271,3 +271,33 @@ def test_more_decode_rows_than_a_grid_has_in_y(gated, fp8):
         return ops.attn_decode_paged(q[a:b], k, v, bt[a:b], ctx[a:b], 0.1, *sc)
 
     assert torch.equal(rows(0, B), torch.cat([rows(0, 40000), rows(40000, B)]))
+
+
+@pytest.mark.parametrize("gqa", [1, 2, 4, 8])
+@pytest.mark.parametrize("L", [2, 33, 1024])         # both keys in a tile, in two waves' tiles, in two shares of the context
+def test_blocklocal_rows_keep_32_bit_exponentials(L, gqa):
+    """A context whose last key dominates and has V = 0, so that the result is the first key's exp(-50..-70) alone, and
+    gates down to exp(-10): their relative error is the result's, which stays a normal number."""
+    B, BS = 200, 16
+    nb = (L + BS - 1) // BS
+    g = torch.Generator().manual_seed(L + gqa)
+    k, v = (torch.zeros(B * nb, 1, BS, D) for _ in range(2))
+    k[..., 0] = -300.0
+    bt = torch.arange(B * nb, dtype=torch.int32).view(B, nb)
+    top, low = torch.arange(B) % 6 + 2.0, -48.0 - torch.arange(B) % 60 / 4
+    for b in range(B):
+        k[b * nb, 0, 0, 0] = low[b]
+        v[b * nb, 0, 0] = torch.rand(D, generator=g).bfloat16().float() + 0.5
+        k[bt[b, (L - 1) // BS], 0, (L - 1) % BS, 0] = top[b]
+    v = v.bfloat16()
+    q = torch.zeros(B, gqa, D)
+    q[..., 0] = 1.0
+    gate = (-10 * torch.rand(B, gqa, generator=g)).bfloat16()
+    dev = lambda t: t.to(DEV)  # noqa: E731
+    out = ops.attn_blocklocal_rows(dev(q.bfloat16()), dev(k.bfloat16()), dev(v), dev(bt),
+                                   torch.full((B,), L, dtype=torch.int32, device=DEV), 1.0, 1024, dev(gate))
+    p = torch.exp((low - top).double()).view(B, 1, 1)
+    ref = p / (1 + p) * v[bt[:, 0].long(), 0, 0].double().view(B, 1, D) * torch.sigmoid(gate.double()).unsqueeze(-1)
+    # the rounding to bf16, and about ten 32-bit ones of 2^-24 before it (exponentials, fold, divisions, gate)
+    half = 2.0 ** (torch.floor(torch.log2(ref.abs())) - 8)
+    assert ((out.double().cpu() - ref).abs() <= half + 10 * 2 ** -24 * ref.abs()).all()
