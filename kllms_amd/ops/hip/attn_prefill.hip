@@ -7,8 +7,8 @@
 //   - SWAPPED QK^T: S = mfma(A=K_tile, B=Q), so a lane's accumulators hold one q-row's
 //     scores and the softmax is in registers (one permlane32_swap merges the halves)
 //   - P goes to bf16 MFMA B-fragments with pack + half swaps; O^T = mfma(A=V^T, B=P).
-//     The paged form multiplies P as two bf16 parts (16 bits of it and more), since
-//     rows behind a cache otherwise take the decode kernel, whose P is fp32
+//     The paged form multiplies P as three bf16 parts, 24 bits: exactly the fp32 P
+//     of the decode kernel, which rows behind a cache otherwise take
 //     V lies in LDS as it lies in memory; ds_read_b64_tr_b16 turns it on the way to
 //     the fragment (staging it transposed took 16 two-byte LDS writes a thread)
 //   - K's 16-byte units are XORed with the row, V's 32-byte slots too: both fragment
@@ -27,8 +27,8 @@
 //
 // Measured, 32 heads / 8 kv heads: one sequence of 7777 rows 612 us (810 TFLOP/s; 2019
 // with V staged transposed, synchronous staging and the mask in every tile), 24 of about
-// 512 rows 157 us (345); 8 segments of 150 rows behind 1536 cached keys 82 us (65 with
-// one part of P; 1017 as single rows).
+// 512 rows 157 us (345); 8 segments of 150 rows behind 1536 cached keys 96 us
+// in a graph (80 with two parts of P, which keep 16 bits; 551 as single rows).
 //
 // MFMA fragment maps (v_mfma_f32_32x32x16_bf16, verified on-device by the
 // mfma_selftest binding):
@@ -207,8 +207,10 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
       }
       // masked scores: fma(-inf, c2, -m) = -inf, whose exponential is 0
       const float m_use = m_run == -INFINITY ? 0.0f : m_run;
-      // 32 keys of P to B-fragment words; paged: also what bf16 leaves of it
-      auto expo = [&](int sub, uint32_t (&hi)[8], uint32_t (&lo)[8]) {
+      // 32 keys of P to B-fragment words; paged: also what bf16 leaves of it, twice (the
+      // differences are exact)
+      constexpr int PARTS = PAGED ? 3 : 1;
+      auto expo = [&](int sub, uint32_t (&w)[PARTS][8]) {
 #pragma unroll
         for (int pr = 0; pr < 8; ++pr) {
           f32x2 p;
@@ -217,11 +219,11 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
             p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[sub][2 * pr + e], c2, -m_use));
             l_run += p[e];
           }
-          hi[pr] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
-          if constexpr (PAGED) {
-            p[0] -= __uint_as_float(hi[pr] << 16);
-            p[1] -= __uint_as_float(hi[pr] & 0xffff0000u);
-            lo[pr] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
+#pragma unroll
+          for (int part = 0; part < PARTS; ++part) {
+            w[part][pr] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
+            p[0] -= __uint_as_float(w[part][pr] << 16);
+            p[1] -= __uint_as_float(w[part][pr] & 0xffff0000u);
           }
         }
       };
@@ -243,12 +245,12 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
         pf.w[3] = r1[1];
         return pf;
       };
-      auto weighted = [&](int sub, const uint32_t (&hi)[8], const uint32_t (&lo)[8]) {
+      auto weighted = [&](int sub, const uint32_t (&w)[PARTS][8]) {
 #pragma unroll
         for (int kw = 0; kw < 2; ++kw) {
-          const PFrag ph = fragment(hi, kw);
-          PFrag pl;
-          if constexpr (PAGED) pl = fragment(lo, kw);
+          PFrag pf[PARTS];
+#pragma unroll
+          for (int part = 0; part < PARTS; ++part) pf[part] = fragment(w[part], kw);
           const int key = sub * 32 + kw * 16 + tr_row;
 #pragma unroll
           for (int dt = 0; dt < 4; ++dt) {
@@ -259,23 +261,24 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
               const char* p = v_lds + kr * 256 + (((dt * 2 + tr_slot) ^ (kr & 7)) << 5) + tr_byte;
               vf.t[rd] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
             }
-            o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.m, ph.m, o_acc[dt], 0, 0, 0);
-            if constexpr (PAGED) o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.m, pl.m, o_acc[dt], 0, 0, 0);
+#pragma unroll
+            for (int part = 0; part < PARTS; ++part)
+              o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.m, pf[part].m, o_acc[dt], 0, 0, 0);
           }
         }
       };
-      uint32_t hi[2][8], lo[2][8];
-      if constexpr (PAGED) {       // one half after the other: the registers of all four parts are not there
+      uint32_t pw[2][PARTS][8];
+      if constexpr (PAGED) {       // one half after the other: the registers of all six parts are not there
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub) {
-          expo(sub, hi[sub], lo[sub]);
-          weighted(sub, hi[sub], lo[sub]);
+          expo(sub, pw[sub]);
+          weighted(sub, pw[sub]);
         }
       } else {
 #pragma unroll
-        for (int sub = 0; sub < 2; ++sub) expo(sub, hi[sub], lo[sub]);
+        for (int sub = 0; sub < 2; ++sub) expo(sub, pw[sub]);
 #pragma unroll
-        for (int sub = 0; sub < 2; ++sub) weighted(sub, hi[sub], lo[sub]);
+        for (int sub = 0; sub < 2; ++sub) weighted(sub, pw[sub]);
       }
     }
     if (more) store_kv(buf ^ 1);

@@ -231,3 +231,33 @@ def test_more_segments_than_a_grid_has_in_y():
         want = ops.attn_segments_paged(q[lo * rows:hi * rows], kc, vc, None, None, 0.1, part, [], tables[lo:hi].contiguous(),
                                        pos[lo:hi])
         assert torch.equal(out[lo * rows:hi * rows], want)
+
+
+@pytest.mark.parametrize("rows", [32, 65, 300])
+@pytest.mark.parametrize("at", [1, 40, 100])          # the second key beside the first, in the other half, in another tile
+def test_segments_against_cache_keep_32_bit_probabilities(at, rows):
+    """Two keys of nearly the same score and V of opposite sign: the result is the difference of their probabilities,
+    2^-14 to 2^-8 of them, and an error of P shows in it at full size."""
+    start, G, rep, BS = 128, 2, 4, 16
+    L, g = start + rows, torch.Generator().manual_seed(rows + at)
+    NB = (L + BS - 1) // BS
+    k, v = torch.zeros(NB * BS, G, D), torch.zeros(NB * BS, G, D)
+    k[..., 0] = -256.0
+    k[0, :, 0], k[at, :, 0], k[at, :, 1] = 1.0, 1.0, -(2.0 ** -4)
+    v[0] = torch.rand(G, D, generator=g).bfloat16().float() + 0.5
+    v[0] = v[0].bfloat16().float()
+    v[at] = -v[0]
+    q = torch.zeros(rows, G * rep, D)
+    q[..., 0] = 1.0
+    q[..., 1] = torch.randint(1, 65, (rows, G * rep), generator=g) * 2.0 ** -10
+    cache = [t.view(NB, BS, G, D).transpose(1, 2).contiguous().bfloat16().to(DEV) for t in (k, v)]
+    bt = torch.arange(NB, dtype=torch.int32, device=DEV).view(1, NB)
+    plan, short = ops.paged_prefill_plan([(start, rows)], DEV)
+    assert plan is not None and not short
+    out = ops.attn_segments_paged(q.bfloat16().to(DEV), *cache, None, None, 1.0, plan, [], bt,
+                                  torch.tensor([start], dtype=torch.int32, device=DEV))
+    p = torch.exp(-(q[..., 1].double() * 2.0 ** -4)).unsqueeze(-1)
+    size = v[0].double().repeat_interleave(rep, 0)
+    ref = (1 - p) / (1 + p) * size
+    # the result's rounding to bf16, and four of 2^-24 in P and its sum
+    assert ((out.double().cpu() - ref).abs() <= 2 ** -8 * ref.abs() + 4 * 2 ** -24 * size).all()
