@@ -313,7 +313,8 @@ class LlamaForCausalLM(nn.Module):
                                     input_ids.shape[0])
             return replace(batch, plans={**(batch.plans or {}), "prefill": plan})
         if (batch.host_segs is not None and batch.seg_tables is not None and self.dtype == torch.bfloat16
-                and self.layers and self.layers[0].self_attn.head_dim == 128):
+                and self.layers and self.layers[0].self_attn.head_dim == 128
+                and ops.paged_prefill_pays(batch.host_segs, self.layers[0].self_attn.num_kv_heads)):
             plan, short = ops.paged_prefill_plan(batch.host_segs, input_ids.device)
             if plan is not None:
                 return replace(batch, plans={**(batch.plans or {}), "paged": (plan, short)})

@@ -139,8 +139,23 @@ def attn_prefill_varlen(
     return torch_ref.attn_prefill_varlen(q, k, v, cu_seqlens, scale)
 
 
-# segments shorter than this attend row by row: a workgroup of the paged prefill kernel has eight 32-row tiles
+# segments shorter than this attend row by row: a workgroup of the paged prefill kernel has eight 32-row tiles. Around
+# the line, 12 segments behind 3000 keys (32 heads, 8 kv heads), paged 190 us; row by row 169 for 16 rows each, 248 for 24,
+# 327 for 31
 PAGED_PREFILL_ROWS = 32
+# A group of up to 256 rows is one workgroup a head, so a step of few groups takes as long as its longest group's keys,
+# one tile after another: 30 ns a key up to 160 rows, 50 above. Row by row every compute unit is busy, 0.03 to 0.05 ns for
+# each row, key and kv head. So the rows have to make 750 row-heads of the longest segment's keys. 32 heads, 8 kv heads, one
+# segment behind 6000 keys: 32 rows 184 us paged, 68 row by row; 64 rows 188, 123; 128 rows 189, 227; four of 32 rows
+# 181, 239. 4 kv heads: 64 rows 188, 93; 256 rows 299, 282; two of 128 193, 286. 32 kv heads, 32 rows behind 3000: 100, 116.
+PAGED_PREFILL_WORK = 750
+
+
+def paged_prefill_pays(segs, kv_heads: int) -> bool:
+    """Whether the long ones of the segments [(start position, rows)] attend together (paged_prefill_plan) or row by
+    row like the short ones."""
+    long = [(start + n, n) for start, n in segs if n >= PAGED_PREFILL_ROWS]
+    return bool(long) and kv_heads * sum(k * n for k, n in long) >= PAGED_PREFILL_WORK * max(k for k, _ in long)
 
 
 def paged_prefill_plan(segs, device) -> tuple:

@@ -1,0 +1,52 @@
+"""Which prompt portions behind a cache attend together on the matrix cores, and which row by row."""
+
+import pytest
+
+from kllms_amd import ops
+
+
+@pytest.mark.parametrize("segs,kv_heads,pays", [
+    ([], 8, False),
+    ([(500, 1)] * 40, 8, False),                    # decode rows
+    ([(3000, 31)] * 12, 8, False),                  # short segments only
+    ([(0, 32)], 8, False), ([(6000, 32)], 8, False), ([(6000, 64)], 8, False),   # too few workgroups for the keys
+    ([(6000, 94)], 8, True), ([(500, 128)], 8, True), ([(2000, 64)] * 2, 8, True), ([(6000, 32)] * 4, 8, True),
+    ([(6000, 128)], 4, False), ([(6000, 188)], 4, True), ([(3000, 32)], 32, True), ([(300, 64)] * 4, 1, False),
+    ([(6000, 40), (10, 300)], 8, False),            # a long context with few rows beside many rows of a short one
+    ([(6000, 40), (10, 300), (5000, 80)], 8, True),
+    ([(1536, 150)] * 8, 8, True),
+])
+def test_rule(segs, kv_heads, pays):
+    assert ops.paged_prefill_pays(segs, kv_heads) is pays
+
+
+def test_one_short_portion_behind_a_long_cache_goes_row_by_row(monkeypatch):
+    """The model asks the rule: a step of one 32-row portion has no plan, one of eight has."""
+    import torch
+
+    from kllms_amd.models.llama import ForwardBatch, LlamaForCausalLM
+
+    model = LlamaForCausalLM.__new__(LlamaForCausalLM)
+    torch.nn.Module.__init__(model)
+    model.dtype = torch.bfloat16
+
+    class Attn:
+        head_dim, num_kv_heads = 128, 8
+
+    class Layer(torch.nn.Module):
+        self_attn = Attn
+
+    model.layers = torch.nn.ModuleList([Layer()])
+    monkeypatch.setattr(ops, "_force_torch", lambda: False)
+    monkeypatch.setattr(ops, "paged_prefill_plan", lambda segs, device: ("plan", []))
+
+    class Ids:
+        is_cuda, device = True, "cpu"
+
+    def planned(segs):
+        batch = ForwardBatch(mode="decode", positions=None, slot_mapping=None, kv_caches=None, host_segs=segs,
+                             seg_tables=torch.zeros(len(segs), 1))
+        return (LlamaForCausalLM._planned(model, Ids, batch).plans or {}).get("paged")
+
+    assert planned([(6000, 32)]) is None
+    assert planned([(1536, 150)] * 8) == ("plan", [])
