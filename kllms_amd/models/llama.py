@@ -261,9 +261,18 @@ class LlamaForCausalLM(nn.Module):
         return mod
 
     # --- forward ------------------------------------------------------------
-    # the fused [gate; up] product of more rows than this is the library's: at 128 rows of 28672 x 4096 it takes 57 us
-    # and 5 for the activation, the few-row kernel 68 (its reads of x grow with the rows), at 64 rows 54 + 5 against 57
+    # rows up to which the fused [gate; up] product is the few-row kernel's, by the weights' size. It saves the
+    # activation's launch, 5 us; the library streams large matrices faster (5.3 TB/s against 4.2 - 5.0) and reads x less.
+    # us, library with activation and few-row kernel, at 1 / 16 / 32 / 64 rows:
+    #   28672 x 4096  63 51 / 64 53 / 59 55 / 57 60 (68 for 57 + 5 at 128)
+    #   27648 x 5120  73 60 / 75 62 / 55 67 / 60 73
+    #   57344 x 8192  178 187 / 175 191 / 174 194 / 184 191
     SILU_ROWS_MAX = 64
+
+    @classmethod
+    def _silu_rows(cls, rows: int, weight: torch.Tensor) -> bool:
+        n = weight.numel()
+        return rows <= (cls.SILU_ROWS_MAX if n < 1 << 27 else 16 if n < 1 << 28 else 0)
 
     def _takes_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> bool:
         """Whether a step runs as _forward_rows: a few decode rows of an unsharded bf16 model on the GPU with the
@@ -294,7 +303,7 @@ class LlamaForCausalLM(nn.Module):
             norm = layers[i + 1].input_layernorm if i + 1 < len(layers) else self.norm
             mlp = layer.mlp
             if isinstance(mlp, LlamaMLP):
-                if T <= self.SILU_ROWS_MAX:
+                if self._silu_rows(T, mlp.gate_up_proj.weight):
                     act = ops.linear_silu_rows(x, mlp.gate_up_proj.weight)
                 else:
                     gate, up = mlp.gate_up_proj(x).split([mlp._i, mlp._i], dim=-1)

@@ -1,4 +1,5 @@
-"""Which prompt portions behind a cache attend together on the matrix cores, and which row by row."""
+"""Rules that choose between two forms of a call: which prompt portions behind a cache attend together on the matrix
+cores, which steps take the few-row [gate; up] product."""
 
 import pytest
 
@@ -16,7 +17,7 @@ from kllms_amd import ops
     ([(6000, 40), (10, 300), (5000, 80)], 8, True),
     ([(1536, 150)] * 8, 8, True),
 ])
-def test_rule(segs, kv_heads, pays):
+def test_portions(segs, kv_heads, pays):
     assert ops.paged_prefill_pays(segs, kv_heads) is pays
 
 
@@ -50,3 +51,13 @@ def test_one_short_portion_behind_a_long_cache_goes_row_by_row(monkeypatch):
 
     assert planned([(6000, 32)]) is None
     assert planned([(1536, 150)] * 8) == ("plan", [])
+
+
+@pytest.mark.parametrize("shape,most", [((1024, 512), 64), ((28672, 4096), 64), ((27648, 5120), 16), ((57344, 8192), 0)])
+def test_gate_up_product(shape, most):
+    import torch
+
+    from kllms_amd.models.llama import LlamaForCausalLM
+
+    w = torch.empty(shape, dtype=torch.bfloat16, device="meta")
+    assert [LlamaForCausalLM._silu_rows(r, w) for r in (1, 16, 17, 64, 65)] == [r <= most for r in (1, 16, 17, 64, 65)]
