@@ -1,4 +1,4 @@
-// Sampling + logprob for gfx950, in two launches.
+// Sampling + logprob for gfx950, in two launches (one for short rows).
 //
 //   sample_part   every row cut into slices, one 256-thread workgroup each: the
 //                 slice's max and argmax, its sum of exp, and - for rows
@@ -110,41 +110,29 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
   return v;
 }
 
-extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
-    SlicePart* __restrict__ parts,        // [B, slices]
-    const float* __restrict__ logits,     // [B, V]
-    const float* __restrict__ temperatures, const float* __restrict__ top_ps,
-    const int* __restrict__ top_ks, const int64_t* __restrict__ seeds,
-    const int64_t* __restrict__ steps,
-    const uint32_t* __restrict__ mask,    // [B, ceil(V/32)] or nullptr
-    int V, int slice) {
-  const int b = blockIdx.y;
+// tokens [lo, hi) of a row by a workgroup of THREADS; the result is thread 0's
+template <int THREADS>
+__device__ __forceinline__ SlicePart slice_part(const float* __restrict__ row, const uint32_t* __restrict__ mrow,
+                                                float temp, bool cuts, uint64_t base, int lo, int hi) {
   const int tid = threadIdx.x;
-  const int lo = blockIdx.x * slice;
-  const int hi = min(V, lo + slice);
-  const float* row = logits + (int64_t)b * V;
-  const uint32_t* mrow = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
-  const float temp = temperatures[b];
-  const bool cuts = temp != 0.0f && truncates(top_ps[b], top_ks[b], V);
   const bool draw = temp != 0.0f && !cuts;
   const float inv_t = (temp > 0.0f) ? 1.0f / temp : 0.0f;
-  const uint64_t base = draw_base(seeds[b], steps[b]);
 
   float m = -INFINITY, sum = 0.0f, ssum = 0.0f, best = -INFINITY;
   int arg = -1, btok = 0;
-  for (int i0 = lo + tid; i0 < hi; i0 += PT * PU) {
+  for (int i0 = lo + tid; i0 < hi; i0 += THREADS * PU) {
     float x[PU];
     bool ok[PU];
 #pragma unroll
     for (int j = 0; j < PU; ++j) {
-      const int i = i0 + j * PT;
+      const int i = i0 + j * THREADS;
       ok[j] = i < hi;
       x[j] = ok[j] ? row[i] : -INFINITY;
     }
     if (mrow) {
 #pragma unroll
       for (int j = 0; j < PU; ++j) {
-        const int i = i0 + j * PT;
+        const int i = i0 + j * THREADS;
         if (ok[j]) ok[j] = (mrow[i >> 5] >> (i & 31)) & 1;
         if (!ok[j]) x[j] = -INFINITY;
       }
@@ -158,7 +146,7 @@ extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
       m = cm;
 #pragma unroll
       for (int j = PU - 1; j >= 0; --j)
-        if (x[j] == cm) arg = i0 + j * PT;
+        if (x[j] == cm) arg = i0 + j * THREADS;
     }
 #pragma unroll
     for (int j = 0; j < PU; ++j) sum += exp_from(x[j], m);
@@ -171,43 +159,63 @@ extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
 #pragma unroll
       for (int j = 0; j < PU; ++j) {
         if (!ok[j]) continue;
-        const float key = draw_key(base, i0 + j * PT, x[j], inv_t);
-        if (key > best) { best = key; btok = i0 + j * PT; }
+        const float key = draw_key(base, i0 + j * THREADS, x[j], inv_t);
+        if (key > best) { best = key; btok = i0 + j * THREADS; }
       }
     }
   }
 
   // fold the threads: max, lowest token at it, rescaled sums, best key
   __shared__ float red[16];
-  __shared__ unsigned long long sh_best[PT / WAVE];
-  __shared__ int sh_arg[PT / WAVE];
-  const float M = block_reduce_max<PT / WAVE>(m, red);
-  const float S = block_reduce_sum<PT / WAVE>(sum * (m == M ? 1.0f : exp_from(m, M)), red);
-  const float SS = cuts ? block_reduce_sum<PT / WAVE>(ssum * (m == M ? 1.0f : __expf((m - M) * inv_t)), red) : 0.0f;
+  __shared__ unsigned long long sh_best[THREADS / WAVE];
+  __shared__ int sh_arg[THREADS / WAVE];
+  const float M = block_reduce_max<THREADS / WAVE>(m, red);
+  const float S = block_reduce_sum<THREADS / WAVE>(sum * (m == M ? 1.0f : exp_from(m, M)), red);
+  const float SS = cuts ? block_reduce_sum<THREADS / WAVE>(ssum * (m == M ? 1.0f : __expf((m - M) * inv_t)), red) : 0.0f;
   int a = (m == M && arg >= 0) ? arg : 0x7fffffff;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) a = min(a, __shfl_xor(a, off));
   const unsigned long long w = wave_max_u64(pack_key(best, btok));
   if ((tid & 63) == 0) { sh_best[tid >> 6] = w; sh_arg[tid >> 6] = a; }
   __syncthreads();
+  SlicePart p;
   if (tid == 0) {
-    SlicePart p;
     p.max = M;
     p.sum = S;
     p.best = sh_best[0];
     p.arg = sh_arg[0];
 #pragma unroll
-    for (int k = 1; k < PT / WAVE; ++k) {
+    for (int k = 1; k < THREADS / WAVE; ++k) {
       p.best = sh_best[k] > p.best ? sh_best[k] : p.best;
       p.arg = min(p.arg, sh_arg[k]);
     }
     if (p.arg == 0x7fffffff) p.arg = -1;
     p.ssum = SS;
-    parts[(int64_t)b * gridDim.x + blockIdx.x] = p;
   }
+  return p;
 }
 
-extern "C" __global__ void __launch_bounds__(NT) sample_final_kernel(
+extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
+    SlicePart* __restrict__ parts,        // [B, slices]
+    const float* __restrict__ logits,     // [B, V]
+    const float* __restrict__ temperatures, const float* __restrict__ top_ps,
+    const int* __restrict__ top_ks, const int64_t* __restrict__ seeds,
+    const int64_t* __restrict__ steps,
+    const uint32_t* __restrict__ mask,    // [B, ceil(V/32)] or nullptr
+    int V, int slice) {
+  const int b = blockIdx.y;
+  const int lo = blockIdx.x * slice;
+  const float temp = temperatures[b];
+  const SlicePart p = slice_part<PT>(logits + (int64_t)b * V, mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr, temp,
+                                     temp != 0.0f && truncates(top_ps[b], top_ks[b], V), draw_base(seeds[b], steps[b]),
+                                     lo, min(V, lo + slice));
+  if (threadIdx.x == 0) parts[(int64_t)b * gridDim.x + blockIdx.x] = p;
+}
+
+
+// WHOLE: a short row's only launch, one slice of all its tokens
+template <bool WHOLE>
+__global__ void __launch_bounds__(NT) sample_final_kernel(
     int64_t* __restrict__ out_tokens,     // [B]
     float* __restrict__ out_logprobs,     // [B]
     const SlicePart* __restrict__ parts,  // [B, slices], slices <= 64
@@ -234,7 +242,17 @@ extern "C" __global__ void __launch_bounds__(NT) sample_final_kernel(
   __shared__ float sh_max, sh_sum, sh_ssum;
   __shared__ int sh_argmax;
   __shared__ unsigned long long sh_best;
-  if (wid == 0) {
+  if constexpr (WHOLE) {
+    const SlicePart p = slice_part<NT>(row, mrow, temp, temp != 0.0f && truncates(top_p, top_k, V),
+                                       draw_base(seeds[b], steps[b]), 0, V);
+    if (tid == 0) {
+      sh_max = p.max;
+      sh_sum = p.sum;
+      sh_ssum = p.ssum;
+      sh_argmax = p.arg < 0 ? 0 : p.arg;
+      sh_best = p.best;
+    }
+  } else if (wid == 0) {
     SlicePart p{-INFINITY, 0.0f, -1, 0.0f, (unsigned long long)NO_KEY << 32};
     if (lane < slices) p = parts[(int64_t)b * slices + lane];
     const float M = wave_reduce_max(p.max);
@@ -589,8 +607,11 @@ extern "C" __global__ void __launch_bounds__(NT) sample_final_kernel(
 
 // rows -> slices: about eight 256-thread workgroups per compute unit, no slice
 // under 2048 tokens (one load round per thread) and at most 64 slices a row (one
-// per lane of sample_final's fold)
+// per lane of sample_final's fold). 0: rows of up to 4096 tokens, half a load round of
+// sample_final's workgroup, take its launch alone: called from Python 9.0 us against 12.5
+// for any number of rows of 300 to 4000 tokens, in a graph 6 to 8 against 8 to 9.5
 extern "C" int sample_slices(int B, int V) {
+  if (V <= 4 * NT) return 0;
   const int most = (V + PT * PU - 1) / (PT * PU);
   const int want = (2048 + B - 1) / B;
   const int n = want < most ? want : most;
@@ -602,17 +623,18 @@ extern "C" void launch_sample(int64_t* tokens, float* logprobs, void* parts, con
                               const int64_t* seeds, const int64_t* steps, const uint32_t* mask, int B,
                               int V, float* dbg, hipStream_t stream) {
   const int n = sample_slices(B, V);
-  const int slice = (V + n - 1) / n;
+  const int slice = n > 0 ? (V + n - 1) / n : V;
   // rows of a launch lie on the grid's y, which ends at 65535
   for (int b = 0; b < B; b += 65535) {
     const int rows = B - b < 65535 ? B - b : 65535;
     SlicePart* p = (SlicePart*)parts + (int64_t)b * n;
     const float* x = logits + (int64_t)b * V;
     const uint32_t* m = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
-    hipLaunchKernelGGL(sample_part_kernel, dim3(n, rows), dim3(PT), 0, stream, p, x, temps + b, top_ps + b,
-                       top_ks + b, seeds + b, steps + b, m, V, slice);
-    hipLaunchKernelGGL(sample_final_kernel, dim3(rows), dim3(NT), 0, stream, tokens + b, logprobs + b,
-                       (const SlicePart*)p, n, x, temps + b, top_ps + b, top_ks + b, seeds + b, steps + b, m, V,
-                       dbg ? dbg + (int64_t)b * 16 : nullptr);
+    if (n > 0)
+      hipLaunchKernelGGL(sample_part_kernel, dim3(n, rows), dim3(PT), 0, stream, p, x, temps + b, top_ps + b,
+                         top_ks + b, seeds + b, steps + b, m, V, slice);
+    hipLaunchKernelGGL(n > 0 ? sample_final_kernel<false> : sample_final_kernel<true>, dim3(rows), dim3(NT), 0, stream,
+                       tokens + b, logprobs + b, (const SlicePart*)p, n, x, temps + b, top_ps + b, top_ks + b,
+                       seeds + b, steps + b, m, V, dbg ? dbg + (int64_t)b * 16 : nullptr);
   }
 }

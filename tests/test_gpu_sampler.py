@@ -169,3 +169,24 @@ def test_top_p_cut_does_not_move(V, temp):
         t, p = ops.sample(*(a[:n] for a in args))
         # the slices' sums in another order: a few fp32 roundings of each level of their tree
         assert torch.equal(t, toks[:n]) and torch.allclose(p, lps[:n], rtol=0, atol=2e-6)
+
+
+@pytest.mark.parametrize("mode", ["plain", "greedy", "masked", "top_k", "top_p", "both", "crowded"])
+@pytest.mark.parametrize("B,V", [(3, 64), (2, 1023), (2, 1025), (40, 4095), (3, 4096), (3, 4097)])
+def test_short_rows_in_one_launch(B, V, mode):
+    """Rows around the length up to which one workgroup does a whole row."""
+    test_draw_matches_float64(B, V, mode)
+
+
+def test_short_rows_without_an_allowed_token():
+    """Nothing allowed, or nothing above -inf: token 0, as in longer rows."""
+    for V in (70, 5000):
+        logits = torch.randn(3, V, device=DEV)
+        logits[1:] = -torch.inf
+        mask = torch.full((3, (V + 31) // 32), -1, dtype=torch.int32, device=DEV)
+        mask[0] = 0
+        for p, k in ((1.0, 0), (0.9, 0), (1.0, 5)):
+            toks, _ = ops.sample(logits, torch.ones(3, device=DEV), torch.full((3,), p, device=DEV),
+                                 torch.full((3,), k, dtype=torch.int32, device=DEV), torch.arange(3, device=DEV),
+                                 torch.zeros(3, dtype=torch.long, device=DEV), mask)
+            assert toks.tolist() == [0, 0, 0]
