@@ -484,7 +484,7 @@ def attn_varlen_mfma(out, q, k, v, grp_start, grp_qpos0, grp_len, scale) -> None
 
 def dense_tile_groups(pieces, device):
     """Host metadata for attn_varlen_mfma: pieces = [(first row, length)];
-    32-row q-tiles of each piece, 8 in a row per workgroup (idle wave slots = -1)."""
+    32-row q-tiles of each piece, 8 per workgroup (idle wave slots = -1)."""
     NW = 8
     gs, gl, gq = [], [], []
     for row0, L in pieces:

@@ -64,7 +64,8 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
     const bf16_t* __restrict__ v,
     const int* __restrict__ grp_start,   // [G] first row of the group's sequence
     const int* __restrict__ grp_len,     // [G] rows of the sequence, 0: idle group
-    const int* __restrict__ grp_q0,      // [G * q0_stride] group's first row within the sequence
+    const int* __restrict__ grp_q0,      // q0_stride 1: [G] group's first row within the sequence, its waves' 32 rows
+                                         // following; 8: [G, 8] first row of each wave, -1: none
     const int* __restrict__ grp_seg,     // PAGED: [G] row of block_tables / seg_pos
     const int* __restrict__ block_tables, const int* __restrict__ seg_pos,  // PAGED: position of a segment's row 0
     float scale, int num_kv_heads, int q_tstride, int kv_tstride, int q0_stride, int block_size, int max_blocks) {
@@ -79,16 +80,28 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
   const int col = lane & 31;       // q-row (B/C col) or K row / V^T row (A row)
 
   const int seqlen = grp_len[grp];
-  const int q0 = grp_q0[grp * q0_stride];
-  if (seqlen <= 0 || q0 >= seqlen) return;
+  int qrow0, rows_end = 0;         // this wave's first row; behind the group's last one
+  if (PAGED || q0_stride == 1) {
+    const int q0 = grp_q0[grp];
+    qrow0 = q0 + wave * QBLK;
+    rows_end = min(seqlen, q0 + NWAVES * QBLK);
+    if (q0 >= seqlen) return;
+  } else {
+    qrow0 = grp_q0[grp * NWAVES + wave];
+#pragma unroll
+    for (int w = 0; w < NWAVES; ++w) {
+      const int r = grp_q0[grp * NWAVES + w];
+      if (r >= 0 && r < seqlen) rows_end = max(rows_end, min(seqlen, r + QBLK));
+    }
+  }
+  if (seqlen <= 0 || rows_end <= 0) return;
   const int seq_start = grp_start[grp];
   const int seg = PAGED ? grp_seg[grp] : 0;
   const int pos0 = PAGED ? seg_pos[seg] : 0;          // keys before the sequence's first row
-  const int qrow0 = q0 + wave * QBLK;
-  const bool active = qrow0 < seqlen;
+  const bool active = qrow0 >= 0 && qrow0 < seqlen;
   const int my_pos = pos0 + qrow0 + col;
   // keys visible to the group's last row, and to this wave's
-  const int kv_end_grp = pos0 + min(seqlen, q0 + NWAVES * QBLK);
+  const int kv_end_grp = pos0 + rows_end;
   const int kv_end_me = active ? pos0 + min(seqlen, qrow0 + QBLK) : 0;
 
   __shared__ __attribute__((aligned(16))) char smem[2][2 * TILE_BYTES];  // [buffer][K | V]
@@ -97,7 +110,7 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
   union QFrag { u32x4 u; bf16x8_mfma m; };
   QFrag q_frag[8];
   {
-    const int row = min(qrow0 + col, seqlen - 1);
+    const int row = active ? min(qrow0 + col, seqlen - 1) : 0;
     const short* qp = (const short*)q + (int64_t)(seq_start + row) * q_tstride + h * DHEAD + half * 8;
     // a negative scale goes into Q's signs: the max below is taken before scaling
     const uint32_t sign = scale < 0.0f ? 0x80008000u : 0u;

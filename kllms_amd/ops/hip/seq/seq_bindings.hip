@@ -503,7 +503,6 @@ void attn_varlen_mfma(torch::Tensor out, torch::Tensor q, torch::Tensor k, torch
   const int ngroups = grp_start.numel();
   TORCH_CHECK(grp_qpos0.numel() == (int64_t)ngroups * 8 && grp_len.numel() == ngroups);
   if (ngroups == 0) return;
-  // a group's tiles follow one another: its first one says where it begins
   launch_attn_prefill((__hip_bfloat16*)out.data_ptr(), (const __hip_bfloat16*)q.data_ptr(),
                       (const __hip_bfloat16*)k.data_ptr(), (const __hip_bfloat16*)v.data_ptr(),
                       grp_start.data_ptr<int>(), grp_len.data_ptr<int>(), grp_qpos0.data_ptr<int>(), 8, ngroups,

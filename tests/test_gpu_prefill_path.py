@@ -261,3 +261,35 @@ def test_segments_against_cache_keep_32_bit_probabilities(at, rows):
     ref = (1 - p) / (1 + p) * size
     # the result's rounding to bf16, and four of 2^-24 in P and its sum
     assert ((out.double().cpu() - ref).abs() <= 2 ** -8 * ref.abs() + 4 * 2 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("H,G", [(4, 4), (8, 2)])
+@pytest.mark.parametrize("seed", range(4))
+def test_packed_tiles_in_any_order(H, G, seed):
+    """Tile tables of attn_varlen_mfma that dense_tile_groups does not make: a group's waves take tiles from anywhere in
+    their piece, with idle ones between them, and rows that begin between tiles."""
+    g = torch.Generator().manual_seed(seed)
+    pieces = [(0, 300), (300, 31), (331, 700)]
+    T = 1031
+    q, k, v = (torch.randn(T, n, D, generator=g).bfloat16().to(DEV) for n in (H, G, G))
+    gs, gl, gq, want = [], [], [], torch.zeros(T, dtype=torch.bool)
+    for row0, n in pieces:
+        tiles = [t for t in torch.randperm((n + 31) // 32, generator=g).tolist() if t % 5 != seed]
+        first = [t * 32 for t in tiles] + ([n - 7, 3] if n > 40 else [])
+        for f in first:
+            want[row0 + f:row0 + min(n, f + 32)] = True
+        while first:
+            slots = [-1] * 8
+            for w in torch.randperm(8, generator=g).tolist()[:5]:
+                if first:
+                    slots[w] = first.pop()
+            gs.append(row0), gl.append(n), gq.extend(slots)
+    gs.append(0), gl.append(300), gq.extend([-1] * 8)               # a group without work
+    t = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    out = torch.full((T, H, D), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.attn_varlen_mfma(out, q, k, v, t(gs), t(gq), t(gl), D ** -0.5)
+    for row0, n in pieces:
+        at = torch.arange(row0, row0 + n)[want[row0:row0 + n]]
+        ref, size = causal64(q[row0:row0 + n].cpu(), k[row0:row0 + n].cpu(), v[row0:row0 + n].cpu(), D ** -0.5, 0)
+        check(out[at.to(DEV)], ref[(at - row0).to(DEV)], size[(at - row0).to(DEV)])
+    assert (out[~want.to(DEV)] == 7.0).all()
