@@ -238,7 +238,8 @@ def linear_rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     return (x.is_cuda and not _force_torch() and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
             and 1 <= x.shape[0] <= LINEAR_ROWS_MAX and x.shape[1] % 128 == 0 and w.shape[0] % 16 == 0
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
-            and w.is_contiguous() and w.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and x.requires_grad))
+            and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
 
 
 def linear_part(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -301,3 +301,29 @@ def test_blocklocal_rows_keep_32_bit_exponentials(L, gqa):
     # the rounding to bf16, and about ten 32-bit ones of 2^-24 before it (exponentials, fold, divisions, gate)
     half = 2.0 ** (torch.floor(torch.log2(ref.abs())) - 8)
     assert ((out.double().cpu() - ref).abs() <= half + 10 * 2 ** -24 * ref.abs()).all()
+
+
+def test_logits_keep_the_heads_gradient_and_bias():
+    """A trainable LM head, or one with a bias, is not the few-row kernel's: it has neither."""
+    from kllms_amd.engine.config import MODEL_PRESETS
+    from kllms_amd.models.llama import LlamaForCausalLM
+
+    with torch.device(DEV):
+        model = LlamaForCausalLM(MODEL_PRESETS["mid-llama"])
+    g = torch.Generator(device=DEV).manual_seed(0)
+    w = model.lm_head.weight
+    w.data.normal_(0, 0.02, generator=g)
+    h = torch.randn(5, w.shape[1], generator=g, device=DEV).bfloat16()
+    want = h.double() @ w.double().t()
+    tol = 2 ** -8 * want.abs() + 1e-3                  # the library rounds to bf16
+    w.requires_grad_(True)
+    out = model.compute_logits(h)
+    out.sum().backward()
+    assert ((out.double() - want).abs() <= tol).all()
+    # the gradient of every row is the sum of h, summed in 32 bits or more and rounded to bf16
+    assert torch.allclose(w.grad.double(), h.double().sum(0).expand_as(w), rtol=2 ** -8, atol=1e-4)
+    with torch.no_grad():
+        assert not model.compute_logits(h).requires_grad
+        model.lm_head.bias = torch.nn.Parameter(torch.randn(w.shape[0], generator=g, device=DEV).bfloat16())
+        full = want + model.lm_head.bias.double()
+        assert ((model.compute_logits(h).double() - full).abs() <= 2 ** -8 * full.abs() + 1e-3).all()
