@@ -283,8 +283,8 @@ class LlamaForCausalLM(nn.Module):
                 and 1 <= input_ids.shape[0] <= ops.LINEAR_ROWS_MAX and self.ctx.world_size == 1
                 and self.dtype == torch.bfloat16 and not ops._force_torch() and at.head_dim == 128
                 and cfg.hidden_size % 128 == 0 and cfg.hidden_size <= 16384 and cfg.intermediate_size % 128 == 0
-                and self.cos_sin.is_contiguous() and input_ids.is_contiguous() and batch.positions.is_contiguous()
-                and batch.slot_mapping.is_contiguous())
+                and self.cos_sin.is_contiguous() and input_ids.is_contiguous()
+                and all(t.is_contiguous() and t.numel() == input_ids.shape[0] for t in (batch.positions, batch.slot_mapping)))
 
     def _forward_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
         """A decode step: weights streamed by the few-row kernel, whose split sums go straight into the next row-wise

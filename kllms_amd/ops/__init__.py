@@ -108,9 +108,11 @@ def rope_store(q, k, v, positions, cos_sin, k_cache, v_cache, slot_mapping, k_sc
             and q.shape[2] == 128 and k.stride(0) == v.stride(0)
             and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 and t.stride(2) == 1 and t.stride(1) == 128
                     for t in (q, k, v))
-            and all(t.dtype == torch.long and t.is_contiguous() for t in (positions, slot_mapping))
+            and all(t.dtype == torch.long and t.is_contiguous() and t.dim() == 1 for t in (positions, slot_mapping))
             and cos_sin.is_contiguous() and k_cache.dtype == v_cache.dtype):
         none = _none(k, torch.float32)
+        if positions.shape[0] != q.shape[0] or slot_mapping.shape[0] != q.shape[0]:      # the rows at their head
+            positions, slot_mapping = positions[:q.shape[0]], slot_mapping[:q.shape[0]]
         _hip_or_raise().rope_store(q, k, v, positions, cos_sin, k_cache, v_cache, slot_mapping,
                                    k_scale if k_scale is not None else none, v_scale if v_scale is not None else none)
         return

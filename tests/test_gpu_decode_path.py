@@ -327,3 +327,27 @@ def test_logits_keep_the_heads_gradient_and_bias():
         model.lm_head.bias = torch.nn.Parameter(torch.randn(w.shape[0], generator=g, device=DEV).bfloat16())
         full = want + model.lm_head.bias.double()
         assert ((model.compute_logits(h).double() - full).abs() <= 2 ** -8 * full.abs() + 1e-3).all()
+
+
+@pytest.mark.parametrize("rows", [3, 70])
+def test_decode_step_takes_the_head_of_longer_rows(rows):
+    """A decode step whose positions and slots lie in larger buffers gives what their heads give."""
+    from dataclasses import replace
+
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+    from kllms_amd.models.llama import ForwardBatch
+
+    eng = LLMEngine(EngineConfig(model="mid-llama", max_kv_blocks=512, use_hip_graphs=False, seed=3))
+    eng.kv.k_all.normal_(), eng.kv.v_all.normal_()
+    ctx = torch.arange(rows) % 15 + 1
+    bt = torch.arange(1, rows + 1, dtype=torch.int32).view(rows, 1)
+    pad = torch.zeros(5, dtype=torch.long)
+    batch = ForwardBatch(mode="decode", positions=torch.cat([ctx - 1, pad]).to(DEV),
+                         slot_mapping=torch.cat([bt[:, 0] * 16 + ctx - 1, pad]).to(DEV), kv_caches=eng.kv.layer_caches(),
+                         block_tables=bt.to(DEV), context_lens=ctx.to(torch.int32).to(DEV))
+    exact = replace(batch, positions=batch.positions[:rows].clone(), slot_mapping=batch.slot_mapping[:rows].clone())
+    ids = torch.arange(rows, device=DEV)
+    with torch.inference_mode():
+        a, b = (eng.model.forward_decode(ids, x) for x in (batch, exact))
+    assert float(((a - b).norm(dim=-1) / b.norm(dim=-1)).max()) < 0.03     # bf16 through two layers, two sets of kernels

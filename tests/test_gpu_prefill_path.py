@@ -293,3 +293,22 @@ def test_packed_tiles_in_any_order(H, G, seed):
         ref, size = causal64(q[row0:row0 + n].cpu(), k[row0:row0 + n].cpu(), v[row0:row0 + n].cpu(), D ** -0.5, 0)
         check(out[at.to(DEV)], ref[(at - row0).to(DEV)], size[(at - row0).to(DEV)])
     assert (out[~want.to(DEV)] == 7.0).all()
+
+
+def test_rope_store_takes_the_head_of_longer_rows():
+    """Positions and slots of a larger buffer: its first T entries, as the two kernels take them; too few are refused."""
+    T, H, G = 40, 4, 2
+    g = torch.Generator(device=DEV).manual_seed(1)
+    rows = torch.randn(T, H + 2 * G, D, generator=g, device=DEV).bfloat16()
+    pos, slots = torch.arange(T + 9, device=DEV), torch.randperm(64, generator=g, device=DEV)
+    cs = torch.randn(64, D, generator=g, device=DEV)
+    got = []
+    for p, s in ((pos, slots), (pos[:T].clone(), slots[:T].clone())):
+        q, k, v = rows.clone().split([H, G, G], 1)
+        kc, vc = (torch.zeros(4, G, 16, D, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        ops.rope_store(q, k, v, p, cs, kc, vc, s)
+        got.append((q.clone(), k.clone(), kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    q, k, v = rows.split([H, G, G], 1)
+    with pytest.raises(RuntimeError):
+        ops.rope_store(q, k, v, pos[:T - 1], cs, kc, vc, slots)
