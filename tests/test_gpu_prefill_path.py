@@ -312,3 +312,22 @@ def test_rope_store_takes_the_head_of_longer_rows():
     q, k, v = rows.split([H, G, G], 1)
     with pytest.raises(RuntimeError):
         ops.rope_store(q, k, v, pos[:T - 1], cs, kc, vc, slots)
+
+
+@pytest.mark.parametrize("rows", [[40, 20], [150, 1, 33], [300]])
+def test_step_segments_together_matches_row_by_row(rows, monkeypatch):
+    """The step of test_step_segments_matches_row_by_row with its long portions on the paged prefill kernel, which the
+    rule on rows and keys would not choose for a model of two kv heads."""
+    from kllms_amd.models.llama import LlamaForCausalLM
+
+    monkeypatch.setattr(ops, "PAGED_PREFILL_WORK", 0)
+    plans, make = [], LlamaForCausalLM._planned
+
+    def planned(self, ids, batch):
+        batch = make(self, ids, batch)
+        plans.append((batch.plans or {}).get("paged"))
+        return batch
+
+    monkeypatch.setattr(LlamaForCausalLM, "_planned", planned)
+    test_step_segments_matches_row_by_row(rows)
+    assert plans[-1] is not None and plans[-1][0] is not None
