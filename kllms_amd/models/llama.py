@@ -342,10 +342,17 @@ class LlamaForCausalLM(nn.Module):
         return hidden
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        # up to 64 rows 57 - 65 us for 32000 x 4096 against the library's 60 - 65 with 5 for the cast; 79 against 63 at 128
-        if (hidden.dim() == 2 and hidden.shape[0] <= 64 and self.lm_head.bias is None
-                and ops.linear_rows_ok(hidden, self.lm_head.weight)):
-            return ops.linear_f32_rows(hidden, self.lm_head.weight)
+        """fp32 [rows, V]. On the GPU the fp32 sums of the bf16 product at every row count: rounded to bf16 at some counts
+        only, near ties between tokens would fall differently as a stream's batch grows."""
+        w = self.lm_head.weight
+        if (hidden.dim() == 2 and hidden.is_cuda and hidden.dtype == w.dtype == torch.bfloat16 and not ops._force_torch()
+                and self.lm_head.bias is None and not (torch.is_grad_enabled() and (hidden.requires_grad or w.requires_grad))):
+            # us, the library and the few-row kernel, weights out of cache, at 1 / 32 / 64 / 128 rows:
+            #   32000 x 4096   59 55 / 59 58 / 61 62 / 63 71        128256 x 2048  121 99 / 127 114 / 135 124 / 149 143
+            #   128256 x 4096  188 193 / 209 215 / 224 230 / 250 261
+            if hidden.shape[0] <= 64 and ops.linear_rows_ok(hidden, w):
+                return ops.linear_f32_rows(hidden, w)
+            return torch.mm(hidden, w.t(), out_dtype=torch.float32)
         return self.lm_head(hidden).float()
 
     def forward_prefill(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:

@@ -351,3 +351,21 @@ def test_decode_step_takes_the_head_of_longer_rows(rows):
     with torch.inference_mode():
         a, b = (eng.model.forward_decode(ids, x) for x in (batch, exact))
     assert float(((a - b).norm(dim=-1) / b.norm(dim=-1)).max()) < 0.03     # bf16 through two layers, two sets of kernels
+
+
+@pytest.mark.parametrize("rows", [1, 5, 64, 65, 128, 300])
+def test_logits_are_32_bit_sums_at_every_row_count(rows):
+    from kllms_amd.engine.config import MODEL_PRESETS
+    from kllms_amd.models.llama import LlamaForCausalLM
+
+    with torch.device(DEV):
+        model = LlamaForCausalLM(MODEL_PRESETS["mid-llama"])
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    w = model.lm_head.weight
+    w.data.normal_(0, 0.02, generator=g)
+    h = torch.randn(rows, w.shape[1], generator=g, device=DEV).bfloat16()
+    out = model.compute_logits(h)
+    assert out.dtype == torch.float32
+    # sums of K products in 32 bits
+    tol = w.shape[1] * 2 ** -24 * (h.double().abs() @ w.double().abs().t().contiguous())
+    assert ((out.double() - h.double() @ w.double().t().contiguous()).abs() <= tol).all()
