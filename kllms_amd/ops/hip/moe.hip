@@ -28,9 +28,12 @@
 // the 8 XCDs in equal runs: an XCD's L2 sees each weight panel once, for its two or
 // three row tiles, and mostly one expert's rows.
 //
-// Measured at 2048 rows, 8 experts of 14336, top 2, width 4096: gate/up 1174 us (820
-// TFLOP/s; 2714 before), down 791 (608: 320 tiles are a round and a quarter; 1347
-// before); with routing around them 1903 us (4358).
+// Measured at 2048 rows, 8 experts of 14336, top 2, width 4096: gate/up 1198 us (803
+// TFLOP/s; 2714 before), down 783 (614: 320 tiles are a round and a quarter; 1347
+// before); with routing around them 1.93 - 2.0 ms (4.36). The one tile serves every row
+// count: the layer at 65 / 128 / 300 / 512 / 1024 rows takes 765 / 771 / 796 / 856 / 1050 us,
+// with 32-row waves over 128-row padding and the routing on the host it took 1195 / 1205 /
+// 1177 / 1751 / 2577; with experts of 3584 and 65 rows 253 (623).
 
 #include "common.h"
 
@@ -274,12 +277,11 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(bf16_t* __restrict__ o
   reinterpret_cast<bf16x8_vec*>(out)[(int64_t)t * nvec + i] = o;
 }
 
-// room for 128 KB of LDS; once per process and kernel is enough, a repeat harmless
+// room for 128 KB of LDS, asked for at each launch: the attribute is the current device's
 template <bool GATEUP>
 static bool lds_ready() {
-  static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_product_kernel<GATEUP>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, MOE_LDS) == hipSuccess;
-  return ok;
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(moe_product_kernel<GATEUP>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, MOE_LDS) == hipSuccess;
 }
 
 // rows S in sorted space; the grid holds the most tiles that S rows of E experts can
