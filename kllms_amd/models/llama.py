@@ -280,6 +280,7 @@ class LlamaForCausalLM(nn.Module):
         cfg = self.cfg
         at = self.layers[0].self_attn if len(self.layers) else None
         return (batch.mode == "decode" and at is not None and input_ids.is_cuda and input_ids.dim() == 1
+                and input_ids.dtype == torch.long
                 and 1 <= input_ids.shape[0] <= ops.LINEAR_ROWS_MAX and self.ctx.world_size == 1
                 and self.dtype == torch.bfloat16 and not ops._force_torch() and at.head_dim == 128
                 and cfg.hidden_size % 128 == 0 and cfg.hidden_size <= 16384 and cfg.intermediate_size % 128 == 0

@@ -369,3 +369,19 @@ def test_logits_are_32_bit_sums_at_every_row_count(rows):
     # sums of K products in 32 bits
     tol = w.shape[1] * 2 ** -24 * (h.double().abs() @ w.double().abs().t().contiguous())
     assert ((out.double() - h.double() @ w.double().t().contiguous()).abs() <= tol).all()
+
+
+def test_decode_step_takes_32_bit_ids():
+    """Ids of 32 bits, which an embedding takes as well, go to the general path."""
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+    from kllms_amd.models.llama import ForwardBatch
+
+    eng = LLMEngine(EngineConfig(model="mid-llama", max_kv_blocks=64, use_hip_graphs=False, seed=3))
+    rows = torch.arange(3, device=DEV)
+    batch = ForwardBatch(mode="decode", positions=torch.zeros_like(rows), slot_mapping=(rows + 8) * eng.kv.block_size,
+                         kv_caches=eng.kv.layer_caches(), block_tables=(rows + 8).to(torch.int32).view(3, 1),
+                         context_lens=torch.ones(3, dtype=torch.int32, device=DEV))
+    with torch.inference_mode():
+        want, got = (eng.model.forward_decode((rows + 5).to(t), batch) for t in (torch.long, torch.int32))
+    assert float(((got - want).norm(dim=-1) / want.norm(dim=-1)).max()) < 0.03     # bf16 through two layers, two sets of kernels
