@@ -840,6 +840,7 @@ class LLMEngine:
         state.ctx += 1
         # ONE device->host transfer per step (tokens + logprobs [+ topk] packed)
         packed = torch.cat(parts).cpu()
+        self._check_ids()
         B = tokens.shape[0]
         tokens_l = [int(x) for x in packed[:B].tolist()]
         logprobs_l = packed[B : 2 * B].tolist()
@@ -859,6 +860,12 @@ class LLMEngine:
             any_done |= s.done
         return any_done
 
+    def _check_ids(self) -> None:
+        """No token of a step whose ids were not all in the vocabulary (the GPU finds that; its results are here by now)."""
+        check = getattr(self.model, "check_ids", None)
+        if check is not None:
+            check()
+
     def _sample_and_append(self, logits: torch.Tensor, streams: List[_Stream]) -> None:
         """Sampling for the FIRST token (from the shared prefill logits);
         subsequent steps go through the device-resident _sample_state path."""
@@ -872,6 +879,7 @@ class LLMEngine:
             self._append_topk(streams, K, tl_idx.reshape(-1).tolist(), tl_vals.reshape(-1).tolist())
         tokens_l = tokens.tolist()
         logprobs_l = logprobs.tolist()
+        self._check_ids()
         for i, s in enumerate(streams):
             tok = tokens_l[i]
             s.step += 1

@@ -117,6 +117,7 @@ class DecodeGraphRunner:
         bs = self._bucket(B)
         if bs is None or batch.block_tables.shape[1] > self.max_blocks_per_seq:
             return self.engine.model.forward_decode(ids, batch)
+        self.engine._check_ids()
         if bs not in self.graphs:
             try:
                 self._capture(bs)

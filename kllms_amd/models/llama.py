@@ -287,12 +287,29 @@ class LlamaForCausalLM(nn.Module):
                 and self.cos_sin.is_contiguous() and input_ids.is_contiguous()
                 and all(t.is_contiguous() and t.numel() == input_ids.shape[0] for t in (batch.positions, batch.slot_mapping)))
 
+    _unknown: Optional[torch.Tensor] = None
+
+    def _unknown_ids(self) -> torch.Tensor:
+        """The flag that a step sets for an id outside the vocabulary: pinned, so that the host reads it without a copy
+        (a copied model's own is not)."""
+        if self._unknown is None or not self._unknown.is_pinned():
+            with torch.inference_mode(False):
+                self._unknown = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
+        return self._unknown
+
+    def check_ids(self) -> None:
+        """Raises if a decode step that has run had an id outside the vocabulary (its logits are NaN). It is
+        known once the step's results have come to the host, and raised before a later step at the latest."""
+        if self._unknown is not None and self._unknown.item():
+            self._unknown.zero_()
+            raise IndexError(f"a decode step had a token id outside the vocabulary of {self.embed_tokens.num_embeddings}")
+
     def _forward_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
         """A decode step: weights streamed by the few-row kernel, whose split sums go straight into the next row-wise
         kernel (8 launches a layer)."""
         layers = self.layers
         x, residual = ops.embed_norm_rows(input_ids, self.embed_tokens.weight, layers[0].input_layernorm.weight,
-                                          layers[0].input_layernorm.eps)
+                                          layers[0].input_layernorm.eps, self._unknown_ids())
         T = x.shape[0]
         for i, layer in enumerate(layers):
             at, norm = layer.self_attn, layer.post_attention_layernorm
@@ -331,6 +348,7 @@ class LlamaForCausalLM(nn.Module):
         return batch
 
     def forward_hidden(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
+        self.check_ids()
         batch = self._planned(input_ids, batch)
         if self._takes_rows(input_ids, batch):
             return self._forward_rows(input_ids, batch)

@@ -259,9 +259,11 @@ def linear_f32_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return _hip_or_raise().linear_rows(x, w, _none(x), 2, 1)
 
 
-def embed_norm_rows(ids, table, weight, eps):
-    """(rms(table[ids]) * weight, table[ids])."""
-    return _hip_or_raise().embed_norm_rows(ids, table, weight, eps)
+def embed_norm_rows(ids, table, weight, eps, unknown=None):
+    """(rms(table[ids]) * weight, table[ids]). An id outside the table gives a row of NaN and sets ``unknown``, one int32
+    of pinned host memory, to 1."""
+    return _hip_or_raise().embed_norm_rows(ids, table, weight, eps,
+                                           unknown if unknown is not None else torch.empty(0, dtype=torch.int32))
 
 
 def add_norm_rows(part, residual, weight, eps):

@@ -390,7 +390,7 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, torch::Tensor bias, 
 // --- row-wise steps of a decode step (decode_rows.hip) -------------------------
 extern "C" void launch_add_norm_rows(bf16_t* out, bf16_t* residual, const float* part, const int64_t* ids,
                                      const bf16_t* table, const bf16_t* w, int S, int M, int n, int64_t vocab,
-                                     float eps, hipStream_t stream);
+                                     float eps, int* unknown, hipStream_t stream);
 extern "C" void launch_rope_store_rows(bf16_t* q_out, const float* part, const bf16_t* bias, const int64_t* positions,
                                        const float* cos_sin, void* k_cache, void* v_cache, float* k_scale,
                                        float* v_scale, const int64_t* slots, int S, int M, int H, int G,
@@ -409,20 +409,24 @@ torch::Tensor add_norm_rows(torch::Tensor part, torch::Tensor residual, torch::T
                   n % 4 == 0 && n <= 16384 && S >= 1 && M >= 1, "add_norm_rows: sizes");
   auto out = torch::empty_like(residual);
   launch_add_norm_rows(bf(out), bf(residual), part.data_ptr<float>(), nullptr, nullptr, cbf(weight), S, M, n, 0,
-                       (float)eps, cur_stream());
+                       (float)eps, nullptr, cur_stream());
   return out;
 }
 
-// (rms(table[ids]) * weight, table[ids])
-std::vector<torch::Tensor> embed_norm_rows(torch::Tensor ids, torch::Tensor table, torch::Tensor weight, double eps) {
+// (rms(table[ids]) * weight, table[ids]); an id outside the table gives a row of NaN and sets unknown (empty, or one
+// int32 of pinned host memory)
+std::vector<torch::Tensor> embed_norm_rows(torch::Tensor ids, torch::Tensor table, torch::Tensor weight, double eps,
+                                           torch::Tensor unknown) {
   CHECK_BF16_CONTIG(table); CHECK_BF16_CONTIG(weight);
   TORCH_CHECK(ids.is_cuda() && ids.is_contiguous() && ids.scalar_type() == at::kLong && ids.dim() == 1);
   const int M = ids.size(0), n = table.size(1);
   TORCH_CHECK(weight.numel() == n && n % 4 == 0 && n <= 16384 && M >= 1, "embed_norm_rows: sizes");
+  TORCH_CHECK(unknown.numel() == 0 || (unknown.numel() == 1 && unknown.scalar_type() == at::kInt && unknown.is_pinned()),
+              "unknown: one int32 of pinned host memory");
   auto residual = torch::empty({M, n}, table.options());
   auto out = torch::empty_like(residual);
   launch_add_norm_rows(bf(out), bf(residual), nullptr, ids.data_ptr<int64_t>(), cbf(table), cbf(weight), 0, M, n,
-                       table.size(0), (float)eps, cur_stream());
+                       table.size(0), (float)eps, unknown.numel() ? unknown.data_ptr<int>() : nullptr, cur_stream());
   return {out, residual};
 }
 

@@ -36,7 +36,7 @@ template <bool EMBED>
 __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
     bf16_t* __restrict__ out, bf16_t* __restrict__ residual, const float* __restrict__ part,
     const int64_t* __restrict__ ids, const bf16_t* __restrict__ table, const bf16_t* __restrict__ w, int S, int M,
-    int n, int64_t vocab, float eps) {
+    int n, int64_t vocab, float eps, int* __restrict__ unknown) {
   __shared__ float red[16];
   const int m = blockIdx.x, tid = threadIdx.x;
   const int nvec = n / 4;
@@ -44,7 +44,9 @@ __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
   bf16x4_vec* ov = reinterpret_cast<bf16x4_vec*>(out + (int64_t)m * n);
   const bf16x4_vec* wv = reinterpret_cast<const bf16x4_vec*>(w);
   const int64_t id = EMBED ? ids[m] : 0;
-  const bool known = id >= 0 && id < vocab;   // an id without a row: NaN, never another's memory
+  // an id without a row: NaN, never another's memory, and *unknown set for the host
+  const bool known = id >= 0 && id < vocab;
+  if (EMBED && !known && unknown && tid == 0) __hip_atomic_store(unknown, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   f32x4 x[DR_VECS];
   float ss = 0.0f;
 #pragma unroll
@@ -83,13 +85,13 @@ __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
 
 extern "C" void launch_add_norm_rows(bf16_t* out, bf16_t* residual, const float* part, const int64_t* ids,
                                      const bf16_t* table, const bf16_t* w, int S, int M, int n, int64_t vocab,
-                                     float eps, hipStream_t stream) {
+                                     float eps, int* unknown, hipStream_t stream) {
   if (ids)
     hipLaunchKernelGGL(add_norm_rows_kernel<true>, dim3(M), dim3(DR_THREADS), 0, stream, out, residual, part, ids,
-                       table, w, S, M, n, vocab, eps);
+                       table, w, S, M, n, vocab, eps, unknown);
   else
     hipLaunchKernelGGL(add_norm_rows_kernel<false>, dim3(M), dim3(DR_THREADS), 0, stream, out, residual, part, ids,
-                       table, w, S, M, n, vocab, eps);
+                       table, w, S, M, n, vocab, eps, unknown);
 }
 
 // qkv sums [S, M, (H + 2G) * 128] (+ bias): q and k rotated (entry i with i + 64), q

@@ -371,6 +371,44 @@ def test_logits_are_32_bit_sums_at_every_row_count(rows):
     assert ((out.double() - h.double() @ w.double().t().contiguous()).abs() <= tol).all()
 
 
+@pytest.mark.parametrize("captured", [False, True])
+@pytest.mark.parametrize("bad", [-1, 2000, 1 << 40])
+def test_an_id_outside_the_vocabulary_is_reported(bad, captured):
+    """The step reads no foreign memory and its logits are NaN; the model raises once it has run, and goes on after that."""
+    import copy
+
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+    from kllms_amd.engine.graph_runner import DecodeGraphRunner
+    from kllms_amd.models.llama import ForwardBatch
+
+    eng = LLMEngine(EngineConfig(model="mid-llama", max_kv_blocks=64, use_hip_graphs=False, seed=3))
+    bad = eng.model.cfg.vocab_size if bad == 2000 else bad
+    rows = torch.arange(3, device=DEV)
+    batch = ForwardBatch(mode="decode", positions=torch.zeros_like(rows), slot_mapping=(rows + 8) * eng.kv.block_size,
+                         kv_caches=eng.kv.layer_caches(), block_tables=(rows + 8).to(torch.int32).view(3, 1),
+                         context_lens=torch.ones(3, dtype=torch.int32, device=DEV))
+    run = DecodeGraphRunner(eng, [4]).run if captured else eng.model.forward_decode
+    good, wrong = rows + 5, torch.tensor([5, bad, 7], device=DEV)
+    with torch.inference_mode():
+        want = run(good, batch).cpu()
+        for _ in range(2):
+            got = run(wrong, batch).cpu()
+            assert got[1].isnan().all() and torch.equal(got[::2], want[::2])
+            with pytest.raises(IndexError, match="outside the vocabulary"):
+                eng._check_ids()
+            assert torch.equal(run(good, batch).cpu(), want)
+        run(wrong, batch).cpu()
+        with pytest.raises(IndexError):     # whoever does not ask is told at the next step
+            run(good, batch)
+        assert torch.equal(run(good, batch).cpu(), want)
+        twin = copy.deepcopy(eng.model)     # its flag is its own
+        twin.forward_decode(wrong, batch).cpu()
+        eng.model.check_ids()
+        with pytest.raises(IndexError):
+            twin.check_ids()
+
+
 def test_decode_step_takes_32_bit_ids():
     """Ids of 32 bits, which an embedding takes as well, go to the general path."""
     from kllms_amd.engine.config import EngineConfig
