@@ -306,7 +306,8 @@ class LlamaForCausalLM(nn.Module):
 
     def _forward_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
         """A decode step: weights streamed by the few-row kernel, whose split sums go straight into the next row-wise
-        kernel (8 launches a layer)."""
+        kernel: 8 launches a layer, one more where attention splits the contexts and one where gate/up is the
+        library's."""
         layers = self.layers
         x, residual = ops.embed_norm_rows(input_ids, self.embed_tokens.weight, layers[0].input_layernorm.weight,
                                           layers[0].input_layernorm.eps, self._unknown_ids())

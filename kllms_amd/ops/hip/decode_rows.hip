@@ -7,7 +7,8 @@
 // agree to the last bits of their sums.
 //
 // Per layer: residual + norm (twice) and rope + cache store, beside attention and
-// four products: 8 launches, where separate reductions, rope, store and activation
+// four products: 8 launches (one more where attention splits the contexts, one where
+// gate/up is the library's), where separate reductions, rope, store and activation
 // took 11. A step of 5 rows (32 heads, width 4096, 6 layers, contexts of 560) went
 // from 948 to 774 us with these and linear_rows.hip, one of 120 rows from 1516 to 1237,
 // one of a single row at width 2048 from 492 to 391.

@@ -11,8 +11,9 @@
 //
 // A matrix of few rows is also split over k (linear_rows_splits); the splits' fp32 sums are left to the consumer, which reads them anyway (rope + store,
 // residual + norm). Forms of the result:
-//   PART  fp32 sums [S, M, N]          BF16  rounded once, bias added before it
-//   F32   fp32, S = 1 (logits)         SILU  silu(gate) * up of a fused [gate; up] matrix
+//   PART  fp32 sums [S, M, N]          SILU  silu(gate) * up of a fused [gate; up] matrix
+//   F32   fp32, S = 1 (logits)         BF16  rounded once, bias added before it: for callers of the
+//                                            binding, the models' products take the other three
 //
 // Measured with the weights out of cache (the library's kernel in brackets), us:
 //   4096 x 4096   5 rows 9 (15.6), 128 rows 15.6 (24.5)
@@ -166,9 +167,16 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
 
 // Waves of a workgroup. Eight halve the reads of x, which at 128 rows and 64 weight rows
 // a workgroup are twice the weights' bytes; they pay where the weights still make enough
-// workgroups: 128 rows, 4096 x 14336 36 us (39.5 with four), 6144 x 4096 21.7 (23.9), but
-// 2048 x 2048 8.5 (6.9); unsplit, 28672 x 4096 with silu at 64 rows 57.4 (59.6), but
-// 16384 x 2048 27.5 (23.0).
+// workgroups. us with four and eight waves, weights out of cache:
+//   PART, 65 / 96 / 128 rows   2048 x 2048  6.3 7.6 / 6.7 8.1 / 7.2 8.9     3072 x 2048  8.4 8.3 / 9.3 9.1 / 10.1 10.2
+//     3072 x 8192  21.7 20.8 / 24.0 22.4 / 26.1 24.5     4096 x 4096  13.6 13.2 / 15.5 14.2 / 16.6 15.6
+//     6144 x 4096  20.0 18.2 / 21.6 19.6 / 22.6 20.7     8192 x 8192  42.4 40.9 / 44.3 41.9 / 46.2 43.5
+//   SILU, 33 / 64 rows   16384 x 2048  22.6 27.0 / 23.0 27.6     16384 x 4096  46.9 51.1 / 46.8 52.2
+//     22016 x 4096  55.5 53.2 / 57.9 54.7     24576 x 3072  41.7 41.5 / 44.8 43.5     28672 x 4096  58.3 60.4 / 61.6 60.5
+//   F32, 33 / 64 rows   16384 x 2048  21.8 26.3 / 22.4 27.6     24576 x 4096  53.6 54.3 / 57.1 56.6
+//     50304 x 2048  56.9 52.0 / 61.3 54.5     128256 x 4096  217.9 220.3 / 240.5 232.5
+// From 200 workgroups of eight waves on (N = 25600) neither side loses more than 4 %; a line at 20000 would gain the
+// sizes between 3 - 6 %.
 static int linear_rows_waves(int M, int N, int form) {
   if (N % 128 != 0) return 4;
   return (form == LR_PART ? M > 64 && N >= 4096 : M > 32 && N >= 200 * 128) ? 8 : 4;
