@@ -295,12 +295,18 @@ void one_shot_allreduce(std::vector<torch::Tensor> bufs) {
 // --- grouped MoE expert GEMMs (moe.hip) --------------------------------------
 extern "C" int launch_moe_gateup(void* act, const void* x, const void* w, const int* sorted_ids, const int* offsets,
                                  const void* zeros, int S, int E, int IN, int K, hipStream_t stream);
-extern "C" int launch_moe_down(void* y, const void* act, const void* w, const int* offsets, int S, int E, int H,
-                               int IN, hipStream_t stream);
+extern "C" int launch_moe_down(void* y, const void* act, const void* w, const int* offsets, float* part, int* count,
+                               int S, int E, int H, int IN, hipStream_t stream);
+extern "C" int64_t moe_down_room(int S, int E, int H, int* zeros);
 extern "C" void launch_moe_sort(int* ids, int* pos, int* offsets, const int64_t* topi, int P, int k, int E,
                                 hipStream_t stream);
 extern "C" void launch_moe_combine(void* out, const void* y, const float* weights, const int* pos, int T, int k,
                                    int H, hipStream_t stream);
+
+// what the products copy to LDS and store in 16-byte pieces: a view that does not begin on such a piece is copied
+static torch::Tensor on_16_bytes(const torch::Tensor& t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t;
+}
 
 void moe_gateup(torch::Tensor act, torch::Tensor x, torch::Tensor w,
                 torch::Tensor sorted_ids, torch::Tensor offsets, torch::Tensor zeros) {
@@ -314,10 +320,14 @@ void moe_gateup(torch::Tensor act, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(act.size(1) == IN && x.size(1) == K && zeros.numel() >= K);
   TORCH_CHECK(sorted_ids.numel() >= act.size(0), "one id per sorted row");
   TORCH_CHECK(offsets.numel() == E + 1);
+  TORCH_CHECK(K < (1 << 24), "moe_gateup: a row of a tile's weights has a 32-bit offset");
   if (act.size(0) == 0) return;
-  TORCH_CHECK(launch_moe_gateup(act.data_ptr(), x.data_ptr(), w.data_ptr(), sorted_ids.data_ptr<int>(),
+  x = on_16_bytes(x), w = on_16_bytes(w), zeros = on_16_bytes(zeros);
+  auto out = on_16_bytes(act);
+  TORCH_CHECK(launch_moe_gateup(out.data_ptr(), x.data_ptr(), w.data_ptr(), sorted_ids.data_ptr<int>(),
                                 offsets.data_ptr<int>(), zeros.data_ptr(), (int)act.size(0), E, IN, K,
-                                cur_stream()) == 0, "moe_gateup: 128 KB of LDS are not available");
+                                cur_stream()) == 0, "moe_gateup: 160 KB of LDS are not available");
+  if (!out.is_same(act)) act.copy_(out);
 }
 
 void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor offsets) {
@@ -328,9 +338,22 @@ void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor
   TORCH_CHECK(H % 64 == 0 && IN % 64 == 0, "H % 64, IN % 64 required");
   TORCH_CHECK(y.size(1) == H && act.size(1) == IN && y.size(0) >= act.size(0));
   TORCH_CHECK(offsets.numel() == E + 1 && offsets.scalar_type() == at::kInt && offsets.is_contiguous());
+  TORCH_CHECK(IN < (1 << 24), "moe_down: a row of a tile's weights has a 32-bit offset");
   if (act.size(0) == 0) return;
-  TORCH_CHECK(launch_moe_down(y.data_ptr(), act.data_ptr(), w.data_ptr(), offsets.data_ptr<int>(), (int)act.size(0), E,
-                              H, IN, cur_stream()) == 0, "moe_down: 128 KB of LDS are not available");
+  act = on_16_bytes(act), w = on_16_bytes(w);
+  auto out = on_16_bytes(y);
+  // partial sums and counters of tiles that are worked on in shares
+  int zeros = 0;
+  const int64_t room = moe_down_room(act.size(0), E, H, &zeros);
+  torch::Tensor part, count;
+  if (room) {
+    part = torch::empty({room}, act.options().dtype(torch::kFloat));
+    count = torch::zeros({zeros}, act.options().dtype(torch::kInt));
+  }
+  TORCH_CHECK(launch_moe_down(out.data_ptr(), act.data_ptr(), w.data_ptr(), offsets.data_ptr<int>(),
+                              room ? part.data_ptr<float>() : nullptr, room ? count.data_ptr<int>() : nullptr, (int)act.size(0), E, H, IN,
+                              cur_stream()) == 0, "moe_down: 160 KB of LDS are not available");
+  if (!out.is_same(y)) y.copy_(out);
 }
 
 // topi [T, k] int64 -> (ids [T * k] token of each sorted place, pos [T, k] sorted place of each pair,

@@ -1,0 +1,281 @@
+// !!! This is a file automatically generated by hipify!!!
+#include "hip/hip_runtime.h"
+// The inner loop of the large bf16 products, for gfx950: a workgroup of 4 waves, one on
+// each SIMD of a compute unit, multiplies 256 rows of W (columns of the result) with 32 * MJ rows of X,
+// acc[i][j] of a wave = 16 columns i by 16 rows j of its 128 columns x 16 * MJ rows, in
+// v_mfma_f32_16x16x32_bf16 (W the A operand, so that a lane ends with 4 neighbouring columns of a row).
+//
+// K goes by 64 ("stages") through a ring of LDS buffers, copied there straight from
+// memory (no registers in between). Rows of 128 bytes; the copy writes LDS in lane
+// order, so the conflict-free order of a row's 16-byte units (XORed with the row) is
+// made by the addresses that the lanes read. A stage has two halves of 32 k:
+//
+//   first    matrix work on window 0 | window 1 is read to registers; barrier: the
+//            buffer is free, the copy of stage s + RING into it starts
+//   second   matrix work on window 1 | barrier before it: stage s + 1 has landed; its
+//            window 0 is read, the copy goes on
+//
+// What bounds it: the matrix units, and around them the issue of the copies. A copy
+// instruction of 1 KB occupies the address unit for 16 cycles; issued in bursts the
+// waves stall on it (1319 TFLOP/s at 8192^3), spread evenly over a stage, one every 5
+// matrix instructions, it stays under them (1490, where the library reaches 1570; 1260
+// with half as deep stages of 64-byte rows, whose requests are twice as many; 1360 with
+// 32x32x16 instructions). The order of issue is pinned by scheduling barriers.
+// One wave per SIMD (128 x 128 of the result) needs 1.0 KB of LDS reads per 4 matrix instructions, half of
+// what eight waves of 128 x 64 need, and all 512 registers: 256 sums, 2 x 64 fragments.
+//
+// Small MJ are for the ends of ragged row ranges and for few rows, where the stream of W
+// is the bound: less matrix work per stage, and more buffers of it in flight.
+
+#pragma once
+
+#include "common.h"
+
+typedef __bf16 bf16x8_mfma __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4_cvt __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+#define TP_N 256           // rows of W of a workgroup
+#define TP_K 64            // k of a stage
+#define TP_THREADS 256
+#define TP_LDS 163840      // all of a compute unit's
+#define TP_SLOTS 32        // compute units of an XCD
+#define TP_SHARES 4        // workgroups that share a tile's K at most
+#define TP_SUMS (256 * 256)
+
+// Which of an XCD's tiles its at-th workgroup takes, and which share of its K. Tiles that
+// make whole rounds of the XCD's compute units are one workgroup's each; those of the
+// last round, if they leave half of the units idle or more, are shared out.
+struct TileShare {
+  int tile, share, shares;
+  float* part;               // [8 XCDs][TP_SLOTS][TP_SUMS], of this tile's shares
+  int* count;                // [8][TP_SLOTS] zeros
+  __device__ __forceinline__ TileShare(int at, int tiles, int stages, float* parts, int* counts, int xcd)
+      : tile(at), share(0), shares(1), part(nullptr), count(nullptr) {
+    const int rest = tiles % TP_SLOTS, full = tiles - rest;
+    if (!parts || at < full || rest == 0) return;
+    shares = max(1, min(min(TP_SLOTS / rest, TP_SHARES), stages / 8));
+    const int r = (at - full) % rest;
+    share = (at - full) / rest;
+    tile = share < shares ? full + r : tiles;
+    part = parts + (int64_t)(xcd * TP_SLOTS + r * shares) * TP_SUMS;
+    count = counts + xcd * TP_SLOTS + r;
+  }
+  __device__ __forceinline__ int first(int stages) const { return (stages + shares - 1) / shares * share; }
+  __device__ __forceinline__ int length(int stages) const {
+    return min((stages + shares - 1) / shares, stages - first(stages));
+  }
+};
+
+#define TP_HOLD __builtin_amdgcn_sched_barrier(0)
+
+// Buffer descriptor of bytes from p on; lanes behind its end read zeros.
+__device__ __forceinline__ u32x4 tp_range(const void* p, uint32_t bytes) {
+  const uint64_t a = (uint64_t)p;
+  u32x4 r;
+  r[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  r[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) & 0xffff;
+  r[2] = __builtin_amdgcn_readfirstlane(bytes);
+  r[3] = 0x00020000;
+  return r;
+}
+
+// Copies of 16 bytes a lane to lds + lane * 16. They are written out because the
+// compiler makes every later LDS read wait for the builtin's; the waits stand in the loop.
+__device__ __forceinline__ void tp_copy(u32x4 range, uint32_t lane_off, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(lane_off), "s"(range),
+               "s"(off), "s"(lds)
+               : "memory");
+}
+
+__device__ __forceinline__ void tp_copy_at(uint64_t at, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(at), "s"(lds) : "memory");
+}
+
+// Rows of an operand in memory order, 8 to a copy: from base on, ``rows`` of them exist (the others read as zeros).
+struct TileRows {
+  u32x4 range;
+  uint32_t lane_off, row8;
+  __device__ __forceinline__ TileRows(const bf16_t* base, int rows, int most, int K, int lane)
+      : range(tp_range(base, (uint32_t)min(max(rows, 0), most) * K * 2)),
+        lane_off((uint32_t)(lane >> 3) * K * 2 + (((lane & 7) ^ (lane >> 3)) << 4)), row8(8u * K * 2) {}
+  __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds) const {
+    tp_copy(range, lane_off, k_off + i * row8, lds);
+  }
+};
+
+// Rows anywhere: at[i] is the address of this lane's 16 bytes of the i-th copy in stage 0.
+template <int MJ>
+struct TileGather {
+  uint64_t at[MJ];
+  __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds) const { tp_copy_at(at[i] + k_off, lds); }
+};
+
+template <int MJ>
+struct TileRing {
+  static constexpr int STRIDE = (TP_N + 32 * MJ) * 128;   // W rows, then X rows
+  static constexpr int RING = TP_LDS / STRIDE < 4 ? TP_LDS / STRIDE : 4;
+};
+
+// acc += W X^T over K; w: this wave's 64 of the 256 rows, x: its 8 * MJ of the 32 * MJ. Ends with all waves past
+// their last LDS read.
+template <int MJ, class X>
+__device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows& w, const X& x, int stages, char* smem) {
+  constexpr int STRIDE = TileRing<MJ>::STRIDE, RING = TileRing<MJ>::RING;
+  constexpr int F = 8 * MJ;              // matrix instructions of a half
+  constexpr int NR = 8 + MJ;             // LDS reads of a half
+  constexpr int ND = 8 + MJ;             // copies of a stage
+  constexpr int RS = F / (2 * NR) > 0 ? F / (2 * NR) : 1;
+  constexpr int P1 = RS * NR + (MJ >= 4 ? 8 : 4);   // first half: all has been read
+  constexpr int DS = (2 * F - P1) / ND;             // a copy every DS instructions from there on
+  constexpr int D1 = (F - 1 - P1) / DS + 1;         // copies in the first half
+  static_assert(P1 < F && DS >= 1 && RING >= 2 && (RING - 1) * ND < 64);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const uint32_t w_put = lds0 + wave * 64 * 128, x_put = lds0 + TP_N * 128 + wave * MJ * 1024;
+  uint32_t w_get[2], x_get[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const uint32_t o = lds0 + col * 128 + (((ks * 4 + grp) ^ (col & 7)) << 4);
+    w_get[ks] = o + (wave >> 1) * 128 * 128;
+    x_get[ks] = o + TP_N * 128 + (wave & 1) * MJ * 16 * 128;
+  }
+  typedef __attribute__((address_space(3))) const bf16x8_mfma* lds_ptr;
+  auto get = [](uint32_t at) { return *(lds_ptr)(uintptr_t)at; };
+  auto put = [&](int d, uint32_t k_off, uint32_t buf) {   // d-th copy of a stage
+    const int i = d < 2 * MJ ? d >> 1 : d - MJ;
+    if (d < 2 * MJ && (d & 1)) x.copy(i, k_off, x_put + buf + i * 1024);
+    else w.copy(i, k_off, w_put + buf + i * 1024);
+  };
+  bf16x8_mfma a[2][8], b[2][MJ];
+  auto read = [&](int ks, int r, uint32_t buf) {
+    if (r < 2 * MJ && !(r & 1)) b[ks][r >> 1] = get(x_get[ks] + buf + (r >> 1) * 2048);
+    else {
+      const int i = r < 2 * MJ ? r >> 1 : r - MJ;
+      a[ks][i] = get(w_get[ks] + buf + i * 2048);
+    }
+  };
+  auto multiply = [&](int ks, int f) {
+    const int i = f / MJ, j = f % MJ;
+    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][i], b[ks][j], acc[i][j], 0, 0, 0);
+    if (f & 1) TP_HOLD;
+  };
+
+#pragma unroll
+  for (int t = 0; t < RING; ++t)         // of fewer stages the last one again: the counts below stand
+#pragma unroll
+    for (int d = 0; d < ND; ++d) put(d, (uint32_t)min(t, stages - 1) * 128, t * STRIDE);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"((RING - 1) * ND) : "memory");
+#pragma unroll
+  for (int r = 0; r < NR; ++r) read(0, r, 0);
+
+  uint32_t buf = 0;
+#pragma unroll 1
+  for (int s = 0; s < stages; ++s) {
+    // behind the last stage that one is copied again and nothing of it used: no branches
+    const uint32_t k_off = (uint32_t)min(s + RING, stages - 1) * 128;
+    TP_HOLD;
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      if (f % RS == 0 && f / RS < NR) read(1, f / RS, buf);
+      if (f == P1) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);           // lgkmcnt(0)
+        asm volatile("s_barrier" ::: "memory");
+        TP_HOLD;
+      }
+      if (f >= P1 && (f - P1) % DS == 0 && (f - P1) / DS < ND) put((f - P1) / DS, k_off, buf);
+      multiply(0, f);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"((RING - 2) * ND + D1) : "memory");
+    TP_HOLD;
+    const uint32_t next = buf == (RING - 1) * STRIDE ? 0u : buf + STRIDE;
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      if (f % RS == 0 && f / RS < NR) read(0, f / RS, next);
+      if ((f + F - P1) % DS == 0 && (f + F - P1) / DS < ND) put((f + F - P1) / DS, k_off, buf);
+      multiply(1, f);
+    }
+    buf = next;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Sums of a tile whose K is shared by ``shares`` workgroups: each leaves its own in part
+// [shares][8 * MJ][threads][4]; the last one to arrive adds them all up, in the order
+// of the shares whoever it is, and goes on (true) with the whole. count: 0 before.
+template <int MJ>
+__device__ __forceinline__ bool tile_fold(f32x4 (&acc)[8][MJ], float* part, int share, int shares, int* count, char* smem) {
+  constexpr int SIZE = 8 * MJ * TP_THREADS;
+  const int tid = threadIdx.x;
+  f32x4* all = reinterpret_cast<f32x4*>(part) + tid;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < MJ; ++j) all[share * SIZE + (i * MJ + j) * TP_THREADS] = acc[i][j];
+  __syncthreads();
+  if (tid == 0) {
+    __threadfence();                     // the workgroup's sums out of this XCD's L2, before the count
+    *reinterpret_cast<int*>(smem) = atomicAdd(count, 1);
+    __threadfence();                     // and nothing older than it in the caches
+  }
+  __syncthreads();
+  if (*reinterpret_cast<const int*>(smem) != shares - 1) return false;
+  __syncthreads();                       // smem is free again
+  // its own share too is read back: kept beside the sum, it would cost the loop above its registers
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+#pragma unroll
+    for (int j = 0; j < MJ; ++j) acc[i][j] = all[(i * MJ + j) * TP_THREADS];
+#pragma unroll 1
+    for (int s = 1; s < shares; ++s) {
+      f32x4 v[MJ];
+#pragma unroll
+      for (int j = 0; j < MJ; ++j) v[j] = all[s * SIZE + (i * MJ + j) * TP_THREADS];
+#pragma unroll
+      for (int j = 0; j < MJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] += v[j][r];
+    }
+    TP_HOLD;
+  }
+  return true;
+}
+
+__device__ __forceinline__ bf16x4_vec tp_pack(float a, float b, float c, float d) {
+  const f32x4 v = {a, b, c, d};
+  return __builtin_bit_cast(bf16x4_vec, __builtin_convertvector(v, bf16x4_cvt));
+}
+
+// A wave's result, 16 * MJ rows by 16 * NI columns, to memory in 16-byte stores of whole rows, by way of its own part
+// of LDS: value(i, j) gives the lane's 4 columns i * 16 + grp * 4.. of row j * 16 + col. Row r goes to out + r *
+// stride; rows and columns of it exist, columns and stride are multiples of 8.
+template <int NI, int MJ, class V>
+__device__ __forceinline__ void tile_store(bf16_t* out, int64_t stride, int rows, int columns, char* smem, V value) {
+  constexpr int UNITS = NI * 2;          // 16-byte units of a row: 8 or 16
+  const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+  char* mine = smem + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * (MJ * 16 * UNITS * 16);
+#pragma unroll
+  for (int j = 0; j < MJ; ++j)
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      *reinterpret_cast<bf16x4_vec*>(mine + (j * 16 + col) * (UNITS * 16) +
+                                     (((i * 2 + (grp >> 1)) ^ (col & (UNITS - 1))) << 4) + (grp & 1) * 8) = value(i, j);
+  // this wave's own part of LDS: in order, only the compiler is held
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int unit = lane % UNITS, r0 = lane / UNITS;
+#pragma unroll
+  for (int k = 0; k < MJ * 16 * UNITS / 64; ++k) {
+    const int r = k * (64 / UNITS) + r0;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(mine + r * (UNITS * 16) + ((unit ^ (r & (UNITS - 1))) << 4));
+    if (r < rows && unit * 8 < columns) *reinterpret_cast<u32x4*>((short*)out + r * stride + unit * 8) = v;
+  }
+}
+
+// room for all of LDS, asked for at each launch: the attribute is the current device's
+static inline bool tp_lds_ready(const void* kernel) {
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, TP_LDS) == hipSuccess;
+}

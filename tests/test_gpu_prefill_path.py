@@ -184,6 +184,33 @@ def test_mixture_products_against_float64(H, I, counts):
     assert ((got.double() - ref).abs() <= lim + 2 ** -8 * ref.abs() + 1e-5).all()
 
 
+@pytest.mark.parametrize("H,I,counts", [
+    (256, 1088, [32, 33, 64, 65, 80, 81, 96, 97, 128, 129]),      # one column tile; down shares its 17 stages in two
+    (1088, 2112, [20, 130, 0, 150, 260, 385, 1]),                 # five column tiles, the last of 64; shares of 33 stages
+])
+def test_mixture_products_at_the_edges_of_row_tiles(H, I, counts):
+    # expert e gets counts[e] + counts[e - 1] rows: 64, 128, 160, 192 and 256 a tile, and parts of two and three tiles
+    test_mixture_products_against_float64(H, I, counts)
+
+
+def test_mixture_products_of_views_off_16_bytes():
+    def off(*shape):
+        n = torch.Size(shape).numel()
+        return torch.randn(n + 1, device=DEV).bfloat16()[1:].view(shape)
+
+    T, H, I, E = 70, 128, 192, 2
+    x, wg, wd = off(T, H), off(E, 2 * I, H), off(E, H, I)
+    ids = torch.arange(T, device=DEV, dtype=torch.int32)
+    offsets = torch.tensor([0, 30, T], device=DEV, dtype=torch.int32)
+    act, y = off(T, I), off(T, H)
+    ops.moe_gateup(act, x, wg, ids, offsets, x)
+    ops.moe_down(y, act, wd, offsets)
+    act2, y2 = torch.empty(T, I, device=DEV, dtype=x.dtype), torch.empty(T, H, device=DEV, dtype=x.dtype)
+    ops.moe_gateup(act2, x.clone(), wg.clone(), ids, offsets, x.clone())
+    ops.moe_down(y2, act2, wd.clone(), offsets)
+    assert torch.equal(act, act2) and torch.equal(y, y2)
+
+
 @pytest.mark.parametrize("T,H", [(65535, 8), (65536, 64), (70001, 2056)])
 def test_mixture_of_more_rows_than_a_grid_has_in_y(T, H):
     g = torch.Generator(device=DEV).manual_seed(T)
