@@ -27,6 +27,8 @@
 
 #pragma once
 
+#include <hip/hip_runtime.h>
+
 #include "common.h"
 
 typedef __bf16 bf16x8_mfma __attribute__((ext_vector_type(8)));
