@@ -105,7 +105,7 @@ class FusedInput(nn.Module):
         self.bias_parts = tuple(bias_parts)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight, self.bias)
+        return ops.linear(x, self.weight, self.bias)
 
     def split(self, y: torch.Tensor, name: str) -> torch.Tensor:
         off, n = self.parts[name]
@@ -213,7 +213,7 @@ class BlockLocalAttention(nn.Module):
                                           sp.scale, sp.mask_size, None, row_map=row_map, out=att)
             if gate is not None:
                 ops.head_gate(att, gate)
-        return F.linear(att.reshape(T, -1), self.o_proj)
+        return ops.linear(att.reshape(T, -1), self.o_proj)
 
 
 class DecayLinearAttention(nn.Module):
@@ -239,7 +239,7 @@ class DecayLinearAttention(nn.Module):
                                   v.unflatten(1, (sp.heads, sp.vdim)), self.decay, st.rec,
                                   batch.state_slots, batch.cu_seqlens, batch.seg_start, step_chunks(batch, sp.dim))
         y = ops.gated_rmsnorm(o.view(o.shape[0], 1, -1), self.norm, gate, self.eps, self.o_proj.dtype)
-        return F.linear(y, self.o_proj)
+        return ops.linear(y, self.o_proj)
 
 
 class ParallelMixer(nn.Module):
@@ -338,7 +338,7 @@ class ChannelDeltaMixer(nn.Module):
             s(y, "b"), a, self.dt_bias, self.A_log, st.rec, batch.state_slots, batch.cu_seqlens,
             batch.seg_start)
         r = ops.gated_rmsnorm(o, self.norm, gate, self.eps, self.o_proj.dtype)
-        return F.linear(r, self.o_proj)
+        return ops.linear(r, self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         m = {pre + n: self.inp.slot(n) for n in self.inp.parts}
@@ -361,12 +361,16 @@ class ClampedGLU(nn.Module):
         self.spec = spec
         self.inp = FusedInput(hidden, [("gate", spec.ff), ("up", spec.ff)], dtype)
         self.down = _param(hidden, spec.ff, dtype=dtype)
+        self._fused = self.inp.weight.shape[0] == 2 * spec.ff      # up's rows follow gate's without a gap
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
+        act = ops.linear_clamped_glu(h, self.inp.weight, self.spec.limit, self.spec.alpha) if self._fused else None
+        if act is not None:
+            return ops.linear(act, self.down)
         y = self.inp(h)
         act = ops.clamped_glu(self.inp.split(y, "gate"), self.inp.split(y, "up"),
                               self.spec.limit, self.spec.alpha)
-        return F.linear(act, self.down)
+        return ops.linear(act, self.down)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         return {pre + "gate": self.inp.slot("gate"), pre + "up": self.inp.slot("up"), pre + "down": self.down}
@@ -403,7 +407,7 @@ class WindowSinkAttention(nn.Module):
         v = s(y, "v").unflatten(1, (sp.kv_heads, sp.vdim))
         ops.qk_norm_store(q, k, v, self.q_norm, self.k_norm, self.eps, st.k, st.v, batch.slot_mapping)
         att = ops.attn_window_sink(q, st, batch, sp, s(y, "g"))
-        return F.linear(att.reshape(T, -1), self.o_proj)
+        return ops.linear(att.reshape(T, -1), self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         m = {pre + n: self.inp.slot(n) for n in self.inp.parts}
@@ -477,7 +481,7 @@ class LatentAttention(nn.Module):
         torch.bmm(lat.transpose(0, 1), self.uv, out=att.view(T, H, V).transpose(0, 1))
         if sp.elem_gate:
             ops.sigmoid_gate_(att, s(y, "g"))
-        return F.linear(att, self.o_proj)
+        return ops.linear(att, self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         m = {pre + n: self.inp.slot(n) for n in self.inp.parts}
@@ -525,7 +529,7 @@ class Retention(nn.Module):
                                   s(y, "v").unflatten(1, (sp.heads, sp.vdim)), s(y, "g"), self.decay, batch.positions,
                                   self.inv_freq, st.rec, batch.state_slots, batch.cu_seqlens, batch.seg_start,
                                   self.eps, self.o_proj.dtype, step_chunks(batch, sp.dim), single_rows(batch))
-        return F.linear(r, self.o_proj)
+        return ops.linear(r, self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         m = {pre + n: self.inp.slot(n) for n in self.inp.parts}
@@ -638,7 +642,7 @@ class PoolWindowAttention(nn.Module):
                                    batch.positions, run, rows)
         att = ops.attn_window_pool_paged(q, st.k, st.v, st.pool_k, st.pool_v, batch.block_tables, batch.token_seg,
                                          batch.positions, sp.scale, sp.softcap, sp.mask_size, run)
-        return F.linear(att.reshape(T, -1), self.o_proj)
+        return ops.linear(att.reshape(T, -1), self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         m = {pre + n: self.inp.slot(n) for n in self.inp.parts}
@@ -729,7 +733,7 @@ class DiffAttention(nn.Module):
                                p.get("v"), st.k, st.v, batch.slot_mapping, single_rows(batch))
         att = ops.attn_diff_paged(q.view(T, sp.heads, 2 * sp.dim), st.k, st.v, batch.block_tables, batch.token_seg,
                                   batch.positions, sp.scale, self.lam, 1.0 - sp.diff, self.eps, self._tiles(batch))
-        return F.linear(att.view(T, -1), self.o_proj)
+        return ops.linear(att.view(T, -1), self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         m = {}
@@ -784,7 +788,7 @@ class Mamba2Mixer(nn.Module):
                                batch.cu_seqlens, batch.seg_start)
         r = ops.gate_group_rmsnorm(o.view(o.shape[0], sp.norm_groups, -1), self.norm, s(y, "z"), self.eps,
                                    self.o_proj.dtype)
-        return F.linear(r, self.o_proj)
+        return ops.linear(r, self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         m = {pre + "in": [self.inp.slot("z"), self.inp.slot("xbc"), self.inp.slot("dt")]}
@@ -812,9 +816,9 @@ class ActFF(nn.Module):
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         if self.inp is not None:
             y = self.inp(h)
-            return F.linear(ops.gelu_glu(self.inp.split(y, "gate"), self.inp.split(y, "up")), self.down)
+            return ops.linear(ops.gelu_glu(self.inp.split(y, "gate"), self.inp.split(y, "up")), self.down)
         act = ops.relu2 if self.spec.act == "relu2" else ops.gelu_tanh
-        return F.linear(act(F.linear(h, self.up)), self.down)
+        return ops.linear(act(F.linear(h, self.up)), self.down)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         if self.inp is not None:
@@ -869,7 +873,7 @@ class WkvMixer(nn.Module):
         o = ops.wkv_recurrence(y[0].unflatten(1, hd), y[1].unflatten(1, hd), y[2].unflatten(1, hd), d,
                                self.w0, self.u, st.rec, batch.state_slots, batch.cu_seqlens, batch.seg_start)
         r = ops.head_rmsnorm_gate(o, self.norm, y[3], self.eps, "silu", self.o_proj.dtype)
-        return F.linear(r, self.o_proj)
+        return ops.linear(r, self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         m = {pre + "mu." + n: self.mu[i] for i, n in enumerate(self.STREAMS)}
@@ -917,7 +921,7 @@ class MlstmMixer(nn.Module):
                               s(y, "v").unflatten(1, (sp.heads, sp.vdim)), z, self.gate_bias, sp.gate_cap,
                               st.rec, batch.state_slots, batch.cu_seqlens, batch.seg_start, self.norm, s(y, "g"),
                               self.eps, self.o_proj.dtype)
-        return F.linear(r, self.o_proj)
+        return ops.linear(r, self.o_proj)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         H = self.spec.heads
@@ -1030,7 +1034,7 @@ class RoutedExperts(nn.Module):
         if self.shared_inp is not None:
             ys = self.shared_inp(h)
             ss = self.shared_inp.split
-            extra = F.linear(self._act(ss(ys, "gate"), ss(ys, "up"), sp.shared.limit), self.shared_down)
+            extra = ops.linear(self._act(ss(ys, "gate"), ss(ys, "up"), sp.shared.limit), self.shared_down)
             gate = ss(ys, "sg")[:, 0] if sp.shared.gated else None
         return ops.moe_combine(rows, h, rowidx, None if on_input else w, h.dtype, extra, gate)
 

@@ -356,6 +356,38 @@ void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor
   if (!out.is_same(y)) y.copy_(out);
 }
 
+// --- products of many rows (linear_tiles.hip) ---------------------------------
+extern "C" int linear_tiles_rows(int64_t M, int64_t N, int64_t K, int act);
+extern "C" int launch_linear_tiles(void* out, const void* x, const void* w, const void* bias, int M, int N, int K, int act,
+                                   int mj, float limit, float alpha, hipStream_t stream);
+
+// act 0: x [M, K] @ w [N, K]^T + bias (or an empty one); 1, 2: w [2 N, K], silu(gate) * up or the clamped form.
+// mj: 32-row steps of a tile, 2 to 8
+torch::Tensor linear_tiles(torch::Tensor x, torch::Tensor w, torch::Tensor bias, int act, int mj, double limit,
+                           double alpha) {
+  CHECK_BF16_CONTIG(x); CHECK_BF16_CONTIG(w);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) && x.device() == w.device(), "x [M, K], w [N, K]");
+  TORCH_CHECK(act >= 0 && act <= 2 && mj >= 2 && mj <= 8, "linear_tiles: act 0 to 2, mj 2 to 8");
+  const int64_t M = x.size(0), K = x.size(1), N = act ? w.size(0) / 2 : w.size(0);
+  TORCH_CHECK(!act || w.size(0) % 2 == 0, "gate and up have the same rows");
+  TORCH_CHECK(K % 64 == 0 && K > 0 && K < (1 << 24) && N % 8 == 0 && N > 0 && N < (1 << 30) && M < (1 << 30),
+              "linear_tiles: K % 64, N % 8 required");
+  TORCH_CHECK(((M + 63) / 64) * ((N + 127) / 128) < (1 << 27), "linear_tiles: too many tiles");
+  const bool biased = bias.numel() > 0;
+  if (biased) {
+    CHECK_BF16_CONTIG(bias);
+    TORCH_CHECK(act == 0 && bias.numel() == N && bias.device() == x.device(), "bias [N] of a plain product");
+  }
+  auto on_16 = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  TORCH_CHECK(on_16(x) && on_16(w) && (!biased || on_16(bias)), "linear_tiles: operands begin on 16 bytes");
+  auto out = torch::empty({M, N}, x.options());
+  if (M == 0) return out;
+  TORCH_CHECK(launch_linear_tiles(out.data_ptr(), x.data_ptr(), w.data_ptr(), biased ? bias.data_ptr() : nullptr, M, N, K,
+                                  act, mj, limit, alpha, cur_stream()) == 0,
+              "linear_tiles: 160 KB of LDS are not available");
+  return out;
+}
+
 // topi [T, k] int64 -> (ids [T * k] token of each sorted place, pos [T, k] sorted place of each pair,
 // offsets [E + 1]); a pair without an expert of 0..E-1 gets pos -1
 std::vector<torch::Tensor> moe_sort(torch::Tensor topi, int64_t E) {
@@ -564,6 +596,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_norm_rows", &embed_norm_rows);
   m.def("rope_store_rows", &rope_store_rows);
   m.def("decode_inputs", &decode_inputs);
+  m.def("linear_tiles", &linear_tiles);
+  m.def("linear_tiles_rows", &linear_tiles_rows);
   m.def("moe_gateup", &moe_gateup);
   m.def("moe_down", &moe_down);
   m.def("moe_sort", &moe_sort);

@@ -55,7 +55,7 @@ __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t*
       const int tok = ids[r];
       xr.at[i] = (uint64_t)(tok >= 0 ? a + (int64_t)tok * K : zeros) + k0 * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
     }
-    tile_product<MJ>(acc, wr, xr, stages, smem);
+    tile_product<MJ>(acc, wr, xr, stages, stages * (blockIdx.x & 7) / 8, smem);
     const int n = n0 + (wave >> 1) * 64;
     tile_store<4, MJ>(out + (int64_t)m * N + n, N, m_end - m, N - n, smem, [&](int i, int j) {
       float v[4];
@@ -70,7 +70,7 @@ __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t*
     const int n_put = n0 + wave * 64, m_put = m0 + wave * MJ * 8;
     const TileRows wr(w + ((int64_t)e * N + n_put) * K + k0, N - n_put, 64, K, lane);
     const TileRows xr(a + (int64_t)m_put * K + k0, m_end - m_put, MJ * 8, K, lane);
-    tile_product<MJ>(acc, wr, xr, stages, smem);
+    tile_product<MJ>(acc, wr, xr, stages, stages * (blockIdx.x & 7) / 8, smem);
     if (sh.shares > 1 && !tile_fold<MJ>(acc, sh.part, sh.share, sh.shares, sh.count, smem)) return;
     const int n = n0 + (wave >> 1) * 128;
     tile_store<8, MJ>(out + (int64_t)m * N + n, N, m_end - m, N - n, smem,

@@ -120,7 +120,8 @@ struct TileRing {
 // acc += W X^T over K; w: this wave's 64 of the 256 rows, x: its 8 * MJ of the 32 * MJ. Ends with all waves past
 // their last LDS read.
 template <int MJ, class X>
-__device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows& w, const X& x, int stages, char* smem) {
+__device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows& w, const X& x, int stages, int start,
+                                             char* smem) {
   constexpr int STRIDE = TileRing<MJ>::STRIDE, RING = TileRing<MJ>::RING;
   constexpr int F = 8 * MJ;              // matrix instructions of a half
   constexpr int NR = 8 + MJ;             // LDS reads of a half
@@ -149,6 +150,10 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows
     if (d < 2 * MJ && (d & 1)) x.copy(i, k_off, x_put + buf + i * 1024);
     else w.copy(i, k_off, w_put + buf + i * 1024);
   };
+  auto k_at = [&](int t) {               // of the t-th stage in work; behind the last one, that one's
+    const int i = min(t, stages - 1) + start;
+    return (uint32_t)(i < stages ? i : i - stages) * 128;
+  };
   bf16x8_mfma a[2][8], b[2][MJ];
   auto read = [&](int ks, int r, uint32_t buf) {
     if (r < 2 * MJ && !(r & 1)) b[ks][r >> 1] = get(x_get[ks] + buf + (r >> 1) * 2048);
@@ -166,7 +171,7 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows
 #pragma unroll
   for (int t = 0; t < RING; ++t)         // of fewer stages the last one again: the counts below stand
 #pragma unroll
-    for (int d = 0; d < ND; ++d) put(d, (uint32_t)min(t, stages - 1) * 128, t * STRIDE);
+    for (int d = 0; d < ND; ++d) put(d, k_at(t), t * STRIDE);
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"((RING - 1) * ND) : "memory");
 #pragma unroll
   for (int r = 0; r < NR; ++r) read(0, r, 0);
@@ -175,7 +180,7 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows
 #pragma unroll 1
   for (int s = 0; s < stages; ++s) {
     // behind the last stage that one is copied again and nothing of it used: no branches
-    const uint32_t k_off = (uint32_t)min(s + RING, stages - 1) * 128;
+    const uint32_t k_off = k_at(s + RING);
     TP_HOLD;
 #pragma unroll
     for (int f = 0; f < F; ++f) {
@@ -200,6 +205,11 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows
     buf = next;
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  // what follows reads sums out of the accumulation registers; it is held off the loop, which must not move them
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < MJ; ++j) asm volatile("" : "+a"(acc[i][j]));
 }
 
 // Sums of a tile whose K is shared by ``shares`` workgroups: each leaves its own in part

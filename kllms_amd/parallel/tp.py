@@ -23,6 +23,8 @@ import torch
 import torch.distributed as dist
 import torch.nn as nn
 
+from .. import ops
+
 
 @dataclass
 class ParallelContext:
@@ -103,7 +105,7 @@ class ColumnParallelLinear(nn.Module):
         return torch.cat(pieces, dim=0)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return torch.nn.functional.linear(x, self.weight, self.bias)
+        return ops.linear(x, self.weight, self.bias)
 
 
 class RowParallelLinear(nn.Module):
@@ -121,7 +123,7 @@ class RowParallelLinear(nn.Module):
         )
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        y = torch.nn.functional.linear(x, self.weight)
+        y = ops.linear(x, self.weight)
         return self.ctx.all_reduce(y)
 
 

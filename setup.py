@@ -30,6 +30,7 @@ SOURCES = [
         "allreduce.hip",
         "moe.hip",
         "linear_rows.hip",
+        "linear_tiles.hip",
         "decode_rows.hip",
         "levenshtein.hip",
     )

@@ -1,0 +1,108 @@
+"""Products of many rows on the tile kernel: edges of its tiles against float64, and the calls that stay with the library."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from kllms_amd import ops
+
+DEV = "cuda:0"
+gpu = pytest.mark.gpu
+
+
+def _operands(M, N, K, gated, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn((2 if gated else 1) * N, K, generator=g, device=DEV) * K ** -0.5).bfloat16()
+    return x, w
+
+
+def _near(got, ref, sums):
+    # half a bf16 step of the result, and fp32 sums of K terms in any order: 2^-24 of the sum of their sizes a step
+    return ((got.double() - ref).abs() <= 2 ** -8 * ref.abs() + sums).all()
+
+
+# one row, one column unit, odd rows behind a tile, a last column tile of 8, one stage and odd numbers of them
+SIZES = [(1, 8, 64), (33, 264, 128), (129, 520, 1088), (257, 256, 2112), (1031, 1288, 192)]
+
+
+@gpu
+@pytest.mark.parametrize("mj", range(2, 9))
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_tiles_against_float64(M, N, K, mj):
+    C = ops._hip_or_raise()
+    x, w = _operands(M, N, K, False)
+    bias = torch.randn(N, device=DEV).bfloat16()
+    ref = x.double() @ w.double().t()
+    slack = K * 2 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert _near(C.linear_tiles(x, w, bias[:0], 0, mj, 0.0, 0.0), ref, slack)
+    assert _near(C.linear_tiles(x, w, bias, 0, mj, 0.0, 0.0), ref + bias.double(), slack + 1e-6)
+    x, w = _operands(M, N, K, True, 1)
+    g, u = (x.double() @ w.double().t()).chunk(2, -1)
+    slack = K * 2 ** -24 * (x.double().abs() @ w.double().abs().t())
+    # the activations' slopes are below 1.1 (silu) and 1.1 * alpha, their values below the other factor
+    slack = 3 * (slack[:, :N] * (u.abs() + 1) + slack[:, N:] * (g.abs() + 1)) + 1e-5
+    assert _near(C.linear_tiles(x, w, bias[:0], 1, mj, 0.0, 0.0), F.silu(g) * u, slack)
+    c, d = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+    assert _near(C.linear_tiles(x, w, bias[:0], 2, mj, 1.5, 1.702), c * torch.sigmoid(1.702 * c) * (d + 1), slack)
+
+
+@gpu
+@pytest.mark.parametrize("M,N,K,act", [(300, 3216, 2048, 0), (1170, 6144, 4096, 0), (777, 8192, 2048, 1), (400, 8192, 2048, 2)])
+def test_entry_points_against_float64(M, N, K, act):
+    x, w = _operands(M, N, K, act > 0, 2)
+    y = x.double() @ w.double().t()
+    if act == 0:
+        got, ref = ops.linear(x, w), y
+    elif act == 1:
+        got, ref = ops.linear_silu(x, w), F.silu(y[:, :N]) * y[:, N:]
+    else:
+        c, d = y[:, :N].clamp(max=7.0), y[:, N:].clamp(-7.0, 7.0)
+        got, ref = ops.linear_clamped_glu(x, w, 7.0, 1.702), c * torch.sigmoid(1.702 * c) * (d + 1)
+    # one rounding to bf16 of values of a normal shape is 0.0017 of them in the 2-norm
+    assert (got.double() - ref).norm() <= 0.002 * ref.norm()
+
+
+@gpu
+def test_extreme_sums_of_the_clamped_form():
+    x, w = _operands(256, 128, 64, True, 3)
+    got = ops._hip_or_raise().linear_tiles((x * 1000).contiguous(), w, x[:0, 0], 2, 2, 7.0, 1.702)
+    y = (x * 1000).double() @ w.double().t()
+    c, d = y[:, :128].clamp(max=7.0), y[:, 128:].clamp(-7.0, 7.0)
+    assert torch.isfinite(got).all()
+    # factors of at most 8 beside slopes below 1.1, as above
+    slack = 64 * 2 ** -24 * ((x.double() * 1000).abs() @ w.double().abs().t())
+    assert _near(got, c * torch.sigmoid(1.702 * c) * (d + 1), 9 * (slack[:, :128] + slack[:, 128:]) + 1e-5)
+
+
+@gpu
+def test_calls_that_stay_with_the_library():
+    x, w = _operands(512, 2048, 1024, False)
+    assert ops._tiles(x, w, 0)
+    assert not ops._tiles(x[:128], w, 0) and not ops._tiles(x.float(), w.float(), 0)
+    assert not ops._tiles(x[:, ::2], w[:, ::2], 0) and not ops._tiles(x[:, :1000].contiguous(), w[:, :1000].contiguous(), 0)
+    assert not ops._tiles(x.t().contiguous().t(), w, 0) and not ops._tiles(x.view(2, 256, 1024), w, 0)
+    off = torch.empty(x.numel() + 1, device=DEV, dtype=x.dtype)[1:].view_as(x).copy_(x)
+    assert not ops._tiles(off, w, 0) and torch.allclose(ops.linear(off, w).float(), ops.linear(x, w).float(), atol=0.05)
+    assert not ops._tiles(x, w, 0, torch.zeros(2048, device=DEV))
+    xg = x.clone().requires_grad_()
+    ops.linear(xg, w).sum().backward()
+    assert xg.grad is not None
+    with torch.no_grad():
+        assert ops._tiles(xg, w, 0)
+    got = torch.func.vmap(lambda t: ops.linear(t, w))(x.view(2, 256, 1024))
+    assert torch.allclose(got.view(512, -1).float(), ops.linear(x, w).float(), atol=0.05)
+
+
+def test_rule_of_the_tiles():
+    if not ops.hip_available():
+        pytest.skip("extension not built")
+    rows = ops._hip_or_raise().linear_tiles_rows
+    assert rows(128, 8192, 2048, 1) == 0                       # few rows
+    assert rows(300, 4096, 14336, 0) == 0                      # long K on few tiles
+    assert rows(7777, 4096, 4096, 0) == 0                      # 496 tiles of the 512 of two rounds
+    assert rows(300, 14336, 4096, 1) == 5                      # 224 tiles of 150 rows
+    assert rows(11700, 4096, 14336, 0) == 8                    # 736 tiles in three rounds
+    for M in range(1, 13000, 97):
+        for N, K, act in ((4096, 4096, 0), (3216, 2048, 0), (14336, 4096, 1)):
+            assert rows(M, N, K, act) in (0, 2, 3, 4, 5, 6, 7, 8)
