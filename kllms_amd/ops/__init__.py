@@ -269,7 +269,7 @@ def _plain_call(*ts: torch.Tensor) -> bool:
 
 
 def _tiles(x: torch.Tensor, w: torch.Tensor, act: int, bias: Optional[torch.Tensor] = None) -> int:
-    """Rows of a tile, in steps of 32, where the tile kernel takes x [M, K] @ w^T, or 0: bf16 on the GPU, contiguous,
+    """Rows of a tile, in steps of 32, + 16 for shares of K, where the tile kernel takes x [M, K] @ w^T, or 0: bf16 on the GPU, contiguous,
     sizes that its 16-byte accesses and 64-deep stages divide, no gradient to keep, and the faster side of the rule."""
     if (x.dim() != 2 or x.shape[0] <= 128 or not x.is_cuda or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16
             or w.dim() != 2 or x.device != w.device or _force_torch()):
@@ -294,20 +294,20 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     """x @ w^T + bias: prompts on the tile kernel where that is the faster one, everything else in the library."""
     mj = _tiles(x, w, 0, bias)
     if mj:
-        return _C.linear_tiles(x, w, bias if bias is not None else _none(x), 0, mj, 0.0, 0.0)
+        return _C.linear_tiles(x, w, bias if bias is not None else _none(x), 0, mj & 15, mj > 15, 0.0, 0.0)
     return torch.nn.functional.linear(x, w, bias)
 
 
 def linear_silu(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     """silu(gate) * up of a fused [gate; up] matrix for prompts, or None where the tile kernel does not take it."""
     mj = _tiles(x, w, 1)
-    return _C.linear_tiles(x, w, _none(x), 1, mj, 0.0, 0.0) if mj else None
+    return _C.linear_tiles(x, w, _none(x), 1, mj & 15, mj > 15, 0.0, 0.0) if mj else None
 
 
 def linear_clamped_glu(x: torch.Tensor, w: torch.Tensor, limit: float, alpha: float) -> Optional[torch.Tensor]:
     """clamped_glu of a fused [gate; up] matrix for prompts, or None where the tile kernel does not take it."""
     mj = _tiles(x, w, 2)
-    return _C.linear_tiles(x, w, _none(x), 2, mj, limit, alpha) if mj else None
+    return _C.linear_tiles(x, w, _none(x), 2, mj & 15, mj > 15, limit, alpha) if mj else None
 
 
 def embed_norm_rows(ids, table, weight, eps, unknown=None):

@@ -358,13 +358,14 @@ void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor
 
 // --- products of many rows (linear_tiles.hip) ---------------------------------
 extern "C" int linear_tiles_rows(int64_t M, int64_t N, int64_t K, int act);
-extern "C" int launch_linear_tiles(void* out, const void* x, const void* w, const void* bias, int M, int N, int K, int act,
-                                   int mj, float limit, float alpha, hipStream_t stream);
+extern "C" int64_t linear_tiles_room(int mj, int* zeros);
+extern "C" int launch_linear_tiles(void* out, const void* x, const void* w, const void* bias, float* part, int* count, int M,
+                                   int N, int K, int act, int mj, float limit, float alpha, hipStream_t stream);
 
 // act 0: x [M, K] @ w [N, K]^T + bias (or an empty one); 1, 2: w [2 N, K], silu(gate) * up or the clamped form.
-// mj: 32-row steps of a tile, 2 to 8
-torch::Tensor linear_tiles(torch::Tensor x, torch::Tensor w, torch::Tensor bias, int act, int mj, double limit,
-                           double alpha) {
+// mj: 32-row steps of a tile, 2 to 8; share: the last round's tiles are shared out over K
+torch::Tensor linear_tiles(torch::Tensor x, torch::Tensor w, torch::Tensor bias, int act, int mj, bool share,
+                           double limit, double alpha) {
   CHECK_BF16_CONTIG(x); CHECK_BF16_CONTIG(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) && x.device() == w.device(), "x [M, K], w [N, K]");
   TORCH_CHECK(act >= 0 && act <= 2 && mj >= 2 && mj <= 8, "linear_tiles: act 0 to 2, mj 2 to 8");
@@ -382,7 +383,14 @@ torch::Tensor linear_tiles(torch::Tensor x, torch::Tensor w, torch::Tensor bias,
   TORCH_CHECK(on_16(x) && on_16(w) && (!biased || on_16(bias)), "linear_tiles: operands begin on 16 bytes");
   auto out = torch::empty({M, N}, x.options());
   if (M == 0) return out;
-  TORCH_CHECK(launch_linear_tiles(out.data_ptr(), x.data_ptr(), w.data_ptr(), biased ? bias.data_ptr() : nullptr, M, N, K,
+  torch::Tensor part, count;
+  if (share) {
+    int zeros = 0;
+    part = torch::empty({linear_tiles_room(mj, &zeros)}, x.options().dtype(torch::kFloat));
+    count = torch::zeros({zeros}, x.options().dtype(torch::kInt));
+  }
+  TORCH_CHECK(launch_linear_tiles(out.data_ptr(), x.data_ptr(), w.data_ptr(), biased ? bias.data_ptr() : nullptr,
+                                  share ? part.data_ptr<float>() : nullptr, share ? count.data_ptr<int>() : nullptr, M, N, K,
                                   act, mj, limit, alpha, cur_stream()) == 0,
               "linear_tiles: 160 KB of LDS are not available");
   return out;

@@ -22,33 +22,36 @@ def _near(got, ref, sums):
     return ((got.double() - ref).abs() <= 2 ** -8 * ref.abs() + sums).all()
 
 
-# one row, one column unit, odd rows behind a tile, a last column tile of 8, one stage and odd numbers of them
-SIZES = [(1, 8, 64), (33, 264, 128), (129, 520, 1088), (257, 256, 2112), (1031, 1288, 192)]
+# one row, one column unit, odd rows behind a tile, a last column tile of 8, one stage and odd numbers of them; shares of
+# 33 stages in two, of 65 in four
+SIZES = [(1, 8, 64), (33, 264, 128), (129, 520, 1088), (257, 256, 2112), (1031, 1288, 192),
+         (70, 2056, 4160)]
 
 
 @gpu
 @pytest.mark.parametrize("mj", range(2, 9))
+@pytest.mark.parametrize("share", [False, True])
 @pytest.mark.parametrize("M,N,K", SIZES)
-def test_tiles_against_float64(M, N, K, mj):
+def test_tiles_against_float64(M, N, K, share, mj):
     C = ops._hip_or_raise()
     x, w = _operands(M, N, K, False)
     bias = torch.randn(N, device=DEV).bfloat16()
     ref = x.double() @ w.double().t()
     slack = K * 2 ** -24 * (x.double().abs() @ w.double().abs().t())
-    assert _near(C.linear_tiles(x, w, bias[:0], 0, mj, 0.0, 0.0), ref, slack)
-    assert _near(C.linear_tiles(x, w, bias, 0, mj, 0.0, 0.0), ref + bias.double(), slack + 1e-6)
+    assert _near(C.linear_tiles(x, w, bias[:0], 0, mj, share, 0.0, 0.0), ref, slack)
+    assert _near(C.linear_tiles(x, w, bias, 0, mj, share, 0.0, 0.0), ref + bias.double(), slack + 1e-6)
     x, w = _operands(M, N, K, True, 1)
     g, u = (x.double() @ w.double().t()).chunk(2, -1)
     slack = K * 2 ** -24 * (x.double().abs() @ w.double().abs().t())
     # the activations' slopes are below 1.1 (silu) and 1.1 * alpha, their values below the other factor
     slack = 3 * (slack[:, :N] * (u.abs() + 1) + slack[:, N:] * (g.abs() + 1)) + 1e-5
-    assert _near(C.linear_tiles(x, w, bias[:0], 1, mj, 0.0, 0.0), F.silu(g) * u, slack)
+    assert _near(C.linear_tiles(x, w, bias[:0], 1, mj, share, 0.0, 0.0), F.silu(g) * u, slack)
     c, d = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
-    assert _near(C.linear_tiles(x, w, bias[:0], 2, mj, 1.5, 1.702), c * torch.sigmoid(1.702 * c) * (d + 1), slack)
+    assert _near(C.linear_tiles(x, w, bias[:0], 2, mj, share, 1.5, 1.702), c * torch.sigmoid(1.702 * c) * (d + 1), slack)
 
 
 @gpu
-@pytest.mark.parametrize("M,N,K,act", [(300, 3216, 2048, 0), (1170, 6144, 4096, 0), (777, 8192, 2048, 1), (400, 8192, 2048, 2)])
+@pytest.mark.parametrize("M,N,K,act", [(300, 3216, 2048, 0), (1170, 6144, 4096, 0), (700, 2048, 8192, 0), (777, 8192, 2048, 1), (400, 8192, 2048, 2)])
 def test_entry_points_against_float64(M, N, K, act):
     x, w = _operands(M, N, K, act > 0, 2)
     y = x.double() @ w.double().t()
@@ -66,7 +69,7 @@ def test_entry_points_against_float64(M, N, K, act):
 @gpu
 def test_extreme_sums_of_the_clamped_form():
     x, w = _operands(256, 128, 64, True, 3)
-    got = ops._hip_or_raise().linear_tiles((x * 1000).contiguous(), w, x[:0, 0], 2, 2, 7.0, 1.702)
+    got = ops._hip_or_raise().linear_tiles((x * 1000).contiguous(), w, x[:0, 0], 2, 2, False, 7.0, 1.702)
     y = (x * 1000).double() @ w.double().t()
     c, d = y[:, :128].clamp(max=7.0), y[:, 128:].clamp(-7.0, 7.0)
     assert torch.isfinite(got).all()
@@ -99,10 +102,11 @@ def test_rule_of_the_tiles():
         pytest.skip("extension not built")
     rows = ops._hip_or_raise().linear_tiles_rows
     assert rows(128, 8192, 2048, 1) == 0                       # few rows
-    assert rows(300, 4096, 14336, 0) == 0                      # long K on few tiles
+    assert rows(256, 4096, 14336, 0) == 0                      # long K on few tiles
+    assert rows(1170, 4096, 14336, 0) == 5 + 16                # 128 tiles of 147 rows, in two shares each
     assert rows(7777, 4096, 4096, 0) == 0                      # 496 tiles of the 512 of two rounds
     assert rows(300, 14336, 4096, 1) == 5                      # 224 tiles of 150 rows
     assert rows(11700, 4096, 14336, 0) == 8                    # 736 tiles in three rounds
     for M in range(1, 13000, 97):
         for N, K, act in ((4096, 4096, 0), (3216, 2048, 0), (14336, 4096, 1)):
-            assert rows(M, N, K, act) in (0, 2, 3, 4, 5, 6, 7, 8)
+            assert rows(M, N, K, act) in (0, 2, 3, 4, 5, 6, 7, 8)      # K below 8192: never shared
