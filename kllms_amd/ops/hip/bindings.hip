@@ -18,7 +18,7 @@ extern "C" void launch_attn_decode(bf16_t*, float*, const bf16_t*, const void*, 
 extern "C" void launch_attn_prefill(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, int, int, float, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill_paged(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, const int*, const int*, const int*, int, float, int, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill_plan(int*, const int*, int, int, hipStream_t);
-extern "C" int sample_slices(int B, int V);
+extern "C" int64_t sample_room(int B, int V, int masked);
 extern "C" void launch_sample(int64_t*, float*, void*, const float*, const float*, const float*, const int*, const int64_t*, const int64_t*, const uint32_t*, int, int, float*, hipStream_t);
 extern "C" __global__ void mfma_selftest_kernel(float*, const bf16_t*, const bf16_t*);
 
@@ -249,8 +249,8 @@ void sample(torch::Tensor tokens, torch::Tensor logprobs, torch::Tensor logits,
   const uint32_t* mptr = mask.numel() > 0
       ? reinterpret_cast<const uint32_t*>(mask.data_ptr<int>()) : nullptr;
   if (B == 0 || V == 0) return;
-  // per-slice results: 6 words each (SlicePart)
-  auto parts = torch::empty({(int64_t)B * sample_slices(B, V) * 3},
+  // per-slice results and lists
+  auto parts = torch::empty({sample_room(B, V, mptr != nullptr)},
                             torch::dtype(torch::kLong).device(logits.device()));
   launch_sample(tokens.data_ptr<int64_t>(), logprobs.data_ptr<float>(), parts.data_ptr(),
                 logits.data_ptr<float>(), temperatures.data_ptr<float>(), top_ps.data_ptr<float>(),

@@ -13,19 +13,16 @@
 // for 120 x 128256 tokens on 1024 SIMDs (the logits alone: 61.6 MB, 13 us at the
 // 4.7 TB/s a copy reaches).
 //
-// Rows with top-p / top-k (sample_final): a 256-bin histogram of the scaled mass
-// and count (per-wave copies: a single one serialises on same-bin LDS atomics)
-// names the boundary bin, up to 3 refinements at 256x finer resolution each
-// (20/256^4 ~ 5e-9 in scaled-logit space: exact up to fp32 rounding of the
-// logits) the threshold in it. Atomics and exponentials are what a sweep costs,
-// so the bins near the max are counted first, with their tokens listed in LDS; a
-// peaked row needs no more. Flat rows take further sweeps, and a boundary bin that
-// outgrows the list is refined by rescans of the row.
+// Rows with top-p / top-k: each slice of a long row lists its highest tokens (slice_list), and sample_final finds the
+// cut in the lists alone where they reach it. It counts their scaled mass and number in 256 bins (per-wave copies: a
+// single one serialises on same-bin LDS atomics), which names the boundary bin, and up to 3 refinements at 256x finer
+// resolution each (20/256^4 ~ 5e-9 in scaled-logit space: exact up to fp32 rounding of the logits) the threshold in it.
+// Rows whose cut lies behind the lists, and rows without any, are swept by their one workgroup: atomics and exponentials
+// are what a sweep costs, so the bins near the max are counted first, with their tokens listed in LDS; flat rows take
+// further sweeps, and a boundary bin that outgrows the list is refined by rescans of the row.
 //
-// Measured, 128256 tokens a row, beside one workgroup per row walking it three to
-// six times: 120 rows, half of them with top-p 0.95 and top-k 50, 79 us (346);
-// 16 masked rows 12.2 us (136). sample_part is 29 us of the former, at its bound;
-// sample_final 52, the slowest truncated row's sweeps.
+// Measured, 128256 tokens a row: 120 rows, half of them with top-p 0.95 and top-k 50, 50 us (79 with sweeps alone, 346 with
+// one workgroup per row walking it three to six times); 8 rows, all truncated, 24 us (52); 16 masked rows 12.2 us.
 //
 // The draw is counter-based: hash(seed, step, token), identical regardless of
 // batch composition and of the slicing. What follows from a sum is so to fp32
@@ -64,14 +61,20 @@ __device__ __forceinline__ float sx_of(float x, float inv_t, float smax) {
 #define PT 256             // threads of a slice's workgroup
 #define PU 8               // logits in flight per thread
 
-// what a slice hands to sample_final: 6 words
+// what a slice hands to sample_final: 10 words
 struct SlicePart {
   float max;
   float sum;                 // sum of exp(x - max)
   int arg;                   // lowest token at the max, -1: none above -inf
   float ssum;                // rows with top-p / top-k: sum of exp((x - max) / temperature)
   unsigned long long best;   // ordered key bits << 32 | token
+  float edge;                // rows with top-p / top-k: the slice's tokens from this logit on are in its list; inf: none
+  int listed;                // how many they are
+  float mass;                // and their sum of exp((x - max) / temperature)
+  int unused;
 };
+
+struct SliceToken { float x; int tok; };
 
 __device__ __forceinline__ unsigned long long pack_key(float key, int tok) {
   uint32_t k = __float_as_uint(key);
@@ -191,8 +194,108 @@ __device__ __forceinline__ SlicePart slice_part(const float* __restrict__ row, c
     }
     if (p.arg == 0x7fffffff) p.arg = -1;
     p.ssum = SS;
+    p.edge = INFINITY;
+    p.listed = 0;
+    p.mass = 0.0f;
   }
   return p;
+}
+
+#define SHORT 1024         // tokens that a slice looks at more closely
+
+// The tokens of [lo, hi) near the slice's max M, for a row that truncates: as deep below it as ``cap`` tokens reach, in
+// steps of 0.3 of scaled logit (2.5 where a step of that holds more than SHORT), and 20 at most. So with top-k up to
+// about cap the cut always lies in the lists: the slice whose list ends first has that many above its end. Two more walks
+// over a slice that the caches still hold, by all workgroups at once, for a walk over the whole row by one. False: not
+// even the first step fits.
+__device__ __forceinline__ bool slice_list(SliceToken* __restrict__ list, int cap, const float* __restrict__ row,
+                                           const uint32_t* __restrict__ mrow, float temp, float M, int lo, int hi,
+                                           float& edge, int& listed, float& mass) {
+  constexpr float STEP = 2.5f, FINE = STEP / 8;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const float inv_t = (temp > 0.0f) ? 1.0f / temp : 0.0f;
+  __shared__ int counts[8], fine[8], put, put2;
+  __shared__ SliceToken near[SHORT];
+  __shared__ float red[16];
+  if (tid < 8) counts[tid] = fine[tid] = 0;
+  if (tid == 8) put = put2 = 0;
+  __syncthreads();
+  auto walk = [&](auto f) {              // f(token, logit, there is one); all lanes take every step
+    for (int i0 = lo; i0 < hi; i0 += PT * PU) {
+      float x[PU];
+#pragma unroll
+      for (int j = 0; j < PU; ++j) x[j] = row[min(i0 + j * PT + tid, hi - 1)];
+#pragma unroll
+      for (int j = 0; j < PU; ++j) {
+        const int i = i0 + j * PT + tid;
+        f(i, x[j], i < hi && (!mrow || ((mrow[i >> 5] >> (i & 31)) & 1)));
+      }
+    }
+  };
+  unsigned long long windows = 0;        // eight counts of 8 bits: a thread has at most 255 tokens
+  walk([&](int, float x, bool ok) {
+    const float d = (M - x) * inv_t * (1.0f / STEP);
+    if (ok && d < 8.0f) windows += 1ull << (8 * (int)d);
+  });
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {          // two counts of 16 bits a word: 64 lanes fit
+    uint32_t w = (uint32_t)(windows >> (16 * k));
+    w = (w & 0xff) | (w & 0xff00) << 8;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) w += __shfl_xor(w, off);
+    if (lane == 0) {
+      atomicAdd(&counts[2 * k], (int)(w & 0xffff));
+      atomicAdd(&counts[2 * k + 1], (int)(w >> 16));
+    }
+  }
+  __syncthreads();
+  int deep = 0, n = 0;
+  while (deep < 8 && n + counts[deep] <= cap) n += counts[deep++];
+  const bool closely = deep < 8 && n + counts[deep] <= SHORT;
+  if (deep == 0 && !closely) return false;
+  const float top = M - (deep + closely) * STEP * temp;
+  walk([&](int i, float x, bool ok) {
+    const bool in = ok && x >= top;
+    const unsigned long long votes = __ballot(in);
+    if (!votes) return;
+    int at = 0;
+    if (lane == 0) at = atomicAdd(&put, (int)__popcll(votes));
+    at = __shfl(at, 0) + (int)__popcll(votes & ((1ull << lane) - 1));
+    if (in && at < SHORT) near[at] = SliceToken{x, i};
+  });
+  __syncthreads();
+  const int found = put;                 // a token at a window's end can fall on the other side of ``top``
+  if (found > SHORT) return false;
+  float from = top;
+  if (closely) {
+    for (int e = tid; e < found; e += PT) {
+      const float d = ((M - near[e].x) * inv_t * (1.0f / STEP) - deep) * 8.0f;
+      if (d >= 0.0f) atomicAdd(&fine[min((int)d, 7)], 1);
+    }
+    __syncthreads();
+    int k = 0;
+    while (k < 8 && n + fine[k] <= cap) n += fine[k++];
+    if (deep == 0 && k == 0) return false;
+    from = M - (deep * STEP + k * FINE) * temp;
+  }
+  float sum = 0.0f;
+  for (int e0 = 0; e0 < found; e0 += PT) {
+    const int e = e0 + tid;
+    const SliceToken t = near[min(e, found - 1)];
+    const bool in = e < found && t.x >= from;
+    const unsigned long long votes = __ballot(in);
+    if (!votes) continue;
+    int at = 0;
+    if (lane == 0) at = atomicAdd(&put2, (int)__popcll(votes));
+    at = __shfl(at, 0) + (int)__popcll(votes & ((1ull << lane) - 1));
+    if (!in) continue;
+    sum += __expf((t.x - M) * inv_t);
+    if (at < cap) list[at] = t;
+  }
+  mass = block_reduce_sum<PT / WAVE>(sum, red);
+  listed = put2;
+  edge = from;
+  return listed <= cap;
 }
 
 extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
@@ -202,13 +305,35 @@ extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
     const int* __restrict__ top_ks, const int64_t* __restrict__ seeds,
     const int64_t* __restrict__ steps,
     const uint32_t* __restrict__ mask,    // [B, ceil(V/32)] or nullptr
+    SliceToken* __restrict__ lists, int cap,   // [B, slices, cap] or nullptr
     int V, int slice) {
   const int b = blockIdx.y;
-  const int lo = blockIdx.x * slice;
+  const int lo = blockIdx.x * slice, hi = min(V, lo + slice);
   const float temp = temperatures[b];
-  const SlicePart p = slice_part<PT>(logits + (int64_t)b * V, mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr, temp,
-                                     temp != 0.0f && truncates(top_ps[b], top_ks[b], V), draw_base(seeds[b], steps[b]),
-                                     lo, min(V, lo + slice));
+  const float* row = logits + (int64_t)b * V;
+  const uint32_t* mrow = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
+  const bool cuts = temp != 0.0f && truncates(top_ps[b], top_ks[b], V);
+  SlicePart p = slice_part<PT>(row, mrow, temp, cuts, draw_base(seeds[b], steps[b]), lo, hi);
+  // a top-k that the lists are long enough for lies in them for sure; where only a share of the mass is asked for the
+  // try costs nothing as long as the chip is not full (16 masked rows of 128256, top-p 0.9: 127 us without, 33 with; 120
+  // flat rows whose nucleus is half of the vocabulary: 292 and 312)
+  if (cuts && lists && ((top_ks[b] > 0 && top_ks[b] <= cap) || (int64_t)gridDim.y * V <= 1 << 22)) {
+    __shared__ float top;
+    // without an allowed token there is nothing to list; a max or a sum that is not finite leaves the row to the sweeps
+    if (threadIdx.x == 0) top = p.arg < 0 ? -INFINITY : p.sum - p.sum == 0.0f ? p.max : INFINITY;
+    __syncthreads();
+    float edge = top, mass = 0.0f;
+    int listed = 0;
+    if (top - top == 0.0f && !slice_list(lists + ((int64_t)b * gridDim.x + blockIdx.x) * cap, cap, row, mrow, temp, top,
+                                         lo, hi, edge, listed, mass)) {
+      edge = INFINITY;
+      listed = 0;
+      mass = 0.0f;
+    }
+    p.edge = edge;
+    p.listed = listed;
+    p.mass = mass;
+  }
   if (threadIdx.x == 0) parts[(int64_t)b * gridDim.x + blockIdx.x] = p;
 }
 
@@ -220,6 +345,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
     float* __restrict__ out_logprobs,     // [B]
     const SlicePart* __restrict__ parts,  // [B, slices], slices <= 64
     int slices,
+    const SliceToken* __restrict__ lists, int cap,   // [B, slices, cap], slices * cap <= SLIST, or nullptr
     const float* __restrict__ logits,     // [B, V]
     const float* __restrict__ temperatures,
     const float* __restrict__ top_ps,
@@ -242,6 +368,9 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   __shared__ float sh_max, sh_sum, sh_ssum;
   __shared__ int sh_argmax;
   __shared__ unsigned long long sh_best;
+  __shared__ float sh_edge;              // all tokens of the row from this logit on are in the slices' lists
+  __shared__ float sh_mass;              // and what those weigh, against the max
+  __shared__ int sh_count[64], sh_total;
   if constexpr (WHOLE) {
     const SlicePart p = slice_part<NT>(row, mrow, temp, temp != 0.0f && truncates(top_p, top_k, V),
                                        draw_base(seeds[b], steps[b]), 0, V);
@@ -253,7 +382,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
       sh_best = p.best;
     }
   } else if (wid == 0) {
-    SlicePart p{-INFINITY, 0.0f, -1, 0.0f, (unsigned long long)NO_KEY << 32};
+    SlicePart p{-INFINITY, 0.0f, -1, 0.0f, (unsigned long long)NO_KEY << 32, -INFINITY, 0, 0.0f, 0};
     if (lane < slices) p = parts[(int64_t)b * slices + lane];
     const float M = wave_reduce_max(p.max);
     const float S = wave_reduce_sum(p.sum * (p.max == M ? 1.0f : exp_from(p.max, M)));
@@ -263,7 +392,16 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) a = min(a, __shfl_xor(a, off));
     const unsigned long long w = wave_max_u64(p.best);
+    const float edge = wave_reduce_max(p.edge);
+    const float lmass = wave_reduce_sum(p.listed == 0 ? 0.0f : p.mass * (p.max == M ? 1.0f : __expf((p.max - M) * inv_t)));
+    int total = p.listed;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
+    sh_count[lane] = p.listed;
     if (lane == 0) {
+      sh_edge = edge;
+      sh_mass = lmass;
+      sh_total = total;
       sh_max = M;
       sh_sum = S;
       sh_ssum = SS;
@@ -413,15 +551,28 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   const float need_mass = top_p < 1.0f ? top_p * (sh_ssum * __expf(sx_of(gmax, inv_t, smax))) : INFINITY;
   const unsigned int need_cnt = (top_k > 0 && top_k < V) ? (unsigned)top_k : 0xffffffffu;
   const uint64_t base = draw_base(seeds[b], steps[b]);
-  clear_hist();
-  if (tid == 0) { sh_listed = 0; sh_best = (unsigned long long)NO_KEY << 32; }
-  __syncthreads();
-  for (int part = 0; part < 3; ++part) {
-    const int from = part == 0 ? 0 : part == 1 ? SNEAR : SMID;
-    const int to = part == 0 ? SNEAR : part == 1 ? SMID : SBINS;
-    sweep(part < 2 ? -to * (SRANGE / SBINS) - 1e-3f : NAN, [&](int i, float x, float sx) {
-      const int bin = coarse_bin(sx);
-      if (bin < from || bin >= to) return;
+  // bins that the slices' lists hold whole; their tokens then stand in for the row if the cut lies there
+  int whole = 0;
+  bool hope = false;
+  if constexpr (!WHOLE)
+    if (lists) {
+      const float deep = -sx_of(sh_edge, inv_t, smax) - 1e-3f;
+      whole = deep > 0.0f ? min((int)(deep * (SBINS / SRANGE)), SBINS) : 0;      // NaN: none
+      hope = (unsigned)sh_total >= need_cnt || sh_mass * 1.001f >= top_p * sh_ssum;
+    }
+  if (tid == 0) sh_best = (unsigned long long)NO_KEY << 32;
+  // where the cut is behind the lists, the sweeps over bins that those hold whole are left out
+  const int after = whole >= SMID ? 2 : whole >= SNEAR ? 1 : 0;
+  for (int part = whole > 0 && hope ? -1 : after; part < 3; part = part < 0 ? after : part + 1) {
+    const int from = part <= after ? 0 : part == 1 ? SNEAR : SMID;
+    const int to = part < 0 ? whole : part == 0 ? SNEAR : part == 1 ? SMID : SBINS;
+    if (part <= after) {
+      __syncthreads();
+      clear_hist();
+      if (tid == 0) sh_listed = 0;
+      __syncthreads();
+    }
+    auto count = [&](int i, float sx, int bin) {
       atomicAdd(&my_mass[bin], __expf(sx));
       atomicAdd(&my_cnt[bin], 1u);
       if (part < 2) {
@@ -431,7 +582,22 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
           list_tok[at] = i;
         }
       }
-    });
+    };
+    if (part < 0) {
+      const SliceToken* mine = lists + (int64_t)b * slices * cap;
+      for (int e = tid; e < slices * cap; e += NT) {
+        if (e % cap >= sh_count[e / cap]) continue;
+        const SliceToken t = mine[e];
+        const float sx = sx_of(t.x, inv_t, smax);
+        const int bin = coarse_bin(sx);
+        if (bin < to) count(t.tok, sx, bin);
+      }
+    } else {
+      sweep(part < 2 ? -to * (SRANGE / SBINS) - 1e-3f : NAN, [&](int i, float, float sx) {
+        const int bin = coarse_bin(sx);
+        if (bin >= from && bin < to) count(i, sx, bin);
+      });
+    }
     __syncthreads();
     fold_hist(from, to);
     __syncthreads();
@@ -465,14 +631,17 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
       }
     }
     __syncthreads();
-    if (sh_cut < SBINS) break;
+    if (sh_cut < SBINS) {
+      if (part >= 0) whole = 0;
+      break;
+    }
   }
 
   // ---- draw over the bins above the boundary --------------------------------
   // afterwards the list holds the boundary bin's tokens, among others, unless
   // they outgrow it
   const int cut = sh_cut;
-  const bool near = cut < SMID && sh_listed <= SLIST;
+  const bool near = (cut < SMID || cut < whole) && sh_listed <= SLIST;   // whole: of the lists that were used, else 0
   const bool fits = near || (cut < SBINS && hist_cnt[cut] <= SLIST);
   float best = -INFINITY;
   int btok = argmax_tok;
@@ -618,12 +787,30 @@ extern "C" int sample_slices(int B, int V) {
   return n < 1 ? 1 : n > 64 ? 64 : n;
 }
 
+// Tokens of a slice's list, or 0: no lists. They cost two more walks over the truncated rows by all workgroups and save
+// the walks of sample_final, one workgroup a row. Worth it on long rows (120 rows of 32000 with top-p and top-k: 33 us
+// without, 37 with; 30 of 50257, masked: 37 and 31) and on as many as leave sample_final the slower part (120 rows of
+// 128256 73 and 61, 250 of 152064 105 and 107; masked, half of them truncated: 171 and 110). Nor have slices lists whose
+// threads would count more than 255 tokens
+static int sample_cap(int B, int V, int n, bool masked) {
+  const int64_t most = masked ? 1 << 26 : 1 << 25;
+  return n > 0 && V > 32768 && (int64_t)B * V <= most && (V + n - 1) / n <= 255 * PT ? SLIST / n : 0;
+}
+
+// words of 8 bytes that a call needs for its slices, and for their lists
+extern "C" int64_t sample_room(int B, int V, int masked) {
+  const int n = sample_slices(B, V);
+  return (int64_t)B * n * (sizeof(SlicePart) / 8 + sample_cap(B, V, n, masked));
+}
+
 extern "C" void launch_sample(int64_t* tokens, float* logprobs, void* parts, const float* logits,
                               const float* temps, const float* top_ps, const int* top_ks,
                               const int64_t* seeds, const int64_t* steps, const uint32_t* mask, int B,
                               int V, float* dbg, hipStream_t stream) {
   const int n = sample_slices(B, V);
   const int slice = n > 0 ? (V + n - 1) / n : V;
+  const int cap = sample_cap(B, V, n, mask != nullptr);
+  SliceToken* lists = cap ? (SliceToken*)((SlicePart*)parts + (int64_t)B * n) : nullptr;   // B is one launch's
   // rows of a launch lie on the grid's y, which ends at 65535
   for (int b = 0; b < B; b += 65535) {
     const int rows = B - b < 65535 ? B - b : 65535;
@@ -632,9 +819,9 @@ extern "C" void launch_sample(int64_t* tokens, float* logprobs, void* parts, con
     const uint32_t* m = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
     if (n > 0)
       hipLaunchKernelGGL(sample_part_kernel, dim3(n, rows), dim3(PT), 0, stream, p, x, temps + b, top_ps + b,
-                         top_ks + b, seeds + b, steps + b, m, V, slice);
+                         top_ks + b, seeds + b, steps + b, m, lists, cap, V, slice);
     hipLaunchKernelGGL(n > 0 ? sample_final_kernel<false> : sample_final_kernel<true>, dim3(rows), dim3(NT), 0, stream,
-                       tokens + b, logprobs + b, (const SlicePart*)p, n, x, temps + b, top_ps + b, top_ks + b,
+                       tokens + b, logprobs + b, (const SlicePart*)p, n, (const SliceToken*)lists, cap, x, temps + b, top_ps + b, top_ks + b,
                        seeds + b, steps + b, m, V, dbg ? dbg + (int64_t)b * 16 : nullptr);
   }
 }

@@ -190,3 +190,26 @@ def test_short_rows_without_an_allowed_token():
                                  torch.full((3,), k, dtype=torch.int32, device=DEV), torch.arange(3, device=DEV),
                                  torch.zeros(3, dtype=torch.long, device=DEV), mask)
             assert toks.tolist() == [0, 0, 0]
+
+
+@pytest.mark.parametrize("B,V", [(1, 131072), (40, 32769), (256, 131072), (257, 131072)])
+@pytest.mark.parametrize("near", [40, 47, 48, 49, 300])
+def test_cut_inside_and_behind_the_slices_lists(B, V, near):
+    """``near`` tokens close to the max in one stretch of the row, and a flat rest 9, 16 or 30 of scaled logit below: a
+    slice lists all of them, or fewer than are asked for, or the cut lies in the rest."""
+    g = torch.Generator().manual_seed(near + V)
+    gap = torch.tensor([9.0, 16.0, 30.0])[torch.arange(B) % 3].unsqueeze(1)
+    logits = torch.rand(B, V, generator=g) - gap
+    logits[:, 100:100 + near] = torch.rand(B, near, generator=g) * 2.0
+    top_k = torch.full((B,), 45, dtype=torch.int32)
+    top_k[1::2] = 301
+    seeds, steps = torch.randint(0, 2**40, (B,), generator=g), torch.randint(0, 99, (B,), generator=g)
+    one = torch.ones(B, device=DEV)
+    toks, _ = ops.sample(logits.to(DEV), one, one, top_k.to(DEV), seeds.to(DEV), steps.to(DEV), None)
+    for b in range(0, B, 1 if B < 100 else 41):
+        x = logits[b].double().numpy()
+        kept = np.argsort(-x, kind="stable")[:int(top_k[b])]
+        key = x + gumbel(int(seeds[b]), int(steps[b]), V)
+        t = int(toks[b])
+        # ties of fp32 logits at the cut may go either way; fast logarithms are off by 4e-7 of the draw's range
+        assert x[t] >= x[kept[-1]] and key[t] >= key[kept].max() - max(1e-3, 4e-7 * V)
