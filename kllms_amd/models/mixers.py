@@ -263,9 +263,22 @@ class ParallelMixer(nn.Module):
         self.right = DecayLinearAttention(ri, hidden, eps, dtype)
         self.left_out = _param(hidden, dtype=torch.float32)
         self.right_out = _param(hidden, dtype=torch.float32)
+        # sizes of the step of few rows (rows_step)
+        self.rows_ok = (le.dim == 128 and le.vdim == 128 and le.values_from_keys and le.head_gate and le.mask_size >= 0
+                        and le.heads // le.kv_heads in (1, 2, 4, 8) and self.inp.weight.shape[0] % 16 == 0
+                        and ri.dim <= 256 and ri.heads * ri.vdim % 128 == 0 and hidden % 128 == 0 and hidden <= 8192)
 
     def cache_spec(self) -> LayerCacheSpec:
         return LayerCacheSpec(kv=self.left.cache_spec(), rec=self.right.cache_spec())
+
+    def rows_step(self, x, h, batch, st: LayerState, w_post, w_next) -> torch.Tensor:
+        """The sublayer with its residual for single decoded rows: ops.hybrid_parallel_rows."""
+        le, p = self.left.spec, self.inp.parts
+        at = [p[n][0] for n in ("left.q", "left.k", "left.g", "right.q", "right.k", "right.v", "right.g")]
+        return ops.hybrid_parallel_rows(x, h, self.inp.weight, self.inp.bias, at, self.left.inv_freq, st.k, st.v,
+                                        self.left.o_proj, self.right.decay, st.rec, self.right.norm, self.right.o_proj,
+                                        self.left_out, self.right_out, w_post, w_next, batch, le.heads, le.scale,
+                                        le.mask_size, self.right.eps)
 
     def forward(self, h: torch.Tensor, batch, st: LayerState):
         y = self.inp(h)
@@ -318,10 +331,20 @@ class ChannelDeltaMixer(nn.Module):
         self.A_log = _param(spec.heads, dtype=torch.float32)
         self.norm = _param(spec.vdim, dtype=torch.float32)
         self.o_proj = _param(hidden, self.hv, dtype=dtype)
+        # sizes of the step of few rows (rows_step)
+        self.rows_ok = (self.inp.weight.shape[0] % 16 == 0 and self.hv % 128 == 0 and spec.dim <= 256 and spec.conv <= 16
+                        and hidden % 128 == 0 and hidden <= 8192)
 
     def cache_spec(self) -> LayerCacheSpec:
         sp = self.spec
         return LayerCacheSpec(rec=(sp.heads, sp.dim, sp.vdim), conv=(self.cp, sp.conv - 1))
+
+    def rows_step(self, x, h, batch, st: LayerState, w_post, w_next) -> torch.Tensor:
+        """The sublayer with its residual for single decoded rows: ops.hybrid_delta_rows."""
+        at = [self.inp.parts[n][0] for n in ("q", "k", "v", "a1", "g1", "b")]
+        return ops.hybrid_delta_rows(x, h, self.inp.weight, at, self.conv, st.conv, self.a2, self.g2, self.dt_bias,
+                                     self.A_log, st.rec, self.norm, self.o_proj, w_post, w_next, batch,
+                                     self.spec.kv_heads, self.eps)
 
     def forward(self, h: torch.Tensor, batch, st: LayerState) -> torch.Tensor:
         sp = self.spec
@@ -362,6 +385,12 @@ class ClampedGLU(nn.Module):
         self.inp = FusedInput(hidden, [("gate", spec.ff), ("up", spec.ff)], dtype)
         self.down = _param(hidden, spec.ff, dtype=dtype)
         self._fused = self.inp.weight.shape[0] == 2 * spec.ff      # up's rows follow gate's without a gap
+        # sizes of the step of few rows (rows_step)
+        self.rows_ok = self._fused and spec.ff % 128 == 0 and hidden % 128 == 0 and hidden <= 8192
+
+    def rows_step(self, x, h, w_post, w_next, eps: float) -> torch.Tensor:
+        """The sublayer with its residual for single decoded rows: ops.hybrid_glu_rows."""
+        return ops.hybrid_glu_rows(x, h, self.inp.weight, self.down, w_post, w_next, self.spec.limit, self.spec.alpha, eps)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         act = ops.linear_clamped_glu(h, self.inp.weight, self.spec.limit, self.spec.alpha) if self._fused else None

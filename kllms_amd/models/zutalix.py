@@ -29,7 +29,7 @@ from ..engine.kvcache import LayerCacheSpec, LayerState
 from ..parallel.tp import ParallelContext
 from .listed import ListedLayerLM
 from .llama import ForwardBatch
-from .mixers import ChannelDeltaMixer, ClampedGLU, ParallelMixer, _param
+from .mixers import ChannelDeltaMixer, ClampedGLU, ParallelMixer, _param, single_rows
 
 
 class HybridLayer(nn.Module):
@@ -50,18 +50,23 @@ class HybridLayer(nn.Module):
             self.mlp = ClampedGLU(spec.mlp, hidden, dtype)
 
     def forward(self, x: torch.Tensor, h: torch.Tensor, batch: ForwardBatch, st: LayerState,
-                next_norm: torch.Tensor) -> torch.Tensor:
+                next_norm: torch.Tensor, rows: bool = False) -> torch.Tensor:
         """x: fp32 residual (updated in place); h = norm1(x) in the model
-        dtype. Returns the next layer's normed input."""
+        dtype. Returns the next layer's normed input. rows: a step of single
+        decoded rows that hybrid_rows_ok admits."""
         after_mix = self.norm2 if self.mlp is not None else next_norm
-        if self.kind == "parallel":
+        if rows and self.mix.rows_ok:
+            h = self.mix.rows_step(x, h, batch, st, self.norm1b, after_mix)
+        elif self.kind == "parallel":
             left, right = self.mix(h, batch, st)
             h = ops.sandwich_residual(x, left, self.norm1b, self.eps, b=right, wa=self.mix.left_out,
                                       wb=self.mix.right_out, w_next=after_mix, out_dtype=h.dtype)
         else:
             y = self.mix(h, batch, st)
             h = ops.sandwich_residual(x, y, self.norm1b, self.eps, w_next=after_mix, out_dtype=h.dtype)
-        if self.mlp is not None:
+        if self.mlp is not None and rows and self.mlp.rows_ok:
+            h = self.mlp.rows_step(x, h, self.norm2b, next_norm, self.eps)
+        elif self.mlp is not None:
             y = self.mlp(h)
             h = ops.sandwich_residual(x, y, self.norm2b, self.eps, w_next=next_norm, out_dtype=h.dtype)
         return h
@@ -145,9 +150,10 @@ class ZutalixForCausalLM(ListedLayerLM):
         x = ops.embed_rmsnorm(input_ids, self.embed_tokens.weight, self.embed_norm, self.eps)
         h = ops.rmsnorm_cast(x, self.layers[0].norm1, self.eps, self.dtype)
         n = len(self.layers)
+        rows = single_rows(batch) and ops.hybrid_rows_ok(x, h, batch)
         for i, layer in enumerate(self.layers):
             nxt = self.layers[i + 1].norm1 if i + 1 < n else self.final_norm
-            h = layer(x, h, batch, batch.kv_caches[i], nxt)
+            h = layer(x, h, batch, batch.kv_caches[i], nxt, rows)
             if self.trace_layers is not None:
                 self.trace_layers.append(x.clone())
         return h

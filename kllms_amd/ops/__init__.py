@@ -625,6 +625,47 @@ def silu_glu(gate, up):
     return gated_act(gate, up, float("inf"), 1.0, 0.0)
 
 
+# --- a hybrid model's step of single decoded rows ----------------------------------
+# GPU-only (ops/hip/seq/seq_steps.hip): callers ask hybrid_rows_ok first.
+
+def hybrid_rows_ok(x, h, batch) -> bool:
+    """Whether a step's sublayers can run as hybrid_*_rows: up to 128 rows, each its own sequence, bf16 on the GPU."""
+    T = h.shape[0]
+    return (_gpu(h) and h.dtype == torch.bfloat16 and x.dtype == torch.float32 and 1 <= T <= LINEAR_ROWS_MAX
+            and batch.context_lens is not None and batch.block_tables is not None and batch.token_seg is not None
+            and batch.block_tables.shape[0] == T and batch.block_tables.is_contiguous()
+            and batch.positions.dtype == torch.long
+            and all(t is not None and t.is_contiguous() and t.numel() == n and t.dtype == torch.int32 for t, n in (
+                (batch.context_lens, T), (batch.state_slots, T), (batch.seg_start, T), (batch.token_seg, T),
+                (batch.cu_seqlens, T + 1), (batch.block_tables, batch.block_tables.numel())))
+            and all(t.is_contiguous() and t.numel() == T and t.dtype == torch.long
+                    for t in (batch.positions, batch.slot_mapping))
+            and not (torch.is_grad_enabled() and (x.requires_grad or h.requires_grad)) and _plain_call(x, h))
+
+
+def hybrid_parallel_rows(x, h, w_in, bias, at, inv_freq, k_cache, v_cache, o_left, decay, state, norm_right, o_right, wa,
+                         wb, w_post, w_next, batch, heads, scale, mask_size, eps):
+    """x (fp32 stream) += the parallel sublayer of h in place, with cache and state; returns the next normed input. at:
+    columns of left q, k, head gates and right q, k, v, gate in h @ w_in^T + bias."""
+    return _seq().hybrid_parallel_rows(
+        x, h, w_in, bias if bias is not None else _none(h), at, inv_freq, k_cache, v_cache, o_left, decay, state,
+        norm_right, o_right, wa, wb, w_post, w_next, batch.positions, batch.slot_mapping, batch.block_tables,
+        batch.context_lens, batch.state_slots, batch.cu_seqlens, batch.seg_start, heads, scale, mask_size, eps)
+
+
+def hybrid_delta_rows(x, h, w_in, at, conv, conv_state, a2, g2, dt_bias, a_log, state, norm, w_out, w_post, w_next, batch,
+                      kv_heads, eps):
+    """The same of a gated-delta-rule sublayer; at: columns of q, k, v, the low-rank inputs and the write strengths."""
+    return _seq().hybrid_delta_rows(x, h, w_in, at, conv, conv_state, a2, g2, dt_bias, a_log, state, norm, w_out, w_post,
+                                    w_next, batch.state_slots, batch.cu_seqlens, batch.seg_start, batch.token_seg,
+                                    kv_heads, eps)
+
+
+def hybrid_glu_rows(x, h, w_in, w_down, w_post, w_next, limit, alpha, eps):
+    """The same of a clamped gated-linear-unit sublayer."""
+    return _seq().hybrid_glu_rows(x, h, w_in, w_down, w_post, w_next, limit, alpha, eps)
+
+
 def embed_bigram(ids, table, bigram, scale, mul_prev, mul_cur, buckets, tok_state, state_slots, cu_seqlens,
                  seg_start, token_seg, out=None):
     """fp32 rows table[id] * scale (+ the hashed bigram row); ``out``: an

@@ -423,7 +423,7 @@ torch::Tensor moe_combine(torch::Tensor y, torch::Tensor weights, torch::Tensor 
 
 // --- products of a few rows (linear_rows.hip) ---------------------------------
 extern "C" void launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
-                                   int K, int x_stride, int form, int splits, hipStream_t stream);
+                                   int K, int x_stride, int form, int splits, float limit, float alpha, hipStream_t stream);
 extern "C" int linear_rows_splits(int M, int N, int K);
 
 // form 0: fp32 sums [S, M, N]; 1: bf16 [M, N] (+ bias); 2: fp32 [M, N]; 3: silu(gate) * up of a fused
@@ -446,7 +446,7 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, torch::Tensor bias, 
            : form == 2 ? torch::empty({M, N}, x.options().dtype(torch::kFloat))
                        : torch::empty({M, form == 3 ? N / 2 : N}, x.options());
   launch_linear_rows(out.data_ptr(), cbf(x), cbf(w), bias.numel() ? cbf(bias) : nullptr, M, N, K,
-                     (int)x.stride(0), (int)form, S, cur_stream());
+                     (int)x.stride(0), (int)form, S, 0.0f, 0.0f, cur_stream());
   return out;
 }
 

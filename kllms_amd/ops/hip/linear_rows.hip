@@ -12,8 +12,8 @@
 // A matrix of few rows is also split over k (linear_rows_splits); the splits' fp32 sums are left to the consumer, which reads them anyway (rope + store,
 // residual + norm). Forms of the result:
 //   PART  fp32 sums [S, M, N]          SILU  silu(gate) * up of a fused [gate; up] matrix
-//   F32   fp32, S = 1 (logits)         BF16  rounded once, bias added before it: for callers of the
-//                                            binding, the models' products take the other three
+//   F32   fp32, S = 1 (logits)         CLAMPED  the clamped gated form of the hybrid family
+//   BF16  rounded once, bias added before it
 //
 // Measured with the weights out of cache (the library's kernel in brackets), us:
 //   4096 x 4096   5 rows 9 (15.6), 128 rows 15.6 (24.5)
@@ -31,7 +31,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 #define LR_KC 128          // k depth of a chunk
 #define LR_STEPS 4         // matrix steps (32 k) of a chunk
 
-enum LinearForm { LR_PART = 0, LR_BF16 = 1, LR_F32 = 2, LR_SILU = 3 };
+enum LinearForm { LR_PART = 0, LR_BF16 = 1, LR_F32 = 2, LR_SILU = 3, LR_CLAMPED = 4 };
 
 union LrFrag {
   u32x4 u;
@@ -41,7 +41,7 @@ union LrFrag {
 template <int MT, int FORM, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
     void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-    const bf16_t* __restrict__ bias, int M, int N, int K, int x_stride, int chunks_per_split) {
+    const bf16_t* __restrict__ bias, int M, int N, int K, int x_stride, int chunks_per_split, float limit, float alpha) {
   __shared__ __attribute__((aligned(16))) u32x4 xs[2][MT * 256];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -49,10 +49,11 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
   const int nchunks = K / LR_KC;
   const int c_begin = blockIdx.y * chunks_per_split;
   const int c_end = min(nchunks, c_begin + chunks_per_split);
-  // weight row of this wave's tile; SILU: the first half of the waves hold gate rows, the others the up rows of
+  // weight row of this wave's tile; gated: the first half of the waves hold gate rows, the others the up rows of
   // the same columns
   constexpr int HW = WAVES / 2;
-  const int n0 = FORM == LR_SILU ? (wave / HW) * (N / 2) + blockIdx.x * (16 * HW) + (wave % HW) * 16
+  constexpr bool GATED = FORM == LR_SILU || FORM == LR_CLAMPED;
+  const int n0 = GATED ? (wave / HW) * (N / 2) + blockIdx.x * (16 * HW) + (wave % HW) * 16
                                  : blockIdx.x * (16 * WAVES) + wave * 16;
   const char* wrow = (const char*)(w + (int64_t)min(n0 + col, N - 1) * K) + grp * 32;
 
@@ -120,7 +121,7 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
 
   // lane (col, grp): rows n0 + grp*4 .. +3 of the weights, row i*16 + col of x
   const int n = n0 + grp * 4;
-  if constexpr (FORM == LR_SILU) {
+  if constexpr (GATED) {
     float* up = reinterpret_cast<float*>(&xs[0][0]);   // [HW waves][MT*16 rows][16]
     static_assert(HW * MT * 16 * 16 * 4 <= sizeof(xs), "the up halves fit the staging buffers");
     if (wave >= HW) {
@@ -137,9 +138,14 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
         bf16x4_vec o;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          // rounded as the separate product's result is
-          const float g = bf16_to_f32(f32_to_bf16(acc[i][r])), v = bf16_to_f32(f32_to_bf16(u[r]));
-          o[r] = f32_to_bf16(g / (1.0f + __expf(-g)) * v);
+          if constexpr (FORM == LR_SILU) {
+            // rounded as the separate product's result is
+            const float g = bf16_to_f32(f32_to_bf16(acc[i][r])), v = bf16_to_f32(f32_to_bf16(u[r]));
+            o[r] = f32_to_bf16(g / (1.0f + __expf(-g)) * v);
+          } else {
+            const float g = fminf(acc[i][r], limit), v = fminf(fmaxf(u[r], -limit), limit);
+            o[r] = f32_to_bf16(g * (1.0f / (1.0f + expf(-alpha * g))) * (v + 1.0f));
+          }
         }
         if (m < M) *reinterpret_cast<bf16x4_vec*>((short*)out + (int64_t)m * (N / 2) + n) = o;
       }
@@ -183,18 +189,20 @@ static int linear_rows_waves(int M, int N, int form) {
 }
 
 extern "C" void launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
-                                   int K, int x_stride, int form, int splits, hipStream_t stream) {
+                                   int K, int x_stride, int form, int splits, float limit, float alpha,
+                                   hipStream_t stream) {
   const int per = (K / LR_KC + splits - 1) / splits;
   const int waves = linear_rows_waves(M, N, form);
   const dim3 grid((N + 16 * waves - 1) / (16 * waves), splits);
 #define LR_GO(MT, F, WV)                                                                                          \
   hipLaunchKernelGGL((linear_rows_kernel<MT, F, WV>), grid, dim3(64 * WV), 0, stream, out, x, w, bias, M, N, K, \
-                     x_stride, per)
+                     x_stride, per, limit, alpha)
 #define LR_FORM(MT, WV)                          \
   switch (form) {                                \
     case LR_PART: LR_GO(MT, LR_PART, WV); break; \
     case LR_BF16: LR_GO(MT, LR_BF16, WV); break; \
     case LR_F32: LR_GO(MT, LR_F32, WV); break;   \
+    case LR_CLAMPED: LR_GO(MT, LR_CLAMPED, WV); break; \
     default: LR_GO(MT, LR_SILU, WV); break;      \
   }
   if (M <= 16) { LR_FORM(1, 4); }

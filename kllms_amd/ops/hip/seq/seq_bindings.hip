@@ -1185,7 +1185,23 @@ void attn_diff_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache, 
   TORCH_CHECK(err == 0, "attn_diff_paged launch: ", hipGetErrorString((hipError_t)err));
 }
 
+// seq_steps.hip
+torch::Tensor hybrid_parallel_rows(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, std::vector<int64_t>,
+                                   torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
+                                   torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
+                                   torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
+                                   torch::Tensor, int64_t, double, int64_t, double);
+torch::Tensor hybrid_delta_rows(torch::Tensor, torch::Tensor, torch::Tensor, std::vector<int64_t>, torch::Tensor,
+                                torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
+                                torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
+                                torch::Tensor, torch::Tensor, int64_t, double);
+torch::Tensor hybrid_glu_rows(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
+                              double, double, double);
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("hybrid_parallel_rows", &hybrid_parallel_rows);
+  m.def("hybrid_delta_rows", &hybrid_delta_rows);
+  m.def("hybrid_glu_rows", &hybrid_glu_rows);
   m.def("embed_rmsnorm", &embed_rmsnorm);
   m.def("rmsnorm_cast", &rmsnorm_cast);
   m.def("sandwich_residual", &sandwich_residual);

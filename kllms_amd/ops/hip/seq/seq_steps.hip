@@ -1,0 +1,249 @@
+// Whole sublayers of a hybrid model's decode step (one row a sequence, up to 128 of them), launched from here one
+// kernel behind the other. A step is some 85 launches of 5 to 17 us, and from Python a launch costs the host 12 to 15 us:
+// it was the bound (40 rows of the 2048-wide preset: 1310 us, the kernels 775). Here it is 2 to 3.
+
+#include <torch/extension.h>
+#include <ATen/hip/HIPContext.h>
+#include <hip/hip_bf16.h>
+
+#include <algorithm>
+
+extern "C" {
+void seq_launch_sandwich_rows(float*, const float*, int, const float*, int, const float*, const float*, const float*,
+                              const float*, void*, int, int, float, hipStream_t);
+void seq_launch_gated_rmsnorm(void*, const float*, const float*, const void*, int, int, int, int, float, int,
+                              int, hipStream_t);
+void seq_launch_rope_pairs_store(void*, const void*, const void*, const int64_t*, const float*, void*, void*,
+                                 const int64_t*, void*, int, int, int, int, int, int, int, int, int, int, int,
+                                 hipStream_t);
+void seq_launch_linear_attn_decay(float*, const void*, const void*, const void*, const float*, float*, float*,
+                                  const int*, const int*, const int*, int, int, int, int, int, int, int, int,
+                                  int, hipStream_t);
+void seq_launch_causal_conv_silu(void*, const void*, const float*, void*, const int*, const int*, const int*,
+                                 const int*, const float*, int, int, int, int, int, int, hipStream_t);
+void seq_launch_gated_delta_rule(float*, const void*, const void*, const void*, const void*, const void*,
+                                 const float*, const float*, float*, float*, float*, float*, float*, float*,
+                                 const int*, const int*, const int*, int, int, int, int, int, int, int, int, int,
+                                 int, int, int, hipStream_t);
+// few-row products and paged decode attention (ops/hip/linear_rows.hip, attn_decode.hip, also part of kllms_amd._C)
+void launch_linear_rows(void*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
+                        int, int, float, float, hipStream_t);
+int linear_rows_splits(int, int, int);
+int attn_decode_splits(int, int, int);
+void launch_attn_decode(__hip_bfloat16*, float*, const __hip_bfloat16*, const void*, const void*, const float*,
+                        const float*, const int*, const int*, const __hip_bfloat16*, int, float, int, int, int, int, int,
+                        int, int, int, int, hipStream_t);
+}
+
+using torch::Tensor;
+
+namespace {
+
+enum { ROWS_PART = 0, ROWS_BF16 = 1, ROWS_CLAMPED = 4 };   // forms of linear_rows
+
+inline hipStream_t cur_stream() { return at::hip::getCurrentHIPStream().stream(); }
+
+inline void check(const Tensor& t, at::ScalarType type, int64_t numel, const char* name) {
+  TORCH_CHECK(t.is_cuda() && t.scalar_type() == type && t.is_contiguous() && t.numel() == numel, name,
+              ": a contiguous GPU tensor of ", numel, " ", toString(type), " values");
+}
+inline void on_16(const Tensor& t, const char* name) {
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, name, " must begin on 16 bytes");
+}
+inline const __hip_bfloat16* bf(const Tensor& t) { return (const __hip_bfloat16*)t.data_ptr(); }
+inline const __hip_bfloat16* bf(const Tensor& t, int64_t col) { return bf(t) + col; }
+
+void check_weight(const Tensor& w, int64_t K, const char* name) {
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == K && K % 128 == 0 && w.size(0) % 16 == 0, name, ": [N, K], N % 16, K % 128");
+  check(w, at::kBFloat16, w.numel(), name);
+  on_16(w, name);
+}
+
+// x [T, K] (contiguous) by w: fp32 sums [S, T, N]
+Tensor part(const Tensor& x, const Tensor& w, int T, hipStream_t st) {
+  const int K = w.size(1), N = w.size(0), S = linear_rows_splits(T, N, K);
+  auto out = torch::empty({S, T, N}, x.options().dtype(torch::kFloat));
+  launch_linear_rows(out.data_ptr(), bf(x), bf(w), nullptr, T, N, K, K, ROWS_PART, S, 0.0f, 0.0f, st);
+  return out;
+}
+
+Tensor rows_bf16(const Tensor& x, const Tensor& w, const Tensor& bias, int T, hipStream_t st) {
+  const int K = w.size(1), N = w.size(0);
+  auto out = torch::empty({T, N}, x.options());
+  launch_linear_rows(out.data_ptr(), bf(x), bf(w), bias.numel() ? bf(bias) : nullptr, T, N, K, K, ROWS_BF16, 1, 0.0f, 0.0f,
+                     st);
+  return out;
+}
+
+struct Rows {
+  int T, W;
+  Rows(const Tensor& x, const Tensor& h) : T(h.size(0)), W(h.size(1)) {
+    TORCH_CHECK(h.dim() == 2 && T >= 1 && T <= 128 && W % 128 == 0 && W <= 8192, "1 to 128 rows of a width % 128, <= 8192");
+    check(h, at::kBFloat16, (int64_t)T * W, "h");
+    check(x, at::kFloat, (int64_t)T * W, "x");
+    on_16(h, "h");
+    on_16(x, "x");
+  }
+  void norm(const Tensor& w, const char* name) const {
+    check(w, at::kFloat, W, name);
+    on_16(w, name);
+  }
+};
+
+}  // namespace
+
+// x (fp32 stream, in place) through a parallel sublayer; h = its normed input. y columns: o_lq, o_lk of the softmax
+// branch's q and k, o_lg of its head gates; o_rq, o_rk, o_rv, o_rg of the recurrent branch. Returns the next normed input
+Tensor hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tensor bias, std::vector<int64_t> at, Tensor inv_freq,
+                            Tensor k_cache, Tensor v_cache, Tensor o_left, Tensor decay, Tensor state, Tensor norm_right,
+                            Tensor o_right, Tensor wa, Tensor wb, Tensor w_post, Tensor w_next, Tensor positions,
+                            Tensor slots, Tensor tables, Tensor lens, Tensor state_slots, Tensor cu, Tensor seg_start,
+                            int64_t heads, double scale, int64_t mask_size, double eps) {
+  const Rows r(x, h);
+  const int T = r.T, W = r.W;
+  check_weight(w_in, W, "w_in");
+  const int N = w_in.size(0);
+  if (bias.numel()) check(bias, at::kBFloat16, N, "bias");
+  TORCH_CHECK(k_cache.dim() == 4 && v_cache.sizes() == k_cache.sizes() && k_cache.size(3) == 128, "caches [NB, G, BS, 128]");
+  check(k_cache, at::kBFloat16, k_cache.numel(), "k_cache");
+  check(v_cache, at::kBFloat16, k_cache.numel(), "v_cache");
+  const int H = heads, G = k_cache.size(1), BS = k_cache.size(2), D = 128;
+  TORCH_CHECK(H % G == 0 && (H / G == 1 || H / G == 2 || H / G == 4 || H / G == 8), "heads to a kv head: 1, 2, 4 or 8");
+  TORCH_CHECK((int64_t)k_cache.size(0) * G * BS < (1LL << 31) && mask_size >= 0);
+  TORCH_CHECK(state.dim() == 4, "state [slots, H, D, V]");
+  const int RH = state.size(1), RD = state.size(2), RV = state.size(3);
+  check(state, at::kFloat, state.numel(), "state");
+  check(decay, at::kFloat, RH, "decay");
+  check(norm_right, at::kFloat, (int64_t)RH * RV, "norm_right");
+  TORCH_CHECK(RD <= 256, "key size above 256 is not supported by the recurrence kernel");
+  check_weight(o_left, (int64_t)H * D, "o_left");
+  check_weight(o_right, (int64_t)RH * RV, "o_right");
+  TORCH_CHECK(o_left.size(0) == W && o_right.size(0) == W);
+  const int64_t sizes[7] = {(int64_t)H * D, (int64_t)G * D, H, (int64_t)RH * RD, (int64_t)RH * RD, (int64_t)RH * RV,
+                            (int64_t)RH * RV};
+  TORCH_CHECK(at.size() == 7, "seven column ranges");
+  for (int i = 0; i < 7; ++i) TORCH_CHECK(at[i] >= 0 && at[i] % 8 == 0 && at[i] + sizes[i] <= N, "columns of w_in");
+  r.norm(wa, "wa"); r.norm(wb, "wb"); r.norm(w_post, "w_post"); r.norm(w_next, "w_next");
+  const int R = inv_freq.numel();
+  check(inv_freq, at::kFloat, R, "inv_freq");
+  TORCH_CHECK(2 * R <= D, "rotary width exceeds the head size");
+  check(positions, at::kLong, T, "positions");
+  check(slots, at::kLong, T, "slots");
+  check(lens, at::kInt, T, "lens");
+  check(state_slots, at::kInt, T, "state_slots");
+  check(cu, at::kInt, T + 1, "cu");
+  check(seg_start, at::kInt, T, "seg_start");
+  TORCH_CHECK(tables.dim() == 2 && tables.size(0) == T, "one table row for each row");
+  check(tables, at::kInt, tables.numel(), "tables");
+  const int width = tables.size(1);
+
+  auto st = cur_stream();
+  const auto f32 = x.options();
+  const Tensor y = rows_bf16(h, w_in, bias, T, st);
+  seq_launch_rope_pairs_store((void*)bf(y, at[0]), bf(y, at[1]), nullptr, positions.data_ptr<int64_t>(),
+                              inv_freq.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
+                              slots.data_ptr<int64_t>(), nullptr, T, H, G, D, D, R, BS, N, N, 0, 0, st);
+  auto att = torch::empty({T, (int64_t)H * D}, h.options());
+  const int64_t longest = mask_size > 0 ? std::min<int64_t>(mask_size, (int64_t)width * BS) : (int64_t)width * BS;
+  const int splits = attn_decode_splits(T, G, (int)std::min<int64_t>(longest, INT32_MAX));
+  auto partials = torch::empty({splits > 1 ? (int64_t)T * H * splits * 130 : 0}, f32);
+  launch_attn_decode((__hip_bfloat16*)att.data_ptr(), partials.data_ptr<float>(), bf(y, at[0]), k_cache.data_ptr(),
+                     v_cache.data_ptr(), nullptr, nullptr, tables.data_ptr<int>(), lens.data_ptr<int>(), bf(y, at[2]), N,
+                     (float)scale, H, G, BS, width, splits, N, T, 0, (int)mask_size, st);
+  auto o = torch::empty({T, (int64_t)RH * RV}, f32), packed = torch::empty({T, (int64_t)RH * (2 * RD + RV)}, f32);
+  seq_launch_linear_attn_decay(o.data_ptr<float>(), bf(y, at[3]), bf(y, at[4]), bf(y, at[5]), decay.data_ptr<float>(),
+                               packed.data_ptr<float>(), state.data_ptr<float>(), state_slots.data_ptr<int>(),
+                               cu.data_ptr<int>(), seg_start.data_ptr<int>(), T, T, RH, RD, RV, N, N, N, 0, st);
+  auto yr = torch::empty({T, (int64_t)RH * RV}, h.options());
+  seq_launch_gated_rmsnorm(yr.data_ptr(), o.data_ptr<float>(), norm_right.data_ptr<float>(), bf(y, at[6]), T, 1, RH * RV, N,
+                           (float)eps, 0, 0, st);
+  const Tensor left = part(att, o_left, T, st), right = part(yr, o_right, T, st);
+  auto out = torch::empty_like(h);
+  seq_launch_sandwich_rows(x.data_ptr<float>(), left.data_ptr<float>(), left.size(0), right.data_ptr<float>(),
+                           right.size(0), wa.data_ptr<float>(), wb.data_ptr<float>(), w_post.data_ptr<float>(),
+                           w_next.data_ptr<float>(), out.data_ptr(), T, W, (float)eps, st);
+  return out;
+}
+
+// The same of a gated-delta-rule sublayer. at: columns of q, k, v, of the two low-rank inputs and of the write strengths
+Tensor hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::vector<int64_t> at, Tensor conv, Tensor conv_state, Tensor a2,
+                         Tensor g2, Tensor dt_bias, Tensor a_log, Tensor state, Tensor norm, Tensor w_out, Tensor w_post,
+                         Tensor w_next, Tensor state_slots, Tensor cu, Tensor seg_start, Tensor token_seg,
+                         int64_t kv_heads, double eps) {
+  const Rows r(x, h);
+  const int T = r.T, W = r.W;
+  check_weight(w_in, W, "w_in");
+  const int N = w_in.size(0);
+  TORCH_CHECK(state.dim() == 4, "state [slots, H, D, V]");
+  const int H = state.size(1), D = state.size(2), V = state.size(3), G = kv_heads;
+  check(state, at::kFloat, state.numel(), "state");
+  TORCH_CHECK(G >= 1 && H % G == 0 && D <= 256, "heads and key size of the recurrence");
+  TORCH_CHECK(a2.dim() == 2 && g2.dim() == 2 && a2.size(0) == (int64_t)H * D && g2.size(0) == (int64_t)H * V);
+  check(a2, at::kBFloat16, a2.numel(), "a2");
+  check(g2, at::kBFloat16, g2.numel(), "g2");
+  const int64_t sizes[6] = {(int64_t)G * D, (int64_t)G * D, (int64_t)H * V, a2.size(1), g2.size(1), H};
+  TORCH_CHECK(at.size() == 6, "six column ranges");
+  for (int i = 0; i < 6; ++i) TORCH_CHECK(at[i] >= 0 && at[i] % 8 == 0 && at[i] + sizes[i] <= N, "columns of w_in");
+  TORCH_CHECK(conv.dim() == 2 && conv_state.dim() == 3, "taps [K, C], history [slots, K - 1, C]");
+  const int K = conv.size(0), C = conv.size(1);
+  for (int i = 0; i < 3; ++i) TORCH_CHECK(at[i] + sizes[i] <= C && C <= N, "the convolution's columns");
+  check(conv, at::kFloat, (int64_t)K * C, "conv");
+  check(conv_state, at::kBFloat16, conv_state.numel(), "conv_state");
+  TORCH_CHECK(K >= 1 && K <= 16 && conv_state.size(1) == K - 1 && conv_state.size(2) == C);
+  check(dt_bias, at::kFloat, (int64_t)H * D, "dt_bias");
+  check(a_log, at::kFloat, H, "a_log");
+  check(norm, at::kFloat, V, "norm");
+  check_weight(w_out, (int64_t)H * V, "w_out");
+  TORCH_CHECK(w_out.size(0) == W);
+  r.norm(w_post, "w_post"); r.norm(w_next, "w_next");
+  check(state_slots, at::kInt, T, "state_slots");
+  check(cu, at::kInt, T + 1, "cu");
+  check(seg_start, at::kInt, T, "seg_start");
+  check(token_seg, at::kInt, T, "token_seg");
+
+  auto st = cur_stream();
+  const auto f32 = x.options();
+  const Tensor y = rows_bf16(h, w_in, Tensor(torch::empty({0}, h.options())), T, st);
+  auto c = torch::empty({T, C}, h.options());
+  seq_launch_causal_conv_silu(c.data_ptr(), y.data_ptr(), conv.data_ptr<float>(), conv_state.data_ptr(),
+                              state_slots.data_ptr<int>(), cu.data_ptr<int>(), seg_start.data_ptr<int>(),
+                              token_seg.data_ptr<int>(), nullptr, T, T, C, K, N, 0, st);
+  const Tensor a = at::linear(y.narrow(1, at[3], sizes[3]), a2), gate = at::linear(y.narrow(1, at[4], sizes[4]), g2);
+  auto o = torch::empty({T, (int64_t)H * V}, f32), qn = torch::empty({T, (int64_t)G * D}, f32),
+       kn = torch::empty({T, (int64_t)G * D}, f32), gd = torch::empty({T, (int64_t)H * D}, f32),
+       vf = torch::empty({T, (int64_t)H * V}, f32), bt = torch::empty({T, H}, f32);
+  seq_launch_gated_delta_rule(o.data_ptr<float>(), bf(c, at[0]), bf(c, at[1]), bf(c, at[2]), bf(y, at[5]), a.data_ptr(),
+                              dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), qn.data_ptr<float>(),
+                              kn.data_ptr<float>(), gd.data_ptr<float>(), vf.data_ptr<float>(), bt.data_ptr<float>(),
+                              state.data_ptr<float>(), state_slots.data_ptr<int>(), cu.data_ptr<int>(),
+                              seg_start.data_ptr<int>(), T, T, H, G, D, V, C, C, C, N, H * D, 0, st);
+  auto yr = torch::empty({T, (int64_t)H * V}, h.options());
+  seq_launch_gated_rmsnorm(yr.data_ptr(), o.data_ptr<float>(), norm.data_ptr<float>(), gate.data_ptr(), T, H, V, H * V,
+                           (float)eps, 0, 0, st);
+  const Tensor p = part(yr, w_out, T, st);
+  auto out = torch::empty_like(h);
+  seq_launch_sandwich_rows(x.data_ptr<float>(), p.data_ptr<float>(), p.size(0), nullptr, 0, nullptr, nullptr,
+                           w_post.data_ptr<float>(), w_next.data_ptr<float>(), out.data_ptr(), T, W, (float)eps, st);
+  return out;
+}
+
+// The same of a clamped gated-linear-unit sublayer, w_in = [gate; up]
+Tensor hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_down, Tensor w_post, Tensor w_next, double limit,
+                       double alpha, double eps) {
+  const Rows r(x, h);
+  check_weight(w_in, r.W, "w_in");
+  const int N = w_in.size(0);
+  TORCH_CHECK(N % 64 == 0, "gate and up in whole tiles");
+  check_weight(w_down, N / 2, "w_down");
+  TORCH_CHECK(w_down.size(0) == r.W);
+  r.norm(w_post, "w_post"); r.norm(w_next, "w_next");
+  auto st = cur_stream();
+  auto act = torch::empty({r.T, N / 2}, h.options());
+  launch_linear_rows(act.data_ptr(), bf(h), bf(w_in), nullptr, r.T, N, r.W, r.W, ROWS_CLAMPED, 1, (float)limit,
+                     (float)alpha, st);
+  const Tensor p = part(act, w_down, r.T, st);
+  auto out = torch::empty_like(h);
+  seq_launch_sandwich_rows(x.data_ptr<float>(), p.data_ptr<float>(), p.size(0), nullptr, 0, nullptr, nullptr,
+                           w_post.data_ptr<float>(), w_next.data_ptr<float>(), out.data_ptr(), r.T, r.W, (float)eps, st);
+  return out;
+}

@@ -34,11 +34,11 @@ HIP_FLAGS = ["-O3", "--offload-arch=gfx950", "-std=c++17", "-fPIC", "-fno-gpu-rd
 EXTENSIONS = {
     "_C_seq": {
         "dir": os.path.join(HIP_DIR, "seq"),
-        # the dense MFMA prefill kernel is shared with _C (one source, two modules)
+        # dense MFMA prefill, paged decode attention and few-row products are shared with _C (one source, two modules)
         "kernels": ["seq_norm.hip", "seq_attn.hip", "seq_recurrent.hip", "seq_parallel.hip", "seq_gated.hip",
                     "seq_latent.hip", "seq_stream.hip", "seq_retention.hip", "seq_diff.hip",
-                    "../attn_prefill.hip"],
-        "bindings": ["seq_bindings.hip"],
+                    "seq_rows.hip", "../attn_prefill.hip", "../attn_decode.hip", "../linear_rows.hip"],
+        "bindings": ["seq_bindings.hip", "seq_steps.hip"],
         "headers": ["seq_common.h"],
     },
 }
