@@ -7,7 +7,12 @@
 // is used whole, and x is read in the same order of k. x goes through LDS in 128-deep
 // chunks, double-buffered, shared by the waves; its 16-byte units are XORed with
 // the row, which keeps the 16-row fragment reads free of bank conflicts. The weights of
-// the next two chunks are in flight while one is multiplied (8 KB a wave).
+// the next DEEP chunks are in flight while one is multiplied (4 KB a wave each), and with AHEAD the chunk's x beside
+// them: loads come back in order, so that a wait for an x that was asked for last is one for all weights before it.
+// (DEEP 4 up to 32 rows, 2 above: there x takes 16 registers a chunk. DEEP 4 without AHEAD does nothing. Us with x asked
+// for one chunk before and so: 16384 x 2048 with silu 1 / 40 rows 19.2 / 22.6 and 18.2 / 19.6, 28672 x 4096 5 rows 52.2
+// and 48.5, 8720 x 2048 in one share 15.6 and 12.3, 4096 x 14336 40 rows 27.9 and 25.9, 2048 x 2048 3.9 and 3.8. Above
+// 64 rows the registers for it cost more workgroups than it gives: 28672 x 4096 120 rows 67 and 70.)
 //
 // A matrix of few rows is also split over k (linear_rows_splits); the splits' fp32 sums are left to the consumer, which reads them anyway (rope + store,
 // residual + norm). Forms of the result:
@@ -16,10 +21,10 @@
 //   BF16  rounded once, bias added before it
 //
 // Measured with the weights out of cache (the library's kernel in brackets), us:
-//   4096 x 4096   5 rows 9 (15.6), 128 rows 15.6 (24.5)
-//   4096 x 14336  5 rows 23.4 (26.7: 5 TB/s either way), 64 rows 30 (42), 128 rows 36 (75.5)
-//   2048 x 8192   1 row 9.2 (12.8), 64 rows 11.9 (22.6)
-//   28672 x 4096  with silu 50 (64 + 5) for 5 rows, 57 (54 + 5) for 64, 68 (57 + 5) for 128
+//   4096 x 4096   5 rows 8.3 (15.6), 128 rows 15.6 (24.5)
+//   4096 x 14336  5 rows 23.7 (26.7: 5 TB/s either way), 64 rows 28.7 (42), 128 rows 36 (75.5)
+//   2048 x 8192   1 row 8.6 (12.8), 64 rows 11.4 (22.6)
+//   28672 x 4096  with silu 48.5 (64 + 5) for 5 rows, 56 (54 + 5) for 64, 68 (57 + 5) for 128
 // Above 64 rows every wave reads all of x from LDS for 16 weight rows, and LDS is the
 // bound where K is not split far.
 
@@ -38,7 +43,7 @@ union LrFrag {
   bf16x8_mfma m;
 };
 
-template <int MT, int FORM, int WAVES>
+template <int MT, int FORM, int WAVES, int DEEP, bool AHEAD>
 __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
     void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
     const bf16_t* __restrict__ bias, int M, int N, int K, int x_stride, int chunks_per_split, float limit, float alpha) {
@@ -61,42 +66,43 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
 #pragma unroll
   for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  u32x4 wr[2][LR_STEPS];
+  u32x4 wr[DEEP][LR_STEPS];
   constexpr int XP = MT * 4 / WAVES;      // passes of a chunk's x over the threads
   static_assert(XP >= 1, "as many 16-byte units as threads");
-  u32x4 xr[XP];
+  constexpr int XD = AHEAD ? DEEP : 1;    // chunks of x in registers
+  u32x4 xr[XD][XP];
   auto load_w = [&](int c, int slot, int st) {
     wr[slot][st] = *reinterpret_cast<const u32x4*>(wrow + (int64_t)c * (LR_KC * 2) + (st >> 1) * 128 + (st & 1) * 16);
   };
   // row tid / 16 of each pass, 16-byte unit tid % 16
   const int xrow = tid >> 4, xunit = tid & 15;
-  auto load_x = [&](int c) {
+  auto load_x = [&](int c, int slot) {
 #pragma unroll
     for (int i = 0; i < XP; ++i)
-      xr[i] = *reinterpret_cast<const u32x4*>((const char*)(x + (int64_t)min(i * 4 * WAVES + xrow, M - 1) * x_stride) +
+      xr[slot][i] = *reinterpret_cast<const u32x4*>((const char*)(x + (int64_t)min(i * 4 * WAVES + xrow, M - 1) * x_stride) +
                                               (int64_t)c * (LR_KC * 2) + xunit * 16);
   };
-  auto store_x = [&](int buf) {
+  auto store_x = [&](int buf, int slot) {
 #pragma unroll
-    for (int i = 0; i < XP; ++i) xs[buf][(i * 4 * WAVES + xrow) * 16 + (xunit ^ (xrow & 15))] = xr[i];
+    for (int i = 0; i < XP; ++i) xs[buf][(i * 4 * WAVES + xrow) * 16 + (xunit ^ (xrow & 15))] = xr[slot][i];
   };
 
   if (c_begin < c_end) {
-    load_x(c_begin);
 #pragma unroll
-    for (int st = 0; st < LR_STEPS; ++st) load_w(c_begin, 0, st);
-    if (c_begin + 1 < c_end) {
+    for (int u = 0; u < DEEP; ++u)
+      if (c_begin + u < c_end) {
+        if (u < XD) load_x(c_begin + u, u);
 #pragma unroll
-      for (int st = 0; st < LR_STEPS; ++st) load_w(c_begin + 1, 1, st);
-    }
-    store_x(0);
+        for (int st = 0; st < LR_STEPS; ++st) load_w(c_begin + u, u, st);
+      }
+    store_x(0, 0);
     __syncthreads();
-    for (int c = c_begin; c < c_end; c += 2) {
+    for (int c = c_begin; c < c_end; c += DEEP) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < DEEP; ++u) {
         if (c + u < c_end) {
           const bool next = c + u + 1 < c_end;
-          if (next) load_x(c + u + 1);
+          if (!AHEAD && next) load_x(c + u + 1, 0);
 #pragma unroll
           for (int st = 0; st < LR_STEPS; ++st) {
             LrFrag a;
@@ -104,15 +110,16 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
               LrFrag b;
-              b.u = xs[u][i * 256 + col * 16 + (((st >> 1) * 8 + grp * 2 + (st & 1)) ^ col)];
+              b.u = xs[u & 1][i * 256 + col * 16 + (((st >> 1) * 8 + grp * 2 + (st & 1)) ^ col)];
               acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, b.m, acc[i], 0, 0, 0);
             }
           }
-          if (c + u + 2 < c_end) {
+          if (c + u + DEEP < c_end) {
+            if constexpr (AHEAD) load_x(c + u + DEEP, u);
 #pragma unroll
-            for (int st = 0; st < LR_STEPS; ++st) load_w(c + u + 2, u, st);
+            for (int st = 0; st < LR_STEPS; ++st) load_w(c + u + DEEP, u, st);
           }
-          if (next) store_x(1 - u);
+          if (next) store_x(1 - (u & 1), (u + 1) % XD);
           __syncthreads();
         }
       }
@@ -194,23 +201,23 @@ extern "C" void launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, 
   const int per = (K / LR_KC + splits - 1) / splits;
   const int waves = linear_rows_waves(M, N, form);
   const dim3 grid((N + 16 * waves - 1) / (16 * waves), splits);
-#define LR_GO(MT, F, WV)                                                                                          \
-  hipLaunchKernelGGL((linear_rows_kernel<MT, F, WV>), grid, dim3(64 * WV), 0, stream, out, x, w, bias, M, N, K, \
-                     x_stride, per, limit, alpha)
-#define LR_FORM(MT, WV)                          \
-  switch (form) {                                \
-    case LR_PART: LR_GO(MT, LR_PART, WV); break; \
-    case LR_BF16: LR_GO(MT, LR_BF16, WV); break; \
-    case LR_F32: LR_GO(MT, LR_F32, WV); break;   \
-    case LR_CLAMPED: LR_GO(MT, LR_CLAMPED, WV); break; \
-    default: LR_GO(MT, LR_SILU, WV); break;      \
+#define LR_GO(MT, F, WV, DEEP)                                                                                        \
+  hipLaunchKernelGGL((linear_rows_kernel<MT, F, WV, DEEP, (MT <= 4)>), grid, dim3(64 * WV), 0, stream, out, x, w, bias, M, \
+                     N, K, x_stride, per, limit, alpha)
+#define LR_FORM(MT, WV, DEEP)                                \
+  switch (form) {                                            \
+    case LR_PART: LR_GO(MT, LR_PART, WV, DEEP); break;       \
+    case LR_BF16: LR_GO(MT, LR_BF16, WV, DEEP); break;       \
+    case LR_F32: LR_GO(MT, LR_F32, WV, DEEP); break;         \
+    case LR_CLAMPED: LR_GO(MT, LR_CLAMPED, WV, DEEP); break; \
+    default: LR_GO(MT, LR_SILU, WV, DEEP); break;            \
   }
-  if (M <= 16) { LR_FORM(1, 4); }
-  else if (M <= 32) { LR_FORM(2, 4); }
-  else if (waves == 8 && M <= 64) { LR_FORM(4, 8); }
-  else if (waves == 8) { LR_FORM(8, 8); }
-  else if (M <= 64) { LR_FORM(4, 4); }
-  else { LR_FORM(8, 4); }
+  if (M <= 16) { LR_FORM(1, 4, 4); }
+  else if (M <= 32) { LR_FORM(2, 4, 4); }
+  else if (waves == 8 && M <= 64) { LR_FORM(4, 8, 2); }
+  else if (waves == 8) { LR_FORM(8, 8, 2); }
+  else if (M <= 64) { LR_FORM(4, 4, 2); }
+  else { LR_FORM(8, 4, 2); }
 #undef LR_FORM
 #undef LR_GO
 }
