@@ -92,7 +92,8 @@ void seq_launch_causal_conv_silu(void*, const void*, const float*, void*, const 
 void seq_launch_gated_delta_rule(float*, const void*, const void*, const void*, const void*, const void*,
                                  const float*, const float*, float*, float*, float*, float*, float*, float*,
                                  const int*, const int*, const int*, int, int, int, int, int, int, int, int, int,
-                                 int, int, int, hipStream_t);
+                                 int, int, int, float*, hipStream_t);
+int64_t seq_delta_chunk_room(int, int, int, int, int, int);
 void seq_launch_dyt_residual(void*, float*, const void*, const float*, const float*, const float*, const float*,
                              const float*, const float*, const int64_t*, const void*, float, int, int, int, hipStream_t);
 void seq_launch_rmsnorm_rows(void*, const void*, const float*, int, int, int, float, int, hipStream_t);
@@ -658,12 +659,15 @@ void gated_delta_rule(torch::Tensor o, torch::Tensor q, torch::Tensor k, torch::
   TORCH_CHECK(state.dim() == 4 && state.size(1) == H && state.size(2) == D && state.size(3) == V);
   TORCH_CHECK(dt_bias.numel() == (int64_t)H * D && a_log.numel() == H && o.numel() == (int64_t)T * H * V);
   if (T == 0 || B == 0) return;
-  // fp32 operands of the recurrence, from the parallel pre-pass: unit q and k,
-  // per-channel decays, values, write strengths
+  // by chunks: their records; else fp32 operands of the recurrence, from the parallel pre-pass: unit q and k, per-channel
+  // decays, values, write strengths
   auto f32 = torch::dtype(torch::kFloat).device(q.device());
-  auto qn = torch::empty({(int64_t)T, (int64_t)G * D}, f32), kn = torch::empty({(int64_t)T, (int64_t)G * D}, f32);
-  auto gd = torch::empty({(int64_t)T, (int64_t)H * D}, f32), vf = torch::empty({(int64_t)T, (int64_t)H * V}, f32);
-  auto bt = torch::empty({(int64_t)T, (int64_t)H}, f32);
+  const int64_t room = seq_delta_chunk_room(T, B, H, G, D, V), t = room ? 0 : T;
+  torch::Tensor rec;
+  if (room) rec = torch::empty({room}, f32);
+  auto qn = torch::empty({t, (int64_t)G * D}, f32), kn = torch::empty({t, (int64_t)G * D}, f32);
+  auto gd = torch::empty({t, (int64_t)H * D}, f32), vf = torch::empty({t, (int64_t)H * V}, f32);
+  auto bt = torch::empty({t, (int64_t)H}, f32);
   seq_launch_gated_delta_rule(o.data_ptr<float>(), q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(),
                               a.data_ptr(), dt_bias.data_ptr<float>(), a_log.data_ptr<float>(),
                               qn.data_ptr<float>(), kn.data_ptr<float>(), gd.data_ptr<float>(),
@@ -671,7 +675,7 @@ void gated_delta_rule(torch::Tensor o, torch::Tensor q, torch::Tensor k, torch::
                               slots.data_ptr<int>(),
                               cu.data_ptr<int>(), seg_start.data_ptr<int>(), T, B, H, G, D, V, (int)q.stride(0),
                               (int)k.stride(0), (int)v.stride(0), (int)beta.stride(0), (int)a.stride(0),
-                              f32flag(q), cur_stream());
+                              f32flag(q), room ? rec.data_ptr<float>() : nullptr, cur_stream());
 }
 
 // ---- parallel-layer family ------------------------------------------------------

@@ -626,13 +626,23 @@ extern "C" void seq_launch_causal_conv_silu(void* y, const void* x, const float*
                                 (T*)conv_state, slots, cu, seg_start, B, C, K, x_stride);)
 }
 
+extern "C" void seq_launch_delta_chunks(float*, const void*, const void*, const void*, const void*, const void*,
+                                        const float*, const float*, float*, float*, const int*, const int*, const int*,
+                                        int, int, int, int, int, int, int, int, int, int, int, hipStream_t);
+
+// rec: room for the form of seq_delta.hip (then qn to bt are not read or written), or nullptr: token by token
 extern "C" void seq_launch_gated_delta_rule(float* o, const void* q, const void* k, const void* v,
                                             const void* beta_logit, const void* a, const float* dt_bias,
                                             const float* a_log, float* qn, float* kn, float* gd, float* vf,
                                             float* bt, float* state, const int* slots, const int* cu,
                                             const int* seg_start, int T_, int B, int H, int G, int D, int V,
                                             int q_stride, int k_stride, int v_stride, int beta_stride,
-                                            int a_stride, int is_f32, hipStream_t st) {
+                                            int a_stride, int is_f32, float* rec, hipStream_t st) {
+  if (rec) {
+    seq_launch_delta_chunks(o, q, k, v, beta_logit, a, dt_bias, a_log, rec, state, slots, cu, seg_start, T_, B, H, G, V,
+                            q_stride, k_stride, v_stride, beta_stride, a_stride, is_f32, st);
+    return;
+  }
   DISPATCH_T(is_f32, hipLaunchKernelGGL(delta_prep_kernel<T>, dim3(T_, G + H), dim3(WAVE), 0, st, qn, kn, gd,
                                         vf, bt, (const T*)q, (const T*)k, (const T*)v, (const T*)beta_logit,
                                         (const T*)a, dt_bias, a_log, H, G, D, V, q_stride, k_stride, v_stride,

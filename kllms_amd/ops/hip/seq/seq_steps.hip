@@ -24,7 +24,7 @@ void seq_launch_causal_conv_silu(void*, const void*, const float*, void*, const 
 void seq_launch_gated_delta_rule(float*, const void*, const void*, const void*, const void*, const void*,
                                  const float*, const float*, float*, float*, float*, float*, float*, float*,
                                  const int*, const int*, const int*, int, int, int, int, int, int, int, int, int,
-                                 int, int, int, hipStream_t);
+                                 int, int, int, float*, hipStream_t);
 // few-row products and paged decode attention (ops/hip/linear_rows.hip, attn_decode.hip, also part of kllms_amd._C)
 void launch_linear_rows(void*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
                         int, int, float, float, hipStream_t);
@@ -216,7 +216,7 @@ Tensor hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::vector<int64_t> a
                               dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), qn.data_ptr<float>(),
                               kn.data_ptr<float>(), gd.data_ptr<float>(), vf.data_ptr<float>(), bt.data_ptr<float>(),
                               state.data_ptr<float>(), state_slots.data_ptr<int>(), cu.data_ptr<int>(),
-                              seg_start.data_ptr<int>(), T, T, H, G, D, V, C, C, C, N, H * D, 0, st);
+                              seg_start.data_ptr<int>(), T, T, H, G, D, V, C, C, C, N, H * D, 0, nullptr, st);
   auto yr = torch::empty({T, (int64_t)H * V}, h.options());
   seq_launch_gated_rmsnorm(yr.data_ptr(), o.data_ptr<float>(), norm.data_ptr<float>(), gate.data_ptr(), T, H, V, H * V,
                            (float)eps, 0, 0, st);

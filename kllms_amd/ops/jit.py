@@ -37,7 +37,7 @@ EXTENSIONS = {
         # dense MFMA prefill, paged decode attention and few-row products are shared with _C (one source, two modules)
         "kernels": ["seq_norm.hip", "seq_attn.hip", "seq_recurrent.hip", "seq_parallel.hip", "seq_gated.hip",
                     "seq_latent.hip", "seq_stream.hip", "seq_retention.hip", "seq_diff.hip",
-                    "seq_rows.hip", "../attn_prefill.hip", "../attn_decode.hip", "../linear_rows.hip"],
+                    "seq_rows.hip", "seq_delta.hip", "../attn_prefill.hip", "../attn_decode.hip", "../linear_rows.hip"],
         "bindings": ["seq_bindings.hip", "seq_steps.hip"],
         "headers": ["seq_common.h"],
     },

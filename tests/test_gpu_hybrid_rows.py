@@ -65,3 +65,42 @@ def test_residual_of_split_sums_against_float64():
     # an activation that rounds to bf16 the other way moves a row by 2^-8 of one of its 128 terms
     assert (x.double() - ref).abs().max() <= 2e-2
     assert ((got.double() - out).abs() <= 2 ** -8 * out.abs() + 2e-2).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,G,V", [(4, 2, 128), (3, 3, 16), (2, 1, 80)])
+@pytest.mark.parametrize("lens", [[64], [16, 17, 200, 31, 1, 300, 0, 33], [300, 64]])
+def test_delta_rule_by_chunks_against_float64(H, G, V, lens, dtype):
+    """Segments fresh and continued, with lengths around the chunk's 16, strong and weak decays."""
+    D, T, B = 64, sum(lens), len(lens)
+    g = torch.Generator().manual_seed(T + V)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    q, k, v, beta = rnd(T, G, D).to(dtype), rnd(T, G, D).to(dtype), rnd(T, H, V).to(dtype), rnd(T, H).to(dtype)
+    a, dt, a_log = (rnd(T, H * D) * 2).to(dtype), rnd(H * D), torch.linspace(-3, 2, H)
+    state = rnd(B + 2, H, D, V)
+    slots = torch.randperm(B + 2, generator=g)[:B].to(torch.int32)
+    start = torch.tensor([7 * (b % 2) for b in range(B)], dtype=torch.int32)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    dev = lambda t: t.to(DEV)  # noqa: E731
+    got_state = dev(state)
+    assert T >= 64 * B                       # else the token-by-token form
+    o = ops.gated_delta_rule(dev(q), dev(k), dev(v), dev(beta), dev(a), dev(dt), dev(a_log), got_state, dev(slots), dev(cu),
+                             dev(start))
+    unit = lambda t: t / torch.sqrt((t * t).sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+    qd, kd = (unit(t.double()).repeat_interleave(H // G, 1) for t in (q, k))
+    qd = qd * D ** -0.5
+    decay = torch.exp(-a_log.double().exp().view(1, H, 1)
+                      * torch.nn.functional.softplus(a.double() + dt.double()).view(T, H, D))
+    for b in range(B):
+        S = state[slots[b]].double() if start[b] else torch.zeros(H, D, V, dtype=torch.float64)
+        size = max(1.0, float(S.abs().max()))
+        for t in range(cu[b], cu[b + 1]):
+            S = S * decay[t].unsqueeze(-1)
+            u = torch.sigmoid(beta[t].double()).unsqueeze(-1) * (v[t].double() - (kd[t].unsqueeze(-2) @ S).squeeze(-2))
+            S = S + kd[t].unsqueeze(-1) * u.unsqueeze(-2)
+            # fp32 sums of 64 products of values of the state's size, carried on by a contraction
+            assert ((qd[t].unsqueeze(-2) @ S).squeeze(-2) - o[t].double().cpu()).abs().max() <= 64 * 2 ** -23 * 8 * size
+            size = max(size, float(v[t].double().abs().max()))
+        assert (S - got_state[slots[b]].double().cpu()).abs().max() <= 64 * 2 ** -23 * 8 * size
+    for s in set(range(B + 2)) - set(slots.tolist()):
+        assert torch.equal(got_state[s].cpu(), state[s])
