@@ -660,7 +660,7 @@ class LLMEngine:
         out = []
         for rows, kind in ((longs, np.int64), (ints, np.int32)):
             rows = [np.asarray(r, dtype=kind) for r in rows]
-            flat = torch.from_numpy(np.concatenate([r.reshape(-1) for r in rows])).to(self.device)
+            flat = ops.upload(torch.from_numpy(np.concatenate([r.reshape(-1) for r in rows])), self.device)
             parts = flat.split([r.size for r in rows])
             out.append([p if r.ndim == 1 else p.view(r.shape) for p, r in zip(parts, rows)])
         return out
