@@ -266,7 +266,7 @@ class ParallelMixer(nn.Module):
         # sizes of the step of few rows (rows_step)
         self.rows_ok = (le.dim == 128 and le.vdim == 128 and le.values_from_keys and le.head_gate and le.mask_size >= 0
                         and le.heads // le.kv_heads in (1, 2, 4, 8) and self.inp.weight.shape[0] % 16 == 0
-                        and ri.dim <= 256 and ri.heads * ri.vdim % 128 == 0 and hidden % 128 == 0 and hidden <= 8192)
+                        and ri.dim <= 256 and ri.dim % 4 == 0 and ri.vdim % 4 == 0 and ri.heads * ri.vdim % 128 == 0 and hidden % 128 == 0 and hidden <= 8192)
 
     def cache_spec(self) -> LayerCacheSpec:
         return LayerCacheSpec(kv=self.left.cache_spec(), rec=self.right.cache_spec())

@@ -13,9 +13,9 @@ void seq_launch_sandwich_rows(float*, const float*, int, const float*, int, cons
                               const float*, void*, int, int, float, hipStream_t);
 void seq_launch_gated_rmsnorm(void*, const float*, const float*, const void*, int, int, int, int, float, int,
                               int, hipStream_t);
-void seq_launch_rope_pairs_store(void*, const void*, const void*, const int64_t*, const float*, void*, void*,
-                                 const int64_t*, void*, int, int, int, int, int, int, int, int, int, int, int,
-                                 hipStream_t);
+void seq_launch_hybrid_split(const float*, int, const void*, const int64_t*, const int64_t*, const float*, void*, void*,
+                             const int64_t*, void*, void*, float*, void*, int, int, int, int, int, int, int, int, int,
+                             hipStream_t);
 void seq_launch_linear_attn_decay(float*, const void*, const void*, const void*, const float*, float*, float*,
                                   const int*, const int*, const int*, int, int, int, int, int, int, int, int,
                                   int, hipStream_t);
@@ -115,7 +115,7 @@ Tensor hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tensor bias, std::v
   check(state, at::kFloat, state.numel(), "state");
   check(decay, at::kFloat, RH, "decay");
   check(norm_right, at::kFloat, (int64_t)RH * RV, "norm_right");
-  TORCH_CHECK(RD <= 256, "key size above 256 is not supported by the recurrence kernel");
+  TORCH_CHECK(RD <= 256 && RD % 4 == 0 && RV % 4 == 0, "key sizes of the recurrence kernel: up to 256, in fours");
   check_weight(o_left, (int64_t)H * D, "o_left");
   check_weight(o_right, (int64_t)RH * RV, "o_right");
   TORCH_CHECK(o_left.size(0) == W && o_right.size(0) == W);
@@ -139,24 +139,28 @@ Tensor hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tensor bias, std::v
 
   auto st = cur_stream();
   const auto f32 = x.options();
-  const Tensor y = rows_bf16(h, w_in, bias, T, st);
-  seq_launch_rope_pairs_store((void*)bf(y, at[0]), bf(y, at[1]), nullptr, positions.data_ptr<int64_t>(),
-                              inv_freq.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
-                              slots.data_ptr<int64_t>(), nullptr, T, H, G, D, D, R, BS, N, N, 0, 0, st);
+  const Tensor y = part(h, w_in, T, st);
+  auto q = torch::empty({T, (int64_t)H * D}, h.options()), head_gate = torch::empty({T, H}, h.options()),
+       gate = torch::empty({T, (int64_t)RH * RV}, h.options());
+  auto packed = torch::empty({T, (int64_t)RH * (2 * RD + RV)}, f32);
+  seq_launch_hybrid_split(y.data_ptr<float>(), y.size(0), bias.numel() ? bias.data_ptr() : nullptr, at.data(),
+                          positions.data_ptr<int64_t>(), inv_freq.data_ptr<float>(), k_cache.data_ptr(),
+                          v_cache.data_ptr(), slots.data_ptr<int64_t>(), q.data_ptr(), head_gate.data_ptr(),
+                          packed.data_ptr<float>(), gate.data_ptr(), T, N, H, G, R, BS, RH, RD, RV, st);
   auto att = torch::empty({T, (int64_t)H * D}, h.options());
   const int64_t longest = mask_size > 0 ? std::min<int64_t>(mask_size, (int64_t)width * BS) : (int64_t)width * BS;
   const int splits = attn_decode_splits(T, G, (int)std::min<int64_t>(longest, INT32_MAX));
   auto partials = torch::empty({splits > 1 ? (int64_t)T * H * splits * 130 : 0}, f32);
-  launch_attn_decode((__hip_bfloat16*)att.data_ptr(), partials.data_ptr<float>(), bf(y, at[0]), k_cache.data_ptr(),
-                     v_cache.data_ptr(), nullptr, nullptr, tables.data_ptr<int>(), lens.data_ptr<int>(), bf(y, at[2]), N,
-                     (float)scale, H, G, BS, width, splits, N, T, 0, (int)mask_size, st);
-  auto o = torch::empty({T, (int64_t)RH * RV}, f32), packed = torch::empty({T, (int64_t)RH * (2 * RD + RV)}, f32);
-  seq_launch_linear_attn_decay(o.data_ptr<float>(), bf(y, at[3]), bf(y, at[4]), bf(y, at[5]), decay.data_ptr<float>(),
+  launch_attn_decode((__hip_bfloat16*)att.data_ptr(), partials.data_ptr<float>(), bf(q), k_cache.data_ptr(),
+                     v_cache.data_ptr(), nullptr, nullptr, tables.data_ptr<int>(), lens.data_ptr<int>(), bf(head_gate), H,
+                     (float)scale, H, G, BS, width, splits, H * D, T, 0, (int)mask_size, st);
+  auto o = torch::empty({T, (int64_t)RH * RV}, f32);
+  seq_launch_linear_attn_decay(o.data_ptr<float>(), nullptr, nullptr, nullptr, decay.data_ptr<float>(),
                                packed.data_ptr<float>(), state.data_ptr<float>(), state_slots.data_ptr<int>(),
-                               cu.data_ptr<int>(), seg_start.data_ptr<int>(), T, T, RH, RD, RV, N, N, N, 0, st);
+                               cu.data_ptr<int>(), seg_start.data_ptr<int>(), T, T, RH, RD, RV, 0, 0, 0, 0, st);
   auto yr = torch::empty({T, (int64_t)RH * RV}, h.options());
-  seq_launch_gated_rmsnorm(yr.data_ptr(), o.data_ptr<float>(), norm_right.data_ptr<float>(), bf(y, at[6]), T, 1, RH * RV, N,
-                           (float)eps, 0, 0, st);
+  seq_launch_gated_rmsnorm(yr.data_ptr(), o.data_ptr<float>(), norm_right.data_ptr<float>(), gate.data_ptr(), T, 1, RH * RV,
+                           RH * RV, (float)eps, 0, 0, st);
   const Tensor left = part(att, o_left, T, st), right = part(yr, o_right, T, st);
   auto out = torch::empty_like(h);
   seq_launch_sandwich_rows(x.data_ptr<float>(), left.data_ptr<float>(), left.size(0), right.data_ptr<float>(),
