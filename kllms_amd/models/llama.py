@@ -3,9 +3,10 @@
 The model runner behind engine.generate() — the native replacement for the
 reference's remote `chat.completions.create` model execution
 (k_llms/resources/completions/completions.py:73). Torch modules orchestrate
-hipBLASLt/rocBLAS GEMMs (via F.linear) while every non-GEMM hot op
-(RMSNorm, RoPE, varlen prefill attention, paged decode attention, SwiGLU,
-KV scatter) dispatches to the hand-written CDNA4 HIP kernels in kllms_amd.ops.
+the products (ops.linear and the few-row kernels, hipBLASLt/rocBLAS where it is
+the faster one) while every other hot op (RMSNorm, RoPE, varlen prefill
+attention, paged decode attention, SwiGLU, KV scatter) dispatches to the
+hand-written CDNA4 HIP kernels in kllms_amd.ops.
 
 Two forward modes driven by ForwardBatch:
 - prefill: packed varlen batch (shared prefill across requests), causal

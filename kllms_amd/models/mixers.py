@@ -9,8 +9,8 @@ side input; differential attention and the dynamic-tanh norm. Each runs on "segm
 portions and single decoded tokens, attention keys found through the block
 table and recurrent state carried in per-sequence slots.
 
-GEMMs go through F.linear (hipBLASLt / rocBLAS); everything between them is a
-kllms_amd.ops kernel. Activations are the model dtype (bf16 when serving,
+Products go through ops.linear (the tile kernel for prompts, else hipBLASLt /
+rocBLAS); everything between them is a kllms_amd.ops kernel. Activations are the model dtype (bf16 when serving,
 fp32 in exact mode); norm weights, recurrence constants, attention weights
 and recurrent state are fp32 in both.
 """

@@ -278,46 +278,28 @@ def _plain_call(*ts: torch.Tensor) -> bool:
             and not torch.compiler.is_compiling() and not torch._C._len_torch_dispatch_stack())
 
 
-def _tiles(x: torch.Tensor, w: torch.Tensor, act: int, bias: Optional[torch.Tensor] = None) -> int:
-    """Rows of a tile, in steps of 32, + 16 for shares of K, where the tile kernel takes x [M, K] @ w^T, or 0: bf16 on the GPU, contiguous,
-    sizes that its 16-byte accesses and 64-deep stages divide, no gradient to keep, and the faster side of the rule."""
-    if (x.dim() != 2 or x.shape[0] <= 128 or not x.is_cuda or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16
-            or w.dim() != 2 or x.device != w.device or _force_torch()):
-        return 0
-    if not (_plain_call(x, w) if bias is None else _plain_call(x, w, bias)):
-        return 0
-    n = w.shape[0] // 2 if act else w.shape[0]
-    k = x.shape[1]
-    if (k % 64 or k == 0 or k >= 1 << 24 or n % 8 or n == 0 or w.shape[1] != k or max(x.shape[0], n) >= 1 << 30
-            or not x.is_contiguous() or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16
-            or x.shape[0] * n >= 1 << 38 or (act and w.shape[0] % 2)):
-        return 0
-    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)):
-        return 0
-    if bias is not None and not (bias.dtype == x.dtype and bias.device == x.device and bias.dim() == 1
-                                 and bias.shape[0] == n and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
-        return 0
-    return _hip_or_raise().linear_tiles_rows(x.shape[0], n, k, act)
+def _try_tiles(x, w, bias, act: int, limit: float = 0.0, alpha: float = 0.0) -> Optional[torch.Tensor]:
+    """The product on the tile kernel, where it takes the call (bf16 on the GPU, more than 128 rows, contiguous, sizes that
+    its 16-byte accesses and 64-deep stages divide, no gradient or transform to serve) and is the faster one."""
+    if x.is_cuda and x.dim() == 2 and x.shape[0] > 128 and not _force_torch():
+        return _hip_or_raise().linear_tiles_try(x, w, bias, act, limit, alpha)
+    return None
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x @ w^T + bias: prompts on the tile kernel where that is the faster one, everything else in the library."""
-    mj = _tiles(x, w, 0, bias)
-    if mj:
-        return _C.linear_tiles(x, w, bias if bias is not None else _none(x), 0, mj & 15, mj > 15, 0.0, 0.0)
-    return torch.nn.functional.linear(x, w, bias)
+    y = _try_tiles(x, w, bias, 0)
+    return y if y is not None else torch.nn.functional.linear(x, w, bias)
 
 
 def linear_silu(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     """silu(gate) * up of a fused [gate; up] matrix for prompts, or None where the tile kernel does not take it."""
-    mj = _tiles(x, w, 1)
-    return _C.linear_tiles(x, w, _none(x), 1, mj & 15, mj > 15, 0.0, 0.0) if mj else None
+    return _try_tiles(x, w, None, 1)
 
 
 def linear_clamped_glu(x: torch.Tensor, w: torch.Tensor, limit: float, alpha: float) -> Optional[torch.Tensor]:
     """clamped_glu of a fused [gate; up] matrix for prompts, or None where the tile kernel does not take it."""
-    mj = _tiles(x, w, 2)
-    return _C.linear_tiles(x, w, _none(x), 2, mj & 15, mj > 15, limit, alpha) if mj else None
+    return _try_tiles(x, w, None, 2, limit, alpha)
 
 
 def embed_norm_rows(ids, table, weight, eps, unknown=None):

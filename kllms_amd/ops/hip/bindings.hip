@@ -396,6 +396,45 @@ torch::Tensor linear_tiles(torch::Tensor x, torch::Tensor w, torch::Tensor bias,
   return out;
 }
 
+// Whether nothing but the values of a tensor is wanted: no subclass, transform or gradient looks on
+static bool plain_values(const torch::Tensor& t) {
+  static const c10::DispatchKeySet others({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot,
+                                           c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                           c10::DispatchKey::FuncTorchVmapMode, c10::DispatchKey::Batched,
+                                           c10::DispatchKey::VmapMode, c10::DispatchKey::Functionalize,
+                                           c10::DispatchKey::FuncTorchDynamicLayerFrontMode,
+                                           c10::DispatchKey::FuncTorchDynamicLayerBackMode});
+  const auto keys = t.key_set() | c10::impl::tls_local_dispatch_key_set().included_;
+  return !keys.has_any(others) && !(at::GradMode::is_enabled() && t.requires_grad()) && !t._fw_grad(0).defined();
+}
+
+// mj of linear_tiles, + 16 for shares, where it takes the call and is the faster side of linear_tiles_rows; 0: the library's
+int64_t linear_tiles_pick(const torch::Tensor& x, const torch::Tensor& w, const std::optional<torch::Tensor>& bias,
+                          int64_t act) {
+  if (x.dim() != 2 || w.dim() != 2 || x.size(0) <= 128 || !x.is_cuda() || x.device() != w.device() ||
+      x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16)
+    return 0;
+  if (!plain_values(x) || !plain_values(w) || torch::jit::tracer::isTracing()) return 0;
+  const int64_t M = x.size(0), K = x.size(1), N = act ? w.size(0) / 2 : w.size(0);
+  auto on_16 = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  if (K % 64 || K == 0 || K >= 1 << 24 || N % 8 || N == 0 || w.size(1) != K || std::max(M, N) >= 1 << 30 ||
+      !x.is_contiguous() || !w.is_contiguous() || !on_16(x) || !on_16(w) || M * N >= (int64_t)1 << 38 ||
+      (act && w.size(0) % 2))
+    return 0;
+  if (bias && !(bias->scalar_type() == at::kBFloat16 && bias->device() == x.device() && bias->dim() == 1 &&
+                bias->size(0) == N && bias->is_contiguous() && on_16(*bias) && plain_values(*bias)))
+    return 0;
+  return linear_tiles_rows(M, N, K, (int)act);
+}
+
+// linear_tiles where linear_tiles_pick takes the call, else nothing. One call: from Python the checks alone are 5 us
+std::optional<torch::Tensor> linear_tiles_try(torch::Tensor x, torch::Tensor w, std::optional<torch::Tensor> bias, int64_t act,
+                                              double limit, double alpha) {
+  const int64_t mj = linear_tiles_pick(x, w, bias, act);
+  if (!mj) return std::nullopt;
+  return linear_tiles(x, w, bias ? *bias : x.new_empty({0}), (int)act, mj & 15, mj > 15, limit, alpha);
+}
+
 // topi [T, k] int64 -> (ids [T * k] token of each sorted place, pos [T, k] sorted place of each pair,
 // offsets [E + 1]); a pair without an expert of 0..E-1 gets pos -1
 std::vector<torch::Tensor> moe_sort(torch::Tensor topi, int64_t E) {
@@ -606,6 +645,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_inputs", &decode_inputs);
   m.def("linear_tiles", &linear_tiles);
   m.def("linear_tiles_rows", &linear_tiles_rows);
+  m.def("linear_tiles_pick", &linear_tiles_pick);
+  m.def("linear_tiles_try", &linear_tiles_try);
   m.def("moe_gateup", &moe_gateup);
   m.def("moe_down", &moe_down);
   m.def("moe_sort", &moe_sort);

@@ -16,8 +16,8 @@
 //   N 4096, K 14336       1170 rows 146, 130    1600 rows 330, 168     3100 rows 334, 280    11700 rows 1303, 1019
 //   N 4096, K 4096        3100 rows  82,  77    4700 rows 139, 125    11700 rows  442,  276
 //   silu N 14336, K 4096   300 rows  81,  72     777 rows 189, 167    3100 rows 698, 557    11700 rows 2099, 2011
-//   silu N 8192, K 2048    300 rows  34,  31     777 rows  60,  47    4700 rows 347, 253     7777 rows  454,  403
-//   N 8720, K 2048         777 rows  34,  33    3100 rows 135,  92     7777 rows 240, 220
+//   silu N 8192, K 2048    300 rows  36,  32     777 rows  61,  51    4700 rows 347, 253     7777 rows  454,  403
+//   N 8720, K 2048        1200 rows  48,  43    3300 rows 138, 107     7777 rows 240, 220
 
 #include "tile_product.h"
 
@@ -142,12 +142,16 @@ extern "C" int linear_tiles_rows(int64_t M, int64_t N, int64_t K, int act) {
   }
   // few rows: the weights' stream bounds, which one tile a column does not keep up
   if (M <= 128) return 0;
-  // long K on few tiles, at K 4096 (library and here, N 4096: 25 us and 43 at 300 rows, 44 and 46 at 1170, 59 and
-  // 58 at 2048; silu N 14336: 81 and 72 at 300). At K 2048 a tile is short enough (N 2048: 19 and 18 at 300 rows); longer
-  // K is shared out (N 4096, K 14336: 63 and 63 at 256 rows, 83 and 74 at 400, 330 and 168 at 1600; N 2048, K 8192: 32
-  // and 35 at 400, 44 and 40 at 700)
+  // Few tiles: the library splits K and makes its tiles smaller. Where both are even (us of the library and here, in a
+  // graph), by results: at K 2048 from 3.5 million (N 2048: 11 and 19 at 300 rows, 20.0 and 20.3 at 1200, 29.8 and 24.5 at
+  // 2600; N 8720: 25 and 28 at 300, 30.7 and 30.6 at 465, 48 and 43 at 1200), at K 4096 from 6.5 (N 4096: 26 and 54 at 300, 48 and 53
+  // at 1200, 58.5 and 56.8 at 1600). Longer K is shared out (N 4096, K 14336: 63 and 63 at 256 rows, 78 and 67 at
+  // 300, 325 and 176 at 1600; N 2048, K 8192: 34 and 36 at 400, 44 and 42 at 600). Gated products save the activation's
+  // launch and pass: ahead from the start at K 2048 (16384 rows of w: 31 and 29 at 140), later at K 4096 (28672: 67 and 69
+  // at 140, 80 and 71 at 200)
   const int64_t outputs = M * N * (act ? 2 : 1);
-  if (K > 2048 && outputs < (K < LT_LONG ? (int64_t)1 << 23 : 1200000)) return 0;
+  const int64_t least_outputs = K >= LT_LONG ? 1200000 : act ? (K > 2048 ? 5000000 : 0) : K > 2048 ? 6500000 : 3500000;
+  if (outputs < least_outputs) return 0;
   // 256 x 256 tiles that fill one or two rounds to 0.92 and more: the library's are 4 to 10 % faster (N 4096, K 4096 /
   // 14336: 3710 rows 94 and 99 / 309 and 339, 8100 rows 184 and 200 / 619 and 699). Below it is not, on balance (2700
   // rows 78 and 77 / 249 and 253; 4200 rows 140 and 125 / 730 and 377; 7600 rows 179 and 195 / 1009 and 696), and

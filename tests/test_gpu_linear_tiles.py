@@ -51,7 +51,7 @@ def test_tiles_against_float64(M, N, K, share, mj):
 
 
 @gpu
-@pytest.mark.parametrize("M,N,K,act", [(300, 3216, 2048, 0), (1170, 6144, 4096, 0), (700, 2048, 8192, 0), (777, 8192, 2048, 1), (400, 8192, 2048, 2)])
+@pytest.mark.parametrize("M,N,K,act", [(1300, 3216, 2048, 0), (1170, 6144, 4096, 0), (700, 2048, 8192, 0), (777, 8192, 2048, 1), (400, 8192, 2048, 2)])
 def test_entry_points_against_float64(M, N, K, act):
     x, w = _operands(M, N, K, act > 0, 2)
     y = x.double() @ w.double().t()
@@ -80,21 +80,29 @@ def test_extreme_sums_of_the_clamped_form():
 
 @gpu
 def test_calls_that_stay_with_the_library():
-    x, w = _operands(512, 2048, 1024, False)
-    assert ops._tiles(x, w, 0)
-    assert not ops._tiles(x[:128], w, 0) and not ops._tiles(x.float(), w.float(), 0)
-    assert not ops._tiles(x[:, ::2], w[:, ::2], 0) and not ops._tiles(x[:, :1000].contiguous(), w[:, :1000].contiguous(), 0)
-    assert not ops._tiles(x.t().contiguous().t(), w, 0) and not ops._tiles(x.view(2, 256, 1024), w, 0)
+    pick = lambda x, w, bias=None: ops._hip_or_raise().linear_tiles_pick(x, w, bias, 0)  # noqa: E731
+    x, w = _operands(2048, 2048, 1024, False)
+    assert pick(x, w) and pick(x, torch.nn.Parameter(w, requires_grad=False))
+    assert not pick(x[:128], w) and not pick(x.float(), w.float())
+    assert not pick(x[:, ::2], w[:, ::2]) and not pick(x[:, :1000].contiguous(), w[:, :1000].contiguous())
+    assert not pick(x.t().contiguous().t(), w) and not pick(x.view(2, 1024, 1024), w)
     off = torch.empty(x.numel() + 1, device=DEV, dtype=x.dtype)[1:].view_as(x).copy_(x)
-    assert not ops._tiles(off, w, 0) and torch.allclose(ops.linear(off, w).float(), ops.linear(x, w).float(), atol=0.05)
-    assert not ops._tiles(x, w, 0, torch.zeros(2048, device=DEV))
+    assert not pick(off, w) and torch.allclose(ops.linear(off, w).float(), ops.linear(x, w).float(), atol=0.05)
+    assert not pick(x, w, torch.zeros(2048, device=DEV))
     xg = x.clone().requires_grad_()
     ops.linear(xg, w).sum().backward()
     assert xg.grad is not None
     with torch.no_grad():
-        assert ops._tiles(xg, w, 0)
-    got = torch.func.vmap(lambda t: ops.linear(t, w))(x.view(2, 256, 1024))
-    assert torch.allclose(got.view(512, -1).float(), ops.linear(x, w).float(), atol=0.05)
+        assert pick(xg, w)
+    got = torch.func.vmap(lambda t: ops.linear(t, w))(x.view(2, 1024, 1024))
+    assert torch.allclose(got.view(2048, -1).float(), ops.linear(x, w).float(), atol=0.05)
+    _, tangent = torch.func.jvp(lambda t: ops.linear(t, w), (x,), (x,))
+    assert torch.allclose(tangent.float(), ops.linear(x, w).float(), atol=0.05)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, x)
+        assert not pick(dual, w)
+    traced = torch.jit.trace(lambda t: ops.linear(t, w), (x,), check_trace=False)
+    assert torch.allclose(traced(x * 2).float(), ops.linear(x * 2, w).float(), atol=0.05)
 
 
 def test_rule_of_the_tiles():
@@ -105,6 +113,7 @@ def test_rule_of_the_tiles():
     assert rows(256, 4096, 14336, 0) == 0                      # long K on few tiles
     assert rows(1170, 4096, 14336, 0) == 5 + 16                # 128 tiles of 147 rows, in two shares each
     assert rows(7777, 4096, 4096, 0) == 0                      # 496 tiles of the 512 of two rounds
+    assert rows(300, 2048, 2048, 0) == 0 and rows(1200, 4096, 4096, 0) == 0
     assert rows(300, 14336, 4096, 1) == 5                      # 224 tiles of 150 rows
     assert rows(11700, 4096, 14336, 0) == 8                    # 736 tiles in three rounds
     for M in range(1, 13000, 97):
