@@ -19,11 +19,11 @@
 //
 // Measured, 8 experts, top 2, us of gate/up and down, beside 256 x 256 tiles of eight waves that were
 // staged through registers:
-//   width 4096, experts of 14336   300 rows  396 + 194 (406 + 328)    1024 rows  525 + 349 (730 + 406)
-//                                 2048 rows  972 + 517 (1175 + 812)
+//   width 4096, experts of 14336   300 rows  356 + 184 (406 + 328)    1024 rows  551 + 343 (730 + 406)
+//                                 2048 rows  896 + 471 (1175 + 812)
 //   width 4096, experts of 7168   6000 rows  1117 + 566: 1260 TFLOP/s (1394 + 847)
-// The layer with its routing at 65 / 150 / 300 / 600 / 1024 / 2048 / 6000 rows, experts of 14336: 622 / 638 / 662 /
-// 714 / 918 / 1400 / 3502 us (741 / 760 / 787 / 907 / 1131 / 1935 / 4622).
+// The layer with its routing at 65 / 150 / 300 / 600 / 1024 / 2048 / 6000 rows, experts of 14336: 582 / 582 / 605 /
+// 666 / 949 / 1431 / 3623 us (741 / 760 / 787 / 907 / 1131 / 1935 / 4622).
 
 #include "tile_product.h"
 

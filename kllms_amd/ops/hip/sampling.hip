@@ -392,16 +392,20 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) a = min(a, __shfl_xor(a, off));
     const unsigned long long w = wave_max_u64(p.best);
-    const float edge = wave_reduce_max(p.edge);
-    const float lmass = wave_reduce_sum(p.listed == 0 ? 0.0f : p.mass * (p.max == M ? 1.0f : __expf((p.max - M) * inv_t)));
-    int total = p.listed;
+    if (lists && temp != 0.0f && truncates(top_p, top_k, V)) {
+      const float edge = wave_reduce_max(p.edge);
+      const float lmass = wave_reduce_sum(p.listed == 0 ? 0.0f : p.mass * (p.max == M ? 1.0f : __expf((p.max - M) * inv_t)));
+      int total = p.listed;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
-    sh_count[lane] = p.listed;
+      for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
+      sh_count[lane] = p.listed;
+      if (lane == 0) {
+        sh_edge = edge;
+        sh_mass = lmass;
+        sh_total = total;
+      }
+    }
     if (lane == 0) {
-      sh_edge = edge;
-      sh_mass = lmass;
-      sh_total = total;
       sh_max = M;
       sh_sum = S;
       sh_ssum = SS;
