@@ -567,9 +567,11 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   if (tid == 0) sh_best = (unsigned long long)NO_KEY << 32;
   // where the cut is behind the lists, the sweeps over bins that those hold whole are left out
   const int after = whole >= SMID ? 2 : whole >= SNEAR ? 1 : 0;
+  bool listing = false;                  // whether the part that found the cut, with those it adds to, listed its tokens
   for (int part = whole > 0 && hope ? -1 : after; part < 3; part = part < 0 ? after : part + 1) {
     const int from = part <= after ? 0 : part == 1 ? SNEAR : SMID;
     const int to = part < 0 ? whole : part == 0 ? SNEAR : part == 1 ? SMID : SBINS;
+    listing = part < 2;
     if (part <= after) {
       __syncthreads();
       clear_hist();
@@ -579,7 +581,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
     auto count = [&](int i, float sx, int bin) {
       atomicAdd(&my_mass[bin], __expf(sx));
       atomicAdd(&my_cnt[bin], 1u);
-      if (part < 2) {
+      if (listing) {
         const int at = atomicAdd(&sh_listed, 1);
         if (at < SLIST) {
           list_sx[at] = sx;
@@ -643,9 +645,11 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
 
   // ---- draw over the bins above the boundary --------------------------------
   // afterwards the list holds the boundary bin's tokens, among others, unless
-  // they outgrow it
+  // they outgrow it. Part 2 lists nothing, and behind the slices' lists it may
+  // end in any bin: their tokens added up in another order can reach a top-p that
+  // the lists' sum missed by its rounding
   const int cut = sh_cut;
-  const bool near = (cut < SMID || cut < whole) && sh_listed <= SLIST;   // whole: of the lists that were used, else 0
+  const bool near = listing && (cut < SMID || cut < whole) && sh_listed <= SLIST;   // whole: of the lists that were used, else 0
   const bool fits = near || (cut < SBINS && hist_cnt[cut] <= SLIST);
   float best = -INFINITY;
   int btok = argmax_tok;

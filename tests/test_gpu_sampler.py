@@ -213,3 +213,36 @@ def test_cut_inside_and_behind_the_slices_lists(B, V, near):
         t = int(toks[b])
         # ties of fp32 logits at the cut may go either way; fast logarithms are off by 4e-7 of the draw's range
         assert x[t] >= x[kept[-1]] and key[t] >= key[kept].max() - max(1e-3, 4e-7 * V)
+
+
+@pytest.mark.parametrize("ulps", [1, 2, 16])
+def test_top_p_a_few_ulps_below_one(ulps):
+    """Rows whose allowed tokens all lie in the slices' lists: whether fp32 sums of their masses reach top_p of the whole
+    depends on the order of the sums, and every order has to end in a draw."""
+    B, V, near = 32, 128256, 400
+    top_p = float(np.float32(1.0) - np.float32(ulps * 2.0 ** -24))
+    g = torch.Generator(device=DEV).manual_seed(ulps)
+    for call in range(32):
+        at = torch.rand(B, V, generator=g, device=DEV).topk(near, -1).indices
+        x = torch.rand(B, near, generator=g, device=DEV)
+        logits = torch.zeros(B, V, device=DEV).scatter_(1, at, x)
+        words = torch.zeros(B, V // 32, dtype=torch.long, device=DEV)
+        words.scatter_add_(1, at // 32, torch.ones_like(at) << (at % 32))
+        mask = torch.where(words >= 2**31, words - 2**32, words).to(torch.int32)
+        seeds = torch.randint(0, 2**40, (B,), generator=g, device=DEV)
+        steps = torch.randint(0, 99, (B,), generator=g, device=DEV)
+        toks, _ = ops.sample(logits, torch.ones(B, device=DEV), torch.full((B,), top_p, device=DEV),
+                             torch.zeros(B, dtype=torch.int32, device=DEV), seeds, steps, mask)
+        at, x, seeds, steps, toks = (t.cpu().numpy() for t in (at, x.double(), seeds, steps, toks))
+        with np.errstate(over="ignore"):
+            base = splitmix(seeds.astype(np.uint64) * np.uint64(0x9E3779B97F4A7C15)
+                            + steps.astype(np.uint64) * np.uint64(0xBF58476D1CE4E5B9))
+            h = splitmix(base[:, None] ^ at.astype(np.uint64)) >> np.uint64(40)
+        u = ((h + np.uint64(1)).astype(np.float32) * np.float32(1.0 / 16777217.0)).astype(np.float64)
+        key = x - np.log(-np.log(u))
+        for b in range(B):
+            won = np.nonzero(at[b] == toks[b])[0]
+            assert won.size == 1
+            # the lowest ten of 400 (a fortieth of the mass at most, the rounding of the sums is 1e-5 of it) may be out
+            kept = np.argsort(-x[b])[:near - 10]
+            assert key[b, won[0]] >= key[b, kept].max() - 1e-3, (call, b)
