@@ -249,14 +249,21 @@ __device__ __forceinline__ bool tile_fold(f32x4 (&acc)[8][MJ], float* part, int 
 #pragma unroll 1
     for (int s0 = 0; s0 < shares; s0 += 2) {
       u32x4 v[2][2][MJ];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int s = s0 + e;            // behind the last share: zeros, as the range ends there
+      auto load = [&](int e) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int j = 0; j < MJ; ++j)
-            v[e][i][j] = __builtin_amdgcn_raw_buffer_load_b128(all, tid * 16, s * SIZE + ((i0 + i) * MJ + j) * TP_THREADS * 16, SC1);
+            v[e][i][j] = __builtin_amdgcn_raw_buffer_load_b128(all, tid * 16, (s0 + e) * SIZE + ((i0 + i) * MJ + j) * TP_THREADS * 16, SC1);
+      };
+      load(0);
+      if (s0 + 1 < shares) {
+        load(1);
+      } else {                           // an odd number of shares: the last one alone, nothing is read behind it
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < MJ; ++j) v[1][i][j] = u32x4{0u, 0u, 0u, 0u};
       }
 #pragma unroll
       for (int e = 0; e < 2; ++e)

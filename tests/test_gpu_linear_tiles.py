@@ -22,8 +22,8 @@ def _near(got, ref, sums):
     return ((got.double() - ref).abs() <= 2 ** -8 * ref.abs() + sums).all()
 
 
-# one row, one column unit, odd rows behind a tile, a last column tile of 8, one stage and odd numbers of them; shares of
-# 33 stages in two, of 65 in four
+# one row, one column unit, odd rows behind a tile, a last column tile of 8, one stage and odd numbers of them; at 17 stages
+# two shares, at 33 and 65 four, where the rule's tiles leave units idle
 SIZES = [(1, 8, 64), (33, 264, 128), (129, 520, 1088), (257, 256, 2112), (1031, 1288, 192),
          (70, 2056, 4160)]
 
@@ -48,6 +48,33 @@ def test_tiles_against_float64(M, N, K, share, mj):
     assert _near(C.linear_tiles(x, w, bias[:0], 1, mj, share, 0.0, 0.0), F.silu(g) * u, slack)
     c, d = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
     assert _near(C.linear_tiles(x, w, bias[:0], 2, mj, share, 1.5, 1.702), c * torch.sigmoid(1.702 * c) * (d + 1), slack)
+
+
+def _shares(M, N, K, mj):
+    """Shares of the last round's tiles on each XCD, and whole rounds before it: (tiles, 256 x 32 mj) dealt to 8 x 32 units."""
+    tiles, stages = -(-M // (32 * mj)) * -(-N // 256), K // 64
+    out = set()
+    for xcd in range(8):
+        n = tiles * (xcd + 1) // 8 - tiles * xcd // 8
+        out.add((max(1, min(32 // (n % 32), 4, stages // 8)) if n % 32 else 1, n // 32))
+    return out
+
+
+# 9 of an XCD's 32 units in three shares; the same behind a whole round; odd numbers of stages in two, three and four shares
+SHARED = [(576, 2048, 1536, 2), (2624, 2048, 1536, 2), (2600, 2040, 2624, 2), (1100, 2048, 1600, 3), (450, 1032, 4160, 4),
+          (3400, 1536, 1088, 8), (2200, 2048, 2112, 2)]
+
+
+@gpu
+@pytest.mark.parametrize("M,N,K,mj", SHARED)
+def test_shares_against_float64(M, N, K, mj):
+    test_tiles_against_float64(M, N, K, True, mj)
+
+
+def test_shares_of_every_kind_are_tested():
+    kinds = set().union(*(_shares(*c) for c in SHARED), *(_shares(*c, 8) for c in SIZES))
+    assert {s for s, _ in kinds} == {1, 2, 3, 4}
+    assert {s for s, rounds in kinds if rounds} >= {3, 4}
 
 
 @gpu
