@@ -122,23 +122,42 @@ __global__ void __launch_bounds__(TP_THREADS, 1) moe_product_kernel(
 }
 
 // topi [P] (P = tokens x choices) -> offsets [E + 1], pos [P] = sorted place of each
-// pair, ids [P] = token of each sorted place. One workgroup: counts by wave ballots,
-// which also give the places (same order as the pairs' within a wave's 64; the order
-// inside an expert matters to nobody).
-__global__ void __launch_bounds__(1024) moe_sort_kernel(int* __restrict__ ids, int* __restrict__ pos,
-                                                        int* __restrict__ offsets, const int64_t* __restrict__ topi,
-                                                        int P, int k, int E) {
-  extern __shared__ int cnt[];           // [E] counts, then cursors
+// pair, ids [P] = token of each sorted place, an expert's in the order of the pairs: which
+// of the products' tiles a row falls into, and with it the order of its sums, is so the
+// same in every call. One workgroup, a run of the pairs to each of its ``waves`` waves
+// that count: by ballots, which also give the places, in a row of counts of its own.
+#define SORT_WAVES 16
+
+__global__ void __launch_bounds__(64 * SORT_WAVES) moe_sort_kernel(int* __restrict__ ids, int* __restrict__ pos,
+                                                                   int* __restrict__ offsets,
+                                                                   const int64_t* __restrict__ topi, int P, int k, int E,
+                                                                   int waves) {
+  extern __shared__ int cnt[];           // [waves][E] counts, then cursors
   const int tid = threadIdx.x, lane = tid & 63;
-  for (int e = tid; e < E; e += 1024) cnt[e] = 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t run = ((int64_t)P + waves * 64 - 1) / (waves * 64) * 64;
+  const int64_t begin = wave < waves ? wave * run : P, end = begin + run < P ? begin + run : P;
+  int* mine = cnt + min(wave, waves - 1) * E;
+  for (int i = tid; i < waves * E; i += 64 * SORT_WAVES) cnt[i] = 0;
   __syncthreads();
-  for (int p0 = 0; p0 < P; p0 += 1024) {
-    const int p = p0 + tid;
-    const int e = p < P ? (int)topi[p] : -1;
+  for (int64_t p0 = begin; p0 < end; p0 += 64) {
+    const int64_t p = p0 + lane;
+    const int e = p < end ? (int)topi[p] : -1;
     for (int c = 0; c < E; ++c) {
       const unsigned long long m = __ballot(e == c);
-      if (m && lane == 0) atomicAdd(&cnt[c], (int)__popcll(m));
+      if (m && lane == 0) mine[c] += (int)__popcll(m);
     }
+  }
+  __syncthreads();
+  // an expert's pairs before each run; its whole number in the first run's place
+  for (int c = tid; c < E; c += 64 * SORT_WAVES) {
+    int at = 0;
+    for (int w = 0; w < waves; ++w) {
+      const int n = cnt[w * E + c];
+      cnt[w * E + c] = at;
+      at += n;
+    }
+    cnt[c] = at;
   }
   __syncthreads();
   if (tid == 0) {
@@ -152,21 +171,23 @@ __global__ void __launch_bounds__(1024) moe_sort_kernel(int* __restrict__ ids, i
     offsets[E] = at;
   }
   __syncthreads();
-  for (int p0 = 0; p0 < P; p0 += 1024) {
-    const int p = p0 + tid;
-    const int e = p < P ? (int)topi[p] : -1;
+  for (int i = E + tid; i < waves * E; i += 64 * SORT_WAVES) cnt[i] += cnt[i % E];
+  __syncthreads();
+  for (int64_t p0 = begin; p0 < end; p0 += 64) {
+    const int64_t p = p0 + lane;
+    const int e = p < end ? (int)topi[p] : -1;
     int place = -1;
     for (int c = 0; c < E; ++c) {
       const unsigned long long m = __ballot(e == c);
       if (!m) continue;
       int first = 0;
-      if (lane == 0) first = atomicAdd(&cnt[c], (int)__popcll(m));
+      if (lane == 0) first = atomicAdd(&mine[c], (int)__popcll(m));
       first = __shfl(first, 0);
       if (e == c) place = first + (int)__popcll(m & ((1ULL << lane) - 1));
     }
-    if (p < P) {
+    if (p < end) {
       pos[p] = place;
-      if (place >= 0) ids[place] = p / k;
+      if (place >= 0) ids[place] = (int)(p / k);
     }
   }
 }
@@ -226,7 +247,10 @@ extern "C" int64_t moe_down_room(int S, int E, int H, int* zeros) {
 
 extern "C" void launch_moe_sort(int* ids, int* pos, int* offsets, const int64_t* topi, int P, int k, int E,
                                 hipStream_t stream) {
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), E * sizeof(int), stream, ids, pos, offsets, topi, P, k, E);
+  const int room = 65536 / (int)sizeof(int);       // of LDS
+  const int waves = E * SORT_WAVES <= room ? SORT_WAVES : room / E;
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(64 * SORT_WAVES), waves * E * sizeof(int), stream, ids, pos, offsets, topi,
+                     P, k, E, waves);
 }
 
 extern "C" void launch_moe_combine(void* out, const void* y, const float* weights, const int* pos, int T, int k,

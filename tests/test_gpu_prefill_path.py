@@ -194,6 +194,23 @@ def test_mixture_products_at_the_edges_of_row_tiles(H, I, counts):
     test_mixture_products_against_float64(H, I, counts)
 
 
+@pytest.mark.parametrize("E", [1, 8, 128, 1024, 1025, 4096])
+@pytest.mark.parametrize("T,k", [(1, 1), (63, 2), (65, 3), (1025, 2), (9001, 2)])
+def test_sort_of_the_mixture_keeps_the_order_of_the_pairs(T, k, E):
+    """Places of one expert in the order of the pairs, so that a row is in the same tile, with the same order of its sums,
+    in every call; an expert out of range has no place."""
+    topi = torch.randint(-1, E + 1, (T, k), generator=torch.Generator().manual_seed(T + E))
+    ids, pos, offsets = ops.moe_sort(topi.to(DEV), E)
+    flat = topi.flatten()
+    order = torch.sort(torch.where((flat >= 0) & (flat < E), flat, E), stable=True).indices
+    n = int(((flat >= 0) & (flat < E)).sum())
+    assert offsets.tolist() == [0] + torch.bincount(flat[order[:n]], minlength=E).cumsum(0).tolist()
+    assert torch.equal(ids[:n].cpu().long(), order[:n] // k)
+    want = torch.full((T * k,), -1)
+    want[order[:n]] = torch.arange(n)
+    assert torch.equal(pos.flatten().cpu().long(), want)
+
+
 def test_mixture_products_of_views_off_16_bytes():
     def off(*shape):
         n = torch.Size(shape).numel()
