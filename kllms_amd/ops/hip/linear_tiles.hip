@@ -68,10 +68,10 @@ __global__ void __launch_bounds__(TP_THREADS, 1) linear_tiles_kernel(bf16_t* __r
   const int64_t k0 = (int64_t)sh.first(K / TP_K) * TP_K;
   const int m = m0 + (wave & 1) * MJ * 16;         // first row of this wave's results
   const int m_put = m0 + wave * MJ * 8;
-  const TileRows xr(x + (int64_t)m_put * K + k0, m_end - m_put, MJ * 8, K, lane);
+  const TileRows xr(x + k0, m_put, m_end, MJ * 8, K, lane);
   // W rows of a gated tile: 64 gate, 64 up, the next 64 gate, 64 up
   const int n_put = ACT ? n0 + (wave >> 1) * 64 : n0 + wave * 64;
-  const TileRows wr(w + ((int64_t)n_put + (ACT ? (int64_t)(wave & 1) * N : 0)) * K + k0, N - n_put, 64, K, lane);
+  const TileRows wr(w + (ACT ? (int64_t)(wave & 1) * N : 0) * K + k0, n_put, N, 64, K, lane);
   // the XCDs begin at different k: rows of a power of two of bytes would have all of them at the same memory channels
   tile_product<MJ>(acc, wr, xr, stages, stages * xcd / 8, smem);
   if (sh.shares > 1 && !tile_fold<MJ>(acc, sh.part, sh.share, sh.shares, sh.count, smem)) return;

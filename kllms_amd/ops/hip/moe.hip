@@ -47,7 +47,7 @@ __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t*
   if constexpr (GATEUP) {
     // W rows of a tile: 64 gate, 64 up, the next 64 gate, 64 up
     const int n_put = n0 + (wave >> 1) * 64;
-    const TileRows wr(w + ((int64_t)e * 2 * N + n_put + (wave & 1) * N) * K + k0, N - n_put, 64, K, lane);
+    const TileRows wr(w + ((int64_t)e * 2 + (wave & 1)) * N * K + k0, n_put, N, 64, K, lane);
     TileGather<MJ> xr;
 #pragma unroll
     for (int i = 0; i < MJ; ++i) {
@@ -68,8 +68,8 @@ __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t*
     });
   } else {
     const int n_put = n0 + wave * 64, m_put = m0 + wave * MJ * 8;
-    const TileRows wr(w + ((int64_t)e * N + n_put) * K + k0, N - n_put, 64, K, lane);
-    const TileRows xr(a + (int64_t)m_put * K + k0, m_end - m_put, MJ * 8, K, lane);
+    const TileRows wr(w + (int64_t)e * N * K + k0, n_put, N, 64, K, lane);
+    const TileRows xr(a + k0, m_put, m_end, MJ * 8, K, lane);
     tile_product<MJ>(acc, wr, xr, stages, stages * (blockIdx.x & 7) / 8, smem);
     if (sh.shares > 1 && !tile_fold<MJ>(acc, sh.part, sh.share, sh.shares, sh.count, smem)) return;
     const int n = n0 + (wave >> 1) * 128;

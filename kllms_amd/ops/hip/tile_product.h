@@ -70,7 +70,7 @@ struct TileShare {
 
 #define TP_HOLD __builtin_amdgcn_sched_barrier(0)
 
-// Buffer descriptor of bytes from p on; lanes behind its end read zeros.
+// Buffer descriptor of bytes from p on; lanes whose own offset is behind its end read zeros.
 __device__ __forceinline__ u32x4 tp_range(const void* p, uint32_t bytes) {
   const uint64_t a = (uint64_t)p;
   u32x4 r;
@@ -83,6 +83,8 @@ __device__ __forceinline__ u32x4 tp_range(const void* p, uint32_t bytes) {
 
 // Copies of 16 bytes a lane to lds + lane * 16. They are written out because the
 // compiler makes every later LDS read wait for the builtin's; the waits stand in the loop.
+// The step to the copy's row is in the lane's offset, which the range check covers: of the scalar offset it
+// only has to hold that it stays within the range (k inside a row), not what a check makes of one beyond it.
 __device__ __forceinline__ void tp_copy(u32x4 range, uint32_t lane_off, uint32_t off, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(lane_off), "s"(range),
                "s"(off), "s"(lds)
@@ -93,16 +95,19 @@ __device__ __forceinline__ void tp_copy_at(uint64_t at, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(at), "s"(lds) : "memory");
 }
 
-// Rows of an operand in memory order, 8 to a copy: from base on, ``rows`` of them exist (the others read as zeros).
+// Rows of an operand in memory order, 8 to a copy: from row ``first`` of p on, those before ``end`` (1 or more) and
+// ``most`` of them at most; the others read as zeros. Behind the end altogether the last row stands in, so that the
+// range always holds a row: what comes of it belongs to rows or columns that are not stored.
 struct TileRows {
   u32x4 range;
-  uint32_t lane_off, row8;
-  __device__ __forceinline__ TileRows(const bf16_t* base, int rows, int most, int K, int lane)
-      : range(tp_range(base, (uint32_t)min(max(rows, 0), most) * K * 2)),
-        lane_off((uint32_t)(lane >> 3) * K * 2 + (((lane & 7) ^ (lane >> 3)) << 4)), row8(8u * K * 2) {}
-  __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds) const {
-    tp_copy(range, lane_off, k_off + i * row8, lds);
+  uint32_t at[8];            // this lane's offset in each copy: the same registers for all operands of one K
+  __device__ __forceinline__ TileRows(const bf16_t* p, int first, int end, int most, int K, int lane)
+      : range(tp_range(p + (int64_t)min(first, end - 1) * K, (uint32_t)min(end - min(first, end - 1), most) * K * 2)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      at[i] = (uint32_t)(i * 8 + (lane >> 3)) * K * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
   }
+  __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds) const { tp_copy(range, at[i], k_off, lds); }
 };
 
 // Rows anywhere: at[i] is the address of this lane's 16 bytes of the i-th copy in stage 0.
