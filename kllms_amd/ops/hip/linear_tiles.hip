@@ -25,12 +25,13 @@
 
 enum { LT_PLAIN = 0, LT_SILU = 1, LT_CLAMPED = 2 };
 
-// exp(x) to fp32's last places: the rounding of x * log2(e) is made good
+// exp(x) to fp32's last places: the rounding of x * log2(e), with that constant split into a high and a low part, is made
+// good where it counts: not above fp32's range, nor below it, where an infinite product would leave nothing of the rest
 __device__ __forceinline__ float lt_exp(float x) {
   const float t = x * 1.44269504088896341f;
   const float rest = __builtin_fmaf(x, 1.44269504088896341f, -t) + x * 1.92596299112661746e-8f;
   const float e = __builtin_amdgcn_exp2f(t);
-  return t < 126.0f ? __builtin_fmaf(e, rest * 0.693147180559945309f, e) : e;
+  return fabsf(t) < 126.0f ? __builtin_fmaf(e, rest * 0.693147180559945309f, e) : e;
 }
 
 template <int ACT, int MJ>

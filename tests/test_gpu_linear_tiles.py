@@ -106,6 +106,21 @@ def test_extreme_sums_of_the_clamped_form():
 
 
 @gpu
+def test_gates_without_a_limit():
+    """Sums behind fp32's range and close to it, with no limit: the gate's sigmoid ends at 0 and 1."""
+    x = torch.ones(8, 64, device=DEV).bfloat16()
+    w = torch.full((16, 64), 0.25, device=DEV).bfloat16()
+    w[:4] = torch.tensor([3e38, 5e36, -5e36, 1e-30], device=DEV).unsqueeze(1)      # inf, 3.2e38, -3.2e38, 6.4e-29
+    got = ops._hip_or_raise().linear_tiles(x, w, x[:0, 0], 2, 2, False, float("inf"), 1.702)
+    g, u = (x.float() @ w.float().t()).chunk(2, -1)
+    ref = g * torch.sigmoid(1.702 * g) * (u + 1)
+    assert torch.isinf(ref[:, 0]).all() and torch.equal(got.isnan(), ref.isnan())
+    assert torch.equal(got.isinf(), ref.bfloat16().isinf())
+    ok = ref.bfloat16().isfinite()
+    assert torch.allclose(got.float()[ok], ref[ok], rtol=2 ** -7)
+
+
+@gpu
 def test_calls_that_stay_with_the_library():
     pick = lambda x, w, bias=None: ops._hip_or_raise().linear_tiles_pick(x, w, bias, 0)  # noqa: E731
     x, w = _operands(2048, 2048, 1024, False)
