@@ -3,6 +3,7 @@
 
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+#include <c10/core/DeviceGuard.h>
 
 #include "common.h"
 
@@ -381,6 +382,8 @@ torch::Tensor linear_tiles(torch::Tensor x, torch::Tensor w, torch::Tensor bias,
   }
   auto on_16 = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
   TORCH_CHECK(on_16(x) && on_16(w) && (!biased || on_16(bias)), "linear_tiles: operands begin on 16 bytes");
+  // as the library: on the device of x, whatever the current one is
+  const c10::DeviceGuard device(x.device());
   auto out = torch::empty({M, N}, x.options());
   if (M == 0) return out;
   torch::Tensor part, count;

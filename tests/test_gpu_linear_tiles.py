@@ -147,6 +147,15 @@ def test_calls_that_stay_with_the_library():
     assert torch.allclose(traced(x * 2).float(), ops.linear(x * 2, w).float(), atol=0.05)
 
 
+@gpu
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="a device that is not the current one takes two")
+def test_operands_of_another_device_than_the_current_one():
+    x, w = _operands(2304, 2048, 1024, False)
+    with torch.cuda.device(1):
+        got = ops.linear(x, w)
+    assert got.device == x.device and torch.equal(got, ops.linear(x, w))
+
+
 def test_rule_of_the_tiles():
     if not ops.hip_available():
         pytest.skip("extension not built")
