@@ -2,6 +2,7 @@
 // Thin launch shims: shape/dtype checks, grid math, current-HIP-stream launch.
 
 #include <torch/extension.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/HIPContext.h>
 #include <c10/core/DeviceGuard.h>
 
@@ -418,6 +419,7 @@ int64_t linear_tiles_pick(const torch::Tensor& x, const torch::Tensor& w, const 
       x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16)
     return 0;
   if (!plain_values(x) || !plain_values(w) || torch::jit::tracer::isTracing()) return 0;
+  if (at::autocast::is_autocast_enabled(at::kCUDA)) return 0;      // the library's product has autocast's type
   const int64_t M = x.size(0), K = x.size(1), N = act ? w.size(0) / 2 : w.size(0);
   auto on_16 = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
   if (K % 64 || K == 0 || K >= 1 << 24 || N % 8 || N == 0 || w.size(1) != K || std::max(M, N) >= 1 << 30 ||

@@ -148,6 +148,18 @@ def test_calls_that_stay_with_the_library():
 
 
 @gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_autocast_decides_the_type_at_every_row_count(dtype):
+    x, w = _operands(2304, 2048, 1024, False)
+    with torch.autocast("cuda", dtype=dtype):
+        for rows in (64, 2304):
+            got = ops.linear(x[:rows], w)
+            assert got.dtype == dtype and torch.equal(got, F.linear(x[:rows], w))
+        assert ops.linear_silu(x, w) is None and ops.linear_clamped_glu(x, w, 7.0, 1.702) is None
+    assert ops.linear(x, w).dtype == torch.bfloat16 and ops.linear_silu(x, w) is not None
+
+
+@gpu
 @pytest.mark.skipif(torch.cuda.device_count() < 2, reason="a device that is not the current one takes two")
 def test_operands_of_another_device_than_the_current_one():
     x, w = _operands(2304, 2048, 1024, False)
