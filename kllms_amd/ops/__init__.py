@@ -271,17 +271,24 @@ def linear_f32_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 # --- products of many rows (prompts) ----------------------------------------------
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
 def _plain_call(*ts: torch.Tensor) -> bool:
     """Whether nothing but the values of these tensors is wanted: no transform, tracer or tensor subclass looks on."""
-    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts) and torch.autograd.forward_ad._current_level < 0
+    return (all(type(t) in _PLAIN for t in ts) and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._len_torch_function_stack()
             and not torch._C._are_functorch_transforms_active() and not torch.jit.is_tracing()
             and not torch.compiler.is_compiling() and not torch._C._len_torch_dispatch_stack())
 
 
 def _try_tiles(x, w, bias, act: int, limit: float = 0.0, alpha: float = 0.0) -> Optional[torch.Tensor]:
     """The product on the tile kernel, where it takes the call (bf16 on the GPU, more than 128 rows, contiguous, sizes that
-    its 16-byte accesses and 64-deep stages divide, no gradient or transform to serve) and is the faster one."""
-    if x.is_cuda and x.dim() == 2 and x.shape[0] > 128 and not _force_torch():
+    its 16-byte accesses and 64-deep stages divide, no gradient or transform to serve) and is the faster one. Subclasses,
+    function modes and the compiler see the library's product, as at every other row count."""
+    if (x.is_cuda and x.dim() == 2 and x.shape[0] > 128 and not torch.compiler.is_compiling()
+            and type(x) in _PLAIN and type(w) in _PLAIN and (bias is None or type(bias) in _PLAIN)
+            and not torch._C._len_torch_function_stack() and not _force_torch()):
         return _hip_or_raise().linear_tiles_try(x, w, bias, act, limit, alpha)
     return None
 

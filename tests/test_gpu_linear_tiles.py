@@ -159,6 +159,35 @@ def test_autocast_decides_the_type_at_every_row_count(dtype):
     assert ops.linear(x, w).dtype == torch.bfloat16 and ops.linear_silu(x, w) is not None
 
 
+class _Tagged(torch.Tensor):
+    pass
+
+
+class _Products(torch.overrides.TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        if func is F.linear:
+            self.seen.append(args[0].shape[0])
+        return func(*args, **(kwargs or {}))
+
+
+@gpu
+def test_subclasses_modes_and_the_compiler_see_the_product():
+    x, w = _operands(2304, 2048, 1024, False)
+    for a, b in ((x.as_subclass(_Tagged), w), (x, w.as_subclass(_Tagged))):
+        for rows in (64, 2304):
+            assert type(ops.linear(a[:rows], b)) is _Tagged
+        assert ops.linear_silu(a, b) is None
+    with _Products() as mode:
+        ops.linear(x[:64], w), ops.linear(x, w)
+    assert mode.seen == [64, 2304]
+    whole = torch.compile(lambda a, b: ops.linear(a, b), backend="eager", fullgraph=True)
+    assert torch.equal(whole(x, w), F.linear(x, w))
+
+
 @gpu
 @pytest.mark.skipif(torch.cuda.device_count() < 2, reason="a device that is not the current one takes two")
 def test_operands_of_another_device_than_the_current_one():
