@@ -124,10 +124,12 @@ class LlamaMLP(nn.Module):
         self._i = cfg.intermediate_size // ctx.world_size
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        act = ops.linear_silu(x, self.gate_up_proj.weight) if self.gate_up_proj.bias is None else None
+        p = self.gate_up_proj
+        plain = ops.only_weights(p, ColumnParallelLinear) and ops.no_global_hooks()
+        act = ops.linear_silu(x, p.weight) if plain and p.bias is None else None
         if act is not None:
             return self.down_proj(act)
-        gate_up = self.gate_up_proj(x)
+        gate_up = p(x)
         gate, up = gate_up.split([self._i, self._i], dim=-1)
         return self.down_proj(ops.silu_mul(gate, up))
 

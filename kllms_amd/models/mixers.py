@@ -271,14 +271,19 @@ class ParallelMixer(nn.Module):
     def cache_spec(self) -> LayerCacheSpec:
         return LayerCacheSpec(kv=self.left.cache_spec(), rec=self.right.cache_spec())
 
-    def rows_step(self, x, h, batch, st: LayerState, w_post, w_next) -> torch.Tensor:
+    def takes_rows(self) -> bool:
+        m = self._modules
+        return (self.rows_ok and ops.only_weights(self, ParallelMixer) and ops.only_weights(m["inp"], FusedInput)
+                and ops.only_weights(m["left"], BlockLocalAttention) and ops.only_weights(m["right"], DecayLinearAttention))
+
+    def rows_step(self, x, h, batch, st: LayerState, w_post, w_next) -> Optional[torch.Tensor]:
         """The sublayer with its residual for single decoded rows: ops.hybrid_parallel_rows."""
-        le, p = self.left.spec, self.inp.parts
+        inp, left, right = (self._modules[n] for n in ("inp", "left", "right"))
+        le, p = left.spec, inp.parts
         at = [p[n][0] for n in ("left.q", "left.k", "left.g", "right.q", "right.k", "right.v", "right.g")]
-        return ops.hybrid_parallel_rows(x, h, self.inp.weight, self.inp.bias, at, self.left.inv_freq, st.k, st.v,
-                                        self.left.o_proj, self.right.decay, st.rec, self.right.norm, self.right.o_proj,
-                                        self.left_out, self.right_out, w_post, w_next, batch, le.heads, le.scale,
-                                        le.mask_size, self.right.eps)
+        return ops.hybrid_parallel_rows(x, h, inp.weight, inp.bias, at, left.inv_freq, st.k, st.v, left.o_proj,
+                                        right.decay, st.rec, right.norm, right.o_proj, self.left_out, self.right_out,
+                                        w_post, w_next, batch, le.heads, le.scale, le.mask_size, right.eps)
 
     def forward(self, h: torch.Tensor, batch, st: LayerState):
         y = self.inp(h)
@@ -339,10 +344,15 @@ class ChannelDeltaMixer(nn.Module):
         sp = self.spec
         return LayerCacheSpec(rec=(sp.heads, sp.dim, sp.vdim), conv=(self.cp, sp.conv - 1))
 
-    def rows_step(self, x, h, batch, st: LayerState, w_post, w_next) -> torch.Tensor:
+    def takes_rows(self) -> bool:
+        return (self.rows_ok and ops.only_weights(self, ChannelDeltaMixer)
+                and ops.only_weights(self._modules["inp"], FusedInput))
+
+    def rows_step(self, x, h, batch, st: LayerState, w_post, w_next) -> Optional[torch.Tensor]:
         """The sublayer with its residual for single decoded rows: ops.hybrid_delta_rows."""
-        at = [self.inp.parts[n][0] for n in ("q", "k", "v", "a1", "g1", "b")]
-        return ops.hybrid_delta_rows(x, h, self.inp.weight, at, self.conv, st.conv, self.a2, self.g2, self.dt_bias,
+        inp = self._modules["inp"]
+        at = [inp.parts[n][0] for n in ("q", "k", "v", "a1", "g1", "b")]
+        return ops.hybrid_delta_rows(x, h, inp.weight, at, self.conv, st.conv, self.a2, self.g2, self.dt_bias,
                                      self.A_log, st.rec, self.norm, self.o_proj, w_post, w_next, batch,
                                      self.spec.kv_heads, self.eps)
 
@@ -388,12 +398,19 @@ class ClampedGLU(nn.Module):
         # sizes of the step of few rows (rows_step)
         self.rows_ok = self._fused and spec.ff % 128 == 0 and hidden % 128 == 0 and hidden <= 8192
 
-    def rows_step(self, x, h, w_post, w_next, eps: float) -> torch.Tensor:
+    def takes_rows(self) -> bool:
+        return (self.rows_ok and ops.only_weights(self, ClampedGLU)
+                and ops.only_weights(self._modules["inp"], FusedInput))
+
+    def rows_step(self, x, h, w_post, w_next, eps: float) -> Optional[torch.Tensor]:
         """The sublayer with its residual for single decoded rows: ops.hybrid_glu_rows."""
-        return ops.hybrid_glu_rows(x, h, self.inp.weight, self.down, w_post, w_next, self.spec.limit, self.spec.alpha, eps)
+        return ops.hybrid_glu_rows(x, h, self._modules["inp"].weight, self.down, w_post, w_next, self.spec.limit,
+                                   self.spec.alpha, eps)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        act = ops.linear_clamped_glu(h, self.inp.weight, self.spec.limit, self.spec.alpha) if self._fused else None
+        act = None
+        if self._fused and ops.only_weights(self.inp, FusedInput) and ops.no_global_hooks():
+            act = ops.linear_clamped_glu(h, self.inp.weight, self.spec.limit, self.spec.alpha)
         if act is not None:
             return ops.linear(act, self.down)
         y = self.inp(h)

@@ -55,21 +55,25 @@ class HybridLayer(nn.Module):
         dtype. Returns the next layer's normed input. rows: a step of single
         decoded rows that hybrid_rows_ok admits."""
         after_mix = self.norm2 if self.mlp is not None else next_norm
-        if rows and self.mix.rows_ok:
-            h = self.mix.rows_step(x, h, batch, st, self.norm1b, after_mix)
+        mix, mlp, done = self.mix, self.mlp, None
+        if rows and type(mix) in (ParallelMixer, ChannelDeltaMixer) and mix.takes_rows():
+            done = mix.rows_step(x, h, batch, st, self.norm1b, after_mix)
+        if done is not None:
+            h = done
         elif self.kind == "parallel":
-            left, right = self.mix(h, batch, st)
-            h = ops.sandwich_residual(x, left, self.norm1b, self.eps, b=right, wa=self.mix.left_out,
-                                      wb=self.mix.right_out, w_next=after_mix, out_dtype=h.dtype)
+            left, right = mix(h, batch, st)
+            h = ops.sandwich_residual(x, left, self.norm1b, self.eps, b=right, wa=mix.left_out,
+                                      wb=mix.right_out, w_next=after_mix, out_dtype=h.dtype)
         else:
-            y = self.mix(h, batch, st)
+            y = mix(h, batch, st)
             h = ops.sandwich_residual(x, y, self.norm1b, self.eps, w_next=after_mix, out_dtype=h.dtype)
-        if self.mlp is not None and rows and self.mlp.rows_ok:
-            h = self.mlp.rows_step(x, h, self.norm2b, next_norm, self.eps)
-        elif self.mlp is not None:
-            y = self.mlp(h)
-            h = ops.sandwich_residual(x, y, self.norm2b, self.eps, w_next=next_norm, out_dtype=h.dtype)
-        return h
+        if mlp is None:
+            return h
+        done = mlp.rows_step(x, h, self.norm2b, next_norm, self.eps) if rows and type(mlp) is ClampedGLU and mlp.takes_rows() else None
+        if done is not None:
+            return done
+        y = mlp(h)
+        return ops.sandwich_residual(x, y, self.norm2b, self.eps, w_next=next_norm, out_dtype=h.dtype)
 
     def checkpoint_map(self, pre: str) -> Dict[str, torch.Tensor]:
         m = {pre + "norm1": self.norm1, pre + "norm1b": self.norm1b}

@@ -282,6 +282,19 @@ def _plain_call(*ts: torch.Tensor) -> bool:
             and not torch.compiler.is_compiling() and not torch._C._len_torch_dispatch_stack())
 
 
+def only_weights(module: torch.nn.Module, kind: type) -> bool:
+    """Whether a call of ``module`` is ``kind``'s forward and nothing else: the class itself, no hooks on it, no forward of
+    the object's own. Asked before a fused call takes a module's weights and passes the module by; hooks on all modules
+    are no_global_hooks()."""
+    d = module.__dict__
+    return type(module) is kind and "forward" not in d and not (
+        d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"])
+
+
+def no_global_hooks() -> bool:
+    return not torch.nn.modules.module._has_any_global_hook()
+
+
 def _try_tiles(x, w, bias, act: int, limit: float = 0.0, alpha: float = 0.0) -> Optional[torch.Tensor]:
     """The product on the tile kernel, where it takes the call (bf16 on the GPU, more than 128 rows, contiguous, sizes that
     its 16-byte accesses and 64-deep stages divide, no gradient or transform to serve) and is the faster one. Subclasses,
@@ -638,13 +651,15 @@ def hybrid_rows_ok(x, h, batch) -> bool:
                 (batch.cu_seqlens, T + 1), (batch.block_tables, batch.block_tables.numel())))
             and all(t.is_contiguous() and t.numel() == T and t.dtype == torch.long
                     for t in (batch.positions, batch.slot_mapping))
-            and not (torch.is_grad_enabled() and (x.requires_grad or h.requires_grad)) and _plain_call(x, h))
+            and not (torch.is_grad_enabled() and (x.requires_grad or h.requires_grad)) and _plain_call(x, h)
+            and no_global_hooks())
 
 
 def hybrid_parallel_rows(x, h, w_in, bias, at, inv_freq, k_cache, v_cache, o_left, decay, state, norm_right, o_right, wa,
                          wb, w_post, w_next, batch, heads, scale, mask_size, eps):
     """x (fp32 stream) += the parallel sublayer of h in place, with cache and state; returns the next normed input. at:
-    columns of left q, k, head gates and right q, k, v, gate in h @ w_in^T + bias."""
+    columns of left q, k, head gates and right q, k, v, gate in h @ w_in^T + bias. None, and nothing done, where the
+    weights do not lie as the kernels read them (contiguous, from 16 bytes on)."""
     return _seq().hybrid_parallel_rows(
         x, h, w_in, bias if bias is not None else _none(h), at, inv_freq, k_cache, v_cache, o_left, decay, state,
         norm_right, o_right, wa, wb, w_post, w_next, batch.positions, batch.slot_mapping, batch.block_tables,
