@@ -1190,16 +1190,16 @@ void attn_diff_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache, 
 }
 
 // seq_steps.hip
-torch::Tensor hybrid_parallel_rows(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, std::vector<int64_t>,
+std::optional<torch::Tensor> hybrid_parallel_rows(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, std::vector<int64_t>,
                                    torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                                    torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                                    torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                                    torch::Tensor, int64_t, double, int64_t, double);
-torch::Tensor hybrid_delta_rows(torch::Tensor, torch::Tensor, torch::Tensor, std::vector<int64_t>, torch::Tensor,
+std::optional<torch::Tensor> hybrid_delta_rows(torch::Tensor, torch::Tensor, torch::Tensor, std::vector<int64_t>, torch::Tensor,
                                 torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                                 torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                                 torch::Tensor, torch::Tensor, int64_t, double);
-torch::Tensor hybrid_glu_rows(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
+std::optional<torch::Tensor> hybrid_glu_rows(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                               double, double, double);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {

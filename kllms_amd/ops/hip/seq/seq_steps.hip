@@ -7,6 +7,7 @@
 #include <hip/hip_bf16.h>
 
 #include <algorithm>
+#include <optional>
 
 extern "C" {
 void seq_launch_sandwich_rows(float*, const float*, int, const float*, int, const float*, const float*, const float*,
@@ -53,10 +54,16 @@ inline void on_16(const Tensor& t, const char* name) {
 inline const __hip_bfloat16* bf(const Tensor& t) { return (const __hip_bfloat16*)t.data_ptr(); }
 inline const __hip_bfloat16* bf(const Tensor& t, int64_t col) { return bf(t) + col; }
 
+// How the kernels here read weights: contiguous and from 16 bytes on. Others are the general sublayers'
+bool lie_whole(std::initializer_list<Tensor> ws) {
+  for (const Tensor& w : ws)
+    if (!w.is_contiguous() || reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) return false;
+  return true;
+}
+
 void check_weight(const Tensor& w, int64_t K, const char* name) {
   TORCH_CHECK(w.dim() == 2 && w.size(1) == K && K % 128 == 0 && w.size(0) % 16 == 0, name, ": [N, K], N % 16, K % 128");
   check(w, at::kBFloat16, w.numel(), name);
-  on_16(w, name);
 }
 
 // x [T, K] (contiguous) by w: fp32 sums [S, T, N]
@@ -84,21 +91,20 @@ struct Rows {
     on_16(h, "h");
     on_16(x, "x");
   }
-  void norm(const Tensor& w, const char* name) const {
-    check(w, at::kFloat, W, name);
-    on_16(w, name);
-  }
+  void norm(const Tensor& w, const char* name) const { check(w, at::kFloat, W, name); }
 };
 
 }  // namespace
 
 // x (fp32 stream, in place) through a parallel sublayer; h = its normed input. y columns: o_lq, o_lk of the softmax
-// branch's q and k, o_lg of its head gates; o_rq, o_rk, o_rv, o_rg of the recurrent branch. Returns the next normed input
-Tensor hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tensor bias, std::vector<int64_t> at, Tensor inv_freq,
+// branch's q and k, o_lg of its head gates; o_rq, o_rk, o_rv, o_rg of the recurrent branch. Returns the next normed input,
+// or nothing where the weights lie otherwise than the kernels read them: then nothing has been done
+std::optional<Tensor> hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tensor bias, std::vector<int64_t> at, Tensor inv_freq,
                             Tensor k_cache, Tensor v_cache, Tensor o_left, Tensor decay, Tensor state, Tensor norm_right,
                             Tensor o_right, Tensor wa, Tensor wb, Tensor w_post, Tensor w_next, Tensor positions,
                             Tensor slots, Tensor tables, Tensor lens, Tensor state_slots, Tensor cu, Tensor seg_start,
                             int64_t heads, double scale, int64_t mask_size, double eps) {
+  if (!lie_whole({w_in, o_left, o_right, wa, wb, w_post, w_next})) return std::nullopt;
   const Rows r(x, h);
   const int T = r.T, W = r.W;
   check_weight(w_in, W, "w_in");
@@ -170,10 +176,11 @@ Tensor hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tensor bias, std::v
 }
 
 // The same of a gated-delta-rule sublayer. at: columns of q, k, v, of the two low-rank inputs and of the write strengths
-Tensor hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::vector<int64_t> at, Tensor conv, Tensor conv_state, Tensor a2,
+std::optional<Tensor> hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::vector<int64_t> at, Tensor conv, Tensor conv_state, Tensor a2,
                          Tensor g2, Tensor dt_bias, Tensor a_log, Tensor state, Tensor norm, Tensor w_out, Tensor w_post,
                          Tensor w_next, Tensor state_slots, Tensor cu, Tensor seg_start, Tensor token_seg,
                          int64_t kv_heads, double eps) {
+  if (!lie_whole({w_in, w_out, w_post, w_next})) return std::nullopt;
   const Rows r(x, h);
   const int T = r.T, W = r.W;
   check_weight(w_in, W, "w_in");
@@ -183,8 +190,6 @@ Tensor hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::vector<int64_t> a
   check(state, at::kFloat, state.numel(), "state");
   TORCH_CHECK(G >= 1 && H % G == 0 && D <= 256, "heads and key size of the recurrence");
   TORCH_CHECK(a2.dim() == 2 && g2.dim() == 2 && a2.size(0) == (int64_t)H * D && g2.size(0) == (int64_t)H * V);
-  check(a2, at::kBFloat16, a2.numel(), "a2");
-  check(g2, at::kBFloat16, g2.numel(), "g2");
   const int64_t sizes[6] = {(int64_t)G * D, (int64_t)G * D, (int64_t)H * V, a2.size(1), g2.size(1), H};
   TORCH_CHECK(at.size() == 6, "six column ranges");
   for (int i = 0; i < 6; ++i) TORCH_CHECK(at[i] >= 0 && at[i] % 8 == 0 && at[i] + sizes[i] <= N, "columns of w_in");
@@ -232,8 +237,9 @@ Tensor hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::vector<int64_t> a
 }
 
 // The same of a clamped gated-linear-unit sublayer, w_in = [gate; up]
-Tensor hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_down, Tensor w_post, Tensor w_next, double limit,
+std::optional<Tensor> hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_down, Tensor w_post, Tensor w_next, double limit,
                        double alpha, double eps) {
+  if (!lie_whole({w_in, w_down, w_post, w_next})) return std::nullopt;
   const Rows r(x, h);
   check_weight(w_in, r.W, "w_in");
   const int N = w_in.size(0);

@@ -47,6 +47,21 @@ def test_rows_steps_against_the_general_sublayers(rows):
         assert (a - b).norm() <= 0.025 * b.norm()
 
 
+def test_rows_steps_with_weights_that_lie_otherwise():
+    """Transposed, or off 16 bytes: what the general sublayers' products take."""
+    eng = LLMEngine(EngineConfig(model="mid-zutalix", device=DEV, seed=0, use_hip_graphs=False, max_kv_blocks=256,
+                                 max_state_slots=40, enable_prefix_caching=False, eos_token_id=-1))
+    ref = _logits(eng, 5, True)
+    for i, layer in enumerate(eng.model.layers):
+        for m in (layer.mix, layer.mlp):
+            if m is not None:
+                w = m.inp.weight.data
+                m.inp.weight.data = (w.t().contiguous().t() if i % 2 == 0
+                                     else w.new_empty(w.numel() + 1)[1:].view_as(w).copy_(w))
+    for a, b in zip(_logits(eng, 5, True), ref):
+        assert (a - b).norm() <= 0.025 * b.norm()      # as above
+
+
 def test_residual_of_split_sums_against_float64():
     C, W, T = ops._seq(), 384, 5
     g = torch.Generator(device=DEV).manual_seed(0)
