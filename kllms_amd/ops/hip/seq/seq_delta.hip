@@ -14,6 +14,10 @@
 //   delta_chunk   a wave per (chunk, head): L and M, the inverse T of I + L by substitution, T beta (P k) and T beta V
 //   delta_scan    a wave per (segment, head, 16 value columns): chunk after chunk, 52 matrix instructions each
 //
+// The matrix instructions add up all 16 tokens, with a zero in L, T or M for those to come, and zero times infinity is
+// NaN: from a token on whose k, write strength or decay is not finite, and in a column from a v on that is not, operands
+// are zeros, and the rows become NaN. So nothing reaches an earlier token, as token by token.
+//
 // Everything stays in fp32 (v_mfma_f32_16x16x4_f32), and no decay is divided by or taken as an exponential of a
 // difference: the P are running products of factors in (0, 1], as token by token. The state's registers are both
 // the B operand of the products and the accumulators of the update: k runs in the order d = 16 m + 4 grp + r.
@@ -21,7 +25,7 @@
 // What bounds them: delta_chunk its records (21 KB a chunk and head: 166 MB in 142 us for 8 x 1000 tokens, 16 heads) and
 // the pairs' sums, delta_scan its matrix instructions, 1700 cycles a chunk, with one wave on a SIMD and two chunks of
 // operands on their way (128 us; 150 with one). Together, us, beside token by token with its pre-pass, 16 heads of 64 x 128:
-// 1 x 100 tokens 38 (47), 1 x 1000 123 (394), 8 x 1000 255 (547), 4 x 2000 322 (850), 64 x 250 of 32 heads of 64 x 64 729 (1158).
+// 1 x 100 tokens 40 (47), 1 x 1000 124 (394), 8 x 1000 262 (547), 4 x 2000 333 (850), 64 x 250 of 32 heads of 64 x 64 714 (1158).
 
 #include "seq_common.h"
 
@@ -48,6 +52,24 @@ __device__ __forceinline__ float row_sum16(float v) {   // over 16 lanes, every 
   return v;
 }
 
+// Not 0 where one of the values is infinite or NaN (no comparison that could be taken for granted: x - x is 0 or NaN)
+__device__ __forceinline__ float not_finite(const f32x4& v) {
+  return (v[0] - v[0]) + (v[1] - v[1]) + ((v[2] - v[2]) + (v[3] - v[3]));
+}
+
+// Rows of a result in matrix layout (row 4 grp + r, column col): the first one of each column whose value is not finite, 16: none
+__device__ __forceinline__ int first_odd_row(const f32x4& v, int col) {
+  int first = 16;
+#pragma unroll
+  for (int r = 3; r >= 0; --r) {
+    const unsigned long long odd = __ballot(v[r] - v[r] != 0.0f) >> col;
+#pragma unroll
+    for (int g = 3; g >= 0; --g)
+      if ((odd >> (g * 16)) & 1) first = min(first, g * 4 + r);
+  }
+  return first;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(WAVE) delta_chunk_kernel(
     float* __restrict__ rec, const T* __restrict__ q_in, const T* __restrict__ k_in, const T* __restrict__ v_in,
@@ -71,6 +93,7 @@ __global__ void __launch_bounds__(WAVE) delta_chunk_kernel(
 
   // unit q and k, q by 1 / sqrt(64), decays and write strengths; behind the segment's end k, q and beta 0, decay 1
   const float rate = expf(a_log[h]);
+  int bad = DC_C;                          // first token with a k, decay or write strength that is not finite
   f32x4 dt;
 #pragma unroll
   for (int x = 0; x < 4; ++x) dt[x] = dt_bias[h * DC_D + col * 4 + x];
@@ -101,8 +124,13 @@ __global__ void __launch_bounds__(WAVE) delta_chunk_kernel(
     *reinterpret_cast<f32x4*>(&k[t][col * 4]) = a;
     *reinterpret_cast<f32x4*>(&q[t][col * 4]) = c;
     *reinterpret_cast<f32x4*>(&g[t][col * 4]) = e;
+    const unsigned long long odd = __ballot(not_finite(a) + not_finite(e) != 0.0f);
+    if (odd && bad == DC_C) bad = i * 4 + __builtin_ctzll(odd) / 16;
   }
-  if (lane < DC_C) beta[lane] = lane < n ? sigmoid_exact(ldf(beta_logit + (int64_t)(t0 + lane) * beta_stride + h)) : 0.0f;
+  float strength = 0.0f;
+  if (lane < n && lane < DC_C) strength = sigmoid_exact(ldf(beta_logit + (int64_t)(t0 + lane) * beta_stride + h));
+  if (lane < DC_C) beta[lane] = strength;
+  if (const unsigned long long odd = __ballot(strength - strength != 0.0f)) bad = min(bad, (int)__builtin_ctzll(odd));
   for (int i = lane; i < DC_C * (DC_C + 1); i += WAVE) (&L[0][0])[i] = (&M[0][0])[i] = 0.0f;
   __syncthreads();
 
@@ -168,6 +196,7 @@ __global__ void __launch_bounds__(WAVE) delta_chunk_kernel(
       kk[t] *= p;
       p *= g[t][d];
     }
+    for (int t = bad; t < DC_C; ++t) k[t][d] = 0.0f;
 #pragma unroll
     for (int t = 0; t < DC_C; t += 4)
       *reinterpret_cast<f32x4*>(r0 + DC_K + d * DC_C + t) = f32x4{kk[t], kk[t + 1], kk[t + 2], kk[t + 3]};
@@ -183,16 +212,33 @@ __global__ void __launch_bounds__(WAVE) delta_chunk_kernel(
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ti[kk], k[kk * 4 + grp][m * 16 + col], acc, 0, 0, 0);
+    if (bad < DC_C) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = grp * 4 + r < bad ? acc[r] : NAN;
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) r0[DC_W + (grp * 4 + r) * DC_D + m * 16 + col] = acc[r];
   }
   for (int v0 = 0; v0 < V; v0 += 16) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, x;     // x[kk]: token 4 kk + grp
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       const int s = kk * 4 + grp;
-      const float x = ldf(v_in + (int64_t)(t0 + min(s, n - 1)) * v_stride + h * V + v0 + col);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ti[kk], s < n ? beta[s] * x : 0.0f, acc, 0, 0, 0);
+      const float v = ldf(v_in + (int64_t)(t0 + min(s, n - 1)) * v_stride + h * V + v0 + col);
+      x[kk] = s < n && s < bad ? beta[s] * v : 0.0f;
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ti[kk], x[kk] - x[kk] == 0.0f ? x[kk] : 0.0f, acc, 0, 0, 0);
+    }
+    if (bad < DC_C || __any(not_finite(x) != 0.0f)) {
+      f32x4 y;                               // as rows 4 grp + r: token 4 kk + g is in lane group g's x[kk]
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float a = __shfl(x[0], r * 16 + col), b = __shfl(x[1], r * 16 + col), c = __shfl(x[2], r * 16 + col),
+                    d = __shfl(x[3], r * 16 + col);
+        y[r] = grp == 0 ? a : grp == 1 ? b : grp == 2 ? c : d;
+      }
+      const int first = min(bad, first_odd_row(y, col));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = grp * 4 + r < first ? acc[r] : NAN;
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) r0[DC_U + (int64_t)(grp * 4 + r) * V + v0 + col] = acc[r];
@@ -250,15 +296,23 @@ __global__ void __launch_bounds__(4 * WAVE, 1) delta_scan_kernel(float* __restri
       u[r] = x.u[r] - (ws[0][r] + ws[1][r]);
       out[r] = qs[0][r] + qs[1][r];
     }
+    f32x4 um;                              // what M takes: in time beside the state's chain, which takes u
+#pragma unroll
+    for (int r = 0; r < 4; ++r) um[r] = u[r] - u[r] == 0.0f ? u[r] : 0.0f;
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
       for (int r = 0; r < 4; ++r) S[m][r] *= x.p[m][r];
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {       // s = 4 grp + kk
-      out = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[kk], u[kk], out, 0, 0, 0);
+      out = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[kk], um[kk], out, 0, 0, 0);
 #pragma unroll
       for (int m = 0; m < 4; ++m) S[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[m][kk], u[kk], S[m], 0, 0, 0);
+    }
+    if (__any(not_finite(u) != 0.0f)) {
+      const int first = first_odd_row(u, col);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[r] = grp * 4 + r < first ? out[r] : NAN;
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {

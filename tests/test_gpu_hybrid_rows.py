@@ -119,3 +119,31 @@ def test_delta_rule_by_chunks_against_float64(H, G, V, lens, dtype):
         assert (S - got_state[slots[b]].double().cpu()).abs().max() <= 64 * 2 ** -23 * 8 * size
     for s in set(range(B + 2)) - set(slots.tolist()):
         assert torch.equal(got_state[s].cpu(), state[s])
+
+
+@pytest.mark.parametrize("name,at", [("q", 10), ("k", 0), ("k", 21), ("v", 16), ("v", 29), ("beta", 37), ("a", 32), ("a", 47)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+def test_delta_rule_by_chunks_keeps_later_tokens_out_of_earlier_ones(name, at, value):
+    """A value that is not finite reaches the tokens from its own on, as token by token, and not those before it in its
+    chunk of 16; one of v stays in its column."""
+    D, H, G, V, T = 64, 2, 1, 48, 80
+    g = torch.Generator().manual_seed(at)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    x = {"q": rnd(T, G, D), "k": rnd(T, G, D), "v": rnd(T, H, V), "beta": rnd(T, H), "a": rnd(T, H * D)}
+    dt, a_log, start = rnd(H * D), torch.zeros(H), rnd(1, H, D, V)
+
+    def run(dev, dtype, op):
+        i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+        state = start.to(dev, torch.float32)
+        args = [x[n].to(dev, dtype) for n in ("q", "k", "v", "beta", "a")]
+        o = op(*args, dt.to(dev), a_log.to(dev), state, i32(0), i32(0, T), i32(5))
+        return o.double().cpu().view(T, H, V), state.double().cpu()
+
+    clean, _ = run(DEV, torch.float32, ops.gated_delta_rule)
+    x[name][at].view(-1)[1] = value
+    o, state = run(DEV, torch.float32, ops.gated_delta_rule)
+    assert torch.equal(o[:at], clean[:at])
+    ref, ref_state = run("cpu", torch.float32, ops.gated_delta_rule)
+    assert torch.equal(o.isfinite(), ref.isfinite()) and torch.equal(state.isfinite(), ref_state.isfinite())
+    ok = ref.isfinite()
+    assert ((o - ref)[ok].abs() <= 64 * 2 ** -23 * 8 * 8).all()      # sums of 64 products, as above; values below 8
