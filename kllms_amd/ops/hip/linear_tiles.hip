@@ -11,8 +11,8 @@
 // compute units. A tile of 32 * MJ rows takes LT_COST[MJ] us for 64 stages of K, so the rows of a tile are those
 // whose rounds cost least (4096 rows of N = K = 4096: 256 tiles of 256; 3100 rows: 224 of 224, 77 us, 88 with 256).
 // Of long K the tiles of a last round that would leave half of the units idle are shared out over it. The library has
-// the advantage where its tiles fill the last round too, and at middling K on few tiles, which it splits and makes
-// smaller; linear_tiles_rows has the lines. Measured, us of the library (with its activation's launch) and here:
+// the advantage where its tiles fill the last round too, and on few tiles, which it splits over K and makes
+// smaller; linear_tiles_ahead has the lines. Measured, us of the library (with its activation's launch) and here:
 //   N 4096, K 14336       1170 rows 146, 130    1600 rows 330, 168     3100 rows 334, 280    11700 rows 1303, 1019
 //   N 4096, K 4096        3100 rows  82,  77    4700 rows 139, 125    11700 rows  442,  276
 //   silu N 14336, K 4096   300 rows  81,  72     777 rows 189, 167    3100 rows 698, 557    11700 rows 2099, 2011
@@ -123,9 +123,55 @@ static const int LT_COST[9] = {0, 0, 44, 49, 60, 68, 77, 88, 97};
 #define LT_UNITS (8 * TP_SLOTS)
 #define LT_LONG 8192       // K from which the last round's tiles may be shared out
 
+// Whether the product is faster here than in the library; rows: of w. The library's time goes by tiles of 256 x 256 in
+// rounds of the compute units as well: by how many rounds they make, and how much of them they fill. Few tiles it splits
+// over K and makes smaller; its third and fifth round cost as much as the next one, and from K 10240 on its short rounds
+// do; where w's rows are no multiple of 256, all do. Gated products save the activation's launch and pass here.
+//
+// Measured in graphs at 78000 sizes, K 64 to 28672, N 256 to 18944, 129 to 12000 rows, us of the library and here:
+//   plain, one round     K 4096, N 4096: 1196 rows 49, 51   2021 66, 64   3493 95, 97     K 2048, N 8192: 593 rows 28, 31
+//     1969 52, 66       K 2048, N 3072: 1755 rows 27, 25    K 14336, N 4096: 521 rows 112, 82    2455 233, 235    3974 304, 345
+//   plain, two           K 2048, N 3072: 5922 rows 83, 70   8984 95, 98    K 4096, N 14336: 1545 rows 159, 167
+//   plain, three, four   K 4096, N 4096: 9513 rows 345, 251    11949 448, 286    N 14336: 3179 rows 431, 298    3702 434, 354
+//   plain, ragged        N 3216, K 2048: 1206 rows 27, 23   4021 59, 46    7710 134, 89
+//   gated                K 1024, N 512: 306 rows 11, 12   2513 17, 13    K 2048, N 1024: 357 rows 14, 19   1124 23, 20
+//     K 4096, N 2048: 339 rows 27, 47   1203 55, 50    K 7168, N 4096: 711 rows 92, 100   3207 315, 313
+// Of the sizes, 35 % of the plain and 71 % of the gated products are taken: 1.18 and 1.27 times as fast in the mean, 13
+// and 4 % of them slower by 3 % or more. (With a least number of results alone, stepped at K 2048, 4096 and 8192, 55 and
+// 84 % were: 1.11 and 1.21, 25 and 11 % slower.)
+static bool linear_tiles_ahead(int64_t M, int64_t rows, int64_t K, bool gated) {
+  // the weights' stream bounds few rows, and one tile a column does not keep it up
+  if (M <= 128) return false;
+  const int64_t tiles = (M + 255) / 256 * ((rows + 255) / 256), rounds = (tiles + LT_UNITS - 1) / LT_UNITS;
+  const double fill = (double)tiles / (rounds * LT_UNITS);
+  const bool ragged = rows % 256 != 0;
+  if (K >= 10240) {                                // the last round shared out over K here
+    if (rounds == 1)
+      return fill > (M >= 700 || K >= 16384 ? 0.08 : 0.1) && fill <= (M >= 700 || gated || K >= 16384 ? 0.5 : 0.25);
+    if (rounds == 2 || (rounds == 4 && !gated)) return fill <= 0.92;
+    return gated || rounds <= 5;
+  }
+  if (gated) {
+    if (K <= 1280) return rounds > 1 || fill > 0.05;
+    if (K <= 2304) return rounds > 1 || fill > 0.2;
+    if (rounds == 1) return K <= 4608 ? fill > (M >= 700 ? 0.3 : 0.4) : M >= 1500 && fill > 0.3 && fill <= 0.84;
+    return rounds > 2 || ragged || fill <= (K <= 4608 ? 0.84 : 0.92);
+  }
+  if (ragged && K >= 256) {
+    if (rounds == 1) return K <= 1280 ? fill > 0.25 : K <= 4608 ? fill > 0.5 : K < 8192 && fill > 0.7 && fill <= 0.84;
+    return K <= 4608 || rounds <= (K < 8192 ? 5 : 4);
+  }
+  if (K <= 640) return K >= 256 && (rounds > 1 || fill > 0.25) && fill <= 0.92;
+  if (rounds == 1) return M >= (K < 8192 ? 1500 : 4000) && fill >= (K <= 2048 ? 0.25 : K < 8192 ? 0.4 : 0.5) && fill <= 0.7;
+  if (rounds == 2) return fill <= 0.7;
+  if (rounds == 4) return fill <= 0.84;
+  return (rounds == 3 || rounds == 5) && fill <= (K >= 2048 ? 0.99 : 0.84);
+}
+
 // MJ of the tiles of a product, + 16 where the last round is shared out over K, or 0 where the library's is the better
 // one; N: columns of the result
 extern "C" int linear_tiles_rows(int64_t M, int64_t N, int64_t K, int act) {
+  if (!linear_tiles_ahead(M, act ? 2 * N : N, K, act != 0)) return 0;
   const int64_t n_tiles = act ? (N + 127) / 128 : (N + 255) / 256, stages = K / TP_K;
   int best = 8;
   double least = 1e30;
@@ -141,25 +187,6 @@ extern "C" int linear_tiles_rows(int64_t M, int64_t N, int64_t K, int act) {
     const double shared = unit / TP_SLOTS * round + round / (shares < stages / 8 ? shares : stages / 8) + 10 + 0.75 * mj * shares;
     if (shared < least) least = shared, best = mj + 16;
   }
-  // few rows: the weights' stream bounds, which one tile a column does not keep up
-  if (M <= 128) return 0;
-  // Few tiles: the library splits K and makes its tiles smaller. Where both are even (us of the library and here, in a
-  // graph), by results: at K 2048 from 3.5 million (N 2048: 11 and 19 at 300 rows, 20.0 and 20.3 at 1200, 29.8 and 24.5 at
-  // 2600; N 8720: 25 and 28 at 300, 30.7 and 30.6 at 465, 48 and 43 at 1200), at K 4096 from 6.5 (N 4096: 26 and 54 at 300, 48 and 53
-  // at 1200, 58.5 and 56.8 at 1600). Longer K is shared out (N 4096, K 14336: 63 and 63 at 256 rows, 78 and 67 at
-  // 300, 325 and 176 at 1600; N 2048, K 8192: 34 and 36 at 400, 44 and 42 at 600). Gated products save the activation's
-  // launch and pass: ahead from the start at K 2048 (16384 rows of w: 31 and 29 at 140), later at K 4096 (28672: 67 and 69
-  // at 140, 80 and 71 at 200)
-  const int64_t outputs = M * N * (act ? 2 : 1);
-  const int64_t least_outputs = K >= LT_LONG ? 1200000 : act ? (K > 2048 ? 5000000 : 0) : K > 2048 ? 6500000 : 3500000;
-  if (outputs < least_outputs) return 0;
-  // 256 x 256 tiles that fill one or two rounds to 0.92 and more: the library's are 4 to 10 % faster (N 4096, K 4096 /
-  // 14336: 3710 rows 94 and 99 / 309 and 339, 8100 rows 184 and 200 / 619 and 699). Below it is not, on balance (2700
-  // rows 78 and 77 / 249 and 253; 4200 rows 140 and 125 / 730 and 377; 7600 rows 179 and 195 / 1009 and 696), and
-  // of three rounds and more, or where a tile is short, it is seldom (12000 rows 450 and 297 / 1359 and 1067)
-  const int64_t tiles = (M + 255) / 256 * n_tiles;
-  const int64_t last = tiles % LT_UNITS ? tiles % LT_UNITS : LT_UNITS;
-  if (!act && K > 2048 && tiles <= 2 * LT_UNITS && last * 25 >= LT_UNITS * 23) return 0;
   return best;
 }
 

@@ -208,6 +208,11 @@ def test_rule_of_the_tiles():
     assert rows(300, 2048, 2048, 0) == 0 and rows(1200, 4096, 4096, 0) == 0
     assert rows(300, 14336, 4096, 1) == 5                      # 224 tiles of 150 rows
     assert rows(11700, 4096, 14336, 0) == 8                    # 736 tiles in three rounds
+    # plain products whose tiles fill the library's rounds, few tiles, gated products of a few workgroups; w's rows no
+    # multiple of 256, where the library has no such tiles
+    assert rows(6000, 8192, 2048, 0) == 0 and rows(700, 6144, 5120, 0) == 0 and rows(129, 128, 2048, 1) == 0
+    assert rows(7700, 3328, 2048, 0) == 0 and rows(7700, 3216, 2048, 0) and rows(7700, 3320, 2048, 0)
+    assert rows(1170, 4096, 8192, 0) == 0 and rows(4400, 2048, 8192, 0) == 5
     for M in range(1, 13000, 97):
         for N, K, act in ((4096, 4096, 0), (3216, 2048, 0), (14336, 4096, 1)):
             assert rows(M, N, K, act) in (0, 2, 3, 4, 5, 6, 7, 8)      # K below 8192: never shared
