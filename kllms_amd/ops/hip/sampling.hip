@@ -298,7 +298,18 @@ __device__ __forceinline__ bool slice_list(SliceToken* __restrict__ list, int ca
   return listed <= cap;
 }
 
-extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
+// Whether a truncated row's slices list their tokens. A top-k that the lists are long enough for lies in them for sure, and
+// in a few rows the try is made for one of a quarter more (the top-k 50 of 8 rows of 128256, whose lists hold 48), and for
+// what a mask leaves of a row (2 masked rows of 50257, top-p 0.9: 61 us without, 30 with; 16 of 128256: 130 and 118).
+// Elsewhere top-p's nucleus is seldom in the lists, and rows whose lists end before their cut pay 3 to 8 % for the try.
+__device__ __forceinline__ bool lists_pay(int rows, int V, int top_k, int cap, bool masked) {
+  const bool few = (int64_t)rows * V <= 1 << 22;
+  return (masked && few) || (top_k > 0 && top_k <= (few ? cap + cap / 4 : cap));
+}
+
+// LISTS: what a call without lists need not carry (its truncated rows are 1 us faster so)
+template <bool LISTS>
+__global__ void __launch_bounds__(PT) sample_part_kernel(
     SlicePart* __restrict__ parts,        // [B, slices]
     const float* __restrict__ logits,     // [B, V]
     const float* __restrict__ temperatures, const float* __restrict__ top_ps,
@@ -314,10 +325,7 @@ extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
   const uint32_t* mrow = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
   const bool cuts = temp != 0.0f && truncates(top_ps[b], top_ks[b], V);
   SlicePart p = slice_part<PT>(row, mrow, temp, cuts, draw_base(seeds[b], steps[b]), lo, hi);
-  // a top-k that the lists are long enough for lies in them for sure; where only a share of the mass is asked for the
-  // try costs nothing as long as the chip is not full (16 masked rows of 128256, top-p 0.9: 127 us without, 33 with; 120
-  // flat rows whose nucleus is half of the vocabulary: 292 and 312)
-  if (cuts && lists && ((top_ks[b] > 0 && top_ks[b] <= cap) || (int64_t)gridDim.y * V <= 1 << 22)) {
+  if (LISTS && cuts && lists_pay(gridDim.y, V, top_ks[b], cap, mask != nullptr)) {
     __shared__ float top;
     // without an allowed token there is nothing to list; a max or a sum that is not finite leaves the row to the sweeps
     if (threadIdx.x == 0) top = p.arg < 0 ? -INFINITY : p.sum - p.sum == 0.0f ? p.max : INFINITY;
@@ -339,7 +347,7 @@ extern "C" __global__ void __launch_bounds__(PT) sample_part_kernel(
 
 
 // WHOLE: a short row's only launch, one slice of all its tokens
-template <bool WHOLE>
+template <bool WHOLE, bool LISTS>
 __global__ void __launch_bounds__(NT) sample_final_kernel(
     int64_t* __restrict__ out_tokens,     // [B]
     float* __restrict__ out_logprobs,     // [B]
@@ -392,7 +400,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) a = min(a, __shfl_xor(a, off));
     const unsigned long long w = wave_max_u64(p.best);
-    if (lists && temp != 0.0f && truncates(top_p, top_k, V)) {
+    if (LISTS && temp != 0.0f && truncates(top_p, top_k, V)) {
       const float edge = wave_reduce_max(p.edge);
       const float lmass = wave_reduce_sum(p.listed == 0 ? 0.0f : p.mass * (p.max == M ? 1.0f : __expf((p.max - M) * inv_t)));
       int total = p.listed;
@@ -558,12 +566,11 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   // bins that the slices' lists hold whole; their tokens then stand in for the row if the cut lies there
   int whole = 0;
   bool hope = false;
-  if constexpr (!WHOLE)
-    if (lists) {
-      const float deep = -sx_of(sh_edge, inv_t, smax) - 1e-3f;
-      whole = deep > 0.0f ? min((int)(deep * (SBINS / SRANGE)), SBINS) : 0;      // NaN: none
-      hope = (unsigned)sh_total >= need_cnt || sh_mass * 1.001f >= top_p * sh_ssum;
-    }
+  if constexpr (LISTS) {
+    const float deep = -sx_of(sh_edge, inv_t, smax) - 1e-3f;
+    whole = deep > 0.0f ? min((int)(deep * (SBINS / SRANGE)), SBINS) : 0;      // NaN: none
+    hope = (unsigned)sh_total >= need_cnt || sh_mass * 1.001f >= top_p * sh_ssum;
+  }
   if (tid == 0) sh_best = (unsigned long long)NO_KEY << 32;
   // where the cut is behind the lists, the sweeps over bins that those hold whole are left out
   const int after = whole >= SMID ? 2 : whole >= SNEAR ? 1 : 0;
@@ -797,12 +804,16 @@ extern "C" int sample_slices(int B, int V) {
 
 // Tokens of a slice's list, or 0: no lists. They cost two more walks over the truncated rows by all workgroups and save
 // the walks of sample_final, one workgroup a row. Worth it on long rows (120 rows of 32000 with top-p and top-k: 33 us
-// without, 37 with; 30 of 50257, masked: 37 and 31) and on as many as leave sample_final the slower part (120 rows of
-// 128256 73 and 61, 250 of 152064 105 and 107; masked, half of them truncated: 171 and 110). Nor have slices lists whose
-// threads would count more than 255 tokens
+// without, 37 with; 30 of 50257, masked: 36 and 31) and in calls of so many rows as leave compute units idle there. us without
+// and with, truncated throughout, masked in brackets: 50257 tokens, 60 rows 37, 33 (39, 35)   120 rows 43, 45 (49, 51)
+// 250 rows 50, 56 (61, 77); 128256 tokens, 120 rows 74, 62 (103, 87)   180 rows 82, 78 (116, 115)   250 rows 90, 91 (127, 141).
+// Larger calls of which a part is not truncated would still gain (250 rows of 128256, half of them 104, 79), but no kernel
+// knows that for less than it gives: a count of the truncated rows in each slice is 2 to 4 us. One or two rows of a
+// shorter vocabulary sample_final is as fast with by itself, unless a mask is on them (2 x 50257: 22, 24 (27, 25); 2 x
+// 128256: 34, 23). Nor have slices lists whose threads would count more than 255 tokens
 static int sample_cap(int B, int V, int n, bool masked) {
-  const int64_t most = masked ? 1 << 26 : 1 << 25;
-  return n > 0 && V > 32768 && (int64_t)B * V <= most && (V + n - 1) / n <= 255 * PT ? SLIST / n : 0;
+  return n > 0 && V > 32768 && B <= (V > 65536 ? 192 : 96) && (masked || (int64_t)B * V >= 120000) &&
+         (V + n - 1) / n <= 255 * PT ? SLIST / n : 0;
 }
 
 // words of 8 bytes that a call needs for its slices, and for their lists
@@ -826,9 +837,10 @@ extern "C" void launch_sample(int64_t* tokens, float* logprobs, void* parts, con
     const float* x = logits + (int64_t)b * V;
     const uint32_t* m = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
     if (n > 0)
-      hipLaunchKernelGGL(sample_part_kernel, dim3(n, rows), dim3(PT), 0, stream, p, x, temps + b, top_ps + b,
-                         top_ks + b, seeds + b, steps + b, m, lists, cap, V, slice);
-    hipLaunchKernelGGL(n > 0 ? sample_final_kernel<false> : sample_final_kernel<true>, dim3(rows), dim3(NT), 0, stream,
+      hipLaunchKernelGGL(lists ? sample_part_kernel<true> : sample_part_kernel<false>, dim3(n, rows), dim3(PT), 0, stream, p, x,
+                         temps + b, top_ps + b, top_ks + b, seeds + b, steps + b, m, lists, cap, V, slice);
+    hipLaunchKernelGGL((n == 0 ? sample_final_kernel<true, false> : lists ? sample_final_kernel<false, true> : sample_final_kernel<false, false>),
+                       dim3(rows), dim3(NT), 0, stream,
                        tokens + b, logprobs + b, (const SlicePart*)p, n, (const SliceToken*)lists, cap, x, temps + b, top_ps + b, top_ks + b,
                        seeds + b, steps + b, m, V, dbg ? dbg + (int64_t)b * 16 : nullptr);
   }

@@ -215,6 +215,11 @@ def test_cut_inside_and_behind_the_slices_lists(B, V, near):
         assert x[t] >= x[kept[-1]] and key[t] >= key[kept].max() - max(1e-3, 4e-7 * V)
 
 
+@pytest.mark.parametrize("B,V", [(2, 50257), (3, 50257), (96, 65536), (97, 65536), (192, 65537), (193, 65537)])
+def test_calls_on_either_side_of_the_lines_for_lists(B, V):
+    test_cut_inside_and_behind_the_slices_lists(B, V, 49)
+
+
 @pytest.mark.parametrize("ulps", [1, 2, 16])
 def test_top_p_a_few_ulps_below_one(ulps):
     """Rows whose allowed tokens all lie in the slices' lists: whether fp32 sums of their masses reach top_p of the whole
