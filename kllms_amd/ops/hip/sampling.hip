@@ -307,8 +307,9 @@ __device__ __forceinline__ bool lists_pay(int rows, int V, int top_k, int cap, b
   return (masked && few) || (top_k > 0 && top_k <= (few ? cap + cap / 4 : cap));
 }
 
-// LISTS: what a call without lists need not carry (its truncated rows are 1 us faster so)
-template <bool LISTS>
+// LISTS 0: what a call without lists need not carry (its truncated rows are 1 us faster so); 2: only if one row in eight of
+// the call is not truncated, which every wave counts for itself
+template <int LISTS>
 __global__ void __launch_bounds__(PT) sample_part_kernel(
     SlicePart* __restrict__ parts,        // [B, slices]
     const float* __restrict__ logits,     // [B, V]
@@ -325,7 +326,18 @@ __global__ void __launch_bounds__(PT) sample_part_kernel(
   const uint32_t* mrow = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
   const bool cuts = temp != 0.0f && truncates(top_ps[b], top_ks[b], V);
   SlicePart p = slice_part<PT>(row, mrow, temp, cuts, draw_base(seeds[b], steps[b]), lo, hi);
-  if (LISTS && cuts && lists_pay(gridDim.y, V, top_ks[b], cap, mask != nullptr)) {
+  bool pays = LISTS && cuts && lists_pay(gridDim.y, V, top_ks[b], cap, mask != nullptr);
+  if (LISTS == 2 && pays) {
+    const int rows = gridDim.y, lane = threadIdx.x & 63;
+    int n = 0;
+#pragma unroll 4
+    for (int r0 = 0; r0 < rows; r0 += WAVE) {
+      const int r = min(r0 + lane, rows - 1);
+      n += __popcll(__ballot(r0 + lane < rows && temperatures[r] != 0.0f && truncates(top_ps[r], top_ks[r], V)));
+    }
+    pays = n * 8 <= rows * 7;
+  }
+  if (pays) {
     __shared__ float top;
     // without an allowed token there is nothing to list; a max or a sum that is not finite leaves the row to the sweeps
     if (threadIdx.x == 0) top = p.arg < 0 ? -INFINITY : p.sum - p.sum == 0.0f ? p.max : INFINITY;
@@ -804,17 +816,20 @@ extern "C" int sample_slices(int B, int V) {
 
 // Tokens of a slice's list, or 0: no lists. They cost two more walks over the truncated rows by all workgroups and save
 // the walks of sample_final, one workgroup a row. Worth it on long rows (120 rows of 32000 with top-p and top-k: 33 us
-// without, 37 with; 30 of 50257, masked: 36 and 31) and in calls of so many rows as leave compute units idle there. us without
-// and with, truncated throughout, masked in brackets: 50257 tokens, 60 rows 37, 33 (39, 35)   120 rows 43, 45 (49, 51)
-// 250 rows 50, 56 (61, 77); 128256 tokens, 120 rows 74, 62 (103, 87)   180 rows 82, 78 (116, 115)   250 rows 90, 91 (127, 141).
-// Larger calls of which a part is not truncated would still gain (250 rows of 128256, half of them 104, 79), but no kernel
-// knows that for less than it gives: a count of the truncated rows in each slice is 2 to 4 us. One or two rows of a
-// shorter vocabulary sample_final is as fast with by itself, unless a mask is on them (2 x 50257: 22, 24 (27, 25); 2 x
-// 128256: 34, 23). Nor have slices lists whose threads would count more than 255 tokens
+// without, 37 with; 30 of 50257, masked: 36 and 31) and on as many as leave compute units idle there (sample_asks). One or
+// two rows of a shorter vocabulary sample_final is as fast with by itself, unless a mask is on them (2 x 50257: 22, 24,
+// masked 27, 25; 2 x 128256: 34, 23). Nor have slices lists whose threads would count more than 255 tokens
 static int sample_cap(int B, int V, int n, bool masked) {
-  return n > 0 && V > 32768 && B <= (V > 65536 ? 192 : 96) && (masked || (int64_t)B * V >= 120000) &&
+  const int64_t tokens = (int64_t)B * V;
+  return n > 0 && V > 32768 && tokens <= (masked ? 1 << 26 : 1 << 25) && (masked || tokens >= 120000) &&
          (V + n - 1) / n <= 255 * PT ? SLIST / n : 0;
 }
+
+// Calls of more rows list only if some are not truncated. us of calls that are truncated throughout, with top-p 0.95 and
+// top-k 50, without lists and with, masked in brackets: 50257 tokens, 60 rows 37, 33 (39, 35)   120 rows 43, 45 (49, 51)   250 rows
+// 50, 56 (61, 77), 54 (67) having asked; 128256 tokens, 120 rows 74, 62 (103, 87)   180 rows 82, 78 (116, 115)   250 rows 90, 91
+// (127, 141), 93 (131) having asked. Half of 250 rows: 55, 45 (65, 56), 47 (58) and 104, 79 (144, 97), 82 (102).
+static bool sample_asks(int B, int V) { return B > (V > 65536 ? 192 : 128); }
 
 // words of 8 bytes that a call needs for its slices, and for their lists
 extern "C" int64_t sample_room(int B, int V, int masked) {
@@ -837,7 +852,7 @@ extern "C" void launch_sample(int64_t* tokens, float* logprobs, void* parts, con
     const float* x = logits + (int64_t)b * V;
     const uint32_t* m = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
     if (n > 0)
-      hipLaunchKernelGGL(lists ? sample_part_kernel<true> : sample_part_kernel<false>, dim3(n, rows), dim3(PT), 0, stream, p, x,
+      hipLaunchKernelGGL(!lists ? sample_part_kernel<0> : sample_asks(B, V) ? sample_part_kernel<2> : sample_part_kernel<1>, dim3(n, rows), dim3(PT), 0, stream, p, x,
                          temps + b, top_ps + b, top_ks + b, seeds + b, steps + b, m, lists, cap, V, slice);
     hipLaunchKernelGGL((n == 0 ? sample_final_kernel<true, false> : lists ? sample_final_kernel<false, true> : sample_final_kernel<false, false>),
                        dim3(rows), dim3(NT), 0, stream,

@@ -215,9 +215,28 @@ def test_cut_inside_and_behind_the_slices_lists(B, V, near):
         assert x[t] >= x[kept[-1]] and key[t] >= key[kept].max() - max(1e-3, 4e-7 * V)
 
 
-@pytest.mark.parametrize("B,V", [(2, 50257), (3, 50257), (96, 65536), (97, 65536), (192, 65537), (193, 65537)])
+@pytest.mark.parametrize("B,V", [(2, 50257), (3, 50257), (128, 65536), (129, 65536), (192, 65537), (193, 65537)])
 def test_calls_on_either_side_of_the_lines_for_lists(B, V):
     test_cut_inside_and_behind_the_slices_lists(B, V, 49)
+
+
+@pytest.mark.parametrize("B,plain", [(129, 15), (129, 16), (129, 17), (300, 37), (300, 38), (300, 300)])
+def test_large_calls_with_rows_that_are_not_truncated(B, plain):
+    """On either side of one row in eight, counted over more rows than a wave has lanes."""
+    V = 32801
+    g = torch.Generator().manual_seed(B + plain)
+    logits = torch.randn(B, V, generator=g) * 2.0
+    top_k = torch.full((B,), 7, dtype=torch.int32)
+    top_k[torch.randperm(B, generator=g)[:plain]] = 0
+    seeds, steps = torch.randint(0, 2**40, (B,), generator=g), torch.randint(0, 99, (B,), generator=g)
+    one = torch.ones(B, device=DEV)
+    toks, _ = ops.sample(logits.to(DEV), one, one, top_k.to(DEV), seeds.to(DEV), steps.to(DEV), None)
+    for b in range(0, B, 7):
+        x = logits[b].double().numpy()
+        kept = np.argsort(-x, kind="stable")[:int(top_k[b]) or V]
+        key = x + gumbel(int(seeds[b]), int(steps[b]), V)
+        t = int(toks[b])
+        assert x[t] >= x[kept[-1]] and key[t] >= key[kept].max() - max(1e-3, 4e-7 * V)      # as above
 
 
 @pytest.mark.parametrize("ulps", [1, 2, 16])
