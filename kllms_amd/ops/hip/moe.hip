@@ -90,25 +90,40 @@ __global__ void __launch_bounds__(TP_THREADS, 1) moe_product_kernel(
   constexpr int BN = GATEUP ? 128 : 256;           // output columns of a workgroup
   const int n_tiles = (N + BN - 1) / BN;
   // (expert, column tile) pairs in turn to the XCDs, the row tiles of one behind each other
-  const int xcd = blockIdx.x & 7;
-  auto columns_of = [&](int e, int& first) {       // this XCD's column tiles of expert e
-    first = (xcd + 8 - (int)((int64_t)e * n_tiles & 7)) & 7;
-    return first < n_tiles ? (n_tiles - first + 7) / 8 : 0;
+  const int xcd = blockIdx.x & 7, lane = threadIdx.x & 63;
+  auto first_of = [&](int e) { return (xcd + 8 - (int)((int64_t)e * n_tiles & 7)) & 7; };   // this XCD's first column tile of e
+  // its tiles of expert e; a lane each: an expert after the other, 128 of them took 25 us a walk
+  auto tiles_of = [&](int e) {
+    if (e >= E) return 0;
+    const int first = first_of(e);
+    return (first < n_tiles ? (n_tiles - first + 7) / 8 : 0) * ((offsets[e + 1] - offsets[e] + 255) / 256);
   };
-  int first = 0, tiles = 0;
+  auto before_and = [&](int n) {                   // over the wave: the sum up to and with this lane
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(n, off);
+      if (lane >= off) n += o;
+    }
+    return n;
+  };
+  int tiles = 0;
   if (part)
-    for (int e = 0; e < E; ++e) tiles += columns_of(e, first) * ((offsets[e + 1] - offsets[e] + 255) / 256);
+    for (int e0 = 0; e0 < E; e0 += 64) tiles += __builtin_amdgcn_readlane(before_and(tiles_of(e0 + lane)), 63);
   const TileShare sh(blockIdx.x >> 3, tiles, K / TP_K, part, count, xcd);
-  int at = sh.tile, e = 0, begin = 0, end = 0, m_tiles = 0;
-  for (; e < E; ++e) {
-    begin = offsets[e];
-    end = offsets[e + 1];
-    m_tiles = (end - begin + 255) / 256;
-    const int mine = columns_of(e, first) * m_tiles;
-    if (at < mine) break;
-    at -= mine;
+  int at = sh.tile, e = E;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int mine = tiles_of(e0 + lane), sum = before_and(mine), all = __builtin_amdgcn_readlane(sum, 63);
+    if (at >= all) {
+      at -= all;
+      continue;
+    }
+    const int found = (int)__builtin_ctzll(__ballot(at < sum));
+    e = e0 + found;
+    at -= __builtin_amdgcn_readlane(sum - mine, found);
+    break;
   }
   if (e >= E) return;
+  const int begin = offsets[e], end = offsets[e + 1], m_tiles = (end - begin + 255) / 256, first = first_of(e);
   // an expert's rows in even parts: its row tiles keep step, and read W from memory once
   const int rows = (end - begin + m_tiles - 1) / m_tiles;
   const int n0 = (first + at / m_tiles * 8) * BN, m0 = begin + at % m_tiles * rows, m_end = min(end, m0 + rows);

@@ -185,9 +185,13 @@ def test_mixture_products_against_float64(H, I, counts):
 
 
 @pytest.mark.parametrize("H,I,counts", [
-    (256, 1088, [32, 33, 64, 65, 80, 81, 96, 97, 128, 129]),      # one column tile; down shares its 17 stages in two
-    (1088, 2112, [20, 130, 0, 150, 260, 385, 1]),                 # five column tiles, the last of 64; shares of 33 stages
-    (2048, 2112, [700, 600, 600, 600, 600, 600, 600, 600]),       # 42 tiles an XCD: a whole round, and ten in three shares
+    (256, 1088, [32, 33, 64, 65, 80, 81, 96, 97, 128, 129]),      # one column tile, 17 stages
+    (1088, 2112, [20, 130, 0, 150, 260, 385, 1]),                 # five column tiles, the last of 64; 33 stages
+    (256, 2624, [32, 33, 64, 65, 80, 81, 96, 97, 128, 129]),      # the same with shares: 41 stages in four
+    (1088, 2624, [20, 130, 0, 150, 260, 385, 1]),
+    (2048, 2624, [700, 600, 600, 600, 600, 600, 600, 600]),       # 42 tiles an XCD: a whole round, and ten in three shares
+    (320, 64, [1] * 60 + [0] * 3 + [2, 300, 0, 1] + [3] * 63),    # experts of more than one walk of a wave's lanes
+    (64, 2624, [5] * 64 + [0] * 64 + [9]),
 ])
 def test_mixture_products_at_the_edges_of_row_tiles(H, I, counts):
     # expert e gets counts[e] + counts[e - 1] rows: 64, 128, 160, 192 and 256 a tile, and parts of two and three tiles
