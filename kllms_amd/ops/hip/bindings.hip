@@ -299,7 +299,7 @@ extern "C" int launch_moe_gateup(void* act, const void* x, const void* w, const 
                                  const void* zeros, int S, int E, int IN, int K, hipStream_t stream);
 extern "C" int launch_moe_down(void* y, const void* act, const void* w, const int* offsets, float* part, int* count,
                                int S, int E, int H, int IN, hipStream_t stream);
-extern "C" int64_t moe_down_room(int S, int E, int H, int* zeros);
+extern "C" int64_t moe_down_room(int S, int E, int H, int IN, int* zeros);
 extern "C" void launch_moe_sort(int* ids, int* pos, int* offsets, const int64_t* topi, int P, int k, int E,
                                 hipStream_t stream);
 extern "C" void launch_moe_combine(void* out, const void* y, const float* weights, const int* pos, int T, int k,
@@ -346,7 +346,7 @@ void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor
   auto out = on_16_bytes(y);
   // partial sums and counters of tiles that are worked on in shares
   int zeros = 0;
-  const int64_t room = moe_down_room(act.size(0), E, H, &zeros);
+  const int64_t room = moe_down_room(act.size(0), E, H, IN, &zeros);
   torch::Tensor part, count;
   if (room) {
     part = torch::empty({room}, act.options().dtype(torch::kFloat));

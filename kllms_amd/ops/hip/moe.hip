@@ -252,12 +252,14 @@ extern "C" int launch_moe_down(void* y, const void* act, const void* w, const in
   return moe_product<false>(y, act, w, nullptr, nullptr, offsets, part, count, S, E, H, IN, stream);
 }
 
-// Whether the last round's tiles may be shared out: with many rounds it is not worth the
-// room. Then floats of ``part`` and zeros of ``count``.
-extern "C" int64_t moe_down_room(int S, int E, int H, int* zeros) {
+// Whether the last round's tiles may be shared out: with many rounds it is not worth the room, and of short K their sums'
+// way through memory takes longer than it saves. us without and with, the zeros' launch included, 8 experts, top 2, 320 rows:
+// width 4096, K 1024 23, 31   2048 46, 51   2560 55, 52   4096 102, 83; width 2048 18, 23   34, 33   54, 40   69, 50. Then floats
+// of ``part`` and zeros of ``count``.
+extern "C" int64_t moe_down_room(int S, int E, int H, int IN, int* zeros) {
   *zeros = 8 * TP_SLOTS;
   const int64_t tiles = (int64_t)(S / 256 + E) * ((H + 255) / 256);
-  return tiles > 8 * 8 * TP_SLOTS ? 0 : (int64_t)8 * TP_SLOTS * TP_SUMS;
+  return tiles > 8 * 8 * TP_SLOTS || IN < 2560 ? 0 : (int64_t)8 * TP_SLOTS * TP_SUMS;
 }
 
 extern "C" void launch_moe_sort(int* ids, int* pos, int* offsets, const int64_t* topi, int P, int k, int E,
