@@ -340,11 +340,14 @@ __global__ void __launch_bounds__(4 * WAVE, 1) delta_scan_kernel(float* __restri
     for (int r = 0; r < 4; ++r) sp[(int64_t)(m * 16 + grp * 4 + r) * V] = S[m][r];
 }
 
-// floats of rec, or 0 where the token-by-token form is taken: other sizes, short segments (below 64 tokens on average the
-// token form may end sooner: 8 x 32 tokens, 16 heads of 64 x 128 25 us, 35 here; 8 x 100 66 and
-// 54), and steps whose records would take more than 1 GB
+// floats of rec, or 0 where the token-by-token form is taken: other sizes, steps whose records would take more than 1 GB, and
+// short segments, where it ends sooner: below 64 tokens on average (8 x 32 tokens, 16 heads of 64 x 128, 25 us and 35 here; 8 x
+// 100 66 and 54), 96 of wide values, whose records are longer (one of 64, 8 heads of 64 x 256, 31 and 37; of 100 45 and 43),
+// and 128 where segments and heads fill the chip without chunks (64 segments, 32 heads of 64 x 128: of 64 tokens 307 and
+// 331, of 100 483 and 511, of 128 612 and 593)
 extern "C" int64_t seq_delta_chunk_room(int T_, int B, int H, int G, int D, int V) {
-  if (D != DC_D || V % 16 != 0 || V < 16 || T_ < 64 * (int64_t)B || H > 65535) return 0;
+  const int least = (int64_t)B * H * V >= 1 << 18 ? 128 : V > 128 ? 96 : 64;
+  if (D != DC_D || V % 16 != 0 || V < 16 || T_ < least * (int64_t)B || H > 65535) return 0;
   const int64_t n = ((int64_t)T_ / DC_C + B) * H * (DC_U + DC_C * V);
   return n <= (int64_t)1 << 28 ? n : 0;
 }
