@@ -26,6 +26,7 @@ void seq_launch_gated_delta_rule(float*, const void*, const void*, const void*, 
                                  const float*, const float*, float*, float*, float*, float*, float*, float*,
                                  const int*, const int*, const int*, int, int, int, int, int, int, int, int, int,
                                  int, int, int, float*, hipStream_t);
+void seq_launch_gated_act(void*, const void*, const void*, int64_t, int, int, float, float, float, int, hipStream_t);
 // few-row products and paged decode attention (ops/hip/linear_rows.hip, attn_decode.hip, also part of kllms_amd._C)
 void launch_linear_rows(void*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
                         int, int, float, float, hipStream_t);
@@ -236,6 +237,11 @@ std::optional<Tensor> hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::ve
   return out;
 }
 
+// Whether the gated product of T rows is the few-row kernel's, which has the activation in it, or the library's and a pass
+// behind it. us of the one and the other by T, w_in of 16384 x 2048: 16 18, 21   64 22, 22   65 30, 23   128 31, 25; 28672 x 4096: 16
+// 52, 70   32 55, 58   40 62, 57   128 75, 61; 22016 x 4096: 16 48, 58   32 52, 47; 57344 x 8192: 1 194, 180   16 192, 185
+static bool glu_on_rows(int T, int64_t n) { return T <= 16 ? n < 1 << 28 : T <= 32 ? n < 1 << 27 : T <= 64 && n <= 1 << 26; }
+
 // The same of a clamped gated-linear-unit sublayer, w_in = [gate; up]
 std::optional<Tensor> hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_down, Tensor w_post, Tensor w_next, double limit,
                        double alpha, double eps) {
@@ -249,8 +255,13 @@ std::optional<Tensor> hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_
   r.norm(w_post, "w_post"); r.norm(w_next, "w_next");
   auto st = cur_stream();
   auto act = torch::empty({r.T, N / 2}, h.options());
-  launch_linear_rows(act.data_ptr(), bf(h), bf(w_in), nullptr, r.T, N, r.W, r.W, ROWS_CLAMPED, 1, (float)limit,
-                     (float)alpha, st);
+  if (glu_on_rows(r.T, w_in.numel())) {
+    launch_linear_rows(act.data_ptr(), bf(h), bf(w_in), nullptr, r.T, N, r.W, r.W, ROWS_CLAMPED, 1, (float)limit,
+                       (float)alpha, st);
+  } else {
+    const Tensor y = at::linear(h, w_in);
+    seq_launch_gated_act(act.data_ptr(), y.data_ptr(), bf(y, N / 2), r.T, N / 2, N, (float)limit, (float)alpha, 1.0f, 0, st);
+  }
   const Tensor p = part(act, w_down, r.T, st);
   auto out = torch::empty_like(h);
   seq_launch_sandwich_rows(x.data_ptr<float>(), p.data_ptr<float>(), p.size(0), nullptr, 0, nullptr, nullptr,

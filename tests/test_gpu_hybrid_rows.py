@@ -62,6 +62,26 @@ def test_rows_steps_with_weights_that_lie_otherwise():
         assert (a - b).norm() <= 0.025 * b.norm()      # as above
 
 
+@pytest.mark.parametrize("T", [1, 64, 65, 128])
+def test_gated_sublayer_against_the_general_one(T):
+    """On the few-row product with the activation in it, and above 64 rows on the library's and a pass."""
+    W, ff = 384, 640
+    g = torch.Generator(device=DEV).manual_seed(T)
+    h = torch.randn(T, W, generator=g, device=DEV).bfloat16()
+    x = torch.randn(T, W, generator=g, device=DEV)
+    w_in = (torch.randn(2 * ff, W, generator=g, device=DEV) * 0.1).bfloat16()
+    w_down = (torch.randn(W, ff, generator=g, device=DEV) * 0.05).bfloat16()
+    post, nxt = (torch.rand(W, generator=g, device=DEV) + 0.5 for _ in range(2))
+    ref = x.clone()
+    y = torch.nn.functional.linear(h, w_in)
+    y = torch.nn.functional.linear(ops.clamped_glu(y[:, :ff], y[:, ff:], 2.0, 1.5), w_down)
+    out = ops.sandwich_residual(ref, y, post, 1e-6, w_next=nxt, out_dtype=torch.bfloat16)
+    got = ops.hybrid_glu_rows(x, h, w_in, w_down, post, nxt, 2.0, 1.5, 1e-6)
+    # the one rounds gate, up and y to bf16 (2^-9 each), the other the activation alone; rows of a normal size
+    assert (x - ref).abs().max() <= 5e-2 and (got.float() - out.float()).abs().max() <= 8e-2
+    assert ((x - ref).norm(dim=1) <= 1e-2 * ref.norm(dim=1)).all()
+
+
 def test_residual_of_split_sums_against_float64():
     C, W, T = ops._seq(), 384, 5
     g = torch.Generator(device=DEV).manual_seed(0)
