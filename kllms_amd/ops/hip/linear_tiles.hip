@@ -14,7 +14,7 @@
 // the advantage where its tiles fill the last round too, and on few tiles, which it splits over K and makes
 // smaller; linear_tiles_ahead has the lines. Measured, us of the library (with its activation's launch) and here:
 //   N 4096, K 14336       1170 rows 146, 130    1600 rows 330, 168     3100 rows 334, 280    11700 rows 1303, 1019
-//   N 4096, K 4096        3100 rows  82,  77    4700 rows 139, 125    11700 rows  442,  276
+//   N 4096, K 4096        4700 rows 139, 125    11700 rows  442,  276
 //   silu N 14336, K 4096   300 rows  81,  72     777 rows 189, 167    3100 rows 698, 557    11700 rows 2099, 2011
 //   silu N 8192, K 2048    300 rows  36,  32     777 rows  61,  51    4700 rows 347, 253     7777 rows  454,  403
 //   N 8720, K 2048        1200 rows  48,  43    3300 rows 138, 107     7777 rows 240, 220
