@@ -54,15 +54,21 @@ class MixtralMoE(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         T, H = x.shape
-        router_logits = self.gate(x).float()                       # [T, E]
-        probs = torch.softmax(router_logits, dim=-1)
-        topw, topi = torch.topk(probs, self.k, dim=-1)             # [T, k]
-        topw = topw / topw.sum(dim=-1, keepdim=True)
+        routed = None
+        if self.gate.bias is None and ops.only_weights(self.gate, nn.Linear) and ops.no_global_hooks():
+            routed = ops.router_top(x, self.gate.weight, self.k, T > 8 * self.E)
+        if routed is not None:
+            topw, topi = routed[:2]                                # [T, k]
+        else:
+            router_logits = self.gate(x).float()                   # [T, E]
+            probs = torch.softmax(router_logits, dim=-1)
+            topw, topi = torch.topk(probs, self.k, dim=-1)
+            topw = topw / topw.sum(dim=-1, keepdim=True)
 
         if T <= 8 * self.E:
             out = self._forward_dense(x, topw, topi)
         elif x.is_cuda:
-            out = self._forward_grouped_hip(x, topw, topi)
+            out = self._forward_grouped_hip(x, topw, topi, *(routed[2:] if routed else ()))
         else:
             out = self._forward_grouped(x, topw, topi)
         return self.ctx.all_reduce(out)
@@ -83,16 +89,19 @@ class MixtralMoE(nn.Module):
         w.scatter_(0, topi.t().long(), topw.t().float())
         return (ye.float() * w.unsqueeze(-1)).sum(dim=0).to(x.dtype)
 
-    def _forward_grouped_hip(self, x: torch.Tensor, topw: torch.Tensor, topi: torch.Tensor) -> torch.Tensor:
-        """Prefill-shape path on GPU, four launches (ops/hip/moe.hip) without a
-        host round trip: pairs sorted by expert, gate/up GEMM with fused
-        silu*mul, down GEMM, and the weighted sum of each token's rows."""
+    def _forward_grouped_hip(self, x: torch.Tensor, topw: torch.Tensor, topi: torch.Tensor, ids=None, pos=None,
+                             offsets=None, cleared=None) -> torch.Tensor:
+        """Prefill-shape path on GPU, three launches (ops/hip/moe.hip) behind the
+        router's two, without a host round trip: gate/up GEMM with fused silu*mul,
+        down GEMM, and the weighted sum of each token's rows. The pairs are sorted
+        here where the router's kernel did not take the call."""
         T, H = x.shape
-        ids, pos, offsets = ops.moe_sort(topi, self.E)
+        if ids is None:
+            ids, pos, offsets = ops.moe_sort(topi, self.E)
         act = torch.empty(T * self.k, self.I, device=x.device, dtype=x.dtype)
         y = torch.empty(T * self.k, H, device=x.device, dtype=x.dtype)
         ops.moe_gateup(act, x, self.w_gate_up, ids, offsets, x)     # every sorted place has a token: no zero rows
-        ops.moe_down(y, act, self.w_down, offsets)
+        ops.moe_down(y, act, self.w_down, offsets, cleared)
         return ops.moe_combine_rows(y, topw, pos)
 
     def _forward_grouped(self, x: torch.Tensor, topw: torch.Tensor, topi: torch.Tensor) -> torch.Tensor:

@@ -399,9 +399,22 @@ def moe_down(
     act: torch.Tensor,
     w_down: torch.Tensor,
     offsets: torch.Tensor,
+    cleared: Optional[torch.Tensor] = None,
 ) -> None:
-    """Grouped MoE down GEMM in sorted-row space (see moe_gateup)."""
-    _hip_or_raise().moe_down(y, act, w_down, offsets)
+    """Grouped MoE down GEMM in sorted-row space (see moe_gateup). ``cleared``: the counters that router_top gives, used up
+    by the call."""
+    _hip_or_raise().moe_down(y, act, w_down, offsets, cleared)
+
+
+def router_top(x: torch.Tensor, gate: torch.Tensor, k: int, places: bool):
+    """Softmax routing of x [T, H] by gate [E, H]: (weights [T, k] fp32 that sum to one, experts [T, k] int32), and with
+    ``places`` the (ids, pos, offsets) of moe_sort and counters for moe_down behind them. None where the kernel does not
+    take the call (up to 32 experts and 8 choices, bf16 on the GPU, H a multiple of 64) or where a subclass, a function
+    mode, a transform, a gradient or the compiler looks on."""
+    if (x.is_cuda and not torch.compiler.is_compiling() and type(x) in _PLAIN and type(gate) in _PLAIN
+            and not torch._C._len_torch_function_stack() and not _force_torch()):
+        return _hip_or_raise().moe_route_try(x, gate, k, places)
+    return None
 
 
 def moe_sort(topi: torch.Tensor, experts: int):

@@ -302,6 +302,11 @@ extern "C" int launch_moe_down(void* y, const void* act, const void* w, const in
 extern "C" int64_t moe_down_room(int S, int E, int H, int IN, int* zeros);
 extern "C" void launch_moe_sort(int* ids, int* pos, int* offsets, const int64_t* topi, int P, int k, int E,
                                 hipStream_t stream);
+extern "C" int moe_route_groups(int T);
+extern "C" void launch_moe_route(int* topi, float* topw, int* rank, int* counts, const void* x, const void* gate, int T, int H,
+                                 int64_t x_stride, int E, int k, hipStream_t stream);
+extern "C" void launch_moe_place(int* ids, int* pos, int* offsets, int* zeros, int n_zeros, const int* topi, const int* rank,
+                                 const int* counts, int T, int k, int E, hipStream_t stream);
 extern "C" void launch_moe_combine(void* out, const void* y, const float* weights, const int* pos, int T, int k,
                                    int H, hipStream_t stream);
 
@@ -332,7 +337,10 @@ void moe_gateup(torch::Tensor act, torch::Tensor x, torch::Tensor w,
   if (!out.is_same(act)) act.copy_(out);
 }
 
-void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor offsets) {
+#define MOE_DOWN_COUNTERS 256
+
+// cleared: MOE_DOWN_COUNTERS int32 zeros that this call uses up, or nothing: it makes its own
+void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor offsets, std::optional<torch::Tensor> cleared) {
   CHECK_BF16_CONTIG(y); CHECK_BF16_CONTIG(act); CHECK_BF16_CONTIG(w);
   const int E = w.size(0);
   const int H = w.size(1);
@@ -350,7 +358,13 @@ void moe_down(torch::Tensor y, torch::Tensor act, torch::Tensor w, torch::Tensor
   torch::Tensor part, count;
   if (room) {
     part = torch::empty({room}, act.options().dtype(torch::kFloat));
-    count = torch::zeros({zeros}, act.options().dtype(torch::kInt));
+    if (cleared) {
+      TORCH_CHECK(cleared->is_cuda() && cleared->scalar_type() == at::kInt && cleared->is_contiguous() &&
+                      cleared->numel() >= zeros, "moe_down: counters");
+      count = *cleared;
+    } else {
+      count = torch::zeros({zeros}, act.options().dtype(torch::kInt));
+    }
   }
   TORCH_CHECK(launch_moe_down(out.data_ptr(), act.data_ptr(), w.data_ptr(), offsets.data_ptr<int>(),
                               room ? part.data_ptr<float>() : nullptr, room ? count.data_ptr<int>() : nullptr, (int)act.size(0), E, H, IN,
@@ -451,6 +465,34 @@ std::vector<torch::Tensor> moe_sort(torch::Tensor topi, int64_t E) {
   launch_moe_sort(ids.data_ptr<int>(), pos.data_ptr<int>(), offsets.data_ptr<int>(), topi.data_ptr<int64_t>(), P,
                   k > 0 ? k : 1, (int)E, cur_stream());
   return {ids, pos, offsets};
+}
+
+// The k experts of each row of x by the router's weights gate [E, H] and their shares (moe_route_kernel), and where
+// ``places`` asks for it what moe_sort gives for them: (topw [T, k] fp32, topi [T, k] int32), then (ids, pos, offsets,
+// counters for moe_down). Nothing where the kernel does not take the call, or where more than its values is wanted.
+std::optional<std::vector<torch::Tensor>> moe_route_try(torch::Tensor x, torch::Tensor gate, int64_t k, bool places) {
+  if (x.dim() != 2 || gate.dim() != 2 || !x.is_cuda() || x.device() != gate.device() || x.scalar_type() != at::kBFloat16 ||
+      gate.scalar_type() != at::kBFloat16 || !plain_values(x) || !plain_values(gate) || torch::jit::tracer::isTracing() ||
+      at::autocast::is_autocast_enabled(at::kCUDA))
+    return std::nullopt;
+  const int64_t T = x.size(0), H = x.size(1), E = gate.size(0);
+  if (T < 1 || T * k >= 1LL << 31 || H < 64 || H % 64 || H >= 1 << 24 || gate.size(1) != H || E < 1 || E > 32 || k < 1 || k > 8 || k > E ||
+      x.stride(1) != 1 || !rows_aligned(x) || !gate.is_contiguous() || reinterpret_cast<uintptr_t>(gate.data_ptr()) % 16)
+    return std::nullopt;
+  const c10::DeviceGuard device(x.device());
+  const int groups = moe_route_groups((int)T);
+  auto i32 = x.options().dtype(torch::kInt);
+  auto topw = torch::empty({T, k}, x.options().dtype(torch::kFloat)), topi = torch::empty({T, k}, i32);
+  auto rank = torch::empty({T * k}, i32), counts = torch::empty({groups, E}, i32);
+  launch_moe_route(topi.data_ptr<int>(), topw.data_ptr<float>(), rank.data_ptr<int>(), counts.data_ptr<int>(), x.data_ptr(),
+                   gate.data_ptr(), (int)T, (int)H, x.stride(0), (int)E, (int)k, cur_stream());
+  if (!places) return std::vector<torch::Tensor>{topw, topi};
+  auto ids = torch::empty({T * k}, i32), pos = torch::empty({T, k}, i32), offsets = torch::empty({E + 1}, i32);
+  auto cleared = torch::empty({MOE_DOWN_COUNTERS}, i32);
+  launch_moe_place(ids.data_ptr<int>(), pos.data_ptr<int>(), offsets.data_ptr<int>(), cleared.data_ptr<int>(),
+                   MOE_DOWN_COUNTERS, topi.data_ptr<int>(), rank.data_ptr<int>(), counts.data_ptr<int>(), (int)T, (int)k, (int)E,
+                   cur_stream());
+  return std::vector<torch::Tensor>{topw, topi, ids, pos, offsets, cleared};
 }
 
 torch::Tensor moe_combine(torch::Tensor y, torch::Tensor weights, torch::Tensor pos) {
@@ -653,7 +695,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_tiles_pick", &linear_tiles_pick);
   m.def("linear_tiles_try", &linear_tiles_try);
   m.def("moe_gateup", &moe_gateup);
-  m.def("moe_down", &moe_down);
+  m.def("moe_down", &moe_down, py::arg("y"), py::arg("act"), py::arg("w"), py::arg("offsets"),
+        py::arg("cleared") = std::nullopt);
+  m.def("moe_route_try", &moe_route_try);
   m.def("moe_sort", &moe_sort);
   m.def("moe_combine", &moe_combine);
   m.def("ipc_allreduce_create", &ipc_allreduce_create);

@@ -1,6 +1,8 @@
 // Grouped mixture-of-experts products for gfx950 (prefill shapes):
 //
-//   moe_sort      (token, choice) pairs grouped by expert, without the host
+//   moe_route     the router: logits, softmax, the top choices and their weights, in one launch
+//   moe_place     the pairs' places grouped by expert, from the counts that moe_route leaves
+//   moe_sort      (token, choice) pairs grouped by expert, without the host, for choices made elsewhere
 //   moe_gateup    act[s, :] = silu(x[tok(s)] Wg[e]^T) * (x[tok(s)] Wu[e]^T)
 //   moe_down      y[s, :]   = act[s] Wd[e]^T
 //   moe_combine   out[t, :] = sum over choices j of w[t, j] y[pos(t, j)], in fp32
@@ -22,8 +24,8 @@
 //   width 4096, experts of 14336   300 rows  356 + 184 (406 + 328)    1024 rows  551 + 343 (730 + 406)
 //                                 2048 rows  896 + 471 (1175 + 812)
 //   width 4096, experts of 7168   6000 rows  1117 + 566: 1260 TFLOP/s (1394 + 847)
-// The layer with its routing at 65 / 150 / 300 / 600 / 1024 / 2048 / 6000 rows, experts of 14336: 582 / 582 / 605 /
-// 666 / 949 / 1431 / 3623 us (741 / 760 / 787 / 907 / 1131 / 1935 / 4622).
+// The layer with a router of seven launches at 65 / 150 / 300 / 600 / 1024 / 2048 / 6000 rows, experts of 14336: 582 / 582 /
+// 605 / 666 / 949 / 1431 / 3623 us (741 / 760 / 787 / 907 / 1131 / 1935 / 4622); moe_route has what it is now.
 
 #include "tile_product.h"
 
@@ -207,6 +209,191 @@ __global__ void __launch_bounds__(64 * SORT_WAVES) moe_sort_kernel(int* __restri
   }
 }
 
+// The router of a mixture layer: z = x gate^T rounded to bf16, as the layer's own product gives it, p = softmax(z) in 32
+// bits, the k largest (of equal ones the lowest expert, as torch takes them; NaN before all) and their shares of their
+// sum. For moe_place: each pair's rank among the group's earlier pairs of its expert, and the group's counts.
+//
+// A workgroup takes 16 rows, one tile of the matrix cores, and its 16 waves share K, so that a row's loads are all in
+// flight at once: with 100 rows the chain of a launch and one trip to memory is the bound, with thousands the stream of
+// x. Seven launches of torch's before (product, conversion, softmax, selection of 18 to 24 us, sorting, sum, quotient) and
+// moe_sort's single workgroup. us of the layer, before and now, 8 experts, top 2: 80 rows of width 2048 and experts of
+// 8192 226, 187; 300 rows 246, 201; 6000 rows 1133, 1061; width 4096 and experts of 7168, 780 rows 426, 385; of 14336,
+// 2048 rows 1401, 1348.
+#define ROUTE_ROWS 16
+#define ROUTE_WAVES 16
+#define ROUTE_EXPERTS 32
+#define ROUTE_TOP 8
+
+template <int NT>                        // tiles of 16 experts
+__global__ void __launch_bounds__(64 * ROUTE_WAVES) moe_route_kernel(
+    int* __restrict__ topi, float* __restrict__ topw, int* __restrict__ rank, int* __restrict__ counts,
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ gate, int T, int H, int64_t x_stride, int E, int k) {
+  constexpr int DEEP = 4;
+  __shared__ float sums[ROUTE_WAVES][ROUTE_ROWS][NT * 16];
+  __shared__ int chosen[ROUTE_ROWS * ROUTE_TOP];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, grp = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int t0 = blockIdx.x * ROUTE_ROWS;
+  // 32 contiguous bytes of a row for each lane group, the same order of k in both operands
+  const char* xr = (const char*)(x + (int64_t)min(t0 + col, T - 1) * x_stride) + grp * 32;
+  const char* gr[NT];
+  f32x4 acc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    gr[n] = (const char*)(gate + (int64_t)min(n * 16 + col, E - 1) * H) + grp * 32;
+    acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const int steps = H / 64;
+  for (int s0 = wave; s0 < steps; s0 += ROUTE_WAVES * DEEP) {
+    bf16x8_mfma a[DEEP][2], b[DEEP][NT][2];
+#pragma unroll
+    for (int u = 0; u < DEEP; ++u) {
+      const int64_t at = (int64_t)min(s0 + u * ROUTE_WAVES, steps - 1) * 128;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        a[u][h] = *reinterpret_cast<const bf16x8_mfma*>(xr + at + h * 16);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) b[u][n][h] = *reinterpret_cast<const bf16x8_mfma*>(gr[n] + at + h * 16);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < DEEP; ++u) {
+      if (s0 + u * ROUTE_WAVES >= steps) break;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][h], b[u][n][h], acc[n], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sums[wave][grp * 4 + r][n * 16 + col] = acc[n][r];
+  __syncthreads();
+  if (tid < ROUTE_ROWS * 16) {           // 16 lanes a row, experts col, col + 16, ..
+    const int row = tid >> 4, t = t0 + row;
+    float p[NT], m = -INFINITY, sum = 0.0f;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      float z = 0.0f;
+#pragma unroll
+      for (int w = 0; w < ROUTE_WAVES; ++w) z += sums[w][row][n * 16 + col];
+      p[n] = n * 16 + col < E ? bf16_to_f32(f32_to_bf16(z)) : -INFINITY;
+      m = fmaxf(m, p[n]);
+    }
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      p[n] = n * 16 + col < E ? expf(p[n] - m) : 0.0f;
+      sum += p[n];
+    }
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    unsigned long long key[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const int e = n * 16 + col;
+      key[n] = e < E ? (unsigned long long)__float_as_uint(p[n] / sum) << 32 | (uint32_t)~e : 0;
+    }
+    float total = 0.0f, mine = 0.0f;
+    int e_mine = -1;
+    for (int j = 0; j < k; ++j) {
+      unsigned long long best = key[0];
+#pragma unroll
+      for (int n = 1; n < NT; ++n) best = key[n] > best ? key[n] : best;
+#pragma unroll
+      for (int off = 8; off > 0; off >>= 1) {
+        const unsigned long long o = __shfl_xor(best, off);
+        best = o > best ? o : best;
+      }
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+        if (key[n] == best) key[n] = 0;
+      const float q = __uint_as_float((uint32_t)(best >> 32));
+      total += q;
+      if (j == col) {
+        mine = q;
+        e_mine = (int)~(uint32_t)best;
+      }
+    }
+    if (col < k) {
+      chosen[row * k + col] = t < T ? e_mine : -1;
+      if (t < T) {
+        topi[(int64_t)t * k + col] = e_mine;
+        topw[(int64_t)t * k + col] = mine / total;
+      }
+    }
+  }
+  __syncthreads();
+  const int pairs = ROUTE_ROWS * k;
+  if (tid < pairs && chosen[tid] >= 0) {
+    const int e = chosen[tid];
+    int n = 0;
+    for (int q = 0; q < tid; ++q) n += chosen[q] == e;
+    rank[(int64_t)t0 * k + tid] = n;
+  } else if (tid >= 512 && tid < 512 + E) {
+    int n = 0;
+    for (int q = 0; q < pairs; ++q) n += chosen[q] == tid - 512;
+    counts[(int64_t)blockIdx.x * E + tid - 512] = n;
+  }
+}
+
+// moe_route's pairs -> offsets, pos and ids as moe_sort gives them: an expert's pairs in their order. A workgroup adds up
+// all groups' counts (6000 rows: 375 groups of 8, read by 256 threads) and places the pairs of 16 groups. ``zeros``: the
+// counters of moe_down's shares, cleared on the way
+#define PLACE_GROUPS 16
+__global__ void __launch_bounds__(256) moe_place_kernel(int* __restrict__ ids, int* __restrict__ pos, int* __restrict__ offsets,
+                                                        int* __restrict__ zeros, int n_zeros, const int* __restrict__ topi,
+                                                        const int* __restrict__ rank, const int* __restrict__ counts, int T,
+                                                        int k, int E) {
+  __shared__ int all[ROUTE_EXPERTS], before[ROUTE_EXPERTS], first[PLACE_GROUPS][ROUTE_EXPERTS];
+  const int tid = threadIdx.x, e = tid % ROUTE_EXPERTS;
+  const int groups = (T + ROUTE_ROWS - 1) / ROUTE_ROWS, g0 = blockIdx.x * PLACE_GROUPS;
+  if (blockIdx.x == 0)
+    for (int i = tid; i < n_zeros; i += 256) zeros[i] = 0;
+  if (tid < ROUTE_EXPERTS) all[tid] = before[tid] = 0;
+  __syncthreads();
+  if (e < E) {
+    int n = 0, n_before = 0;
+#pragma unroll 8
+    for (int g = tid / ROUTE_EXPERTS; g < groups; g += 256 / ROUTE_EXPERTS) {
+      const int c = counts[(int64_t)g * E + e];
+      n += c;
+      if (g < g0) n_before += c;
+    }
+    atomicAdd(&all[e], n);
+    atomicAdd(&before[e], n_before);
+  }
+  __syncthreads();
+  if (tid < ROUTE_EXPERTS) {
+    int upto = all[e];
+#pragma unroll
+    for (int off = 1; off < ROUTE_EXPERTS; off <<= 1) {
+      const int o = __shfl_up(upto, off);
+      if (e >= off) upto += o;
+    }
+    if (blockIdx.x == 0 && e < E) {
+      offsets[e + 1] = upto;
+      if (e == 0) offsets[0] = 0;
+    }
+    int at = upto - all[e] + before[e];
+#pragma unroll
+    for (int i = 0; i < PLACE_GROUPS; ++i) {
+      first[i][e] = at;
+      if (g0 + i < groups && e < E) at += counts[(int64_t)(g0 + i) * E + e];
+    }
+  }
+  __syncthreads();
+  const int64_t p0 = (int64_t)g0 * ROUTE_ROWS * k;
+  const int n = (int)min((int64_t)PLACE_GROUPS * ROUTE_ROWS * k, (int64_t)T * k - p0);
+  for (int i = tid; i < n; i += 256) {
+    const int place = first[i / (ROUTE_ROWS * k)][topi[p0 + i]] + rank[p0 + i];
+    pos[p0 + i] = place;
+    ids[place] = (int)((p0 + i) / k);
+  }
+}
+
 // tokens on the grid's x: y and z stop at 65535, a packed prompt batch does not
 __global__ void __launch_bounds__(256) moe_combine_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ y,
                                                           const float* __restrict__ weights,
@@ -268,6 +455,21 @@ extern "C" void launch_moe_sort(int* ids, int* pos, int* offsets, const int64_t*
   const int waves = E * SORT_WAVES <= room ? SORT_WAVES : room / E;
   hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(64 * SORT_WAVES), waves * E * sizeof(int), stream, ids, pos, offsets, topi,
                      P, k, E, waves);
+}
+
+// E up to ROUTE_EXPERTS, k up to ROUTE_TOP and E, H a multiple of 64, rows on 16 bytes; counts: [ceil(T / 16), E]
+extern "C" int moe_route_groups(int T) { return (T + ROUTE_ROWS - 1) / ROUTE_ROWS; }
+
+extern "C" void launch_moe_route(int* topi, float* topw, int* rank, int* counts, const void* x, const void* gate, int T, int H,
+                                 int64_t x_stride, int E, int k, hipStream_t stream) {
+  hipLaunchKernelGGL(E <= 16 ? moe_route_kernel<1> : moe_route_kernel<2>, dim3(moe_route_groups(T)), dim3(64 * ROUTE_WAVES), 0,
+                     stream, topi, topw, rank, counts, (const bf16_t*)x, (const bf16_t*)gate, T, H, x_stride, E, k);
+}
+
+extern "C" void launch_moe_place(int* ids, int* pos, int* offsets, int* zeros, int n_zeros, const int* topi, const int* rank,
+                                 const int* counts, int T, int k, int E, hipStream_t stream) {
+  hipLaunchKernelGGL(moe_place_kernel, dim3((moe_route_groups(T) + PLACE_GROUPS - 1) / PLACE_GROUPS), dim3(256), 0, stream, ids,
+                     pos, offsets, zeros, n_zeros, topi, rank, counts, T, k, E);
 }
 
 extern "C" void launch_moe_combine(void* out, const void* y, const float* weights, const int* pos, int T, int k,

@@ -1,5 +1,7 @@
 """Causal prefill attention, packed and against the paged cache, against float64 at the edges of its tiles."""
 
+import math
+
 import pytest
 import torch
 
@@ -380,3 +382,70 @@ def test_step_segments_together_matches_row_by_row(rows, monkeypatch):
     monkeypatch.setattr(LlamaForCausalLM, "_planned", planned)
     test_step_segments_matches_row_by_row(rows)
     assert plans[-1] is not None and plans[-1][0] is not None
+
+
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 255, 256, 257, 4113])
+@pytest.mark.parametrize("E,k,H", [(1, 1, 64), (2, 2, 64), (8, 2, 4096), (16, 3, 1088), (17, 8, 4160), (32, 8, 2048)])
+def test_router_against_torch_and_the_sort(T, E, k, H):
+    """Whole-number logits are exact in every order of the sums, so that choices, ties among them (the lowest expert
+    first) and places are compared to the last; the weights are fp32 quotients of exponentials: a few places of 2^-24."""
+    g = torch.Generator().manual_seed(T * 37 + E)
+    x = (torch.rand(T, H, generator=g) < 16 / H).float() * torch.randint(-3, 4, (T, H), generator=g)
+    gate = torch.randint(-1, 2, (E, H), generator=g).float()
+    z = (x @ gate.t()).bfloat16().float()
+    want = torch.sort(-z, dim=1, stable=True).indices[:, :k]
+    p = torch.softmax(z.double(), 1).gather(1, want)
+    if T > 3:
+        x[3] = math.nan
+    wide = torch.zeros(T, H + 8, dtype=torch.bfloat16)     # rows of a wider matrix
+    wide[:, :H] = x
+    topw, topi, ids, pos, offsets, cleared = ops.router_top(wide.to(DEV)[:, :H], gate.bfloat16().to(DEV), k, True)
+    plain = [t for t in range(T) if t != 3 or T <= 3]
+    assert torch.equal(topi.cpu()[plain].long(), want[plain])
+    assert torch.allclose(topw.cpu().double()[plain], (p / p.sum(1, keepdim=True))[plain], rtol=2 ** -20, atol=0)
+    if T > 3:
+        assert topw[3].isnan().all() and sorted(set(topi[3].tolist())) == sorted(topi[3].tolist())
+        assert 0 <= int(topi.min()) and int(topi.max()) < E
+    for a, b in zip((ids, pos, offsets), ops.moe_sort(topi, E)):
+        assert torch.equal(a, b)
+    assert not cleared.any()
+
+
+def test_router_leaves_other_calls_to_torch():
+    x, gate = torch.randn(40, 128, device=DEV).bfloat16(), torch.randn(8, 128, device=DEV).bfloat16()
+    assert ops.router_top(x, gate, 2, False) is not None
+    assert ops.router_top(x.float(), gate.float(), 2, False) is None
+    assert ops.router_top(x, gate, 9, False) is None
+    assert ops.router_top(x[:, :96].contiguous(), gate[:, :96].contiguous(), 2, False) is None
+    assert ops.router_top(x.t()[:40, :], gate, 2, False) is None
+    assert ops.router_top(x, torch.randn(33, 128, device=DEV).bfloat16(), 2, False) is None
+    assert ops.router_top(x, gate.requires_grad_(), 2, False) is None
+    with torch.autocast("cuda", torch.float16):
+        assert ops.router_top(x, gate.detach(), 2, False) is None
+
+
+def test_mixture_layer_with_a_hooked_router():
+    """The layer through the router's kernel and through the module, whose hook must run: the same up to the choices, which
+    whole-number logits make the same."""
+    from kllms_amd.engine.config import ModelArchConfig
+    from kllms_amd.models.mixtral import MixtralMoE
+    from kllms_amd.parallel.tp import ParallelContext
+    cfg = ModelArchConfig(arch="mixtral", vocab_size=64, hidden_size=256, intermediate_size=128, num_layers=1, num_heads=2,
+                          num_kv_heads=1, num_experts=8, num_experts_per_tok=2)
+    g = torch.Generator().manual_seed(5)
+    with torch.device(DEV):
+        moe = MixtralMoE(cfg, ParallelContext(), torch.bfloat16)
+    with torch.no_grad():
+        moe.gate.weight.copy_(torch.randint(-1, 2, moe.gate.weight.shape, generator=g))
+        for p in (moe.w_gate_up, moe.w_down):
+            p.copy_(torch.randn(p.shape, generator=g) * 0.05)
+    for T in (7, 64, 65, 300):
+        x = (torch.randint(-2, 3, (T, 256), generator=g) * (torch.rand(T, 256, generator=g) < 0.05)).bfloat16().to(DEV)
+        got = moe(x)
+        seen = []
+        h = moe.gate.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+        want = moe(x)
+        h.remove()
+        assert seen == [(T, 8)]
+        # weights apart by fp32 rounding, the result rounded to bf16 once (2^-9)
+        assert torch.allclose(got.float(), want.float(), rtol=2 ** -7, atol=1e-4 * float(want.float().abs().max()))
