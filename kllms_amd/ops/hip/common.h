@@ -101,11 +101,6 @@ __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
   return x ^ (x >> 31);
 }
 
-__device__ __forceinline__ float u64_to_uniform(uint64_t h) {
-  // (0, 1]: use top 24 bits
-  return ((float)((h >> 40) + 1)) * (1.0f / 16777217.0f);
-}
-
 #define HIP_CHECK_LAUNCH()                                                     \
   do {                                                                         \
     hipError_t e_ = hipGetLastError();                                         \

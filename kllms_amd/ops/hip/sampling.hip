@@ -9,7 +9,7 @@
 // Why split: one workgroup per row leaves a 120-row batch on 120 of 256 compute
 // units and a 16-row one on 16, and walks the row three times. The draw, not
 // memory, bounds the split form: per 64 tokens the two 64-bit products of the
-// hash, three transcendentals and the compare take about 280 issue cycles, 27 us
+// hash, three transcendentals and the compares take about 230 issue cycles, 22 us
 // for 120 x 128256 tokens on 1024 SIMDs (the logits alone: 61.6 MB, 13 us at the
 // 4.7 TB/s a copy reaches).
 //
@@ -22,7 +22,8 @@
 // further sweeps, and a boundary bin that outgrows the list is refined by rescans of the row.
 //
 // Measured, 128256 tokens a row: 120 rows, half of them with top-p 0.95 and top-k 50, 50 us (79 with sweeps alone, 346 with
-// one workgroup per row walking it three to six times); 8 rows, all truncated, 24 us (52); 16 masked rows 12.2 us.
+// one workgroup per row walking it three to six times); 8 rows, all truncated, 24 us (52). With the draw of slice_part:
+// 43.7 us for the 120 rows, 8.8 us for 16 masked ones.
 //
 // The draw is counter-based: hash(seed, step, token), identical regardless of
 // batch composition and of the slicing. What follows from a sum is so to fp32
@@ -31,6 +32,8 @@
 // token whose share ends within that of top_p may be in at one batch size and out at
 // another). Slices by V alone cost up to 20% (250 rows of 152064: 75 us -> 90).
 // temperature == 0 -> greedy.
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -89,11 +92,40 @@ __device__ __forceinline__ uint64_t draw_base(int64_t seed, int64_t step) {
   return splitmix64((uint64_t)seed * 0x9E3779B97F4A7C15ULL + (uint64_t)step * 0xBF58476D1CE4E5B9ULL);
 }
 
-__device__ __forceinline__ float draw_key(uint64_t base, int tok, float x, float inv_t) {
-  const float u = u64_to_uniform(splitmix64(base ^ (uint64_t)tok));
-  const float gumbel = -__logf(-__logf(u));
-  return x * inv_t + gumbel;
-}
+// splitmix64 of a row's base ^ token, the upper word without its last step, which leaves the 24 bits that are used as they
+// are. What of it is the row's alone is worked out once: the upper half of the first sum has two values, by the carry.
+// In words of 32 bits: a shift of 64 issues at a fraction of the rate
+struct Draw {
+  uint32_t lo, hi;           // of the base, the upper half with the constant added
+  uint32_t far0, far1;       // product of the mixed upper half without and with a carry
+  float inv_t;
+  __device__ __forceinline__ Draw(uint64_t base, float inv)
+      : lo((uint32_t)base), hi((uint32_t)(base >> 32) + 0x9E3779B9u), inv_t(inv) {
+    far0 = (hi ^ (hi >> 30)) * 0x1CE4E5B9u;
+    far1 = ((hi + 1) ^ ((hi + 1) >> 30)) * 0x1CE4E5B9u;
+  }
+  __device__ __forceinline__ uint32_t word(int tok) const {
+    const uint32_t s = (lo ^ (uint32_t)tok) + 0x7F4A7C15u;
+    const bool carry = s < 0x7F4A7C15u;
+    const uint32_t a = s ^ __builtin_amdgcn_alignbit(hi + carry, s, 30);
+    const uint64_t p = (uint64_t)a * 0x1CE4E5B9u;
+    uint32_t ph = (uint32_t)(p >> 32) + a * 0xBF58476Du + (carry ? far1 : far0);
+    const uint32_t pl = (uint32_t)p ^ __builtin_amdgcn_alignbit(ph, (uint32_t)p, 27);
+    ph ^= ph >> 27;
+    return __umulhi(pl, 0x133111EBu) + pl * 0x94D049BBu + ph * 0x133111EBu;
+  }
+  __device__ __forceinline__ float key(int tok, float x) const {
+    const float u = (float)((word(tok) >> 8) + 1) * (1.0f / 16777217.0f);   // (0, 1]
+    const float gumbel = -__logf(-__logf(u));
+    return x * inv_t + gumbel;
+  }
+  // key up to rounding: the logarithms as the hardware has them
+  __device__ __forceinline__ float near(int tok, float x) const {
+    constexpr float LN2 = 0.693147180559945309f;
+    const float u = (float)((word(tok) >> 8) + 1) * (1.0f / 16777217.0f);
+    return __builtin_fmaf(x, inv_t, -LN2 * __builtin_amdgcn_logf(-LN2 * __builtin_amdgcn_logf(u)));
+  }
+};
 
 __device__ __forceinline__ bool truncates(float top_p, int top_k, int V) {
   return (top_p < 1.0f) || (top_k > 0 && top_k < V);
@@ -113,87 +145,206 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
   return v;
 }
 
-// tokens [lo, hi) of a row by a workgroup of THREADS; the result is thread 0's
+// op over the wave's 64 values, in all lanes, without a trip through LDS: all lanes take part
+template <class T, class Op>
+__device__ __forceinline__ T wave_fold(T v, Op op) {
+  auto bits = [](T x) { return __builtin_bit_cast(int, x); };
+  auto back = [](int x) { return __builtin_bit_cast(T, x); };
+  v = op(v, back(__builtin_amdgcn_mov_dpp(bits(v), 0xB1, 0xf, 0xf, false)));    // neighbours
+  v = op(v, back(__builtin_amdgcn_mov_dpp(bits(v), 0x4E, 0xf, 0xf, false)));    // pairs of a quad
+  v = op(v, back(__builtin_amdgcn_mov_dpp(bits(v), 0x141, 0xf, 0xf, false)));   // quads of 8
+  v = op(v, back(__builtin_amdgcn_mov_dpp(bits(v), 0x140, 0xf, 0xf, false)));   // halves of a row of 16
+  const auto rows = __builtin_amdgcn_permlane16_swap((unsigned)bits(v), (unsigned)bits(v), false, false);
+  v = op(back((int)rows[0]), back((int)rows[1]));
+  const auto halves = __builtin_amdgcn_permlane32_swap((unsigned)bits(v), (unsigned)bits(v), false, false);
+  return op(back((int)halves[0]), back((int)halves[1]));
+}
+
+// tokens [lo, hi) of a row by a workgroup of THREADS, lo a multiple of 64; the result is thread 0's. strip: room for the tokens of a masked row
+// that are allowed, PU * 64 a wave, or nullptr.
+//
+// The draw: what bounds a slice is the issue of its arithmetic, and the hash alone is half of that. So a token's key is not
+// worked out to the last bit (two logarithms with their corrections are a third of it); a lane keeps its highest and
+// second highest key up to rounding. The exact key is made for the highest of each lane; where it then is not clear that
+// no lane's second one can win, the wave makes all of its keys. The draw is so the same to the last bit as with all keys.
+// Of a masked row the allowed tokens are packed first, so that waves work on 64 of them at a time, and the mask is read a
+// word for 32 lanes. us with all keys made and now, masked with one token in eight allowed in brackets: 120 rows of 128256
+// 38.9, 29.2 (44.9, 20.4)   16 rows 11.5, 10.0 (12.1, 8.8)   250 rows of 152064 74.5, 56.8 (90.3, 36.6); 120 greedy rows take 17.
 template <int THREADS>
 __device__ __forceinline__ SlicePart slice_part(const float* __restrict__ row, const uint32_t* __restrict__ mrow,
-                                                float temp, bool cuts, uint64_t base, int lo, int hi) {
-  const int tid = threadIdx.x;
+                                                float temp, bool cuts, uint64_t base, int lo, int hi,
+                                                SliceToken* __restrict__ strip) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool draw = temp != 0.0f && !cuts;
   const float inv_t = (temp > 0.0f) ? 1.0f / temp : 0.0f;
 
-  float m = -INFINITY, sum = 0.0f, ssum = 0.0f, best = -INFINITY;
-  int arg = -1, btok = 0;
-  for (int i0 = lo + tid; i0 < hi; i0 += THREADS * PU) {
-    float x[PU];
-    bool ok[PU];
+  float m = -INFINITY, sum = 0.0f, ssum = 0.0f;
+  float first = -INFINITY, second = -INFINITY;     // highest keys
+  int arg = -1, at = -1;
+  const Draw rng(base, inv_t);
+  auto consider = [&](int tok, float x) {          // -inf and NaN change nothing
+    const float v = rng.near(tok, x);
+    if (v > first) at = tok;
+    second = __builtin_amdgcn_fmed3f(second, first, v);
+    first = fmaxf(first, v);
+  };
+  auto higher = [&](float cm) {
+    sum *= exp_from(m, cm);
+    ssum *= m == -INFINITY ? 0.0f : __expf((m - cm) * inv_t);
+    m = cm;
+  };
+  // the wave's allowed tokens among the 64 from i0 + j * THREADS on, for all j: whole words of the mask, the same for all
+  // lanes (lo is a multiple of 64)
+  auto allowed = [&](int i0, auto whole, uint64_t (&votes)[PU]) {
+    const uint32_t* words = mrow + (i0 >> 5);
 #pragma unroll
     for (int j = 0; j < PU; ++j) {
-      const int i = i0 + j * THREADS;
-      ok[j] = i < hi;
-      x[j] = ok[j] ? row[i] : -INFINITY;
+      if constexpr (whole()) {
+        votes[j] = words[j * (THREADS / 32)] | (uint64_t)words[j * (THREADS / 32) + 1] << 32;
+      } else {
+        const int n = max(min(hi - (i0 + j * THREADS), 64), 0);
+        votes[j] = n == 0 ? 0 : (words[j * (THREADS / 32)] | (n > 32 ? (uint64_t)words[j * (THREADS / 32) + 1] << 32 : 0)) & ~0ull >> (64 - n);
+      }
+    }
+  };
+  // a wave's lanes stay together: 64 tokens from i0 on, and from each THREADS behind
+  auto round = [&](int i0, auto whole) {
+    float x[PU];
+    const float* from = row + i0;
+#pragma unroll
+    for (int j = 0; j < PU; ++j) x[j] = from[whole() ? j * THREADS + lane : min(j * THREADS + lane, hi - 1 - i0)];
+    uint64_t votes[PU];
+    if (mrow) allowed(i0, whole, votes);
+    if (mrow && strip) {
+      SliceToken* mine = strip + wave * (PU * WAVE);
+      int n = 0;
+#pragma unroll
+      for (int j = 0; j < PU; ++j) {
+        if (__builtin_amdgcn_inverse_ballot_w64(votes[j]))
+          mine[n + __builtin_amdgcn_mbcnt_hi((uint32_t)(votes[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)votes[j], 0))] =
+              SliceToken{x[j], i0 + j * THREADS + lane};
+        n += (int)__popcll(votes[j]);
+      }
+      // the strip is this wave's own: in-order LDS, only the compiler is held
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (int e0 = 0; e0 < n; e0 += WAVE) {
+        const SliceToken t = mine[min(e0 + lane, n - 1)];
+        const float v = e0 + lane < n ? t.x : -INFINITY;
+        if (v > m) {
+          higher(v);
+          arg = t.tok;
+        }
+        sum += exp_from(v, m);
+        if (cuts && v != -INFINITY) ssum += __expf((v - m) * inv_t);
+        if (draw) consider(t.tok, v);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      return;
     }
     if (mrow) {
 #pragma unroll
-      for (int j = 0; j < PU; ++j) {
-        const int i = i0 + j * THREADS;
-        if (ok[j]) ok[j] = (mrow[i >> 5] >> (i & 31)) & 1;
-        if (!ok[j]) x[j] = -INFINITY;
-      }
+      for (int j = 0; j < PU; ++j) x[j] = __builtin_amdgcn_inverse_ballot_w64(votes[j]) ? x[j] : -INFINITY;
+    } else if (!whole()) {
+#pragma unroll
+      for (int j = 0; j < PU; ++j) x[j] = i0 + j * THREADS + lane < hi ? x[j] : -INFINITY;
     }
     float cm = x[0];
 #pragma unroll
     for (int j = 1; j < PU; ++j) cm = fmaxf(cm, x[j]);
     if (cm > m) {
-      sum *= exp_from(m, cm);
-      ssum *= m == -INFINITY ? 0.0f : __expf((m - cm) * inv_t);
-      m = cm;
+      higher(cm);
 #pragma unroll
       for (int j = PU - 1; j >= 0; --j)
-        if (x[j] == cm) arg = i0 + j * THREADS;
+        if (x[j] == cm) arg = i0 + j * THREADS + lane;
     }
+    const float near = m == -INFINITY ? 0.0f : m;  // -inf adds nothing, also before a finite token
 #pragma unroll
-    for (int j = 0; j < PU; ++j) sum += exp_from(x[j], m);
+    for (int j = 0; j < PU; ++j) sum += __expf(x[j] - near);
     if (cuts) {
 #pragma unroll
-      for (int j = 0; j < PU; ++j)   // as exp_from: -inf adds nothing, also before the thread has seen a finite token
+      for (int j = 0; j < PU; ++j)
         if (x[j] != -INFINITY) ssum += __expf((x[j] - m) * inv_t);
     }
     if (draw) {
 #pragma unroll
-      for (int j = 0; j < PU; ++j) {
-        if (!ok[j]) continue;
-        const float key = draw_key(base, i0 + j * THREADS, x[j], inv_t);
-        if (key > best) { best = key; btok = i0 + j * THREADS; }
+      for (int j = 0; j < PU; ++j) consider(i0 + j * THREADS + lane, x[j]);
+    }
+  };
+  int i0 = lo + wave * WAVE;
+  for (; i0 + THREADS * (PU - 1) + WAVE <= hi; i0 += THREADS * PU) round(i0, std::true_type{});
+  if (i0 < hi) round(i0, std::false_type{});
+
+  auto most = [](float a, float b) { return fmaxf(a, b); };
+  auto plus = [](float a, float b) { return a + b; };
+  float best = -INFINITY;
+  if (draw) {
+    if (at >= 0) {
+      const float key = rng.key(at, row[at]);
+      if (key > best) best = key;
+    }
+    const float top = wave_fold(best, most);
+    // an infinite key (u of one) is so in both forms
+    const bool open = second != -INFINITY && (top == INFINITY ? second == top : !(second < top - (1e-3f + 1e-6f * fabsf(top))));
+    if (__any(open) || (top != -INFINITY && __popcll(__ballot(best == top)) > 1)) {
+      best = -INFINITY;
+      for (int i0 = lo + wave * WAVE; i0 < hi; i0 += THREADS * PU) {
+        float x[PU];
+        uint64_t votes[PU];
+#pragma unroll
+        for (int j = 0; j < PU; ++j) x[j] = row[min(i0 + j * THREADS + lane, hi - 1)];
+        if (mrow) allowed(i0, std::false_type{}, votes);
+#pragma unroll
+        for (int j = 0; j < PU; ++j) {
+          const int tok = i0 + j * THREADS + lane;
+          const bool ok = mrow ? (votes[j] >> lane & 1) != 0 : tok < hi;
+          const float key = rng.key(tok, x[j]);
+          if (ok && key > best) { best = key; at = tok; }
+        }
       }
     }
   }
 
-  // fold the threads: max, lowest token at it, rescaled sums, best key
-  __shared__ float red[16];
-  __shared__ unsigned long long sh_best[THREADS / WAVE];
-  __shared__ int sh_arg[THREADS / WAVE];
-  const float M = block_reduce_max<THREADS / WAVE>(m, red);
-  const float S = block_reduce_sum<THREADS / WAVE>(sum * (m == M ? 1.0f : exp_from(m, M)), red);
-  const float SS = cuts ? block_reduce_sum<THREADS / WAVE>(ssum * (m == M ? 1.0f : __expf((m - M) * inv_t)), red) : 0.0f;
-  int a = (m == M && arg >= 0) ? arg : 0x7fffffff;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) a = min(a, __shfl_xor(a, off));
-  const unsigned long long w = wave_max_u64(pack_key(best, btok));
-  if ((tid & 63) == 0) { sh_best[tid >> 6] = w; sh_arg[tid >> 6] = a; }
+  // fold the lanes, then the waves: max, lowest token at it, rescaled sums, best key
+  __shared__ float sh_m[THREADS / WAVE], sh_s[THREADS / WAVE], sh_ss[THREADS / WAVE], sh_key[THREADS / WAVE];
+  __shared__ int sh_tok[THREADS / WAVE], sh_arg[THREADS / WAVE];
+  const float M = wave_fold(m, most);
+  const float S = wave_fold(sum * (m == M ? 1.0f : exp_from(m, M)), plus);
+  const float SS = cuts ? wave_fold(ssum * (m == M ? 1.0f : m == -INFINITY ? 0.0f : __expf((m - M) * inv_t)), plus) : 0.0f;
+  const int a = wave_fold((m == M && arg >= 0) ? arg : 0x7fffffff, [](int p, int q) { return min(p, q); });
+  const float K = wave_fold(best, most);
+  const int tok = wave_fold(best == K ? at : -1, [](int p, int q) { return max(p, q); });   // of equal keys the last token
+  if (lane == 0) {
+    sh_m[wave] = M;
+    sh_s[wave] = S;
+    sh_ss[wave] = SS;
+    sh_arg[wave] = a;
+    sh_key[wave] = K;
+    sh_tok[wave] = tok;
+  }
   __syncthreads();
   SlicePart p;
   if (tid == 0) {
-    p.max = M;
-    p.sum = S;
-    p.best = sh_best[0];
-    p.arg = sh_arg[0];
+    p.max = sh_m[0];
 #pragma unroll
-    for (int k = 1; k < THREADS / WAVE; ++k) {
-      p.best = sh_best[k] > p.best ? sh_best[k] : p.best;
-      p.arg = min(p.arg, sh_arg[k]);
+    for (int k = 1; k < THREADS / WAVE; ++k) p.max = fmaxf(p.max, sh_m[k]);
+    p.sum = p.ssum = 0.0f;
+    p.arg = 0x7fffffff;
+    p.best = 0;
+#pragma unroll
+    for (int k = 0; k < THREADS / WAVE; ++k) {
+      const float mk = sh_m[k];
+      p.sum += sh_s[k] * (mk == p.max ? 1.0f : exp_from(mk, p.max));
+      if (cuts) p.ssum += sh_ss[k] * (mk == p.max ? 1.0f : mk == -INFINITY ? 0.0f : __expf((mk - p.max) * inv_t));
+      if (mk == p.max) p.arg = min(p.arg, sh_arg[k]);
+      const unsigned long long w = pack_key(sh_key[k], max(sh_tok[k], 0));
+      p.best = w > p.best ? w : p.best;
     }
     if (p.arg == 0x7fffffff) p.arg = -1;
-    p.ssum = SS;
     p.edge = INFINITY;
     p.listed = 0;
     p.mass = 0.0f;
@@ -210,12 +361,11 @@ __device__ __forceinline__ SlicePart slice_part(const float* __restrict__ row, c
 // even the first step fits.
 __device__ __forceinline__ bool slice_list(SliceToken* __restrict__ list, int cap, const float* __restrict__ row,
                                            const uint32_t* __restrict__ mrow, float temp, float M, int lo, int hi,
-                                           float& edge, int& listed, float& mass) {
+                                           SliceToken* __restrict__ near, float& edge, int& listed, float& mass) {
   constexpr float STEP = 2.5f, FINE = STEP / 8;
   const int tid = threadIdx.x, lane = tid & 63;
   const float inv_t = (temp > 0.0f) ? 1.0f / temp : 0.0f;
   __shared__ int counts[8], fine[8], put, put2;
-  __shared__ SliceToken near[SHORT];
   __shared__ float red[16];
   if (tid < 8) counts[tid] = fine[tid] = 0;
   if (tid == 8) put = put2 = 0;
@@ -325,7 +475,9 @@ __global__ void __launch_bounds__(PT) sample_part_kernel(
   const float* row = logits + (int64_t)b * V;
   const uint32_t* mrow = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
   const bool cuts = temp != 0.0f && truncates(top_ps[b], top_ks[b], V);
-  SlicePart p = slice_part<PT>(row, mrow, temp, cuts, draw_base(seeds[b], steps[b]), lo, hi);
+  __shared__ SliceToken room[PT * PU];   // a masked row's allowed tokens, or what slice_list looks at
+  static_assert(SHORT <= PT * PU);
+  SlicePart p = slice_part<PT>(row, mrow, temp, cuts, draw_base(seeds[b], steps[b]), lo, hi, room);
   bool pays = LISTS && cuts && lists_pay(gridDim.y, V, top_ks[b], cap, mask != nullptr);
   if (LISTS == 2 && pays) {
     const int rows = gridDim.y, lane = threadIdx.x & 63;
@@ -345,7 +497,7 @@ __global__ void __launch_bounds__(PT) sample_part_kernel(
     float edge = top, mass = 0.0f;
     int listed = 0;
     if (top - top == 0.0f && !slice_list(lists + ((int64_t)b * gridDim.x + blockIdx.x) * cap, cap, row, mrow, temp, top,
-                                         lo, hi, edge, listed, mass)) {
+                                         lo, hi, room, edge, listed, mass)) {
       edge = INFINITY;
       listed = 0;
       mass = 0.0f;
@@ -393,7 +545,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   __shared__ int sh_count[64], sh_total;
   if constexpr (WHOLE) {
     const SlicePart p = slice_part<NT>(row, mrow, temp, temp != 0.0f && truncates(top_p, top_k, V),
-                                       draw_base(seeds[b], steps[b]), 0, V);
+                                       draw_base(seeds[b], steps[b]), 0, V, nullptr);
     if (tid == 0) {
       sh_max = p.max;
       sh_sum = p.sum;
@@ -574,7 +726,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   // rounded: at a scaled max of 3000 up to 1e-4 apart, which the factor takes out
   const float need_mass = top_p < 1.0f ? top_p * (sh_ssum * __expf(sx_of(gmax, inv_t, smax))) : INFINITY;
   const unsigned int need_cnt = (top_k > 0 && top_k < V) ? (unsigned)top_k : 0xffffffffu;
-  const uint64_t base = draw_base(seeds[b], steps[b]);
+  const Draw rng(draw_base(seeds[b], steps[b]), inv_t);
   // bins that the slices' lists hold whole; their tokens then stand in for the row if the cut lies there
   int whole = 0;
   bool hope = false;
@@ -673,7 +825,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   float best = -INFINITY;
   int btok = argmax_tok;
   auto consider = [&](int i, float x) {
-    const float key = draw_key(base, i, x, inv_t);
+    const float key = rng.key(i, x);
     if (key > best) { best = key; btok = i; }
   };
   if (near) {
@@ -801,17 +953,20 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   }
 }
 
-// rows -> slices: about eight 256-thread workgroups per compute unit, no slice
-// under 2048 tokens (one load round per thread) and at most 64 slices a row (one
+// rows -> slices: at most eight 256-thread workgroups per compute unit, which are there at once (120 rows in 18 slices were
+// 2160, whose last ones ran alone), and whole load rounds of 2048 tokens as far as may be; at most 64 slices a row (one
 // per lane of sample_final's fold). 0: rows of up to 4096 tokens, half a load round of
 // sample_final's workgroup, take its launch alone: called from Python 9.0 us against 12.5
 // for any number of rows of 300 to 4000 tokens, in a graph 6 to 8 against 8 to 9.5
 extern "C" int sample_slices(int B, int V) {
   if (V <= 4 * NT) return 0;
   const int most = (V + PT * PU - 1) / (PT * PU);
-  const int want = (2048 + B - 1) / B;
-  const int n = want < most ? want : most;
-  return n < 1 ? 1 : n > 64 ? 64 : n;
+  const int want = 2048 / B;
+  int n = want < most ? want : most;
+  n = n < 1 ? 1 : n > 64 ? 64 : n;
+  if ((int64_t)B * n < 1024) return n;   // compute units are left over
+  const int rounds = (V + n * PT * PU - 1) / (n * PT * PU);
+  return (V + rounds * PT * PU - 1) / (rounds * PT * PU);
 }
 
 // Tokens of a slice's list, or 0: no lists. They cost two more walks over the truncated rows by all workgroups and save
@@ -842,7 +997,7 @@ extern "C" void launch_sample(int64_t* tokens, float* logprobs, void* parts, con
                               const int64_t* seeds, const int64_t* steps, const uint32_t* mask, int B,
                               int V, float* dbg, hipStream_t stream) {
   const int n = sample_slices(B, V);
-  const int slice = n > 0 ? (V + n - 1) / n : V;
+  const int slice = n > 0 ? ((V + n - 1) / n + 63) / 64 * 64 : V;    // whole words of the masks
   const int cap = sample_cap(B, V, n, mask != nullptr);
   SliceToken* lists = cap ? (SliceToken*)((SlicePart*)parts + (int64_t)B * n) : nullptr;   // B is one launch's
   // rows of a launch lie on the grid's y, which ends at 65535

@@ -270,3 +270,57 @@ def test_top_p_a_few_ulps_below_one(ulps):
             # the lowest ten of 400 (a fortieth of the mass at most, the rounding of the sums is 1e-5 of it) may be out
             kept = np.argsort(-x[b])[:near - 10]
             assert key[b, won[0]] >= key[b, kept].max() - 1e-3, (call, b)
+
+
+def draws(seed, step, V):
+    with np.errstate(over="ignore"):
+        base = splitmix(np.uint64(seed) * np.uint64(0x9E3779B97F4A7C15) + np.uint64(step) * np.uint64(0xBF58476D1CE4E5B9))
+    return splitmix(base ^ np.arange(V, dtype=np.uint64)) >> np.uint64(40)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("B,V", [(1, 2049), (3, 6145), (1, 16447), (40, 50257), (200, 32801), (700, 8193)])
+def test_flat_rows_draw_the_highest_hash(B, V, masked):
+    """Equal logits: the draw is the hash's alone, lanes hold several near the top and ties are of equal hashes."""
+    mask, ok = None, np.ones((B, V), dtype=bool)
+    if masked:
+        bits = torch.rand(B, (V + 31) // 32 * 32, generator=torch.Generator().manual_seed(V)) < 0.1
+        bits[:, V - 1] = True
+        w = (bits.view(B, -1, 32).long() << torch.arange(32)).sum(-1)
+        mask = torch.where(w >= 2**31, w - 2**32, w).to(torch.int32).to(DEV)
+        ok = bits[:, :V].numpy()
+    one = torch.ones(B, device=DEV)
+    seeds = torch.arange(B) * 7919 + V
+    toks, lps = ops.sample(torch.full((B, V), 3.25, device=DEV), one, one, torch.zeros(B, dtype=torch.int32, device=DEV),
+                           seeds.to(DEV), torch.full((B,), 3, device=DEV), mask)
+    for b in range(B):
+        h = np.where(ok[b], draws(int(seeds[b]), 3, V).astype(np.int64), -1)
+        assert h[int(toks[b])] == h.max()
+        assert abs(float(lps[b]) + np.log(ok[b].sum())) < 1e-5 * np.log(V) + 1e-6
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_a_uniform_of_one_wins(masked):
+    """One hash in 2^24 gives u = 1 in float32, an infinite key: it is drawn whatever its logit, unless masked."""
+    V = 131072
+    found = [(s, int(h.argmax())) for s in range(600) for h in (draws(s, 1, V),) if int(h.max()) == 0xffffff][:3]
+    assert found, "600 rows of 2^17 have about 4.7"
+    B = len(found)
+    seeds = torch.tensor([s for s, _ in found])
+    at = [t for _, t in found]
+    logits = torch.randn(B, V, generator=torch.Generator().manual_seed(1))
+    logits[range(B), at] = -40.0
+    mask = None
+    if masked:
+        mask = torch.full((B, V // 32), -1, dtype=torch.int32)
+        for b in range(0, B, 2):
+            mask[b, at[b] // 32] ^= torch.tensor(1 << (at[b] % 32) if at[b] % 32 < 31 else -2**31, dtype=torch.int32)
+        mask = mask.to(DEV)
+    one = torch.ones(B, device=DEV)
+    toks, _ = ops.sample(logits.to(DEV), one, one, torch.zeros(B, dtype=torch.int32, device=DEV), seeds.to(DEV),
+                         one.long(), mask)
+    for b in range(B):
+        if masked and b % 2 == 0:
+            assert int(toks[b]) != at[b]
+        else:
+            assert int(toks[b]) == at[b]
