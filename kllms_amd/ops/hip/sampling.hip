@@ -23,7 +23,9 @@
 //
 // Measured, 128256 tokens a row: 120 rows, half of them with top-p 0.95 and top-k 50, 50 us (79 with sweeps alone, 346 with
 // one workgroup per row walking it three to six times); 8 rows, all truncated, 24 us (52). With the draw of slice_part:
-// 43.7 us for the 120 rows, 8.8 us for 16 masked ones.
+// 43.7 us for the 120 rows, 8.8 us for 16 masked ones. With lists that each thread places its own tokens in (by ballots and
+// a counter in LDS 8.6 us of a slice's 22, now 4.4 of 16) and the cut made from tokens in registers (12 us a row, now 8):
+// 36 us for the 120 rows, 17 for 7 truncated ones.
 //
 // The draw is counter-based: hash(seed, step, token), identical regardless of
 // batch composition and of the slicing. What follows from a sum is so to fp32
@@ -158,6 +160,26 @@ __device__ __forceinline__ T wave_fold(T v, Op op) {
   v = op(back((int)rows[0]), back((int)rows[1]));
   const auto halves = __builtin_amdgcn_permlane32_swap((unsigned)bits(v), (unsigned)bits(v), false, false);
   return op(back((int)halves[0]), back((int)halves[1]));
+}
+
+// sums up to and with each lane, likewise: shifts in rows of 16, then the rows' ends to the rows behind them
+template <class T>
+__device__ __forceinline__ T wave_scan(T v) {
+  auto bits = [](T x) { return __builtin_bit_cast(int, x); };
+  auto back = [](int x) { return __builtin_bit_cast(T, x); };
+  v += back(__builtin_amdgcn_update_dpp(0, bits(v), 0x111, 0xf, 0xf, false));
+  v += back(__builtin_amdgcn_update_dpp(0, bits(v), 0x112, 0xf, 0xf, false));
+  v += back(__builtin_amdgcn_update_dpp(0, bits(v), 0x114, 0xf, 0xf, false));
+  v += back(__builtin_amdgcn_update_dpp(0, bits(v), 0x118, 0xf, 0xf, false));
+  v += back(__builtin_amdgcn_update_dpp(0, bits(v), 0x142, 0xa, 0xf, false));
+  v += back(__builtin_amdgcn_update_dpp(0, bits(v), 0x143, 0xc, 0xf, false));
+  return v;
+}
+
+// the lane before's value, 0 in the first
+template <class T>
+__device__ __forceinline__ T wave_before(T v) {
+  return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, false));
 }
 
 // tokens [lo, hi) of a row by a workgroup of THREADS, lo a multiple of 64; the result is thread 0's. strip: room for the tokens of a masked row
@@ -363,14 +385,16 @@ __device__ __forceinline__ bool slice_list(SliceToken* __restrict__ list, int ca
                                            const uint32_t* __restrict__ mrow, float temp, float M, int lo, int hi,
                                            SliceToken* __restrict__ near, float& edge, int& listed, float& mass) {
   constexpr float STEP = 2.5f, FINE = STEP / 8;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float inv_t = (temp > 0.0f) ? 1.0f / temp : 0.0f;
-  __shared__ int counts[8], fine[8], put, put2;
-  __shared__ float red[16];
+  __shared__ __attribute__((aligned(16))) int counts[8];
+  __shared__ int fine[8], put, taken[PT / WAVE];
+  __shared__ float red[PT / WAVE];
   if (tid < 8) counts[tid] = fine[tid] = 0;
-  if (tid == 8) put = put2 = 0;
+  if (tid == 8) put = 0;
   __syncthreads();
-  auto walk = [&](auto f) {              // f(token, logit, there is one); all lanes take every step
+  auto window = [&](float x) { return (M - x) * inv_t * (1.0f / STEP); };
+  auto walk = [&](auto f) {              // f(token, logit, there is one)
     for (int i0 = lo; i0 < hi; i0 += PT * PU) {
       float x[PU];
 #pragma unroll
@@ -382,44 +406,57 @@ __device__ __forceinline__ bool slice_list(SliceToken* __restrict__ list, int ca
       }
     }
   };
+  auto plus = [](int p, int q) { return p + q; };
   unsigned long long windows = 0;        // eight counts of 8 bits: a thread has at most 255 tokens
   walk([&](int, float x, bool ok) {
-    const float d = (M - x) * inv_t * (1.0f / STEP);
+    const float d = window(x);
     if (ok && d < 8.0f) windows += 1ull << (8 * (int)d);
   });
 #pragma unroll
   for (int k = 0; k < 4; ++k) {          // two counts of 16 bits a word: 64 lanes fit
     uint32_t w = (uint32_t)(windows >> (16 * k));
-    w = (w & 0xff) | (w & 0xff00) << 8;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) w += __shfl_xor(w, off);
+    w = (uint32_t)wave_fold((int)((w & 0xff) | (w & 0xff00) << 8), plus);
     if (lane == 0) {
       atomicAdd(&counts[2 * k], (int)(w & 0xffff));
       atomicAdd(&counts[2 * k + 1], (int)(w >> 16));
     }
   }
   __syncthreads();
-  int deep = 0, n = 0;
-  while (deep < 8 && n + counts[deep] <= cap) n += counts[deep++];
-  const bool closely = deep < 8 && n + counts[deep] <= SHORT;
+  int in_window[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) in_window[k] = counts[k];
+  int deep = 0, n = 0, next = 0;         // whole windows, their tokens, those of the window behind them
+  bool more = true;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    if (more && n + in_window[k] <= cap) n += in_window[k], deep = k + 1;
+    else if (more) next = in_window[k], more = false;
+  }
+  const bool closely = deep < 8 && n + next <= SHORT;
   if (deep == 0 && !closely) return false;
-  const float top = M - (deep + closely) * STEP * temp;
+  const int steps = deep + closely;
+  // each thread's tokens behind those of the threads before it: their number is in its windows
+  int mine = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) mine += k < steps ? (int)(windows >> (8 * k) & 0xff) : 0;
+  const int upto = wave_scan(mine);
+  if (lane == 63) taken[wave] = upto;
+  __syncthreads();
+  int at = upto - mine, found = 0;
+#pragma unroll
+  for (int w = 0; w < PT / WAVE; ++w) {
+    at += w < wave ? taken[w] : 0;
+    found += taken[w];
+  }
+  if (found > SHORT) return false;
   walk([&](int i, float x, bool ok) {
-    const bool in = ok && x >= top;
-    const unsigned long long votes = __ballot(in);
-    if (!votes) return;
-    int at = 0;
-    if (lane == 0) at = atomicAdd(&put, (int)__popcll(votes));
-    at = __shfl(at, 0) + (int)__popcll(votes & ((1ull << lane) - 1));
-    if (in && at < SHORT) near[at] = SliceToken{x, i};
+    if (ok && window(x) < (float)steps) near[at++] = SliceToken{x, i};
   });
   __syncthreads();
-  const int found = put;                 // a token at a window's end can fall on the other side of ``top``
-  if (found > SHORT) return false;
-  float from = top;
+  float from = M - steps * STEP * temp;
   if (closely) {
     for (int e = tid; e < found; e += PT) {
-      const float d = ((M - near[e].x) * inv_t * (1.0f / STEP) - deep) * 8.0f;
+      const float d = (window(near[e].x) - deep) * 8.0f;
       if (d >= 0.0f) atomicAdd(&fine[min((int)d, 7)], 1);
     }
     __syncthreads();
@@ -432,19 +469,24 @@ __device__ __forceinline__ bool slice_list(SliceToken* __restrict__ list, int ca
   for (int e0 = 0; e0 < found; e0 += PT) {
     const int e = e0 + tid;
     const SliceToken t = near[min(e, found - 1)];
-    const bool in = e < found && t.x >= from;
+    const bool in = e < found && t.x >= from;      // a token at a window's end can fall on the other side of ``from``
     const unsigned long long votes = __ballot(in);
     if (!votes) continue;
     int at = 0;
-    if (lane == 0) at = atomicAdd(&put2, (int)__popcll(votes));
+    if (lane == 0) at = atomicAdd(&put, (int)__popcll(votes));
     at = __shfl(at, 0) + (int)__popcll(votes & ((1ull << lane) - 1));
     if (!in) continue;
     sum += __expf((t.x - M) * inv_t);
     if (at < cap) list[at] = t;
   }
-  mass = block_reduce_sum<PT / WAVE>(sum, red);
-  listed = put2;
-  edge = from;
+  sum = wave_fold(sum, [](float p, float q) { return p + q; });
+  if (lane == 0) red[wave] = sum;
+  __syncthreads();
+  mass = 0.0f;
+#pragma unroll
+  for (int w = 0; w < PT / WAVE; ++w) mass += red[w];
+  listed = put;
+  edge = from + (4e-7f * fabsf(M) + 1e-5f * temp);   // above what the windows' rounding can have left out
   return listed <= cap;
 }
 
@@ -457,9 +499,8 @@ __device__ __forceinline__ bool lists_pay(int rows, int V, int top_k, int cap, b
   return (masked && few) || (top_k > 0 && top_k <= (few ? cap + cap / 4 : cap));
 }
 
-// LISTS 0: what a call without lists need not carry (its truncated rows are 1 us faster so); 2: only if one row in eight of
-// the call is not truncated, which every wave counts for itself
-template <int LISTS>
+// LISTS false: what a call without lists need not carry (its truncated rows are 1 us faster so)
+template <bool LISTS>
 __global__ void __launch_bounds__(PT) sample_part_kernel(
     SlicePart* __restrict__ parts,        // [B, slices]
     const float* __restrict__ logits,     // [B, V]
@@ -478,17 +519,7 @@ __global__ void __launch_bounds__(PT) sample_part_kernel(
   __shared__ SliceToken room[PT * PU];   // a masked row's allowed tokens, or what slice_list looks at
   static_assert(SHORT <= PT * PU);
   SlicePart p = slice_part<PT>(row, mrow, temp, cuts, draw_base(seeds[b], steps[b]), lo, hi, room);
-  bool pays = LISTS && cuts && lists_pay(gridDim.y, V, top_ks[b], cap, mask != nullptr);
-  if (LISTS == 2 && pays) {
-    const int rows = gridDim.y, lane = threadIdx.x & 63;
-    int n = 0;
-#pragma unroll 4
-    for (int r0 = 0; r0 < rows; r0 += WAVE) {
-      const int r = min(r0 + lane, rows - 1);
-      n += __popcll(__ballot(r0 + lane < rows && temperatures[r] != 0.0f && truncates(top_ps[r], top_ks[r], V)));
-    }
-    pays = n * 8 <= rows * 7;
-  }
+  const bool pays = LISTS && cuts && lists_pay(gridDim.y, V, top_ks[b], cap, mask != nullptr);
   if (pays) {
     __shared__ float top;
     // without an allowed token there is nothing to list; a max or a sum that is not finite leaves the row to the sweeps
@@ -536,7 +567,24 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   const float top_p = top_ps[b];
   const int top_k = top_ks[b];
   const float inv_t = (temp > 0.0f) ? 1.0f / temp : 0.0f;
+  const bool cuts = temp != 0.0f && truncates(top_p, top_k, V);
+  const Draw rng(draw_base(seeds[b], steps[b]), inv_t);
 
+  __shared__ float hist_mass[NW * SBINS];
+  __shared__ unsigned int hist_cnt[NW * SBINS];
+  auto clear_hist = [&]() {
+    for (int i = tid; i < NW * SBINS; i += NT) {
+      hist_mass[i] = 0.0f;
+      hist_cnt[i] = 0;
+    }
+  };
+  // the lists are on their way before it is known how much of them counts
+  SliceToken ahead[SLIST / NT];
+  if (LISTS && cuts) {
+#pragma unroll
+    for (int k = 0; k < SLIST / NT; ++k)
+      ahead[k] = lists[(int64_t)b * slices * cap + min(tid + k * NT, slices * cap - 1)];
+  }
   __shared__ float sh_max, sh_sum, sh_ssum;
   __shared__ int sh_argmax;
   __shared__ unsigned long long sh_best;
@@ -544,8 +592,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   __shared__ float sh_mass;              // and what those weigh, against the max
   __shared__ int sh_count[64], sh_total;
   if constexpr (WHOLE) {
-    const SlicePart p = slice_part<NT>(row, mrow, temp, temp != 0.0f && truncates(top_p, top_k, V),
-                                       draw_base(seeds[b], steps[b]), 0, V, nullptr);
+    const SlicePart p = slice_part<NT>(row, mrow, temp, cuts, draw_base(seeds[b], steps[b]), 0, V, nullptr);
     if (tid == 0) {
       sh_max = p.max;
       sh_sum = p.sum;
@@ -556,20 +603,20 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   } else if (wid == 0) {
     SlicePart p{-INFINITY, 0.0f, -1, 0.0f, (unsigned long long)NO_KEY << 32, -INFINITY, 0, 0.0f, 0};
     if (lane < slices) p = parts[(int64_t)b * slices + lane];
-    const float M = wave_reduce_max(p.max);
-    const float S = wave_reduce_sum(p.sum * (p.max == M ? 1.0f : exp_from(p.max, M)));
+    auto most = [](float v, float w) { return fmaxf(v, w); };
+    auto plus = [](float v, float w) { return v + w; };
+    const float M = wave_fold(p.max, most);
+    const float S = wave_fold(p.sum * (p.max == M ? 1.0f : exp_from(p.max, M)), plus);
     // a slice without an allowed token has nothing to add
-    const float SS = wave_reduce_sum(p.arg < 0 ? 0.0f : p.ssum * (p.max == M ? 1.0f : __expf((p.max - M) * inv_t)));
-    int a = (p.max == M && p.arg >= 0) ? p.arg : 0x7fffffff;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) a = min(a, __shfl_xor(a, off));
-    const unsigned long long w = wave_max_u64(p.best);
-    if (LISTS && temp != 0.0f && truncates(top_p, top_k, V)) {
-      const float edge = wave_reduce_max(p.edge);
-      const float lmass = wave_reduce_sum(p.listed == 0 ? 0.0f : p.mass * (p.max == M ? 1.0f : __expf((p.max - M) * inv_t)));
-      int total = p.listed;
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
+    const float scale = p.max == M ? 1.0f : __expf((p.max - M) * inv_t);
+    const float SS = cuts ? wave_fold(p.arg < 0 ? 0.0f : p.ssum * scale, plus) : 0.0f;
+    const int a = wave_fold((p.max == M && p.arg >= 0) ? p.arg : 0x7fffffff, [](int v, int w) { return min(v, w); });
+    unsigned long long w = 0;
+    if (!cuts) w = wave_max_u64(p.best);
+    if (LISTS && cuts) {
+      const float edge = wave_fold(p.edge, most);
+      const float lmass = wave_fold(p.listed == 0 ? 0.0f : p.mass * scale, plus);
+      const int total = wave_fold(p.listed, [](int v, int w) { return v + w; });
       sh_count[lane] = p.listed;
       if (lane == 0) {
         sh_edge = edge;
@@ -585,11 +632,12 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
       sh_best = w;
     }
   }
+  if (cuts) clear_hist();                // beside the fold
   __syncthreads();
   const float gmax = sh_max;
   const float gsum_unscaled = sh_sum;
   const int argmax_tok = sh_argmax;
-  if (temp == 0.0f || !truncates(top_p, top_k, V)) {
+  if (!cuts) {
     if (tid == 0) {
       const int tok = (temp == 0.0f || (uint32_t)(sh_best >> 32) == NO_KEY) ? argmax_tok
                                                                            : (int)(sh_best & 0xffffffffu);
@@ -599,20 +647,12 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
     return;
   }
 
-  __shared__ float hist_mass[NW * SBINS];
-  __shared__ unsigned int hist_cnt[NW * SBINS];
-  __shared__ float list_sx[SLIST];
+  __shared__ float list_x[SLIST];
   __shared__ int list_tok[SLIST];
   __shared__ int sh_listed;
   const float smax = gmax * inv_t;
   float* my_mass = hist_mass + wid * SBINS;
   unsigned int* my_cnt = hist_cnt + wid * SBINS;
-  auto clear_hist = [&]() {
-    for (int i = tid; i < NW * SBINS; i += NT) {
-      hist_mass[i] = 0.0f;
-      hist_cnt[i] = 0;
-    }
-  };
   // fold the per-wave histograms over bins [from, to): thread j owns bin j; the
   // copy of wave 0 becomes the whole
   auto fold_hist = [&](int from, int to) {
@@ -688,17 +728,8 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
       ms += m[k];
       cs += c[k];
     }
-    float mi = ms;
-    unsigned int ci = cs;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const float mo = __shfl_up(mi, off);
-      const unsigned int co = __shfl_up(ci, off);
-      if (lane >= off) { mi += mo; ci += co; }
-    }
-    float mb = __shfl_up(mi, 1);
-    unsigned int cb = __shfl_up(ci, 1);
-    if (lane == 0) { mb = 0.0f; cb = 0; }
+    float mb = wave_before(wave_scan(ms));
+    unsigned int cb = wave_before(wave_scan(cs));
     int hit = -1;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -714,9 +745,9 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
     const unsigned long long any = __ballot(hit >= 0);
     if (!any) return -1;
     const int src = __ffsll(any) - 1;
-    before_mass = __shfl(mb, src);
-    before_cnt = __shfl(cb, src);
-    return __shfl(hit, src);
+    before_mass = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mb), src));
+    before_cnt = __builtin_amdgcn_readlane(cb, src);
+    return __builtin_amdgcn_readlane(hit, src);
   };
 
   // ---- histogram of the scaled mass, boundary bin --------------------------
@@ -726,7 +757,6 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   // rounded: at a scaled max of 3000 up to 1e-4 apart, which the factor takes out
   const float need_mass = top_p < 1.0f ? top_p * (sh_ssum * __expf(sx_of(gmax, inv_t, smax))) : INFINITY;
   const unsigned int need_cnt = (top_k > 0 && top_k < V) ? (unsigned)top_k : 0xffffffffu;
-  const Draw rng(draw_base(seeds[b], steps[b]), inv_t);
   // bins that the slices' lists hold whole; their tokens then stand in for the row if the cut lies there
   int whole = 0;
   bool hope = false;
@@ -738,41 +768,128 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   if (tid == 0) sh_best = (unsigned long long)NO_KEY << 32;
   // where the cut is behind the lists, the sweeps over bins that those hold whole are left out
   const int after = whole >= SMID ? 2 : whole >= SNEAR ? 1 : 0;
+  float best = -INFINITY, best_x = 0.0f;
+  int btok = argmax_tok;
+  auto consider = [&](int i, float x) {
+    const float key = rng.key(i, x);
+    if (key > best) { best = key; best_x = x; btok = i; }
+  };
+  auto finish = [&]() {
+    const float K = wave_fold(best, [](float v, float w) { return fmaxf(v, w); });
+    const int tok = wave_fold(best == K ? btok : -1, [](int v, int w) { return max(v, w); });
+    if (lane == 0) atomicMax(&sh_best, pack_key(K, tok));
+    __syncthreads();
+    const bool drawn = (uint32_t)(sh_best >> 32) != NO_KEY;
+    if (drawn ? pack_key(best, btok) == sh_best : tid == 0) {
+      out_tokens[b] = btok;
+      out_logprobs[b] = (drawn ? best_x : row[btok]) - gmax - __logf(gsum_unscaled);
+    }
+  };
+  bool fresh = true;                     // the histogram is clear
+  int start = whole > 0 && hope ? -1 : after;
+  if constexpr (LISTS) {
+    // A cut in the lists, and few tokens in its bin: their order is made by one wave, and a thread's tokens stay in
+    // registers. Anything else is left to the general way below
+    if (start < 0 && !dbg) {
+      float sx[SLIST / NT];
+      int bin[SLIST / NT];
+      if (tid == 0) sh_listed = 0;
+#pragma unroll
+      for (int k = 0; k < SLIST / NT; ++k) {
+        const int e = tid + k * NT;
+        sx[k] = sx_of(ahead[k].x, inv_t, smax);
+        bin[k] = e < slices * cap && e % cap < sh_count[e / cap] ? coarse_bin(sx[k]) : SBINS;
+        if (bin[k] >= whole) bin[k] = SBINS;
+        if (bin[k] < SBINS) {
+          atomicAdd(&my_mass[bin[k]], __expf(sx[k]));
+          atomicAdd(&my_cnt[bin[k]], 1u);
+        }
+      }
+      __syncthreads();
+      fold_hist(0, whole);
+      __syncthreads();
+      if (wid == 0) {
+        float before_mass = 0.0f;
+        unsigned int before_cnt = 0;
+        const int cut_bin = find_cut(whole, need_mass, need_cnt, before_mass, before_cnt);
+        if (lane == 0) {
+          sh_cut = cut_bin;
+          sh_need_mass = need_mass - before_mass;
+          sh_need_cnt = need_cnt == 0xffffffffu ? need_cnt : need_cnt - before_cnt;
+        }
+      }
+      __syncthreads();
+      const int cut = sh_cut;
+      const unsigned int n = cut < 0 ? 0 : hist_cnt[cut];
+      if (cut >= 0 && n <= WAVE) {
+#pragma unroll
+        for (int k = 0; k < SLIST / NT; ++k)
+          if (bin[k] == cut) {
+            const int at = atomicAdd(&sh_listed, 1);
+            list_x[at] = ahead[k].x;
+            list_tok[at] = ahead[k].tok;
+          }
+#pragma unroll
+        for (int k = 0; k < SLIST / NT; ++k)
+          if (bin[k] < cut) consider(ahead[k].tok, ahead[k].x);
+        __syncthreads();
+        if (wid == 0) {
+          // what of the bin lies above a token; equal ones are in or out together, as in the general way
+          const float x = list_x[lane < (int)n ? lane : 0], s = sx_of(x, inv_t, smax), e = __expf(s);
+          float above = 0.0f;
+          unsigned int higher = 0;
+          for (unsigned int j = 0; j < n; ++j) {
+            const bool over = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s), j)) > s;
+            above += over ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), j)) : 0.0f;
+            higher += over;
+          }
+          if (lane < (int)n && above < sh_need_mass && higher < sh_need_cnt) consider(list_tok[lane], x);
+        }
+        finish();
+        return;
+      }
+      fresh = false;
+      if (cut < 0) start = after;
+    }
+  }
   bool listing = false;                  // whether the part that found the cut, with those it adds to, listed its tokens
-  for (int part = whole > 0 && hope ? -1 : after; part < 3; part = part < 0 ? after : part + 1) {
+  for (int part = start; part < 3; part = part < 0 ? after : part + 1) {
     const int from = part <= after ? 0 : part == 1 ? SNEAR : SMID;
     const int to = part < 0 ? whole : part == 0 ? SNEAR : part == 1 ? SMID : SBINS;
     listing = part < 2;
     if (part <= after) {
-      __syncthreads();
-      clear_hist();
+      if (!fresh) {
+        __syncthreads();
+        clear_hist();
+      }
+      fresh = false;
       if (tid == 0) sh_listed = 0;
       __syncthreads();
     }
-    auto count = [&](int i, float sx, int bin) {
+    auto count = [&](int i, float x, float sx, int bin) {
       atomicAdd(&my_mass[bin], __expf(sx));
       atomicAdd(&my_cnt[bin], 1u);
       if (listing) {
         const int at = atomicAdd(&sh_listed, 1);
         if (at < SLIST) {
-          list_sx[at] = sx;
+          list_x[at] = x;
           list_tok[at] = i;
         }
       }
     };
     if (part < 0) {
-      const SliceToken* mine = lists + (int64_t)b * slices * cap;
-      for (int e = tid; e < slices * cap; e += NT) {
-        if (e % cap >= sh_count[e / cap]) continue;
-        const SliceToken t = mine[e];
-        const float sx = sx_of(t.x, inv_t, smax);
+#pragma unroll
+      for (int k = 0; k < SLIST / NT; ++k) {
+        const int e = tid + k * NT;
+        if (e >= slices * cap || e % cap >= sh_count[e / cap]) continue;
+        const float sx = sx_of(ahead[k].x, inv_t, smax);
         const int bin = coarse_bin(sx);
-        if (bin < to) count(t.tok, sx, bin);
+        if (bin < to) count(ahead[k].tok, ahead[k].x, sx, bin);
       }
     } else {
-      sweep(part < 2 ? -to * (SRANGE / SBINS) - 1e-3f : NAN, [&](int i, float, float sx) {
+      sweep(part < 2 ? -to * (SRANGE / SBINS) - 1e-3f : NAN, [&](int i, float x, float sx) {
         const int bin = coarse_bin(sx);
-        if (bin >= from && bin < to) count(i, sx, bin);
+        if (bin >= from && bin < to) count(i, x, sx, bin);
       });
     }
     __syncthreads();
@@ -822,16 +939,10 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   const int cut = sh_cut;
   const bool near = listing && (cut < SMID || cut < whole) && sh_listed <= SLIST;   // whole: of the lists that were used, else 0
   const bool fits = near || (cut < SBINS && hist_cnt[cut] <= SLIST);
-  float best = -INFINITY;
-  int btok = argmax_tok;
-  auto consider = [&](int i, float x) {
-    const float key = rng.key(i, x);
-    if (key > best) { best = key; btok = i; }
-  };
   if (near) {
     const int n = sh_listed;
     for (int e = tid; e < n; e += NT)
-      if (coarse_bin(list_sx[e]) < cut) consider(list_tok[e], row[list_tok[e]]);
+      if (coarse_bin(sx_of(list_x[e], inv_t, smax)) < cut) consider(list_tok[e], list_x[e]);
   } else {
     __syncthreads();
     if (tid == 0) sh_listed = 0;
@@ -843,7 +954,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
       } else if (fits && bin == cut) {
         const int at = atomicAdd(&sh_listed, 1);
         if (at < SLIST) {
-          list_sx[at] = sx;
+          list_x[at] = x;
           list_tok[at] = i;
         }
       }
@@ -851,14 +962,16 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
   }
   __syncthreads();
   const int listed = min(sh_listed, SLIST);
-  // f(token, sx) over the boundary bin's tokens
+  // f(token, x, sx) over the boundary bin's tokens
   auto boundary = [&](auto f) {
     if (fits) {
-      for (int e = tid; e < listed; e += NT)
-        if (coarse_bin(list_sx[e]) == cut) f(list_tok[e], list_sx[e]);
+      for (int e = tid; e < listed; e += NT) {
+        const float x = list_x[e], sx = sx_of(x, inv_t, smax);
+        if (coarse_bin(sx) == cut) f(list_tok[e], x, sx);
+      }
     } else {
       sweep(NAN, [&](int i, float x, float sx) {
-        if (coarse_bin(sx) == cut) f(i, sx);
+        if (coarse_bin(sx) == cut) f(i, x, sx);
       });
     }
   };
@@ -875,7 +988,7 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
     const float sel_invw = sh_sel_invw;
     clear_hist();
     __syncthreads();
-    boundary([&](int, float sx) {
+    boundary([&](int, float, float sx) {
       // membership = the EXACT bin the previous level counted this token
       // into equals its boundary bin (bit-identical re-evaluation)
       if (!sel_coarse && min(max((int)((sel_hi - sx) * sel_invw), 0), SBINS - 1) != sel_cut) return;
@@ -902,9 +1015,8 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
           before_mass += bn < SBINS - 1 ? hist_mass[bn] : 0.0f;
           before_cnt += bn < SBINS - 1 ? hist_cnt[bn] : 0u;
         }
-        before_mass = wave_reduce_sum(before_mass);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) before_cnt += __shfl_xor(before_cnt, off);
+        before_mass = wave_fold(before_mass, [](float v, float w) { return v + w; });
+        before_cnt = wave_fold(before_cnt, [](unsigned int v, unsigned int w) { return v + w; });
       }
       if (lane == 0) {
         const float subw = (hi - lo) / SBINS;
@@ -939,18 +1051,11 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
     // the threshold stays in sx space (converting it back to x loses the
     // refined margin to fp32 rounding), exclusive at its lower edge as the bins
     const float thresh = sh_lo;
-    boundary([&](int i, float sx) {
-      if (sx > thresh) consider(i, row[i]);
+    boundary([&](int i, float x, float sx) {
+      if (sx > thresh) consider(i, x);
     });
   }
-  const unsigned long long w = wave_max_u64(pack_key(best, btok));
-  if (lane == 0) atomicMax(&sh_best, w);
-  __syncthreads();
-  if (tid == 0) {
-    const int tok = (int)(sh_best & 0xffffffffu);
-    out_tokens[b] = tok;
-    out_logprobs[b] = row[tok] - gmax - __logf(gsum_unscaled);
-  }
+  finish();
 }
 
 // rows -> slices: at most eight 256-thread workgroups per compute unit, which are there at once (120 rows in 18 slices were
@@ -969,22 +1074,18 @@ extern "C" int sample_slices(int B, int V) {
   return (V + rounds * PT * PU - 1) / (rounds * PT * PU);
 }
 
-// Tokens of a slice's list, or 0: no lists. They cost two more walks over the truncated rows by all workgroups and save
-// the walks of sample_final, one workgroup a row. Worth it on long rows (120 rows of 32000 with top-p and top-k: 33 us
-// without, 37 with; 30 of 50257, masked: 36 and 31) and on as many as leave compute units idle there (sample_asks). One or
-// two rows of a shorter vocabulary sample_final is as fast with by itself, unless a mask is on them (2 x 50257: 22, 24,
-// masked 27, 25; 2 x 128256: 34, 23). Nor have slices lists whose threads would count more than 255 tokens
+// Tokens of a slice's list, or 0: no lists. They cost two more walks over the truncated rows by all workgroups and save the
+// walks of sample_final, one workgroup a row, so they pay on all but the smallest calls, up to the rows at which
+// sample_final's workgroups fill the chip by themselves. us without lists and with, top-p 0.95 and top-k 50, all rows truncated,
+// masked with one in eight allowed in brackets:
+//   1 row of 32000 14.6, 17.8 (13.6, 18.6)   50257 14.0, 16.9 (30.9, 19.1)   128256 19.4, 16.6 (30.9, 18.1)   8 rows of 8192 18.9, 18.5
+//   (18.9, 16.7)   40 of 32000 28.4, 20.1 (27.1, 21.4)   120 of 50257 39.1, 31.0 (40.9, 34.1)   250 of 32000 37.7, 33.1 (37.8,
+//   38.6)   250 of 152064 102.7, 83.0 (121.1, 105.4)   512 of 50257 85.3, 69.0 (88.0, 88.0)   1024 of 32000 103.9, 121.4 (107.6, 160.7)
+// and half of the rows truncated: 120 of 32000 31.9, 22.7 (31.4, 23.0)   512 of 50257 67.0, 53.0 (63.3, 68.2). Nor have slices
+// lists whose threads would count more than 255 tokens.
 static int sample_cap(int B, int V, int n, bool masked) {
-  const int64_t tokens = (int64_t)B * V;
-  return n > 0 && V > 32768 && tokens <= (masked ? 1 << 26 : 1 << 25) && (masked || tokens >= 120000) &&
-         (V + n - 1) / n <= 255 * PT ? SLIST / n : 0;
+  return n > 0 && B <= (masked ? 256 : 512) && (int64_t)B * V >= (masked ? 50000 : 120000) && (V + n - 1) / n <= 255 * PT ? SLIST / n : 0;
 }
-
-// Calls of more rows list only if some are not truncated. us of calls that are truncated throughout, with top-p 0.95 and
-// top-k 50, without lists and with, masked in brackets: 50257 tokens, 60 rows 37, 33 (39, 35)   120 rows 43, 45 (49, 51)   250 rows
-// 50, 56 (61, 77), 54 (67) having asked; 128256 tokens, 120 rows 74, 62 (103, 87)   180 rows 82, 78 (116, 115)   250 rows 90, 91
-// (127, 141), 93 (131) having asked. Half of 250 rows: 55, 45 (65, 56), 47 (58) and 104, 79 (144, 97), 82 (102).
-static bool sample_asks(int B, int V) { return B > (V > 65536 ? 192 : 128); }
 
 // words of 8 bytes that a call needs for its slices, and for their lists
 extern "C" int64_t sample_room(int B, int V, int masked) {
@@ -1007,7 +1108,7 @@ extern "C" void launch_sample(int64_t* tokens, float* logprobs, void* parts, con
     const float* x = logits + (int64_t)b * V;
     const uint32_t* m = mask ? mask + (int64_t)b * ((V + 31) / 32) : nullptr;
     if (n > 0)
-      hipLaunchKernelGGL(!lists ? sample_part_kernel<0> : sample_asks(B, V) ? sample_part_kernel<2> : sample_part_kernel<1>, dim3(n, rows), dim3(PT), 0, stream, p, x,
+      hipLaunchKernelGGL(lists ? sample_part_kernel<true> : sample_part_kernel<false>, dim3(n, rows), dim3(PT), 0, stream, p, x,
                          temps + b, top_ps + b, top_ks + b, seeds + b, steps + b, m, lists, cap, V, slice);
     hipLaunchKernelGGL((n == 0 ? sample_final_kernel<true, false> : lists ? sample_final_kernel<false, true> : sample_final_kernel<false, false>),
                        dim3(rows), dim3(NT), 0, stream,

@@ -324,3 +324,30 @@ def test_a_uniform_of_one_wins(masked):
             assert int(toks[b]) != at[b]
         else:
             assert int(toks[b]) == at[b]
+
+
+@pytest.mark.parametrize("near", [50, 63, 64, 65, 200])
+@pytest.mark.parametrize("width", [0.0, 1e-6, 0.05])
+@pytest.mark.parametrize("B,V", [(1, 131072), (3, 50257), (40, 32000), (512, 8192), (513, 8192)])
+def test_cut_in_a_crowded_bin_of_the_lists(B, V, near, width):
+    """The highest tokens, spread over the row's slices, within a bin of the histogram or equal: one wave orders up to 64
+    of them, more are refined."""
+    g = torch.Generator().manual_seed(near + V)
+    logits = torch.rand(B, V, generator=g) - 12.0
+    at = torch.arange(near) * (V // near) + 7
+    logits[:, at] = 1.0 - width * torch.rand(B, near, generator=g)
+    k = torch.tensor([45, 10, 1])[torch.arange(B) % 3].int()
+    top_p = torch.tensor([1.0, 0.95])[torch.arange(B) % 2]
+    seeds, steps = torch.randint(0, 2**40, (B,), generator=g), torch.randint(0, 99, (B,), generator=g)
+    toks, _ = ops.sample(logits.to(DEV), torch.ones(B, device=DEV), top_p.to(DEV), k.to(DEV), seeds.to(DEV), steps.to(DEV), None)
+    for b in range(0, B, 1 if B < 100 else 41):
+        x = logits[b].double().numpy()
+        order = np.argsort(-x, kind="stable")
+        p = np.exp(x[order] - x.max())
+        before = (np.cumsum(p) - p) / p.sum()
+        lim = int(k[b])
+        must = order[:lim][before[:lim] < float(top_p[b]) - 1e-4]
+        low = x[must[-1]] - 1e-6 - (1e-4 if top_p[b] < 1 else 0.0)      # tokens that tie with the last one may be in
+        t = int(toks[b])
+        key = x + gumbel(int(seeds[b]), int(steps[b]), V)
+        assert x[t] >= low and key[t] >= key[must].max() - max(1e-3, 4e-7 * V)
