@@ -82,6 +82,10 @@ class LlamaAttention(nn.Module):
         self._kv = self.num_kv_heads * self.head_dim
 
     def forward(self, hidden: torch.Tensor, batch: ForwardBatch, cos_sin: torch.Tensor) -> torch.Tensor:
+        return self.o_proj(self.attend(hidden, batch, cos_sin).reshape(hidden.shape[0], -1))
+
+    def attend(self, hidden: torch.Tensor, batch: ForwardBatch, cos_sin: torch.Tensor) -> torch.Tensor:
+        """The heads' results [T, H, D]; keys and values are stored."""
         T = hidden.shape[0]
         qkv = self.qkv_proj(hidden)
         # strided views into the fused QKV row — the HIP kernels take the
@@ -94,10 +98,8 @@ class LlamaAttention(nn.Module):
         ops.rope_store(q, k, v, batch.positions, cos_sin, k_cache, v_cache, batch.slot_mapping, k_scale, v_scale)
 
         if batch.mode == "prefill":
-            out = ops.attn_prefill_varlen(q, k, v, batch.cu_seqlens, self.scale, (batch.plans or {}).get("prefill"))
-        else:
-            out = self.attend_cache(q, batch)
-        return self.o_proj(out.reshape(T, -1))
+            return ops.attn_prefill_varlen(q, k, v, batch.cu_seqlens, self.scale, (batch.plans or {}).get("prefill"))
+        return self.attend_cache(q, batch)
 
     def attend_cache(self, q: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
         """Attention of decode-mode rows q [T, H, D] against the paged cache."""
@@ -124,14 +126,17 @@ class LlamaMLP(nn.Module):
         self._i = cfg.intermediate_size // ctx.world_size
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        return self.down_proj(self.activate(x))
+
+    def activate(self, x: torch.Tensor) -> torch.Tensor:
+        """silu(gate) * up."""
         p = self.gate_up_proj
         plain = ops.only_weights(p, ColumnParallelLinear) and ops.no_global_hooks()
         act = ops.linear_silu(x, p.weight) if plain and p.bias is None else None
         if act is not None:
-            return self.down_proj(act)
-        gate_up = p(x)
-        gate, up = gate_up.split([self._i, self._i], dim=-1)
-        return self.down_proj(ops.silu_mul(gate, up))
+            return act
+        gate, up = p(x).split([self._i, self._i], dim=-1)
+        return ops.silu_mul(gate, up)
 
 
 class RMSNormModule(nn.Module):
@@ -267,12 +272,10 @@ class LlamaForCausalLM(nn.Module):
         return mod
 
     # --- forward ------------------------------------------------------------
-    # rows up to which the fused [gate; up] product is the few-row kernel's, by the weights' size. It saves the
-    # activation's launch, 5 us; the library streams large matrices faster (5.3 TB/s against 4.2 - 5.0) and reads x less.
-    # us, library with activation and few-row kernel, at 1 / 16 / 32 / 64 rows:
-    #   28672 x 4096  63 51 / 64 53 / 59 55 / 57 60 (68 for 57 + 5 at 128)
-    #   27648 x 5120  73 60 / 75 62 / 55 67 / 60 73
-    #   57344 x 8192  178 187 / 175 191 / 174 194 / 184 191
+    # rows up to which the fused [gate; up] product of any width is the few-row kernel's, which saves the activation's
+    # launch. us, library with activation and few-row kernel, at 1 / 32 / 64 / 128 rows:
+    #   27648 x 5120  82 55 / 57 59 / 60 62 / 70 85        24576 x 3072  53 31 / 36 37 at 64 / 43 49
+    #   37888 x 3584  61 62 / 62 64 at 16 / 71 71 / 73 88
     SILU_ROWS_MAX = 64
 
     @classmethod
@@ -280,18 +283,63 @@ class LlamaForCausalLM(nn.Module):
         n = weight.numel()
         return rows <= (cls.SILU_ROWS_MAX if n < 1 << 27 else 16 if n < 1 << 28 else 0)
 
+    # More, of a width that is a power of two: the others' stages take a third longer at many rows. At 1 / 32 / 64 / 128 / 256
+    # rows, 256 beside the better of library and tiles:
+    #   28672 x 4096  65 42 / 55 42 / 55 43 / 58 50 / 69 63        16384 x 2048  20 14 / 20 14 / 21 15 / 24 19 / 30 26
+    #   22016 x 4096  53 33 / 48 41 / 46 38 / 49 47 / 66 60        57344 x 8192  181 163 / 182 169 / 198 175 / 203 197 / 239 309
+    @staticmethod
+    def _silu_streams(rows: int, weight: torch.Tensor) -> bool:
+        n, width = weight.shape
+        return width & (width - 1) == 0 and rows <= (ops.LINEAR_SILU_MAX if n <= 32768 else ops.LINEAR_ROWS_MAX)
+
     def _takes_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> bool:
         """Whether a step runs as _forward_rows: a few decode rows of an unsharded bf16 model on the GPU with the
         sizes that the few-row kernels divide."""
+        return batch.mode == "decode" and input_ids.shape[0] <= ops.LINEAR_ROWS_MAX and self._rows_fit(input_ids, batch)
+
+    def _rows_fit(self, input_ids: torch.Tensor, batch: ForwardBatch) -> bool:
         cfg = self.cfg
         at = self.layers[0].self_attn if len(self.layers) else None
-        return (batch.mode == "decode" and at is not None and input_ids.is_cuda and input_ids.dim() == 1
-                and input_ids.dtype == torch.long
-                and 1 <= input_ids.shape[0] <= ops.LINEAR_ROWS_MAX and self.ctx.world_size == 1
+        return (batch.mode in ("decode", "prefill") and at is not None and input_ids.is_cuda and input_ids.dim() == 1
+                and input_ids.dtype == torch.long and input_ids.shape[0] >= 1 and self.ctx.world_size == 1
                 and self.dtype == torch.bfloat16 and not ops._force_torch() and at.head_dim == 128
                 and cfg.hidden_size % 128 == 0 and cfg.hidden_size <= 16384 and cfg.intermediate_size % 128 == 0
                 and self.cos_sin.is_contiguous() and input_ids.is_contiguous()
                 and all(t.is_contiguous() and t.numel() == input_ids.shape[0] for t in (batch.positions, batch.slot_mapping)))
+
+    def _takes_short(self, input_ids: torch.Tensor, batch: ForwardBatch) -> bool:
+        """Whether more decode rows than _takes_rows takes, or a short prompt, run as _forward_rows: up to the rows at which
+        the few-row products are the faster ones, and where nothing but the modules' own forwards would run. us of the
+        library's product and of linear_part with the reading of its sums, at 160 / 256 / 384 rows:
+          4096 x 4096    27 19 / 23 23 / 25 29      4096 x 14336  84 43 / 63 53 / 78 66      6144 x 4096   28 24 / 40 31 / 36 40
+          2048 x 8192    26 17 / 27 22 / 33 26      8192 x 8192   54 43 / 76 58 / 62 73      10240 x 8192  67 71 / 88 94"""
+        rows = input_ids.shape[0]
+        if not (batch.mode == "prefill" or rows > ops.LINEAR_ROWS_MAX) or rows > ops.LINEAR_PART_MAX:
+            return False
+        if not self._rows_fit(input_ids, batch):
+            return False
+        at = self.layers[0].self_attn
+        widest = max(at.qkv_proj.weight.shape[0], self.cfg.hidden_size)
+        most = ops.LINEAR_PART_MAX if widest <= 6144 else 256 if widest <= 8192 else ops.LINEAR_ROWS_MAX
+        return rows <= most and self._only_weights(input_ids, batch)
+
+    def _only_weights(self, input_ids: torch.Tensor, batch: ForwardBatch) -> bool:
+        """Whether the layers' modules are the plain ones and nothing looks on at their calls."""
+        plain = ops.only_weights
+        if not (ops.no_global_hooks() and ops.plain_call(input_ids, batch.positions, batch.slot_mapping)
+                and plain(self.embed_tokens, nn.Embedding)
+                and not (torch.is_grad_enabled() and any(p.requires_grad for p in self.parameters()))):
+            return False
+        for layer in self.layers:
+            at, mlp = layer.self_attn, layer.mlp
+            if not (plain(layer, self.layer_cls) and plain(at, LlamaAttention) and plain(at.qkv_proj, ColumnParallelLinear)
+                    and plain(at.o_proj, RowParallelLinear)):
+                return False
+            if isinstance(mlp, LlamaMLP) and not (plain(mlp, LlamaMLP) and plain(mlp.gate_up_proj, ColumnParallelLinear)
+                                                  and plain(mlp.down_proj, RowParallelLinear)
+                                                  and mlp.gate_up_proj.bias is None):
+                return False
+        return True
 
     _unknown: Optional[torch.Tensor] = None
 
@@ -311,9 +359,9 @@ class LlamaForCausalLM(nn.Module):
             raise IndexError(f"a decode step had a token id outside the vocabulary of {self.embed_tokens.num_embeddings}")
 
     def _forward_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
-        """A decode step: weights streamed by the few-row kernel, whose split sums go straight into the next row-wise
-        kernel: 8 launches a layer, one more where attention splits the contexts and one where gate/up is the
-        library's."""
+        """A decode step or a short prompt: weights streamed by the few-row kernel, whose split sums go straight into the
+        next row-wise kernel: 8 launches a layer, one more where attention splits the contexts and one where gate/up is the
+        library's. A prompt's fused projection stays whole: its attention reads the keys and values as rows."""
         layers = self.layers
         x, residual = ops.embed_norm_rows(input_ids, self.embed_tokens.weight, layers[0].input_layernorm.weight,
                                           layers[0].input_layernorm.eps, self._unknown_ids())
@@ -321,18 +369,18 @@ class LlamaForCausalLM(nn.Module):
         for i, layer in enumerate(layers):
             at, norm = layer.self_attn, layer.post_attention_layernorm
             k_cache, v_cache, k_scale, v_scale = batch.kv_caches[at.layer_idx]
-            q = ops.rope_store_rows(ops.linear_part(x, at.qkv_proj.weight), at.qkv_proj.bias, at.num_heads,
-                                    batch.positions, self.cos_sin, k_cache, v_cache, batch.slot_mapping, k_scale, v_scale)
-            att = at.attend_cache(q, batch)
+            if batch.mode == "prefill":
+                att = at.attend(x, batch, self.cos_sin)
+            else:
+                q = ops.rope_store_rows(ops.linear_part(x, at.qkv_proj.weight), at.qkv_proj.bias, at.num_heads,
+                                        batch.positions, self.cos_sin, k_cache, v_cache, batch.slot_mapping, k_scale, v_scale)
+                att = at.attend_cache(q, batch)
             x = ops.add_norm_rows(ops.linear_part(att.view(T, -1), at.o_proj.weight), residual, norm.weight, norm.eps)
             norm = layers[i + 1].input_layernorm if i + 1 < len(layers) else self.norm
             mlp = layer.mlp
             if isinstance(mlp, LlamaMLP):
-                if self._silu_rows(T, mlp.gate_up_proj.weight):
-                    act = ops.linear_silu_rows(x, mlp.gate_up_proj.weight)
-                else:
-                    gate, up = mlp.gate_up_proj(x).split([mlp._i, mlp._i], dim=-1)
-                    act = ops.silu_mul(gate, up)
+                w = mlp.gate_up_proj.weight
+                act = (ops.linear_silu_rows(x, w) if self._silu_rows(T, w) or self._silu_streams(T, w) else mlp.activate(x))
                 x = ops.add_norm_rows(ops.linear_part(act, mlp.down_proj.weight), residual, norm.weight, norm.eps)
             else:
                 x, residual = ops.fused_add_rmsnorm(mlp(x), residual, norm.weight, norm.eps)
@@ -357,7 +405,7 @@ class LlamaForCausalLM(nn.Module):
     def forward_hidden(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
         self.check_ids()
         batch = self._planned(input_ids, batch)
-        if self._takes_rows(input_ids, batch):
+        if self._takes_rows(input_ids, batch) or self._takes_short(input_ids, batch):
             return self._forward_rows(input_ids, batch)
         hidden = self.embed_tokens(input_ids)
         residual = None
@@ -373,10 +421,13 @@ class LlamaForCausalLM(nn.Module):
         w = self.lm_head.weight
         if (hidden.dim() == 2 and hidden.is_cuda and hidden.dtype == w.dtype == torch.bfloat16 and not ops._force_torch()
                 and self.lm_head.bias is None and not (torch.is_grad_enabled() and (hidden.requires_grad or w.requires_grad))):
-            # us, the library and the few-row kernel, weights out of cache, at 1 / 32 / 64 / 128 rows:
-            #   32000 x 4096   59 55 / 59 58 / 61 62 / 63 71        128256 x 2048  121 99 / 127 114 / 135 124 / 149 143
-            #   128256 x 4096  188 193 / 209 215 / 224 230 / 250 261
-            if hidden.shape[0] <= 64 and ops.linear_rows_ok(hidden, w):
+            # us, the library and the few-row kernel, weights out of cache, at 1 / 32 / 64 / 96 / 128 rows:
+            #   32000 x 4096   61 49 / 60 51 / 61 52 / 62 55 / 64 60        128256 x 2048  114 94 / 122 106 / 127 117 / 137 131 / 139 143
+            #   128256 x 4096  188 177 / 209 197 / 223 207 / 239 222 / 250 244
+            #   152064 x 3584  230 193 / 263 211 / 224 225 / 240 253 / 255 279
+            K = w.shape[1]
+            most = 64 if K & (K - 1) else 128 if K >= 4096 else 96
+            if hidden.shape[0] <= most and ops.linear_rows_ok(hidden, w):
                 return ops.linear_f32_rows(hidden, w)
             return torch.mm(hidden, w.t(), out_dtype=torch.float32)
         return self.lm_head(hidden).float()

@@ -242,6 +242,8 @@ def attn_decode_paged(
 # GPU-only: callers ask linear_rows_ok first and keep F.linear for everything else.
 
 LINEAR_ROWS_MAX = 128
+LINEAR_PART_MAX = 384      # of linear_part
+LINEAR_SILU_MAX = 256      # of linear_silu_rows
 
 
 def linear_rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -280,6 +282,11 @@ def _plain_call(*ts: torch.Tensor) -> bool:
             and not torch._C._len_torch_function_stack()
             and not torch._C._are_functorch_transforms_active() and not torch.jit.is_tracing()
             and not torch.compiler.is_compiling() and not torch._C._len_torch_dispatch_stack())
+
+
+def plain_call(*ts: torch.Tensor) -> bool:
+    """_plain_call without autocast, under which the library's products have its type."""
+    return _plain_call(*ts) and not torch.is_autocast_enabled("cuda")
 
 
 def only_weights(module: torch.nn.Module, kind: type) -> bool:

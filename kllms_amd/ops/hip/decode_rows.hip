@@ -10,8 +10,8 @@
 // four products: 8 launches (one more where attention splits the contexts, one where
 // gate/up is the library's), where separate reductions, rope, store and activation
 // took 11. A step of 5 rows (32 heads, width 4096, 6 layers, contexts of 560) went
-// from 948 to 774 us with these and linear_rows.hip, one of 120 rows from 1516 to 1237,
-// one of a single row at width 2048 from 492 to 391.
+// from 948 to 774 us with these and few-row products through registers, and to 686 with those of linear_rows.hip; one of
+// 120 rows from 1516 to 1237 and 1122, one of a single row at width 2048 from 492 to 391 and 344.
 
 #include "common.h"
 

@@ -1,233 +1,224 @@
-// Products of a few rows with a weight matrix, y[M, N] = x[M, K] W[N, K]^T, M <= 128
-// (the projections of a decode step), for gfx950.
+// Products of a few rows with a weight matrix, y[M, N] = x[M, K] W[N, K]^T (the projections of a decode step or of a
+// short prompt), for gfx950, on the ring of tile_product.h.
 //
-// The weights' stream is the bound: 64 weight rows per 256-thread workgroup (128 per 512
-// for many rows of x), 16 per wave, each read once and straight from memory to matrix fragments (16x16x32) - a
-// lane group takes 32 contiguous bytes of its row in two loads, so every 128-byte line
-// is used whole, and x is read in the same order of k. x goes through LDS in 128-deep
-// chunks, double-buffered, shared by the waves; its 16-byte units are XORed with
-// the row, which keeps the 16-row fragment reads free of bank conflicts. The weights of
-// the next DEEP chunks are in flight while one is multiplied (4 KB a wave each), and with AHEAD the chunk's x beside
-// them: loads come back in order, so that a wait for an x that was asked for last is one for all weights before it.
-// (DEEP 4 up to 32 rows, 2 above: there x takes 16 registers a chunk. DEEP 4 without AHEAD does nothing. Us with x asked
-// for one chunk before and so: 16384 x 2048 with silu 1 / 40 rows 19.2 / 22.6 and 18.2 / 19.6, 28672 x 4096 5 rows 52.2
-// and 48.5, 8720 x 2048 in one share 15.6 and 12.3, 4096 x 14336 40 rows 27.9 and 25.9, 2048 x 2048 3.9 and 3.8. Above
-// 64 rows the registers for it cost more workgroups than it gives: 28672 x 4096 120 rows 67 and 70.)
+// The weights' stream is the bound, and bytes in flight are what keeps it up: W and x go from memory to LDS without
+// registers in between, 64 deep in k, and a workgroup has all its buffers on their way from its first instruction on -
+// 60 to 150 KB of a compute unit. (Weights loaded to registers two to four chunks ahead, with x through two LDS buffers,
+// streamed 28672 x 4096 at 4.6 TB/s for 5 rows and at 3.4 for 96; so it is 5.7 and 5.2.) A workgroup takes 64 or 128 rows of
+// W; MJ tiles of 32 rows of x are multiplied at once, so that LDS is read once for 16 * MJ rows and not for 16.
 //
-// A matrix of few rows is also split over k (linear_rows_splits); the splits' fp32 sums are left to the consumer, which reads them anyway (rope + store,
-// residual + norm). Forms of the result:
+// A matrix of few rows is also split over k (linear_rows_splits); the splits' fp32 sums are left to the consumer, which
+// reads them anyway (rope + store, residual + norm). Forms of the result:
 //   PART  fp32 sums [S, M, N]          SILU  silu(gate) * up of a fused [gate; up] matrix
 //   F32   fp32, S = 1 (logits)         CLAMPED  the clamped gated form of the hybrid family
 //   BF16  rounded once, bias added before it
 //
-// Measured with the weights out of cache (the library's kernel in brackets), us:
-//   4096 x 4096   5 rows 8.3 (15.6), 128 rows 15.6 (24.5)
-//   4096 x 14336  5 rows 23.7 (26.7: 5 TB/s either way), 64 rows 28.7 (42), 128 rows 36 (75.5)
-//   2048 x 8192   1 row 8.6 (12.8), 64 rows 11.4 (22.6)
-//   28672 x 4096  with silu 48.5 (64 + 5) for 5 rows, 56 (54 + 5) for 64, 68 (57 + 5) for 128
-// Above 64 rows every wave reads all of x from LDS for 16 weight rows, and LDS is the
-// bound where K is not split far.
+// Measured in graphs, weights out of cache, us with the weights through registers and now:
+//   PART  4096 x 4096   5 rows 8.5, 8.1   40 rows 10.0, 8.7   96 14.3, 11.0     6144 x 4096   5 rows 11.6, 11.1   64 15.9, 12.9
+//     4096 x 14336   5 rows 23.7, 23.3   40 26.4, 24.9   96 35.0, 30.6     2048 x 8192   16 rows 9.2, 8.6   128 16.6, 12.4
+//     2048 x 2048   5 rows 3.9, 4.3   128 7.4, 6.2
+//   SILU  28672 x 4096   5 rows 51.0, 41.0   64 55.7, 42.7   128 69.2, 50.0 (library and activation 60.2)
+//     16384 x 2048   1 row 17.6, 13.5   40 20.1, 13.7   96 29.2, 16.4 (22.3)
+//   F32   32000 x 4096   5 rows 54.6, 44.8 (library 59.9)   128 76.8, 59.8 (65.4)     128256 x 4096   1 row 202.7, 176.9 (188.7)
+// and against the library above 128 rows:
+//   PART  4096 x 4096   192 rows 32.8, 14.6   256 23.3, 17.5   384 25.2, 22.6     4096 x 14336   192 103, 39.4   384 82.4, 55.6
+//   SILU  28672 x 4096   160 rows 63.4, 53.5   256 72.6, 63.5     16384 x 2048   192 31.1, 22.3   256 35.3, 25.8
 
-#include "common.h"
+#include <atomic>
 
-typedef __bf16 bf16x8_mfma __attribute__((ext_vector_type(8)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-#define LR_KC 128          // k depth of a chunk
-#define LR_STEPS 4         // matrix steps (32 k) of a chunk
+#include "tile_product.h"
 
 enum LinearForm { LR_PART = 0, LR_BF16 = 1, LR_F32 = 2, LR_SILU = 3, LR_CLAMPED = 4 };
 
-union LrFrag {
-  u32x4 u;
-  bf16x8_mfma m;
-};
-
-template <int MT, int FORM, int WAVES, int DEEP, bool AHEAD>
-__global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(
-    void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-    const bf16_t* __restrict__ bias, int M, int N, int K, int x_stride, int chunks_per_split, float limit, float alpha) {
-  __shared__ __attribute__((aligned(16))) u32x4 xs[2][MT * 256];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = lane & 15, grp = lane >> 4;
-  const int nchunks = K / LR_KC;
-  const int c_begin = blockIdx.y * chunks_per_split;
-  const int c_end = min(nchunks, c_begin + chunks_per_split);
-  // weight row of this wave's tile; gated: the first half of the waves hold gate rows, the others the up rows of
-  // the same columns
-  constexpr int HW = WAVES / 2;
+// Workgroups by share of k, then by rows of W, then by rows of x: those of an XCD have the same part of x in its L2, and
+// the row tiles of a part of W run side by side.
+template <int NI, int MJ, int FORM, int KB>
+__global__ void __launch_bounds__(TP_THREADS, 1) linear_rows_kernel(
+    void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const bf16_t* __restrict__ bias,
+    int M, int N, int K, int x_stride, int m_tiles, int splits, float limit, float alpha) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr bool GATED = FORM == LR_SILU || FORM == LR_CLAMPED;
-  const int n0 = GATED ? (wave / HW) * (N / 2) + blockIdx.x * (16 * HW) + (wave % HW) * 16
-                                 : blockIdx.x * (16 * WAVES) + wave * 16;
-  const char* wrow = (const char*)(w + (int64_t)min(n0 + col, N - 1) * K) + grp * 32;
-
-  f32x4 acc[MT];
+  constexpr int BN = GATED ? 16 * NI : 32 * NI;    // columns of the result
+  const int columns = GATED ? N / 2 : N;
+  const int n_tiles = (columns + BN - 1) / BN, all = n_tiles * splits * m_tiles, xcd = blockIdx.x & 7;
+  const int begin = (int)((int64_t)all * xcd >> 3), items = (int)((int64_t)all * (xcd + 1) >> 3) - begin;
+  const int at = blockIdx.x >> 3;
+  if (at >= items) return;
+  const int item = begin + at, rest = item / m_tiles, share = rest / n_tiles, n0 = rest % n_tiles * BN;
+  const int rows = (M + m_tiles - 1) / m_tiles;    // even parts
+  const int m0 = item % m_tiles * rows, m_end = min(M, m0 + rows);
+  const uint32_t stages_all = K / TP_K, first = stages_all * share / splits;      // both far below 2^16
+  const int stages = (int)(stages_all * (share + 1) / splits - first);
+  const int64_t k0 = (int64_t)first * TP_K;
+  const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  f32x4 acc[NI][MJ];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  u32x4 wr[DEEP][LR_STEPS];
-  constexpr int XP = MT * 4 / WAVES;      // passes of a chunk's x over the threads
-  static_assert(XP >= 1, "as many 16-byte units as threads");
-  constexpr int XD = AHEAD ? DEEP : 1;    // chunks of x in registers
-  u32x4 xr[XD][XP];
-  auto load_w = [&](int c, int slot, int st) {
-    wr[slot][st] = *reinterpret_cast<const u32x4*>(wrow + (int64_t)c * (LR_KC * 2) + (st >> 1) * 128 + (st & 1) * 16);
-  };
-  // row tid / 16 of each pass, 16-byte unit tid % 16
-  const int xrow = tid >> 4, xunit = tid & 15;
-  auto load_x = [&](int c, int slot) {
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int i = 0; i < XP; ++i)
-      xr[slot][i] = *reinterpret_cast<const u32x4*>((const char*)(x + (int64_t)min(i * 4 * WAVES + xrow, M - 1) * x_stride) +
-                                              (int64_t)c * (LR_KC * 2) + xunit * 16);
-  };
-  auto store_x = [&](int buf, int slot) {
+    for (int j = 0; j < MJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const TileRows xr(x + k0, m0 + wave * MJ * 8, m_end, MJ * 8, x_stride, lane);
+  // W rows of a gated tile: 8 * NI gate, the same of up, the next gate, their up
+  const int n_put = GATED ? n0 + (wave >> 1) * (8 * NI) : n0 + wave * (8 * NI);
+  const TileRows wr(w + (GATED ? (int64_t)(wave & 1) * columns : 0) * K + k0, n_put, columns, 8 * NI, K, lane);
+  // the XCDs begin at different k: rows of a power of two of bytes would have all of them at the same memory channels
+  tile_product<MJ, NI, KB * 1024>(acc, wr, xr, stages, stages * xcd / 8, smem);
+  if constexpr (FORM == LR_SILU && MJ > 4) {       // many rows: whole lines
+    const int m = m0 + (wave & 1) * MJ * 16, n = n0 + (wave >> 1) * (BN / 2);
+    tile_store<NI / 2, MJ>((bf16_t*)out + (int64_t)m * columns + n, columns, m_end - m, columns - n, smem, [&](int i, int j) {
+      float v[4];
 #pragma unroll
-    for (int i = 0; i < XP; ++i) xs[buf][(i * 4 * WAVES + xrow) * 16 + (xunit ^ (xrow & 15))] = xr[slot][i];
-  };
-
-  if (c_begin < c_end) {
-#pragma unroll
-    for (int u = 0; u < DEEP; ++u)
-      if (c_begin + u < c_end) {
-        if (u < XD) load_x(c_begin + u, u);
-#pragma unroll
-        for (int st = 0; st < LR_STEPS; ++st) load_w(c_begin + u, u, st);
+      for (int r = 0; r < 4; ++r) {
+        const float g = acc[i][j][r];
+        v[r] = g / (1.0f + __expf(-g)) * acc[i + NI / 2][j][r];
       }
-    store_x(0, 0);
-    __syncthreads();
-    for (int c = c_begin; c < c_end; c += DEEP) {
-#pragma unroll
-      for (int u = 0; u < DEEP; ++u) {
-        if (c + u < c_end) {
-          const bool next = c + u + 1 < c_end;
-          if (!AHEAD && next) load_x(c + u + 1, 0);
-#pragma unroll
-          for (int st = 0; st < LR_STEPS; ++st) {
-            LrFrag a;
-            a.u = wr[u][st];
-#pragma unroll
-            for (int i = 0; i < MT; ++i) {
-              LrFrag b;
-              b.u = xs[u & 1][i * 256 + col * 16 + (((st >> 1) * 8 + grp * 2 + (st & 1)) ^ col)];
-              acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, b.m, acc[i], 0, 0, 0);
-            }
-          }
-          if (c + u + DEEP < c_end) {
-            if constexpr (AHEAD) load_x(c + u + DEEP, u);
-#pragma unroll
-            for (int st = 0; st < LR_STEPS; ++st) load_w(c + u + DEEP, u, st);
-          }
-          if (next) store_x(1 - (u & 1), (u + 1) % XD);
-          __syncthreads();
-        }
-      }
-    }
+      return tp_pack(v[0], v[1], v[2], v[3]);
+    });
+    return;
   }
-
-  // lane (col, grp): rows n0 + grp*4 .. +3 of the weights, row i*16 + col of x
-  const int n = n0 + grp * 4;
-  if constexpr (GATED) {
-    float* up = reinterpret_cast<float*>(&xs[0][0]);   // [HW waves][MT*16 rows][16]
-    static_assert(HW * MT * 16 * 16 * 4 <= sizeof(xs), "the up halves fit the staging buffers");
-    if (wave >= HW) {
+  const int m = m0 + (wave & 1) * MJ * 16 + col, n = n0 + (wave >> 1) * (BN / 2) + grp * 4;
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
-        *reinterpret_cast<f32x4*>(up + (((wave - HW) * MT + i) * 16 + col) * 16 + grp * 4) = acc[i];
-    }
-    __syncthreads();
-    if (wave < HW) {
+  for (int j = 0; j < MJ; ++j) {
+    const int mr = m + j * 16;
+    if (mr >= m_end) continue;
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int m = i * 16 + col;
-        const f32x4 u = *reinterpret_cast<const f32x4*>(up + ((wave * MT + i) * 16 + col) * 16 + grp * 4);
-        bf16x4_vec o;
+    for (int i = 0; i < (GATED ? NI / 2 : NI); ++i) {
+      const int nc = n + i * 16;
+      if (nc >= columns) continue;
+      if constexpr (GATED) {
+        float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
+          const float g = acc[i][j][r], u = acc[i + NI / 2][j][r];
           if constexpr (FORM == LR_SILU) {
-            // rounded as the separate product's result is
-            const float g = bf16_to_f32(f32_to_bf16(acc[i][r])), v = bf16_to_f32(f32_to_bf16(u[r]));
-            o[r] = f32_to_bf16(g / (1.0f + __expf(-g)) * v);
+            v[r] = g / (1.0f + __expf(-g)) * u;
           } else {
-            const float g = fminf(acc[i][r], limit), v = fminf(fmaxf(u[r], -limit), limit);
-            o[r] = f32_to_bf16(g * (1.0f / (1.0f + expf(-alpha * g))) * (v + 1.0f));
+            const float gc = fminf(g, limit), uc = fminf(fmaxf(u, -limit), limit);
+            v[r] = gc * (1.0f / (1.0f + expf(-alpha * gc))) * (uc + 1.0f);
           }
         }
-        if (m < M) *reinterpret_cast<bf16x4_vec*>((short*)out + (int64_t)m * (N / 2) + n) = o;
-      }
-    }
-  } else {
-    if (n >= N) return;
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int m = i * 16 + col;
-      if (m >= M) continue;
-      if constexpr (FORM == LR_PART) {
-        *reinterpret_cast<f32x4*>((float*)out + ((int64_t)blockIdx.y * M + m) * N + n) = acc[i];
-      } else if constexpr (FORM == LR_F32) {
-        *reinterpret_cast<f32x4*>((float*)out + (int64_t)m * N + n) = acc[i];
-      } else {
+        *reinterpret_cast<bf16x4_vec*>((short*)out + (int64_t)mr * columns + nc) = tp_pack(v[0], v[1], v[2], v[3]);
+      } else if constexpr (FORM == LR_BF16) {
         bf16x4_vec o;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          o[r] = f32_to_bf16(acc[i][r] + (bias ? bf16_to_f32(((const short*)bias)[n + r]) : 0.0f));
-        *reinterpret_cast<bf16x4_vec*>((short*)out + (int64_t)m * N + n) = o;
+        for (int r = 0; r < 4; ++r) o[r] = f32_to_bf16(acc[i][j][r] + (bias ? bf16_to_f32(((const short*)bias)[nc + r]) : 0.0f));
+        *reinterpret_cast<bf16x4_vec*>((short*)out + (int64_t)mr * N + nc) = o;
+      } else {
+        *reinterpret_cast<f32x4*>((float*)out + ((int64_t)share * M + mr) * N + nc) = acc[i][j];
       }
     }
   }
 }
 
-// Waves of a workgroup. Eight halve the reads of x, which at 128 rows and 64 weight rows
-// a workgroup are twice the weights' bytes; they pay where the weights still make enough
-// workgroups. us with four and eight waves, weights out of cache:
-//   PART, 65 / 96 / 128 rows   2048 x 2048  6.3 7.6 / 6.7 8.1 / 7.2 8.9     3072 x 2048  8.4 8.3 / 9.3 9.1 / 10.1 10.2
-//     3072 x 8192  21.7 20.8 / 24.0 22.4 / 26.1 24.5     4096 x 4096  13.6 13.2 / 15.5 14.2 / 16.6 15.6
-//     6144 x 4096  20.0 18.2 / 21.6 19.6 / 22.6 20.7     8192 x 8192  42.4 40.9 / 44.3 41.9 / 46.2 43.5
-//   SILU, 33 / 64 rows   16384 x 2048  22.6 27.0 / 23.0 27.6     16384 x 4096  46.9 51.1 / 46.8 52.2
-//     22016 x 4096  55.5 53.2 / 57.9 54.7     24576 x 3072  41.7 41.5 / 44.8 43.5     28672 x 4096  58.3 60.4 / 61.6 60.5
-//   F32, 33 / 64 rows   16384 x 2048  21.8 26.3 / 22.4 27.6     24576 x 4096  53.6 54.3 / 57.1 56.6
-//     50304 x 2048  56.9 52.0 / 61.3 54.5     128256 x 4096  217.9 220.3 / 240.5 232.5
-// From 200 workgroups of eight waves on (N = 25600) neither side loses more than 4 %; a line at 20000 would gain the
-// sizes between 3 - 6 %.
-static int linear_rows_waves(int M, int N, int form) {
-  if (N % 128 != 0) return 4;
-  return (form == LR_PART ? M > 64 && N >= 4096 : M > 32 && N >= 200 * 128) ? 8 : 4;
-}
+#define LR_UNITS 256       // compute units
 
-extern "C" void launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
-                                   int K, int x_stride, int form, int splits, float limit, float alpha,
-                                   hipStream_t stream) {
-  const int per = (K / LR_KC + splits - 1) / splits;
-  const int waves = linear_rows_waves(M, N, form);
-  const dim3 grid((N + 16 * waves - 1) / (16 * waves), splits);
-#define LR_GO(MT, F, WV, DEEP)                                                                                        \
-  hipLaunchKernelGGL((linear_rows_kernel<MT, F, WV, DEEP, (MT <= 4)>), grid, dim3(64 * WV), 0, stream, out, x, w, bias, M, \
-                     N, K, x_stride, per, limit, alpha)
-#define LR_FORM(MT, WV, DEEP)                                \
-  switch (form) {                                            \
-    case LR_PART: LR_GO(MT, LR_PART, WV, DEEP); break;       \
-    case LR_BF16: LR_GO(MT, LR_BF16, WV, DEEP); break;       \
-    case LR_F32: LR_GO(MT, LR_F32, WV, DEEP); break;         \
-    case LR_CLAMPED: LR_GO(MT, LR_CLAMPED, WV, DEEP); break; \
-    default: LR_GO(MT, LR_SILU, WV, DEEP); break;            \
+// Tiles of a product: rows of W 32 * ni, rows of x 32 * mj in m_tiles parts, KB of LDS (80: two workgroups to a compute
+// unit, whose streams fill each other's beginnings and ends).
+struct LinearPlan {
+  int ni, mj, m_tiles, kb;
+};
+
+// Up to 128 rows one part of x, so that W is read once; above, two or more read it from the L2 where the splits they
+// replace would cost more in sums (4096 x 4096, 384 rows, with the sums' reading: four parts in two splits 25.1 us, one in
+// eight above 30). 64 rows of W to a tile where 128 would leave half of the compute
+// units idle (4096 x 4096, 5 rows: 8.0 us, 8.4; silu 16384 x 2048 13.5, 15.2; but 18432 x 4096, 144 tiles of 128 rows, 35.2,
+// 30.7) or make more workgroups than there are (silu 37888 x 3584, 16 rows: 57, 64); 128 of a long matrix at many rows of x,
+// whose reading by all of them weighs more (4096 x 14336, 128 rows: 40.8 us with the sums' reading, 37.9).
+static LinearPlan linear_plan(int M, int N, int K, int form) {
+  LinearPlan p;
+  const bool gated = form == LR_SILU || form == LR_CLAMPED;
+  if (M <= 128) {
+    p.m_tiles = 1;
+    p.mj = (M + 31) / 32;
+    if (form == LR_PART)
+      p.ni = N >= 5120 || (p.mj == 4 && N >= 4096 && K >= 8192) ? 4 : 2;
+    else if (gated)
+      p.ni = N <= 256 * 64 || (N > 256 * 128 && p.mj == 1) ? 2 : 4;
+    else
+      p.ni = p.mj > 1 && N >= 192 * 128 ? 4 : 2;
+  } else {
+    p.ni = 4;
+    p.m_tiles = gated ? (N > 256 * 64 ? 1 : 2) : N >= 4096 ? 2 : (M + 95) / 96;
+    p.mj = ((M + p.m_tiles - 1) / p.m_tiles + 31) / 32;
   }
-  if (M <= 16) { LR_FORM(1, 4, 4); }
-  else if (M <= 32) { LR_FORM(2, 4, 4); }
-  else if (waves == 8 && M <= 64) { LR_FORM(4, 8, 2); }
-  else if (waves == 8) { LR_FORM(8, 8, 2); }
-  else if (M <= 64) { LR_FORM(4, 4, 2); }
-  else { LR_FORM(8, 4, 2); }
-#undef LR_FORM
-#undef LR_GO
+  p.kb = p.ni == 2 || p.mj <= 2 ? 80 : 160;
+  return p;
 }
 
-// splits of k for the PART form: about 800 workgroups, 512 (256 of eight waves) where
-// the rows' sums weigh more (M > 32), and two chunks at least
+// room for the kernel's LDS; the attribute is asked for once a device
+static bool lr_lds_ready(const void* kernel, std::atomic<uint64_t>& devices) {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return false;
+  const uint64_t bit = 1ull << (device & 63);
+  if (device < 64 && (devices.load(std::memory_order_relaxed) & bit)) return true;
+  if (!tp_lds_ready(kernel)) return false;
+  if (device < 64) devices.fetch_or(bit, std::memory_order_relaxed);
+  return true;
+}
+
+template <int NI, int MJ, int FORM, int KB>
+static int linear_rows_go(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N, int K, int x_stride,
+                          int m_tiles, int splits, float limit, float alpha, hipStream_t stream) {
+  static std::atomic<uint64_t> devices{0};
+  if (!lr_lds_ready(reinterpret_cast<const void*>(linear_rows_kernel<NI, MJ, FORM, KB>), devices)) return -1;
+  constexpr int LDS = TileRing<MJ, NI, KB * 1024>::STRIDE * TileRing<MJ, NI, KB * 1024>::RING;
+  const int64_t all = (int64_t)((N + 32 * NI - 1) / (32 * NI)) * splits * m_tiles;
+  hipLaunchKernelGGL((linear_rows_kernel<NI, MJ, FORM, KB>), dim3((all + 7) / 8 * 8), dim3(TP_THREADS), LDS, stream, out, x, w, bias,
+                     M, N, K, x_stride, m_tiles, splits, limit, alpha);
+  return 0;
+}
+
+template <int FORM>
+static int linear_rows_form(const LinearPlan& p, void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
+                            int K, int x_stride, int splits, float limit, float alpha, hipStream_t stream) {
+#define LR_CASE(NI, MJ)                                                                                              \
+  if (p.ni == NI && p.mj == MJ)                                                                                      \
+    return linear_rows_go<NI, MJ, FORM, (NI == 2 || MJ <= 2 ? 80 : 160)>(out, x, w, bias, M, N, K, x_stride, p.m_tiles, splits, limit, \
+                                                                         alpha, stream)
+  LR_CASE(2, 1);
+  LR_CASE(2, 2);
+  LR_CASE(2, 3);
+  LR_CASE(2, 4);
+  LR_CASE(4, 1);
+  LR_CASE(4, 2);
+  LR_CASE(4, 3);
+  LR_CASE(4, 4);
+  if constexpr (FORM == LR_PART || FORM == LR_SILU) {
+    LR_CASE(4, 5);
+    LR_CASE(4, 6);
+  }
+  if constexpr (FORM == LR_SILU) {
+    LR_CASE(4, 7);
+    LR_CASE(4, 8);
+  }
+#undef LR_CASE
+  return -1;
+}
+
+// Rows up to which a form is taken
+extern "C" int linear_rows_most(int form) { return form == LR_PART ? 384 : form == LR_SILU ? 256 : 128; }
+
+// 0, or -1 where the LDS cannot be had
+extern "C" int launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N, int K,
+                                  int x_stride, int form, int splits, float limit, float alpha, hipStream_t stream) {
+  const LinearPlan p = linear_plan(M, N, K, form);
+#define LR_FORM(F) \
+  case F: return linear_rows_form<F>(p, out, x, w, bias, M, N, K, x_stride, splits, limit, alpha, stream)
+  switch (form) {
+    LR_FORM(LR_PART);
+    LR_FORM(LR_BF16);
+    LR_FORM(LR_F32);
+    LR_FORM(LR_SILU);
+    LR_FORM(LR_CLAMPED);
+  }
+#undef LR_FORM
+  return -1;
+}
+
+// splits of k for the PART form: one workgroup for each compute unit, and four stages of 64 at least
 extern "C" int linear_rows_splits(int M, int N, int K) {
-  const int waves = linear_rows_waves(M, N, LR_PART);
-  const int tiles = (N + 16 * waves - 1) / (16 * waves), chunks = K / LR_KC;
-  int s = ((M <= 32 ? 800 : 2048 / waves) + tiles / 2) / tiles;
-  s = s < chunks / 2 ? s : chunks / 2;
-  return s < 1 ? 1 : s;
+  const LinearPlan p = linear_plan(M, N, K, LR_PART);
+  const int tiles = (N + 32 * p.ni - 1) / (32 * p.ni) * p.m_tiles, most = K / TP_K / 4;
+  const int s = (LR_UNITS + 8) / tiles;
+  return s < 1 || most < 1 ? 1 : s < most ? s : most;
 }

@@ -28,7 +28,7 @@ void seq_launch_gated_delta_rule(float*, const void*, const void*, const void*, 
                                  int, int, int, float*, hipStream_t);
 void seq_launch_gated_act(void*, const void*, const void*, int64_t, int, int, float, float, float, int, hipStream_t);
 // few-row products and paged decode attention (ops/hip/linear_rows.hip, attn_decode.hip, also part of kllms_amd._C)
-void launch_linear_rows(void*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
+int launch_linear_rows(void*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
                         int, int, float, float, hipStream_t);
 int linear_rows_splits(int, int, int);
 int attn_decode_splits(int, int, int);
@@ -42,6 +42,7 @@ using torch::Tensor;
 namespace {
 
 enum { ROWS_PART = 0, ROWS_BF16 = 1, ROWS_CLAMPED = 4 };   // forms of linear_rows
+constexpr const char* NO_LDS = "160 KB of LDS are not available";
 
 inline hipStream_t cur_stream() { return at::hip::getCurrentHIPStream().stream(); }
 
@@ -71,15 +72,15 @@ void check_weight(const Tensor& w, int64_t K, const char* name) {
 Tensor part(const Tensor& x, const Tensor& w, int T, hipStream_t st) {
   const int K = w.size(1), N = w.size(0), S = linear_rows_splits(T, N, K);
   auto out = torch::empty({S, T, N}, x.options().dtype(torch::kFloat));
-  launch_linear_rows(out.data_ptr(), bf(x), bf(w), nullptr, T, N, K, K, ROWS_PART, S, 0.0f, 0.0f, st);
+  TORCH_CHECK(launch_linear_rows(out.data_ptr(), bf(x), bf(w), nullptr, T, N, K, K, ROWS_PART, S, 0.0f, 0.0f, st) == 0, NO_LDS);
   return out;
 }
 
 Tensor rows_bf16(const Tensor& x, const Tensor& w, const Tensor& bias, int T, hipStream_t st) {
   const int K = w.size(1), N = w.size(0);
   auto out = torch::empty({T, N}, x.options());
-  launch_linear_rows(out.data_ptr(), bf(x), bf(w), bias.numel() ? bf(bias) : nullptr, T, N, K, K, ROWS_BF16, 1, 0.0f, 0.0f,
-                     st);
+  TORCH_CHECK(launch_linear_rows(out.data_ptr(), bf(x), bf(w), bias.numel() ? bf(bias) : nullptr, T, N, K, K, ROWS_BF16, 1, 0.0f,
+                                 0.0f, st) == 0, NO_LDS);
   return out;
 }
 
@@ -238,9 +239,10 @@ std::optional<Tensor> hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::ve
 }
 
 // Whether the gated product of T rows is the few-row kernel's, which has the activation in it, or the library's and a pass
-// behind it. us of the one and the other by T, w_in of 16384 x 2048: 16 18, 21   64 22, 22   65 30, 23   128 31, 25; 28672 x 4096: 16
-// 52, 70   32 55, 58   40 62, 57   128 75, 61; 22016 x 4096: 16 48, 58   32 52, 47; 57344 x 8192: 1 194, 180   16 192, 185
-static bool glu_on_rows(int T, int64_t n) { return T <= 16 ? n < 1 << 28 : T <= 32 ? n < 1 << 27 : T <= 64 && n <= 1 << 26; }
+// behind it. us of the one and the other by T, w_in of 16384 x 2048: 1 13.8, 19.6   64 15.2, 20.6   128 18.8, 23.6; 28672 x 4096: 16
+// 41.6, 62.8   128 50.9, 57.5; 57344 x 8192: 16 166, 186   128 197, 203; of other widths than powers of two the stages take a
+// third longer at many rows: 27648 x 5120 16 57, 82   64 62, 60   128 85, 70; 24576 x 3072 96 41, 39   128 49, 43
+static bool glu_on_rows(int T, int K) { return T <= 64 || (K & (K - 1)) == 0; }
 
 // The same of a clamped gated-linear-unit sublayer, w_in = [gate; up]
 std::optional<Tensor> hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_down, Tensor w_post, Tensor w_next, double limit,
@@ -255,9 +257,9 @@ std::optional<Tensor> hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_
   r.norm(w_post, "w_post"); r.norm(w_next, "w_next");
   auto st = cur_stream();
   auto act = torch::empty({r.T, N / 2}, h.options());
-  if (glu_on_rows(r.T, w_in.numel())) {
-    launch_linear_rows(act.data_ptr(), bf(h), bf(w_in), nullptr, r.T, N, r.W, r.W, ROWS_CLAMPED, 1, (float)limit,
-                       (float)alpha, st);
+  if (glu_on_rows(r.T, r.W)) {
+    TORCH_CHECK(launch_linear_rows(act.data_ptr(), bf(h), bf(w_in), nullptr, r.T, N, r.W, r.W, ROWS_CLAMPED, 1, (float)limit,
+                                   (float)alpha, st) == 0, NO_LDS);
   } else {
     const Tensor y = at::linear(h, w_in);
     seq_launch_gated_act(act.data_ptr(), y.data_ptr(), bf(y, N / 2), r.T, N / 2, N, (float)limit, (float)alpha, 1.0f, 0, st);

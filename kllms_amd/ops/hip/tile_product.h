@@ -23,11 +23,16 @@
 // what eight waves of 128 x 64 need, and all 512 registers: 256 sums, 2 x 64 fragments.
 //
 // Small MJ are for the ends of ragged row ranges and for few rows, where the stream of W
-// is the bound: less matrix work per stage, and more buffers of it in flight.
+// is the bound: less matrix work per stage, and more buffers of it in flight. So are NI of 2 and 4, tiles of 64 and 128
+// rows of W for products that it bounds from end to end (linear_rows.hip). One loop for all of their stages: with the last
+// ones in a loop of their own, without copies, the sums moved between registers in every stage (28672 x 4096, 256 rows:
+// 82 us; 64 so).
 
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -108,6 +113,12 @@ struct TileRows {
       at[i] = (uint32_t)(i * 8 + (lane >> 3)) * K * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
   }
   __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds) const { tp_copy(range, at[i], k_off, lds); }
+  // zeros, without a look at memory, where not ``live``
+  __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds, bool live) const {
+    u32x4 r = range;
+    r[2] = live ? r[2] : 0;
+    tp_copy(r, at[i], k_off, lds);
+  }
 };
 
 // Rows anywhere: at[i] is the address of this lane's 16 bytes of the i-th copy in stage 0.
@@ -117,67 +128,78 @@ struct TileGather {
   __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds) const { tp_copy_at(at[i] + k_off, lds); }
 };
 
-template <int MJ>
+template <int MJ, int NI = 8, int BYTES = TP_LDS>
 struct TileRing {
-  static constexpr int STRIDE = (TP_N + 32 * MJ) * 128;   // W rows, then X rows
-  static constexpr int RING = TP_LDS / STRIDE < 4 ? TP_LDS / STRIDE : 4;
+  static constexpr int STRIDE = (32 * NI + 32 * MJ) * 128;   // W rows, then X rows
+  static constexpr int MOST = NI == 8 ? 4 : 8;
+  static constexpr int RING = BYTES / STRIDE < MOST ? BYTES / STRIDE : MOST;
 };
 
-// acc += W X^T over K; w: this wave's 64 of the 256 rows, x: its 8 * MJ of the 32 * MJ. Ends with all waves past
-// their last LDS read.
-template <int MJ, class X>
-__device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows& w, const X& x, int stages, int start,
+// acc += W X^T over K; w: this wave's 8 * NI of the 32 * NI rows (64 of 256), x: its 8 * MJ of the 32 * MJ. Ends with all
+// waves past their last LDS read. NI 4, tiles of 128 columns, is for few rows: half the sums, more buffers in flight.
+template <int MJ, int NI = 8, int BYTES = TP_LDS, class X>
+__device__ __forceinline__ void tile_product(f32x4 (&acc)[NI][MJ], const TileRows& w, const X& x, int stages, int start,
                                              char* smem) {
-  constexpr int STRIDE = TileRing<MJ>::STRIDE, RING = TileRing<MJ>::RING;
-  constexpr int F = 8 * MJ;              // matrix instructions of a half
-  constexpr int NR = 8 + MJ;             // LDS reads of a half
-  constexpr int ND = 8 + MJ;             // copies of a stage
+  constexpr int STRIDE = TileRing<MJ, NI, BYTES>::STRIDE, RING = TileRing<MJ, NI, BYTES>::RING;
+  constexpr int G = NI * MJ;             // matrix instructions of a half
+  constexpr int NR = NI + MJ;            // LDS reads of a half
+  constexpr int ND = NI + MJ;            // copies of a stage
+  constexpr int F = G > NR + 3 ? G : NR + 3;   // places for them, the reads and the copies
+  constexpr int BOTH = NI < MJ ? NI : MJ;   // reads and copies go by turns while both operands have some
   constexpr int RS = F / (2 * NR) > 0 ? F / (2 * NR) : 1;
-  constexpr int P1 = RS * NR + (MJ >= 4 ? 8 : 4);   // first half: all has been read
+  constexpr int P1 = RS * NR + (NI < 8 ? (F - RS * NR) / 2 : MJ >= 4 ? 8 : 4);   // first half: all has been read
   constexpr int DS = (2 * F - P1) / ND;             // a copy every DS instructions from there on
   constexpr int D1 = (F - 1 - P1) / DS + 1;         // copies in the first half
+  constexpr bool LEAN = NI < 8;          // few stages: what is behind the last is out of the copies' range, and not read
   static_assert(P1 < F && DS >= 1 && RING >= 2 && (RING - 1) * ND < 64);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, grp = lane >> 4;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
-  const uint32_t w_put = lds0 + wave * 64 * 128, x_put = lds0 + TP_N * 128 + wave * MJ * 1024;
+  const uint32_t w_put = lds0 + wave * NI * 1024, x_put = lds0 + NI * 4096 + wave * MJ * 1024;
   uint32_t w_get[2], x_get[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     const uint32_t o = lds0 + col * 128 + (((ks * 4 + grp) ^ (col & 7)) << 4);
-    w_get[ks] = o + (wave >> 1) * 128 * 128;
-    x_get[ks] = o + TP_N * 128 + (wave & 1) * MJ * 16 * 128;
+    w_get[ks] = o + (wave >> 1) * NI * 16 * 128;
+    x_get[ks] = o + NI * 4096 + (wave & 1) * MJ * 16 * 128;
   }
   typedef __attribute__((address_space(3))) const bf16x8_mfma* lds_ptr;
   auto get = [](uint32_t at) { return *(lds_ptr)(uintptr_t)at; };
+  bool live = true;                      // the stage that is copied exists
   auto put = [&](int d, uint32_t k_off, uint32_t buf) {   // d-th copy of a stage
-    const int i = d < 2 * MJ ? d >> 1 : d - MJ;
-    if (d < 2 * MJ && (d & 1)) x.copy(i, k_off, x_put + buf + i * 1024);
-    else w.copy(i, k_off, w_put + buf + i * 1024);
+    const int i = d < 2 * BOTH ? d >> 1 : d - BOTH;
+    if constexpr (LEAN) {
+      if (d < 2 * BOTH ? d & 1 : MJ > NI) x.copy(i, k_off, x_put + buf + i * 1024, live);
+      else w.copy(i, k_off, w_put + buf + i * 1024, live);
+    } else {
+      if (d < 2 * BOTH ? d & 1 : MJ > NI) x.copy(i, k_off, x_put + buf + i * 1024);
+      else w.copy(i, k_off, w_put + buf + i * 1024);
+    }
   };
   auto k_at = [&](int t) {               // of the t-th stage in work; behind the last one, that one's
     const int i = min(t, stages - 1) + start;
     return (uint32_t)(i < stages ? i : i - stages) * 128;
   };
-  bf16x8_mfma a[2][8], b[2][MJ];
+  bf16x8_mfma a[2][NI], b[2][MJ];
   auto read = [&](int ks, int r, uint32_t buf) {
-    if (r < 2 * MJ && !(r & 1)) b[ks][r >> 1] = get(x_get[ks] + buf + (r >> 1) * 2048);
-    else {
-      const int i = r < 2 * MJ ? r >> 1 : r - MJ;
-      a[ks][i] = get(w_get[ks] + buf + i * 2048);
-    }
+    const int i = r < 2 * BOTH ? r >> 1 : r - BOTH;
+    if (r < 2 * BOTH ? !(r & 1) : MJ > NI) b[ks][i] = get(x_get[ks] + buf + i * 2048);
+    else a[ks][i] = get(w_get[ks] + buf + i * 2048);
   };
   auto multiply = [&](int ks, int f) {
+    if (f >= G) return;
     const int i = f / MJ, j = f % MJ;
     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][i], b[ks][j], acc[i][j], 0, 0, 0);
     if (f & 1) TP_HOLD;
   };
 
 #pragma unroll
-  for (int t = 0; t < RING; ++t)         // of fewer stages the last one again: the counts below stand
+  for (int t = 0; t < RING; ++t) {       // of fewer stages the last one again: the counts below stand
+    live = t < stages;
 #pragma unroll
     for (int d = 0; d < ND; ++d) put(d, k_at(t), t * STRIDE);
+  }
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"((RING - 1) * ND) : "memory");
 #pragma unroll
   for (int r = 0; r < NR; ++r) read(0, r, 0);
@@ -187,6 +209,7 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows
   for (int s = 0; s < stages; ++s) {
     // behind the last stage that one is copied again and nothing of it used: no branches
     const uint32_t k_off = k_at(s + RING);
+    live = s + RING < stages;
     TP_HOLD;
 #pragma unroll
     for (int f = 0; f < F; ++f) {
@@ -213,7 +236,7 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[8][MJ], const TileRows
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   // what follows reads sums out of the accumulation registers; it is held off the loop, which must not move them
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < MJ; ++j) asm volatile("" : "+a"(acc[i][j]));
 }

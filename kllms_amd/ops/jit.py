@@ -57,7 +57,7 @@ def module_path(name: str) -> str:
 def source_digest(name: str) -> str:
     ext = EXTENSIONS[name]
     h = hashlib.sha256(" ".join(HIP_FLAGS).encode())
-    shared = ["../common.h"] if any(f.startswith("../") for f in ext["kernels"]) else []
+    shared = ["../common.h", "../tile_product.h"] if any(f.startswith("../") for f in ext["kernels"]) else []
     for f in ext["headers"] + shared + ext["kernels"] + ext["bindings"]:
         with open(os.path.join(ext["dir"], f), "rb") as fh:
             h.update(f.encode() + b"\0" + fh.read())

@@ -423,3 +423,73 @@ def test_decode_step_takes_32_bit_ids():
     with torch.inference_mode():
         want, got = (eng.model.forward_decode((rows + 5).to(t), batch) for t in (torch.long, torch.int32))
     assert float(((got - want).norm(dim=-1) / want.norm(dim=-1)).max()) < 0.03     # bf16 through two layers, two sets of kernels
+
+
+@pytest.mark.parametrize("M", [1, 31, 32, 33, 96, 97, 129, 192, 193, 256, 257, 384])
+@pytest.mark.parametrize("N,K,splits", [(16, 128, 1), (80, 128, 2), (4112, 640, 5), (5136, 1152, 17), (2064, 4224, 3), (4096, 8192, 0)])
+def test_linear_rows_tiles_and_splits(M, N, K, splits):
+    """Tiles of 64 and 128 rows of W with a ragged last one, parts of x of uneven length, fewer stages than buffers, splits
+    of uneven length, one stage each at most."""
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(N, K, generator=g) * 0.05).bfloat16().to(DEV)
+    ref = x.double() @ w.double().t()
+    tol = K * 2 ** -24 * (x.double().abs() @ w.double().abs().t())
+    part = ops._hip_or_raise().linear_rows(x, w, ops._none(x), 0, splits)
+    assert splits == 0 or part.shape[0] == min(splits, K // 64)
+    assert ((part.double().sum(0) - ref).abs() <= tol).all()
+    if M <= 256 and N % 64 == 0:
+        gate, up = ref.chunk(2, -1)
+        tg, tu = tol.chunk(2, -1)
+        full = torch.nn.functional.silu(gate) * up
+        # the sums' error through silu(g) * u (slope below 1.1 in g), a fast exponential, the result's rounding
+        assert ((ops.linear_silu_rows(x, w).double() - full).abs()
+                <= 1.1 * tg * (up.abs() + tu) + tu * gate.abs() + 2 ** -8 * full.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("N", [128, 192, 16320, 16448, 20544, 32896])
+@pytest.mark.parametrize("M", [5, 40, 128, 129, 256])
+def test_gated_rows_at_the_lines_of_their_tiles(M, N):
+    K = 256
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(N, K, generator=g) * 0.05).bfloat16().to(DEV)
+    ref = x.double() @ w.double().t()
+    gate, up = ref.chunk(2, -1)
+    tg, tu = (K * 2 ** -24 * (x.double().abs() @ w.double().abs().t())).chunk(2, -1)
+    full = torch.nn.functional.silu(gate) * up
+    assert ((ops.linear_silu_rows(x, w).double() - full).abs()
+            <= 1.1 * tg * (up.abs() + tu) + tu * gate.abs() + 2 ** -8 * full.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("preset", ["mid-llama", "mid-qwen", "mid-mixtral"])
+@pytest.mark.parametrize("lens", [[1], [7, 20], [128], [100, 29], [384], [200, 185]])
+def test_short_prompts_match_general_path(preset, lens):
+    """A short prompt through the few-row products against the same model's general kernels, which a hook on any of its
+    modules brings back, both within bf16 rounding of each other; the cache rows of the first layer are the same."""
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+    from kllms_amd.models.llama import ForwardBatch
+
+    eng = LLMEngine(EngineConfig(model=preset, max_kv_blocks=256, use_hip_graphs=False, seed=3))
+    seqs = [eng.kv.alloc_sequence(n) for n in lens]
+    slots = torch.tensor([x for s in seqs for x in eng.kv.prefill_slot_mapping(s)])
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    batch = ForwardBatch(mode="prefill", positions=torch.tensor([p for n in lens for p in range(n)]).to(DEV),
+                         slot_mapping=slots.to(DEV), kv_caches=eng.kv.layer_caches(), cu_seqlens=cu.to(DEV))
+    ids = torch.randint(0, 2000, (sum(lens),), generator=torch.Generator().manual_seed(sum(lens))).to(DEV)
+    m = eng.model
+    with torch.inference_mode():
+        assert m._takes_short(ids, batch) == (sum(lens) <= 384)
+        got, kv = m.forward_prefill(ids, batch), eng.kv.k_all.clone()
+        for owner in (m.embed_tokens, m.layers[0], m.layers[0].self_attn, m.layers[0].self_attn.qkv_proj, m.layers[1].self_attn.o_proj):
+            seen = []
+            h = owner.register_forward_hook(lambda *a: seen.append(1))
+            want = m.forward_prefill(ids, batch)
+            h.remove()
+            assert seen
+        with torch.autocast("cuda", torch.bfloat16):
+            assert not m._takes_short(ids, batch)
+    off = (got - want).norm(dim=-1) / want.norm(dim=-1)
+    assert float(off.max()) < (0.5 if preset == "mid-mixtral" else 0.05)      # a routed row may change its experts
+    assert torch.equal(kv[0], eng.kv.k_all[0])
