@@ -1,11 +1,15 @@
 """A hybrid model's step of single decoded rows, sublayer by sublayer in native code, against the general sublayers."""
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
 from kllms_amd import ops
-from kllms_amd.engine.config import EngineConfig
+from kllms_amd.engine.config import ChannelDeltaSpec, EngineConfig
 from kllms_amd.engine.engine import LLMEngine
+from kllms_amd.engine.kvcache import LayerState
+from kllms_amd.models.mixers import ChannelDeltaMixer
 
 DEV = "cuda:0"
 pytestmark = pytest.mark.gpu
@@ -100,6 +104,41 @@ def test_gated_sublayer_against_the_general_one(T):
     # the one rounds gate, up and y to bf16 (2^-9 each), the other the activation alone; rows of a normal size
     assert (x - ref).abs().max() <= 5e-2 and (got.float() - out.float()).abs().max() <= 8e-2
     assert ((x - ref).norm(dim=1) <= 1e-2 * ref.norm(dim=1)).all()
+
+
+@pytest.mark.parametrize("T", [1, 9])
+@pytest.mark.parametrize("H,G,D,V,taps,ranks", [(2, 2, 64, 64, 4, (16, 8)), (4, 2, 64, 128, 4, (64, 56)), (3, 1, 40, 128, 2, (16, 72)),
+                                                (4, 1, 256, 32, 3, (16, 8)), (2, 2, 256, 192, 16, (8, 32)),
+                                                (8, 2, 128, 160, 5, (136, 16))])
+def test_delta_sublayer_against_the_general_one(T, H, G, D, V, taps, ranks):
+    """One, two and three heads to a key head, keys that fill the row groups and do not, values in one block of columns and
+    more, few taps and many, ranks within and above one pass; fresh rows and carried ones, slots in any order."""
+    W, eps = 256, 1e-5
+    g = torch.Generator(device=DEV).manual_seed(H * D + V)
+    spec = ChannelDeltaSpec(heads=H, kv_heads=G, dim=D, vdim=V, conv=taps, decay_rank=ranks[0], gate_rank=ranks[1])
+    mix = ChannelDeltaMixer(spec, W, eps, torch.bfloat16).to(DEV)
+    for n, p in mix.checkpoint_map("").items():
+        p.data.copy_(torch.randn(p.shape, generator=g, device=DEV) * (1.0 if p.dim() == 1 else p.shape[-1] ** -0.5))
+    start = torch.randint(0, 2, (T,), generator=g, device=DEV, dtype=torch.int32) * 7
+    start[0] = 7
+    rows = torch.arange(T + 1, device=DEV, dtype=torch.int32)
+    batch = SimpleNamespace(state_slots=torch.randperm(T + 2, generator=g, device=DEV)[:T].int(), cu_seqlens=rows, seg_start=start,
+                            token_seg=rows[:T].contiguous())
+    states = [LayerState(rec=torch.randn(T + 2, H, D, V, generator=g, device=DEV) * 0.2,
+                         conv=torch.randn(T + 2, taps - 1, mix.cp, generator=g, device=DEV).bfloat16())]
+    states.append(LayerState(rec=states[0].rec.clone(), conv=states[0].conv.clone()))
+    h = torch.randn(T, W, generator=g, device=DEV).bfloat16()
+    x = torch.randn(T, W, generator=g, device=DEV)
+    ref = x.clone()
+    post, nxt = (torch.rand(W, generator=g, device=DEV) + 0.5 for _ in range(2))
+    with torch.no_grad():
+        out = ops.sandwich_residual(ref, mix(h, batch, states[0]), post, eps, w_next=nxt, out_dtype=torch.bfloat16)
+        got = mix.rows_step(x, h, batch, states[1], post, nxt)
+    # the same roundings of values summed in another order: some go the other way, 2^-8 of a term each
+    for a, b in ((x, ref), (got, out), (states[1].rec, states[0].rec)):
+        assert (a.double() - b.double()).norm() <= 1e-2 * b.double().norm()
+    assert (states[1].conv.double() - states[0].conv.double()).abs().max() <= 2 ** -7 * states[0].conv.double().abs().max()
+    assert (states[1].conv != states[0].conv).float().mean() <= 0.02
 
 
 def test_residual_of_split_sums_against_float64():
