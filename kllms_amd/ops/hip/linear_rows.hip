@@ -32,9 +32,11 @@ enum LinearForm { LR_PART = 0, LR_BF16 = 1, LR_F32 = 2, LR_SILU = 3, LR_CLAMPED 
 
 // Workgroups by share of k, then by rows of W, then by rows of x: those of an XCD have the same part of x in its L2, and
 // the row tiles of a part of W run side by side.
+// more: the bias (BF16), or a second matrix (PART): then K is both matrices' and the halves of the splits are two products, of
+// x's first M rows with w and of the next M with more.
 template <int NI, int MJ, int FORM, int KB>
 __global__ void __launch_bounds__(TP_THREADS, 1) linear_rows_kernel(
-    void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const bf16_t* __restrict__ bias,
+    void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const bf16_t* __restrict__ more,
     int M, int N, int K, int x_stride, int m_tiles, int splits, float limit, float alpha) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr bool GATED = FORM == LR_SILU || FORM == LR_CLAMPED;
@@ -57,10 +59,22 @@ __global__ void __launch_bounds__(TP_THREADS, 1) linear_rows_kernel(
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < MJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const TileRows xr(x + k0, m0 + wave * MJ * 8, m_end, MJ * 8, x_stride, lane);
   // W rows of a gated tile: 8 * NI gate, the same of up, the next gate, their up
   const int n_put = GATED ? n0 + (wave >> 1) * (8 * NI) : n0 + wave * (8 * NI);
-  const TileRows wr(w + (GATED ? (int64_t)(wave & 1) * columns : 0) * K + k0, n_put, columns, 8 * NI, K, lane);
+  const bf16_t* wk = w + (GATED ? (int64_t)(wave & 1) * columns : 0) * K + k0;
+  const bf16_t* xk = x + k0;
+  int w_row = K;
+  if constexpr (FORM == LR_PART) {
+    if (more) {
+      w_row = K / 2;
+      if (2 * share >= splits) {
+        wk = more + (k0 - w_row);
+        xk += (int64_t)M * x_stride - w_row;
+      }
+    }
+  }
+  const TileRows xr(xk, m0 + wave * MJ * 8, m_end, MJ * 8, x_stride, lane);
+  const TileRows wr(wk, n_put, columns, 8 * NI, w_row, lane);
   // the XCDs begin at different k: rows of a power of two of bytes would have all of them at the same memory channels
   tile_product<MJ, NI, KB * 1024>(acc, wr, xr, stages, stages * xcd / 8, smem);
   if constexpr (FORM == LR_SILU && MJ > 4) {       // many rows: whole lines
@@ -101,7 +115,7 @@ __global__ void __launch_bounds__(TP_THREADS, 1) linear_rows_kernel(
       } else if constexpr (FORM == LR_BF16) {
         bf16x4_vec o;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = f32_to_bf16(acc[i][j][r] + (bias ? bf16_to_f32(((const short*)bias)[nc + r]) : 0.0f));
+        for (int r = 0; r < 4; ++r) o[r] = f32_to_bf16(acc[i][j][r] + (more ? bf16_to_f32(((const short*)more)[nc + r]) : 0.0f));
         *reinterpret_cast<bf16x4_vec*>((short*)out + (int64_t)mr * N + nc) = o;
       } else {
         *reinterpret_cast<f32x4*>((float*)out + ((int64_t)share * M + mr) * N + nc) = acc[i][j];
@@ -157,23 +171,23 @@ static bool lr_lds_ready(const void* kernel, std::atomic<uint64_t>& devices) {
 }
 
 template <int NI, int MJ, int FORM, int KB>
-static int linear_rows_go(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N, int K, int x_stride,
+static int linear_rows_go(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* more, int M, int N, int K, int x_stride,
                           int m_tiles, int splits, float limit, float alpha, hipStream_t stream) {
   static std::atomic<uint64_t> devices{0};
   if (!lr_lds_ready(reinterpret_cast<const void*>(linear_rows_kernel<NI, MJ, FORM, KB>), devices)) return -1;
   constexpr int LDS = TileRing<MJ, NI, KB * 1024>::STRIDE * TileRing<MJ, NI, KB * 1024>::RING;
   const int64_t all = (int64_t)((N + 32 * NI - 1) / (32 * NI)) * splits * m_tiles;
-  hipLaunchKernelGGL((linear_rows_kernel<NI, MJ, FORM, KB>), dim3((all + 7) / 8 * 8), dim3(TP_THREADS), LDS, stream, out, x, w, bias,
+  hipLaunchKernelGGL((linear_rows_kernel<NI, MJ, FORM, KB>), dim3((all + 7) / 8 * 8), dim3(TP_THREADS), LDS, stream, out, x, w, more,
                      M, N, K, x_stride, m_tiles, splits, limit, alpha);
   return 0;
 }
 
 template <int FORM>
-static int linear_rows_form(const LinearPlan& p, void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
+static int linear_rows_form(const LinearPlan& p, void* out, const bf16_t* x, const bf16_t* w, const bf16_t* more, int M, int N,
                             int K, int x_stride, int splits, float limit, float alpha, hipStream_t stream) {
 #define LR_CASE(NI, MJ)                                                                                              \
   if (p.ni == NI && p.mj == MJ)                                                                                      \
-    return linear_rows_go<NI, MJ, FORM, (NI == 2 || MJ <= 2 ? 80 : 160)>(out, x, w, bias, M, N, K, x_stride, p.m_tiles, splits, limit, \
+    return linear_rows_go<NI, MJ, FORM, (NI == 2 || MJ <= 2 ? 80 : 160)>(out, x, w, more, M, N, K, x_stride, p.m_tiles, splits, limit, \
                                                                          alpha, stream)
   LR_CASE(2, 1);
   LR_CASE(2, 2);
@@ -221,4 +235,10 @@ extern "C" int linear_rows_splits(int M, int N, int K) {
   const int tiles = (N + 32 * p.ni - 1) / (32 * p.ni) * p.m_tiles, most = K / TP_K / 4;
   const int s = (LR_UNITS + 8) / tiles;
   return s < 1 || most < 1 ? 1 : s < most ? s : most;
+}
+
+// PART sums of two products of one size, x [2, M, K] with w and w2 [N, K]: [S, M, N], the first half of the (even) S the one's
+extern "C" int launch_linear_rows_two(float* out, const bf16_t* x, const bf16_t* w, const bf16_t* w2, int M, int N, int K,
+                                      int splits, hipStream_t stream) {
+  return linear_rows_form<LR_PART>(linear_plan(M, N, K, LR_PART), out, x, w, w2, M, N, 2 * K, K, splits, 0.0f, 0.0f, stream);
 }

@@ -524,9 +524,7 @@ extern "C" void seq_launch_linear_attn_decay(float* o, const void* q, const void
                                              int v_stride, int is_f32, hipStream_t st) {
   const int64_t n = (int64_t)T_ * H * (2 * D + V);
   const int grid = (int)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384);
-  if (q == nullptr) {
-    // packed has been filled already
-  } else if (D % 8 == 0 && V % 8 == 0 && q_stride % 8 == 0 && k_stride % 8 == 0 && v_stride % 8 == 0 &&
+  if (D % 8 == 0 && V % 8 == 0 && q_stride % 8 == 0 && k_stride % 8 == 0 && v_stride % 8 == 0 &&
              aligned16(q) && aligned16(k) && aligned16(v) && aligned16(packed)) {
     const int g8 = (int)((n / 8 + 255) / 256 < 16384 ? (n / 8 + 255) / 256 : 16384);
     DISPATCH_T(is_f32, hipLaunchKernelGGL(linear_prep_v8_kernel<T>, dim3(g8), dim3(256), 0, st, packed,

@@ -1,10 +1,10 @@
 // Row-wise passes of a hybrid model's step of few rows, straight from the split sums of the product before them
 // (fp32, as linear_rows leaves them). First the residual epilogue, a [SA, T, W], b [SB, T, W]:
-//   y = a, or (rms(a) wa + rms(b) wb) / 2;  x += rms(y) w_post;  out = rms(x) w_next in bf16
+//   y = a, or (rms(a) wa + rms(b / rms(what b is of)) wb) / 2;  x += rms(y) w_post;  out = rms(x) w_next in bf16
 //
 // A row is one workgroup's: its sums are the bytes, 64 to 128 KB of them, and the three reductions the chain behind. Four
-// columns a thread and load, kept in registers through all passes. 40 rows of 2048 in 8 shares: 5.2 us
-// of a step, 7.8 with two branches (4.8 and 6.5 from bf16 products, which took 12 and 12 to 17 us themselves, 5.3 now).
+// columns a thread and load, kept in registers through all passes. 40 rows of 2048 in 8 shares: 4.7 us
+// of a step, 8.6 with two branches (4.8 and 6.5 from bf16 products, which took 12 and 12 to 17 us themselves).
 
 #include "seq_common.h"
 
@@ -17,7 +17,8 @@ template <bool DUAL>
 __global__ void __launch_bounds__(SR_THREADS) sandwich_rows_kernel(
     float* __restrict__ x, const float* __restrict__ a, int SA, const float* __restrict__ b, int SB,
     const float* __restrict__ wa, const float* __restrict__ wb, const float* __restrict__ w_post,
-    const float* __restrict__ w_next, bfraw* __restrict__ out, int T_, int W, float eps) {
+    const float* __restrict__ w_next, bfraw* __restrict__ out, int T_, int W, float eps,
+    const float* __restrict__ squares, int heads, float per) {
   __shared__ float scratch[16];
   const int t = blockIdx.x, tid = threadIdx.x, nvec = W / 4;
   const int64_t plane = (int64_t)T_ * W;
@@ -44,8 +45,13 @@ __global__ void __launch_bounds__(SR_THREADS) sandwich_rows_kernel(
   f32x4 y[SR_VECS];
   float ss = sums(a, SA, y);
   if constexpr (DUAL) {
+    // b is of a product whose rows' norm is put off to here
+    float sq = 0.0f;
+    for (int i = tid % WAVE; i < heads; i += WAVE) sq += squares[(int64_t)t * heads + i];
     f32x4 z[SR_VECS];
-    const float sb = sums(b, SB, z);
+    float sb = sums(b, SB, z);
+    const float rs = 1.0f / sqrtf(wave_sum(sq) * per + eps);
+    sb *= rs * rs;
     const float ra = 1.0f / sqrtf(block_sum(ss, scratch) * inv_w + eps);
     const float rb = 1.0f / sqrtf(block_sum(sb, scratch) * inv_w + eps);
     ss = 0.0f;
@@ -56,7 +62,7 @@ __global__ void __launch_bounds__(SR_THREADS) sandwich_rows_kernel(
       const f32x4 ga = reinterpret_cast<const f32x4*>(wa)[i], gb = reinterpret_cast<const f32x4*>(wb)[i];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        y[k][e] = 0.5f * (y[k][e] * ra * ga[e] + z[k][e] * rb * gb[e]);
+        y[k][e] = 0.5f * (y[k][e] * ra * ga[e] + z[k][e] * rs * rb * gb[e]);
         ss += y[k][e] * y[k][e];
       }
     }
@@ -89,100 +95,192 @@ __global__ void __launch_bounds__(SR_THREADS) sandwich_rows_kernel(
   }
 }
 
-// b nullptr: one branch
+// b nullptr: one branch. squares [T, heads]: sums of squares of which per times the row's total is the mean that b's rows are
+// still to be normalised by
 extern "C" void seq_launch_sandwich_rows(float* x, const float* a, int SA, const float* b, int SB, const float* wa,
                                          const float* wb, const float* w_post, const float* w_next, void* out, int T_,
-                                         int W, float eps, hipStream_t st) {
-  if (b)
-    hipLaunchKernelGGL(sandwich_rows_kernel<true>, dim3(T_), dim3(SR_THREADS), 0, st, x, a, SA, b, SB, wa, wb, w_post,
-                       w_next, (bfraw*)out, T_, W, eps);
-  else
-    hipLaunchKernelGGL(sandwich_rows_kernel<false>, dim3(T_), dim3(SR_THREADS), 0, st, x, a, SA, b, SB, wa, wb, w_post,
-                       w_next, (bfraw*)out, T_, W, eps);
+                                         int W, float eps, const float* squares, int heads, float per, hipStream_t st) {
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(T_), dim3(SR_THREADS), 0, st, x, a, SA, b, SB, wa, wb, w_post, w_next, (bfraw*)out, T_, W,
+                       eps, squares, heads, per);
+  };
+  b ? go(sandwich_rows_kernel<true>) : go(sandwich_rows_kernel<false>);
 }
 
-// What a parallel sublayer's input product, as split sums part [S, T, N], is wanted for, in one pass: sums (+ bias), then
-// left q rotated in pairs and rounded, left k rotated into the cache with itself as the value, head gates and the right
-// gate rounded, and silu of the right q, k, v in the recurrence's order. Four columns a thread; at: first columns of left
-// q, k, head gates and right q, k, v, gate, all multiples of 8.
+// What a parallel sublayer's input product, as split sums part [S, T, N], is wanted for, in one launch: sums (+ bias), then for
+// the softmax branch left q rotated in pairs and rounded, left k rotated into the cache with itself as the value and the head
+// gates rounded (four columns a thread); and the recurrent branch up to its norm, a workgroup a row's head: silu of q, k, v,
+// the step of the recurrence, and o w sigmoid(gate) in bf16 with the head's sum of o^2, from which the branch's norm over all
+// heads is one factor a row for the pass behind the output product. at: first columns of left q, k, head gates and right q, k,
+// v, gate, all multiples of 8.
 //
-// Bound by the sums' bytes (5.6 MB for 40 rows of 8720 in 4 shares) and a launch. In place of a product in one share (21 us
-// of it), the rotation's pass and the silu pass (8 us): a step of 40 rows 699 us before, 678 with it, of 2 rows 635 and 586.
+// Bound by the state's bytes (32 KB a head of 64 x 128, read and written). A thread keeps four columns of DR rows of the state.
+// In place of a pass over the sums, the recurrence and the norm (4.5, 14.5 and 5 us for 40 rows of 16 heads): 12.9 us, with 8
+// rows 6.8 (15).
 struct SplitColumns { int at[7]; };
 
-__global__ void __launch_bounds__(256) hybrid_split_kernel(
+#define PR_THREADS 512
+#define DR_BLOCK 128           // columns of the state at a time
+
+template <int DR>
+__global__ void __launch_bounds__(PR_THREADS, DR <= 8 ? 4 : 2) parallel_rows_kernel(
     const float* __restrict__ part, int S, const bfraw* __restrict__ bias, SplitColumns cols,
     const int64_t* __restrict__ positions, const float* __restrict__ inv_freq, bfraw* __restrict__ k_cache,
-    bfraw* __restrict__ v_cache, const int64_t* __restrict__ slots, bfraw* __restrict__ q_out,
-    bfraw* __restrict__ head_gate, float* __restrict__ packed, bfraw* __restrict__ gate, int T_, int N, int H, int G,
-    int R, int BS, int RH, int RD, int RV) {
-  const int t = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;
-  if (c >= N) return;
-  float x[4] = {};
-  const float* p = part + (int64_t)t * N + c;
-#pragma unroll 4
-  for (int s = 0; s < S; ++s) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(p + (int64_t)s * T_ * N);
+    bfraw* __restrict__ v_cache, const int64_t* __restrict__ cache_slots, bfraw* __restrict__ q_out,
+    bfraw* __restrict__ head_gate, const float* __restrict__ decay, float* __restrict__ state,
+    const float* __restrict__ norm, bfraw* __restrict__ z, float* __restrict__ squares,
+    const int* __restrict__ slots, const int* __restrict__ cu, const int* __restrict__ seg_start, int T_, int N, int H,
+    int G, int R, int BS, int RH, int RD, int RV) {
+  extern __shared__ float lds[];
+  const int tid = threadIdx.x, plane = T_ * N;
+  if ((int)blockIdx.x >= RH) {
+    const int t = blockIdx.y, i = ((blockIdx.x - RH) * PR_THREADS + tid) * 4;
+    const int nq = H * 128, nk = G * 128;
+    if (i >= nq + nk + H) return;
+    const bool is_q = i < nq, is_k = !is_q && i < nq + nk;
+    const int o = is_q ? i : is_k ? i - nq : i - nq - nk, c = cols.at[is_q ? 0 : is_k ? 1 : 2] + o;
+    const float* p = part + (int64_t)t * N + c;
+    float x[4] = {};
+    for (int s0 = 0; s0 < S; s0 += 8) {
+      f32x4 v[8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] += v[e];
-  }
-  if (bias) {
+      for (int s = 0; s < 8; ++s) v[s] = *reinterpret_cast<const f32x4*>(p + (int64_t)min(s0 + s, S - 1) * plane);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] += ldf(bias + c + e);
-  }
-  auto put = [](bfraw* o, const float (&v)[4]) {
-    *reinterpret_cast<uint2*>(o) = make_uint2(bf_bits(v[0]) | (bf_bits(v[1]) << 16), bf_bits(v[2]) | (bf_bits(v[3]) << 16));
-  };
-  auto in = [&](int i, int n) { return c >= cols.at[i] && c < cols.at[i] + n; };
-  const bool is_q = in(0, H * 128);
-  if (is_q || in(1, G * 128)) {
-    const int o = c - cols.at[is_q ? 0 : 1], dim = o % 128;
+      for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] += s0 + s < S ? v[s][e] : 0.0f;
+    }
+    if (bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] += ldf(bias + c + e);
+    }
+    auto put = [](bfraw* to, const float (&v)[4]) {
+      *reinterpret_cast<uint2*>(to) = make_uint2(bf_bits(v[0]) | (bf_bits(v[1]) << 16), bf_bits(v[2]) | (bf_bits(v[3]) << 16));
+    };
+    if (!is_q && !is_k) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (o + e < H) stf(head_gate + (int64_t)t * H + o + e, x[e]);
+      return;
+    }
+    const int dim = o % 128;
     float y[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int k = 0; k < 2; ++k) {
       float sn = 0.0f, cs = 1.0f;
-      if (dim / 2 + i < R) sincosf((float)positions[t] * inv_freq[dim / 2 + i], &sn, &cs);
-      y[2 * i] = x[2 * i] * cs - x[2 * i + 1] * sn;
-      y[2 * i + 1] = x[2 * i + 1] * cs + x[2 * i] * sn;
+      if (dim / 2 + k < R) sincosf((float)positions[t] * inv_freq[dim / 2 + k], &sn, &cs);
+      y[2 * k] = x[2 * k] * cs - x[2 * k + 1] * sn;
+      y[2 * k + 1] = x[2 * k + 1] * cs + x[2 * k] * sn;
     }
     if (is_q) {
-      put(q_out + (int64_t)t * H * 128 + o, y);
+      put(q_out + (int64_t)t * nq + o, y);
     } else {
-      const int64_t slot = slots[t], row = (slot / BS * G + o / 128) * BS + slot % BS;
+      const int64_t slot = cache_slots[t], row = (slot / BS * G + o / 128) * BS + slot % BS;
       put(k_cache + row * 128 + dim, y);
       put(v_cache + row * 128 + dim, x);
     }
-  } else if (in(2, H)) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (c + e < cols.at[2] + H) stf(head_gate + (int64_t)t * H + c - cols.at[2] + e, x[e]);
-  } else if (in(6, RH * RV)) {
-    put(gate + (int64_t)t * RH * RV + c - cols.at[6], x);
-  } else {
-#pragma unroll
-    for (int i = 3; i < 6; ++i) {
-      const int w = i == 5 ? RV : RD;    // a multiple of 4
-      if (!in(i, RH * w)) continue;
-      const int o = c - cols.at[i], h = o / w;
-      float* to = packed + ((int64_t)t * RH + h) * (2 * RD + RV) + (i - 3) * RD + o % w;
-      f32x4 y;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) y[e] = silu_exact(x[e]);
-      *reinterpret_cast<f32x4*>(to) = y;
-    }
+    return;
   }
+  const int b = blockIdx.y, h = blockIdx.x, t = cu[b];
+  if (cu[b + 1] == t) return;                         // the whole workgroup
+  const bool fresh = seg_start[b] == 0;
+  float* const qs = lds, *const ks = qs + RD, *const vs = ks + RD, *const gate = vs + RV;
+  float* const red = gate + RV;                       // RD and RV are multiples of 4
+  const float dec = decay[h];
+  float* const head = state + ((int64_t)slots[b] * RH + h) * RD * RV;
+  f32x4 st[DR];
+  auto fetch = [&](int c0, int V4, int RG) {
+    const int quad = tid % V4, rg = tid / V4;
+#pragma unroll
+    for (int i = 0; i < DR; ++i) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(head + (int64_t)min(i * RG + rg, RD - 1) * RV + c0 + quad * 4);
+      st[i] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : v;
+    }
+  };
+  const int n = 2 * (RD + RV);
+  float v[8], add = 0.0f;
+  const float* p;
+  auto column = [&](int i) {
+    i = min(i, n - 1);
+    const int c = i < RD ? cols.at[3] + h * RD + i : i < 2 * RD ? cols.at[4] + h * RD + i - RD
+                : i < 2 * RD + RV ? cols.at[5] + h * RV + i - 2 * RD : cols.at[6] + h * RV + i - 2 * RD - RV;
+    p = part + (int64_t)t * N + c;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) v[s] = p[(int64_t)min(s, S - 1) * plane];
+    if (bias) add = ldf(bias + c);
+  };
+  column(tid);
+  const int first4 = min(RV, DR_BLOCK) / 4;
+  fetch(0, first4, PR_THREADS / first4);
+  for (int i = tid; i < n; i += PR_THREADS) {
+    if (i >= PR_THREADS) column(i);
+    float x = 0.0f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) x += s < S ? v[s] : 0.0f;
+    for (int s = 8; s < S; ++s) x += p[(int64_t)s * plane];
+    x += add;
+    lds[i] = i < 2 * RD + RV ? silu_exact(x) : sigmoid_exact(__uint_as_float(bf_bits(x) << 16));
+  }
+  __syncthreads();
+  float ss = 0.0f;
+  for (int c0 = 0; c0 < RV; c0 += DR_BLOCK) {
+    const int VB = min(RV - c0, DR_BLOCK), V4 = VB / 4, RG = PR_THREADS / V4, quad = tid % V4, rg = tid / V4;
+    if (c0 > 0) fetch(c0, V4, RG);
+    f32x4 read = {0.f, 0.f, 0.f, 0.f};
+    if (rg < RG) {
+      const f32x4 val = *reinterpret_cast<const f32x4*>(vs + c0 + quad * 4);
+#pragma unroll
+      for (int i = 0; i < DR; ++i) {
+        const int d = i * RG + rg;
+        const float k = ks[min(d, RD - 1)], q = d < RD ? qs[min(d, RD - 1)] : 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          st[i][e] = dec * st[i][e] + k * val[e];
+          read[e] += st[i][e] * q;
+        }
+        if (d < RD) *reinterpret_cast<f32x4*>(head + (int64_t)d * RV + c0 + quad * 4) = st[i];
+      }
+      *reinterpret_cast<f32x4*>(red + rg * VB + quad * 4) = read;
+    }
+    __syncthreads();
+    if (tid < VB) {
+      float o = 0.0f;
+#pragma unroll 8
+      for (int i = 0; i < RG; ++i) o += red[i * VB + tid];
+      ss += o * o;
+      const int c = c0 + tid;
+      stf(z + ((int64_t)t * RH + h) * RV + c, o * norm[h * RV + c] * gate[c]);
+    }
+    __syncthreads();
+  }
+  ss = block_sum(ss, red);
+  if (tid == 0) squares[(int64_t)t * RH + h] = ss;
 }
 
-extern "C" void seq_launch_hybrid_split(const float* part, int S, const void* bias, const int64_t* at,
-                                        const int64_t* positions, const float* inv_freq, void* k_cache, void* v_cache,
-                                        const int64_t* slots, void* q_out, void* head_gate, float* packed, void* gate,
-                                        int T_, int N, int H, int G, int R, int BS, int RH, int RD, int RV,
-                                        hipStream_t st) {
+static inline size_t parallel_rows_lds(int RD, int RV) { return (size_t)(2 * (RD + RV) + PR_THREADS * 4) * sizeof(float); }
+
+// what a workgroup keeps within 64 KB
+extern "C" bool seq_parallel_rows_takes(int RD, int RV) { return RD <= 256 && parallel_rows_lds(RD, RV) <= 65536; }
+
+extern "C" void seq_launch_parallel_rows(const float* part, int S, const void* bias, const int64_t* at,
+                                         const int64_t* positions, const float* inv_freq, void* k_cache, void* v_cache,
+                                         const int64_t* cache_slots, void* q_out, void* head_gate, const float* decay,
+                                         float* state, const float* norm, void* z, float* squares,
+                                         const int* slots, const int* cu, const int* seg_start, int T_, int N, int H, int G,
+                                         int R, int BS, int RH, int RD, int RV, hipStream_t st) {
   SplitColumns cols;
   for (int i = 0; i < 7; ++i) cols.at[i] = (int)at[i];
-  hipLaunchKernelGGL(hybrid_split_kernel, dim3((N / 4 + 255) / 256, T_), dim3(256), 0, st, part, S, (const bfraw*)bias,
-                     cols, positions, inv_freq, (bfraw*)k_cache, (bfraw*)v_cache, slots, (bfraw*)q_out, (bfraw*)head_gate,
-                     packed, (bfraw*)gate, T_, N, H, G, R, BS, RH, RD, RV);
+  const int left = (H * 128 + G * 128 + H + 4 * PR_THREADS - 1) / (4 * PR_THREADS);
+  const int RG = PR_THREADS / ((RV < DR_BLOCK ? RV : DR_BLOCK) / 4), rows = (RD + RG - 1) / RG;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(RH + left, T_), dim3(PR_THREADS), parallel_rows_lds(RD, RV), st, part, S,
+                       (const bfraw*)bias, cols, positions, inv_freq, (bfraw*)k_cache, (bfraw*)v_cache, cache_slots,
+                       (bfraw*)q_out, (bfraw*)head_gate, decay, state, norm, (bfraw*)z, squares, slots, cu,
+                       seg_start, T_, N, H, G, R, BS, RH, RD, RV);
+  };
+  if (rows <= 4) go(parallel_rows_kernel<4>);
+  else if (rows <= 8) go(parallel_rows_kernel<8>);
+  else go(parallel_rows_kernel<16>);
 }
 
 // A gated-delta-rule sublayer between its input product (split sums part [S, T, N]) and its output product, single tokens:
@@ -201,7 +299,6 @@ struct DeltaColumns { int at[6]; };
 
 #define DR_THREADS 512
 #define DR_OUTS 6             // low-rank outputs of eight lanes at a time: registers
-#define DR_BLOCK 128           // columns of the state at a time
 
 template <int DR, int HP, int TAPS>
 __global__ void __launch_bounds__(DR_THREADS, DR * HP <= 8 ? 4 : 2) delta_rows_kernel(

@@ -1,5 +1,5 @@
 // Whole sublayers of a hybrid model's decode step (one row a sequence, up to 128 of them), launched from here one
-// kernel behind the other. A step is some 60 launches of 4 to 18 us, and from Python a launch costs the host 12 to 15 us:
+// kernel behind the other. A step is some 50 launches of 4 to 18 us, and from Python a launch costs the host 12 to 15 us:
 // it was the bound (85 launches for 40 rows of the 2048-wide preset: 1310 us, the kernels 775). Here it is 2 to 3.
 
 #include <torch/extension.h>
@@ -11,15 +11,11 @@
 
 extern "C" {
 void seq_launch_sandwich_rows(float*, const float*, int, const float*, int, const float*, const float*, const float*,
-                              const float*, void*, int, int, float, hipStream_t);
-void seq_launch_gated_rmsnorm(void*, const float*, const float*, const void*, int, int, int, int, float, int,
-                              int, hipStream_t);
-void seq_launch_hybrid_split(const float*, int, const void*, const int64_t*, const int64_t*, const float*, void*, void*,
-                             const int64_t*, void*, void*, float*, void*, int, int, int, int, int, int, int, int, int,
-                             hipStream_t);
-void seq_launch_linear_attn_decay(float*, const void*, const void*, const void*, const float*, float*, float*,
-                                  const int*, const int*, const int*, int, int, int, int, int, int, int, int,
-                                  int, hipStream_t);
+                              const float*, void*, int, int, float, const float*, int, float, hipStream_t);
+bool seq_parallel_rows_takes(int, int);
+void seq_launch_parallel_rows(const float*, int, const void*, const int64_t*, const int64_t*, const float*, void*, void*,
+                              const int64_t*, void*, void*, const float*, float*, const float*, void*, float*, const int*,
+                              const int*, const int*, int, int, int, int, int, int, int, int, int, hipStream_t);
 bool seq_delta_rows_takes(int, int, int, int, int, int, int);
 void seq_launch_delta_rows(const float*, int, const int64_t*, const float*, void*, int, int, const void*, int, const void*, int,
                            const float*, const float*, float*, const float*, void*, const int*, const int*, const int*, int,
@@ -28,6 +24,8 @@ void seq_launch_gated_act(void*, const void*, const void*, int64_t, int, int, fl
 // few-row products and paged decode attention (ops/hip/linear_rows.hip, attn_decode.hip, also part of kllms_amd._C)
 int launch_linear_rows(void*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
                         int, int, float, float, hipStream_t);
+int launch_linear_rows_two(float*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
+                           hipStream_t);
 int linear_rows_splits(int, int, int);
 int attn_decode_splits(int, int, int);
 void launch_attn_decode(__hip_bfloat16*, float*, const __hip_bfloat16*, const void*, const void*, const float*,
@@ -96,7 +94,7 @@ std::optional<Tensor> hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tens
                             Tensor o_right, Tensor wa, Tensor wb, Tensor w_post, Tensor w_next, Tensor positions,
                             Tensor slots, Tensor tables, Tensor lens, Tensor state_slots, Tensor cu, Tensor seg_start,
                             int64_t heads, double scale, int64_t mask_size, double eps) {
-  if (!lie_whole({w_in, o_left, o_right, wa, wb, w_post, w_next})) return std::nullopt;
+  if (!lie_whole({w_in, o_left, o_right, state, wa, wb, w_post, w_next})) return std::nullopt;
   const Rows r(x, h);
   const int T = r.T, W = r.W;
   check_weight(w_in, W, "w_in");
@@ -134,36 +132,43 @@ std::optional<Tensor> hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tens
   TORCH_CHECK(tables.dim() == 2 && tables.size(0) == T, "one table row for each row");
   check(tables, at::kInt, tables.numel(), "tables");
   const int width = tables.size(1);
+  if (!seq_parallel_rows_takes(RD, RV)) return std::nullopt;
 
   auto st = cur_stream();
   const auto f32 = x.options();
   const Tensor y = part(h, w_in, T, st);
-  auto q = torch::empty({T, (int64_t)H * D}, h.options()), head_gate = torch::empty({T, H}, h.options()),
-       gate = torch::empty({T, (int64_t)RH * RV}, h.options());
-  auto packed = torch::empty({T, (int64_t)RH * (2 * RD + RV)}, f32);
-  seq_launch_hybrid_split(y.data_ptr<float>(), y.size(0), bias.numel() ? bias.data_ptr() : nullptr, at.data(),
-                          positions.data_ptr<int64_t>(), inv_freq.data_ptr<float>(), k_cache.data_ptr(),
-                          v_cache.data_ptr(), slots.data_ptr<int64_t>(), q.data_ptr(), head_gate.data_ptr(),
-                          packed.data_ptr<float>(), gate.data_ptr(), T, N, H, G, R, BS, RH, RD, RV, st);
-  auto att = torch::empty({T, (int64_t)H * D}, h.options());
+  const int KL = H * D, KR = RH * RV;
+  auto q = torch::empty({T, (int64_t)KL}, h.options()), head_gate = torch::empty({T, H}, h.options());
+  auto both = torch::empty({(int64_t)T * (KL + KR)}, h.options());     // the left branch's rows, then the right one's
+  auto squares = torch::empty({T, RH}, f32);
+  seq_launch_parallel_rows(y.data_ptr<float>(), y.size(0), bias.numel() ? bias.data_ptr() : nullptr, at.data(),
+                           positions.data_ptr<int64_t>(), inv_freq.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
+                           slots.data_ptr<int64_t>(), q.data_ptr(), head_gate.data_ptr(), decay.data_ptr<float>(),
+                           state.data_ptr<float>(), norm_right.data_ptr<float>(),
+                           (void*)bf(both, (int64_t)T * KL), squares.data_ptr<float>(), state_slots.data_ptr<int>(),
+                           cu.data_ptr<int>(), seg_start.data_ptr<int>(), T, N, H, G, R, BS, RH, RD, RV, st);
   const int64_t longest = mask_size > 0 ? std::min<int64_t>(mask_size, (int64_t)width * BS) : (int64_t)width * BS;
   const int splits = attn_decode_splits(T, G, (int)std::min<int64_t>(longest, INT32_MAX));
   auto partials = torch::empty({splits > 1 ? (int64_t)T * H * splits * 130 : 0}, f32);
-  launch_attn_decode((__hip_bfloat16*)att.data_ptr(), partials.data_ptr<float>(), bf(q), k_cache.data_ptr(),
+  launch_attn_decode((__hip_bfloat16*)both.data_ptr(), partials.data_ptr<float>(), bf(q), k_cache.data_ptr(),
                      v_cache.data_ptr(), nullptr, nullptr, tables.data_ptr<int>(), lens.data_ptr<int>(), bf(head_gate), H,
-                     (float)scale, H, G, BS, width, splits, H * D, T, 0, (int)mask_size, st);
-  auto o = torch::empty({T, (int64_t)RH * RV}, f32);
-  seq_launch_linear_attn_decay(o.data_ptr<float>(), nullptr, nullptr, nullptr, decay.data_ptr<float>(),
-                               packed.data_ptr<float>(), state.data_ptr<float>(), state_slots.data_ptr<int>(),
-                               cu.data_ptr<int>(), seg_start.data_ptr<int>(), T, T, RH, RD, RV, 0, 0, 0, 0, st);
-  auto yr = torch::empty({T, (int64_t)RH * RV}, h.options());
-  seq_launch_gated_rmsnorm(yr.data_ptr(), o.data_ptr<float>(), norm_right.data_ptr<float>(), gate.data_ptr(), T, 1, RH * RV,
-                           RH * RV, (float)eps, 0, 0, st);
-  const Tensor left = part(att, o_left, T, st), right = part(yr, o_right, T, st);
+                     (float)scale, H, G, BS, width, splits, KL, T, 0, (int)mask_size, st);
+  Tensor left, right;
+  if (KL == KR) {    // one launch, half as many sums of each: 40 rows, 2048 x 2048 each, 6.2 us, two launches 5.3 each
+    const int S = std::max(linear_rows_splits(T, W, 2 * KL) & ~1, 2);
+    const Tensor sums = torch::empty({S, T, (int64_t)W}, f32);
+    TORCH_CHECK(launch_linear_rows_two(sums.data_ptr<float>(), bf(both), bf(o_left), bf(o_right), T, W, KL, S, st) == 0, NO_LDS);
+    left = sums.narrow(0, 0, S / 2);
+    right = sums.narrow(0, S / 2, S / 2);
+  } else {
+    left = part(both, o_left, T, st);
+    right = part(both.narrow(0, (int64_t)T * KL, (int64_t)T * KR), o_right, T, st);
+  }
   auto out = torch::empty_like(h);
   seq_launch_sandwich_rows(x.data_ptr<float>(), left.data_ptr<float>(), left.size(0), right.data_ptr<float>(),
                            right.size(0), wa.data_ptr<float>(), wb.data_ptr<float>(), w_post.data_ptr<float>(),
-                           w_next.data_ptr<float>(), out.data_ptr(), T, W, (float)eps, st);
+                           w_next.data_ptr<float>(), out.data_ptr(), T, W, (float)eps, squares.data_ptr<float>(), RH,
+                           1.0f / (float)KR, st);
   return out;
 }
 
@@ -217,7 +222,7 @@ std::optional<Tensor> hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::ve
   const Tensor p = part(yr, w_out, T, st);
   auto out = torch::empty_like(h);
   seq_launch_sandwich_rows(x.data_ptr<float>(), p.data_ptr<float>(), p.size(0), nullptr, 0, nullptr, nullptr,
-                           w_post.data_ptr<float>(), w_next.data_ptr<float>(), out.data_ptr(), T, W, (float)eps, st);
+                           w_post.data_ptr<float>(), w_next.data_ptr<float>(), out.data_ptr(), T, W, (float)eps, nullptr, 0, 0.0f, st);
   return out;
 }
 
@@ -250,6 +255,6 @@ std::optional<Tensor> hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_
   const Tensor p = part(act, w_down, r.T, st);
   auto out = torch::empty_like(h);
   seq_launch_sandwich_rows(x.data_ptr<float>(), p.data_ptr<float>(), p.size(0), nullptr, 0, nullptr, nullptr,
-                           w_post.data_ptr<float>(), w_next.data_ptr<float>(), out.data_ptr(), r.T, r.W, (float)eps, st);
+                           w_post.data_ptr<float>(), w_next.data_ptr<float>(), out.data_ptr(), r.T, r.W, (float)eps, nullptr, 0, 0.0f, st);
   return out;
 }

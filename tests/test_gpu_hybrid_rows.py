@@ -6,10 +6,11 @@ import pytest
 import torch
 
 from kllms_amd import ops
-from kllms_amd.engine.config import ChannelDeltaSpec, EngineConfig
+from kllms_amd.engine.config import (BlockAttnSpec, ChannelDeltaSpec, DecayLinearAttnSpec, EngineConfig, ParallelMixerSpec,
+                                     RotarySpec)
 from kllms_amd.engine.engine import LLMEngine
 from kllms_amd.engine.kvcache import LayerState
-from kllms_amd.models.mixers import ChannelDeltaMixer
+from kllms_amd.models.mixers import ChannelDeltaMixer, ParallelMixer
 
 DEV = "cuda:0"
 pytestmark = pytest.mark.gpu
@@ -139,6 +140,49 @@ def test_delta_sublayer_against_the_general_one(T, H, G, D, V, taps, ranks):
         assert (a.double() - b.double()).norm() <= 1e-2 * b.double().norm()
     assert (states[1].conv.double() - states[0].conv.double()).abs().max() <= 2 ** -7 * states[0].conv.double().abs().max()
     assert (states[1].conv != states[0].conv).float().mean() <= 0.02
+
+
+@pytest.mark.parametrize("T", [1, 9])
+@pytest.mark.parametrize("G,RH,RD,RV", [(2, 16, 64, 128), (4, 2, 40, 192), (4, 4, 256, 32)])
+def test_parallel_sublayer_against_the_general_one(T, G, RH, RD, RV):
+    """Output products of one size (one launch) and of two, keys that fill the row groups and do not, values in one block of
+    columns and more; fresh rows and carried ones, slots in any order."""
+    W, H, eps, BS, blocks = 256, 16, 1e-5, 16, 4
+    g = torch.Generator(device=DEV).manual_seed(RH * RD + RV)
+    spec = ParallelMixerSpec(left=BlockAttnSpec(heads=H, kv_heads=G, dim=128, vdim=128, scale=0.1, mask_size=32,
+                                                rot=RotarySpec(dims=96)),
+                             right=DecayLinearAttnSpec(heads=RH, dim=RD, vdim=RV, decay=[0.5 + 0.4 * i / RH for i in range(RH)]))
+    mix = ParallelMixer(spec, W, eps, torch.bfloat16).to(DEV)
+    for n, p in mix.checkpoint_map("").items():
+        p.data.copy_(torch.randn(p.shape, generator=g, device=DEV) * (1.0 if p.dim() == 1 else p.shape[-1] ** -0.5))
+    rows = torch.arange(T + 1, device=DEV, dtype=torch.int32)
+    positions = torch.randint(0, BS * blocks, (T,), generator=g, device=DEV)
+    positions[0] = BS * blocks - 1
+    tables = torch.randperm(T * blocks, generator=g, device=DEV).int().view(T, blocks)
+    start = torch.where(torch.randint(0, 2, (T,), generator=g, device=DEV) > 0, positions, 0).int()
+    start[0] = positions[0]
+    batch = SimpleNamespace(
+        mode="decode", host_segs=None, plans=None, positions=positions, context_lens=(positions + 1).int(), block_tables=tables,
+        slot_mapping=tables.gather(1, (positions // BS)[:, None]).squeeze(1).long() * BS + positions % BS,
+        state_slots=torch.randperm(T + 2, generator=g, device=DEV)[:T].int(), cu_seqlens=rows, seg_start=start,
+        token_seg=rows[:T].contiguous())
+    cache = torch.randn(2, T * blocks, G, BS, 128, generator=g, device=DEV).bfloat16()
+    rec = torch.randn(T + 2, RH, RD, RV, generator=g, device=DEV) * 0.2
+    states = [LayerState(k=cache[0].clone(), v=cache[1].clone(), rec=rec.clone()) for _ in range(2)]
+    h = torch.randn(T, W, generator=g, device=DEV).bfloat16()
+    x = torch.randn(T, W, generator=g, device=DEV)
+    ref = x.clone()
+    post, nxt = (torch.rand(W, generator=g, device=DEV) + 0.5 for _ in range(2))
+    with torch.no_grad():
+        left, right = mix(h, batch, states[0])
+        out = ops.sandwich_residual(ref, left, post, eps, b=right, wa=mix.left_out, wb=mix.right_out, w_next=nxt,
+                                    out_dtype=torch.bfloat16)
+        got = mix.rows_step(x, h, batch, states[1], post, nxt)
+    # bf16 roundings at other places (q, k, v before their use, the branches' sums): 2^-9 of each, in a few steps behind another
+    for a, b in ((x, ref), (got, out), (states[1].rec, states[0].rec)):
+        assert (a.double() - b.double()).norm() <= 1.5e-2 * b.double().norm()
+    for a, b in ((states[1].k, states[0].k), (states[1].v, states[0].v)):
+        assert ((a.double() - b.double()).abs() <= 2 ** -6 * b.double().abs() + 2e-2).all()
 
 
 def test_residual_of_split_sums_against_float64():
