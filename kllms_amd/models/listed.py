@@ -16,6 +16,8 @@ from typing import Dict, Iterable, Optional, Tuple
 import torch
 import torch.nn as nn
 
+from .. import ops
+
 
 class ListedLayerLM(nn.Module):
     # the engine keeps a recurrent-state slot per sequence and feeds segment
@@ -56,7 +58,13 @@ class ListedLayerLM(nn.Module):
         self._after_load()
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        return self.lm_head(hidden).float()
+        head = self.lm_head
+        if (ops.only_weights(head, nn.Linear) and head.bias is None and ops.plain_call(hidden, head.weight)
+                and ops.no_global_hooks()):
+            out = ops.linear_f32(hidden, head.weight)
+            if out is not None:
+                return out
+        return head(hidden).float()
 
     def forward_prefill(self, input_ids: torch.Tensor, batch) -> torch.Tensor:
         """Logits of the LAST row of each segment: [n_seg, V]."""

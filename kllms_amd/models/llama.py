@@ -416,20 +416,10 @@ class LlamaForCausalLM(nn.Module):
         return hidden
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        """fp32 [rows, V]. On the GPU the fp32 sums of the bf16 product at every row count: rounded to bf16 at some counts
-        only, near ties between tokens would fall differently as a stream's batch grows."""
-        w = self.lm_head.weight
-        if (hidden.dim() == 2 and hidden.is_cuda and hidden.dtype == w.dtype == torch.bfloat16 and not ops._force_torch()
-                and self.lm_head.bias is None and not (torch.is_grad_enabled() and (hidden.requires_grad or w.requires_grad))):
-            # us, the library and the few-row kernel, weights out of cache, at 1 / 32 / 64 / 96 / 128 rows:
-            #   32000 x 4096   61 49 / 60 51 / 61 52 / 62 55 / 64 60        128256 x 2048  114 94 / 122 106 / 127 117 / 137 131 / 139 143
-            #   128256 x 4096  188 177 / 209 197 / 223 207 / 239 222 / 250 244
-            #   152064 x 3584  230 193 / 263 211 / 224 225 / 240 253 / 255 279
-            K = w.shape[1]
-            most = 64 if K & (K - 1) else 128 if K >= 4096 else 96
-            if hidden.shape[0] <= most and ops.linear_rows_ok(hidden, w):
-                return ops.linear_f32_rows(hidden, w)
-            return torch.mm(hidden, w.t(), out_dtype=torch.float32)
+        """fp32 [rows, V]."""
+        out = ops.linear_f32(hidden, self.lm_head.weight) if self.lm_head.bias is None else None
+        if out is not None:
+            return out
         return self.lm_head(hidden).float()
 
     def forward_prefill(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:

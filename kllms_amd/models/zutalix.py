@@ -151,8 +151,7 @@ class ZutalixForCausalLM(ListedLayerLM):
     # --- forward ------------------------------------------------------------------
     def forward_hidden(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
         assert batch.seg_start is not None, "this model takes segment batches"
-        x = ops.embed_rmsnorm(input_ids, self.embed_tokens.weight, self.embed_norm, self.eps)
-        h = ops.rmsnorm_cast(x, self.layers[0].norm1, self.eps, self.dtype)
+        x, h = ops.embed_rmsnorm(input_ids, self.embed_tokens.weight, self.embed_norm, self.eps, w_next=self.layers[0].norm1)
         n = len(self.layers)
         rows = single_rows(batch) and ops.hybrid_rows_ok(x, h, batch)
         for i, layer in enumerate(self.layers):

@@ -271,6 +271,24 @@ def linear_f32_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return _hip_or_raise().linear_rows(x, w, _none(x), 2, 1)
 
 
+def linear_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """fp32 x @ w^T from the fp32 sums of the bf16 product at every row count (rounded to bf16 at some counts only, near ties
+    between tokens would fall differently as a stream's batch grows); None where that is not to be had: not bf16 on the GPU,
+    or wanted for a gradient."""
+    if not (x.dim() == 2 and x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and not _force_torch()
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+        return None
+    # us, the library and the few-row kernel, weights out of cache, at 1 / 32 / 64 / 96 / 128 rows:
+    #   32000 x 4096   61 49 / 60 51 / 61 52 / 62 55 / 64 60        128256 x 2048  114 94 / 122 106 / 127 117 / 137 131 / 139 143
+    #   128256 x 4096  188 177 / 209 197 / 223 207 / 239 222 / 250 244
+    #   152064 x 3584  230 193 / 263 211 / 224 225 / 240 253 / 255 279
+    K = w.shape[1]
+    most = 64 if K & (K - 1) else 128 if K >= 4096 else 96
+    if x.shape[0] <= most and linear_rows_ok(x, w):
+        return linear_f32_rows(x, w)
+    return torch.mm(x, w.t(), out_dtype=torch.float32)
+
+
 # --- products of many rows (prompts) ----------------------------------------------
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
@@ -483,15 +501,18 @@ def _none(ref: torch.Tensor, dtype=None) -> torch.Tensor:
     return t
 
 
-def embed_rmsnorm(ids, table, weight, eps, pos_table=None, positions=None):
-    """fp32 rms(table[ids] (+ pos_table[positions])) * weight."""
+def embed_rmsnorm(ids, table, weight, eps, pos_table=None, positions=None, w_next=None):
+    """fp32 x = rms(table[ids] (+ pos_table[positions])) * weight; with w_next also rms(x) * w_next in the table's dtype."""
     if _gpu(table):
         out = torch.empty((ids.numel(), table.shape[1]), dtype=torch.float32, device=table.device)
+        nxt = torch.empty(out.shape, dtype=table.dtype, device=table.device) if w_next is not None else _none(table)
         has = pos_table is not None
         _seq().embed_rmsnorm(out, ids, table, weight, eps, pos_table if has else _none(table),
-                             positions if has else _none(table, torch.long))
-        return out
-    return torch_ref.embed_rmsnorm(ids, table, weight, eps, pos_table, positions)
+                             positions if has else _none(table, torch.long),
+                             w_next if w_next is not None else _none(table, torch.float32), nxt)
+        return (out, nxt) if w_next is not None else out
+    out = torch_ref.embed_rmsnorm(ids, table, weight, eps, pos_table, positions)
+    return (out, torch_ref.rmsnorm_cast(out, w_next, eps, table.dtype)) if w_next is not None else out
 
 
 def rmsnorm_cast(x, weight, eps, out_dtype):

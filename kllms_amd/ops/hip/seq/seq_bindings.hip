@@ -8,8 +8,8 @@
 #include <hip/hip_bf16.h>
 
 extern "C" {
-void seq_launch_embed_rmsnorm(float*, const int64_t*, const void*, const float*, const void*, const int64_t*, int,
-                              int, float, int, hipStream_t);
+void seq_launch_embed_rmsnorm(float*, const int64_t*, const void*, const float*, const void*, const int64_t*, const float*,
+                              void*, int, int, float, int, hipStream_t);
 void seq_launch_gelu_tanh(void*, const void*, int64_t, int, int, int, hipStream_t);
 void seq_launch_scale_softcap(float*, int64_t, float, float, hipStream_t);
 void seq_launch_scale_rows(void*, const void*, const int*, const float*, int, int, int, hipStream_t);
@@ -134,7 +134,7 @@ static int f32flag(const torch::Tensor& t) { return t.scalar_type() == at::kFloa
 
 // pos_table / positions: empty tensors for an embedding without position rows
 void embed_rmsnorm(torch::Tensor out, torch::Tensor ids, torch::Tensor table, torch::Tensor w, double eps,
-                   torch::Tensor pos_table, torch::Tensor positions) {
+                   torch::Tensor pos_table, torch::Tensor positions, torch::Tensor w_next, torch::Tensor next) {
   CHECK_F32C(out); CHECK_I64C(ids); CHECK_ACT(table); CHECK_F32C(w);
   TORCH_CHECK(table.is_contiguous() && table.dim() == 2);
   const int T = ids.numel(), W = table.size(1);
@@ -144,11 +144,16 @@ void embed_rmsnorm(torch::Tensor out, torch::Tensor ids, torch::Tensor table, to
     CHECK_ACT(pos_table); CHECK_SAME(pos_table, table); CHECK_I64C(positions);
     TORCH_CHECK(pos_table.is_contiguous() && pos_table.dim() == 2 && pos_table.size(1) == W && positions.numel() == T);
   }
+  const bool more = w_next.numel() > 0;
+  if (more) {
+    CHECK_F32C(w_next); CHECK_SAME(next, table);
+    TORCH_CHECK(w_next.numel() == W && next.is_contiguous() && next.numel() == (int64_t)T * W);
+  }
   if (T == 0) return;
   seq_launch_embed_rmsnorm(out.data_ptr<float>(), ids.data_ptr<int64_t>(), table.data_ptr(),
                            w.data_ptr<float>(), pos ? pos_table.data_ptr() : nullptr,
-                           pos ? positions.data_ptr<int64_t>() : nullptr, T, W, (float)eps, f32flag(table),
-                           cur_stream());
+                           pos ? positions.data_ptr<int64_t>() : nullptr, more ? w_next.data_ptr<float>() : nullptr,
+                           more ? next.data_ptr() : nullptr, T, W, (float)eps, f32flag(table), cur_stream());
 }
 
 void gelu_tanh(torch::Tensor out, torch::Tensor x) {

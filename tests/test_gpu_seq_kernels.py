@@ -205,3 +205,22 @@ def test_gated_delta_rule_runs_match_single_tokens(D, V):
         o2[rows] = ops.gated_delta_rule(*(t[rows].contiguous() for t in x), dt, alog, s2, slots[live].contiguous(),
                                         c1, t1)
     assert torch.equal(o1, o2) and torch.equal(s1, s2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W", [8, 100, 2048, 2056, 4104, 8192, 8200])
+def test_embedding_with_the_first_norm(W, dtype):
+    """One, two and four pieces of a row, whole and ragged; widths of the column-by-column kernel (not in eights, above 8192)."""
+    g = torch.Generator(device=DEV).manual_seed(W)
+    ids = torch.randint(0, 50, (5,), generator=g, device=DEV)
+    table = torch.randn(50, W, generator=g, device=DEV).to(dtype)
+    pos = torch.randn(9, W, generator=g, device=DEV).to(dtype)
+    positions = torch.randint(0, 9, (5,), generator=g, device=DEV)
+    w, nxt = (torch.rand(W, generator=g, device=DEV) + 0.5 for _ in range(2))
+    for more in ((None, None), (pos, positions)):
+        x, h = ops.embed_rmsnorm(ids, table, w, 1e-6, *more, w_next=nxt)
+        rx = torch_ref.embed_rmsnorm(ids, table, w, 1e-6, *more)
+        rh = torch_ref.rmsnorm_cast(rx, nxt, 1e-6, dtype)
+        assert torch.equal(x, ops.embed_rmsnorm(ids, table, w, 1e-6, *more))
+        close(x, rx, torch.float32)
+        close(h, rh, dtype)
