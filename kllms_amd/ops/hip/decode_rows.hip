@@ -10,30 +10,40 @@
 // four products: 8 launches (one more where attention splits the contexts, one where
 // gate/up is the library's), where separate reductions, rope, store and activation
 // took 11. A step of 5 rows (32 heads, width 4096, 6 layers, contexts of 560) went
-// from 948 to 774 us with these and few-row products through registers, and to 686 with those of linear_rows.hip; one of
-// 120 rows from 1516 to 1237 and 1122, one of a single row at width 2048 from 492 to 391 and 344.
+// from 948 to 774 us with these and few-row products through registers, and to 681 with those of linear_rows.hip; one of
+// 120 rows from 1516 to 1237 and 1122, one of a single row at width 2048 from 492 to 391 and 338.
 
 #include "common.h"
 
 #define DR_THREADS 1024
 
-// sum of the splits of part [S, M, n4 * 4] at (m, vector i)
-__device__ __forceinline__ f32x4 split_sum(const float* __restrict__ part, int S, int64_t MN, int64_t at) {
-  f32x4 a = *reinterpret_cast<const f32x4*>(part + at);
-#pragma unroll 4
-  for (int s = 1; s < S; ++s) {
-    const f32x4 b = *reinterpret_cast<const f32x4*>(part + s * MN + at);
+// Sum of the splits of part [S, ...] at `at`, in their order. The loads of two, four or eight splits go out together, those
+// past the last one to its place: a loop over S waits for each load by itself where S is no multiple of what is unrolled (the
+// steps above with such a loop: 688, and 344 for the single row).
+template <int B, typename V>
+__device__ __forceinline__ V splits_of(const float* __restrict__ part, int s0, int S, int64_t plane, int64_t at, V sum) {
+  V v[B];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) a[j] += b[j];
-  }
-  return a;
+  for (int s = 0; s < B; ++s) v[s] = *reinterpret_cast<const V*>(part + min(s0 + s, S - 1) * plane + at);
+#pragma unroll
+  for (int s = 0; s < B; ++s)
+    if (s0 + s < S) sum += v[s];
+  return sum;
+}
+template <typename V>
+__device__ __forceinline__ V split_sum(const float* __restrict__ part, int S, int64_t plane, int64_t at) {
+  const V zero = {};
+  if (S <= 2) return splits_of<2>(part, 0, S, plane, at, zero);
+  if (S <= 4) return splits_of<4>(part, 0, S, plane, at, zero);
+  V sum = splits_of<8>(part, 0, S, plane, at, zero);
+  for (int s0 = 8; s0 < S; s0 += 8) sum = splits_of<8>(part, s0, S, plane, at, sum);
+  return sum;
 }
 
 // residual[m] += sum of splits (written back, bf16), or residual[m] = table[ids[m]]
 // (EMBED); out[m] = rms(residual[m]) * w. One workgroup per row, the row in registers:
-// rows of up to 4 * DR_THREADS * DR_VECS elements.
-#define DR_VECS 4
-template <bool EMBED>
+// rows of up to 4 * DR_THREADS * VECS elements.
+template <bool EMBED, int VECS>
 __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
     bf16_t* __restrict__ out, bf16_t* __restrict__ residual, const float* __restrict__ part,
     const int64_t* __restrict__ ids, const bf16_t* __restrict__ table, const bf16_t* __restrict__ w, int S, int M,
@@ -48,18 +58,20 @@ __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
   // an id without a row: NaN, never another's memory, and *unknown set for the host
   const bool known = id >= 0 && id < vocab;
   if (EMBED && !known && unknown && tid == 0) __hip_atomic_store(unknown, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  f32x4 x[DR_VECS];
+  f32x4 x[VECS];
+  bf16x4_vec g[VECS];
   float ss = 0.0f;
 #pragma unroll
-  for (int k = 0; k < DR_VECS; ++k) {
+  for (int k = 0; k < VECS; ++k) {
     const int i = tid + k * DR_THREADS;
     if (i >= nvec) break;
+    g[k] = wv[i];
     bf16x4_vec r;
     if constexpr (EMBED) {
       r = known ? reinterpret_cast<const bf16x4_vec*>(table + id * n)[i] : bf16x4_vec{0x7fc0, 0x7fc0, 0x7fc0, 0x7fc0};
     } else {
       r = rv[i];
-      const f32x4 a = split_sum(part, S, (int64_t)M * n, (int64_t)m * n + i * 4);
+      const f32x4 a = split_sum<f32x4>(part, S, (int64_t)M * n, (int64_t)m * n + i * 4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) r[j] = f32_to_bf16(bf16_to_f32(r[j]) + bf16_to_f32(f32_to_bf16(a[j])));
     }
@@ -73,13 +85,12 @@ __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
   ss = block_reduce_sum<16>(ss, red);
   const float inv = rsqrtf(ss / n + eps);
 #pragma unroll
-  for (int k = 0; k < DR_VECS; ++k) {
+  for (int k = 0; k < VECS; ++k) {
     const int i = tid + k * DR_THREADS;
     if (i >= nvec) break;
-    const bf16x4_vec g = wv[i];
     bf16x4_vec o;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = f32_to_bf16(x[k][j] * inv * bf16_to_f32(g[j]));
+    for (int j = 0; j < 4; ++j) o[j] = f32_to_bf16(x[k][j] * inv * bf16_to_f32(g[k][j]));
     ov[i] = o;
   }
 }
@@ -87,12 +98,13 @@ __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
 extern "C" void launch_add_norm_rows(bf16_t* out, bf16_t* residual, const float* part, const int64_t* ids,
                                      const bf16_t* table, const bf16_t* w, int S, int M, int n, int64_t vocab,
                                      float eps, int* unknown, hipStream_t stream) {
-  if (ids)
-    hipLaunchKernelGGL(add_norm_rows_kernel<true>, dim3(M), dim3(DR_THREADS), 0, stream, out, residual, part, ids,
-                       table, w, S, M, n, vocab, eps, unknown);
-  else
-    hipLaunchKernelGGL(add_norm_rows_kernel<false>, dim3(M), dim3(DR_THREADS), 0, stream, out, residual, part, ids,
-                       table, w, S, M, n, vocab, eps, unknown);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(M), dim3(DR_THREADS), 0, stream, out, residual, part, ids, table, w, S, M, n, vocab, eps,
+                       unknown);
+  };
+  const bool narrow = n <= 4 * DR_THREADS;
+  if (ids) narrow ? go(add_norm_rows_kernel<true, 1>) : go(add_norm_rows_kernel<true, 4>);
+  else narrow ? go(add_norm_rows_kernel<false, 1>) : go(add_norm_rows_kernel<false, 4>);
 }
 
 // qkv sums [S, M, (H + 2G) * 128] (+ bias): q and k rotated (entry i with i + 64), q
@@ -110,22 +122,28 @@ __global__ void __launch_bounds__(256) rope_store_rows_kernel(
   if (head >= H + 2 * G) return;
   const int N = (H + 2 * G) * 128;
   const int64_t MN = (int64_t)M * N;
-  const float* p = part + (int64_t)m * N + head * 128 + lane;
-  float a = 0.0f, b = 0.0f;
-#pragma unroll 4
-  for (int s = 0; s < S; ++s) {
-    a += p[s * MN];
-    b += p[s * MN + 64];
+  // what is not the sums' is asked for before them
+  const bool turned = head < H + G;
+  const int64_t slot = head < H ? 0 : slots[m];
+  float c = 0.0f, sn = 0.0f, lo_bias = 0.0f, hi_bias = 0.0f;
+  if (turned) {
+    const float* cs = cos_sin + positions[m] * 128;
+    c = cs[lane];
+    sn = cs[64 + lane];
   }
   if (bias) {
-    a += bf16_to_f32(((const short*)bias)[head * 128 + lane]);
-    b += bf16_to_f32(((const short*)bias)[head * 128 + lane + 64]);
+    lo_bias = bf16_to_f32(((const short*)bias)[head * 128 + lane]);
+    hi_bias = bf16_to_f32(((const short*)bias)[head * 128 + lane + 64]);
+  }
+  const int64_t at = (int64_t)m * N + head * 128 + lane;
+  float a = split_sum<float>(part, S, MN, at), b = split_sum<float>(part + 64, S, MN, at);
+  if (bias) {
+    a += lo_bias;
+    b += hi_bias;
   }
   a = bf16_to_f32(f32_to_bf16(a));
   b = bf16_to_f32(f32_to_bf16(b));
-  if (head < H + G) {
-    const float* cs = cos_sin + positions[m] * 128;
-    const float c = cs[lane], sn = cs[64 + lane];
+  if (turned) {
     const float x = a, y = b;
     a = x * c - y * sn;
     b = y * c + x * sn;
@@ -139,7 +157,6 @@ __global__ void __launch_bounds__(256) rope_store_rows_kernel(
   }
   const bool is_k = head < H + G;
   const int g = head - H - (is_k ? 0 : G);
-  const int64_t slot = slots[m];
   const int64_t row = ((slot / block_size) * G + g) * block_size + slot % block_size;
   if constexpr (FP8) {
     const float x = bf16_to_f32(lo), y = bf16_to_f32(hi);

@@ -3,94 +3,130 @@
 //   y = a, or (rms(a) wa + rms(b / rms(what b is of)) wb) / 2;  x += rms(y) w_post;  out = rms(x) w_next in bf16
 //
 // A row is one workgroup's: its sums are the bytes, 64 to 128 KB of them, and the three reductions the chain behind. Four
-// columns a thread and load, kept in registers through all passes. 40 rows of 2048 in 8 shares: 4.7 us
-// of a step, 8.6 with two branches (4.8 and 6.5 from bf16 products, which took 12 and 12 to 17 us themselves).
+// columns a thread and load, kept in registers through all passes, and all loads before the first wait. 40 rows of 2048 in 8
+// shares: 3.9 us of a step, with two branches of 4 shares 5.4 (4.7 and 8.3 with the loads one by one behind the shares that
+// fill a batch, and three of the norms' weights behind the sums).
 
 #include "seq_common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define SR_THREADS 512
-#define SR_VECS 4          // W <= 4 * 4 * 512
 
-template <bool DUAL>
+// Sums of S splits a plane apart, in their order; the loads of four or eight go out together, those past the last one to its
+// place
+__device__ __forceinline__ f32x4 split_sum(const float* __restrict__ p, int S, int64_t plane) {
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  if (S <= 4) {
+    f32x4 v[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) v[s] = *reinterpret_cast<const f32x4*>(p + min(s, S - 1) * plane);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      if (s < S) sum += v[s];
+    return sum;
+  }
+  for (int s0 = 0; s0 < S; s0 += 8) {
+    f32x4 v[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) v[s] = *reinterpret_cast<const f32x4*>(p + min(s0 + s, S - 1) * plane);
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      if (s0 + s < S) sum += v[s];
+  }
+  return sum;
+}
+
+// VECS: W <= 4 * VECS * SR_THREADS
+template <bool DUAL, int VECS>
 __global__ void __launch_bounds__(SR_THREADS) sandwich_rows_kernel(
     float* __restrict__ x, const float* __restrict__ a, int SA, const float* __restrict__ b, int SB,
     const float* __restrict__ wa, const float* __restrict__ wb, const float* __restrict__ w_post,
     const float* __restrict__ w_next, bfraw* __restrict__ out, int T_, int W, float eps,
     const float* __restrict__ squares, int heads, float per) {
-  __shared__ float scratch[16];
+  __shared__ float scratch[2][16];
   const int t = blockIdx.x, tid = threadIdx.x, nvec = W / 4;
   const int64_t plane = (int64_t)T_ * W;
   const float inv_w = 1.0f / (float)W;
-  auto sums = [&](const float* p, int S, f32x4 (&v)[SR_VECS]) {
-    float ss = 0.0f;
-#pragma unroll
-    for (int k = 0; k < SR_VECS; ++k) {
-      v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const int i = tid + k * SR_THREADS;
-      if (i >= nvec) break;
-      const float* q = p + (int64_t)t * W + i * 4;
-#pragma unroll 8
-      for (int s = 0; s < S; ++s) {
-        const f32x4 u = *reinterpret_cast<const f32x4*>(q + s * plane);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[k][e] += u[e];
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ss += v[k][e] * v[k][e];
-    }
-    return ss;
-  };
-  f32x4 y[SR_VECS];
-  float ss = sums(a, SA, y);
-  if constexpr (DUAL) {
-    // b is of a product whose rows' norm is put off to here
-    float sq = 0.0f;
+  f32x4 y[VECS], z[VECS], old[VECS], post[VECS], next[VECS], ga[VECS], gb[VECS];
+  float ss = 0.0f, sb = 0.0f, sq = 0.0f;
+  // b is of a product whose rows' norm is put off to here
+  if constexpr (DUAL)
     for (int i = tid % WAVE; i < heads; i += WAVE) sq += squares[(int64_t)t * heads + i];
-    f32x4 z[SR_VECS];
-    float sb = sums(b, SB, z);
-    const float rs = 1.0f / sqrtf(wave_sum(sq) * per + eps);
-    sb *= rs * rs;
-    const float ra = 1.0f / sqrtf(block_sum(ss, scratch) * inv_w + eps);
-    const float rb = 1.0f / sqrtf(block_sum(sb, scratch) * inv_w + eps);
-    ss = 0.0f;
 #pragma unroll
-    for (int k = 0; k < SR_VECS; ++k) {
-      const int i = tid + k * SR_THREADS;
-      if (i >= nvec) break;
-      const f32x4 ga = reinterpret_cast<const f32x4*>(wa)[i], gb = reinterpret_cast<const f32x4*>(wb)[i];
+  for (int k = 0; k < VECS; ++k) {
+    const int i = tid + k * SR_THREADS;
+    if (i >= nvec) break;
+    const int64_t at = (int64_t)t * W + i * 4;
+    old[k] = *reinterpret_cast<const f32x4*>(x + at);
+    post[k] = reinterpret_cast<const f32x4*>(w_post)[i];
+    next[k] = reinterpret_cast<const f32x4*>(w_next)[i];
+    if constexpr (DUAL) {
+      ga[k] = reinterpret_cast<const f32x4*>(wa)[i];
+      gb[k] = reinterpret_cast<const f32x4*>(wb)[i];
+      z[k] = split_sum(b + at, SB, plane);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sb += z[k][e] * z[k][e];
+    }
+    y[k] = split_sum(a + at, SA, plane);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss += y[k][e] * y[k][e];
+  }
+  if constexpr (DUAL) {
+    const float rs = 1.0f / sqrtf(group_sum<1>(sq) * per + eps);
+    // both sums over the row behind one barrier
+    const int lane = tid % WAVE, wave = tid / WAVE;
+    ss = group_sum<1>(ss);
+    sb = group_sum<1>(sb * rs * rs);
+    if (lane == 0) { scratch[0][wave] = ss; scratch[1][wave] = sb; }
+    __syncthreads();
+    ss = sb = 0.0f;
+#pragma unroll
+    for (int i = 0; i < SR_THREADS / WAVE; ++i) { ss += scratch[0][i]; sb += scratch[1][i]; }
+    const float ra = 1.0f / sqrtf(ss * inv_w + eps), rb = 1.0f / sqrtf(sb * inv_w + eps);
+    ss = 0.0f;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < VECS; ++k) {
+      if (tid + k * SR_THREADS >= nvec) break;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        y[k][e] = 0.5f * (y[k][e] * ra * ga[e] + z[k][e] * rs * rb * gb[e]);
+        y[k][e] = 0.5f * (y[k][e] * ra * ga[k][e] + z[k][e] * rs * rb * gb[k][e]);
         ss += y[k][e] * y[k][e];
       }
     }
   }
-  const float ry = 1.0f / sqrtf(block_sum(ss, scratch) * inv_w + eps);
+  // two sums, one behind the other, each in a place of its own
+  auto row_sum = [&](float v, float* place) {
+    v = group_sum<1>(v);
+    if (tid % WAVE == 0) place[tid / WAVE] = v;
+    __syncthreads();
+    v = 0.0f;
+#pragma unroll
+    for (int i = 0; i < SR_THREADS / WAVE; ++i) v += place[i];
+    return v;
+  };
+  const float ry = 1.0f / sqrtf(row_sum(ss, scratch[0]) * inv_w + eps);
   float sx = 0.0f;
 #pragma unroll
-  for (int k = 0; k < SR_VECS; ++k) {
+  for (int k = 0; k < VECS; ++k) {
     const int i = tid + k * SR_THREADS;
     if (i >= nvec) break;
-    f32x4* px = reinterpret_cast<f32x4*>(x + (int64_t)t * W) + i;
-    const f32x4 old = *px, g = reinterpret_cast<const f32x4*>(w_post)[i];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      y[k][e] = old[e] + y[k][e] * ry * g[e];
+      y[k][e] = old[k][e] + y[k][e] * ry * post[k][e];
       sx += y[k][e] * y[k][e];
     }
-    *px = y[k];
+    reinterpret_cast<f32x4*>(x + (int64_t)t * W)[i] = y[k];
   }
-  const float rx = 1.0f / sqrtf(block_sum(sx, scratch) * inv_w + eps);
+  const float rx = 1.0f / sqrtf(row_sum(sx, scratch[1]) * inv_w + eps);
 #pragma unroll
-  for (int k = 0; k < SR_VECS; ++k) {
+  for (int k = 0; k < VECS; ++k) {
     const int i = tid + k * SR_THREADS;
     if (i >= nvec) break;
-    const f32x4 g = reinterpret_cast<const f32x4*>(w_next)[i];
     uint2 o;
-    o.x = bf_bits(y[k][0] * rx * g[0]) | (bf_bits(y[k][1] * rx * g[1]) << 16);
-    o.y = bf_bits(y[k][2] * rx * g[2]) | (bf_bits(y[k][3] * rx * g[3]) << 16);
+    o.x = bf_bits(y[k][0] * rx * next[k][0]) | (bf_bits(y[k][1] * rx * next[k][1]) << 16);
+    o.y = bf_bits(y[k][2] * rx * next[k][2]) | (bf_bits(y[k][3] * rx * next[k][3]) << 16);
     reinterpret_cast<uint2*>(out + (int64_t)t * W)[i] = o;
   }
 }
@@ -104,7 +140,9 @@ extern "C" void seq_launch_sandwich_rows(float* x, const float* a, int SA, const
     hipLaunchKernelGGL(kernel, dim3(T_), dim3(SR_THREADS), 0, st, x, a, SA, b, SB, wa, wb, w_post, w_next, (bfraw*)out, T_, W,
                        eps, squares, heads, per);
   };
-  b ? go(sandwich_rows_kernel<true>) : go(sandwich_rows_kernel<false>);
+  const bool narrow = W <= 4 * SR_THREADS;
+  if (b) narrow ? go(sandwich_rows_kernel<true, 1>) : go(sandwich_rows_kernel<true, 4>);
+  else narrow ? go(sandwich_rows_kernel<false, 1>) : go(sandwich_rows_kernel<false, 4>);
 }
 
 // What a parallel sublayer's input product, as split sums part [S, T, N], is wanted for, in one launch: sums (+ bias), then for

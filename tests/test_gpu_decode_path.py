@@ -493,3 +493,13 @@ def test_short_prompts_match_general_path(preset, lens):
     off = (got - want).norm(dim=-1) / want.norm(dim=-1)
     assert float(off.max()) < (0.5 if preset == "mid-mixtral" else 0.05)      # a routed row may change its experts
     assert torch.equal(kv[0], eng.kv.k_all[0])
+
+
+@pytest.mark.parametrize("S,M,n", [(4, 3, 4096), (9, 2, 2048), (17, 5, 4100), (16, 1, 16384)])
+def test_add_norm_rows_at_the_batches_of_splits(S, M, n):
+    test_add_and_embed_norm_rows(S, M, n)
+
+
+@pytest.mark.parametrize("S,M", [(2, 3), (4, 1), (5, 7), (9, 2), (17, 5)])
+def test_rope_store_rows_at_the_batches_of_splits(S, M):
+    test_rope_store_rows(S, M, 8, 2, 16, True, False)

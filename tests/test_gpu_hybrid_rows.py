@@ -205,6 +205,28 @@ def test_residual_of_split_sums_against_float64():
     assert ((got.double() - out).abs() <= 2 ** -8 * out.abs() + 2e-2).all()
 
 
+@pytest.mark.parametrize("W,ff", [(128, 1152), (256, 2304), (128, 4352), (2176, 640), (4224, 1280)])
+def test_residual_of_many_split_sums_against_float64(W, ff):
+    """4, 9 and 17 splits; rows of more than one vector a thread, the last one ragged."""
+    C, T = ops._seq(), 5
+    g = torch.Generator(device=DEV).manual_seed(ff)
+    h = torch.randn(T, W, generator=g, device=DEV).bfloat16()
+    x = torch.randn(T, W, generator=g, device=DEV)
+    w_in = (torch.randn(2 * ff, W, generator=g, device=DEV) * W ** -0.5).bfloat16()
+    w_down = (torch.randn(W, ff, generator=g, device=DEV) * ff ** -0.5).bfloat16()
+    post, nxt = (torch.rand(W, generator=g, device=DEV) + 0.5 for _ in range(2))
+    gate, up = (h.double() @ w_in.double().t()).chunk(2, -1)
+    gate, up = gate.clamp(max=2.0), up.clamp(-2.0, 2.0)
+    act = (gate * torch.sigmoid(1.5 * gate) * (up + 1)).bfloat16().double()
+    y = act @ w_down.double().t()
+    ref = x.double() + y / torch.sqrt((y * y).mean(-1, keepdim=True) + 1e-6) * post.double()
+    out = ref / torch.sqrt((ref * ref).mean(-1, keepdim=True) + 1e-6) * nxt.double()
+    got = C.hybrid_glu_rows(x, h, w_in, w_down, post, nxt, 2.0, 1.5, 1e-6)
+    # as above, of more terms: 2^-8 of the few activations whose rounding falls the other way
+    assert (x.double() - ref).abs().max() <= 2e-2
+    assert ((got.double() - out).abs() <= 2 ** -8 * out.abs() + 2e-2).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("H,G,V", [(4, 2, 128), (3, 3, 16), (2, 1, 80)])
 @pytest.mark.parametrize("lens", [[64], [16, 17, 200, 31, 1, 300, 0, 33], [300, 64]])
