@@ -224,3 +224,32 @@ def test_embedding_with_the_first_norm(W, dtype):
         assert torch.equal(x, ops.embed_rmsnorm(ids, table, w, 1e-6, *more))
         close(x, rx, torch.float32)
         close(h, rh, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,G,D,Dv,R,pad", [(16, 4, 128, 128, 48, 0), (3, 1, 128, 128, 64, 8), (5, 2, 24, 40, 4, 16), (4, 4, 8, 8, 0, 8),
+                                            (2, 1, 512, 16, 256, 0), (3, 2, 40, 40, 6, 0), (2, 2, 16, 16, 8, 3)])
+def test_rope_pairs_store_by_rows(H, G, D, Dv, R, pad, dtype):
+    """A workgroup to a row: more and fewer pieces than threads, none, some and all entries turned, strided rows; and what the
+    kernel of a wave to a head keeps: pairs not in fours, rows not in eights."""
+    T, NB, BS = 7, 9, 4
+    fused = rnd(T, H * D + G * D + G * Dv + pad, dtype=dtype, seed=1)
+    pos = torch.arange(T, device=DEV) * 517
+    slots = torch.randperm(NB * BS, generator=torch.Generator().manual_seed(2))[:T].to(DEV)
+    inv_freq = torch.rand(R, generator=torch.Generator().manual_seed(3)).to(DEV)
+    for own_values in (True, False):
+        if not own_values and Dv != D:
+            continue
+        res = []
+        for impl in (ops, torch_ref):
+            f = fused.clone()
+            q, k = f[:, :H * D].unflatten(1, (H, D)), f[:, H * D:(H + G) * D].unflatten(1, (G, D))
+            v = f[:, (H + G) * D:(H + G) * D + G * Dv].unflatten(1, (G, Dv)) if own_values else None
+            k1, v1 = rnd(NB, G, BS, D, dtype=dtype, seed=4), rnd(NB, G, BS, Dv, dtype=dtype, seed=5)
+            fresh = torch.zeros(T, 2, G, D, dtype=dtype, device=DEV) if impl is ops and Dv == D else None
+            impl.rope_pairs_store(q, k, v, pos, inv_freq, k1, v1, slots, *([fresh] if fresh is not None else []))
+            res.append((f, k1, v1))
+            if fresh is not None:
+                assert torch.equal(fresh[:, 0], k1[slots // BS, :, slots % BS]) and torch.equal(fresh[:, 1], v1[slots // BS, :, slots % BS])
+        for a, b in zip(*res):
+            close(a, b, dtype)
