@@ -392,15 +392,7 @@ def sample(
     dbg: Optional[torch.Tensor] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     if logits.is_cuda and not _force_torch():
-        B = logits.shape[0]
-        tokens = torch.empty(B, dtype=torch.long, device=logits.device)
-        logprobs = torch.empty(B, dtype=torch.float32, device=logits.device)
-        _hip_or_raise().sample(
-            tokens, logprobs, logits, temperatures, top_ps, top_ks, seeds, steps,
-            mask if mask is not None else _none(logits, torch.int32),
-            dbg if dbg is not None else _none(logits, torch.float32),
-        )
-        return tokens, logprobs
+        return _hip_or_raise().sample(logits, temperatures, top_ps, top_ks, seeds, steps, mask, dbg)
     return torch_ref.sample(logits, temperatures, top_ps, top_ks, seeds, steps, mask)
 
 

@@ -242,22 +242,24 @@ void attn_prefill_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cach
                             BS, (int)tables.size(1), cur_stream());
 }
 
-void sample(torch::Tensor tokens, torch::Tensor logprobs, torch::Tensor logits,
-            torch::Tensor temperatures, torch::Tensor top_ps, torch::Tensor top_ks,
-            torch::Tensor seeds, torch::Tensor steps, torch::Tensor mask,
-            torch::Tensor dbg) {
+// (tokens, logprobs). The results are allocated here: 16 rows take 8.8 us on the device, and from Python the two allocations
+// kept it waiting
+std::tuple<torch::Tensor, torch::Tensor> sample(torch::Tensor logits, torch::Tensor temperatures, torch::Tensor top_ps,
+                                                torch::Tensor top_ks, torch::Tensor seeds, torch::Tensor steps,
+                                                std::optional<torch::Tensor> mask, std::optional<torch::Tensor> dbg) {
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() && logits.scalar_type() == at::kFloat);
   const int B = logits.size(0), V = logits.size(1);
-  const uint32_t* mptr = mask.numel() > 0
-      ? reinterpret_cast<const uint32_t*>(mask.data_ptr<int>()) : nullptr;
-  if (B == 0 || V == 0) return;
+  const auto whole = torch::dtype(torch::kLong).device(logits.device());
+  auto tokens = torch::empty({B}, whole), logprobs = torch::empty({B}, logits.options());
+  const uint32_t* mptr = mask && mask->numel() > 0 ? reinterpret_cast<const uint32_t*>(mask->data_ptr<int>()) : nullptr;
+  if (B == 0 || V == 0) return {tokens, logprobs};
   // per-slice results and lists
-  auto parts = torch::empty({sample_room(B, V, mptr != nullptr)},
-                            torch::dtype(torch::kLong).device(logits.device()));
+  auto parts = torch::empty({sample_room(B, V, mptr != nullptr)}, whole);
   launch_sample(tokens.data_ptr<int64_t>(), logprobs.data_ptr<float>(), parts.data_ptr(),
                 logits.data_ptr<float>(), temperatures.data_ptr<float>(), top_ps.data_ptr<float>(),
                 top_ks.data_ptr<int>(), seeds.data_ptr<int64_t>(), steps.data_ptr<int64_t>(), mptr,
-                B, V, dbg.numel() ? dbg.data_ptr<float>() : nullptr, cur_stream());
+                B, V, dbg && dbg->numel() ? dbg->data_ptr<float>() : nullptr, cur_stream());
+  return {tokens, logprobs};
 }
 
 torch::Tensor mfma_selftest(torch::Tensor A, torch::Tensor B) {
