@@ -10,8 +10,10 @@
 // four products: 8 launches (one more where attention splits the contexts, one where
 // gate/up is the library's), where separate reductions, rope, store and activation
 // took 11. A step of 5 rows (32 heads, width 4096, 6 layers, contexts of 560) went
-// from 948 to 774 us with these and few-row products through registers, and to 681 with those of linear_rows.hip; one of
-// 120 rows from 1516 to 1237 and 1122, one of a single row at width 2048 from 492 to 391 and 338.
+// from 948 to 774 us with these and few-row products through registers, and to 676 with those of linear_rows.hip; one of
+// 120 rows from 1516 to 1237 and 1114, one of a single row at width 2048 from 492 to 391 and 330.
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -38,6 +40,29 @@ __device__ __forceinline__ V split_sum(const float* __restrict__ part, int S, in
   V sum = splits_of<8>(part, 0, S, plane, at, zero);
   for (int s0 = 8; s0 < S; s0 += 8) sum = splits_of<8>(part, s0, S, plane, at, sum);
   return sum;
+}
+
+// Sum over the workgroup, for all its threads. The chain of a row runs through it: register moves within a wave and one
+// barrier, where shuffles through LDS and two took 0.6 us longer.
+__device__ __forceinline__ float row_sum(float v, float* scratch) {
+  auto moved = [](float x, auto how) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), decltype(how)::value, 0xf, 0xf, false));
+  };
+  auto over_wave = [&](float x, bool halves) {
+    x += moved(x, std::integral_constant<int, 0xb1>());    // quad_perm 1 0 3 2
+    x += moved(x, std::integral_constant<int, 0x4e>());    // quad_perm 2 3 0 1
+    x += moved(x, std::integral_constant<int, 0x141>());   // row_half_mirror
+    x += moved(x, std::integral_constant<int, 0x140>());   // row_mirror
+    if (!halves) return x;
+    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+  };
+  v = over_wave(v, true);
+  if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return over_wave(scratch[threadIdx.x & 15], false);      // 16 waves
 }
 
 // residual[m] += sum of splits (written back, bf16), or residual[m] = table[ids[m]]
@@ -82,7 +107,7 @@ __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
       ss += x[k][j] * x[k][j];
     }
   }
-  ss = block_reduce_sum<16>(ss, red);
+  ss = row_sum(ss, red);
   const float inv = rsqrtf(ss / n + eps);
 #pragma unroll
   for (int k = 0; k < VECS; ++k) {

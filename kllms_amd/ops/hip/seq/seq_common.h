@@ -46,8 +46,14 @@ __device__ __forceinline__ float wave_max(float v) {
 // Gated delta rule, 8 prompts of 1000 tokens, D = V = 64: 826 us with xor shuffles, 659 so.
 template <int COLS>
 __device__ __forceinline__ float group_sum(float v) {
+  if constexpr (COLS == 1) {
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0xb1, 0xf, 0xf, false));   // quad_perm 1 0 3 2
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x4e, 0xf, 0xf, false));   // quad_perm 2 3 0 1
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x141, 0xf, 0xf, false));  // row_half_mirror
+  } else {
 #pragma unroll
-  for (int off = COLS; off < 8; off <<= 1) v += __shfl_xor(v, off);
+    for (int off = COLS; off < 8; off <<= 1) v += __shfl_xor(v, off);
+  }
   if constexpr (COLS <= 8)
     v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x128, 0xf, 0xf, false));  // row_ror:8
   if constexpr (COLS <= 16) {

@@ -4,7 +4,7 @@
 //
 // A row is one workgroup's: its sums are the bytes, 64 to 128 KB of them, and the three reductions the chain behind. Four
 // columns a thread and load, kept in registers through all passes, and all loads before the first wait. 40 rows of 2048 in 8
-// shares: 3.9 us of a step, with two branches of 4 shares 5.4 (4.7 and 8.3 with the loads one by one behind the shares that
+// shares: 3.9 us of a step, with two branches of 4 shares 4.8 (4.7 and 8.3 with the loads one by one behind the shares that
 // fill a batch, and three of the norms' weights behind the sums).
 
 #include "seq_common.h"
