@@ -270,13 +270,14 @@ __global__ void __launch_bounds__(PR_THREADS, DR <= 8 ? 4 : 2) parallel_rows_ker
 #pragma unroll
       for (int i = 0; i < DR; ++i) {
         const int d = i * RG + rg;
-        const float k = ks[min(d, RD - 1)], q = d < RD ? qs[min(d, RD - 1)] : 0.0f;
+        const bool on = d < RD;
+        const float k = ks[min(d, RD - 1)], q = on ? qs[min(d, RD - 1)] : 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          st[i][e] = dec * st[i][e] + k * val[e];
+          st[i][e] = on ? dec * st[i][e] + k * val[e] : 0.0f;
           read[e] += st[i][e] * q;
         }
-        if (d < RD) *reinterpret_cast<f32x4*>(head + (int64_t)d * RV + c0 + quad * 4) = st[i];
+        if (on) *reinterpret_cast<f32x4*>(head + (int64_t)d * RV + c0 + quad * 4) = st[i];
       }
       *reinterpret_cast<f32x4*>(red + rg * VB + quad * 4) = read;
     }
@@ -520,7 +521,7 @@ __global__ void __launch_bounds__(DR_THREADS, DR * HP <= 8 ? 4 : 2) delta_rows_k
           const float dc = dec[(hh + p) * D + d], k = on ? ks[d] : 0.0f, q = on ? qs[d] : 0.0f;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            st[p][i][e] *= dc;
+            st[p][i][e] = on ? st[p][i][e] * dc : 0.0f;
             pred[e] += st[p][i][e] * k;
             read[e] += st[p][i][e] * q;
           }
@@ -576,7 +577,7 @@ static inline size_t delta_rows_lds(int rep, int D, int V, int ranks, int HP) {
 // a workgroup keeps within 64 KB
 extern "C" bool seq_delta_rows_takes(int H, int G, int D, int V, int K, int RA, int RB) {
   const int rep = H / G;
-  return D <= 256 && V % 4 == 0 && K >= 2 && K <= 16 && RA % 8 == 0 && RB % 8 == 0 &&
+  return D <= 256 && V % 4 == 0 && K >= 2 && K <= 16 && RA >= 8 && RA % 8 == 0 && RB >= 8 && RB % 8 == 0 &&
          delta_rows_lds(rep, D, V, RA + RB, rep % 2 == 0 ? 2 : 1) <= 65536;
 }
 
