@@ -511,6 +511,7 @@ torch::Tensor moe_combine(torch::Tensor y, torch::Tensor weights, torch::Tensor 
 
 // --- products of a few rows (linear_rows.hip) ---------------------------------
 extern "C" int linear_rows_most(int form);
+extern "C" int64_t linear_rows_strides();
 extern "C" int launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
                                    int K, int x_stride, int form, int splits, float limit, float alpha, hipStream_t stream);
 extern "C" int linear_rows_splits(int M, int N, int K);
@@ -529,13 +530,15 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, torch::Tensor bias, 
               "linear_rows: M in 1..", linear_rows_most((int)form), ", K a multiple of 128, N of 16");
   TORCH_CHECK(bias.numel() == 0 || (form == 1 && bias.numel() == N && bias.is_contiguous() &&
                                     bias.scalar_type() == at::kBFloat16), "bias: bf16 [N], bf16 form only");
+  if (x.stride(0) >= linear_rows_strides()) x = x.contiguous();    // one row is contiguous whatever its stride
+  const int x_stride = M == 1 ? K : (int)x.stride(0);
   int S = 1;
   if (form == 0) S = splits > 0 ? (int)std::min<int64_t>(splits, K / 64) : linear_rows_splits(M, N, K);
   auto out = form == 0 ? torch::empty({S, M, N}, x.options().dtype(torch::kFloat))
            : form == 2 ? torch::empty({M, N}, x.options().dtype(torch::kFloat))
                        : torch::empty({M, form == 3 ? N / 2 : N}, x.options());
   TORCH_CHECK(launch_linear_rows(out.data_ptr(), cbf(x), cbf(w), bias.numel() ? cbf(bias) : nullptr, M, N, K,
-                                 (int)x.stride(0), (int)form, S, 0.0f, 0.0f, cur_stream()) == 0,
+                                 x_stride, (int)form, S, 0.0f, 0.0f, cur_stream()) == 0,
               "linear_rows: 160 KB of LDS are not available");
   return out;
 }

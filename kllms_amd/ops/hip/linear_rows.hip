@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(TP_THREADS, 1) linear_rows_kernel(
       }
     }
   }
-  const TileRows xr(xk, m0 + wave * MJ * 8, m_end, MJ * 8, x_stride, lane);
+  const TileRows xr(xk, m0 + wave * MJ * 8, m_end, MJ * 8, x_stride, stages * TP_K, lane);
   const TileRows wr(wk, n_put, columns, 8 * NI, w_row, lane);
   // the XCDs begin at different k: rows of a power of two of bytes would have all of them at the same memory channels
   tile_product<MJ, NI, KB * 1024>(acc, wr, xr, stages, stages * xcd / 8, smem);
@@ -212,7 +212,10 @@ static int linear_rows_form(const LinearPlan& p, void* out, const bf16_t* x, con
 // Rows up to which a form is taken
 extern "C" int linear_rows_most(int form) { return form == LR_PART ? 384 : form == LR_SILU ? 256 : 128; }
 
-// 0, or -1 where the LDS cannot be had
+// x_stride from which on 64 rows' offsets would leave 32 bits
+extern "C" int64_t linear_rows_strides() { return 1 << 25; }
+
+// 0, or -1 where the LDS cannot be had. x_stride: any below linear_rows_strides(), 0 and less than K too
 extern "C" int launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N, int K,
                                   int x_stride, int form, int splits, float limit, float alpha, hipStream_t stream) {
   const LinearPlan p = linear_plan(M, N, K, form);

@@ -102,12 +102,17 @@ __device__ __forceinline__ void tp_copy_at(uint64_t at, uint32_t lds) {
 
 // Rows of an operand in memory order, 8 to a copy: from row ``first`` of p on, those before ``end`` (1 or more) and
 // ``most`` of them at most; the others read as zeros. Behind the end altogether the last row stands in, so that the
-// range always holds a row: what comes of it belongs to rows or columns that are not stored.
+// range always holds a row: what comes of it belongs to rows or columns that are not stored. K: elements from a row to the
+// next, width: those of a row that are read. The range ends with the last row's: rows may overlap or be one and the same
+// (K below width), and then what does not exist reads others' values, for rows that are not stored either.
 struct TileRows {
   u32x4 range;
   uint32_t at[8];            // this lane's offset in each copy: the same registers for all operands of one K
   __device__ __forceinline__ TileRows(const bf16_t* p, int first, int end, int most, int K, int lane)
-      : range(tp_range(p + (int64_t)min(first, end - 1) * K, (uint32_t)min(end - min(first, end - 1), most) * K * 2)) {
+      : TileRows(p, first, end, most, K, K, lane) {}
+  __device__ __forceinline__ TileRows(const bf16_t* p, int first, int end, int most, int K, int width, int lane)
+      : range(tp_range(p + (int64_t)min(first, end - 1) * K,
+                       ((uint32_t)(min(end - min(first, end - 1), most) - 1) * K + width) * 2)) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       at[i] = (uint32_t)(i * 8 + (lane >> 3)) * K * 2 + (((lane & 7) ^ (lane >> 3)) << 4);

@@ -503,3 +503,48 @@ def test_add_norm_rows_at_the_batches_of_splits(S, M, n):
 @pytest.mark.parametrize("S,M", [(2, 3), (4, 1), (5, 7), (9, 2), (17, 5)])
 def test_rope_store_rows_at_the_batches_of_splits(S, M):
     test_rope_store_rows(S, M, 8, 2, 16, True, False)
+
+
+@pytest.mark.parametrize("M", [1, 2, 5, 64, 128, 129, 384])
+@pytest.mark.parametrize("stride", [0, 8, 120, 512, 648, (1 << 25) - 8, 1 << 25])
+@pytest.mark.parametrize("N,K", [(64, 640), (5184, 640)])
+def test_linear_rows_of_repeated_and_overlapping_rows(M, stride, N, K):
+    """Rows that are one and the same, that overlap, and that lie further apart than 32 bits of offsets reach over a tile."""
+    if stride > K + 8 and M > 5:
+        M = 65 if stride < 1 << 25 and M == 128 and N == 64 else 5       # 4 GiB of rows once
+    g = torch.Generator(device=DEV).manual_seed(M + stride + N)
+    x = torch.empty((M - 1) * stride + K, dtype=torch.bfloat16, device=DEV).as_strided((M, K), (stride, 1))
+    for m in range(M):
+        x[m].normal_(generator=g)
+    w = (torch.randn(N, K, generator=g, device=DEV) * 0.05).bfloat16()
+    xd, wt = x.double().contiguous(), w.double().t().contiguous()
+    ref = xd @ wt
+    tol = K * 2 ** -24 * (xd.abs() @ wt.abs())
+    C, none = ops._hip_or_raise(), ops._none(x)
+    for splits in (0, 1, 5):
+        assert ((C.linear_rows(x, w, none, 0, splits).double().sum(0) - ref).abs() <= tol).all()
+    if M <= 256:
+        gate, up = ref.chunk(2, -1)
+        tg, tu = tol.chunk(2, -1)
+        full = torch.nn.functional.silu(gate) * up
+        assert ((ops.linear_silu_rows(x, w).double() - full).abs()
+                <= 1.1 * tg * (up.abs() + tu) + tu * gate.abs() + 2 ** -8 * full.abs() + 1e-6).all()
+    if M <= 128:
+        assert ops.linear_rows_ok(x, w)
+        assert ((ops.linear_f32(x, w).double() - ref).abs() <= tol).all()
+        assert ((C.linear_rows(x, w, none, 1, 1).double() - ref).abs() <= tol + 2 ** -8 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("preset", ["mid-llama", "mid-zutalix"])
+@pytest.mark.parametrize("rows", [1, 5, 64, 128])
+def test_logits_of_one_row_repeated(preset, rows):
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+
+    m = LLMEngine(EngineConfig(model=preset, max_kv_blocks=64, use_hip_graphs=False, seed=3)).model
+    w = m.lm_head.weight
+    h = torch.randn(1, w.shape[1], generator=torch.Generator().manual_seed(rows)).bfloat16().to(DEV)
+    with torch.inference_mode():
+        out = m.compute_logits(h.expand(rows, -1))
+    tol = w.shape[1] * 2 ** -24 * (h.double().abs() @ w.double().abs().t().contiguous())
+    assert ((out.double() - h.double() @ w.double().t().contiguous()).abs() <= tol).all()
