@@ -821,7 +821,8 @@ __global__ void __launch_bounds__(NT) sample_final_kernel(
       __syncthreads();
       const int cut = sh_cut;
       const unsigned int n = cut < 0 ? 0 : hist_cnt[cut];
-      if (cut >= 0 && n <= WAVE) {
+      // with no mass left to fill (top-p 0) what ties with the max is in, which the general way finds
+      if (cut >= 0 && n <= WAVE && sh_need_mass > 0.0f) {
 #pragma unroll
         for (int k = 0; k < SLIST / NT; ++k)
           if (bin[k] == cut) {

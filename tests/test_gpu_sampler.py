@@ -351,3 +351,21 @@ def test_cut_in_a_crowded_bin_of_the_lists(B, V, near, width):
         t = int(toks[b])
         key = x + gumbel(int(seeds[b]), int(steps[b]), V)
         assert x[t] >= low and key[t] >= key[must].max() - max(1e-3, 4e-7 * V)
+
+
+@pytest.mark.parametrize("top_k", [0, 30])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("B,V", [(2, 50257), (7, 128256), (40, 32000), (3, 3000), (600, 8192)])
+def test_top_p_zero_draws_among_the_highest(B, V, masked, top_k):
+    """Top-p 0 leaves what ties with the max, with the slices' lists and without: the draw is among those."""
+    g = torch.Generator().manual_seed(V + B)
+    logits = torch.randn(B, V, generator=g) - 6.0
+    at = [7, V // 3, V // 2 + 1, V - 2]
+    logits[:, at] = 2.5
+    mask = torch.full((B, (V + 31) // 32), -1, dtype=torch.int32).to(DEV) if masked else None
+    seeds, steps = torch.randint(0, 2**40, (B,), generator=g), torch.randint(0, 99, (B,), generator=g)
+    toks, _ = ops.sample(logits.to(DEV), torch.ones(B, device=DEV), torch.zeros(B, device=DEV),
+                         torch.full((B,), top_k, dtype=torch.int32, device=DEV), seeds.to(DEV), steps.to(DEV), mask)
+    for b in range(0, B, 1 if B < 100 else 41):
+        h = draws(int(seeds[b]), int(steps[b]), V)[at]
+        assert int(toks[b]) in at and h[at.index(int(toks[b]))] == h.max()
