@@ -324,22 +324,28 @@ class LlamaForCausalLM(nn.Module):
         return rows <= most and self._only_weights(input_ids, batch)
 
     def _only_weights(self, input_ids: torch.Tensor, batch: ForwardBatch) -> bool:
-        """Whether the layers' modules are the plain ones and nothing looks on at their calls."""
+        """Whether the layers' modules are the plain ones, nothing looks on at their calls, and their weights are such as the
+        few-row products read. Other weights are the library's."""
         plain = ops.only_weights
         if not (ops.no_global_hooks() and ops.plain_call(input_ids, batch.positions, batch.slot_mapping)
                 and plain(self.embed_tokens, nn.Embedding)
                 and not (torch.is_grad_enabled() and any(p.requires_grad for p in self.parameters()))):
             return False
+        read = [self.embed_tokens.weight]
         for layer in self.layers:
             at, mlp = layer.self_attn, layer.mlp
-            if not (plain(layer, self.layer_cls) and plain(at, LlamaAttention) and plain(at.qkv_proj, ColumnParallelLinear)
-                    and plain(at.o_proj, RowParallelLinear)):
+            qkv, o = at.qkv_proj, at.o_proj
+            if not (plain(layer, self.layer_cls) and plain(at, LlamaAttention) and plain(qkv, ColumnParallelLinear)
+                    and plain(o, RowParallelLinear)):
                 return False
-            if isinstance(mlp, LlamaMLP) and not (plain(mlp, LlamaMLP) and plain(mlp.gate_up_proj, ColumnParallelLinear)
-                                                  and plain(mlp.down_proj, RowParallelLinear)
-                                                  and mlp.gate_up_proj.bias is None):
-                return False
-        return True
+            read += (qkv.weight, o.weight) if qkv.bias is None else (qkv.weight, o.weight, qkv.bias)
+            if isinstance(mlp, LlamaMLP):
+                up, down = mlp.gate_up_proj, mlp.down_proj
+                if not (plain(mlp, LlamaMLP) and plain(up, ColumnParallelLinear) and plain(down, RowParallelLinear)
+                        and up.bias is None):
+                    return False
+                read += (up.weight, down.weight)
+        return ops.rows_weights_ok(read, input_ids)
 
     _unknown: Optional[torch.Tensor] = None
 

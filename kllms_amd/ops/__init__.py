@@ -14,7 +14,7 @@ by numerics tests to produce the oracle on-device).
 from __future__ import annotations
 
 import os
-from typing import Optional, Tuple
+from typing import Optional, Sequence, Tuple
 
 import torch
 
@@ -254,6 +254,11 @@ def linear_rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
             and w.is_contiguous() and w.data_ptr() % 16 == 0
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+
+
+def rows_weights_ok(ws: Sequence[torch.Tensor], like: torch.Tensor) -> bool:
+    """Whether the few-row kernels read all of these: plain bf16 tensors on ``like``'s device, contiguous, on 16 bytes."""
+    return all(type(w) in _PLAIN for w in ws) and _hip_or_raise().rows_weights_ok(ws, like)
 
 
 def linear_part(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

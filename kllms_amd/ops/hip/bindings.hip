@@ -543,6 +543,15 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, torch::Tensor bias, 
   return out;
 }
 
+// What linear_rows and the row-wise steps ask of weights. One call for a model's: from Python a question is 1 us
+bool rows_weights_ok(const std::vector<torch::Tensor>& ws, const torch::Tensor& like) {
+  for (const auto& w : ws)
+    if (w.layout() != at::kStrided || w.device() != like.device() || w.scalar_type() != at::kBFloat16 || !plain_values(w) ||
+        !w.is_contiguous() || reinterpret_cast<uintptr_t>(w.data_ptr()) % 16)
+      return false;
+  return true;
+}
+
 // --- row-wise steps of a decode step (decode_rows.hip) -------------------------
 extern "C" void launch_add_norm_rows(bf16_t* out, bf16_t* residual, const float* part, const int64_t* ids,
                                      const bf16_t* table, const bf16_t* w, int S, int M, int n, int64_t vocab,
@@ -693,6 +702,7 @@ void ipc_allreduce_destroy(int64_t ctx) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("levenshtein_pairs", &levenshtein_pairs);
   m.def("linear_rows", &linear_rows);
+  m.def("rows_weights_ok", &rows_weights_ok);
   m.def("add_norm_rows", &add_norm_rows);
   m.def("embed_norm_rows", &embed_norm_rows);
   m.def("rope_store_rows", &rope_store_rows);

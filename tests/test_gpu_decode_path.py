@@ -548,3 +548,55 @@ def test_logits_of_one_row_repeated(preset, rows):
         out = m.compute_logits(h.expand(rows, -1))
     tol = w.shape[1] * 2 ** -24 * (h.double().abs() @ w.double().abs().t().contiguous())
     assert ((out.double() - h.double() @ w.double().t().contiguous()).abs() <= tol).all()
+
+
+class _Tagged(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("which", ["qkv_proj", "o_proj", "gate_up_proj", "down_proj", "embed_tokens", "bias"])
+@pytest.mark.parametrize("how", ["transposed", "off 16 bytes", "subclass"])
+def test_short_prompts_with_weights_that_lie_otherwise(which, how):
+    """What the few-row products do not read the library does, in whole prompts and in portions of more than 128 rows."""
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+
+    eng = LLMEngine(EngineConfig(model="mid-qwen", max_kv_blocks=64, use_hip_graphs=False, enable_prefix_caching=False, seed=3))
+    ids = torch.randint(0, 2000, (200,), generator=torch.Generator().manual_seed(1))
+
+    def run():
+        out = []
+        for n in (100, 200):
+            if n > 128:
+                s = eng.open_sequence()
+                out.append(eng.step_segments([(s, ids[:n].tolist(), [n - 1])]).double())
+                eng.kv.free_sequence(s)
+            s = eng.kv.alloc_sequence(n)
+            batch = ForwardBatch(mode="prefill", positions=torch.arange(n, device=DEV), kv_caches=eng.kv.layer_caches(),
+                                 slot_mapping=torch.tensor(eng.kv.prefill_slot_mapping(s), device=DEV),
+                                 cu_seqlens=torch.tensor([0, n], dtype=torch.int32, device=DEV))
+            taken = eng.model._takes_short(ids[:n].to(DEV), batch)
+            out.append(eng.model.forward_prefill(ids[:n].to(DEV), batch).double())
+            eng.kv.free_sequence(s)
+        return out, taken
+
+    from kllms_amd.models.llama import ForwardBatch
+    with torch.inference_mode():
+        want, taken = run()
+        assert taken
+        for layer in eng.model.layers:
+            m = {"embed_tokens": eng.model.embed_tokens, "bias": layer.self_attn.qkv_proj}.get(which)
+            m = m if m is not None else getattr(layer.self_attn if which[:2] in ("qk", "o_") else layer.mlp, which)
+            name = "bias" if which == "bias" else "weight"
+            w = getattr(m, name).data
+            if how == "transposed":
+                w = torch.stack((w, w), -1)[..., 0] if w.dim() == 1 else w.t().contiguous().t()
+            elif how == "off 16 bytes":
+                w = w.new_empty(w.numel() + 1)[1:].view_as(w).copy_(w)
+            else:
+                w = w.as_subclass(_Tagged)
+            setattr(m, name, torch.nn.Parameter(w, requires_grad=False))
+        got, taken = run()
+    assert not taken
+    for a, b in zip(got, want):
+        assert (a - b).norm() <= 0.05 * b.norm()      # bf16 through two layers, two sets of kernels
