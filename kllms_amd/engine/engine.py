@@ -15,7 +15,7 @@ from __future__ import annotations
 
 import time
 from dataclasses import dataclass, field
-from typing import Any, List, Optional, Tuple
+from typing import Any, List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -366,10 +366,17 @@ class LLMEngine:
         return logits
 
     # --- main entry -----------------------------------------------------------
+    def check_prompt(self, ids: Sequence[int]) -> None:
+        """Refuses a prompt with an id outside the vocabulary before anything of it is computed or kept."""
+        if len(ids) and not 0 <= min(ids) <= max(ids) < self.arch.vocab_size:
+            raise IndexError(f"a prompt has a token id outside the vocabulary of {self.arch.vocab_size}")
+
     @torch.inference_mode()
     def generate(self, requests: List[GenRequest]) -> List[RequestOutput]:
         if not requests:
             return []
+        for r in requests:
+            self.check_prompt(r.prompt_ids)
         # admission control: bound concurrent decode streams; excess requests
         # are served in sub-batches (same results, sequential batches)
         total_streams = sum(max(1, r.n) for r in requests)

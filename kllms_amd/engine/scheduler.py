@@ -97,6 +97,11 @@ class BatchScheduler:
     # --- public -----------------------------------------------------------
     def submit(self, request: GenRequest) -> Future:
         fut: Future = Future()
+        try:                       # here, not at admission: other requests of the batch are not this one's
+            self.engine.check_prompt(request.prompt_ids)
+        except IndexError as e:
+            fut.set_exception(e)
+            return fut
         self._queue.put(_Ticket(request=request, future=fut))
         self._ensure_thread()
         return fut

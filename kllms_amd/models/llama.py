@@ -328,7 +328,7 @@ class LlamaForCausalLM(nn.Module):
         few-row products read. Other weights are the library's."""
         plain = ops.only_weights
         if not (ops.no_global_hooks() and ops.plain_call(input_ids, batch.positions, batch.slot_mapping)
-                and plain(self.embed_tokens, nn.Embedding)
+                and plain(self.embed_tokens, nn.Embedding)    # its result is written to
                 and not (torch.is_grad_enabled() and any(p.requires_grad for p in self.parameters()))):
             return False
         read = [self.embed_tokens.weight]
@@ -358,20 +358,23 @@ class LlamaForCausalLM(nn.Module):
         return self._unknown
 
     def check_ids(self) -> None:
-        """Raises if a decode step that has run had an id outside the vocabulary (its logits are NaN). It is
+        """Raises if a step on the paged cache that has run had an id outside the vocabulary (its logits are NaN). It is
         known once the step's results have come to the host, and raised before a later step at the latest."""
         if self._unknown is not None and self._unknown.item():
             self._unknown.zero_()
-            raise IndexError(f"a decode step had a token id outside the vocabulary of {self.embed_tokens.num_embeddings}")
+            raise IndexError(f"a step had a token id outside the vocabulary of {self.embed_tokens.num_embeddings}")
 
     def _forward_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
         """A decode step or a short prompt: weights streamed by the few-row kernel, whose split sums go straight into the
         next row-wise kernel: 8 launches a layer, one more where attention splits the contexts and one where gate/up is the
         library's. A prompt's fused projection stays whole: its attention reads the keys and values as rows."""
-        layers = self.layers
-        x, residual = ops.embed_norm_rows(input_ids, self.embed_tokens.weight, layers[0].input_layernorm.weight,
-                                          layers[0].input_layernorm.eps, self._unknown_ids())
-        T = x.shape[0]
+        layers, norm = self.layers, self.layers[0].input_layernorm
+        T = input_ids.shape[0]
+        if batch.mode == "decode":
+            x, residual = ops.embed_norm_rows(input_ids, self.embed_tokens.weight, norm.weight, norm.eps, self._unknown_ids())
+        else:              # a prompt's ids are the caller's: the embedding refuses them in the call
+            residual = self.embed_tokens(input_ids)
+            x = ops.rmsnorm(residual, norm.weight, norm.eps)
         for i, layer in enumerate(layers):
             at, norm = layer.self_attn, layer.post_attention_layernorm
             k_cache, v_cache, k_scale, v_scale = batch.kv_caches[at.layer_idx]

@@ -600,3 +600,44 @@ def test_short_prompts_with_weights_that_lie_otherwise(which, how):
     assert not taken
     for a, b in zip(got, want):
         assert (a - b).norm() <= 0.05 * b.norm()      # bf16 through two layers, two sets of kernels
+
+
+@pytest.mark.parametrize("tokens", [40, 200])
+def test_a_prompt_with_an_id_outside_the_vocabulary_is_refused(tokens):
+    """In the call, each time, and nothing of it is kept for other prompts."""
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import GenRequest, LLMEngine
+    from kllms_amd.engine.sampling import SamplingParams
+
+    eng = LLMEngine(EngineConfig(model="mid-llama", max_kv_blocks=128, use_hip_graphs=False, seed=3, prefix_cache_min_tokens=16))
+    ids = torch.randint(0, 2000, (tokens,), generator=torch.Generator().manual_seed(1)).tolist()
+    good = [GenRequest(prompt_ids=ids, n=1, sampling=SamplingParams(temperature=0.0, max_tokens=4))]
+    bad = [GenRequest(prompt_ids=ids[:5] + [eng.arch.vocab_size] + ids[6:], n=1,
+                      sampling=SamplingParams(temperature=0.0, max_tokens=4))]
+    for _ in range(2):
+        with pytest.raises(IndexError, match="outside the vocabulary"):
+            eng.generate(bad)
+        assert not eng.prefix_cache.match(bad[0].prompt_ids, 16)
+        assert len(eng.generate(good)[0].streams[0].token_ids) == 4
+
+
+@pytest.mark.parametrize("tokens", [1, 100, 300])
+def test_prompts_look_their_ids_up_in_the_embedding(tokens, monkeypatch):
+    """Which refuses an id without a row in the call; steps on the paged cache report it."""
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+    from kllms_amd.models.llama import ForwardBatch
+
+    eng = LLMEngine(EngineConfig(model="mid-llama", max_kv_blocks=128, use_hip_graphs=False, seed=3))
+    seen = []
+    looked_up = torch.nn.functional.embedding
+    monkeypatch.setattr(torch.nn.functional, "embedding", lambda i, *a: (seen.append(i.numel()), looked_up(i, *a))[1])
+    s = eng.kv.alloc_sequence(tokens)
+    batch = ForwardBatch(mode="prefill", positions=torch.arange(tokens, device=DEV), kv_caches=eng.kv.layer_caches(),
+                         slot_mapping=torch.tensor(eng.kv.prefill_slot_mapping(s), device=DEV),
+                         cu_seqlens=torch.tensor([0, tokens], dtype=torch.int32, device=DEV))
+    ids = torch.arange(tokens, device=DEV)
+    with torch.inference_mode():
+        assert eng.model._takes_short(ids, batch)
+        eng.model.forward_prefill(ids, batch)
+        assert seen == [tokens]

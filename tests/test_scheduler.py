@@ -75,6 +75,25 @@ class TestScheduler:
         sched.shutdown()
         assert len(ok.streams) == 1
 
+    @pytest.mark.parametrize("chunk", [None, 16])
+    @pytest.mark.parametrize("bad", [-1, 512, 1 << 40])
+    def test_an_id_outside_the_vocabulary_is_its_own_requests_error(self, bad, chunk):
+        """Also beside other requests of one admission, for whole and chunked prompts, and again for the same prompt."""
+        eng = LLMEngine(EngineConfig(model="tiny-llama", max_kv_blocks=512, use_hip_graphs=False, device="cpu", seed=0,
+                                     prefill_chunk_tokens=chunk))
+        wrong = list(range(2, 42)) + [bad] + [3] * 20
+        sched = BatchScheduler(eng, admit_wait_s=0.05)
+        futs = [sched.submit(greedy_req(p)) for p in ([1, 2, 3], wrong, [4] * 30, wrong)]
+        for f in futs[1::2]:
+            with pytest.raises(IndexError, match="outside the vocabulary"):
+                f.result(timeout=60)
+        assert [len(f.result(timeout=60).streams) for f in futs[::2]] == [1, 1]
+        sched.shutdown()
+        for _ in range(2):
+            with pytest.raises(IndexError, match="outside the vocabulary"):
+                eng.generate([greedy_req([1, 2, 3]), greedy_req(wrong)])
+        assert not eng.prefix_cache.match(wrong, 1)
+
 
 class TestAsyncClientScheduling:
     def test_concurrent_async_calls(self):
