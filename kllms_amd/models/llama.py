@@ -312,7 +312,12 @@ class LlamaForCausalLM(nn.Module):
         the few-row products are the faster ones, and where nothing but the modules' own forwards would run. us of the
         library's product and of linear_part with the reading of its sums, at 160 / 256 / 384 rows:
           4096 x 4096    27 19 / 23 23 / 25 29      4096 x 14336  84 43 / 63 53 / 78 66      6144 x 4096   28 24 / 40 31 / 36 40
-          2048 x 8192    26 17 / 27 22 / 33 26      8192 x 8192   54 43 / 76 58 / 62 73      10240 x 8192  67 71 / 88 94"""
+          2048 x 8192    26 17 / 27 22 / 33 26      8192 x 8192   54 43 / 76 58 / 62 73      10240 x 8192  67 71 / 88 94
+          3072 x 8192    32 26 / 38 29 / 47 35      3584 x 18944  111 54 / 130 63 / 89 72    5120 x 5120   42 29 / 55 39 / 44 42
+        Whole prompts through four layers in the library and so, us at 24 / 160 / 256 / 320 / 384 tokens:
+          1024  228 172 / 275 237 / 290 267 / 314 294 / 323 301      1280  271 210 / 333 311 / 372 363 / 383 385 / 387 394
+          2560  397 335 / 591 533 / 672 597 / 675 619 / 701 654      3072  392 337 / 573 526 / 693 650 / 675 653 / 737 693
+          3584  927 575 / 1095 822 / 1303 1009 / 1174 1074 / 1219 1145      5120  707 621 / 1123 931 / 1470 1148 / 1281 1282 / 1314 1307"""
         rows = input_ids.shape[0]
         if not (batch.mode == "prefill" or rows > ops.LINEAR_ROWS_MAX) or rows > ops.LINEAR_PART_MAX:
             return False
@@ -321,6 +326,8 @@ class LlamaForCausalLM(nn.Module):
         at = self.layers[0].self_attn
         widest = max(at.qkv_proj.weight.shape[0], self.cfg.hidden_size)
         most = ops.LINEAR_PART_MAX if widest <= 6144 else 256 if widest <= 8192 else ops.LINEAR_ROWS_MAX
+        if 1024 < self.cfg.hidden_size < 1536:
+            most = 288
         return rows <= most and self._only_weights(input_ids, batch)
 
     def _only_weights(self, input_ids: torch.Tensor, batch: ForwardBatch) -> bool:

@@ -134,10 +134,18 @@ struct LinearPlan {
 
 // Up to 128 rows one part of x, so that W is read once; above, two or more read it from the L2 where the splits they
 // replace would cost more in sums (4096 x 4096, 384 rows, with the sums' reading: four parts in two splits 25.1 us, one in
-// eight above 30). 64 rows of W to a tile where 128 would leave half of the compute
-// units idle (4096 x 4096, 5 rows: 8.0 us, 8.4; silu 16384 x 2048 13.5, 15.2; but 18432 x 4096, 144 tiles of 128 rows, 35.2,
-// 30.7) or make more workgroups than there are (silu 37888 x 3584, 16 rows: 57, 64); 128 of a long matrix at many rows of x,
-// whose reading by all of them weighs more (4096 x 14336, 128 rows: 40.8 us with the sums' reading, 37.9).
+// eight above 30). Four parts of a small matrix, three of a wider one, two from N 4096 or 2^24 weights on: these leave it fewer
+// splits in any case, and each part reads all of W. us with the sums' reading, in parts of up to 96 rows and so, library last, at
+// 160 / 256 / 320 / 384 rows:
+//   2048 x 2048  15.4 12.3 15 / 16.2 14.3 15 / 17.7 17.4 17 / 19.0 18.7 16    1024 x 4096  16.0 12.4 15 / 21.3 14.6 15 / 17.7 17.5 18 / 19.2 19.1 19
+//   3072 x 3072  18.3 17.0 20 / 20.5 20.5 22 / 24.8 22.9 22 / 25.9 26.1 24    3072 x 8192  26.0 25.7 32 / 31.2 28.7 38 / 40.4 32.8 38 / 42.8 35.2 47
+//   3072 x 12288  37.1 36.7 48 / 45.4 42.6 56 / 67.5 46.8 57 / 71.3 50.0 73   3584 x 18944  54.1 53.6 111 / 63.9 62.7 130 / 83.2 66.7 86 / 88.2 72.3 89
+// 64 rows of W to a tile where 128 would leave half of the compute units idle (4096 x 4096, 5 rows: 8.0 us, 8.4; silu
+// 16384 x 2048 13.5, 15.2; but 18432 x 4096, 144 tiles of 128 rows, 35.2, 30.7) or make more workgroups than there are (silu
+// 37888 x 3584, 16 rows: 57, 64), and of PART up to N 5632, and near 8192 at few rows, where they fill the compute units as well
+// (with 128 rows and with 64: 5120 x 5120 1 row 17.1, 15.4   128 28.5, 26.8; 8192 x 6144 1 row 28.0, 26.8; but 6144 x 6144 128 rows
+// 31.1, 38.7); 128 of a long matrix at many rows of x, whose reading by all of them weighs more (4096 x 14336, 128 rows: 40.8 us
+// with the sums' reading, 37.9; 5120 x 13824, 96 rows 40.3, 38.7).
 static LinearPlan linear_plan(int M, int N, int K, int form) {
   LinearPlan p;
   const bool gated = form == LR_SILU || form == LR_CLAMPED;
@@ -145,14 +153,15 @@ static LinearPlan linear_plan(int M, int N, int K, int form) {
     p.m_tiles = 1;
     p.mj = (M + 31) / 32;
     if (form == LR_PART)
-      p.ni = N >= 5120 || (p.mj == 4 && N >= 4096 && K >= 8192) ? 4 : 2;
+      p.ni = (N <= 5632 && !(p.mj == 4 && N >= 4096 && K >= 8192) && !(N >= 5120 && K > 8192)) ||
+                     (p.mj == 1 && N >= 7680 && N <= 8448) ? 2 : 4;
     else if (gated)
       p.ni = N <= 256 * 64 || (N > 256 * 128 && p.mj == 1) ? 2 : 4;
     else
       p.ni = p.mj > 1 && N >= 192 * 128 ? 4 : 2;
   } else {
     p.ni = 4;
-    p.m_tiles = gated ? (N > 256 * 64 ? 1 : 2) : N >= 4096 ? 2 : (M + 95) / 96;
+    p.m_tiles = gated ? (N > 256 * 64 ? 1 : 2) : N >= 4096 || (int64_t)N * K >= 1 << 24 ? 2 : N >= 3072 ? 3 : 4;
     p.mj = ((M + p.m_tiles - 1) / p.m_tiles + 31) / 32;
   }
   p.kb = p.ni == 2 || p.mj <= 2 ? 80 : 160;

@@ -447,6 +447,18 @@ def test_linear_rows_tiles_and_splits(M, N, K, splits):
                 <= 1.1 * tg * (up.abs() + tu) + tu * gate.abs() + 2 ** -8 * full.abs() + 1e-6).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(m, n, 512) for m in (1, 32, 33, 128) for n in (5104, 5120, 5632, 5648, 7664, 7680, 8448, 8464)]
+                         + [(m, n, k) for m in (129, 130, 193, 289, 384) for n, k in ((3056, 640), (3072, 640), (2048, 8064), (2048, 8192))]
+                         + [(97, 5120, 8192), (97, 5120, 8320), (96, 5120, 8320)])
+def test_linear_rows_at_the_lines_of_their_tiles(M, N, K):
+    """Where the split sums go from tiles of 64 rows of W to 128 and back, and from four parts of x to three and two."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) * 0.05).bfloat16()
+    xd, wt = x.double(), w.double().t().contiguous()
+    assert ((ops.linear_part(x, w).double().sum(0) - xd @ wt).abs() <= K * 2 ** -24 * (xd.abs() @ wt.abs())).all()
+
+
 @pytest.mark.parametrize("N", [128, 192, 16320, 16448, 20544, 32896])
 @pytest.mark.parametrize("M", [5, 40, 128, 129, 256])
 def test_gated_rows_at_the_lines_of_their_tiles(M, N):
