@@ -573,7 +573,7 @@ static inline size_t delta_rows_lds(int rep, int D, int V, int ranks, int HP) {
   return ((size_t)2 * D + rep * (2 * V + D + 1) + V + ranks + 1 + 3 + HP * (DR_BLOCK + 2 * DR_THREADS * 4)) * sizeof(float);
 }
 
-// false, and nothing done, for sizes it is not written for: value sizes and ranks in fours and eights, keys up to 256, what
+// false for sizes it is not written for: value sizes and ranks in fours and eights, keys up to 256, what
 // a workgroup keeps within 64 KB
 extern "C" bool seq_delta_rows_takes(int H, int G, int D, int V, int K, int RA, int RB) {
   const int rep = H / G;

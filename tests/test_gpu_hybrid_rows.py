@@ -142,6 +142,29 @@ def test_delta_sublayer_against_the_general_one(T, H, G, D, V, taps, ranks):
     assert (states[1].conv != states[0].conv).float().mean() <= 0.02
 
 
+@pytest.mark.parametrize("T", [1, 9, 128])
+@pytest.mark.parametrize("H,G,D,V,taps,ranks", [(4, 2, 64, 64, 4, (20, 60)), (64, 32, 32, 130, 4, (16, 16)),
+                                                (8, 1, 256, 512, 4, (64, 72))])
+def test_delta_sublayers_of_other_sizes_stay_native(T, H, G, D, V, taps, ranks):
+    """Ranks not in eights, values not in fours, more than a workgroup keeps: the sublayer's launches one by one."""
+    test_delta_sublayer_against_the_general_one(T, H, G, D, V, taps, ranks)
+
+
+@pytest.mark.parametrize("name", ["a2", "g2"])
+@pytest.mark.parametrize("how", ["transposed", "off 16 bytes"])
+def test_delta_sublayers_with_low_rank_weights_that_lie_otherwise(name, how, monkeypatch):
+    step = ChannelDeltaMixer.rows_step
+
+    def moved(self, *a):
+        w = getattr(self, name).data
+        getattr(self, name).data = (w.t().contiguous().t() if how == "transposed"
+                                    else w.new_empty(w.numel() + 1)[1:].view_as(w).copy_(w))
+        return step(self, *a)
+
+    monkeypatch.setattr(ChannelDeltaMixer, "rows_step", moved)
+    test_delta_sublayer_against_the_general_one(9, 4, 2, 64, 64, 4, (16, 8))
+
+
 @pytest.mark.parametrize("T", [1, 9])
 @pytest.mark.parametrize("G,RH,RD,RV", [(2, 16, 64, 128), (4, 2, 40, 192), (4, 4, 256, 32)])
 def test_parallel_sublayer_against_the_general_one(T, G, RH, RD, RV):
