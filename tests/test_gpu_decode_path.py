@@ -183,8 +183,9 @@ def test_decode_rows_match_general_path(preset, rows):
     ids = torch.randint(0, 2000, (rows,), generator=g).to(DEV)
     with torch.inference_mode():
         assert eng.model._takes_rows(ids, batch) == (rows <= 128)
+        assert eng.model._takes_rows(ids, batch) != eng.model._takes_short(ids, batch)     # the latter: more rows
         got = eng.model.forward_decode(ids, batch)
-        eng.model._takes_rows = lambda *a: False
+        eng.model._takes_rows = eng.model._takes_short = lambda *a: False
         want = eng.model.forward_decode(ids, batch)
     # bf16 activations through two layers; a routed row may change its experts
     off = (got - want).norm(dim=-1) / want.norm(dim=-1)
@@ -476,9 +477,10 @@ def test_gated_rows_at_the_lines_of_their_tiles(M, N):
 
 @pytest.mark.parametrize("preset", ["mid-llama", "mid-qwen", "mid-mixtral"])
 @pytest.mark.parametrize("lens", [[1], [7, 20], [128], [100, 29], [384], [200, 185]])
-def test_short_prompts_match_general_path(preset, lens):
+def test_short_prompts_match_general_path(preset, lens, monkeypatch):
     """A short prompt through the few-row products against the same model's general kernels, which a hook on any of its
-    modules brings back, both within bf16 rounding of each other; the cache rows of the first layer are the same."""
+    modules brings back, both within bf16 rounding of each other at every row (of a mixture: every row whose experts are the
+    same); the cache rows of the first layer are the same."""
     from kllms_amd.engine.config import EngineConfig
     from kllms_amd.engine.engine import LLMEngine
     from kllms_amd.models.llama import ForwardBatch
@@ -491,8 +493,16 @@ def test_short_prompts_match_general_path(preset, lens):
                          slot_mapping=slots.to(DEV), kv_caches=eng.kv.layer_caches(), cu_seqlens=cu.to(DEV))
     ids = torch.randint(0, 2000, (sum(lens),), generator=torch.Generator().manual_seed(sum(lens))).to(DEV)
     m = eng.model
+    route, experts = ops.router_top, []
+    monkeypatch.setattr(ops, "router_top", lambda *a: (lambda r: (experts.append(r[1].sort(-1)[0]), r)[1])(route(*a)))
+
+    def hidden():
+        experts.clear()
+        return m.forward_hidden(ids, batch).float(), list(experts)
+
     with torch.inference_mode():
         assert m._takes_short(ids, batch) == (sum(lens) <= 384)
+        rows, chosen = hidden()
         got, kv = m.forward_prefill(ids, batch), eng.kv.k_all.clone()
         for owner in (m.embed_tokens, m.layers[0], m.layers[0].self_attn, m.layers[0].self_attn.qkv_proj, m.layers[1].self_attn.o_proj):
             seen = []
@@ -502,8 +512,18 @@ def test_short_prompts_match_general_path(preset, lens):
             assert seen
         with torch.autocast("cuda", torch.bfloat16):
             assert not m._takes_short(ids, batch)
+        h = m.embed_tokens.register_forward_hook(lambda *a: None)
+        general, chosen_too = hidden()
+        h.remove()
     off = (got - want).norm(dim=-1) / want.norm(dim=-1)
     assert float(off.max()) < (0.5 if preset == "mid-mixtral" else 0.05)      # a routed row may change its experts
+    same = torch.ones(sum(lens), dtype=torch.bool, device=DEV)
+    assert len(chosen) == len(chosen_too) == (m.cfg.num_layers if preset == "mid-mixtral" else 0)
+    for a, b in zip(chosen, chosen_too):
+        same &= (a == b).all(-1)
+    off = ((rows - general).norm(dim=-1) / general.norm(dim=-1))[same]
+    # two layers, each some six roundings to bf16 (2^-9) apart
+    assert float(same.float().mean()) >= 0.9 and float(off.max()) < 0.02
     assert torch.equal(kv[0], eng.kv.k_all[0])
 
 
