@@ -3,8 +3,9 @@
 // graph) and little else, so each of these kernels does all the work that lies
 // between two products, and takes the previous product's fp32 split sums as they are
 // (linear_rows.hip), which saves the reduction's launch. The sums are rounded to bf16
-// where a whole product's result would be: a step of few rows and one of many then
-// agree to the last bits of their sums.
+// where a whole product's result would be: these products of a step of few rows and of
+// one of many then agree to the last bits of their sums. (Not so gate and up: with the
+// activation in the product they stay in fp32, from the library they come in bf16.)
 //
 // Per layer: residual + norm (twice) and rope + cache store, beside attention and
 // four products: 8 launches (one more where attention splits the contexts, one where

@@ -7,11 +7,11 @@
 //                 top-k find their threshold and draw here
 //
 // Why split: one workgroup per row leaves a 120-row batch on 120 of 256 compute
-// units and a 16-row one on 16, and walks the row three times. The draw, not
-// memory, bounds the split form: per 64 tokens the two 64-bit products of the
-// hash, three transcendentals and the compares take about 230 issue cycles, 22 us
-// for 120 x 128256 tokens on 1024 SIMDs (the logits alone: 61.6 MB, 13 us at the
-// 4.7 TB/s a copy reaches).
+// units and a 16-row one on 16, and walks the row three times. Arithmetic, not
+// memory, bounds the split form: per token the hash in 32-bit products, two
+// logarithms, the exponential of the sum and the compares, 28 us for 120 x 128256
+// tokens where greedy rows take 17 (the logits alone: 61.6 MB, 13 us at the 4.7 TB/s
+// a copy reaches), 35 where all rows are truncated and listed instead of drawn.
 //
 // Rows with top-p / top-k: each slice of a long row lists its highest tokens (slice_list), and sample_final finds the
 // cut in the lists alone where they reach it. It counts their scaled mass and number in 256 bins (per-wave copies: a

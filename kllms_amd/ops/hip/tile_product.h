@@ -328,7 +328,7 @@ __device__ __forceinline__ bf16x4_vec tp_pack(float a, float b, float c, float d
 // stride; rows and columns of it exist, columns and stride are multiples of 8.
 template <int NI, int MJ, class V>
 __device__ __forceinline__ void tile_store(bf16_t* out, int64_t stride, int rows, int columns, char* smem, V value) {
-  constexpr int UNITS = NI * 2;          // 16-byte units of a row: 8 or 16
+  constexpr int UNITS = NI * 2;          // 16-byte units of a row: 4, 8 or 16
   const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
   char* mine = smem + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * (MJ * 16 * UNITS * 16);
 #pragma unroll
