@@ -5,10 +5,10 @@ top-k-routed mixture of experts. Experts are TP-SHARDED, not
 expert-parallel — every rank holds a 1/tp slice of every expert, so routing
 needs no all-to-all and the layer keeps the dense model's two all-reduces.
 
-Expert compute has two regimes: decode shapes run a DENSE batched GEMM over
-all experts (same HBM traffic as routed compute when nearly every expert is
-touched; hipGraph-friendly because shapes are data-independent), prefill
-shapes bucket tokens per expert and run grouped GEMMs.
+On the GPU the experts run as grouped products over tokens bucketed by expert
+(ops/hip/moe.hip), at every row count and without a host round trip, so that a
+hipGraph replays them. Few rows that those kernels do not take (other types or
+sizes, a gradient) run a DENSE batched GEMM over all experts.
 
 Router semantics match Mixtral: softmax over ALL expert logits (fp32), top-k
 (default 2), renormalize the selected weights.
@@ -54,9 +54,10 @@ class MixtralMoE(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         T, H = x.shape
+        grouped = x.is_cuda and (T > 8 * self.E or self._takes_grouped(x))
         routed = None
         if self.gate.bias is None and ops.only_weights(self.gate, nn.Linear) and ops.no_global_hooks():
-            routed = ops.router_top(x, self.gate.weight, self.k, T > 8 * self.E)
+            routed = ops.router_top(x, self.gate.weight, self.k, grouped)
         if routed is not None:
             topw, topi = routed[:2]                                # [T, k]
         else:
@@ -65,25 +66,41 @@ class MixtralMoE(nn.Module):
             topw, topi = torch.topk(probs, self.k, dim=-1)
             topw = topw / topw.sum(dim=-1, keepdim=True)
 
-        if T <= 8 * self.E:
-            out = self._forward_dense(x, topw, topi)
-        elif x.is_cuda:
+        if grouped:
             out = self._forward_grouped_hip(x, topw, topi, *(routed[2:] if routed else ()))
+        elif T <= 8 * self.E:
+            out = self._forward_dense(x, topw, topi)
         else:
             out = self._forward_grouped(x, topw, topi)
         return self.ctx.all_reduce(out)
 
+    def _takes_grouped(self, x: torch.Tensor) -> bool:
+        """Whether few rows run as the grouped products. They read the chosen experts alone, where a batched product reads all:
+        us of the layer, 8 experts, top 2, and batched, at 1 / 5 / 16 / 64 rows: width 512, experts of 1024 41 124 / 42 141 /
+        44 141 / 41 132; 2048, 8192 76 195 / 159 304 / 186 245 / 188 298; 4096, 14336 172 543 / 396 674 / 520 622 / 526 695"""
+        gu, down = self.w_gate_up, self.w_down
+        return (x.shape[0] >= 1 and self.E <= 4096 and x.dtype == gu.dtype == down.dtype == torch.bfloat16 and not ops._force_torch()
+                and x.shape[1] % 64 == 0 and self.I % 64 == 0 and x.shape[1] < 1 << 24 and self.I < 1 << 24
+                and x.is_contiguous() and gu.is_contiguous() and down.is_contiguous() and ops.plain_call(x, gu, down)
+                and not (torch.is_grad_enabled() and (x.requires_grad or gu.requires_grad or down.requires_grad)))
+
     def _forward_dense(self, x: torch.Tensor, topw: torch.Tensor, topi: torch.Tensor) -> torch.Tensor:
-        """Decode-shape path: with few tokens and top-k routing, (nearly)
-        every expert's weights stream from HBM anyway, so computing ALL
-        experts with batched GEMMs costs the same memory traffic as exact
-        routing, needs no token bucketing, and replays cleanly in a hipGraph
-        (no data-dependent shapes)."""
+        """Few tokens in batched GEMMs over all experts: no token bucketing, no
+        data-dependent shapes. On the GPU the weights are the left operands: a
+        batched bf16 product whose right operand is a transposed view has
+        faulted there."""
         T = x.shape[0]
-        xb = x.unsqueeze(0).expand(self.E, T, -1)                     # [E, T, H]
-        gu2 = torch.bmm(xb, self.w_gate_up.transpose(1, 2)).view(self.E * T, 2 * self.I)
-        act = ops.silu_mul(gu2[:, : self.I], gu2[:, self.I:]).view(self.E, T, self.I)
-        ye = torch.bmm(act, self.w_down.transpose(1, 2))              # [E, T, H]
+        if x.is_cuda:
+            n = max(T, 2)                                       # a single column takes three times two's time
+            xt = x.t().unsqueeze(0).expand(self.E, -1, n).contiguous()            # [E, H, n]
+            gu2 = torch.bmm(self.w_gate_up, xt).transpose(1, 2).reshape(self.E * n, 2 * self.I)
+            act = ops.silu_mul(gu2[:, : self.I], gu2[:, self.I:]).view(self.E, n, self.I)
+            ye = torch.bmm(self.w_down, act.transpose(1, 2).contiguous())[:, :, :T].transpose(1, 2)      # [E, T, H]
+        else:
+            xb = x.unsqueeze(0).expand(self.E, T, -1)                             # [E, T, H]
+            gu2 = torch.bmm(xb, self.w_gate_up.transpose(1, 2)).view(self.E * T, 2 * self.I)
+            act = ops.silu_mul(gu2[:, : self.I], gu2[:, self.I:]).view(self.E, T, self.I)
+            ye = torch.bmm(act, self.w_down.transpose(1, 2))                      # [E, T, H]
         # combine: weight[e, t] = topw where topi == e else 0
         w = torch.zeros(self.E, T, device=x.device, dtype=torch.float32)
         w.scatter_(0, topi.t().long(), topw.t().float())
@@ -91,10 +108,10 @@ class MixtralMoE(nn.Module):
 
     def _forward_grouped_hip(self, x: torch.Tensor, topw: torch.Tensor, topi: torch.Tensor, ids=None, pos=None,
                              offsets=None, cleared=None) -> torch.Tensor:
-        """Prefill-shape path on GPU, three launches (ops/hip/moe.hip) behind the
-        router's two, without a host round trip: gate/up GEMM with fused silu*mul,
-        down GEMM, and the weighted sum of each token's rows. The pairs are sorted
-        here where the router's kernel did not take the call."""
+        """The path on the GPU, three launches (ops/hip/moe.hip) behind the router's
+        two, without a host round trip: gate/up GEMM with fused silu*mul, down GEMM,
+        and the weighted sum of each token's rows. The pairs are sorted here where
+        the router's kernel did not take the call."""
         T, H = x.shape
         if ids is None:
             ids, pos, offsets = ops.moe_sort(topi, self.E)

@@ -449,3 +449,49 @@ def test_mixture_layer_with_a_hooked_router():
         assert seen == [(T, 8)]
         # weights apart by fp32 rounding, the result rounded to bf16 once (2^-9)
         assert torch.allclose(got.float(), want.float(), rtol=2 ** -7, atol=1e-4 * float(want.float().abs().max()))
+
+
+@pytest.mark.parametrize("T", [1, 2, 16, 32])
+@pytest.mark.parametrize("H,I,E,k,how", [(512, 1024, 8, 2, ""), (64, 64, 4, 1, ""), (256, 192, 32, 8, ""), (512, 2624, 8, 2, ""),
+                                         (128, 64, 40, 2, ""), (128, 96, 4, 2, "size"), (256, 128, 8, 2, "rows"),
+                                         (256, 128, 8, 2, "transposed"), (256, 128, 8, 2, "gradient")])
+def test_mixture_layer_of_few_rows(T, H, I, E, k, how):
+    """As grouped products, and as batched ones where those do not take the call, against float64 on the layer's routing."""
+    from kllms_amd.engine.config import ModelArchConfig
+    from kllms_amd.models.mixtral import MixtralMoE
+    from kllms_amd.parallel.tp import ParallelContext
+    cfg = ModelArchConfig(arch="mixtral", vocab_size=64, hidden_size=H, intermediate_size=I, num_layers=1, num_heads=2,
+                          num_kv_heads=1, num_experts=E, num_experts_per_tok=k)
+    g = torch.Generator(device=DEV).manual_seed(T + H + I)
+    with torch.device(DEV):
+        moe = MixtralMoE(cfg, ParallelContext(), torch.bfloat16)
+    with torch.no_grad():
+        for p in moe.parameters():
+            p.copy_(torch.randn(p.shape, generator=g, device=DEV) * p.shape[-1] ** -0.5)
+    x = torch.randn(T, H, generator=g, device=DEV).bfloat16()
+    if how == "rows":
+        x = torch.cat((x, x), 1)[:, :H] if T > 1 else torch.stack((x, x), -1)[..., 0]
+    elif how == "transposed":
+        moe.w_down.data = moe.w_down.data.transpose(1, 2).contiguous().transpose(1, 2)
+    elif how == "gradient":
+        x.requires_grad_()
+    assert moe._takes_grouped(x) == (how == "")
+    got = moe(x)
+    if how == "gradient":
+        got.float().sum().backward()
+        assert x.grad.isfinite().all() and x.grad.norm() > 0
+        x = x.detach()
+    p = torch.softmax((x.double() @ moe.gate.weight.double().t().contiguous()).bfloat16().float(), -1)
+    topw, topi = torch.topk(p, k, -1)
+    sure = torch.topk(p, min(k + 1, E), -1)[0]
+    sure = (sure[:, k - 1] > 1.02 * sure[:, k]) if E > k else torch.ones(T, dtype=torch.bool, device=DEV)
+    topw = (topw / topw.sum(-1, keepdim=True)).double()
+    want = torch.zeros(T, H, dtype=torch.float64, device=DEV)
+    for t in range(T):
+        for w, e in zip(topw[t], topi[t].tolist()):
+            gate, up = (moe.w_gate_up[e].double() @ x[t].double()).chunk(2)
+            want[t] += w * (moe.w_down[e].double() @ (torch.nn.functional.silu(gate) * up))
+    # gate, up, act, each expert's row and the sum are rounded to bf16 (2^-9 each); rows whose choice is not a close one
+    off = (got.double() - want).norm(dim=-1) / want.norm(dim=-1)
+    assert sure.float().mean() >= 0.5 or T < 8
+    assert (off[sure] <= 0.015).all()
