@@ -101,8 +101,8 @@ class LlamaAttention(nn.Module):
             return ops.attn_prefill_varlen(q, k, v, batch.cu_seqlens, self.scale, (batch.plans or {}).get("prefill"))
         return self.attend_cache(q, batch)
 
-    def attend_cache(self, q: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
-        """Attention of decode-mode rows q [T, H, D] against the paged cache."""
+    def attend_cache(self, q: torch.Tensor, batch: ForwardBatch, arrived: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """Attention of decode-mode rows q [T, H, D] against the paged cache; ``arrived``: zeros of ops.attn_decode_paged."""
         k_cache, v_cache, k_scale, v_scale = batch.kv_caches[self.layer_idx]
         paged = (batch.plans or {}).get("paged")
         if paged is not None and k_scale is None:
@@ -111,7 +111,7 @@ class LlamaAttention(nn.Module):
                                            plan, short, batch.seg_tables, batch.seg_start)
         return ops.attn_decode_paged(
             q, k_cache, v_cache, batch.block_tables, batch.context_lens, self.scale,
-            k_scale, v_scale,
+            k_scale, v_scale, arrived,
         )
 
 
@@ -378,7 +378,10 @@ class LlamaForCausalLM(nn.Module):
         layers, norm = self.layers, self.layers[0].input_layernorm
         T = input_ids.shape[0]
         if batch.mode == "decode":
-            x, residual = ops.embed_norm_rows(input_ids, self.embed_tokens.weight, norm.weight, norm.eps, self._unknown_ids())
+            # zeroed by the first launch, and zero again after each layer's attention
+            arrived = torch.empty(T * layers[0].self_attn.num_kv_heads, dtype=torch.int32, device=input_ids.device)
+            x, residual = ops.embed_norm_rows(input_ids, self.embed_tokens.weight, norm.weight, norm.eps, self._unknown_ids(),
+                                              arrived)
         else:              # a prompt's ids are the caller's: the embedding refuses them in the call
             residual = self.embed_tokens(input_ids)
             x = ops.rmsnorm(residual, norm.weight, norm.eps)
@@ -390,7 +393,7 @@ class LlamaForCausalLM(nn.Module):
             else:
                 q = ops.rope_store_rows(ops.linear_part(x, at.qkv_proj.weight), at.qkv_proj.bias, at.num_heads,
                                         batch.positions, self.cos_sin, k_cache, v_cache, batch.slot_mapping, k_scale, v_scale)
-                att = at.attend_cache(q, batch)
+                att = at.attend_cache(q, batch, arrived)
             x = ops.add_norm_rows(ops.linear_part(att.view(T, -1), at.o_proj.weight), residual, norm.weight, norm.eps)
             norm = layers[i + 1].input_layernorm if i + 1 < len(layers) else self.norm
             mlp = layer.mlp

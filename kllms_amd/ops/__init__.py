@@ -225,14 +225,17 @@ def attn_decode_paged(
     scale: float,
     k_scale: Optional[torch.Tensor] = None,
     v_scale: Optional[torch.Tensor] = None,
+    arrived: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
+    """``arrived``: an int32 zero for each row and kv head, zero again afterwards; with it, contexts that several workgroups
+    share are merged in the same launch."""
     if q.is_cuda and not _force_torch():
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         none = _none(q, torch.float32)
         _hip_or_raise().attn_decode_paged(
             out, q, k_cache, v_cache, block_tables, context_lens, scale,
             k_scale if k_scale is not None else none,
-            v_scale if v_scale is not None else none, none)
+            v_scale if v_scale is not None else none, none, -1, arrived)
         return out
     return torch_ref.attn_decode_paged(q, k_cache, v_cache, block_tables, context_lens, scale,
                                        k_scale, v_scale)
@@ -352,11 +355,11 @@ def linear_clamped_glu(x: torch.Tensor, w: torch.Tensor, limit: float, alpha: fl
     return _try_tiles(x, w, None, 2, limit, alpha)
 
 
-def embed_norm_rows(ids, table, weight, eps, unknown=None):
+def embed_norm_rows(ids, table, weight, eps, unknown=None, clear=None):
     """(rms(table[ids]) * weight, table[ids]). An id outside the table gives a row of NaN and sets ``unknown``, one int32
-    of pinned host memory, to 1."""
+    of pinned host memory, to 1. ``clear``: int32 values on the GPU that the launch zeroes."""
     return _hip_or_raise().embed_norm_rows(ids, table, weight, eps,
-                                           unknown if unknown is not None else torch.empty(0, dtype=torch.int32))
+                                           unknown if unknown is not None else torch.empty(0, dtype=torch.int32), clear)
 
 
 def add_norm_rows(part, residual, weight, eps):

@@ -3,21 +3,22 @@
 // Flash decoding over 32-key tiles, one tile per WAVE: a wave takes every
 // (Z*4)-th tile of its (stream, kv head), keeps its own running max and sum, and
 // the four waves of a workgroup fold once at the end. Z workgroups share a
-// context; their partials are merged by a second launch (none with Z = 1).
+// context; their partials are merged by the last of them to arrive, or by a second
+// launch where the caller has no counters for that.
 //
-// What bounds it is bytes in flight: a wave issues the K and V loads of a whole
-// tile (16 KB in bf16, 64 registers a lane) before it uses any, so twelve waves
-// keep 192 KB in flight per compute unit, and no barrier stands between a wave's
-// scores, softmax and weighted sum. (64-key tiles leave two waves per SIMD, and
-// loading the next tile ahead spills: 43 and 126 us where this takes 36.)
+// What bounds it is bytes in flight, and for contexts that lie in the L2 the address
+// units. A wave has the K and V rows of its next tile (16 KB in bf16, 64 registers a
+// lane) on their way while it works on one, twelve waves a compute unit. Rows are read
+// whole, 16 neighbouring lanes each (with the fragments' own pattern, four lanes in
+// four rows, an instruction occupies the address unit for 64 cycles and not 16), and
+// turned by way of a strip of LDS that is the wave's own: no barriers.
 //
-//   scores   S[key][head] on the matrix cores (16x16x32): K rows go from memory to
-//            fragments as they lie - lane group g takes dims 32g..32g+31 of its
-//            row, 64 contiguous bytes in four loads, and Q is read in the same
-//            order (a dot product does not care which order its terms have)
+//   scores   S[key][column] on the matrix cores (16x16x32); column n is head n % GQA
 //   softmax  fp32, head per lane column, exchanges over the four lane groups only
-//   P V      fp32 on the vector unit: 16 lanes x 8 dims span a V row, four keys at
-//            a time; P crosses lanes through a wave-private LDS strip
+//   P V      on the matrix cores: P in three bf16 parts, which are its 32 bits, in
+//            columns of their own: n / GQA is the part. The scores' lanes hold P as
+//            the product reads it; V comes turned from the strip (ds_read_b64_tr_b16).
+//            On the vector unit P V was 360 of a tile's 550 instructions
 //
 // Workgroups are laid out kv head fastest: with 8 kv heads each XCD serves one of
 // them, and the streams of a request, neighbours in the batch, find their shared
@@ -28,11 +29,13 @@
 // only its last token's aligned block of mask_size positions, and each head's result
 // passes a sigmoid gate (the block-local layers of the hybrid family).
 //
-// Measured with the merge, 32 heads / 8 kv heads, beside 256-key workgroups with
-// block-wide passes: 120 streams of 560 keys 36.5 us (68), 5 streams 8.5 us (23), 16
-// fp8 streams of 5850 keys 49 us (109, 198 MB: 4 TB/s); 16 / 4 heads, one stream of
-// 170 keys 7.8 us (21); block-local, 40 rows of 600 keys, 16 / 4 heads,
-// 20.5 us (81 with a workgroup per row and q-head).
+// Measured in graphs, 32 heads / 8 kv heads, against rows read as fragments, P V on the vector unit and merges in a launch of
+// their own, us: 120 streams, five to a prompt, of 560 keys 33.5, 25.1; 40, eight to a prompt, of 2000 41, 28; prompts of their
+// own: 128 streams of 700 77, 71 (5.5 TB/s), 24 of 2500 48.6, 42.4; 16 fp8 streams of 6000 45.5, 40; 5 streams of 560 8.4, 7.4;
+// 16 / 4 heads, one of 150 7.5, 5.6; block-local, 100 rows of 600, 16 / 4 heads 15.5, 11.5. Without groups of heads, 8 / 8, 40
+// streams of 600: 22.4, 23.2; fp8 15.9, 17.2: there P V is a quarter of the vector work, and fewer registers let one wave more in.
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -40,6 +43,8 @@ typedef __bf16 bf16x8_mfma __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4_cvt __attribute__((ext_vector_type(4)));
 
 #define NTHREADS 256
 #define TKEYS 32           // keys of a wave's tile
@@ -56,10 +61,8 @@ __device__ __forceinline__ Frag fp8x8_to_bf16(u32x2 v) {
   Frag f;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i], false);
-    const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i], true);
-    f.u[2 * i] = __builtin_amdgcn_perm(__float_as_uint(lo[1]), __float_as_uint(lo[0]), 0x07060302u);
-    f.u[2 * i + 1] = __builtin_amdgcn_perm(__float_as_uint(hi[1]), __float_as_uint(hi[0]), 0x07060302u);
+    f.u[2 * i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)v[i], 1.0f, false));
+    f.u[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)v[i], 1.0f, true));
   }
   return f;
 }
@@ -70,6 +73,21 @@ __device__ __forceinline__ int first_key(int L, int mask_size) {
   return mask_size > 0 ? max(L - 1, 0) / mask_size * mask_size : 0;
 }
 
+// Workgroups that share a context of so many tiles (attn_decode_shares): one up to ``few`` tiles a wave, then ``mid`` or as many
+// as leave a wave eight, ``most`` at most; no more than its rounds of tiles take.
+struct DecodeShares {
+  int few, mid, most, grid;
+};
+__host__ __device__ __forceinline__ int shares_of(int tiles, const DecodeShares& s) {
+  const int rounds = (tiles + 3) / 4;
+  if (rounds <= s.few) return 1;
+  int z = (rounds + 7) / 8;
+  z = z < s.mid ? s.mid : z;
+  z = z > s.most ? s.most : z;
+  const int each = (rounds + z - 1) / z;
+  return (rounds + each - 1) / each;
+}
+
 // LOCAL (block-local layers): exponentials to the last place, as those layers' other kernels
 // have them; __expf of an argument of -70 is off by 3e-6. 40 rows of 600 keys, 16 / 4 heads,
 // in a graph: 17.0 us, 15.9 with __expf
@@ -78,15 +96,34 @@ __device__ __forceinline__ float exp_of(float x) {
   return LOCAL ? expf(x) : __expf(x);
 }
 
+// v of lane from + more
+__device__ __forceinline__ int lane_value(int v, int from, int more) { return __builtin_amdgcn_ds_bpermute(from * 4 + more * 4, v); }
+
 template <bool LOCAL>
 __device__ __forceinline__ float head_gate(const bf16_t* __restrict__ gate, int stride, int b, int h) {
   if (!gate) return 1.0f;
   return 1.0f / (1.0f + exp_of<LOCAL>(-bf16_to_f32(((const short*)gate)[(int64_t)b * stride + h])));
 }
 
-template <int GQA, bool FP8, bool LOCAL>
+#define DECODE_SHARES 16   // of a context at most that are merged in the same launch
+#define FAR 16             // loads and stores past the L2, from and to other XCDs' workgroups
+
+// A wave's strip of LDS: K of its tile, then V, 32 rows of 128 bf16; after the last one its sums, rows of SUM_PITCH floats
+#define SUM_PITCH 132
+template <int GQA>
+struct Strip {
+  static constexpr int SETS = GQA == 8 ? 2 : 1;               // sets of 16 columns
+  static constexpr int SUMS = 3 * GQA * SUM_PITCH * 4;
+  static constexpr int BYTES = ((SUMS > TKEYS * 256 ? SUMS : TKEYS * 256) + 255) / 256 * 256;
+};
+
+// KV: what the cache holds
+enum { KV_BF16 = 0, KV_FP8 = 1, KV_FP8_ANY = 2 };   // fp8 in blocks of a multiple of four keys, and in others
+
+template <int GQA, int KV, bool LOCAL>
 __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
-    float* __restrict__ partials, bf16_t* __restrict__ out,  // out: written when gridDim.z == 1
+    float* __restrict__ partials,
+    bf16_t* __restrict__ out,            // written where one workgroup has the context, or by the last one with ``arrived``
     const bf16_t* __restrict__ q,        // [B, H, 128], row stride q_tstride
     const char* __restrict__ k_cache,    // [NB, KVH, BS, 128], bf16 or fp8
     const char* __restrict__ v_cache,
@@ -95,75 +132,126 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
     const int* __restrict__ block_tables,  // [B, max_blocks]
     const int* __restrict__ context_lens,  // [B]
     const bf16_t* __restrict__ gate, int gate_stride,  // [B, H] logits of the heads' sigmoid gates, or nullptr
-    float scale, int block_size, int max_blocks, int q_tstride, int mask_size) {
+    int* __restrict__ arrived,           // [B, KVH] zeros, zeros again afterwards, or nullptr: a second launch merges
+    float scale, int block_size, uint32_t block_inverse, int max_blocks, int q_tstride, int mask_size, DecodeShares shares) {
+  constexpr int SETS = Strip<GQA>::SETS;
+  constexpr bool FP8 = KV != KV_BF16;
   const int g_kv = blockIdx.x, num_kv_heads = gridDim.x;
   const int b = blockIdx.y;
-  const int z = blockIdx.z, Z = gridDim.z;
+  const int z = blockIdx.z;
   const int L = context_lens[b];
   const int first = first_key(L, mask_size);
   const int tiles = (L - first + TKEYS - 1) / TKEYS;
-  if (z * 4 >= tiles && Z > 1) return;   // no keys here: the merge skips this partial
+  const int Z = shares_of(tiles, shares);
+  if (z >= Z) return;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 15, grp = lane >> 4;
 
-  __shared__ __attribute__((aligned(16))) float p_lds[4][TKEYS * GQA];
-  __shared__ float o_lds[4][GQA * 128];
+  __shared__ __attribute__((aligned(16))) char strips[4][Strip<GQA>::BYTES];
   __shared__ float m_lds[4][GQA], l_lds[4][GQA];
-  float* p_me = p_lds[wave];
+  char* const strip = strips[wave];
 
+  // column n of the products is head n % GQA
   Frag qf[4];
   {
-    const short* qp = (const short*)q + (int64_t)b * q_tstride + (g_kv * GQA + min(col, GQA - 1)) * 128 + grp * 32;
+    const short* qp = (const short*)q + (int64_t)b * q_tstride + (g_kv * GQA + col % GQA) * 128 + grp * 8;
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-      qf[s].u = col < GQA ? *reinterpret_cast<const u32x4*>(qp + s * 8) : u32x4{0, 0, 0, 0};
+    for (int s = 0; s < 4; ++s) qf[s].u = *reinterpret_cast<const u32x4*>(qp + s * 32);
   }
   const int* bt = block_tables + (int64_t)b * max_blocks;
 
-  float m_run = -INFINITY, l_run = 0.0f;   // of head ``col``; l_run: this lane's keys only
-  float o[GQA][8];
+  float m_run = -INFINITY, l_run = 0.0f;   // of head col % GQA; l_run: this lane's keys only
+  f32x4 o[SETS][8];
 #pragma unroll
-  for (int h = 0; h < GQA; ++h)
+  for (int e = 0; e < SETS; ++e)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[h][j] = 0.0f;
+    for (int i = 0; i < 8; ++i) o[e][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // cache row of key first + tile * 32 + (lane & 31); keys behind the context repeat its
-  // last row
-  auto row_of = [&](int tile) {
-    const int kc = min(first + tile * TKEYS + (lane & (TKEYS - 1)), L - 1);
-    return (bt[kc / block_size] * num_kv_heads + g_kv) * block_size + kc % block_size;
+  // key first + tile * 32 + (lane & 31); those behind the context repeat its last one
+  auto key_of = [&](int tile) { return min(first + tile * TKEYS + (lane & (TKEYS - 1)), L - 1); };
+  // key / block_size by its reciprocal, which is off by one at most
+  auto block_of = [&](int key) {
+    const int n = (int)__umulhi((uint32_t)key, block_inverse), rest = key - n * block_size;
+    return n - (rest < 0) + (rest >= block_size);
   };
-  const int t0 = z * 4 + wave;
-  int row_next = t0 < tiles ? row_of(t0) : 0;
-#pragma unroll 1
-  for (int t = t0; t < tiles; t += Z * 4) {
-    const int base = first + t * TKEYS;
-    const int rowi = row_next;
-    float ks = 1.0f, vs = 1.0f;
-    if constexpr (FP8) { ks = k_scale[rowi]; vs = v_scale[rowi]; }
-    u32x4 kraw[TKEYS / 16][FP8 ? 2 : 4];
+  auto row_of = [&](int tile, int block) {
+    const int key = key_of(tile);
+    return (block * num_kv_heads + g_kv) * block_size + (key - block_of(key) * block_size);
+  };
+  typedef __attribute__((address_space(3))) char* lds_t;
+  typedef __attribute__((address_space(3))) u32x4* lds_vec;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_t)strip;
+  const int row8 = FP8 ? lane >> 3 : grp, turn_row = grp * 4 + (col >> 2);
+  // where this lane's 16 bytes of the strip lie: stored, read as K (row col), read turned as V. The rest is an XOR
+  uint32_t put_at = lds0 + row8 * 256 + (((FP8 ? (lane & 7) * 2 : col) ^ row8) << 4);
+  uint32_t key_at = lds0 + col * 256 + ((grp ^ col) << 4);
+  uint32_t turn_at = lds0 + turn_row * 256 + ((((col & 3) >> 1) ^ turn_row) << 4) + (col & 1) * 8;
+  // Whole rows go to registers, 16 lanes each (8 in fp8), and from there to the strip, their 16-byte units XORed with the row
+  constexpr int LOADS = FP8 ? TKEYS / 8 : TKEYS / 4;
+  u32x4 kraw[LOADS], vraw[LOADS];
+  f32x4 ks[2], vs[2];                    // scales of this lane's keys tt*16 + grp*4 + r
+  auto load = [&](u32x4 (&to)[LOADS], const char* cache, int row) {
 #pragma unroll
-    for (int tt = 0; tt < TKEYS / 16; ++tt) {
-      const int64_t r = __shfl(rowi, tt * 16 + col);
-      const u32x4* kp = reinterpret_cast<const u32x4*>(k_cache + r * (FP8 ? 128 : 256) + grp * (FP8 ? 32 : 64));
-#pragma unroll
-      for (int s = 0; s < (FP8 ? 2 : 4); ++s) kraw[tt][s] = kp[s];
+    for (int i = 0; i < LOADS; ++i) {
+      const int64_t r = lane_value(row, FP8 ? lane >> 3 : grp, i * (FP8 ? 8 : 4));
+      to[i] = *reinterpret_cast<const u32x4*>(cache + (FP8 ? r * 128 + (lane & 7) * 16 : r * 256 + col * 16));
     }
-    u32x4 vraw[TKEYS / 4];
+  };
+  auto load_scales = [&](f32x4 (&to)[2], const float* scales, int row) {
 #pragma unroll
-    for (int i = 0; i < TKEYS / 4; ++i) {
-      const int64_t r = __shfl(rowi, i * 4 + grp);
-      if constexpr (FP8) {
-        const u32x2 v = *reinterpret_cast<const u32x2*>(v_cache + r * 128 + col * 8);
-        vraw[i][0] = v[0];
-        vraw[i][1] = v[1];
+    for (int tt = 0; tt < 2; ++tt) {
+      if constexpr (KV == KV_FP8) {        // behind the context the last row's four
+        to[tt] = *reinterpret_cast<const f32x4*>(scales + (lane_value(row, grp * 4, tt * 16) & ~3));
       } else {
-        vraw[i] = *reinterpret_cast<const u32x4*>(v_cache + r * 256 + col * 16);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) to[tt][r] = scales[lane_value(row, grp * 4, tt * 16 + r)];
       }
     }
-    row_next = row_of(min(t + Z * 4, tiles - 1));
-
-    // ---- scores: lane (col, grp) holds keys tt*16 + grp*4 + r of head col ----
+  };
+  auto load_k = [&](int row) {
+    if constexpr (FP8) load_scales(ks, k_scale, row);
+    load(kraw, k_cache, row);
+  };
+  auto load_v = [&](int row) {
+    if constexpr (FP8) load_scales(vs, v_scale, row);
+    load(vraw, v_cache, row);
+  };
+  auto store = [&](const u32x4 (&from)[LOADS]) {
+    const uint32_t put = put_at;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      if constexpr (FP8) {
+        const uint32_t at = put ^ ((i & 1) << 7);
+        *(lds_vec)(uintptr_t)(at + i * 2048) = fp8x8_to_bf16(u32x2{from[i][0], from[i][1]}).u;
+        *(lds_vec)(uintptr_t)((at ^ 16) + i * 2048) = fp8x8_to_bf16(u32x2{from[i][2], from[i][3]}).u;
+      } else {
+        *(lds_vec)(uintptr_t)((put ^ ((i & 3) << 6)) + i * 1024) = from[i];
+      }
+    }
+  };
+  // the strip is this wave's own: in-order LDS, only the compiler is held
+  auto hold = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  const int step = Z * 4;
+  int t = z * 4 + wave, row = 0, block = 0;  // row of this lane's key in the next tile; the block of the one behind it
+  auto tile = [&](auto more) {
+    const int base = first + t * TKEYS;
+    // not eighteen addresses for the whole loop
+    asm volatile("" : "+v"(put_at), "+v"(key_at), "+v"(turn_at));
+    // ---- scores: lane (col, grp) holds keys tt*16 + grp*4 + r of head col % GQA ----
+    store(kraw);
+    const f32x4 ks_now[2] = {ks[0], ks[1]}, vs_now[2] = {vs[0], vs[1]};
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (more) {
+      row = row_of(t + step, block);
+      block = bt[block_of(key_of(min(t + 2 * step, tiles - 1)))];
+      load_k(row);
+    }
+    hold();
+    __builtin_amdgcn_sched_barrier(0);
     float sc[TKEYS / 16][4];
     float tmax = -INFINITY;
 #pragma unroll
@@ -172,101 +260,110 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         Frag kf;
-        if constexpr (FP8)
-          kf = fp8x8_to_bf16(u32x2{kraw[tt][s >> 1][(s & 1) * 2], kraw[tt][s >> 1][(s & 1) * 2 + 1]});
-        else
-          kf.u = kraw[tt][s];
+        kf.u = *(lds_vec)(uintptr_t)((key_at ^ (s << 6)) + tt * 4096);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.m, qf[s].m, acc, 0, 0, 0);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int key = tt * 16 + grp * 4 + r;
         float x = acc[r] * scale;
-        if constexpr (FP8) x *= __shfl(ks, key);
-        sc[tt][r] = base + key < L ? x : -INFINITY;
+        if constexpr (FP8) x *= ks_now[tt][r];
+        sc[tt][r] = base + tt * 16 + grp * 4 + r < L ? x : -INFINITY;
         tmax = fmaxf(tmax, sc[tt][r]);
       }
     }
+    hold();
+    __builtin_amdgcn_sched_barrier(0);
+    store(vraw);
+    if constexpr (more) load_v(row);
+    __builtin_amdgcn_sched_barrier(0);
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
     const float m_new = fmaxf(m_run, tmax);
-    const float alpha = (m_run == -INFINITY) ? 0.0f : exp_of<LOCAL>(m_run - m_new);
-    m_run = m_new;
-    l_run *= alpha;
+    if (__any(m_new > m_run)) {
+      const float alpha = (m_run == -INFINITY) ? 0.0f : exp_of<LOCAL>(m_run - m_new);
+      l_run *= alpha;
 #pragma unroll
-    for (int tt = 0; tt < TKEYS / 16; ++tt)
+      for (int e = 0; e < SETS; ++e)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[e][i] *= alpha;
+    }
+    m_run = m_new;
+    // P in three bf16 parts, which are its 32 bits: column n of the product has part n / GQA
+    Frag pf[SETS];
+#pragma unroll
+    for (int tt = 0; tt < TKEYS / 16; ++tt) {
+      float part[3][4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float p = (sc[tt][r] == -INFINITY) ? 0.0f : exp_of<LOCAL>(sc[tt][r] - m_new);
+        float p = (sc[tt][r] == -INFINITY) ? 0.0f : exp_of<LOCAL>(sc[tt][r] - m_new);
         l_run += p;
-        if (col < GQA) p_me[(tt * 16 + grp * 4 + r) * GQA + col] = p;
+        if constexpr (FP8) p *= vs_now[tt][r];
+        part[0][r] = p;
       }
-    // the strip is this wave's own: in-order LDS, only the compiler is held
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int h = 0; h < GQA; ++h) {
-      const float a = __shfl(alpha, h);
+      for (int e = 0; e < 2; ++e) {
+        const f32x4 x = {part[e][0], part[e][1], part[e][2], part[e][3]};
+        const u32x2 packed = __builtin_bit_cast(u32x2, __builtin_convertvector(x, bf16x4_cvt));
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[h][j] *= a;
+        for (int r = 0; r < 4; ++r)
+          part[e + 1][r] = part[e][r] - __uint_as_float(r & 1 ? packed[r >> 1] & 0xffff0000u : packed[r >> 1] << 16);
+      }
+#pragma unroll
+      for (int e = 0; e < SETS; ++e) {
+        const int mine = GQA == 8 ? (e == 0 ? col / GQA : 2) : col / GQA;
+        f32x4 x;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = mine == 0 ? part[0][r] : mine == 1 ? part[1][r] : part[2][r];
+        const u32x2 packed = __builtin_bit_cast(u32x2, __builtin_convertvector(x, bf16x4_cvt));
+        pf[e].u[tt * 2] = packed[0];
+        pf[e].u[tt * 2 + 1] = packed[1];
+      }
     }
-
-    // ---- P V: lane (col, grp) adds dims col*8.. of keys i*4 + grp ------------
+    hold();
+    // ---- P V: dims 16 i.. by 16 columns; lane (col, grp) has the same keys of either operand ----
 #pragma unroll
-    for (int i = 0; i < TKEYS / 4; ++i) {
-      float p[GQA];
+    for (int i0 = 0; i0 < 8; i0 += 4) {
+      union { s16x4 half[2]; bf16x8_mfma m; } vf[4];
 #pragma unroll
-      for (int h = 0; h < GQA; ++h) p[h] = p_me[(i * 4 + grp) * GQA + h];
-      if constexpr (FP8) {
-        const float s = __shfl(vs, i * 4 + grp);
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int h = 0; h < GQA; ++h) p[h] *= s;
-      }
-      float v[8];
+        for (int tt = 0; tt < 2; ++tt)
+          vf[i].half[tt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) s16x4*)(uintptr_t)((turn_at ^ ((i0 + i) << 5)) + tt * 4096));
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int w = 0; w < (FP8 ? 2 : 4); ++w) {
-        if constexpr (FP8) {
-          const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)vraw[i][w], false);
-          const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)vraw[i][w], true);
-          v[4 * w] = lo[0];
-          v[4 * w + 1] = lo[1];
-          v[4 * w + 2] = hi[0];
-          v[4 * w + 3] = hi[1];
-        } else {
-          v[2 * w] = __uint_as_float(vraw[i][w] << 16);
-          v[2 * w + 1] = __uint_as_float(vraw[i][w] & 0xffff0000u);
-        }
-      }
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int h = 0; h < GQA; ++h)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[h][j] += p[h] * v[j];
+        for (int e = 0; e < SETS; ++e)
+          o[e][i0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i].m, pf[e].m, o[e][i0 + i], 0, 0, 0);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    hold();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (t < tiles) {
+    row = row_of(t, bt[block_of(key_of(t))]);
+    block = bt[block_of(key_of(min(t + step, tiles - 1)))];
+    asm volatile("" : "+v"(block));        // here, not behind K and V
+    __builtin_amdgcn_sched_barrier(0);
+    load_k(row);
+    __builtin_amdgcn_sched_barrier(0);
+    load_v(row);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+    for (; t + step < tiles; t += step) tile(std::true_type());
+    tile(std::false_type());
   }
 
-  // ---- fold the lane groups' keys, then the waves ---------------------------
+  // ---- fold the lane groups' keys, then the parts and the waves ---------------------------
   l_run += __shfl_xor(l_run, 16);
   l_run += __shfl_xor(l_run, 32);
-  // halves, then odd and even rows of 16 lanes: each exchange sums two values and
-  // leaves one in either part, so a lane ends with dims 2*grp' and 2*grp'+1 of its
-  // eight, grp' = the part it landed in
+  float* const sums = reinterpret_cast<float*>(strip);
 #pragma unroll
-  for (int h = 0; h < GQA; ++h) {
-    float half[4];
+  for (int e = 0; e < SETS; ++e) {
+    const int n = e * 16 + col;            // part n / GQA of head n % GQA
+    if (n < 3 * GQA) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[h][j]), __float_as_uint(o[h][j + 4]), false, false);
-      half[j] = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);   // lanes 0-31: dim j, 32-63: dim j + 4
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(half[j]), __float_as_uint(half[j + 2]), false, false);
-      const float v = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);  // even rows: dim j, odd rows: dim j + 2
-      o_lds[wave][h * 128 + col * 8 + (lane >> 5) * 4 + (grp & 1) * 2 + j] = v;
+      for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(sums + n * SUM_PITCH + i * 16 + grp * 4) = o[e][i];
     }
   }
   if (lane < GQA) {
@@ -274,7 +371,7 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
     l_lds[wave][lane] = l_run;
   }
   __syncthreads();
-  float* base = partials + (((int64_t)b * num_kv_heads + g_kv) * Z + z) * GQA * PART_STRIDE;
+  float* base = partials + (((int64_t)b * num_kv_heads + g_kv) * gridDim.z + z) * GQA * PART_STRIDE;
   for (int i = tid; i < GQA * 128; i += NTHREADS) {
     const int h = i >> 7, d = i & 127;
     float M = m_lds[0][h];
@@ -284,33 +381,112 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float e = m_lds[w][h] == -INFINITY ? 0.0f : exp_of<LOCAL>(m_lds[w][h] - M);   // a wave without a tile
-      acc += o_lds[w][i] * e;
+      const float* s = reinterpret_cast<const float*>(strips[w]) + h * SUM_PITCH + d;
+      acc += (s[0] + (s[GQA * SUM_PITCH] + s[2 * GQA * SUM_PITCH])) * e;
       l += l_lds[w][h] * e;
     }
     if (Z == 1) {
       const float v = (l > 0.0f ? acc / l : 0.0f) * head_gate<LOCAL>(gate, gate_stride, b, g_kv * GQA + h);
       ((short*)out)[((int64_t)b * num_kv_heads * GQA + g_kv * GQA + h) * 128 + d] = f32_to_bf16(v);
-    } else {
+    } else if (!arrived) {
       base[h * PART_STRIDE + d] = acc;
       if (d == 0) {
         base[h * PART_STRIDE + 128] = M;
         base[h * PART_STRIDE + 129] = l;
       }
+    } else {
+      const auto far = __builtin_amdgcn_make_buffer_rsrc(base, 0, GQA * PART_STRIDE * 4, 0x00020000);
+      const int at = h * PART_STRIDE * 4;
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc), far, at + d * 4, 0, FAR);
+      if (d == 0) __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(M), __float_as_uint(l)}, far, at + 512, 0, FAR);
     }
   }
+  if (Z == 1 || !arrived) return;
+  // ---- the last workgroup to arrive merges the partials, in their order ----------------------
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  int* const last = reinterpret_cast<int*>(strips[0]);
+  if (tid == 0) {
+    int* const count = arrived + (int64_t)b * num_kv_heads + g_kv;
+    *last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == Z - 1;
+    if (*last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!*last) return;
+  // 32 lanes a head, 4 dims each, all loads before the first wait
+  const float* all = base - (int64_t)z * GQA * PART_STRIDE;
+  const auto far = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(all), 0, Z * GQA * PART_STRIDE * 4, 0x00020000);
+  const int h = tid >> 5, d = (tid & 31) * 4;
+  if (h >= GQA) return;
+  f32x4 part[DECODE_SHARES];
+  float m[DECODE_SHARES], l[DECODE_SHARES], M = -INFINITY;
+#pragma unroll
+  for (int e0 = 0; e0 < DECODE_SHARES; e0 += 4)
+    if (e0 < Z) {
+#pragma unroll
+      for (int e = e0; e < e0 + 4; ++e) {  // behind the last one zeros
+        const int at = (e * GQA + h) * PART_STRIDE * 4;
+        const auto ml = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(far, at + 512, 0, FAR));
+        part[e] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(far, at + d * 4, 0, FAR));
+        m[e] = ml[0];
+        l[e] = ml[1];
+      }
+    }
+#pragma unroll
+  for (int e = 0; e < DECODE_SHARES; ++e)
+    if (e < Z) M = fmaxf(M, m[e]);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  float sum = 0.0f;
+#pragma unroll
+  for (int e = 0; e < DECODE_SHARES; ++e)
+    if (e < Z) {
+      const float w = m[e] == -INFINITY ? 0.0f : exp_of<LOCAL>(m[e] - M);
+      sum += l[e] * w;
+      acc += part[e] * w;
+    }
+  const float open = head_gate<LOCAL>(gate, gate_stride, b, g_kv * GQA + h);
+  bf16x4_vec v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = f32_to_bf16((sum > 0.0f ? acc[r] / sum : 0.0f) * open);
+  *reinterpret_cast<bf16x4_vec*>((short*)out + ((int64_t)b * num_kv_heads * GQA + g_kv * GQA + h) * 128 + d) = v;
 }
 
-// Workgroups per context: about 640 in all, and never more than the longest
-// context has groups of four tiles. Below that the chip is not full, above it the
-// merge and the workgroups' fixed part (lengths, table, fold: 4 us) cost more than
-// the shorter loops give. With the merge, bf16, 960 (stream, kv head) pairs of 560
-// keys: 36.5 us with 1, 42 with 2, 47 with 8; fp8, 128 pairs of 5850 keys: 114 with
-// 1, 58 with 3, 49 with 4 to 6, 54 with 24.
-extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx) {
-  const int most = (max_ctx + 4 * TKEYS - 1) / (4 * TKEYS);
-  const int want = (640 + B * num_kv_heads / 2) / (B * num_kv_heads);
-  const int z = want < most ? want : most;
-  return z < 1 ? 1 : z;
+// Rows of one launch: they lie on the grid's y, which ends at 65535. Steps with a row
+// per token (prompt portions on the fp8 cache, short segments) can have more and go out
+// in several launches; on x, beside the kv heads, every workgroup would divide.
+#define MAX_ROWS 65535
+
+// Shares of a context at most, as long as the chip is not full: 256 workgroups in all for contexts of medium length, whose merge
+// (2 us, 3 in its own launch) weighs most, and for long ones what fills whole rounds of the compute units best: a workgroup more
+// on some of them than on others is waited for. us, 32 / 8 heads, by workgroups in all:
+//   24 streams of 560  192 13.8   384 17.7   768 16.6          of 2500  192 44.3   384 46.0   576 47.1   768 43.6
+//   16 of 6000, fp8  256 44.3   384 46.1   512 41.7   640 46.2   768 43.3       bf16  256 72.1   384 77.7   512 73.7   640 77.6
+//   40 of 2000  320 68.3   640 62.8   960 62.0    40 of 560  320 22.0   640 23.2    8 of 1500  64 21.5   128 16.3   256 15.3   640 15.7
+static DecodeShares attn_decode_shares(int B, int num_kv_heads, int max_ctx, bool fp8, bool joined) {
+  const int64_t pairs = (int64_t)B * num_kv_heads;
+  const int cap = joined ? DECODE_SHARES : 32;
+  DecodeShares s;
+  s.few = joined ? 3 : 1;
+  s.mid = pairs >= 256 ? 1 : (int)(256 / pairs > cap ? cap : 256 / pairs);
+  // long ones: what fills whole rounds of the compute units best
+  s.most = 1;
+  double best = 0.0;
+  for (int z = 1; z <= cap && (z == 1 || pairs * z <= 1024); ++z) {
+    if (pairs * z < (fp8 ? 512 : 256) && z < cap && pairs * (z + 1) <= 1024) continue;
+    const double fill = (double)(pairs * z) / ((pairs * z + 255) / 256 * 256);
+    if (fill > best + 0.02) best = fill, s.most = z;
+  }
+  s.most = s.most < s.mid ? s.mid : s.most;
+  const int rounds = (max_ctx + 4 * TKEYS - 1) / (4 * TKEYS);
+  int z = s.mid > (rounds + 7) / 8 ? s.mid : (rounds + 7) / 8;     // shares_of of any context up to max_ctx is no more
+  z = z > s.most ? s.most : z;
+  s.grid = rounds <= s.few ? 1 : z < rounds ? z : rounds;
+  return s;
+}
+
+// workgroups per context of a launch: room for partials where more than one
+extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx, int fp8, int joined) {
+  return attn_decode_shares(B < MAX_ROWS ? B : MAX_ROWS, num_kv_heads, max_ctx, fp8 != 0, joined != 0).grid;
 }
 
 // merge the partials of a (stream, q head): two dims per lane, the partials dealt
@@ -320,13 +496,14 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(
     bf16_t* __restrict__ out,            // [B, H, 128]
     const float* __restrict__ partials,  // [B, KVH, Z, gqa, 130]
     const int* __restrict__ context_lens, const bf16_t* __restrict__ gate, int gate_stride, int gqa, int Z,
-    int mask_size) {
+    int mask_size, DecodeShares shares) {
   const int b = blockIdx.y, h = blockIdx.x, num_q_heads = gridDim.x;
   const int g_kv = h / gqa, g = h % gqa;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int L = context_lens[b];
   const int tiles = (L - first_key(L, mask_size) + TKEYS - 1) / TKEYS;
-  const int n = min(Z, (tiles + 3) / 4);
+  const int n = shares_of(tiles, shares);
+  if (n == 1) return;                    // its one workgroup has written the result
   const float* base = partials + (((int64_t)b * (num_q_heads / gqa) + g_kv) * Z * gqa + g) * PART_STRIDE;
   const int64_t step = (int64_t)gqa * PART_STRIDE;
   float m = -INFINITY;
@@ -355,34 +532,40 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(
   }
 }
 
-// Rows of one launch: they lie on the grid's y, which ends at 65535. Steps with a row
-// per token (prompt portions on the fp8 cache, short segments) can have more and go out
-// in several launches; on x, beside the kv heads, every workgroup would divide.
-#define MAX_ROWS 65535
-
 // picks the GQA instantiation (the binding admits 1, 2, 4, 8); mask_size: -1 plain decode,
 // from 0 on a block-local layer's (bf16 caches); partials: room for
 // min(B, MAX_ROWS) * KVH * splits * gqa * 130 floats when splits > 1
 extern "C" void launch_attn_decode(
-    bf16_t* out, float* partials, const bf16_t* q, const void* k_cache, const void* v_cache,
+    bf16_t* out, float* partials, int* arrived, const bf16_t* q, const void* k_cache, const void* v_cache,
     const float* k_scale, const float* v_scale, const int* block_tables, const int* context_lens,
     const bf16_t* gate, int gate_stride, float scale, int num_q_heads, int num_kv_heads, int block_size,
-    int max_blocks, int splits, int q_tstride, int B, int cache_fp8, int mask_size, hipStream_t stream) {
+    int max_blocks, int max_ctx, int q_tstride, int B, int cache_fp8, int mask_size, hipStream_t stream) {
   const int gqa = num_q_heads / num_kv_heads;
   const bool local = mask_size >= 0;
+  const DecodeShares sh = attn_decode_shares(B < MAX_ROWS ? B : MAX_ROWS, num_kv_heads, max_ctx, cache_fp8 != 0, arrived != nullptr);
+  const int splits = sh.grid;
+  const bool quads = block_size % 4 == 0 && (reinterpret_cast<uintptr_t>(k_scale) | reinterpret_cast<uintptr_t>(v_scale)) % 16 == 0;
+  const uint32_t block_inverse = block_size > 1 ? (uint32_t)(((1ull << 32) + block_size - 1) / block_size) : ~0u;
   for (int b0 = 0; b0 < B; b0 += MAX_ROWS) {
     const int rows = B - b0 < MAX_ROWS ? B - b0 : MAX_ROWS;
     const dim3 grid(num_kv_heads, rows, splits);
     bf16_t* o = out + (int64_t)b0 * num_q_heads * 128;
     const bf16_t* q0 = q + (int64_t)b0 * q_tstride;
     const int* bt = block_tables + (int64_t)b0 * max_blocks;
+    int* a0 = arrived ? arrived + (int64_t)b0 * num_kv_heads : nullptr;
     const bf16_t* g0 = gate ? gate + (int64_t)b0 * gate_stride : nullptr;
 #define LAUNCH(G, F, L)                                                                            \
   hipLaunchKernelGGL((attn_decode_tiles<G, F, L>), grid, dim3(NTHREADS), 0, stream, partials, o, q0, \
                      (const char*)k_cache, (const char*)v_cache, k_scale, v_scale, bt,             \
-                     context_lens + b0, g0, gate_stride, scale, block_size, max_blocks, q_tstride, mask_size)
+                     context_lens + b0, g0, gate_stride, a0, scale, block_size, block_inverse, max_blocks, q_tstride, \
+                     mask_size, sh)
 #define DISPATCH(G) \
-  do { if (cache_fp8) LAUNCH(G, true, false); else if (local) LAUNCH(G, false, true); else LAUNCH(G, false, false); } while (0)
+  do {                                                                                             \
+    if (cache_fp8 && quads) LAUNCH(G, KV_FP8, false);                                              \
+    else if (cache_fp8) LAUNCH(G, KV_FP8_ANY, false);                                              \
+    else if (local) LAUNCH(G, KV_BF16, true);                                                      \
+    else LAUNCH(G, KV_BF16, false);                                                                \
+  } while (0)
     switch (gqa) {
       case 1: DISPATCH(1); break;
       case 2: DISPATCH(2); break;
@@ -391,9 +574,9 @@ extern "C" void launch_attn_decode(
     }
 #undef DISPATCH
 #undef LAUNCH
-    if (splits > 1)
+    if (splits > 1 && !arrived)
       hipLaunchKernelGGL(local && !cache_fp8 ? attn_decode_merge_kernel<true> : attn_decode_merge_kernel<false>,
                          dim3(num_q_heads, rows), dim3(256), 0, stream, o, partials, context_lens + b0, g0,
-                         gate_stride, gqa, splits, mask_size);
+                         gate_stride, gqa, splits, mask_size, sh);
   }
 }

@@ -15,8 +15,8 @@ extern "C" __global__ void silu_mul_kernel(bf16_t*, const bf16_t*, const bf16_t*
 extern "C" __global__ void rope_kernel(bf16_t*, bf16_t*, const int64_t*, const float*, int, int, int, int, int);
 extern "C" __global__ void store_kv_kernel(const bf16_t*, const bf16_t*, bf16_t*, bf16_t*, const int64_t*, int, int, int, int, int);
 extern "C" __global__ void store_kv_fp8_kernel(const bf16_t*, const bf16_t*, unsigned char*, unsigned char*, float*, float*, const int64_t*, int, int, int, int, int);
-extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx);
-extern "C" void launch_attn_decode(bf16_t*, float*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, const bf16_t*, int, float, int, int, int, int, int, int, int, int, int, hipStream_t);
+extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx, int fp8, int joined);
+extern "C" void launch_attn_decode(bf16_t*, float*, int*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, const bf16_t*, int, float, int, int, int, int, int, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, int, int, float, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill_paged(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, const int*, const int*, const int*, int, float, int, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill_plan(int*, const int*, int, int, hipStream_t);
@@ -152,7 +152,7 @@ void rope_store(torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor
 void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                        torch::Tensor v_cache, torch::Tensor block_tables,
                        torch::Tensor context_lens, double scale,
-                       torch::Tensor k_scale, torch::Tensor v_scale, torch::Tensor gate, int64_t mask_size) {
+                       torch::Tensor k_scale, torch::Tensor v_scale, torch::Tensor gate, int64_t mask_size, std::optional<torch::Tensor> arrived) {
   CHECK_BF16_CONTIG(out); CHECK_BF16_ROWS(q); CHECK_KV_CACHE(k_cache); CHECK_KV_CACHE(v_cache);
   const int B = q.size(0), H = q.size(1), D = q.size(2);
   const int KVH = k_cache.size(1), BS = k_cache.size(2);
@@ -170,7 +170,11 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
     TORCH_CHECK(gate.is_cuda() && gate.scalar_type() == at::kBFloat16 && gate.dim() == 2 && gate.size(0) == B &&
                     gate.size(1) == H && gate.stride(1) == 1, "gate must be a bf16 [B, H] row view");
   const int64_t longest = mask_size > 0 ? std::min<int64_t>(mask_size, (int64_t)max_blocks * BS) : (int64_t)max_blocks * BS;
-  const int splits = attn_decode_splits(B, KVH, (int)longest);
+  const int longest32 = (int)std::min<int64_t>(longest, INT32_MAX);
+  const int splits = attn_decode_splits(B, KVH, longest32, k_cache.scalar_type() == at::kFloat8_e4m3fn, arrived.has_value());
+  if (arrived)
+    TORCH_CHECK(arrived->is_cuda() && arrived->is_contiguous() && arrived->scalar_type() == at::kInt &&
+                    arrived->numel() >= (int64_t)B * KVH, "arrived: an int32 zero for each row and kv head");
   auto partials = torch::empty({splits > 1 ? (int64_t)B * KVH * splits * gqa * 130 : 0},
                                torch::dtype(torch::kFloat).device(q.device()));
   const int cache_fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn ? 1 : 0;
@@ -180,11 +184,11 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
                 "fp8 attn_decode requires [NB, KVH, BS] fp32 k_scale/v_scale");
   }
   launch_attn_decode(
-      bf(out), partials.data_ptr<float>(), cbf(q), k_cache.data_ptr(), v_cache.data_ptr(),
+      bf(out), partials.data_ptr<float>(), arrived ? arrived->data_ptr<int>() : nullptr, cbf(q), k_cache.data_ptr(), v_cache.data_ptr(),
       cache_fp8 ? k_scale.data_ptr<float>() : nullptr,
       cache_fp8 ? v_scale.data_ptr<float>() : nullptr,
       block_tables.data_ptr<int>(), context_lens.data_ptr<int>(), gate.numel() ? cbf(gate) : nullptr,
-      gate.numel() ? (int)gate.stride(0) : 0, (float)scale, H, KVH, BS, max_blocks, splits, (int)q.stride(0), B,
+      gate.numel() ? (int)gate.stride(0) : 0, (float)scale, H, KVH, BS, max_blocks, longest32, (int)q.stride(0), B,
       cache_fp8, (int)mask_size, cur_stream());
 }
 
@@ -555,7 +559,7 @@ bool rows_weights_ok(const std::vector<torch::Tensor>& ws, const torch::Tensor& 
 // --- row-wise steps of a decode step (decode_rows.hip) -------------------------
 extern "C" void launch_add_norm_rows(bf16_t* out, bf16_t* residual, const float* part, const int64_t* ids,
                                      const bf16_t* table, const bf16_t* w, int S, int M, int n, int64_t vocab,
-                                     float eps, int* unknown, hipStream_t stream);
+                                     float eps, int* unknown, int* clear, int clears, hipStream_t stream);
 extern "C" void launch_rope_store_rows(bf16_t* q_out, const float* part, const bf16_t* bias, const int64_t* positions,
                                        const float* cos_sin, void* k_cache, void* v_cache, float* k_scale,
                                        float* v_scale, const int64_t* slots, int S, int M, int H, int G,
@@ -574,24 +578,27 @@ torch::Tensor add_norm_rows(torch::Tensor part, torch::Tensor residual, torch::T
                   n % 4 == 0 && n <= 16384 && S >= 1 && M >= 1, "add_norm_rows: sizes");
   auto out = torch::empty_like(residual);
   launch_add_norm_rows(bf(out), bf(residual), part.data_ptr<float>(), nullptr, nullptr, cbf(weight), S, M, n, 0,
-                       (float)eps, nullptr, cur_stream());
+                       (float)eps, nullptr, nullptr, 0, cur_stream());
   return out;
 }
 
 // (rms(table[ids]) * weight, table[ids]); an id outside the table gives a row of NaN and sets unknown (empty, or one
-// int32 of pinned host memory)
+// int32 of pinned host memory). clear: int32 values that are zeroed beside
 std::vector<torch::Tensor> embed_norm_rows(torch::Tensor ids, torch::Tensor table, torch::Tensor weight, double eps,
-                                           torch::Tensor unknown) {
+                                           torch::Tensor unknown, std::optional<torch::Tensor> clear) {
   CHECK_BF16_CONTIG(table); CHECK_BF16_CONTIG(weight);
   TORCH_CHECK(ids.is_cuda() && ids.is_contiguous() && ids.scalar_type() == at::kLong && ids.dim() == 1);
   const int M = ids.size(0), n = table.size(1);
   TORCH_CHECK(weight.numel() == n && n % 4 == 0 && n <= 16384 && M >= 1, "embed_norm_rows: sizes");
   TORCH_CHECK(unknown.numel() == 0 || (unknown.numel() == 1 && unknown.scalar_type() == at::kInt && unknown.is_pinned()),
               "unknown: one int32 of pinned host memory");
+  TORCH_CHECK(!clear || (clear->is_cuda() && clear->is_contiguous() && clear->scalar_type() == at::kInt &&
+                         clear->numel() <= INT32_MAX), "clear: int32 values");
   auto residual = torch::empty({M, n}, table.options());
   auto out = torch::empty_like(residual);
   launch_add_norm_rows(bf(out), bf(residual), nullptr, ids.data_ptr<int64_t>(), cbf(table), cbf(weight), 0, M, n,
-                       table.size(0), (float)eps, unknown.numel() ? unknown.data_ptr<int>() : nullptr, cur_stream());
+                       table.size(0), (float)eps, unknown.numel() ? unknown.data_ptr<int>() : nullptr,
+                       clear ? clear->data_ptr<int>() : nullptr, clear ? (int)clear->numel() : 0, cur_stream());
   return {out, residual};
 }
 
@@ -704,7 +711,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_rows", &linear_rows);
   m.def("rows_weights_ok", &rows_weights_ok);
   m.def("add_norm_rows", &add_norm_rows);
-  m.def("embed_norm_rows", &embed_norm_rows);
+  m.def("embed_norm_rows", &embed_norm_rows, py::arg("ids"), py::arg("table"), py::arg("weight"), py::arg("eps"),
+        py::arg("unknown"), py::arg("clear") = py::none());
   m.def("rope_store_rows", &rope_store_rows);
   m.def("decode_inputs", &decode_inputs);
   m.def("linear_tiles", &linear_tiles);
@@ -729,7 +737,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_store", &rope_store);
   m.def("attn_decode_paged", &attn_decode_paged, py::arg("out"), py::arg("q"), py::arg("k_cache"),
         py::arg("v_cache"), py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"), py::arg("k_scale"),
-        py::arg("v_scale"), py::arg("gate"), py::arg("mask_size") = -1);
+        py::arg("v_scale"), py::arg("gate"), py::arg("mask_size") = -1, py::arg("arrived") = py::none());
   m.def("attn_prefill", &attn_prefill);
   m.def("attn_prefill_plan", &attn_prefill_plan);
   m.def("attn_prefill_paged", &attn_prefill_paged);

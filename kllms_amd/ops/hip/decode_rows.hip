@@ -67,14 +67,16 @@ __device__ __forceinline__ float row_sum(float v, float* scratch) {
 }
 
 // residual[m] += sum of splits (written back, bf16), or residual[m] = table[ids[m]]
-// (EMBED); out[m] = rms(residual[m]) * w. One workgroup per row, the row in registers:
+// (EMBED, which also zeroes ``clear``); out[m] = rms(residual[m]) * w. One workgroup per row, the row in registers:
 // rows of up to 4 * DR_THREADS * VECS elements.
 template <bool EMBED, int VECS>
 __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
     bf16_t* __restrict__ out, bf16_t* __restrict__ residual, const float* __restrict__ part,
     const int64_t* __restrict__ ids, const bf16_t* __restrict__ table, const bf16_t* __restrict__ w, int S, int M,
-    int n, int64_t vocab, float eps, int* __restrict__ unknown) {
+    int n, int64_t vocab, float eps, int* __restrict__ unknown, int* __restrict__ clear, int clears) {
   __shared__ float red[16];
+  if constexpr (EMBED)
+    for (int i = blockIdx.x * DR_THREADS + threadIdx.x; i < clears; i += gridDim.x * DR_THREADS) clear[i] = 0;
   const int m = blockIdx.x, tid = threadIdx.x;
   const int nvec = n / 4;
   bf16x4_vec* rv = reinterpret_cast<bf16x4_vec*>(residual + (int64_t)m * n);
@@ -123,10 +125,10 @@ __global__ void __launch_bounds__(DR_THREADS) add_norm_rows_kernel(
 
 extern "C" void launch_add_norm_rows(bf16_t* out, bf16_t* residual, const float* part, const int64_t* ids,
                                      const bf16_t* table, const bf16_t* w, int S, int M, int n, int64_t vocab,
-                                     float eps, int* unknown, hipStream_t stream) {
+                                     float eps, int* unknown, int* clear, int clears, hipStream_t stream) {
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(M), dim3(DR_THREADS), 0, stream, out, residual, part, ids, table, w, S, M, n, vocab, eps,
-                       unknown);
+                       unknown, clear, clears);
   };
   const bool narrow = n <= 4 * DR_THREADS;
   if (ids) narrow ? go(add_norm_rows_kernel<true, 1>) : go(add_norm_rows_kernel<true, 4>);

@@ -35,8 +35,8 @@ int launch_linear_rows(void*, const __hip_bfloat16*, const __hip_bfloat16*, cons
 int launch_linear_rows_two(float*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
                            hipStream_t);
 int linear_rows_splits(int, int, int);
-int attn_decode_splits(int, int, int);
-void launch_attn_decode(__hip_bfloat16*, float*, const __hip_bfloat16*, const void*, const void*, const float*,
+int attn_decode_splits(int, int, int, int, int);
+void launch_attn_decode(__hip_bfloat16*, float*, int*, const __hip_bfloat16*, const void*, const void*, const float*,
                         const float*, const int*, const int*, const __hip_bfloat16*, int, float, int, int, int, int, int,
                         int, int, int, int, hipStream_t);
 }
@@ -156,11 +156,12 @@ std::optional<Tensor> hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tens
                            (void*)bf(both, (int64_t)T * KL), squares.data_ptr<float>(), state_slots.data_ptr<int>(),
                            cu.data_ptr<int>(), seg_start.data_ptr<int>(), T, N, H, G, R, BS, RH, RD, RV, st);
   const int64_t longest = mask_size > 0 ? std::min<int64_t>(mask_size, (int64_t)width * BS) : (int64_t)width * BS;
-  const int splits = attn_decode_splits(T, G, (int)std::min<int64_t>(longest, INT32_MAX));
+  const int longest32 = (int)std::min<int64_t>(longest, INT32_MAX);
+  const int splits = attn_decode_splits(T, G, longest32, 0, 0);
   auto partials = torch::empty({splits > 1 ? (int64_t)T * H * splits * 130 : 0}, f32);
-  launch_attn_decode((__hip_bfloat16*)both.data_ptr(), partials.data_ptr<float>(), bf(q), k_cache.data_ptr(),
+  launch_attn_decode((__hip_bfloat16*)both.data_ptr(), partials.data_ptr<float>(), nullptr, bf(q), k_cache.data_ptr(),
                      v_cache.data_ptr(), nullptr, nullptr, tables.data_ptr<int>(), lens.data_ptr<int>(), bf(head_gate), H,
-                     (float)scale, H, G, BS, width, splits, KL, T, 0, (int)mask_size, st);
+                     (float)scale, H, G, BS, width, longest32, KL, T, 0, (int)mask_size, st);
   Tensor left, right;
   if (KL == KR) {    // one launch, half as many sums of each: 40 rows, 2048 x 2048 each, 6.2 us, two launches 5.3 each
     const int S = std::max(linear_rows_splits(T, W, 2 * KL) & ~1, 2);

@@ -70,6 +70,27 @@ def test_paged_decode_tiles(gqa, KVH, BS, ctx, width, fp8):
     assert (err <= 2 ** -8 * ref.abs() + 2e-5).all(), err.max()
 
 
+# lengths at the edges of tiles, of rounds of four and of the lines where more workgroups share a context (3, 8 and 16 rounds);
+# in one launch with counters, and with the merge in a second
+@pytest.mark.parametrize("joined", [True, False])
+@pytest.mark.parametrize("gqa,KVH,BS,fp8", [(1, 3, 16, False), (2, 2, 1, True), (4, 4, 16, False), (4, 8, 4, True), (4, 2, 6, True),
+                                            (8, 1, 16, False), (8, 2, 32, True)])
+@pytest.mark.parametrize("ctx", [[384], [385, 1, 33], [1024, 1025, 31, 32], [2048, 2049, 640, 641, 5], [4200, 90],
+                                 [513 + 17 * i for i in range(70)]])
+def test_shared_contexts(ctx, gqa, KVH, BS, fp8, joined):
+    q, k, v, ks, vs, bt, n = paged_case(len(ctx), KVH, gqa, BS, ctx, fp8, seed=gqa + len(ctx) + BS, width=-(-8192 // BS))
+    dev = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    arrived = torch.zeros(len(ctx) * KVH, dtype=torch.int32, device=DEV) if joined else None
+    args = (dev(q), dev(k), dev(v), dev(bt), dev(n), D ** -0.5, dev(ks), dev(vs), arrived)
+    out = ops.attn_decode_paged(*args)
+    ref = attention64(q, k, v, ks, vs, bt, n, D ** -0.5)
+    err = (out.double().cpu() - ref).abs()
+    # one bf16 rounding of the result (2^-9), fp32 sums before it
+    assert (err <= 2 ** -8 * ref.abs() + 2e-5).all(), err.max()
+    assert torch.equal(ops.attn_decode_paged(*args), out)
+    assert arrived is None or not arrived.any()
+
+
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 64, 65, 128])
 @pytest.mark.parametrize("N,K", [(16, 128), (48, 256), (64, 384), (192, 1280), (2048, 2048)])
 def test_linear_rows(M, N, K):
@@ -113,8 +134,9 @@ def test_add_and_embed_norm_rows(S, M, n):
     assert ((out.double() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5).all()
     table = torch.randn(11, n, generator=g).bfloat16().to(DEV)
     ids = torch.randint(0, 11, (M,), generator=g).to(DEV)
-    out, row = ops.embed_norm_rows(ids, table, w, 1e-5)
-    assert torch.equal(row, table[ids])
+    clear = torch.ones(1500, dtype=torch.int32, device=DEV)
+    out, row = ops.embed_norm_rows(ids, table, w, 1e-5, None, clear)
+    assert torch.equal(row, table[ids]) and not clear.any()
     r = row.double()
     ref = r / torch.sqrt((r * r).mean(-1, keepdim=True) + 1e-5) * w.double()
     assert ((out.double() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5).all()
