@@ -108,7 +108,7 @@ class LlamaAttention(nn.Module):
         if paged is not None and k_scale is None:
             plan, short = paged
             return ops.attn_segments_paged(q, k_cache, v_cache, batch.block_tables, batch.context_lens, self.scale,
-                                           plan, short, batch.seg_tables, batch.seg_start)
+                                           plan, short, batch.seg_tables, batch.seg_start, batch.plans.get("few", False))
         return ops.attn_decode_paged(
             q, k_cache, v_cache, batch.block_tables, batch.context_lens, self.scale,
             k_scale, v_scale, arrived,
@@ -418,7 +418,8 @@ class LlamaForCausalLM(nn.Module):
                 and ops.paged_prefill_pays(batch.host_segs, self.layers[0].self_attn.num_kv_heads)):
             plan, short = ops.paged_prefill_plan(batch.host_segs, input_ids.device)
             if plan is not None:
-                return replace(batch, plans={**(batch.plans or {}), "paged": (plan, short)})
+                return replace(batch, plans={**(batch.plans or {}), "paged": (plan, short),
+                                             "few": ops.paged_prefill_few(batch.host_segs)})
         return batch
 
     def forward_hidden(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:

@@ -170,6 +170,14 @@ def paged_prefill_pays(segs, kv_heads: int) -> bool:
     return bool(long) and kv_heads * sum(k * n for k, n in long) >= PAGED_PREFILL_WORK * max(k for k, _ in long)
 
 
+def paged_prefill_few(segs) -> bool:
+    """Whether the long ones of the segments [(start position, rows)] have up to 64 rows each, behind enough keys that four
+    waves share a row tile's (their sums take 2 us to meet): 32 heads, one of 37 rows behind 1536 52 us and 33, one of 33 behind
+    5 6.5 and 9.4."""
+    long = [(start + n, n) for start, n in segs if n >= PAGED_PREFILL_ROWS]
+    return bool(long) and max(n for _, n in long) <= 64 and max(k for k, _ in long) >= 512
+
+
 def paged_prefill_plan(segs, device) -> tuple:
     """(groups [4, G] on the device, [(first row, rows)] left to row-by-row attention) for segments
     [(start position, rows)] packed in that order; groups None when every segment is short."""
@@ -188,10 +196,11 @@ def paged_prefill_plan(segs, device) -> tuple:
     return plan, short
 
 
-def attn_segments_paged(q, k_cache, v_cache, block_tables, context_lens, scale, plan, short, seg_tables, seg_start):
-    """Rows of long segments on the matrix cores against the paged bf16 cache, the others row by row (GPU only)."""
+def attn_segments_paged(q, k_cache, v_cache, block_tables, context_lens, scale, plan, short, seg_tables, seg_start, few=False):
+    """Rows of long segments on the matrix cores against the paged bf16 cache, the others row by row (GPU only). ``few``: no
+    segment of the plan has more than 64 rows."""
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    _hip_or_raise().attn_prefill_paged(out, q, k_cache, v_cache, plan, seg_tables, seg_start, scale)
+    _hip_or_raise().attn_prefill_paged(out, q, k_cache, v_cache, plan, seg_tables, seg_start, scale, few)
     f = _none(q, torch.float32)
     for r, n in short:
         _hip_or_raise().attn_decode_paged(out[r:r + n], q[r:r + n], k_cache, v_cache, block_tables[r:r + n],

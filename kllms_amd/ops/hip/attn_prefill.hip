@@ -2,8 +2,9 @@
 // sequences, keys either from the same packed rows or from the paged cache.
 //
 //   - an 8-wave workgroup serves 8 consecutive 32-row q-tiles of ONE (sequence,
-//     q-head); 64 keys at a time are staged in LDS for all waves, double-buffered:
-//     the next 64 are on their way to registers while these are multiplied
+//     q-head); 128 keys at a time are staged in LDS for all waves, double-buffered:
+//     the next 128 are on their way there, without registers in between, while these
+//     are multiplied, 64 at a time
 //   - SWAPPED QK^T: S = mfma(A=K_tile, B=Q), so a lane's accumulators hold one q-row's
 //     scores and the softmax is in registers (one permlane32_swap merges the halves)
 //   - P goes to bf16 MFMA B-fragments with pack + half swaps; O^T = mfma(A=V^T, B=P).
@@ -11,24 +12,32 @@
 //     of the decode kernel, which rows behind a cache otherwise take
 //     V lies in LDS as it lies in memory; ds_read_b64_tr_b16 turns it on the way to
 //     the fragment (staging it transposed took 16 two-byte LDS writes a thread)
-//   - K's 16-byte units are XORed with the row, V's 32-byte slots too: both fragment
-//     reads are free of bank conflicts
+//   - K's 16-byte units are XORed with the row, V's 32-byte slots with v_turn of it:
+//     both fragment reads are free of bank conflicts
+//   - where no group has more than 64 rows (the tail of a chat behind a long cache) four
+//     waves share a q-tile, 32 keys of each stage each, and their sums meet in LDS
 //
-// What bounds it: per 32 x 32 scores 16 matrix instructions (512 cycles of a SIMD)
-// stand beside about 500 vector cycles of softmax - half of them the exponentials at a
-// quarter of the rate - and two waves per SIMD overlap the two. So the softmax is kept
-// lean: base-2 exponentials of one fma each, the mask only where a tile crosses the
-// diagonal or the end, the packed conversion instruction, and a running max that is
-// renewed only when it grows by more than 8 (P stays below e^8, fine in fp32 and bf16).
+// What bounds it: a SIMD's two waves, which a barrier keeps in step, do their 32 matrix
+// instructions of a tile (1024 cycles) and their softmax (about 1000 cycles, half of
+// them the exponentials at a quarter of the rate) at the same times, so that the two
+// add up: 3600 cycles for both, matrix and vector units busy 41 and 43 % each. So the
+// barriers are few, the softmax is kept lean - base-2 exponentials of one fma each, the
+// mask only where a tile crosses the diagonal or the end, the packed conversion
+// instruction, and a running max that is renewed only when it grows by more than 8 (P
+// stays below e^8, fine in fp32 and bf16) - and P V has priority over the other wave.
+// Taken back: waves in turns, one at its products while the other is at its softmax,
+// with barriers between (a turn took 2400 cycles); the next tile's scores ahead of this
+// one's softmax (3 % faster for long sequences, 15 % slower for short and paged ones);
+// 64 rows a wave, whose sums and scores the registers do not hold.
 //
 // Grid: q-heads fastest, the heads of a kv head 8 apart, so that with 8 kv heads an
 // XCD's L2 serves one of them; groups of rows longest first, since causal groups
 // differ in length.
 //
-// Measured, 32 heads / 8 kv heads: one sequence of 7777 rows 612 us (810 TFLOP/s; 2019
-// with V staged transposed, synchronous staging and the mask in every tile), 24 of about
-// 512 rows 157 us (345); 8 segments of 150 rows behind 1536 cached keys 96 us
-// in a graph (80 with two parts of P, which keep 16 bits; 551 as single rows).
+// Measured in graphs, 32 heads / 8 kv heads, with 64 keys a stage by way of registers and
+// so, us: one sequence of 7777 rows 548, 502 (986 TFLOP/s), 24 of about 550 177, 142; 16 / 4
+// heads, 8 of 1000 76, 67; 8 segments of 160 rows behind 1536 cached keys 98, 95, 12 of 45
+// behind 2000 135, 85, one of 37 behind 1536 52, 33.
 //
 // MFMA fragment maps (v_mfma_f32_32x32x16_bf16, verified on-device by the
 // mfma_selftest binding):
@@ -47,16 +56,22 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 #define QBLK 32
-#define KVBLK 64                   // staged keys per barrier round
+#define STAGE 128                  // keys staged per barrier round
 #define DHEAD 128
 #define NWAVES 8
-#define TILE_BYTES (KVBLK * 256)   // K or V of a round
+#define STAGE_BYTES (STAGE * 256)  // K or V of a stage
+#define LDS_BYTES (4 * STAGE_BYTES)
+#define SHARE_FLOATS (66 * 64)     // sums of a wave, its maxima and row sums
 
 __device__ __forceinline__ int acc_row(int r, int half) {
   return (r & 3) + 8 * (r >> 2) + 4 * half;   // C/D row map
 }
 
-template <bool PAGED>
+// V's 32-byte slots of a row are XORed with this: the rows of a turned read, 4 by 2 slots, lie in all banks
+__device__ __forceinline__ int v_turn(int row) { return (row & 3) * 2 + (row >> 2 & 1); }
+
+// SHARED: PAGED, groups of up to 64 rows: four waves share a q-tile, each with 32 keys of a stage
+template <bool PAGED, bool SHARED>
 __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
     bf16_t* __restrict__ out,       // [T, H, D] contiguous
     const bf16_t* __restrict__ q,   // [T, H, D], token stride q_tstride
@@ -68,7 +83,7 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
                                          // following; 8: [G, 8] first row of each wave, -1: none
     const int* __restrict__ grp_seg,     // PAGED: [G] row of block_tables / seg_pos
     const int* __restrict__ block_tables, const int* __restrict__ seg_pos,  // PAGED: position of a segment's row 0
-    float scale, int num_kv_heads, int q_tstride, int kv_tstride, int q0_stride, int block_size, int max_blocks) {
+    float scale, int num_kv_heads, int q_tstride, int kv_tstride, int q0_stride, int block_size, uint32_t block_inverse, int max_blocks) {
   const int grp = blockIdx.y;
   const int num_q_heads = gridDim.x;
   const int g_kv = blockIdx.x % num_kv_heads;
@@ -81,11 +96,13 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
 
   const int seqlen = grp_len[grp];
   int qrow0, rows_end = 0;         // this wave's first row; behind the group's last one
+  constexpr int SHARES = SHARED ? 4 : 1;
+  const int share = wave % SHARES;
   if (PAGED || q0_stride == 1) {
     const int q0 = grp_q0[grp];
-    qrow0 = q0 + wave * QBLK;
-    rows_end = min(seqlen, q0 + NWAVES * QBLK);
     if (q0 >= seqlen) return;
+    rows_end = min(seqlen, q0 + NWAVES / SHARES * QBLK);
+    qrow0 = q0 + wave / SHARES * QBLK;
   } else {
     qrow0 = grp_q0[grp * NWAVES + wave];
 #pragma unroll
@@ -98,13 +115,13 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
   const int seq_start = grp_start[grp];
   const int seg = PAGED ? grp_seg[grp] : 0;
   const int pos0 = PAGED ? seg_pos[seg] : 0;          // keys before the sequence's first row
-  const bool active = qrow0 >= 0 && qrow0 < seqlen;
+  const bool active = qrow0 >= 0 && qrow0 < rows_end;
   const int my_pos = pos0 + qrow0 + col;
   // keys visible to the group's last row, and to this wave's
   const int kv_end_grp = pos0 + rows_end;
-  const int kv_end_me = active ? pos0 + min(seqlen, qrow0 + QBLK) : 0;
+  const int kv_end_me = active ? pos0 + min(rows_end, qrow0 + QBLK) : 0;
 
-  __shared__ __attribute__((aligned(16))) char smem[2][2 * TILE_BYTES];  // [buffer][K | V]
+  extern __shared__ __attribute__((aligned(1024))) char smem[];          // [buffer][K | V]
 
   // ---- Q fragments (B-operand): 8 d-slices of 16 --------------------------
   union QFrag { u32x4 u; bf16x8_mfma m; };
@@ -125,177 +142,216 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
   const float c2 = fmaxf(fabsf(scale) * 1.44269504088896340736f, 1e-30f);
   const float THR2 = 8.0f * 1.44269504088896340736f;
 
-  // ---- staging: one key per 8 threads, 32 bytes of K and of V each ---------
-  const int st_key = tid >> 3, st_piece = tid & 7;
-  u32x4 rk[2], rv[2];
+  // ---- staging: straight to LDS, a copy has four rows, a wave COPIES of them of K and of V --------
+  constexpr int COPIES = STAGE / NWAVES / 4;
   const int* bt = PAGED ? block_tables + (int64_t)seg * max_blocks : nullptr;
-  auto row_of = [&](int kt) -> int64_t {              // element offset of this thread's key
-    const int key = min(kt + st_key, kv_end_grp - 1);
-    if constexpr (PAGED)
-      return (((int64_t)bt[key / block_size] * num_kv_heads + g_kv) * block_size + key % block_size) * DHEAD;
-    else
-      return (int64_t)(seq_start + key) * kv_tstride + g_kv * DHEAD;
+  typedef __attribute__((address_space(3))) char* lds_t;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_t)smem;
+  const int st_row = wave * (COPIES * 4) + (lane >> 4), st_unit = lane & 15;
+  int st_block[COPIES];                            // PAGED: of the stage that is asked for next
+  // key / block_size by its reciprocal, which is off by one at most
+  auto block_of = [&](int key) {
+    const int n = (int)__umulhi((uint32_t)key, block_inverse), rest = key - n * block_size;
+    return n - (rest < 0) + (rest >= block_size);
   };
-  auto load_kv = [&](int64_t row) {
-    const u32x4* kp = reinterpret_cast<const u32x4*>((const short*)k + row) + st_piece * 2;
-    const u32x4* vp = reinterpret_cast<const u32x4*>((const short*)v + row) + st_piece * 2;
-    rk[0] = kp[0];
-    rk[1] = kp[1];
-    rv[0] = vp[0];
-    rv[1] = vp[1];
+  auto st_key = [&](int kt, int i) { return min(kt + st_row + i * 4, kv_end_grp - 1); };
+  auto ask_blocks = [&](int kt) {
+    if constexpr (PAGED) {
+#pragma unroll
+      for (int i = 0; i < COPIES; ++i) st_block[i] = bt[block_of(st_key(kt, i))];
+    }
   };
-  auto store_kv = [&](int buf) {
-    char* kb = smem[buf] + st_key * 256;
-    *reinterpret_cast<u32x4*>(kb + (((st_piece * 2) ^ (st_key & 15)) << 4)) = rk[0];
-    *reinterpret_cast<u32x4*>(kb + (((st_piece * 2 + 1) ^ (st_key & 15)) << 4)) = rk[1];
-    u32x4* vb = reinterpret_cast<u32x4*>(smem[buf] + TILE_BYTES + st_key * 256 + ((st_piece ^ (st_key & 7)) << 5));
-    vb[0] = rv[0];
-    vb[1] = rv[1];
+  auto stage = [&](int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) {
+      const int r = st_row + i * 4, key = st_key(kt, i);
+      int64_t row;
+      if constexpr (PAGED) row = (((int64_t)st_block[i] * num_kv_heads + g_kv) * block_size + (key - block_of(key) * block_size)) * DHEAD;
+      else row = (int64_t)(seq_start + key) * kv_tstride + g_kv * DHEAD;
+      const uint32_t to = lds0 + buf * 2 * STAGE_BYTES + (wave * COPIES + i) * 1024;
+      const uint64_t ka = (uint64_t)((const short*)k + row + ((st_unit ^ (r & 15)) << 3));
+      const uint64_t va = (uint64_t)((const short*)v + row + ((st_unit ^ (v_turn(r) << 1)) << 3));
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(ka), "s"(to) : "memory");
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(va), "s"(to + STAGE_BYTES) : "memory");
+    }
   };
 
   f32x16 o_acc[4] = {};
   float m_run = -INFINITY;
   float l_run = 0.0f;
 
-  load_kv(row_of(0));
-  int64_t row_next = row_of(KVBLK);
-  store_kv(0);
-  __syncthreads();
+  constexpr int SUBS = SHARED ? 1 : 2, TILE = SUBS * 32;       // 32-key parts and keys of a wave's tile
+  auto tile = [&](int ks, int kt, int buf) {
+    const char* k_lds = smem + buf * 2 * STAGE_BYTES + (kt - ks) * 256;
+    // ---- QK^T: S[key][qrow], 32 keys each ----------------------------
+    f32x16 s_acc[SUBS] = {};
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+#pragma unroll
+      for (int sub = 0; sub < SUBS; ++sub) {
+        const int krow = col + sub * 32;
+        const bf16x8_mfma a = *reinterpret_cast<const bf16x8_mfma*>(
+            k_lds + krow * 256 + (((s * 2 + half) ^ (krow & 15)) << 4));
+        s_acc[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, q_frag[s].m, s_acc[sub], 0, 0, 0);
+      }
+    }
+    if (kt + TILE > pos0 + qrow0 || kt + TILE > kv_end_grp) {
+      // rows see keys up to their own position, which also ends the sequence
+#pragma unroll
+      for (int sub = 0; sub < SUBS; ++sub)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = kt + sub * 32 + acc_row(r, half);
+          if (key > my_pos || key >= kv_end_grp) s_acc[sub][r] = -INFINITY;
+        }
+    }
+
+    // ---- online softmax (row = lane-local) --------------------------------
+    float tmax = s_acc[0][0];
+#pragma unroll
+    for (int sub = 0; sub < SUBS; ++sub)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s_acc[sub][r]);
+    {
+      auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
+      tmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * c2;
+    }
+    // the running max is renewed per row (lane) and only when it grows by more
+    // than THR2; the first tile always renews it, a tile without a visible key never
+    float alpha = 1.0f;
+    if (!(tmax <= m_run + THR2)) {
+      const float m_new = fmaxf(m_run, tmax);
+      alpha = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+    }
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_acc[dt][r] *= alpha;
+      l_run *= alpha;
+    }
+    // masked scores: fma(-inf, c2, -m) = -inf, whose exponential is 0
+    const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+    // 32 keys of P to B-fragment words; paged: also what bf16 leaves of it, twice (the
+    // differences are exact)
+    constexpr int PARTS = PAGED ? 3 : 1;
+    auto expo = [&](int sub, uint32_t (&w)[PARTS][8]) {
+#pragma unroll
+      for (int pr = 0; pr < 8; ++pr) {
+        f32x2 p;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[sub][2 * pr + e], c2, -m_use));
+          l_run += p[e];
+        }
+#pragma unroll
+        for (int part = 0; part < PARTS; ++part) {
+          w[part][pr] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
+          p[0] -= __uint_as_float(w[part][pr] << 16);
+          p[1] -= __uint_as_float(w[part][pr] & 0xffff0000u);
+        }
+      }
+    };
+
+    // ---- PV: O^T += V^T x P, 16 keys at a time ------------------------------
+    const char* v_lds = k_lds + STAGE_BYTES;
+    // this lane's share of a transposed read: row (lane & 15) / 4, 4 elements
+    const int tr_row = half * 8 + ((lane & 15) >> 2);
+    const int tr_byte = (lane & 3) * 8;
+    const int tr_slot = (lane >> 4) & 1;
+    union PFrag { uint32_t w[4]; bf16x8_mfma m; };
+    auto fragment = [&](const uint32_t (&packs)[8], int kw) {
+      PFrag pf;
+      auto r0 = __builtin_amdgcn_permlane32_swap(packs[4 * kw + 0], packs[4 * kw + 2], false, false);
+      auto r1 = __builtin_amdgcn_permlane32_swap(packs[4 * kw + 1], packs[4 * kw + 3], false, false);
+      pf.w[0] = r0[0];
+      pf.w[1] = r1[0];
+      pf.w[2] = r0[1];
+      pf.w[3] = r1[1];
+      return pf;
+    };
+    auto weighted = [&](int sub, const uint32_t (&w)[PARTS][8]) {
+#pragma unroll
+      for (int kw = 0; kw < 2; ++kw) {
+        PFrag pf[PARTS];
+#pragma unroll
+        for (int part = 0; part < PARTS; ++part) pf[part] = fragment(w[part], kw);
+        const int key = sub * 32 + kw * 16 + tr_row;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          union { s16x4 t[2]; bf16x8_mfma m; } vf;
+#pragma unroll
+          for (int rd = 0; rd < 2; ++rd) {
+            const int kr = key + rd * 4;
+            const char* p = v_lds + kr * 256 + (((dt * 2 + tr_slot) ^ v_turn(kr)) << 5) + tr_byte;
+            vf.t[rd] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+          }
+#pragma unroll
+          for (int part = 0; part < PARTS; ++part)
+            o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.m, pf[part].m, o_acc[dt], 0, 0, 0);
+        }
+      }
+    };
+    uint32_t pw[SUBS][PARTS][8];
+    if constexpr (PAGED) {       // one half after the other: the registers of all six parts are not there
+#pragma unroll
+      for (int sub = 0; sub < SUBS; ++sub) {
+        expo(sub, pw[sub]);
+        weighted(sub, pw[sub]);
+      }
+    } else {
+#pragma unroll
+      for (int sub = 0; sub < SUBS; ++sub) expo(sub, pw[sub]);
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int sub = 0; sub < SUBS; ++sub) weighted(sub, pw[sub]);
+      __builtin_amdgcn_s_setprio(0);
+    }
+  };
+  ask_blocks(0);
+  stage(0, 0);
+  ask_blocks(STAGE);
   int buf = 0;
-  for (int kt = 0; kt < kv_end_grp; kt += KVBLK, buf ^= 1) {
-    const bool more = kt + KVBLK < kv_end_grp;
-    if (more) {
-      load_kv(row_next);
-      row_next = row_of(kt + 2 * KVBLK);
+  for (int ks = 0; ks < kv_end_grp; ks += STAGE, buf ^= 1) {
+    // this stage is there, and the last one's buffer is free
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (ks + STAGE < kv_end_grp) {
+      stage(ks + STAGE, buf ^ 1);
+      ask_blocks(ks + 2 * STAGE);
     }
-    if (kt < kv_end_me) {
-      const char* k_lds = smem[buf];
-      // ---- QK^T: S[key][qrow], two 32-key halves ----------------------------
-      f32x16 s_acc[2] = {};
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-          const int krow = col + sub * 32;
-          const bf16x8_mfma a = *reinterpret_cast<const bf16x8_mfma*>(
-              k_lds + krow * 256 + (((s * 2 + half) ^ (krow & 15)) << 4));
-          s_acc[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, q_frag[s].m, s_acc[sub], 0, 0, 0);
-        }
-      }
-      if (kt + KVBLK > pos0 + qrow0 || kt + KVBLK > kv_end_grp) {
-        // rows see keys up to their own position, which also ends the sequence
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = kt + sub * 32 + acc_row(r, half);
-            if (key > my_pos || key >= kv_end_grp) s_acc[sub][r] = -INFINITY;
-          }
-      }
+    const int end = min(ks + STAGE, kv_end_me);
+#pragma unroll 1
+    for (int kt = ks + share * TILE; kt < end; kt += SHARES * TILE) tile(ks, kt, buf);
+  }
 
-      // ---- online softmax (row = lane-local) --------------------------------
-      float tmax = s_acc[0][0];
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s_acc[sub][r]);
-      {
-        auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
-        tmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * c2;
-      }
-      // the running max is renewed per row (lane) and only when it grows by more
-      // than THR2; the first tile always renews it, a tile without a visible key never
-      float alpha = 1.0f;
-      if (!(tmax <= m_run + THR2)) {
-        const float m_new = fmaxf(m_run, tmax);
-        alpha = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
-        m_run = m_new;
-      }
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) o_acc[dt][r] *= alpha;
-        l_run *= alpha;
-      }
-      // masked scores: fma(-inf, c2, -m) = -inf, whose exponential is 0
-      const float m_use = m_run == -INFINITY ? 0.0f : m_run;
-      // 32 keys of P to B-fragment words; paged: also what bf16 leaves of it, twice (the
-      // differences are exact)
-      constexpr int PARTS = PAGED ? 3 : 1;
-      auto expo = [&](int sub, uint32_t (&w)[PARTS][8]) {
-#pragma unroll
-        for (int pr = 0; pr < 8; ++pr) {
-          f32x2 p;
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[sub][2 * pr + e], c2, -m_use));
-            l_run += p[e];
-          }
-#pragma unroll
-          for (int part = 0; part < PARTS; ++part) {
-            w[part][pr] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
-            p[0] -= __uint_as_float(w[part][pr] << 16);
-            p[1] -= __uint_as_float(w[part][pr] & 0xffff0000u);
-          }
-        }
-      };
-
-      // ---- PV: O^T += V^T x P, 16 keys at a time ------------------------------
-      const char* v_lds = smem[buf] + TILE_BYTES;
-      // this lane's share of a transposed read: row (lane & 15) / 4, 4 elements
-      const int tr_row = half * 8 + ((lane & 15) >> 2);
-      const int tr_byte = (lane & 3) * 8;
-      const int tr_slot = (lane >> 4) & 1;
-      union PFrag { uint32_t w[4]; bf16x8_mfma m; };
-      auto fragment = [&](const uint32_t (&packs)[8], int kw) {
-        PFrag pf;
-        auto r0 = __builtin_amdgcn_permlane32_swap(packs[4 * kw + 0], packs[4 * kw + 2], false, false);
-        auto r1 = __builtin_amdgcn_permlane32_swap(packs[4 * kw + 1], packs[4 * kw + 3], false, false);
-        pf.w[0] = r0[0];
-        pf.w[1] = r1[0];
-        pf.w[2] = r0[1];
-        pf.w[3] = r1[1];
-        return pf;
-      };
-      auto weighted = [&](int sub, const uint32_t (&w)[PARTS][8]) {
-#pragma unroll
-        for (int kw = 0; kw < 2; ++kw) {
-          PFrag pf[PARTS];
-#pragma unroll
-          for (int part = 0; part < PARTS; ++part) pf[part] = fragment(w[part], kw);
-          const int key = sub * 32 + kw * 16 + tr_row;
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt) {
-            union { s16x4 t[2]; bf16x8_mfma m; } vf;
-#pragma unroll
-            for (int rd = 0; rd < 2; ++rd) {
-              const int kr = key + rd * 4;
-              const char* p = v_lds + kr * 256 + (((dt * 2 + tr_slot) ^ (kr & 7)) << 5) + tr_byte;
-              vf.t[rd] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
-            }
-#pragma unroll
-            for (int part = 0; part < PARTS; ++part)
-              o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.m, pf[part].m, o_acc[dt], 0, 0, 0);
-          }
-        }
-      };
-      uint32_t pw[2][PARTS][8];
-      if constexpr (PAGED) {       // one half after the other: the registers of all six parts are not there
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-          expo(sub, pw[sub]);
-          weighted(sub, pw[sub]);
-        }
-      } else {
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) expo(sub, pw[sub]);
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) weighted(sub, pw[sub]);
-      }
-    }
-    if (more) store_kv(buf ^ 1);
+  // ---- the shares' sums, lane by lane, to the first of a q-tile's waves ----------
+  if constexpr (SHARED) {
     __syncthreads();
+    // of both q-tiles the other three: 6 of 16.5 KB
+    float* const sums = reinterpret_cast<float*>(smem) + (wave - wave / SHARES - (share > 0)) * SHARE_FLOATS + lane;
+    if (share > 0) {
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sums[(dt * 16 + r) * 64] = o_acc[dt][r];
+      sums[64 * 64] = m_run;
+      sums[65 * 64] = l_run;
+    }
+    __syncthreads();
+    if (share > 0) return;
+    for (int e = 0; e < SHARES - 1; ++e) {
+      const float* theirs = sums + e * SHARE_FLOATS;
+      const float m = theirs[64 * 64], m_new = fmaxf(m_run, m);
+      const float a = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+      const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
+      m_run = m_new;
+      l_run = l_run * a + theirs[65 * 64] * w;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_acc[dt][r] = o_acc[dt][r] * a + theirs[(dt * 16 + r) * 64] * w;
+    }
   }
 
   // ---- epilogue: merge half-sums, normalize, write O ----------------------
@@ -303,7 +359,7 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
     l_run = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
-  if (active && qrow0 + col < seqlen) {
+  if (active && qrow0 + col < rows_end) {
     const float inv_l = (l_run > 0.0f) ? 1.0f / l_run : 0.0f;
     bf16_t* op = out + (((int64_t)(seq_start + qrow0 + col)) * num_q_heads + h) * DHEAD;
 #pragma unroll
@@ -324,27 +380,40 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
 // least, so many short prompts have as many)
 #define MAX_GROUPS 65535
 
-extern "C" void launch_attn_prefill(bf16_t* out, const bf16_t* q, const bf16_t* k, const bf16_t* v,
-                                    const int* grp_start, const int* grp_len, const int* grp_q0, int q0_stride,
-                                    int ngroups, float scale, int num_q_heads, int num_kv_heads, int q_tstride,
-                                    int kv_tstride, hipStream_t stream) {
-  for (int g = 0; g < ngroups; g += MAX_GROUPS)
-    hipLaunchKernelGGL(attn_prefill_kernel<false>, dim3(num_q_heads, ngroups - g < MAX_GROUPS ? ngroups - g : MAX_GROUPS),
-                       dim3(64 * NWAVES), 0, stream, out, q, k, v, grp_start + g, grp_len + g,
-                       grp_q0 + (int64_t)g * q0_stride, nullptr, nullptr, nullptr, scale, num_kv_heads, q_tstride,
-                       kv_tstride, q0_stride, 1, 0);
+// room for the kernels' LDS; asked for at each launch: the attribute is the current device's
+static bool prefill_lds_ready(const void* kernel) {
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) == hipSuccess;
 }
 
-extern "C" void launch_attn_prefill_paged(bf16_t* out, const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache,
-                                          const int* grp_start, const int* grp_len, const int* grp_q0,
-                                          const int* grp_seg, const int* block_tables, const int* seg_pos, int ngroups,
-                                          float scale, int num_q_heads, int num_kv_heads, int q_tstride,
-                                          int block_size, int max_blocks, hipStream_t stream) {
+// 0, or -1 where the LDS cannot be had
+extern "C" int launch_attn_prefill(bf16_t* out, const bf16_t* q, const bf16_t* k, const bf16_t* v,
+                                   const int* grp_start, const int* grp_len, const int* grp_q0, int q0_stride,
+                                   int ngroups, float scale, int num_q_heads, int num_kv_heads, int q_tstride,
+                                   int kv_tstride, hipStream_t stream) {
+  if (!prefill_lds_ready(reinterpret_cast<const void*>(attn_prefill_kernel<false, false>))) return -1;
   for (int g = 0; g < ngroups; g += MAX_GROUPS)
-    hipLaunchKernelGGL(attn_prefill_kernel<true>, dim3(num_q_heads, ngroups - g < MAX_GROUPS ? ngroups - g : MAX_GROUPS),
-                       dim3(64 * NWAVES), 0, stream, out, q, k_cache, v_cache, grp_start + g, grp_len + g, grp_q0 + g,
-                       grp_seg + g, block_tables, seg_pos, scale, num_kv_heads, q_tstride, 0, 1, block_size,
+    hipLaunchKernelGGL((attn_prefill_kernel<false, false>), dim3(num_q_heads, ngroups - g < MAX_GROUPS ? ngroups - g : MAX_GROUPS),
+                       dim3(64 * NWAVES), LDS_BYTES, stream, out, q, k, v, grp_start + g, grp_len + g,
+                       grp_q0 + (int64_t)g * q0_stride, nullptr, nullptr, nullptr, scale, num_kv_heads, q_tstride,
+                       kv_tstride, q0_stride, 1, ~0u, 0);
+  return 0;
+}
+
+// few: no group has more than 64 rows
+extern "C" int launch_attn_prefill_paged(bf16_t* out, const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache,
+                                         const int* grp_start, const int* grp_len, const int* grp_q0,
+                                         const int* grp_seg, const int* block_tables, const int* seg_pos, int ngroups,
+                                         float scale, int num_q_heads, int num_kv_heads, int q_tstride,
+                                         int block_size, int max_blocks, int few, hipStream_t stream) {
+  const auto kernel = few ? attn_prefill_kernel<true, true> : attn_prefill_kernel<true, false>;
+  if (!prefill_lds_ready(reinterpret_cast<const void*>(kernel))) return -1;
+  const uint32_t inverse = block_size > 1 ? (uint32_t)(((1ull << 32) + block_size - 1) / block_size) : ~0u;
+  for (int g = 0; g < ngroups; g += MAX_GROUPS)
+    hipLaunchKernelGGL(kernel, dim3(num_q_heads, ngroups - g < MAX_GROUPS ? ngroups - g : MAX_GROUPS),
+                       dim3(64 * NWAVES), LDS_BYTES, stream, out, q, k_cache, v_cache, grp_start + g, grp_len + g, grp_q0 + g,
+                       grp_seg + g, block_tables, seg_pos, scale, num_kv_heads, q_tstride, 0, 1, block_size, inverse,
                        max_blocks);
+  return 0;
 }
 
 // Groups of 256 rows of each sequence cu[i]..cu[i+1], into plan [3, G] (start, length,

@@ -17,8 +17,8 @@ extern "C" __global__ void store_kv_kernel(const bf16_t*, const bf16_t*, bf16_t*
 extern "C" __global__ void store_kv_fp8_kernel(const bf16_t*, const bf16_t*, unsigned char*, unsigned char*, float*, float*, const int64_t*, int, int, int, int, int);
 extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx, int fp8, int joined);
 extern "C" void launch_attn_decode(bf16_t*, float*, int*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, const bf16_t*, int, float, int, int, int, int, int, int, int, int, int, hipStream_t);
-extern "C" void launch_attn_prefill(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, int, int, float, int, int, int, int, hipStream_t);
-extern "C" void launch_attn_prefill_paged(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, const int*, const int*, const int*, int, float, int, int, int, int, int, hipStream_t);
+extern "C" int launch_attn_prefill(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, int, int, float, int, int, int, int, hipStream_t);
+extern "C" int launch_attn_prefill_paged(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, const int*, const int*, const int*, int, float, int, int, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill_plan(int*, const int*, int, int, hipStream_t);
 extern "C" int64_t sample_room(int B, int V, int masked);
 extern "C" void launch_sample(int64_t*, float*, void*, const float*, const float*, const float*, const int*, const int64_t*, const int64_t*, const uint32_t*, int, int, float*, hipStream_t);
@@ -220,15 +220,16 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k, torch::Te
   if (!rows_aligned(q)) q = q.contiguous();
   if (!rows_aligned(k) || !rows_aligned(v)) { k = k.contiguous(); v = v.contiguous(); }
   const int* p = plan.data_ptr<int>();
-  launch_attn_prefill(bf(out), cbf(q), cbf(k), cbf(v), p, p + G, p + 2 * G, 1, G, (float)scale, H, KVH,
-                      (int)q.stride(0), (int)k.stride(0), cur_stream());
+  TORCH_CHECK(launch_attn_prefill(bf(out), cbf(q), cbf(k), cbf(v), p, p + G, p + 2 * G, 1, G, (float)scale, H, KVH,
+                                  (int)q.stride(0), (int)k.stride(0), cur_stream()) == 0,
+              "attn_prefill: 128 KB of LDS are not available");
 }
 
 // rows of segments against the paged cache (bf16): plan [4, G] int32 (first row, rows, first row within the
 // segment, segment), tables [n, MAXB], pos [n] = position of each segment's first row. The segments' own keys and
-// values are in the cache already.
+// values are in the cache already. few: no segment of the plan has more than 64 rows.
 void attn_prefill_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache, torch::Tensor v_cache,
-                        torch::Tensor plan, torch::Tensor tables, torch::Tensor pos, double scale) {
+                        torch::Tensor plan, torch::Tensor tables, torch::Tensor pos, double scale, bool few) {
   CHECK_BF16_CONTIG(out); CHECK_BF16_ROWS(q); CHECK_BF16_CONTIG(k_cache); CHECK_BF16_CONTIG(v_cache);
   const int H = q.size(1), KVH = k_cache.size(1), BS = k_cache.size(2);
   TORCH_CHECK(q.size(2) == 128 && k_cache.size(3) == 128 && v_cache.sizes() == k_cache.sizes() && H % KVH == 0,
@@ -241,9 +242,10 @@ void attn_prefill_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cach
   if (G == 0) return;
   if (!rows_aligned(q)) q = q.contiguous();
   const int* p = plan.data_ptr<int>();
-  launch_attn_prefill_paged(bf(out), cbf(q), cbf(k_cache), cbf(v_cache), p, p + G, p + 2 * G, p + 3 * G,
-                            tables.data_ptr<int>(), pos.data_ptr<int>(), G, (float)scale, H, KVH, (int)q.stride(0),
-                            BS, (int)tables.size(1), cur_stream());
+  TORCH_CHECK(launch_attn_prefill_paged(bf(out), cbf(q), cbf(k_cache), cbf(v_cache), p, p + G, p + 2 * G, p + 3 * G,
+                                        tables.data_ptr<int>(), pos.data_ptr<int>(), G, (float)scale, H, KVH, (int)q.stride(0),
+                                        BS, (int)tables.size(1), few, cur_stream()) == 0,
+              "attn_prefill_paged: 128 KB of LDS are not available");
 }
 
 // (tokens, logprobs). The results are allocated here: 16 rows take 8.8 us on the device, and from Python the two allocations
@@ -740,7 +742,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("v_scale"), py::arg("gate"), py::arg("mask_size") = -1, py::arg("arrived") = py::none());
   m.def("attn_prefill", &attn_prefill);
   m.def("attn_prefill_plan", &attn_prefill_plan);
-  m.def("attn_prefill_paged", &attn_prefill_paged);
+  m.def("attn_prefill_paged", &attn_prefill_paged, py::arg("out"), py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
+        py::arg("plan"), py::arg("tables"), py::arg("pos"), py::arg("scale"), py::arg("few") = false);
   m.def("sample", &sample);
   m.def("mfma_selftest", &mfma_selftest);
   m.def("one_shot_allreduce", &one_shot_allreduce);

@@ -108,9 +108,9 @@ int seq_launch_attn_diff_paged(void*, const void*, const void*, const void*, con
 
 // dense varlen causal MFMA prefill kernel (ops/hip/attn_prefill.hip, also part
 // of kllms_amd._C): bf16, head size 128, 8 q-tiles of 32 rows per workgroup
-extern "C" void launch_attn_prefill(__hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*,
-                                    const __hip_bfloat16*, const int*, const int*, const int*, int, int, float, int,
-                                    int, int, int, hipStream_t);
+extern "C" int launch_attn_prefill(__hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*,
+                                   const __hip_bfloat16*, const int*, const int*, const int*, int, int, float, int,
+                                   int, int, int, hipStream_t);
 
 static inline hipStream_t cur_stream() { return at::hip::getCurrentHIPStream().stream(); }
 
@@ -509,10 +509,11 @@ void attn_varlen_mfma(torch::Tensor out, torch::Tensor q, torch::Tensor k, torch
   const int ngroups = grp_start.numel();
   TORCH_CHECK(grp_qpos0.numel() == (int64_t)ngroups * 8 && grp_len.numel() == ngroups);
   if (ngroups == 0) return;
-  launch_attn_prefill((__hip_bfloat16*)out.data_ptr(), (const __hip_bfloat16*)q.data_ptr(),
-                      (const __hip_bfloat16*)k.data_ptr(), (const __hip_bfloat16*)v.data_ptr(),
-                      grp_start.data_ptr<int>(), grp_len.data_ptr<int>(), grp_qpos0.data_ptr<int>(), 8, ngroups,
-                      (float)scale, H, G, (int)q.stride(0), (int)k.stride(0), cur_stream());
+  TORCH_CHECK(launch_attn_prefill((__hip_bfloat16*)out.data_ptr(), (const __hip_bfloat16*)q.data_ptr(),
+                                  (const __hip_bfloat16*)k.data_ptr(), (const __hip_bfloat16*)v.data_ptr(),
+                                  grp_start.data_ptr<int>(), grp_len.data_ptr<int>(), grp_qpos0.data_ptr<int>(), 8, ngroups,
+                                  (float)scale, H, G, (int)q.stride(0), (int)k.stride(0), cur_stream()) == 0,
+              "128 KB of LDS are not available");
 }
 
 static void check_segments(const torch::Tensor& slots, const torch::Tensor& cu, const torch::Tensor& seg_start,
