@@ -4,7 +4,7 @@
 // The weights' stream is the bound, and bytes in flight are what keeps it up: W and x go from memory to LDS without
 // registers in between, 64 deep in k, and a workgroup has all its buffers on their way from its first instruction on -
 // 60 to 150 KB of a compute unit. (Weights loaded to registers two to four chunks ahead, with x through two LDS buffers,
-// streamed 28672 x 4096 at 4.6 TB/s for 5 rows and at 3.4 for 96; so it is 5.7 and 5.2.) A workgroup takes 64 or 128 rows of
+// streamed 28672 x 4096 at 4.6 TB/s for 5 rows and at 3.4 for 96; so it is 5.7 and 5.2, 6.2 with the streaming hint.) A workgroup takes 64 or 128 rows of
 // W; MJ tiles of 32 rows of x are multiplied at once, so that LDS is read once for 16 * MJ rows and not for 16.
 //
 // A matrix of few rows is also split over k (linear_rows_splits); the splits' fp32 sums are left to the consumer, which
@@ -13,7 +13,8 @@
 //   F32   fp32, S = 1 (logits)         CLAMPED  the clamped gated form of the hybrid family
 //   BF16  rounded once, bias added before it
 //
-// Measured in graphs, weights out of cache, us with the weights through registers and now:
+// Measured in graphs, weights out of cache, us with the weights through registers and so, both without the streaming hint of
+// large matrices (LR_ONCE has what that gives):
 //   PART  4096 x 4096   5 rows 8.5, 8.1   40 rows 10.0, 8.7   96 14.3, 11.0     6144 x 4096   5 rows 11.6, 11.1   64 15.9, 12.9
 //     4096 x 14336   5 rows 23.7, 23.3   40 26.4, 24.9   96 35.0, 30.6     2048 x 8192   16 rows 9.2, 8.6   128 16.6, 12.4
 //     2048 x 2048   5 rows 3.9, 4.3   128 7.4, 6.2
@@ -33,8 +34,8 @@ enum LinearForm { LR_PART = 0, LR_BF16 = 1, LR_F32 = 2, LR_SILU = 3, LR_CLAMPED 
 // Workgroups by share of k, then by rows of W, then by rows of x: those of an XCD have the same part of x in its L2, and
 // the row tiles of a part of W run side by side.
 // more: the bias (BF16), or a second matrix (PART): then K is both matrices' and the halves of the splits are two products, of
-// x's first M rows with w and of the next M with more.
-template <int NI, int MJ, int FORM, int KB>
+// x's first M rows with w and of the next M with more. ONCE: W passes the caches by (LR_ONCE)
+template <int NI, int MJ, int FORM, int KB, bool ONCE>
 __global__ void __launch_bounds__(TP_THREADS, 1) linear_rows_kernel(
     void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const bf16_t* __restrict__ more,
     int M, int N, int K, int x_stride, int m_tiles, int splits, float limit, float alpha) {
@@ -74,7 +75,7 @@ __global__ void __launch_bounds__(TP_THREADS, 1) linear_rows_kernel(
     }
   }
   const TileRows xr(xk, m0 + wave * MJ * 8, m_end, MJ * 8, x_stride, stages * TP_K, lane);
-  const TileRows wr(wk, n_put, columns, 8 * NI, w_row, lane);
+  const TileRowsOf<ONCE> wr(wk, n_put, columns, 8 * NI, w_row, lane);
   // the XCDs begin at different k: rows of a power of two of bytes would have all of them at the same memory channels
   tile_product<MJ, NI, KB * 1024>(acc, wr, xr, stages, stages * xcd / 8, smem);
   if constexpr (FORM == LR_SILU && MJ > 4) {       // many rows: whole lines
@@ -179,14 +180,26 @@ static bool lr_lds_ready(const void* kernel, std::atomic<uint64_t>& devices) {
   return true;
 }
 
-template <int NI, int MJ, int FORM, int KB>
+// Bytes of a matrix from which on its rows are loaded with the streaming hint (nt). A model whose matrices are as large does not
+// fit the last-level cache (256 MB) from one step to the next: without the hint they push out of it, and of the L2, what the
+// step reads again (x, sums, keys of shared prompts) and hit nothing themselves. us without and with, 900 MB of weights in turn:
+//   PART  4096 x 4096   5 rows 8.1, 7.7   120 rows 12.4, 12.2     6144 x 4096   5 rows 11.3, 10.6   120 16.4, 16.1
+//     4096 x 14336   5 rows 23.8, 20.9   120 32.7, 31.5   384 59.7, 58.6     2048 x 8192   1 row 8.9, 8.2   120 12.3, 12.2
+//   SILU  28672 x 4096   5 rows 41.6, 37.6 (6.2 TB/s)   120 49.6, 46.9   256 64.3, 63.5     16384 x 2048   1 row 14.4, 13.1
+//   F32   32000 x 4096   5 rows 46.6, 41.3   120 54.9, 51.7
+// Weights that do fit lose by it, at many rows above all: 130 MB of 16384 x 2048 1 row 12.9, 11.9   100 rows 13.8, 16.6; 200 MB of
+// 2048 x 2048 4.2, 4.2 and 5.8, 6.4; 30 MB of 1024 x 1024 3.6, 3.6 and 5.0, 5.2; 100 MB of 4096 x 1024 6.2, 6.3 and 8.1, 9.7.
+// From widths of 2048 on a layer has 120 MB; below, the matrices are smaller than this.
+#define LR_ONCE (8 << 20)
+
+template <int NI, int MJ, int FORM, int KB, bool ONCE>
 static int linear_rows_go(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* more, int M, int N, int K, int x_stride,
                           int m_tiles, int splits, float limit, float alpha, hipStream_t stream) {
   static std::atomic<uint64_t> devices{0};
-  if (!lr_lds_ready(reinterpret_cast<const void*>(linear_rows_kernel<NI, MJ, FORM, KB>), devices)) return -1;
+  if (!lr_lds_ready(reinterpret_cast<const void*>(linear_rows_kernel<NI, MJ, FORM, KB, ONCE>), devices)) return -1;
   constexpr int LDS = TileRing<MJ, NI, KB * 1024>::STRIDE * TileRing<MJ, NI, KB * 1024>::RING;
   const int64_t all = (int64_t)((N + 32 * NI - 1) / (32 * NI)) * splits * m_tiles;
-  hipLaunchKernelGGL((linear_rows_kernel<NI, MJ, FORM, KB>), dim3((all + 7) / 8 * 8), dim3(TP_THREADS), LDS, stream, out, x, w, more,
+  hipLaunchKernelGGL((linear_rows_kernel<NI, MJ, FORM, KB, ONCE>), dim3((all + 7) / 8 * 8), dim3(TP_THREADS), LDS, stream, out, x, w, more,
                      M, N, K, x_stride, m_tiles, splits, limit, alpha);
   return 0;
 }
@@ -194,10 +207,14 @@ static int linear_rows_go(void* out, const bf16_t* x, const bf16_t* w, const bf1
 template <int FORM>
 static int linear_rows_form(const LinearPlan& p, void* out, const bf16_t* x, const bf16_t* w, const bf16_t* more, int M, int N,
                             int K, int x_stride, int splits, float limit, float alpha, hipStream_t stream) {
+  // of two matrices K is both's
+  const bool once = (int64_t)N * K * (int64_t)sizeof(bf16_t) >= LR_ONCE;
 #define LR_CASE(NI, MJ)                                                                                              \
   if (p.ni == NI && p.mj == MJ)                                                                                      \
-    return linear_rows_go<NI, MJ, FORM, (NI == 2 || MJ <= 2 ? 80 : 160)>(out, x, w, more, M, N, K, x_stride, p.m_tiles, splits, limit, \
-                                                                         alpha, stream)
+    return once ? linear_rows_go<NI, MJ, FORM, (NI == 2 || MJ <= 2 ? 80 : 160), true>(out, x, w, more, M, N, K, x_stride, p.m_tiles, \
+                                                                                      splits, limit, alpha, stream)  \
+                : linear_rows_go<NI, MJ, FORM, (NI == 2 || MJ <= 2 ? 80 : 160), false>(out, x, w, more, M, N, K, x_stride, p.m_tiles, \
+                                                                                       splits, limit, alpha, stream)
   LR_CASE(2, 1);
   LR_CASE(2, 2);
   LR_CASE(2, 3);

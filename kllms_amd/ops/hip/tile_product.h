@@ -90,10 +90,17 @@ __device__ __forceinline__ u32x4 tp_range(const void* p, uint32_t bytes) {
 // compiler makes every later LDS read wait for the builtin's; the waits stand in the loop.
 // The step to the copy's row is in the lane's offset, which the range check covers: of the scalar offset it
 // only has to hold that it stays within the range (k inside a row), not what a check makes of one beyond it.
+// ONCE: the caches need not hold it for longer than it takes (nt).
+template <bool ONCE = false>
 __device__ __forceinline__ void tp_copy(u32x4 range, uint32_t lane_off, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(lane_off), "s"(range),
-               "s"(off), "s"(lds)
-               : "memory");
+  if constexpr (ONCE)
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds" ::"v"(lane_off), "s"(range),
+                 "s"(off), "s"(lds)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(lane_off), "s"(range),
+                 "s"(off), "s"(lds)
+                 : "memory");
 }
 
 __device__ __forceinline__ void tp_copy_at(uint64_t at, uint32_t lds) {
@@ -105,26 +112,28 @@ __device__ __forceinline__ void tp_copy_at(uint64_t at, uint32_t lds) {
 // range always holds a row: what comes of it belongs to rows or columns that are not stored. K: elements from a row to the
 // next, width: those of a row that are read. The range ends with the last row's: rows may overlap or be one and the same
 // (K below width), and then what does not exist reads others' values, for rows that are not stored either.
-struct TileRows {
+template <bool ONCE>
+struct TileRowsOf {
   u32x4 range;
   uint32_t at[8];            // this lane's offset in each copy: the same registers for all operands of one K
-  __device__ __forceinline__ TileRows(const bf16_t* p, int first, int end, int most, int K, int lane)
-      : TileRows(p, first, end, most, K, K, lane) {}
-  __device__ __forceinline__ TileRows(const bf16_t* p, int first, int end, int most, int K, int width, int lane)
+  __device__ __forceinline__ TileRowsOf(const bf16_t* p, int first, int end, int most, int K, int lane)
+      : TileRowsOf(p, first, end, most, K, K, lane) {}
+  __device__ __forceinline__ TileRowsOf(const bf16_t* p, int first, int end, int most, int K, int width, int lane)
       : range(tp_range(p + (int64_t)min(first, end - 1) * K,
                        ((uint32_t)(min(end - min(first, end - 1), most) - 1) * K + width) * 2)) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       at[i] = (uint32_t)(i * 8 + (lane >> 3)) * K * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
   }
-  __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds) const { tp_copy(range, at[i], k_off, lds); }
+  __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds) const { tp_copy<ONCE>(range, at[i], k_off, lds); }
   // zeros, without a look at memory, where not ``live``
   __device__ __forceinline__ void copy(int i, uint32_t k_off, uint32_t lds, bool live) const {
     u32x4 r = range;
     r[2] = live ? r[2] : 0;
-    tp_copy(r, at[i], k_off, lds);
+    tp_copy<ONCE>(r, at[i], k_off, lds);
   }
 };
+typedef TileRowsOf<false> TileRows;
 
 // Rows anywhere: at[i] is the address of this lane's 16 bytes of the i-th copy in stage 0.
 template <int MJ>
@@ -142,8 +151,8 @@ struct TileRing {
 
 // acc += W X^T over K; w: this wave's 8 * NI of the 32 * NI rows (64 of 256), x: its 8 * MJ of the 32 * MJ. Ends with all
 // waves past their last LDS read. NI 4, tiles of 128 columns, is for few rows: half the sums, more buffers in flight.
-template <int MJ, int NI = 8, int BYTES = TP_LDS, class X>
-__device__ __forceinline__ void tile_product(f32x4 (&acc)[NI][MJ], const TileRows& w, const X& x, int stages, int start,
+template <int MJ, int NI = 8, int BYTES = TP_LDS, class W, class X>
+__device__ __forceinline__ void tile_product(f32x4 (&acc)[NI][MJ], const W& w, const X& x, int stages, int start,
                                              char* smem) {
   constexpr int STRIDE = TileRing<MJ, NI, BYTES>::STRIDE, RING = TileRing<MJ, NI, BYTES>::RING;
   constexpr int G = NI * MJ;             // matrix instructions of a half

@@ -482,6 +482,28 @@ def test_linear_rows_at_the_lines_of_their_tiles(M, N, K):
     assert ((ops.linear_part(x, w).double().sum(0) - xd @ wt).abs() <= K * 2 ** -24 * (xd.abs() @ wt.abs())).all()
 
 
+@pytest.mark.parametrize("N,K", [(2032, 2048), (2064, 2048), (1984, 2048), (2112, 2048), (32768, 128), (32704, 128)])
+@pytest.mark.parametrize("M", [1, 33, 128, 160])
+def test_linear_rows_around_the_streaming_line(M, N, K):
+    """A little below 8 MB of weights, and from there on, where they pass the caches by: each form, with ragged tiles."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) * 0.05).bfloat16()
+    xd, wt = x.double(), w.double().t().contiguous()
+    ref, tol = xd @ wt, K * 2 ** -24 * (xd.abs() @ wt.abs())     # fp32 sums of K products
+    assert ((ops.linear_part(x, w).double().sum(0) - ref).abs() <= tol).all()
+    if M <= 128:
+        got = ops._hip_or_raise().linear_rows(x, w, ops._none(x), 1, 1).double()
+        assert ((got - ref).abs() <= tol + 2 ** -8 * ref.abs()).all()
+        assert ((ops.linear_f32_rows(x, w).double() - ref).abs() <= tol).all()
+    if N % 64 == 0:
+        gate, up = ref.chunk(2, -1)
+        tg, tu = tol.chunk(2, -1)
+        full = torch.nn.functional.silu(gate) * up
+        assert ((ops.linear_silu_rows(x, w).double() - full).abs()
+                <= 1.1 * tg * (up.abs() + tu) + tu * gate.abs() + 2 ** -8 * full.abs() + 1e-6).all()
+
+
 @pytest.mark.parametrize("N", [128, 192, 16320, 16448, 20544, 32896])
 @pytest.mark.parametrize("M", [5, 40, 128, 129, 256])
 def test_gated_rows_at_the_lines_of_their_tiles(M, N):
