@@ -30,8 +30,8 @@
 // passes a sigmoid gate (the block-local layers of the hybrid family).
 //
 // Measured in graphs, 32 heads / 8 kv heads, against rows read as fragments, P V on the vector unit and merges in a launch of
-// their own, us: 120 streams, five to a prompt, of 560 keys 33.5, 25.1; 40, eight to a prompt, of 2000 41, 28; prompts of their
-// own: 128 streams of 700 77, 71 (5.5 TB/s), 24 of 2500 48.6, 42.4; 16 fp8 streams of 6000 45.5, 40; 5 streams of 560 8.4, 7.4;
+// their own, us, without the streaming hint (DECODE_ONCE): 120 streams, five to a prompt, of 560 keys 33.5, 25.1; 40, eight to
+// a prompt, of 2000 41, 28; prompts of their own: 128 streams of 700 77, 71 (5.5 TB/s), 24 of 2500 48.6, 42.4; 16 fp8 streams of 6000 45.5, 40; 5 streams of 560 8.4, 7.4;
 // 16 / 4 heads, one of 150 7.5, 5.6; block-local, 100 rows of 600, 16 / 4 heads 15.5, 11.5. Without groups of heads, 8 / 8, 40
 // streams of 600: 22.4, 23.2; fp8 15.9, 17.2: there P V is a quarter of the vector work, and fewer registers let one wave more in.
 
@@ -117,11 +117,18 @@ struct Strip {
   static constexpr int BYTES = ((SUMS > TKEYS * 256 ? SUMS : TKEYS * 256) + 255) / 256 * 256;
 };
 
+// Bytes of a layer's keys and values from which on they are loaded with the streaming hint (nt), unless the stream before or
+// behind this one begins with the same block: a shared prompt is read again, from the L2. Layers of as much do not lie in the
+// last-level cache (256 MB) any more when the next step comes to them. Steps of six layers, 32 / 8 heads, us without and with:
+// 128 streams of 700 1297, 1225; 24 of 2500 910, 881; 40 of 600 794, 782; 8 of 1500 655, 652; one of 7800 629, 617; 16 fp8 streams of
+// 6000 857, 830. Prompts of 3000 shared by eight streams each with the hint 941, without 892.
+#define DECODE_ONCE (16 << 20)
+
 // KV: what the cache holds
 enum { KV_BF16 = 0, KV_FP8 = 1, KV_FP8_ANY = 2 };   // fp8 in blocks of a multiple of four keys, and in others
 
-template <int GQA, int KV, bool LOCAL>
-__global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
+template <int GQA, int KV, bool LOCAL, bool ONCE>
+__device__ __forceinline__ void decode_share(
     float* __restrict__ partials,
     bf16_t* __restrict__ out,            // written where one workgroup has the context, or by the last one with ``arrived``
     const bf16_t* __restrict__ q,        // [B, H, 128], row stride q_tstride
@@ -133,22 +140,22 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
     const int* __restrict__ context_lens,  // [B]
     const bf16_t* __restrict__ gate, int gate_stride,  // [B, H] logits of the heads' sigmoid gates, or nullptr
     int* __restrict__ arrived,           // [B, KVH] zeros, zeros again afterwards, or nullptr: a second launch merges
-    float scale, int block_size, uint32_t block_inverse, int max_blocks, int q_tstride, int mask_size, DecodeShares shares) {
+    float scale, int block_size, uint32_t block_inverse, int max_blocks, int q_tstride, int mask_size, DecodeShares shares,
+    int L, int first, int tiles, int Z, char (&strips)[4][Strip<GQA>::BYTES], float (&m_lds)[4][GQA], float (&l_lds)[4][GQA]) {
   constexpr int SETS = Strip<GQA>::SETS;
   constexpr bool FP8 = KV != KV_BF16;
   const int g_kv = blockIdx.x, num_kv_heads = gridDim.x;
   const int b = blockIdx.y;
   const int z = blockIdx.z;
-  const int L = context_lens[b];
-  const int first = first_key(L, mask_size);
-  const int tiles = (L - first + TKEYS - 1) / TKEYS;
-  const int Z = shares_of(tiles, shares);
-  if (z >= Z) return;
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int col = lane & 15, grp = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // asked for anew behind the loop, whose registers are all taken
+  auto lane_now = [] {
+    int all = -1;
+    asm volatile("" : "+s"(all));
+    return (int)__builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
+  };
+  const int lane = lane_now(), col = lane & 15, grp = lane >> 4;
 
-  __shared__ __attribute__((aligned(16))) char strips[4][Strip<GQA>::BYTES];
-  __shared__ float m_lds[4][GQA], l_lds[4][GQA];
   char* const strip = strips[wave];
 
   // column n of the products is head n % GQA
@@ -194,7 +201,9 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int64_t r = lane_value(row, FP8 ? lane >> 3 : grp, i * (FP8 ? 8 : 4));
-      to[i] = *reinterpret_cast<const u32x4*>(cache + (FP8 ? r * 128 + (lane & 7) * 16 : r * 256 + col * 16));
+      const u32x4* at = reinterpret_cast<const u32x4*>(cache + (FP8 ? r * 128 + (lane & 7) * 16 : r * 256 + col * 16));
+      if constexpr (ONCE) to[i] = __builtin_nontemporal_load(at);
+      else to[i] = *at;
     }
   };
   auto load_scales = [&](f32x4 (&to)[2], const float* scales, int row) {
@@ -355,20 +364,21 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
   }
 
   // ---- fold the lane groups' keys, then the parts and the waves ---------------------------
+  const int end_lane = lane_now(), tid = wave * 64 + end_lane;
   l_run += __shfl_xor(l_run, 16);
   l_run += __shfl_xor(l_run, 32);
   float* const sums = reinterpret_cast<float*>(strip);
 #pragma unroll
   for (int e = 0; e < SETS; ++e) {
-    const int n = e * 16 + col;            // part n / GQA of head n % GQA
+    const int n = e * 16 + (end_lane & 15);  // part n / GQA of head n % GQA
     if (n < 3 * GQA) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(sums + n * SUM_PITCH + i * 16 + grp * 4) = o[e][i];
+      for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(sums + n * SUM_PITCH + i * 16 + (end_lane >> 4) * 4) = o[e][i];
     }
   }
-  if (lane < GQA) {
-    m_lds[wave][lane] = m_run;
-    l_lds[wave][lane] = l_run;
+  if (end_lane < GQA) {
+    m_lds[wave][end_lane] = m_run;
+    l_lds[wave][end_lane] = l_run;
   }
   __syncthreads();
   float* base = partials + (((int64_t)b * num_kv_heads + g_kv) * gridDim.z + z) * GQA * PART_STRIDE;
@@ -449,6 +459,52 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
 #pragma unroll
   for (int r = 0; r < 4; ++r) v[r] = f32_to_bf16((sum > 0.0f ? acc[r] / sum : 0.0f) * open);
   *reinterpret_cast<bf16x4_vec*>((short*)out + ((int64_t)b * num_kv_heads * GQA + g_kv * GQA + h) * 128 + d) = v;
+}
+
+template <int GQA, int KV, bool LOCAL>
+__global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
+    float* __restrict__ partials,
+    bf16_t* __restrict__ out,            // written where one workgroup has the context, or by the last one with ``arrived``
+    const bf16_t* __restrict__ q,        // [B, H, 128], row stride q_tstride
+    const char* __restrict__ k_cache,    // [NB, KVH, BS, 128], bf16 or fp8
+    const char* __restrict__ v_cache,
+    const float* __restrict__ k_scale,   // [NB, KVH, BS] per-row dequant (FP8 only)
+    const float* __restrict__ v_scale,
+    const int* __restrict__ block_tables,  // [B, max_blocks]
+    const int* __restrict__ context_lens,  // [B]
+    const bf16_t* __restrict__ gate, int gate_stride,  // [B, H] logits of the heads' sigmoid gates, or nullptr
+    int* __restrict__ arrived,           // [B, KVH] zeros, zeros again afterwards, or nullptr: a second launch merges
+    float scale, int block_size, uint32_t block_inverse, int max_blocks, int q_tstride, int mask_size, DecodeShares shares, int rows) {
+  __shared__ __attribute__((aligned(16))) char strips[4][Strip<GQA>::BYTES];
+  __shared__ float m_lds[4][GQA], l_lds[4][GQA];
+  const int b = blockIdx.y;
+  const bool after = b > 0, ahead = b + 1 < rows;
+  int L = context_lens[b], own = 0, prev = 0, next = 0;
+  if constexpr (!LOCAL) {                  // beside the length, not behind it
+    const int* bt = block_tables + (int64_t)b * max_blocks;
+    own = bt[0];
+    prev = bt[after ? -max_blocks : 0];
+    next = bt[ahead ? max_blocks : 0];
+    asm volatile("" : "+s"(L), "+s"(own), "+s"(prev), "+s"(next));
+  }
+  const int first = first_key(L, mask_size);
+  const int tiles = (L - first + TKEYS - 1) / TKEYS;
+  const int Z = shares_of(tiles, shares);
+  if ((int)blockIdx.z >= Z) return;
+#define DECODE_SHARE(ONCE)                                                                                                    \
+  decode_share<GQA, KV, LOCAL, ONCE>(partials, out, q, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens, gate,   \
+                                     gate_stride, arrived, scale, block_size, block_inverse, max_blocks, q_tstride, mask_size, \
+                                     shares, L, first, tiles, Z, strips, m_lds, l_lds)
+  // both sides whole: with the loops alone twice in one body it spilled registers
+  if constexpr (!LOCAL) {
+    const bool shared = (after && prev == own) || (ahead && next == own);
+    if (!shared && (int64_t)L * rows * gridDim.x * (KV == KV_BF16 ? 512 : 256) >= DECODE_ONCE) {
+      DECODE_SHARE(true);
+      return;
+    }
+  }
+  DECODE_SHARE(false);
+#undef DECODE_SHARE
 }
 
 // Rows of one launch: they lie on the grid's y, which ends at 65535. Steps with a row
@@ -558,7 +614,7 @@ extern "C" void launch_attn_decode(
   hipLaunchKernelGGL((attn_decode_tiles<G, F, L>), grid, dim3(NTHREADS), 0, stream, partials, o, q0, \
                      (const char*)k_cache, (const char*)v_cache, k_scale, v_scale, bt,             \
                      context_lens + b0, g0, gate_stride, a0, scale, block_size, block_inverse, max_blocks, q_tstride, \
-                     mask_size, sh)
+                     mask_size, sh, rows)
 #define DISPATCH(G) \
   do {                                                                                             \
     if (cache_fp8 && quads) LAUNCH(G, KV_FP8, false);                                              \
