@@ -12,7 +12,7 @@
 //
 // What bounds them: with a few hundred rows an expert or fewer, the stream of W from memory;
 // above, the matrix units. So the row tiles of an expert are even parts of its rows, in
-// tiles of 64, 128, 160, 192 or 256 rows: they keep step, and the 2 or 3 of a column run side
+// tiles of 64, 128, 160, 192, 224 or 256 rows: they keep step, and the 2 or 3 of a column run side
 // by side on one XCD, whose L2 then sees a panel of W once. (256 rows a tile and a small one
 // for the rest: the small ones run ahead, and read W again: at 1024 rows gate/up 603 us
 // instead of 525.) Column tiles go to the 8 XCDs in turn, which gives each the same share of
@@ -25,7 +25,12 @@
 //                                 2048 rows  896 + 471 (1175 + 812)
 //   width 4096, experts of 7168   6000 rows  1117 + 566: 1260 TFLOP/s (1394 + 847)
 // The layer with a router of seven launches at 65 / 150 / 300 / 600 / 1024 / 2048 / 6000 rows, experts of 14336: 582 / 582 /
-// 605 / 666 / 949 / 1431 / 3623 us (741 / 760 / 787 / 907 / 1131 / 1935 / 4622); moe_route has what it is now.
+// 605 / 666 / 949 / 1431 / 3623 us (741 / 760 / 787 / 907 / 1131 / 1935 / 4622); moe_route has what it was after that.
+//
+// W is read once for the row tiles side by side and is loaded with the streaming hint, which leaves the L2 to x; tiles of 224
+// rows are for parts of 193 to 224, a tenth less than a tile of 256. The layer, us without the two and with: 10 rows 487, 454;
+// 300 563, 541; 1024 889, 883; 1600 1144, 1057; 2048 1377, 1370; 2600 1720, 1610; experts of 7168, 3300 rows 1105, 1016, 6000
+// 1739, 1736; width 2048, experts of 8192, 600 rows 227, 219.
 
 #include "tile_product.h"
 
@@ -49,7 +54,7 @@ __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t*
   if constexpr (GATEUP) {
     // W rows of a tile: 64 gate, 64 up, the next 64 gate, 64 up
     const int n_put = n0 + (wave >> 1) * 64;
-    const TileRows wr(w + ((int64_t)e * 2 + (wave & 1)) * N * K + k0, n_put, N, 64, K, lane);
+    const TileRowsOf<true> wr(w + ((int64_t)e * 2 + (wave & 1)) * N * K + k0, n_put, N, 64, K, lane);
     TileGather<MJ> xr;
 #pragma unroll
     for (int i = 0; i < MJ; ++i) {
@@ -70,7 +75,7 @@ __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t*
     });
   } else {
     const int n_put = n0 + wave * 64, m_put = m0 + wave * MJ * 8;
-    const TileRows wr(w + (int64_t)e * N * K + k0, n_put, N, 64, K, lane);
+    const TileRowsOf<true> wr(w + (int64_t)e * N * K + k0, n_put, N, 64, K, lane);
     const TileRows xr(a + k0, m_put, m_end, MJ * 8, K, lane);
     tile_product<MJ>(acc, wr, xr, stages, stages * (blockIdx.x & 7) / 8, smem);
     if (sh.shares > 1 && !tile_fold<MJ>(acc, sh.part, sh.share, sh.shares, sh.count, smem)) return;
@@ -130,7 +135,8 @@ __global__ void __launch_bounds__(TP_THREADS, 1) moe_product_kernel(
   const int rows = (end - begin + m_tiles - 1) / m_tiles;
   const int n0 = (first + at / m_tiles * 8) * BN, m0 = begin + at % m_tiles * rows, m_end = min(end, m0 + rows);
 #define MOE_TILE(MJ) moe_tile<GATEUP, MJ>(out, a, w, ids, zeros, e, m0, m_end, n0, N, K, sh, smem)
-  if (rows > 192) MOE_TILE(8);
+  if (rows > 224) MOE_TILE(8);
+  else if (rows > 192) MOE_TILE(7);
   else if (rows > 160) MOE_TILE(6);
   else if (rows > 128) MOE_TILE(5);
   else if (rows > 64) MOE_TILE(4);

@@ -198,9 +198,11 @@ def test_mixture_products_against_float64(H, I, counts):
     (2048, 2624, [700, 600, 600, 600, 600, 600, 600, 600]),       # 42 tiles an XCD: a whole round, and ten in three shares
     (320, 64, [1] * 60 + [0] * 3 + [2, 300, 0, 1] + [3] * 63),    # experts of more than one walk of a wave's lanes
     (64, 2624, [5] * 64 + [0] * 64 + [9]),
+    (320, 320, [96, 96, 97, 112, 112, 113, 224, 224, 225]),      # tiles of 224 rows, and their edges in one and two parts
+    (64, 2624, [96, 96, 97, 112, 112, 113, 224, 224, 225]),
 ])
 def test_mixture_products_at_the_edges_of_row_tiles(H, I, counts):
-    # expert e gets counts[e] + counts[e - 1] rows: 64, 128, 160, 192 and 256 a tile, and parts of two and three tiles
+    # expert e gets counts[e] + counts[e - 1] rows: 64, 128, 160, 192, 224 and 256 a tile, and parts of two and three tiles
     test_mixture_products_against_float64(H, I, counts)
 
 
