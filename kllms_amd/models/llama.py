@@ -416,10 +416,11 @@ class LlamaForCausalLM(nn.Module):
         if (batch.host_segs is not None and batch.seg_tables is not None and self.dtype == torch.bfloat16
                 and self.layers and self.layers[0].self_attn.head_dim == 128
                 and ops.paged_prefill_pays(batch.host_segs, self.layers[0].self_attn.num_kv_heads)):
-            plan, short = ops.paged_prefill_plan(batch.host_segs, input_ids.device)
+            at = self.layers[0].self_attn
+            few = hasattr(at, "num_heads") and ops.paged_prefill_few(batch.host_segs, at.num_heads)
+            plan, short = ops.paged_prefill_plan(batch.host_segs, input_ids.device, *([64] if few else []))
             if plan is not None:
-                return replace(batch, plans={**(batch.plans or {}), "paged": (plan, short),
-                                             "few": ops.paged_prefill_few(batch.host_segs)})
+                return replace(batch, plans={**(batch.plans or {}), "paged": (plan, short), "few": few})
         return batch
 
     def forward_hidden(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:

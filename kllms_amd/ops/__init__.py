@@ -13,6 +13,7 @@ by numerics tests to produce the oracle on-device).
 
 from __future__ import annotations
 
+import heapq
 import os
 from typing import Optional, Sequence, Tuple
 
@@ -170,21 +171,48 @@ def paged_prefill_pays(segs, kv_heads: int) -> bool:
     return bool(long) and kv_heads * sum(k * n for k, n in long) >= PAGED_PREFILL_WORK * max(k for k, _ in long)
 
 
-def paged_prefill_few(segs) -> bool:
-    """Whether the long ones of the segments [(start position, rows)] have up to 64 rows each, behind enough keys that four
-    waves share a row tile's (their sums take 2 us to meet): 32 heads, one of 37 rows behind 1536 52 us and 33, one of 33 behind
-    5 6.5 and 9.4."""
+# us of a workgroup that goes over k keys: four waves to a row tile and 64 rows a workgroup; one wave to a row tile and up to
+# 128 rows, and up to 256, where a SIMD has two of them. Measured, one segment, at 512 / 1536 / 4000 keys: 20, 36, 76; 26, 55,
+# 127; 41, 86, 199.
+_PAGED_GROUP = {64: (12, 1 / 63), 128: (11, 1 / 34), 256: (16, 1 / 22)}
+
+
+def paged_prefill_few(segs, heads: int) -> bool:
+    """Whether the long ones of the segments [(start position, rows)] are dealt out in groups of 64 rows, whose four waves
+    share each row tile's keys (their sums take 2 us to meet), and not of 256. Few segments leave the chip idle otherwise; with
+    many, the keys are staged four times as often. 32 / 8 heads, us, groups of 256 and of 64:
+      behind 512    1 segment of 64 rows 24, 19   146 37, 20   512 53, 28     4 of 146 37, 34   300 44, 59     8 of 146 40, 52
+      behind 1536   1 of 64 52, 34   146 82, 36   512 98, 47     2 of 300 87, 70     4 of 146 83, 63   256 88, 82     8 of 65 56, 62
+        146 88, 99    12 of 64 103, 70   96 106, 95
+      behind 4000   1 of 146 190, 76     4 of 256 203, 166     8 of 146 197, 212    12 of 128 259, 240
+    One of 33 rows behind 5, whatever the rule says of it: 6.5, 9.4."""
     long = [(start + n, n) for start, n in segs if n >= PAGED_PREFILL_ROWS]
-    return bool(long) and max(n for _, n in long) <= 64 and max(k for k, _ in long) >= 512
+    if max((k for k, _ in long), default=0) < 512:
+        return False
+
+    def cost(size):
+        """Of all groups, longest first, on as many at a time as compute units have their heads."""
+        groups = []
+        for k, n in long:
+            for r in range(0, n, size):
+                rows = min(size, n - r)
+                at, key = _PAGED_GROUP[64 if size == 64 else 128 if rows <= 128 else 256]
+                groups.append(at + (k - n + r + rows) * key)
+        lanes = [0.0] * max(1, 256 // heads)
+        for us in sorted(groups, reverse=True):
+            heapq.heapreplace(lanes, lanes[0] + us)
+        return max(lanes)
+
+    return cost(64) < cost(256)
 
 
-def paged_prefill_plan(segs, device) -> tuple:
-    """(groups [4, G] on the device, [(first row, rows)] left to row-by-row attention) for segments
+def paged_prefill_plan(segs, device, rows: int = 256) -> tuple:
+    """(groups [4, G] of up to ``rows`` rows on the device, [(first row, rows)] left to row-by-row attention) for segments
     [(start position, rows)] packed in that order; groups None when every segment is short."""
     groups, short, row = [], [], 0
     for i, (_, n) in enumerate(segs):
         if n >= PAGED_PREFILL_ROWS:
-            groups.extend((row, n, r, i) for r in range(0, n, 256))
+            groups.extend((row, n, r, i) for r in range(0, n, rows))
         elif n and short and short[-1][0] + short[-1][1] == row:
             short[-1] = (short[-1][0], short[-1][1] + n)
         elif n:
@@ -197,8 +225,8 @@ def paged_prefill_plan(segs, device) -> tuple:
 
 
 def attn_segments_paged(q, k_cache, v_cache, block_tables, context_lens, scale, plan, short, seg_tables, seg_start, few=False):
-    """Rows of long segments on the matrix cores against the paged bf16 cache, the others row by row (GPU only). ``few``: no
-    segment of the plan has more than 64 rows."""
+    """Rows of long segments on the matrix cores against the paged bf16 cache, the others row by row (GPU only). ``few``: the
+    plan's groups are of 64 rows."""
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     _hip_or_raise().attn_prefill_paged(out, q, k_cache, v_cache, plan, seg_tables, seg_start, scale, few)
     f = _none(q, torch.float32)

@@ -14,8 +14,9 @@
 //     the fragment (staging it transposed took 16 two-byte LDS writes a thread)
 //   - K's 16-byte units are XORed with the row, V's 32-byte slots with v_turn of it:
 //     both fragment reads are free of bank conflicts
-//   - where no group has more than 64 rows (the tail of a chat behind a long cache) four
-//     waves share a q-tile, 32 keys of each stage each, and their sums meet in LDS
+//   - where few segments (the tail of a chat behind a long cache) would leave the chip idle,
+//     groups are of 64 rows and four waves share a q-tile, 32 keys of each stage each; their
+//     sums meet in LDS
 //
 // What bounds it: a SIMD's two waves, which a barrier keeps in step, do their 32 matrix
 // instructions of a tile (1024 cycles) and their softmax (about 1000 cycles, half of
@@ -37,7 +38,8 @@
 // Measured in graphs, 32 heads / 8 kv heads, with 64 keys a stage by way of registers and
 // so, us: one sequence of 7777 rows 548, 502 (986 TFLOP/s), 24 of about 550 177, 142; 16 / 4
 // heads, 8 of 1000 76, 67; 8 segments of 160 rows behind 1536 cached keys 98, 95, 12 of 45
-// behind 2000 135, 85, one of 37 behind 1536 52, 33.
+// behind 2000 135, 85, one of 37 behind 1536 52, 33; in groups of 64 rows where that is faster
+// (paged_prefill_few), one of 146 behind 1536 82, 36, of 512 98, 47, four of 146 83, 63.
 //
 // MFMA fragment maps (v_mfma_f32_32x32x16_bf16, verified on-device by the
 // mfma_selftest binding):
@@ -70,7 +72,7 @@ __device__ __forceinline__ int acc_row(int r, int half) {
 // V's 32-byte slots of a row are XORed with this: the rows of a turned read, 4 by 2 slots, lie in all banks
 __device__ __forceinline__ int v_turn(int row) { return (row & 3) * 2 + (row >> 2 & 1); }
 
-// SHARED: PAGED, groups of up to 64 rows: four waves share a q-tile, each with 32 keys of a stage
+// SHARED: PAGED, groups of 64 rows: four waves share a q-tile, each with 32 keys of a stage
 template <bool PAGED, bool SHARED>
 __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
     bf16_t* __restrict__ out,       // [T, H, D] contiguous
@@ -399,7 +401,7 @@ extern "C" int launch_attn_prefill(bf16_t* out, const bf16_t* q, const bf16_t* k
   return 0;
 }
 
-// few: no group has more than 64 rows
+// few: groups of 64 rows
 extern "C" int launch_attn_prefill_paged(bf16_t* out, const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache,
                                          const int* grp_start, const int* grp_len, const int* grp_q0,
                                          const int* grp_seg, const int* block_tables, const int* seg_pos, int ngroups,

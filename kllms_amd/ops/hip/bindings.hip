@@ -227,7 +227,7 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k, torch::Te
 
 // rows of segments against the paged cache (bf16): plan [4, G] int32 (first row, rows, first row within the
 // segment, segment), tables [n, MAXB], pos [n] = position of each segment's first row. The segments' own keys and
-// values are in the cache already. few: no segment of the plan has more than 64 rows.
+// values are in the cache already. few: the plan's groups are of 64 rows.
 void attn_prefill_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache, torch::Tensor v_cache,
                         torch::Tensor plan, torch::Tensor tables, torch::Tensor pos, double scale, bool few) {
   CHECK_BF16_CONTIG(out); CHECK_BF16_ROWS(q); CHECK_BF16_CONTIG(k_cache); CHECK_BF16_CONTIG(v_cache);

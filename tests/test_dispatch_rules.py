@@ -21,6 +21,18 @@ def test_portions(segs, kv_heads, pays):
     assert ops.paged_prefill_pays(segs, kv_heads) is pays
 
 
+@pytest.mark.parametrize("segs,heads,few", [
+    ([], 32, False), ([(3000, 31)] * 2, 32, False),                              # nothing on the matrix cores
+    ([(447, 64)], 32, False), ([(448, 64)], 32, True), ([(5, 400)], 32, False),  # keys that are few
+    ([(1536, 146)], 32, True), ([(1536, 512)] * 2, 32, True), ([(1536, 256)] * 4, 32, True), ([(1536, 300)] * 4, 32, False),
+    ([(1536, 128)] * 4, 32, True), ([(1536, 65)] * 8, 32, False), ([(1536, 146)] * 8, 32, False), ([(1536, 146)] * 8, 16, True),
+    ([(1536, 64)] * 12, 32, True), ([(4000, 128)] * 12, 32, True), ([(4000, 40), (10, 4000)], 32, False),
+    ([(4000, 40), (3000, 1)] * 2, 32, True),                                      # decode rows beside do not count
+])
+def test_groups_of_portions(segs, heads, few):
+    assert ops.paged_prefill_few(segs, heads) is few
+
+
 def test_one_short_portion_behind_a_long_cache_goes_row_by_row(monkeypatch):
     """The model asks the rule: a step of one 32-row portion has no plan, one of eight has."""
     import torch

@@ -63,11 +63,13 @@ def test_plan_covers_many_sequences():
     assert got == want
 
 
-# the last two: four waves to a row tile, at the edges of their tiles and stages of keys and of the row tiles
+# few: four waves to a row tile, at the edges of their tiles and stages of keys, of the row tiles and of the groups
+@pytest.mark.parametrize("few", [False, True])
 @pytest.mark.parametrize("H,G,BS", [(8, 2, 16), (32, 8, 16), (4, 4, 5), (4, 2, 1)])
 @pytest.mark.parametrize("segs", [[(0, 40)], [(17, 32), (1000, 300), (3, 1), (5, 2)], [(255, 1), (64, 257), (0, 31), (700, 33)],
-                                  [(576, 32), (95, 64), (0, 33), (1151, 1), (1, 63)], [(480, 32), (2000, 47)]])
-def test_segments_against_cache(H, G, BS, segs):
+                                  [(576, 32), (95, 64), (0, 33), (1151, 1), (1, 63)], [(480, 32), (2000, 47)],
+                                  [(600, 65), (31, 128), (1, 129), (128, 192), (97, 95)]])
+def test_segments_against_cache(H, G, BS, segs, few):
     g = torch.Generator().manual_seed(sum(n for _, n in segs) + H)
     NB = sum((s + n + BS - 1) // BS for s, n in segs) + 2
     perm = torch.randperm(NB, generator=g).tolist()
@@ -79,15 +81,14 @@ def test_segments_against_cache(H, G, BS, segs):
         bt[i, :m] = torch.tensor([perm.pop() for _ in range(m)], dtype=torch.int32)
     T = sum(n for _, n in segs)
     q = torch.randn(T, H + 1, D, generator=g).bfloat16().to(DEV)[:, :H]
-    plan, short = ops.paged_prefill_plan(segs, DEV)
+    plan, short = ops.paged_prefill_plan(segs, DEV, *([64] if few else []))
     row_seg = torch.tensor([i for i, (_, n) in enumerate(segs) for _ in range(n)])
     ctx = torch.tensor([s + j + 1 for s, n in segs for j in range(n)], dtype=torch.int32)
     if plan is None:
         return
     out = ops.attn_segments_paged(q, kc.to(DEV), vc.to(DEV), bt[row_seg].to(DEV), ctx.to(DEV), D ** -0.5, plan, short,
                                   bt.to(DEV), torch.tensor([s for s, _ in segs], dtype=torch.int32).to(DEV),
-                                  ops.paged_prefill_few(segs))
-    assert ops.paged_prefill_few(segs) == (segs[0][0] in (576, 480))
+                                  few)
     r = 0
     for i, (s, n) in enumerate(segs):
         at = torch.arange(s + n)
