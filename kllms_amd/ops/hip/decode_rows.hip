@@ -8,11 +8,11 @@
 // activation in the product they stay in fp32, from the library they come in bf16.)
 //
 // Per layer: residual + norm (twice) and rope + cache store, beside attention and
-// four products: 8 launches (one more where attention splits the contexts, one where
-// gate/up is the library's), where separate reductions, rope, store and activation
+// four products: 8 launches (one more where gate/up is the library's), where separate reductions, rope, store and activation
 // took 11. A step of 5 rows (32 heads, width 4096, 6 layers, contexts of 560) went
 // from 948 to 774 us with these and few-row products through registers, and to 676 with those of linear_rows.hip; one of
-// 120 rows from 1516 to 1237 and 1114, one of a single row at width 2048 from 492 to 391 and 330.
+// 120 rows from 1516 to 1237 and 1114, one of a single row at width 2048 from 492 to 391 and 330. (With the merge in
+// attention's launch and weights that pass the caches by they are at 612, 1024 and 284.)
 
 #include <type_traits>
 
