@@ -209,7 +209,7 @@ __device__ __forceinline__ void decode_share(
   auto load_scales = [&](f32x4 (&to)[2], const float* scales, int row) {
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
-      if constexpr (KV == KV_FP8) {        // behind the context the last row's four
+      if constexpr (KV == KV_FP8) {        // whole quads: of the last one also what lies behind the context
         to[tt] = *reinterpret_cast<const f32x4*>(scales + (lane_value(row, grp * 4, tt * 16) & ~3));
       } else {
 #pragma unroll
@@ -306,7 +306,8 @@ __device__ __forceinline__ void decode_share(
       for (int r = 0; r < 4; ++r) {
         float p = (sc[tt][r] == -INFINITY) ? 0.0f : exp_of<LOCAL>(sc[tt][r] - m_new);
         l_run += p;
-        if constexpr (FP8) p *= vs_now[tt][r];
+        // scales behind the context are what another sequence left there, infinities too
+        if constexpr (FP8) p = base + tt * 16 + grp * 4 + r < L ? p * vs_now[tt][r] : 0.0f;
         part[0][r] = p;
       }
 #pragma unroll

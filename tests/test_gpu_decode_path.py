@@ -10,8 +10,8 @@ DEV = "cuda"
 D = 128
 
 
-def paged_case(B, KVH, gqa, BS, ctx, fp8, seed=0, width=None):
-    """q, caches, scales, block tables, lengths; blocks shuffled, streams 0 and 1 share their full blocks."""
+def paged_case(B, KVH, gqa, BS, ctx, fp8, seed=0, width=None, shared=True):
+    """q, caches, scales, block tables, lengths; blocks shuffled, streams 0 and 1 share their full blocks unless not ``shared``."""
     g = torch.Generator().manual_seed(seed)
     need = [max(1, (c + BS - 1) // BS) for c in ctx]
     NB = sum(need) + 3
@@ -19,7 +19,7 @@ def paged_case(B, KVH, gqa, BS, ctx, fp8, seed=0, width=None):
     bt = torch.zeros((B, width or max(need)), dtype=torch.int32)
     for b in range(B):
         own = [perm.pop() for _ in range(need[b])]
-        if b == 1:
+        if b == 1 and shared:
             own[:min(ctx[0], ctx[1]) // BS] = bt[0, :min(ctx[0], ctx[1]) // BS].tolist()
         bt[b, :need[b]] = torch.tensor(own, dtype=torch.int32)
     k, v = ((torch.randn(NB, KVH, BS, D, generator=g) * s).bfloat16() for s in (1.0, 1.0))
@@ -90,6 +90,26 @@ def test_shared_contexts(ctx, gqa, KVH, BS, fp8, joined):
     assert (err <= 2 ** -8 * ref.abs() + 2e-5).all(), err.max()
     assert torch.equal(ops.attn_decode_paged(*args), out)
     assert arrived is None or not arrived.any()
+
+
+@pytest.mark.parametrize("left", [float("inf"), float("nan")])
+@pytest.mark.parametrize("gqa,KVH,BS,fp8", [(4, 2, 16, True), (1, 2, 4, True), (8, 1, 32, True), (2, 2, 6, True), (4, 2, 16, False)])
+@pytest.mark.parametrize("ctx", [[1, 2, 3, 5], [33, 62, 127, 130], [385, 514, 1027, 2049]])
+def test_what_lies_behind_the_context_is_not_read(ctx, gqa, KVH, BS, fp8, left):
+    """Blocks are given to the next sequence as they are: keys, values and scales of the one before, which may have overflowed."""
+    q, k, v, ks, vs, bt, n = paged_case(len(ctx), KVH, gqa, BS, ctx, fp8, seed=sum(ctx) + BS, shared=False)
+    ref = attention64(q, k, v, ks, vs, bt, n, D ** -0.5)
+    for b, c in enumerate(ctx):
+        blk, at = int(bt[b, (c - 1) // BS]), (c - 1) % BS + 1
+        for t in (k, v):
+            (t.view(torch.uint8) if fp8 else t)[blk, :, at:] = 0x7f if fp8 else left
+        for t in (ks, vs) if fp8 else ():
+            t[blk, :, at:] = left
+    dev = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    out = ops.attn_decode_paged(dev(q), dev(k), dev(v), dev(bt), dev(n), D ** -0.5, dev(ks), dev(vs))
+    err = (out.double().cpu() - ref).abs()
+    # one bf16 rounding of the result (2^-9), fp32 sums before it
+    assert (err <= 2 ** -8 * ref.abs() + 2e-5).all(), err.max()
 
 
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 64, 65, 128])
