@@ -393,7 +393,8 @@ __device__ __forceinline__ void decode_share(
     for (int w = 0; w < 4; ++w) {
       const float e = m_lds[w][h] == -INFINITY ? 0.0f : exp_of<LOCAL>(m_lds[w][h] - M);   // a wave without a tile
       const float* s = reinterpret_cast<const float*>(strips[w]) + h * SUM_PITCH + d;
-      acc += (s[0] + (s[GQA * SUM_PITCH] + s[2 * GQA * SUM_PITCH])) * e;
+      // an infinite value times what is left of P, which may be 0 or negative, is no number: P's first part alone then
+      acc += (isinf(s[0]) ? s[0] : s[0] + (s[GQA * SUM_PITCH] + s[2 * GQA * SUM_PITCH])) * e;
       l += l_lds[w][h] * e;
     }
     if (Z == 1) {

@@ -112,6 +112,33 @@ def test_what_lies_behind_the_context_is_not_read(ctx, gqa, KVH, BS, fp8, left):
     assert (err <= 2 ** -8 * ref.abs() + 2e-5).all(), err.max()
 
 
+@pytest.mark.parametrize("joined", [True, False])
+@pytest.mark.parametrize("gqa,KVH,BS,fp8", [(1, 2, 16, False), (2, 3, 16, False), (4, 2, 16, False), (8, 1, 16, False), (4, 2, 16, True)])
+@pytest.mark.parametrize("ctx", [[5, 40], [700, 1300]])
+def test_infinite_values_give_infinities(ctx, gqa, KVH, BS, fp8, joined):
+    """One key with an infinite value in some dims (in fp8 an infinite scale): those of the result are infinite, the others as ever."""
+    q, k, v, ks, vs, bt, n = paged_case(len(ctx), KVH, gqa, BS, ctx, fp8, seed=sum(ctx), shared=False)
+    q = q * 0.1                                                   # no weight near the smallest numbers
+    for b, c in enumerate(ctx):
+        blk, at = int(bt[b, (c // 2) // BS]), (c // 2) % BS
+        if fp8:
+            v.view(torch.uint8)[blk, :, at] &= 0x80               # signed zeros, which stay: 0 * inf
+            v.view(torch.uint8)[blk, :, at, 1::3] |= 0x31
+            vs[blk, :, at] = float("inf")
+        else:
+            v[blk, :, at, 1::6], v[blk, :, at, 4::6] = float("inf"), -float("inf")
+    dev = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    arrived = torch.zeros(len(ctx) * KVH, dtype=torch.int32, device=DEV) if joined else None
+    out = ops.attn_decode_paged(dev(q), dev(k), dev(v), dev(bt), dev(n), D ** -0.5, dev(ks), dev(vs), arrived).double().cpu()
+    ref = attention64(q, k, v, ks, vs, bt, n, D ** -0.5)
+    assert torch.equal(out[..., 1::3], ref[..., 1::3]) and ref[..., 1::3].isinf().all()
+    if not fp8:
+        rest = torch.arange(D) % 3 != 1
+        err = (out - ref)[..., rest].abs()
+        # one bf16 rounding of the result (2^-9), fp32 sums before it
+        assert (err <= 2 ** -8 * ref[..., rest].abs() + 2e-5).all(), err.max()
+
+
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 64, 65, 128])
 @pytest.mark.parametrize("N,K", [(16, 128), (48, 256), (64, 384), (192, 1280), (2048, 2048)])
 def test_linear_rows(M, N, K):
