@@ -164,6 +164,10 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
   const int max_blocks = block_tables.size(1);
   TORCH_CHECK((int64_t)k_cache.size(0) * KVH * BS < (1LL << 31), "attn_decode: cache rows exceed 32-bit indexing");
   if (B == 0) return;
+  if (max_blocks == 0) {       // every context is empty: the kernel looks at a row's first block before its length
+    out.zero_();
+    return;
+  }
   // 16-byte query loads
   if (q.stride(0) % 8 != 0 || reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 != 0) q = q.contiguous();
   if (gate.numel() > 0)

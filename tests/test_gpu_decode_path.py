@@ -112,6 +112,14 @@ def test_what_lies_behind_the_context_is_not_read(ctx, gqa, KVH, BS, fp8, left):
     assert (err <= 2 ** -8 * ref.abs() + 2e-5).all(), err.max()
 
 
+def test_empty_tables():
+    """Rows without a context, and a table without a column: zeros."""
+    q, k, v, _, _, bt, n = (t if t is None else t.to(DEV) for t in paged_case(3, 2, 4, 16, [40, 5, 17], False))
+    out = ops.attn_decode_paged(q, k, v, bt[:, :0].contiguous(), n * 0, 0.1)
+    assert not out.any()
+    assert torch.equal(ops.attn_decode_paged(q, k, v, bt, n * 0, 0.1), out)
+
+
 @pytest.mark.parametrize("joined", [True, False])
 @pytest.mark.parametrize("gqa,KVH,BS,fp8", [(1, 2, 16, False), (2, 3, 16, False), (4, 2, 16, False), (8, 1, 16, False), (4, 2, 16, True)])
 @pytest.mark.parametrize("ctx", [[5, 40], [700, 1300]])
