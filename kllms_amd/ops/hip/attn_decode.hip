@@ -535,7 +535,7 @@ static DecodeShares attn_decode_shares(int B, int num_kv_heads, int max_ctx, boo
     if (fill > best + 0.02) best = fill, s.most = z;
   }
   s.most = s.most < s.mid ? s.mid : s.most;
-  const int rounds = (max_ctx + 4 * TKEYS - 1) / (4 * TKEYS);
+  const int rounds = (int)(((int64_t)max_ctx + 4 * TKEYS - 1) / (4 * TKEYS));
   int z = s.mid > (rounds + 7) / 8 ? s.mid : (rounds + 7) / 8;     // shares_of of any context up to max_ctx is no more
   z = z > s.most ? s.most : z;
   s.grid = rounds <= s.few ? 1 : z < rounds ? z : rounds;

@@ -121,6 +121,17 @@ def test_empty_tables():
 
 
 @pytest.mark.parametrize("joined", [True, False])
+def test_a_table_of_more_positions_than_32_bits(joined):
+    """As many columns as make 2^31 positions: the shares of a context are those of a table that is just wide enough."""
+    q, k, v, _, _, bt, n = (t if t is None else t.to(DEV) for t in paged_case(1, 2, 4, 16, [5000], False))
+    arrived = torch.zeros(2, dtype=torch.int32, device=DEV) if joined else None
+    wide = torch.zeros((1, 2 ** 27), dtype=torch.int32, device=DEV)
+    wide[:, :bt.shape[1]] = bt
+    want = ops.attn_decode_paged(q, k, v, bt, n, 0.1, None, None, arrived)
+    assert torch.equal(ops.attn_decode_paged(q, k, v, wide, n, 0.1, None, None, arrived), want)
+
+
+@pytest.mark.parametrize("joined", [True, False])
 @pytest.mark.parametrize("gqa,KVH,BS,fp8", [(1, 2, 16, False), (2, 3, 16, False), (4, 2, 16, False), (8, 1, 16, False), (4, 2, 16, True)])
 @pytest.mark.parametrize("ctx", [[5, 40], [700, 1300]])
 def test_infinite_values_give_infinities(ctx, gqa, KVH, BS, fp8, joined):
