@@ -378,7 +378,8 @@ class LlamaForCausalLM(nn.Module):
         T = input_ids.shape[0]
         if batch.mode == "decode":
             # zeroed by the first launch, and zero again after each layer's attention
-            arrived = torch.empty(T * layers[0].self_attn.num_kv_heads, dtype=torch.int32, device=input_ids.device)
+            arrived = torch.empty(T * layers[0].self_attn.num_kv_heads * ops.ATTN_COUNTER_GAP, dtype=torch.int32,
+                                  device=input_ids.device)
             x, residual = ops.embed_norm_rows(input_ids, self.embed_tokens.weight, norm.weight, norm.eps, self._unknown_ids(),
                                               arrived)
         else:              # a prompt's ids are the caller's: the embedding refuses them in the call

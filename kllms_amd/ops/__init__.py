@@ -253,6 +253,11 @@ def attn_blocklocal_rows(q, k_cache, v_cache, block_tables, context_lens, scale,
     return out
 
 
+# 32 ints, a line of the L2: workgroups that count in one line wait for each other. One stream of 2000 keys, 32 / 8 heads,
+# 128 workgroups: 9.7 us with the eight counters beside each other, 8.9 with this between them; two 11.1, 9.3
+ATTN_COUNTER_GAP = 32
+
+
 def attn_decode_paged(
     q: torch.Tensor,
     k_cache: torch.Tensor,
@@ -265,7 +270,7 @@ def attn_decode_paged(
     arrived: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """``arrived``: an int32 zero for each row and kv head, zero again afterwards; with it, contexts that several workgroups
-    share are merged in the same launch."""
+    share are merged in the same launch. Zeros for ATTN_COUNTER_GAP times as many keep the counters in cache lines of their own."""
     if q.is_cuda and not _force_torch():
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         none = _none(q, torch.float32)

@@ -3,8 +3,8 @@
 // Flash decoding over 32-key tiles, one tile per WAVE: a wave takes every
 // (Z*4)-th tile of its (stream, kv head), keeps its own running max and sum, and
 // the four waves of a workgroup fold once at the end. Z workgroups share a
-// context; their partials are merged by the last of them to arrive, or by a second
-// launch where the caller has no counters for that.
+// context (attn_decode_shares); their partials are merged by the last of them to
+// arrive, or by a second launch where the caller has no counters for that.
 //
 // What bounds it is bytes in flight, and for contexts that lie in the L2 the address
 // units. A wave has the K and V rows of its next tile (16 KB in bf16, 64 registers a
@@ -32,9 +32,12 @@
 // Measured in graphs, 32 heads / 8 kv heads, against rows read as fragments, P V on the vector unit and merges in a launch of
 // their own, us, without the streaming hint (DECODE_ONCE): 120 streams, five to a prompt, of 560 keys 33.5, 25.1; 40, eight to
 // a prompt, of 2000 41, 28; prompts of their own: 128 streams of 700 77, 71 (5.5 TB/s), 24 of 2500 48.6, 42.4; 16 fp8 streams of 6000 45.5, 40; 5 streams of 560 8.4, 7.4;
-// 16 / 4 heads, one of 150 7.5, 5.6; block-local, 100 rows of 600, 16 / 4 heads 15.5, 11.5. Without groups of heads, 8 / 8, 40
-// streams of 600: 22.4, 23.2; fp8 15.9, 17.2: there P V is a quarter of the vector work, and fewer registers let one wave more in.
+// 16 / 4 heads, one of 150 7.5, 5.6; block-local, 100 rows of 600, 16 / 4 heads 15.5, 11.5.
+//
+// Without groups of heads, 8 / 8, 40 streams of 600: 22.4, 23.2; fp8 15.9, 17.2: there P V is a quarter of the vector work, and
+// fewer registers let one wave more in.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -73,18 +76,24 @@ __device__ __forceinline__ int first_key(int L, int mask_size) {
   return mask_size > 0 ? max(L - 1, 0) / mask_size * mask_size : 0;
 }
 
-// Workgroups that share a context of so many tiles (attn_decode_shares): one up to ``few`` tiles a wave, then ``mid`` or as many
-// as leave a wave eight, ``most`` at most; no more than its rounds of tiles take.
+// How many workgroups share a context of so many rounds of four tiles, a tile for each wave (attn_decode_shares): one up to
+// ``few`` rounds. Above, the last of ``most`` from whose ``from`` on it is, no more than ``lo`` or one for every ``per`` rounds,
+// and of those as many as are all equally long.
 struct DecodeShares {
-  int few, mid, most, grid;
+  int few, lo, per, most[3], from[3];
+  int grid;                  // of no context more
+  bool joined;               // merged in the same launch
 };
+__host__ __device__ __forceinline__ int most_of(int rounds, const DecodeShares& s) {
+  int z = (rounds + s.per - 1) / s.per, most = rounds >= s.from[1] ? s.most[1] : s.most[0];
+  most = rounds >= s.from[2] ? s.most[2] : most;
+  z = z < s.lo ? s.lo : z;
+  return z < most ? z : most;
+}
 __host__ __device__ __forceinline__ int shares_of(int tiles, const DecodeShares& s) {
   const int rounds = (tiles + 3) / 4;
   if (rounds <= s.few) return 1;
-  int z = (rounds + 7) / 8;
-  z = z < s.mid ? s.mid : z;
-  z = z > s.most ? s.most : z;
-  const int each = (rounds + z - 1) / z;
+  const int z = most_of(rounds, s), each = (rounds + z - 1) / z;
   return (rounds + each - 1) / each;
 }
 
@@ -105,7 +114,7 @@ __device__ __forceinline__ float head_gate(const bf16_t* __restrict__ gate, int 
   return 1.0f / (1.0f + exp_of<LOCAL>(-bf16_to_f32(((const short*)gate)[(int64_t)b * stride + h])));
 }
 
-#define DECODE_SHARES 16   // of a context at most that are merged in the same launch
+#define MERGED 16          // partials of a thread that are on their way at once when they are merged in the same launch
 #define FAR 16             // loads and stores past the L2, from and to other XCDs' workgroups
 
 // A wave's strip of LDS: K of its tile, then V, 32 rows of 128 bf16; after the last one its sums, rows of SUM_PITCH floats
@@ -139,7 +148,7 @@ __device__ __forceinline__ void decode_share(
     const int* __restrict__ block_tables,  // [B, max_blocks]
     const int* __restrict__ context_lens,  // [B]
     const bf16_t* __restrict__ gate, int gate_stride,  // [B, H] logits of the heads' sigmoid gates, or nullptr
-    int* __restrict__ arrived,           // [B, KVH] zeros, zeros again afterwards, or nullptr: a second launch merges
+    int* __restrict__ arrived, int apart,  // [B, KVH] zeros, ``apart`` ints from each other, zeros again afterwards, or nullptr
     float scale, int block_size, uint32_t block_inverse, int max_blocks, int q_tstride, int mask_size, DecodeShares shares,
     int L, int first, int tiles, int Z, char (&strips)[4][Strip<GQA>::BYTES], float (&m_lds)[4][GQA], float (&l_lds)[4][GQA]) {
   constexpr int SETS = Strip<GQA>::SETS;
@@ -383,27 +392,35 @@ __device__ __forceinline__ void decode_share(
   }
   __syncthreads();
   float* base = partials + (((int64_t)b * num_kv_heads + g_kv) * gridDim.z + z) * GQA * PART_STRIDE;
-  for (int i = tid; i < GQA * 128; i += NTHREADS) {
-    const int h = i >> 7, d = i & 127;
+  // dims of a thread: one round for all of them. (Four of each group size: 0.8 us more without groups)
+  constexpr int VEC = GQA > 2 ? GQA / 2 : 1;
+  if (tid * VEC < GQA * 128) {
+    const int h = tid * VEC >> 7, d = tid * VEC & 127;
     float M = m_lds[0][h];
 #pragma unroll
     for (int w = 1; w < 4; ++w) M = fmaxf(M, m_lds[w][h]);
-    float acc = 0.0f, l = 0.0f;
+    float acc[VEC] = {}, l = 0.0f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float e = m_lds[w][h] == -INFINITY ? 0.0f : exp_of<LOCAL>(m_lds[w][h] - M);   // a wave without a tile
       const float* s = reinterpret_cast<const float*>(strips[w]) + h * SUM_PITCH + d;
-      // an infinite value times what is left of P, which may be 0 or negative, is no number: P's first part alone then.
-      // (Asked of the first part itself, the others are read in a branch behind it, 0.4 us a launch)
-      const float all = s[0] + (s[GQA * SUM_PITCH] + s[2 * GQA * SUM_PITCH]);
-      acc += (all == all ? all : s[0]) * e;
+#pragma unroll
+      for (int r = 0; r < VEC; ++r) {
+        // an infinite value times what is left of P, which may be 0 or negative, is no number: P's first part alone then.
+        // (Asked of the first part itself, the others are read in a branch behind it, 0.4 us a launch)
+        const float all = s[r] + (s[GQA * SUM_PITCH + r] + s[2 * GQA * SUM_PITCH + r]);
+        acc[r] += (all == all ? all : s[r]) * e;
+      }
       l += l_lds[w][h] * e;
     }
     if (Z == 1) {
-      const float v = (l > 0.0f ? acc / l : 0.0f) * head_gate<LOCAL>(gate, gate_stride, b, g_kv * GQA + h);
-      ((short*)out)[((int64_t)b * num_kv_heads * GQA + g_kv * GQA + h) * 128 + d] = f32_to_bf16(v);
+      const float open = head_gate<LOCAL>(gate, gate_stride, b, g_kv * GQA + h);
+      short* const to = (short*)out + ((int64_t)b * num_kv_heads * GQA + g_kv * GQA + h) * 128 + d;
+#pragma unroll
+      for (int r = 0; r < VEC; ++r) to[r] = f32_to_bf16((l > 0.0f ? acc[r] / l : 0.0f) * open);
     } else if (!arrived) {
-      base[h * PART_STRIDE + d] = acc;
+#pragma unroll
+      for (int r = 0; r < VEC; ++r) base[h * PART_STRIDE + d + r] = acc[r];
       if (d == 0) {
         base[h * PART_STRIDE + 128] = M;
         base[h * PART_STRIDE + 129] = l;
@@ -411,7 +428,14 @@ __device__ __forceinline__ void decode_share(
     } else {
       const auto far = __builtin_amdgcn_make_buffer_rsrc(base, 0, GQA * PART_STRIDE * 4, 0x00020000);
       const int at = h * PART_STRIDE * 4;
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc), far, at + d * 4, 0, FAR);
+      if constexpr (VEC == 4) {
+        const u32x4 all = {__float_as_uint(acc[0]), __float_as_uint(acc[1]), __float_as_uint(acc[2]), __float_as_uint(acc[3])};
+        __builtin_amdgcn_raw_buffer_store_b128(all, far, at + d * 4, 0, FAR);
+      } else if constexpr (VEC == 2) {
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(acc[0]), __float_as_uint(acc[1])}, far, at + d * 4, 0, FAR);
+      } else {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[0]), far, at + d * 4, 0, FAR);
+      }
       if (d == 0) __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(M), __float_as_uint(l)}, far, at + 512, 0, FAR);
     }
   }
@@ -421,43 +445,72 @@ __device__ __forceinline__ void decode_share(
   __syncthreads();
   int* const last = reinterpret_cast<int*>(strips[0]);
   if (tid == 0) {
-    int* const count = arrived + (int64_t)b * num_kv_heads + g_kv;
+    int* const count = arrived + ((int64_t)b * num_kv_heads + g_kv) * apart;
     *last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == Z - 1;
     if (*last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   if (!*last) return;
-  // 32 lanes a head, 4 dims each, all loads before the first wait
+  // 32 lanes a head, 4 dims each, and as many sets of heads as there are threads for, a partial each in turn; the loads of
+  // MERGED partials before the first wait. (Without the sets 16 partials took 0.5 us more)
+  constexpr int SETS_OF_HEADS = NTHREADS / (32 * GQA);
   const float* all = base - (int64_t)z * GQA * PART_STRIDE;
   const auto far = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(all), 0, Z * GQA * PART_STRIDE * 4, 0x00020000);
-  const int h = tid >> 5, d = (tid & 31) * 4;
-  if (h >= GQA) return;
-  f32x4 part[DECODE_SHARES];
-  float m[DECODE_SHARES], l[DECODE_SHARES], M = -INFINITY;
-#pragma unroll
-  for (int e0 = 0; e0 < DECODE_SHARES; e0 += 4)
-    if (e0 < Z) {
-#pragma unroll
-      for (int e = e0; e < e0 + 4; ++e) {  // behind the last one zeros
-        const int at = (e * GQA + h) * PART_STRIDE * 4;
-        const auto ml = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(far, at + 512, 0, FAR));
-        part[e] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(far, at + d * 4, 0, FAR));
-        m[e] = ml[0];
-        l[e] = ml[1];
-      }
-    }
-#pragma unroll
-  for (int e = 0; e < DECODE_SHARES; ++e)
-    if (e < Z) M = fmaxf(M, m[e]);
+  const int h = (tid >> 5) % GQA, d = (tid & 31) * 4, set = tid / (32 * GQA);
+  float M = -INFINITY, sum = 0.0f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  float sum = 0.0f;
+#pragma unroll 1
+  for (int z0 = 0; z0 < Z; z0 += MERGED * SETS_OF_HEADS) {
+    f32x4 part[MERGED];
+    float m[MERGED], l[MERGED];
 #pragma unroll
-  for (int e = 0; e < DECODE_SHARES; ++e)
-    if (e < Z) {
-      const float w = m[e] == -INFINITY ? 0.0f : exp_of<LOCAL>(m[e] - M);
-      sum += l[e] * w;
-      acc += part[e] * w;
+    for (int e0 = 0; e0 < MERGED; e0 += 4)
+      if (z0 + e0 * SETS_OF_HEADS < Z) {
+#pragma unroll
+        for (int e = e0; e < e0 + 4; ++e) {  // behind the last one zeros
+          const int mine = z0 + e * SETS_OF_HEADS + set, at = (mine * GQA + h) * PART_STRIDE * 4;
+          const auto ml = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(far, at + 512, 0, FAR));
+          part[e] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(far, at + d * 4, 0, FAR));
+          m[e] = mine < Z ? ml[0] : -INFINITY;
+          l[e] = ml[1];
+        }
+      }
+    const float before = M;
+#pragma unroll
+    for (int e = 0; e < MERGED; ++e)
+      if (z0 + e * SETS_OF_HEADS < Z) M = fmaxf(M, m[e]);
+    const float a = before == -INFINITY ? 0.0f : exp_of<LOCAL>(before - M);
+    sum *= a;
+    acc *= a;
+#pragma unroll
+    for (int e = 0; e < MERGED; ++e)
+      if (z0 + e * SETS_OF_HEADS < Z) {
+        const float w = m[e] == -INFINITY ? 0.0f : exp_of<LOCAL>(m[e] - M);
+        sum += l[e] * w;
+        acc += part[e] * w;
+      }
+  }
+  if constexpr (SETS_OF_HEADS > 1) {       // the sets' sums meet in LDS, behind the one word that said who was last
+    f32x4* const sums_of = reinterpret_cast<f32x4*>(strips[1]);
+    f32x2* const ml_of = reinterpret_cast<f32x2*>(strips[2]);
+    sums_of[tid] = acc;
+    ml_of[tid] = f32x2{M, sum};
+    __syncthreads();
+    if (set > 0) return;
+    float top = M;
+#pragma unroll
+    for (int e = 1; e < SETS_OF_HEADS; ++e) top = fmaxf(top, ml_of[tid + e * 32 * GQA][0]);
+    const float a = M == -INFINITY ? 0.0f : exp_of<LOCAL>(M - top);
+    sum *= a;
+    acc *= a;
+#pragma unroll
+    for (int e = 1; e < SETS_OF_HEADS; ++e) {
+      const f32x2 ml = ml_of[tid + e * 32 * GQA];
+      const float w = ml[0] == -INFINITY ? 0.0f : exp_of<LOCAL>(ml[0] - top);
+      sum += ml[1] * w;
+      acc += sums_of[tid + e * 32 * GQA] * w;
     }
+  }
   const float open = head_gate<LOCAL>(gate, gate_stride, b, g_kv * GQA + h);
   bf16x4_vec v;
 #pragma unroll
@@ -477,7 +530,7 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
     const int* __restrict__ block_tables,  // [B, max_blocks]
     const int* __restrict__ context_lens,  // [B]
     const bf16_t* __restrict__ gate, int gate_stride,  // [B, H] logits of the heads' sigmoid gates, or nullptr
-    int* __restrict__ arrived,           // [B, KVH] zeros, zeros again afterwards, or nullptr: a second launch merges
+    int* __restrict__ arrived, int apart,  // [B, KVH] zeros, ``apart`` ints from each other, zeros again afterwards, or nullptr
     float scale, int block_size, uint32_t block_inverse, int max_blocks, int q_tstride, int mask_size, DecodeShares shares, int rows) {
   __shared__ __attribute__((aligned(16))) char strips[4][Strip<GQA>::BYTES];
   __shared__ float m_lds[4][GQA], l_lds[4][GQA];
@@ -497,7 +550,7 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
   if ((int)blockIdx.z >= Z) return;
 #define DECODE_SHARE(ONCE)                                                                                                    \
   decode_share<GQA, KV, LOCAL, ONCE>(partials, out, q, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens, gate,   \
-                                     gate_stride, arrived, scale, block_size, block_inverse, max_blocks, q_tstride, mask_size, \
+                                     gate_stride, arrived, apart, scale, block_size, block_inverse, max_blocks, q_tstride, mask_size, \
                                      shares, L, first, tiles, Z, strips, m_lds, l_lds)
   // both sides whole: with the loops alone twice in one body it spilled registers
   if constexpr (!LOCAL) {
@@ -516,37 +569,53 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
 // in several launches; on x, beside the kv heads, every workgroup would divide.
 #define MAX_ROWS 65535
 
-// Shares of a context at most, as long as the chip is not full: 256 workgroups in all for contexts of medium length, whose merge
-// (2 us, 3 in its own launch) weighs most, and for long ones what fills whole rounds of the compute units best: a workgroup more
-// on some of them than on others is waited for. us, 32 / 8 heads, by workgroups in all:
-//   24 streams of 560  192 13.8   384 17.7   768 16.6          of 2500  192 44.3   384 46.0   576 47.1   768 43.6
-//   16 of 6000, fp8  256 44.3   384 46.1   512 41.7   640 46.2   768 43.3       bf16  256 72.1   384 77.7   512 73.7   640 77.6
-//   40 of 2000  320 68.3   640 62.8   960 62.0    40 of 560  320 22.0   640 23.2    8 of 1500  64 21.5   128 16.3   256 15.3   640 15.7
-static DecodeShares attn_decode_shares(int B, int num_kv_heads, int max_ctx, bool fp8, bool joined) {
+// What is best for contexts of one length is one workgroup a compute unit, 256 in all, or two or three of them on each; in
+// between, some units work on one more than others and are waited for. Their number also has to cover contexts of different
+// lengths, whose longest has the same number as all: so the longer ones have two or three a unit, the sooner the slower
+// a round is (fp8, one head a kv head). us by workgroups in all:
+//   32 / 8 heads, bf16   one of 7800 168 12.1   248 12.2   488 14.4      5 of 7800 160 31.0   240 30.0   320 35.0   440 30.9   640 32.9
+//     16 of 2000 128 27.0   256 25.4   384 27.6   512 25.9   768 26.3      16 / 4, one of 131072 64 90   128 54.8   256 49.4   344 58.9
+//     12 of 2500 to 7800 192 50.9   480 47.6      24 of 1300 to 4500 192 61.4   768 53.2      one each, 40 of 2000 64.7, 640 60.5   960 58.4
+//   fp8   5 of 7800 240 22.4   320 22.9   440 20.9   640 23.4      16 / 4, 40 of 1500 160 21.1   320 20.3   480 17.8   640 19.6
+//   8 / 8   5 of 700 to 7800 240 23.0   440 24.8   fp8 240 19.5   440 16.0 (the lengths of one launch differ: 16.1 with 640 of all)
+// Counted over the launch's lengths by each workgroup, so that all are equally long, they took 0.6 us more and gained nothing.
+// A merge in its own launch takes 1 us more, at the start; one of eight heads for very few contexts, by a single
+// workgroup each, the longer the more: 8 / 1 heads, one of 7800 12.1, in a launch of its own 10.8; of 131072 32.1, 22.4.
+static DecodeShares attn_decode_shares(int B, int num_kv_heads, int gqa, int max_ctx, bool fp8, bool local, bool joined) {
   const int64_t pairs = (int64_t)B * num_kv_heads;
-  const int cap = joined ? DECODE_SHARES : 32;
+  if (gqa == 8 && pairs <= 2 && max_ctx > 24 * 4 * TKEYS) joined = false;
   DecodeShares s;
-  s.few = joined ? 3 : 1;
-  s.mid = pairs >= 256 ? 1 : (int)(256 / pairs > cap ? cap : 256 / pairs);
-  // long ones: what fills whole rounds of the compute units best
-  s.most = 1;
-  double best = 0.0;
-  for (int z = 1; z <= cap && (z == 1 || pairs * z <= 1024); ++z) {
-    if (pairs * z < (fp8 ? 512 : 256) && z < cap && pairs * (z + 1) <= 1024) continue;
-    const double fill = (double)(pairs * z) / ((pairs * z + 255) / 256 * 256);
-    if (fill > best + 0.02) best = fill, s.most = z;
+  s.joined = joined;
+  s.few = joined ? 3 : local ? 1 : 2;
+  if (pairs <= 256) {
+    s.lo = joined ? 32 : 48;
+    s.per = joined ? 16 : 4;
+    for (int i = 0; i < 3; ++i) {
+      s.most[i] = (int)std::min<int64_t>(256 * (i + 1) / pairs, 128);
+      s.from[i] = i == 0 ? 0 : (fp8 || gqa == 1 ? 2 * i : 2 * i + 2) * s.most[i];
+      // not where it fills the units less
+      if (i && (int64_t)s.most[i] * pairs * i + 24 * i * (i + 1) < (int64_t)s.most[i - 1] * pairs * (i + 1)) s.most[i] = s.most[i - 1], s.from[i] = INT32_MAX;
+    }
+  } else {                                   // those that fill whole rounds of the units best, one for every eight rounds
+    s.lo = 1;
+    s.per = 8;
+    s.most[0] = 1;
+    s.from[1] = s.from[2] = INT32_MAX;
+    double best = 0.0;
+    for (int z = 1; z == 1 || pairs * z <= 1024; ++z) {
+      if (pairs * z < 512 && fp8 && pairs * (z + 1) <= 1024) continue;
+      const double fill = (double)(pairs * z) / ((pairs * z + 255) / 256 * 256);
+      if (fill > best + 0.02) best = fill, s.most[0] = z;
+    }
   }
-  s.most = s.most < s.mid ? s.mid : s.most;
   const int rounds = (int)(((int64_t)max_ctx + 4 * TKEYS - 1) / (4 * TKEYS));
-  int z = s.mid > (rounds + 7) / 8 ? s.mid : (rounds + 7) / 8;     // shares_of of any context up to max_ctx is no more
-  z = z > s.most ? s.most : z;
-  s.grid = rounds <= s.few ? 1 : z < rounds ? z : rounds;
+  s.grid = rounds <= s.few ? 1 : std::min(most_of(rounds, s), rounds);
   return s;
 }
 
 // workgroups per context of a launch: room for partials where more than one
-extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx, int fp8, int joined) {
-  return attn_decode_shares(B < MAX_ROWS ? B : MAX_ROWS, num_kv_heads, max_ctx, fp8 != 0, joined != 0).grid;
+extern "C" int attn_decode_splits(int B, int num_kv_heads, int gqa, int max_ctx, int fp8, int local, int joined) {
+  return attn_decode_shares(B < MAX_ROWS ? B : MAX_ROWS, num_kv_heads, gqa, max_ctx, fp8 != 0, local != 0, joined != 0).grid;
 }
 
 // merge the partials of a (stream, q head): two dims per lane, the partials dealt
@@ -596,14 +665,15 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(
 // from 0 on a block-local layer's (bf16 caches); partials: room for
 // min(B, MAX_ROWS) * KVH * splits * gqa * 130 floats when splits > 1
 extern "C" void launch_attn_decode(
-    bf16_t* out, float* partials, int* arrived, const bf16_t* q, const void* k_cache, const void* v_cache,
+    bf16_t* out, float* partials, int* arrived, int apart, const bf16_t* q, const void* k_cache, const void* v_cache,
     const float* k_scale, const float* v_scale, const int* block_tables, const int* context_lens,
     const bf16_t* gate, int gate_stride, float scale, int num_q_heads, int num_kv_heads, int block_size,
     int max_blocks, int max_ctx, int q_tstride, int B, int cache_fp8, int mask_size, hipStream_t stream) {
   const int gqa = num_q_heads / num_kv_heads;
   const bool local = mask_size >= 0;
-  const DecodeShares sh = attn_decode_shares(B < MAX_ROWS ? B : MAX_ROWS, num_kv_heads, max_ctx, cache_fp8 != 0, arrived != nullptr);
+  const DecodeShares sh = attn_decode_shares(B < MAX_ROWS ? B : MAX_ROWS, num_kv_heads, gqa, max_ctx, cache_fp8 != 0, local, arrived != nullptr);
   const int splits = sh.grid;
+  if (!sh.joined) arrived = nullptr;
   const bool quads = block_size % 4 == 0 && (reinterpret_cast<uintptr_t>(k_scale) | reinterpret_cast<uintptr_t>(v_scale)) % 16 == 0;
   const uint32_t block_inverse = block_size > 1 ? (uint32_t)(((1ull << 32) + block_size - 1) / block_size) : ~0u;
   for (int b0 = 0; b0 < B; b0 += MAX_ROWS) {
@@ -612,12 +682,12 @@ extern "C" void launch_attn_decode(
     bf16_t* o = out + (int64_t)b0 * num_q_heads * 128;
     const bf16_t* q0 = q + (int64_t)b0 * q_tstride;
     const int* bt = block_tables + (int64_t)b0 * max_blocks;
-    int* a0 = arrived ? arrived + (int64_t)b0 * num_kv_heads : nullptr;
+    int* a0 = arrived ? arrived + (int64_t)b0 * num_kv_heads * apart : nullptr;
     const bf16_t* g0 = gate ? gate + (int64_t)b0 * gate_stride : nullptr;
 #define LAUNCH(G, F, L)                                                                            \
   hipLaunchKernelGGL((attn_decode_tiles<G, F, L>), grid, dim3(NTHREADS), 0, stream, partials, o, q0, \
                      (const char*)k_cache, (const char*)v_cache, k_scale, v_scale, bt,             \
-                     context_lens + b0, g0, gate_stride, a0, scale, block_size, block_inverse, max_blocks, q_tstride, \
+                     context_lens + b0, g0, gate_stride, a0, apart, scale, block_size, block_inverse, max_blocks, q_tstride, \
                      mask_size, sh, rows)
 #define DISPATCH(G) \
   do {                                                                                             \

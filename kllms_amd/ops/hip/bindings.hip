@@ -15,8 +15,8 @@ extern "C" __global__ void silu_mul_kernel(bf16_t*, const bf16_t*, const bf16_t*
 extern "C" __global__ void rope_kernel(bf16_t*, bf16_t*, const int64_t*, const float*, int, int, int, int, int);
 extern "C" __global__ void store_kv_kernel(const bf16_t*, const bf16_t*, bf16_t*, bf16_t*, const int64_t*, int, int, int, int, int);
 extern "C" __global__ void store_kv_fp8_kernel(const bf16_t*, const bf16_t*, unsigned char*, unsigned char*, float*, float*, const int64_t*, int, int, int, int, int);
-extern "C" int attn_decode_splits(int B, int num_kv_heads, int max_ctx, int fp8, int joined);
-extern "C" void launch_attn_decode(bf16_t*, float*, int*, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, const bf16_t*, int, float, int, int, int, int, int, int, int, int, int, hipStream_t);
+extern "C" int attn_decode_splits(int B, int num_kv_heads, int gqa, int max_ctx, int fp8, int local, int joined);
+extern "C" void launch_attn_decode(bf16_t*, float*, int*, int, const bf16_t*, const void*, const void*, const float*, const float*, const int*, const int*, const bf16_t*, int, float, int, int, int, int, int, int, int, int, int, hipStream_t);
 extern "C" int launch_attn_prefill(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, int, int, float, int, int, int, int, hipStream_t);
 extern "C" int launch_attn_prefill_paged(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, const int*, const int*, const int*, const int*, const int*, int, float, int, int, int, int, int, int, hipStream_t);
 extern "C" void launch_attn_prefill_plan(int*, const int*, int, int, hipStream_t);
@@ -175,10 +175,14 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
                     gate.size(1) == H && gate.stride(1) == 1, "gate must be a bf16 [B, H] row view");
   const int64_t longest = mask_size > 0 ? std::min<int64_t>(mask_size, (int64_t)max_blocks * BS) : (int64_t)max_blocks * BS;
   const int longest32 = (int)std::min<int64_t>(longest, INT32_MAX);
-  const int splits = attn_decode_splits(B, KVH, longest32, k_cache.scalar_type() == at::kFloat8_e4m3fn, arrived.has_value());
-  if (arrived)
+  const int splits = attn_decode_splits(B, KVH, gqa, longest32, k_cache.scalar_type() == at::kFloat8_e4m3fn, mask_size >= 0,
+                                        arrived.has_value());
+  int apart = 1;
+  if (arrived) {
     TORCH_CHECK(arrived->is_cuda() && arrived->is_contiguous() && arrived->scalar_type() == at::kInt &&
                     arrived->numel() >= (int64_t)B * KVH, "arrived: an int32 zero for each row and kv head");
+    apart = (int)std::min<int64_t>(arrived->numel() / ((int64_t)B * KVH), 32);
+  }
   auto partials = torch::empty({splits > 1 ? (int64_t)B * KVH * splits * gqa * 130 : 0},
                                torch::dtype(torch::kFloat).device(q.device()));
   const int cache_fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn ? 1 : 0;
@@ -188,7 +192,7 @@ void attn_decode_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache
                 "fp8 attn_decode requires [NB, KVH, BS] fp32 k_scale/v_scale");
   }
   launch_attn_decode(
-      bf(out), partials.data_ptr<float>(), arrived ? arrived->data_ptr<int>() : nullptr, cbf(q), k_cache.data_ptr(), v_cache.data_ptr(),
+      bf(out), partials.data_ptr<float>(), arrived ? arrived->data_ptr<int>() : nullptr, apart, cbf(q), k_cache.data_ptr(), v_cache.data_ptr(),
       cache_fp8 ? k_scale.data_ptr<float>() : nullptr,
       cache_fp8 ? v_scale.data_ptr<float>() : nullptr,
       block_tables.data_ptr<int>(), context_lens.data_ptr<int>(), gate.numel() ? cbf(gate) : nullptr,
@@ -741,6 +745,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_inplace", &rope_inplace);
   m.def("store_kv", &store_kv);
   m.def("rope_store", &rope_store);
+  // workgroups of a context at most, by rows, kv heads, heads of each, positions of the table, fp8, block-local, counters
+  m.def("attn_decode_splits", &attn_decode_splits);
   m.def("attn_decode_paged", &attn_decode_paged, py::arg("out"), py::arg("q"), py::arg("k_cache"),
         py::arg("v_cache"), py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"), py::arg("k_scale"),
         py::arg("v_scale"), py::arg("gate"), py::arg("mask_size") = -1, py::arg("arrived") = py::none());

@@ -35,8 +35,8 @@ int launch_linear_rows(void*, const __hip_bfloat16*, const __hip_bfloat16*, cons
 int launch_linear_rows_two(float*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
                            hipStream_t);
 int linear_rows_splits(int, int, int);
-int attn_decode_splits(int, int, int, int, int);
-void launch_attn_decode(__hip_bfloat16*, float*, int*, const __hip_bfloat16*, const void*, const void*, const float*,
+int attn_decode_splits(int, int, int, int, int, int, int);
+void launch_attn_decode(__hip_bfloat16*, float*, int*, int, const __hip_bfloat16*, const void*, const void*, const float*,
                         const float*, const int*, const int*, const __hip_bfloat16*, int, float, int, int, int, int, int,
                         int, int, int, int, hipStream_t);
 }
@@ -157,9 +157,9 @@ std::optional<Tensor> hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tens
                            cu.data_ptr<int>(), seg_start.data_ptr<int>(), T, N, H, G, R, BS, RH, RD, RV, st);
   const int64_t longest = mask_size > 0 ? std::min<int64_t>(mask_size, (int64_t)width * BS) : (int64_t)width * BS;
   const int longest32 = (int)std::min<int64_t>(longest, INT32_MAX);
-  const int splits = attn_decode_splits(T, G, longest32, 0, 0);
+  const int splits = attn_decode_splits(T, G, H / G, longest32, 0, 1, 0);
   auto partials = torch::empty({splits > 1 ? (int64_t)T * H * splits * 130 : 0}, f32);
-  launch_attn_decode((__hip_bfloat16*)both.data_ptr(), partials.data_ptr<float>(), nullptr, bf(q), k_cache.data_ptr(),
+  launch_attn_decode((__hip_bfloat16*)both.data_ptr(), partials.data_ptr<float>(), nullptr, 1, bf(q), k_cache.data_ptr(),
                      v_cache.data_ptr(), nullptr, nullptr, tables.data_ptr<int>(), lens.data_ptr<int>(), bf(head_gate), H,
                      (float)scale, H, G, BS, width, longest32, KL, T, 0, (int)mask_size, st);
   Tensor left, right;

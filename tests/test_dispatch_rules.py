@@ -33,6 +33,22 @@ def test_groups_of_portions(segs, heads, few):
     assert ops.paged_prefill_few(segs, heads) is few
 
 
+@pytest.mark.skipif(not ops.hip_available(), reason="the extension is not built")
+@pytest.mark.parametrize("rows,kv_heads,group,keys,fp8,most", [
+    (1, 8, 4, 384, 0, 1), (1, 8, 4, 512, 0, 4), (1, 8, 4, 2048, 0, 16), (2, 8, 4, 8192, 0, 16), (5, 8, 4, 8192, 0, 12),
+    (1, 8, 4, 32768, 0, 32), (1, 4, 4, 131072, 0, 64), (1, 1, 4, 131072, 0, 64), (1, 1, 8, 131072, 0, 128),    # few long contexts
+    (20, 8, 4, 8192, 0, 3), (20, 8, 4, 1000, 0, 1), (20, 8, 4, 1000, 1, 3), (40, 8, 4, 8192, 0, 3), (128, 8, 4, 8192, 0, 1),
+])
+def test_shares_of_a_context(rows, kv_heads, group, keys, fp8, most):
+    """Few contexts fill the chip also where they are long; no more partials than fit 1024 workgroups' room."""
+    splits = ops._hip_or_raise().attn_decode_splits
+    assert splits(rows, kv_heads, group, keys, fp8, 0, 1) == most
+    for r in (1, 3, 17, 100, 255, 1000, 70000):
+        for joined in (0, 1):
+            z = splits(r, kv_heads, group, 1 << 20, fp8, 0, joined)
+            assert z == 1 or r * kv_heads * z <= 1024
+
+
 def test_one_short_portion_behind_a_long_cache_goes_row_by_row(monkeypatch):
     """The model asks the rule: a step of one 32-row portion has no plan, one of eight has."""
     import torch

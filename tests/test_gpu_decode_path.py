@@ -92,6 +92,25 @@ def test_shared_contexts(ctx, gqa, KVH, BS, fp8, joined):
     assert arrived is None or not arrived.any()
 
 
+# shares that a thread merges one after the other, and counters in lines of their own
+@pytest.mark.parametrize("gap", [0, 1, 32])
+@pytest.mark.parametrize("gqa,KVH,BS,fp8", [(1, 1, 16, False), (1, 2, 16, True), (1, 2, 5, True), (2, 2, 8, True), (4, 1, 16, False),
+                                            (8, 1, 16, False), (8, 1, 16, True)])
+@pytest.mark.parametrize("ctx", [[6300], [17000, 40, 900], [140000]])
+def test_few_long_contexts(ctx, gqa, KVH, BS, fp8, gap):
+    q, k, v, ks, vs, bt, n = paged_case(len(ctx), KVH, gqa, BS, ctx, fp8, seed=gqa + len(ctx) + BS, shared=False)
+    dev = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    arrived = torch.zeros(len(ctx) * KVH * gap, dtype=torch.int32, device=DEV) if gap else None
+    args = (dev(q), dev(k), dev(v), dev(bt), dev(n), D ** -0.5, dev(ks), dev(vs), arrived)
+    out = ops.attn_decode_paged(*args)
+    ref = attention64(q, k, v, ks, vs, bt, n, D ** -0.5)
+    err = (out.double().cpu() - ref).abs()
+    # one bf16 rounding of the result (2^-9), fp32 sums before it
+    assert (err <= 2 ** -8 * ref.abs() + 2e-5).all(), err.max()
+    assert torch.equal(ops.attn_decode_paged(*args), out)
+    assert arrived is None or not arrived.any()
+
+
 @pytest.mark.parametrize("left", [float("inf"), float("nan")])
 @pytest.mark.parametrize("gqa,KVH,BS,fp8", [(4, 2, 16, True), (1, 2, 4, True), (8, 1, 32, True), (2, 2, 6, True), (4, 2, 16, False)])
 @pytest.mark.parametrize("ctx", [[1, 2, 3, 5], [33, 62, 127, 130], [385, 514, 1027, 2049]])
