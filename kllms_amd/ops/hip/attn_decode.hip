@@ -34,8 +34,11 @@
 // a prompt, of 2000 41, 28; prompts of their own: 128 streams of 700 77, 71 (5.5 TB/s), 24 of 2500 48.6, 42.4; 16 fp8 streams of 6000 45.5, 40; 5 streams of 560 8.4, 7.4;
 // 16 / 4 heads, one of 150 7.5, 5.6; block-local, 100 rows of 600, 16 / 4 heads 15.5, 11.5.
 //
-// Without groups of heads, 8 / 8, 40 streams of 600: 22.4, 23.2; fp8 15.9, 17.2: there P V is a quarter of the vector work, and
-// fewer registers let one wave more in.
+// Without groups of heads P V is a quarter of the vector work, and stays on the vector unit: a lane loads the V rows of the keys
+// whose scores it has, P is where it is needed, and V needs no strip. 8 / 8 heads, us with the fragments' own loads, by way of the
+// matrix cores and so: one stream of 2000 8.0, 8.8, 7.2; 16 of 2000 31.9, 25.3, 24.8; 40 of 500 22.1, 19.9, 18.2; fp8: one of 2000
+// 7.2, 8.4, 7.0; 40 of 500 14.0, 14.1, 12.6; 120 of 20, which is four waves to a SIMD or three 5.4, 8.0, 5.4. Where two heads have
+// a kv head it is one as the other.
 
 #include <algorithm>
 #include <type_traits>
@@ -152,7 +155,7 @@ __device__ __forceinline__ void decode_share(
     float scale, int block_size, uint32_t block_inverse, int max_blocks, int q_tstride, int mask_size, DecodeShares shares,
     int L, int first, int tiles, int Z, char (&strips)[4][Strip<GQA>::BYTES], float (&m_lds)[4][GQA], float (&l_lds)[4][GQA]) {
   constexpr int SETS = Strip<GQA>::SETS;
-  constexpr bool FP8 = KV != KV_BF16;
+  constexpr bool FP8 = KV != KV_BF16, ONE = GQA == 1;
   const int g_kv = blockIdx.x, num_kv_heads = gridDim.x;
   const int b = blockIdx.y;
   const int z = blockIdx.z;
@@ -177,7 +180,8 @@ __device__ __forceinline__ void decode_share(
   const int* bt = block_tables + (int64_t)b * max_blocks;
 
   float m_run = -INFINITY, l_run = 0.0f;   // of head col % GQA; l_run: this lane's keys only
-  f32x4 o[SETS][8];
+  f32x4 o[SETS][8];                      // ONE: the first DIMS floats are this lane's dims, of its keys alone
+  constexpr int DIMS = FP8 ? 16 : 8;
 #pragma unroll
   for (int e = 0; e < SETS; ++e)
 #pragma unroll
@@ -203,13 +207,17 @@ __device__ __forceinline__ void decode_share(
   uint32_t key_at = lds0 + col * 256 + ((grp ^ col) << 4);
   uint32_t turn_at = lds0 + turn_row * 256 + ((((col & 3) >> 1) ^ turn_row) << 4) + (col & 1) * 8;
   // Whole rows go to registers, 16 lanes each (8 in fp8), and from there to the strip, their 16-byte units XORed with the row
+  // (ONE: V's stay there, a lane's are of the keys whose scores it has)
   constexpr int LOADS = FP8 ? TKEYS / 8 : TKEYS / 4;
   u32x4 kraw[LOADS], vraw[LOADS];
   f32x4 ks[2], vs[2];                    // scales of this lane's keys tt*16 + grp*4 + r
-  auto load = [&](u32x4 (&to)[LOADS], const char* cache, int row) {
+  auto load = [&](u32x4 (&to)[LOADS], const char* cache, int row, auto own) {
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      const int64_t r = lane_value(row, FP8 ? lane >> 3 : grp, i * (FP8 ? 8 : 4));
+      int64_t r;
+      if constexpr (!own) r = lane_value(row, FP8 ? lane >> 3 : grp, i * (FP8 ? 8 : 4));
+      else if constexpr (FP8) r = lane_value(row, grp * 4 + (lane >> 3 & 1), (i >> 1) * 16 + (i & 1) * 2);
+      else r = lane_value(row, grp * 4, (i >> 2) * 16 + (i & 3));
       const u32x4* at = reinterpret_cast<const u32x4*>(cache + (FP8 ? r * 128 + (lane & 7) * 16 : r * 256 + col * 16));
       if constexpr (ONCE) to[i] = __builtin_nontemporal_load(at);
       else to[i] = *at;
@@ -226,13 +234,13 @@ __device__ __forceinline__ void decode_share(
       }
     }
   };
-  auto load_k = [&](int row) {
-    if constexpr (FP8) load_scales(ks, k_scale, row);
-    load(kraw, k_cache, row);
+  auto load_k = [&](int row, auto scales) {
+    if constexpr (FP8 && scales) load_scales(ks, k_scale, row);
+    load(kraw, k_cache, row, std::false_type());
   };
   auto load_v = [&](int row) {
     if constexpr (FP8) load_scales(vs, v_scale, row);
-    load(vraw, v_cache, row);
+    load(vraw, v_cache, row, std::bool_constant<ONE>());
   };
   auto store = [&](const u32x4 (&from)[LOADS]) {
     const uint32_t put = put_at;
@@ -261,12 +269,13 @@ __device__ __forceinline__ void decode_share(
     asm volatile("" : "+v"(put_at), "+v"(key_at), "+v"(turn_at));
     // ---- scores: lane (col, grp) holds keys tt*16 + grp*4 + r of head col % GQA ----
     store(kraw);
+    // ONE: the scales themselves, which are loaded anew behind their use: registers for a fourth wave
     const f32x4 ks_now[2] = {ks[0], ks[1]}, vs_now[2] = {vs[0], vs[1]};
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (more) {
       row = row_of(t + step, block);
       block = bt[block_of(key_of(min(t + 2 * step, tiles - 1)))];
-      load_k(row);
+      load_k(row, std::bool_constant<!ONE>());
     }
     hold();
     __builtin_amdgcn_sched_barrier(0);
@@ -284,16 +293,19 @@ __device__ __forceinline__ void decode_share(
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         float x = acc[r] * scale;
-        if constexpr (FP8) x *= ks_now[tt][r];
+        if constexpr (FP8) x *= ONE ? ks[tt][r] : ks_now[tt][r];
         sc[tt][r] = base + tt * 16 + grp * 4 + r < L ? x : -INFINITY;
         tmax = fmaxf(tmax, sc[tt][r]);
       }
     }
-    hold();
-    __builtin_amdgcn_sched_barrier(0);
-    store(vraw);
-    if constexpr (more) load_v(row);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (more && FP8 && ONE) load_scales(ks, k_scale, row);
+    if constexpr (!ONE) {
+      hold();
+      __builtin_amdgcn_sched_barrier(0);
+      store(vraw);
+      if constexpr (more) load_v(row);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
     const float m_new = fmaxf(m_run, tmax);
@@ -303,9 +315,40 @@ __device__ __forceinline__ void decode_share(
 #pragma unroll
       for (int e = 0; e < SETS; ++e)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[e][i] *= alpha;
+        for (int i = 0; i < (ONE ? DIMS / 4 : 8); ++i) o[e][i] *= alpha;
     }
     m_run = m_new;
+    if constexpr (ONE) {
+#pragma unroll
+      for (int tt = 0; tt < TKEYS / 16; ++tt) {
+        float p[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          p[r] = (sc[tt][r] == -INFINITY) ? 0.0f : exp_of<LOCAL>(sc[tt][r] - m_new);
+          l_run += p[r];
+          if constexpr (FP8) p[r] = base + tt * 16 + grp * 4 + r < L ? p[r] * vs[tt][r] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < LOADS / 2; ++i) {
+          const u32x4 v = vraw[tt * (LOADS / 2) + i];
+          const float even = p[FP8 ? i * 2 : i], odd = p[FP8 ? i * 2 + 1 : i], w = FP8 && lane & 8 ? odd : even;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if constexpr (FP8) {
+              const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[u], false), hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[u], true);
+              o[0][u] += w * f32x4{lo[0], lo[1], hi[0], hi[1]};
+            } else {
+              o[0][u >> 1][(u & 1) * 2] += w * __uint_as_float(v[u] << 16);
+              o[0][u >> 1][(u & 1) * 2 + 1] += w * __uint_as_float(v[u] & 0xffff0000u);
+            }
+          }
+        }
+      }
+      if constexpr (more) load_v(row);
+      hold();
+      __builtin_amdgcn_sched_barrier(0);
+      return;
+    }
     // P in three bf16 parts, which are its 32 bits: column n of the product has part n / GQA
     Frag pf[SETS];
 #pragma unroll
@@ -364,7 +407,7 @@ __device__ __forceinline__ void decode_share(
     block = bt[block_of(key_of(min(t + step, tiles - 1)))];
     asm volatile("" : "+v"(block));        // here, not behind K and V
     __builtin_amdgcn_sched_barrier(0);
-    load_k(row);
+    load_k(row, std::true_type());
     __builtin_amdgcn_sched_barrier(0);
     load_v(row);
     __builtin_amdgcn_sched_barrier(0);
@@ -381,7 +424,11 @@ __device__ __forceinline__ void decode_share(
 #pragma unroll
   for (int e = 0; e < SETS; ++e) {
     const int n = e * 16 + (end_lane & 15);  // part n / GQA of head n % GQA
-    if (n < 3 * GQA) {
+    if constexpr (ONE) {                     // a sum for each set of keys
+      f32x4* const to = reinterpret_cast<f32x4*>(sums + (end_lane >> (FP8 ? 3 : 4)) * SUM_PITCH + (end_lane & (FP8 ? 7 : 15)) * DIMS);
+#pragma unroll
+      for (int i = 0; i < DIMS / 4; ++i) to[i] = o[0][i];
+    } else if (n < 3 * GQA) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(sums + n * SUM_PITCH + i * 16 + (end_lane >> 4) * 4) = o[e][i];
     }
@@ -408,8 +455,15 @@ __device__ __forceinline__ void decode_share(
       for (int r = 0; r < VEC; ++r) {
         // an infinite value times what is left of P, which may be 0 or negative, is no number: P's first part alone then.
         // (Asked of the first part itself, the others are read in a branch behind it, 0.4 us a launch)
-        const float all = s[r] + (s[GQA * SUM_PITCH + r] + s[2 * GQA * SUM_PITCH + r]);
-        acc[r] += (all == all ? all : s[r]) * e;
+        if constexpr (ONE) {
+          float all = s[0];
+#pragma unroll
+          for (int i = 1; i < (FP8 ? 8 : 4); ++i) all += s[i * SUM_PITCH];
+          acc[r] += all * e;
+        } else {
+          const float all = s[r] + (s[GQA * SUM_PITCH + r] + s[2 * GQA * SUM_PITCH + r]);
+          acc[r] += (all == all ? all : s[r]) * e;
+        }
       }
       l += l_lds[w][h] * e;
     }
@@ -519,7 +573,7 @@ __device__ __forceinline__ void decode_share(
 }
 
 template <int GQA, int KV, bool LOCAL>
-__global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
+__global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : GQA == 1 && KV != KV_FP8_ANY ? 4 : 3) void attn_decode_tiles(
     float* __restrict__ partials,
     bf16_t* __restrict__ out,            // written where one workgroup has the context, or by the last one with ``arrived``
     const bf16_t* __restrict__ q,        // [B, H, 128], row stride q_tstride
@@ -571,19 +625,20 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : 3) void attn_decode_tiles(
 
 // What is best for contexts of one length is one workgroup a compute unit, 256 in all, or two or three of them on each; in
 // between, some units work on one more than others and are waited for. Their number also has to cover contexts of different
-// lengths, whose longest has the same number as all: so the longer ones have two or three a unit, the sooner the slower
-// a round is (fp8, one head a kv head). us by workgroups in all:
+// lengths, whose longest has the same number as all: so the longer ones have two or three a unit, in fp8, whose rounds are
+// slower, sooner. us by workgroups in all:
 //   32 / 8 heads, bf16   one of 7800 168 12.1   248 12.2   488 14.4      5 of 7800 160 31.0   240 30.0   320 35.0   440 30.9   640 32.9
 //     16 of 2000 128 27.0   256 25.4   384 27.6   512 25.9   768 26.3      16 / 4, one of 131072 64 90   128 54.8   256 49.4   344 58.9
 //     12 of 2500 to 7800 192 50.9   480 47.6      24 of 1300 to 4500 192 61.4   768 53.2      one each, 40 of 2000 64.7, 640 60.5   960 58.4
 //   fp8   5 of 7800 240 22.4   320 22.9   440 20.9   640 23.4      16 / 4, 40 of 1500 160 21.1   320 20.3   480 17.8   640 19.6
+//     7 of 7000 392 25.3   728 27.2      30 of 600 240 12.2   480 13.5
 //   8 / 8   5 of 700 to 7800 240 23.0   440 24.8   fp8 240 19.5   440 16.0 (the lengths of one launch differ: 16.1 with 640 of all)
 // Counted over the launch's lengths by each workgroup, so that all are equally long, they took 0.6 us more and gained nothing.
-// A merge in its own launch takes 1 us more, at the start; one of eight heads for very few contexts, by a single
-// workgroup each, the longer the more: 8 / 1 heads, one of 7800 12.1, in a launch of its own 10.8; of 131072 32.1, 22.4.
+// A merge in its own launch takes 1 us more, but many partials of eight heads take a single workgroup longer. 8 / 1 heads, one
+// of 500 7.8, in a launch of its own 8.4; of 7800 12.1, 11.0; of 32768 19.0, 14.5; of 131072 32.1, 22.5: so where tables are long.
 static DecodeShares attn_decode_shares(int B, int num_kv_heads, int gqa, int max_ctx, bool fp8, bool local, bool joined) {
   const int64_t pairs = (int64_t)B * num_kv_heads;
-  if (gqa == 8 && pairs <= 2 && max_ctx > 24 * 4 * TKEYS) joined = false;
+  if (gqa == 8 && pairs <= 2 && max_ctx > 16384) joined = false;
   DecodeShares s;
   s.joined = joined;
   s.few = joined ? 3 : local ? 1 : 2;
@@ -592,9 +647,11 @@ static DecodeShares attn_decode_shares(int B, int num_kv_heads, int gqa, int max
     s.per = joined ? 16 : 4;
     for (int i = 0; i < 3; ++i) {
       s.most[i] = (int)std::min<int64_t>(256 * (i + 1) / pairs, 128);
-      s.from[i] = i == 0 ? 0 : (fp8 || gqa == 1 ? 2 * i : 2 * i + 2) * s.most[i];
-      // not where it fills the units less
-      if (i && (int64_t)s.most[i] * pairs * i + 24 * i * (i + 1) < (int64_t)s.most[i - 1] * pairs * (i + 1)) s.most[i] = s.most[i - 1], s.from[i] = INT32_MAX;
+      s.from[i] = i == 0 ? 0 : std::max(6, (fp8 ? 2 * i : 2 * i + 2) * s.most[i]);
+      // not where it fills the units less, nor, in fp8 and with groups, three a unit where it does not fill them better
+      const int64_t full = (int64_t)s.most[i] * pairs * i, before = i ? (int64_t)s.most[i - 1] * pairs * (i + 1) : 0;
+      const int by = fp8 && gqa > 1 && i == 2 ? -24 * i * (i + 1) : 24 * i * (i + 1);
+      if (i && full + by < before) s.most[i] = s.most[i - 1], s.from[i] = INT32_MAX;
     }
   } else {                                   // those that fill whole rounds of the units best, one for every eight rounds
     s.lo = 1;
