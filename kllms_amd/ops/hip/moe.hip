@@ -27,16 +27,14 @@
 // The layer with a router of seven launches at 65 / 150 / 300 / 600 / 1024 / 2048 / 6000 rows, experts of 14336: 582 / 582 /
 // 605 / 666 / 949 / 1431 / 3623 us (741 / 760 / 787 / 907 / 1131 / 1935 / 4622); moe_route has what it was after that.
 //
-// W is read once for the row tiles side by side and is loaded with the streaming hint, which leaves the L2 to x; tiles of 224
-// rows are for parts of 193 to 224, a tenth less than a tile of 256. The layer, us without the two and with: 10 rows 487, 454;
-// 300 563, 541; 1024 889, 883; 1600 1144, 1057; 2048 1377, 1370; 2600 1720, 1610; experts of 7168, 3300 rows 1105, 1016, 6000
-// 1739, 1736; width 2048, experts of 8192, 600 rows 227, 219.
+// Tiles of 224 rows are for parts of 193 to 224, a tenth less than a tile of 256. The layer, us without them and with: 1600
+// rows 1144, 1057; 2600 1720, 1610; experts of 7168, 3300 rows 1105, 1016. When W has the streaming hint: moe_once.
 
 #include "tile_product.h"
 
 // one tile; GATEUP: a = x [T, K] gathered by ids, w [E, 2 * N, K] (gate at [0, N), up behind), out [S, N].
 // Down: a = act [S, K], w [E, N, K], out [S, N]
-template <bool GATEUP, int MJ>
+template <bool GATEUP, bool ONCE, int MJ>
 __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t* __restrict__ a,
                                          const bf16_t* __restrict__ w, const int* __restrict__ ids,
                                          const bf16_t* __restrict__ zeros, int e, int m0, int m_end, int n0, int N,
@@ -54,7 +52,7 @@ __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t*
   if constexpr (GATEUP) {
     // W rows of a tile: 64 gate, 64 up, the next 64 gate, 64 up
     const int n_put = n0 + (wave >> 1) * 64;
-    const TileRowsOf<true> wr(w + ((int64_t)e * 2 + (wave & 1)) * N * K + k0, n_put, N, 64, K, lane);
+    const TileRowsOf<ONCE> wr(w + ((int64_t)e * 2 + (wave & 1)) * N * K + k0, n_put, N, 64, K, lane);
     TileGather<MJ> xr;
 #pragma unroll
     for (int i = 0; i < MJ; ++i) {
@@ -75,7 +73,7 @@ __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t*
     });
   } else {
     const int n_put = n0 + wave * 64, m_put = m0 + wave * MJ * 8;
-    const TileRowsOf<true> wr(w + (int64_t)e * N * K + k0, n_put, N, 64, K, lane);
+    const TileRowsOf<ONCE> wr(w + (int64_t)e * N * K + k0, n_put, N, 64, K, lane);
     const TileRows xr(a + k0, m_put, m_end, MJ * 8, K, lane);
     tile_product<MJ>(acc, wr, xr, stages, stages * (blockIdx.x & 7) / 8, smem);
     if (sh.shares > 1 && !tile_fold<MJ>(acc, sh.part, sh.share, sh.shares, sh.count, smem)) return;
@@ -88,7 +86,7 @@ __device__ __forceinline__ void moe_tile(bf16_t* __restrict__ out, const bf16_t*
 // offsets [E + 1]: row range of each expert in sorted space; ids [S]: token index of a
 // sorted row, or -1 (a row of zeros, [K]). Down: part, count: room for the shares of
 // tiles, or nullptr: every tile is one workgroup's.
-template <bool GATEUP>
+template <bool GATEUP, bool ONCE>
 __global__ void __launch_bounds__(TP_THREADS, 1) moe_product_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
     const int* __restrict__ ids, const bf16_t* __restrict__ zeros, const int* __restrict__ offsets,
@@ -134,7 +132,7 @@ __global__ void __launch_bounds__(TP_THREADS, 1) moe_product_kernel(
   // an expert's rows in even parts: its row tiles keep step, and read W from memory once
   const int rows = (end - begin + m_tiles - 1) / m_tiles;
   const int n0 = (first + at / m_tiles * 8) * BN, m0 = begin + at % m_tiles * rows, m_end = min(end, m0 + rows);
-#define MOE_TILE(MJ) moe_tile<GATEUP, MJ>(out, a, w, ids, zeros, e, m0, m_end, n0, N, K, sh, smem)
+#define MOE_TILE(MJ) moe_tile<GATEUP, ONCE, MJ>(out, a, w, ids, zeros, e, m0, m_end, n0, N, K, sh, smem)
   if (rows > 224) MOE_TILE(8);
   else if (rows > 192) MOE_TILE(7);
   else if (rows > 160) MOE_TILE(6);
@@ -422,17 +420,39 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(bf16_t* __restrict__ o
   reinterpret_cast<bf16x8_vec*>(out)[(int64_t)t * nvec + i] = o;
 }
 
+// Whether the products load W with the streaming hint, which leaves the caches to x: where the weights of all experts are
+// themselves too large for the 256 MB last-level cache, so that no call finds anything of the one before, and few enough
+// rows go to an expert that its W is read by one row tile, or two. Smaller ones stay in the cache from layer to layer or
+// from call to call in part, and the hint gives that up. us without and with, 8 experts, width and size of an expert:
+//   gate/up  1024x4096 (134 MB), 1024 tokens, 2 choices 58, 61   2048x4096 (268 MB) alone 4 tokens 36, 37; 600 56, 58
+//            2048x6144 (402 MB) 32 tokens 84, 80; 800 113, 112   2048x8192 (537 MB) 4 tokens 85, 81; 300 117, 107; 800 131, 127
+//            4096x14336 (1879 MB) 32 tokens 341, 316; 800 422, 417
+//     but with 256 rows an expert and more 2048x8192 168, 171; 4096x14336 532, 539; 2048x6144, 512 rows 213, 217
+//   down     2048x4096 (134 MB) alone 32 tokens 32, 54; 1024 73, 93   2048x6144 (201 MB) 2048 tokens 141, 157
+//            4096x7168 (470 MB) 4 tokens 96, 93; 300 124, 120; 1024 175, 172   4096x14336 (940 MB) 2048 tokens 564, 558
+#define MOE_ONCE_BYTES ((int64_t)320 << 20)
+static bool moe_once(bool gateup, int64_t S, int64_t E, int64_t N, int64_t K) {
+  return E * (gateup ? 2 : 1) * N * K * 2 >= MOE_ONCE_BYTES && S <= E * (gateup ? 224 : 512);
+}
+
 // rows S in sorted space; the grid holds the most tiles that S rows of E experts can make
 // on an XCD, eightfold, and a round for shares. Returns 0, or -1 where the LDS cannot be had
+template <bool GATEUP, bool ONCE>
+static int moe_product_of(void* out, const void* a, const void* w, const int* ids, const void* zeros, const int* offsets,
+                          float* part, int* count, int S, int E, int N, int K, hipStream_t stream) {
+  if (!tp_lds_ready(reinterpret_cast<const void*>(moe_product_kernel<GATEUP, ONCE>))) return -1;
+  const int64_t n_tiles = GATEUP ? (N + 127) / 128 : (N + 255) / 256;
+  const int64_t blocks = (S / 256 + E) * ((n_tiles + 7) / 8) + (part ? TP_SLOTS : 0);
+  hipLaunchKernelGGL((moe_product_kernel<GATEUP, ONCE>), dim3(blocks * 8), dim3(TP_THREADS), TP_LDS, stream, (bf16_t*)out,
+                     (const bf16_t*)a, (const bf16_t*)w, ids, (const bf16_t*)zeros, offsets, part, count, E, N, K);
+  return 0;
+}
+
 template <bool GATEUP>
 static int moe_product(void* out, const void* a, const void* w, const int* ids, const void* zeros, const int* offsets,
                        float* part, int* count, int S, int E, int N, int K, hipStream_t stream) {
-  if (!tp_lds_ready(reinterpret_cast<const void*>(moe_product_kernel<GATEUP>))) return -1;
-  const int64_t n_tiles = GATEUP ? (N + 127) / 128 : (N + 255) / 256;
-  const int64_t blocks = (S / 256 + E) * ((n_tiles + 7) / 8) + (part ? TP_SLOTS : 0);
-  hipLaunchKernelGGL(moe_product_kernel<GATEUP>, dim3(blocks * 8), dim3(TP_THREADS), TP_LDS, stream, (bf16_t*)out,
-                     (const bf16_t*)a, (const bf16_t*)w, ids, (const bf16_t*)zeros, offsets, part, count, E, N, K);
-  return 0;
+  const auto product = moe_once(GATEUP, S, E, N, K) ? moe_product_of<GATEUP, true> : moe_product_of<GATEUP, false>;
+  return product(out, a, w, ids, zeros, offsets, part, count, S, E, N, K, stream);
 }
 
 extern "C" int launch_moe_gateup(void* act, const void* x, const void* w, const int* sorted_ids, const int* offsets,

@@ -207,6 +207,30 @@ def test_mixture_products_at_the_edges_of_row_tiles(H, I, counts):
     test_mixture_products_against_float64(H, I, counts)
 
 
+@pytest.mark.parametrize("counts", [[1, 64, 0], [65, 130, 200], [225, 0, 600], [0, 9000, 3000]])
+def test_mixture_products_of_weights_beyond_the_cache(counts):
+    """How W is loaded, which its size and the rows of an expert decide, is not to be seen in the results: the first experts
+    alone give the same bits as with all others behind them, whose products have more than 320 MB of W to read. The last one's
+    experts have too many rows for the difference."""
+    E, H, I, few = 21, 4096, 2048, len(counts)
+    g = torch.Generator(device=DEV).manual_seed(sum(counts))
+    wg = torch.empty(E, 2 * I, H, device=DEV, dtype=torch.bfloat16).normal_(0, H ** -0.5, generator=g)
+    wd = torch.empty(E, H, I, device=DEV, dtype=torch.bfloat16).normal_(0, I ** -0.5, generator=g)
+    S = sum(counts)
+    x = torch.randn(S, H, device=DEV, generator=g).bfloat16()
+    ids = torch.randperm(S, device=DEV, generator=g).to(torch.int32)
+    ends = torch.tensor([0] + counts).cumsum(0)
+    got = []
+    for n in (few, E):
+        offsets = torch.cat([ends, ends[-1:].expand(n - few)]).to(device=DEV, dtype=torch.int32)
+        act, y = torch.empty(S, I, device=DEV, dtype=x.dtype), torch.empty(S, H, device=DEV, dtype=x.dtype)
+        ops.moe_gateup(act, x, wg[:n], ids, offsets, x)
+        ops.moe_down(y, act, wd[:n], offsets)
+        got.append((act, y))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert torch.isfinite(got[0][1]).all() and got[0][1].abs().amax(1).gt(0).all()
+
+
 @pytest.mark.parametrize("E", [1, 8, 128, 1024, 1025, 4096])
 @pytest.mark.parametrize("T,k", [(1, 1), (63, 2), (65, 3), (1025, 2), (9001, 2)])
 def test_sort_of_the_mixture_keeps_the_order_of_the_pairs(T, k, E):
