@@ -24,6 +24,8 @@ class ListedLayerLM(nn.Module):
     # batches; prefix-block reuse is off (state cannot be rebuilt from blocks)
     stateful = True
 
+    _once = False           # ops.weights_once, of a model whose steps run on the few-row products
+
     trace_layers: Optional[list] = None   # debugging: residual after each layer run
 
     def checkpoint_map(self) -> Dict[str, torch.Tensor]:
@@ -61,7 +63,7 @@ class ListedLayerLM(nn.Module):
         head = self.lm_head
         if (ops.only_weights(head, nn.Linear) and head.bias is None and ops.plain_call(hidden, head.weight)
                 and ops.no_global_hooks()):
-            out = ops.linear_f32(hidden, head.weight)
+            out = ops.linear_f32(hidden, head.weight, self._once)
             if out is not None:
                 return out
         return head(hidden).float()

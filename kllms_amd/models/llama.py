@@ -177,6 +177,7 @@ class LlamaDecoderLayer(nn.Module):
 
 class LlamaForCausalLM(nn.Module):
     layer_cls = LlamaDecoderLayer
+    _once = False           # ops.weights_once
 
     def __init__(self, cfg: ModelArchConfig, ctx: Optional[ParallelContext] = None, dtype=torch.bfloat16):
         super().__init__()
@@ -194,6 +195,7 @@ class LlamaForCausalLM(nn.Module):
         # every rank — no logits gather needed.
         self.lm_head = nn.Linear(cfg.hidden_size, cfg.vocab_size, bias=False, dtype=dtype)
         self.lm_head.weight.requires_grad_(False)
+        self._once = ops.weights_once(self)
         self.register_buffer(
             "cos_sin",
             build_cos_sin_cache(cfg.head_dim_, cfg.max_position_embeddings, cfg.rope_theta, "cpu",
@@ -374,7 +376,7 @@ class LlamaForCausalLM(nn.Module):
     def _forward_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
         """A decode step or a short prompt: weights streamed by the few-row kernel, whose split sums go straight into the
         next row-wise kernel: 8 launches a layer, one more where gate/up is the library's. A prompt's fused projection stays whole: its attention reads the keys and values as rows."""
-        layers, norm = self.layers, self.layers[0].input_layernorm
+        layers, norm, once = self.layers, self.layers[0].input_layernorm, self._once
         T = input_ids.shape[0]
         if batch.mode == "decode":
             # zeroed by the first launch, and zero again after each layer's attention
@@ -391,16 +393,16 @@ class LlamaForCausalLM(nn.Module):
             if batch.mode == "prefill":
                 att = at.attend(x, batch, self.cos_sin)
             else:
-                q = ops.rope_store_rows(ops.linear_part(x, at.qkv_proj.weight), at.qkv_proj.bias, at.num_heads,
+                q = ops.rope_store_rows(ops.linear_part(x, at.qkv_proj.weight, once), at.qkv_proj.bias, at.num_heads,
                                         batch.positions, self.cos_sin, k_cache, v_cache, batch.slot_mapping, k_scale, v_scale)
                 att = at.attend_cache(q, batch, arrived)
-            x = ops.add_norm_rows(ops.linear_part(att.view(T, -1), at.o_proj.weight), residual, norm.weight, norm.eps)
+            x = ops.add_norm_rows(ops.linear_part(att.view(T, -1), at.o_proj.weight, once), residual, norm.weight, norm.eps)
             norm = layers[i + 1].input_layernorm if i + 1 < len(layers) else self.norm
             mlp = layer.mlp
             if isinstance(mlp, LlamaMLP):
                 w = mlp.gate_up_proj.weight
-                act = (ops.linear_silu_rows(x, w) if self._silu_rows(T, w) or self._silu_streams(T, w) else mlp.activate(x))
-                x = ops.add_norm_rows(ops.linear_part(act, mlp.down_proj.weight), residual, norm.weight, norm.eps)
+                act = (ops.linear_silu_rows(x, w, once) if self._silu_rows(T, w) or self._silu_streams(T, w) else mlp.activate(x))
+                x = ops.add_norm_rows(ops.linear_part(act, mlp.down_proj.weight, once), residual, norm.weight, norm.eps)
             else:
                 x, residual = ops.fused_add_rmsnorm(mlp(x), residual, norm.weight, norm.eps)
         return x
@@ -438,7 +440,7 @@ class LlamaForCausalLM(nn.Module):
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """fp32 [rows, V]."""
-        out = ops.linear_f32(hidden, self.lm_head.weight) if self.lm_head.bias is None else None
+        out = ops.linear_f32(hidden, self.lm_head.weight, self._once) if self.lm_head.bias is None else None
         if out is not None:
             return out
         return self.lm_head(hidden).float()

@@ -263,7 +263,8 @@ class ParallelMixer(nn.Module):
         self.right = DecayLinearAttention(ri, hidden, eps, dtype)
         self.left_out = _param(hidden, dtype=torch.float32)
         self.right_out = _param(hidden, dtype=torch.float32)
-        # sizes of the step of few rows (rows_step)
+        # sizes of the step of few rows (rows_step), and how it reads its weights: ops.weights_once of the model
+        self.once = False
         self.rows_ok = (le.dim == 128 and le.vdim == 128 and le.values_from_keys and le.head_gate and le.mask_size >= 0
                         and le.heads // le.kv_heads in (1, 2, 4, 8) and self.inp.weight.shape[0] % 16 == 0
                         and ri.dim <= 256 and ri.dim % 4 == 0 and ri.vdim % 4 == 0 and ri.heads * ri.vdim % 128 == 0 and hidden % 128 == 0 and hidden <= 8192)
@@ -283,7 +284,7 @@ class ParallelMixer(nn.Module):
         at = [p[n][0] for n in ("left.q", "left.k", "left.g", "right.q", "right.k", "right.v", "right.g")]
         return ops.hybrid_parallel_rows(x, h, inp.weight, inp.bias, at, left.inv_freq, st.k, st.v, left.o_proj,
                                         right.decay, st.rec, right.norm, right.o_proj, self.left_out, self.right_out,
-                                        w_post, w_next, batch, le.heads, le.scale, le.mask_size, right.eps)
+                                        w_post, w_next, batch, le.heads, le.scale, le.mask_size, right.eps, self.once)
 
     def forward(self, h: torch.Tensor, batch, st: LayerState):
         y = self.inp(h)
@@ -336,7 +337,8 @@ class ChannelDeltaMixer(nn.Module):
         self.A_log = _param(spec.heads, dtype=torch.float32)
         self.norm = _param(spec.vdim, dtype=torch.float32)
         self.o_proj = _param(hidden, self.hv, dtype=dtype)
-        # sizes of the step of few rows (rows_step)
+        # sizes of the step of few rows (rows_step), and how it reads its weights: ops.weights_once of the model
+        self.once = False
         self.rows_ok = (self.inp.weight.shape[0] % 16 == 0 and self.hv % 128 == 0 and spec.dim <= 256 and spec.conv <= 16
                         and hidden % 128 == 0 and hidden <= 8192)
 
@@ -354,7 +356,7 @@ class ChannelDeltaMixer(nn.Module):
         at = [inp.parts[n][0] for n in ("q", "k", "v", "a1", "g1", "b")]
         return ops.hybrid_delta_rows(x, h, inp.weight, at, self.conv, st.conv, self.a2, self.g2, self.dt_bias,
                                      self.A_log, st.rec, self.norm, self.o_proj, w_post, w_next, batch,
-                                     self.spec.kv_heads, self.eps)
+                                     self.spec.kv_heads, self.eps, self.once)
 
     def forward(self, h: torch.Tensor, batch, st: LayerState) -> torch.Tensor:
         sp = self.spec
@@ -395,7 +397,8 @@ class ClampedGLU(nn.Module):
         self.inp = FusedInput(hidden, [("gate", spec.ff), ("up", spec.ff)], dtype)
         self.down = _param(hidden, spec.ff, dtype=dtype)
         self._fused = self.inp.weight.shape[0] == 2 * spec.ff      # up's rows follow gate's without a gap
-        # sizes of the step of few rows (rows_step)
+        # sizes of the step of few rows (rows_step), and how it reads its weights: ops.weights_once of the model
+        self.once = False
         self.rows_ok = self._fused and spec.ff % 128 == 0 and hidden % 128 == 0 and hidden <= 8192
 
     def takes_rows(self) -> bool:
@@ -405,7 +408,7 @@ class ClampedGLU(nn.Module):
     def rows_step(self, x, h, w_post, w_next, eps: float) -> Optional[torch.Tensor]:
         """The sublayer with its residual for single decoded rows: ops.hybrid_glu_rows."""
         return ops.hybrid_glu_rows(x, h, self._modules["inp"].weight, self.down, w_post, w_next, self.spec.limit,
-                                   self.spec.alpha, eps)
+                                   self.spec.alpha, eps, self.once)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         act = None

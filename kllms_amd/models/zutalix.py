@@ -101,6 +101,11 @@ class ZutalixForCausalLM(ListedLayerLM):
         self.final_norm = _param(W, dtype=torch.float32)
         self.lm_head = nn.Linear(W, cfg.vocab_size, bias=False, dtype=dtype)
         self.lm_head.weight.requires_grad_(False)
+        self._once = ops.weights_once(self)
+        for layer in self.layers:
+            for m in (layer.mix, layer.mlp):
+                if m is not None:
+                    m.once = self._once
 
     # --- cache layout ---------------------------------------------------------
     def cache_layout(self) -> List[LayerCacheSpec]:

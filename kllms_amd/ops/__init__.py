@@ -306,22 +306,33 @@ def rows_weights_ok(ws: Sequence[torch.Tensor], like: torch.Tensor) -> bool:
     return all(type(w) in _PLAIN for w in ws) and _hip_or_raise().rows_weights_ok(ws, like)
 
 
-def linear_part(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+WEIGHTS_ONCE_BYTES = 320 << 20
+
+
+def weights_once(model: torch.nn.Module) -> bool:
+    """``once`` of the few-row products in a model's steps: whether the matrices that every step reads are too many to stay in
+    the 256 MB last-level cache until the next one. Tables, of which a step reads rows, and stacks of experts, of which it
+    reads some, do not count: without them it is a model whose steps hit nothing for certain."""
+    return sum(p.numel() * p.element_size() for m in model.modules() if not isinstance(m, torch.nn.Embedding)
+               for p in m.parameters(recurse=False) if p.dim() == 2) >= WEIGHTS_ONCE_BYTES
+
+
+def linear_part(x: torch.Tensor, w: torch.Tensor, once: bool = False) -> torch.Tensor:
     """fp32 sums [S, M, N] of x @ w^T over S shares of K; the consumer adds them up."""
-    return _hip_or_raise().linear_rows(x, w, _none(x), 0, 0)
+    return _hip_or_raise().linear_rows(x, w, _none(x), 0, 0, once)
 
 
-def linear_silu_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def linear_silu_rows(x: torch.Tensor, w: torch.Tensor, once: bool = False) -> torch.Tensor:
     """silu(gate) * up of a fused [gate; up] matrix, bf16."""
-    return _hip_or_raise().linear_rows(x, w, _none(x), 3, 1)
+    return _hip_or_raise().linear_rows(x, w, _none(x), 3, 1, once)
 
 
-def linear_f32_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def linear_f32_rows(x: torch.Tensor, w: torch.Tensor, once: bool = False) -> torch.Tensor:
     """fp32 x @ w^T without a rounding to bf16 (logits)."""
-    return _hip_or_raise().linear_rows(x, w, _none(x), 2, 1)
+    return _hip_or_raise().linear_rows(x, w, _none(x), 2, 1, once)
 
 
-def linear_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+def linear_f32(x: torch.Tensor, w: torch.Tensor, once: bool = False) -> Optional[torch.Tensor]:
     """fp32 x @ w^T from the fp32 sums of the bf16 product at every row count (rounded to bf16 at some counts only, near ties
     between tokens would fall differently as a stream's batch grows); None where that is not to be had: not bf16 on the GPU,
     or wanted for a gradient."""
@@ -335,7 +346,7 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     K = w.shape[1]
     most = 64 if K & (K - 1) else 128 if K >= 4096 else 96
     if x.shape[0] <= most and linear_rows_ok(x, w):
-        return linear_f32_rows(x, w)
+        return linear_f32_rows(x, w, once)
     return torch.mm(x, w.t(), out_dtype=torch.float32)
 
 
@@ -739,27 +750,27 @@ def hybrid_rows_ok(x, h, batch) -> bool:
 
 
 def hybrid_parallel_rows(x, h, w_in, bias, at, inv_freq, k_cache, v_cache, o_left, decay, state, norm_right, o_right, wa,
-                         wb, w_post, w_next, batch, heads, scale, mask_size, eps):
+                         wb, w_post, w_next, batch, heads, scale, mask_size, eps, once=False):
     """x (fp32 stream) += the parallel sublayer of h in place, with cache and state; returns the next normed input. at:
     columns of left q, k, head gates and right q, k, v, gate in h @ w_in^T + bias. None, and nothing done, where the
     weights do not lie as the kernels read them (contiguous, from 16 bytes on)."""
     return _seq().hybrid_parallel_rows(
         x, h, w_in, bias if bias is not None else _none(h), at, inv_freq, k_cache, v_cache, o_left, decay, state,
         norm_right, o_right, wa, wb, w_post, w_next, batch.positions, batch.slot_mapping, batch.block_tables,
-        batch.context_lens, batch.state_slots, batch.cu_seqlens, batch.seg_start, heads, scale, mask_size, eps)
+        batch.context_lens, batch.state_slots, batch.cu_seqlens, batch.seg_start, heads, scale, mask_size, eps, once)
 
 
 def hybrid_delta_rows(x, h, w_in, at, conv, conv_state, a2, g2, dt_bias, a_log, state, norm, w_out, w_post, w_next, batch,
-                      kv_heads, eps):
+                      kv_heads, eps, once=False):
     """The same of a gated-delta-rule sublayer; at: columns of q, k, v, the low-rank inputs and the write strengths."""
     return _seq().hybrid_delta_rows(x, h, w_in, at, conv, conv_state, a2, g2, dt_bias, a_log, state, norm, w_out, w_post,
                                     w_next, batch.state_slots, batch.cu_seqlens, batch.seg_start, batch.token_seg,
-                                    kv_heads, eps)
+                                    kv_heads, eps, once)
 
 
-def hybrid_glu_rows(x, h, w_in, w_down, w_post, w_next, limit, alpha, eps):
+def hybrid_glu_rows(x, h, w_in, w_down, w_post, w_next, limit, alpha, eps, once=False):
     """The same of a clamped gated-linear-unit sublayer."""
-    return _seq().hybrid_glu_rows(x, h, w_in, w_down, w_post, w_next, limit, alpha, eps)
+    return _seq().hybrid_glu_rows(x, h, w_in, w_down, w_post, w_next, limit, alpha, eps, once)
 
 
 def embed_bigram(ids, table, bigram, scale, mul_prev, mul_cur, buckets, tok_state, state_slots, cu_seqlens,

@@ -527,12 +527,13 @@ torch::Tensor moe_combine(torch::Tensor y, torch::Tensor weights, torch::Tensor 
 extern "C" int linear_rows_most(int form);
 extern "C" int64_t linear_rows_strides();
 extern "C" int launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N,
-                                   int K, int x_stride, int form, int splits, float limit, float alpha, hipStream_t stream);
+                                   int K, int x_stride, int form, int splits, float limit, float alpha, bool once,
+                                   hipStream_t stream);
 extern "C" int linear_rows_splits(int M, int N, int K);
 
 // form 0: fp32 sums [S, M, N]; 1: bf16 [M, N] (+ bias); 2: fp32 [M, N]; 3: silu(gate) * up of a fused
-// [gate; up] matrix, bf16 [M, N / 2]
-torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, torch::Tensor bias, int64_t form, int64_t splits) {
+// [gate; up] matrix, bf16 [M, N / 2]. once: the weights of the caller's step do not stay in the caches until its next
+torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, torch::Tensor bias, int64_t form, int64_t splits, bool once) {
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 &&
                   x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
               "x must be a bf16 [M, K] row view, 16-byte aligned");
@@ -552,7 +553,7 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, torch::Tensor bias, 
            : form == 2 ? torch::empty({M, N}, x.options().dtype(torch::kFloat))
                        : torch::empty({M, form == 3 ? N / 2 : N}, x.options());
   TORCH_CHECK(launch_linear_rows(out.data_ptr(), cbf(x), cbf(w), bias.numel() ? cbf(bias) : nullptr, M, N, K,
-                                 x_stride, (int)form, S, 0.0f, 0.0f, cur_stream()) == 0,
+                                 x_stride, (int)form, S, 0.0f, 0.0f, once, cur_stream()) == 0,
               "linear_rows: 160 KB of LDS are not available");
   return out;
 }
@@ -718,7 +719,8 @@ void ipc_allreduce_destroy(int64_t ctx) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("levenshtein_pairs", &levenshtein_pairs);
-  m.def("linear_rows", &linear_rows);
+  m.def("linear_rows", &linear_rows, py::arg("x"), py::arg("w"), py::arg("bias"), py::arg("form"), py::arg("splits"),
+        py::arg("once") = false);
   m.def("rows_weights_ok", &rows_weights_ok);
   m.def("add_norm_rows", &add_norm_rows);
   m.def("embed_norm_rows", &embed_norm_rows, py::arg("ids"), py::arg("table"), py::arg("weight"), py::arg("eps"),

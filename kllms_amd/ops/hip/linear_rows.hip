@@ -180,17 +180,19 @@ static bool lr_lds_ready(const void* kernel, std::atomic<uint64_t>& devices) {
   return true;
 }
 
-// Bytes of a matrix from which on its rows are loaded with the streaming hint (nt). A model whose matrices are as large does not
-// fit the last-level cache (256 MB) from one step to the next: without the hint they push out of it, and of the L2, what the
-// step reads again (x, sums, keys of shared prompts) and hit nothing themselves. us without and with, 900 MB of weights in turn:
-//   PART  4096 x 4096   5 rows 8.1, 7.7   120 rows 12.4, 12.2     6144 x 4096   5 rows 11.3, 10.6   120 16.4, 16.1
-//     4096 x 14336   5 rows 23.8, 20.9   120 32.7, 31.5   384 59.7, 58.6     2048 x 8192   1 row 8.9, 8.2   120 12.3, 12.2
-//   SILU  28672 x 4096   5 rows 41.6, 37.6 (6.2 TB/s)   120 49.6, 46.9   256 64.3, 63.5     16384 x 2048   1 row 14.4, 13.1
-//   F32   32000 x 4096   5 rows 46.6, 41.3   120 54.9, 51.7
-// Weights that do fit lose by it, at many rows above all: 130 MB of 16384 x 2048 1 row 12.9, 11.9   100 rows 13.8, 16.6; 200 MB of
-// 2048 x 2048 4.2, 4.2 and 5.8, 6.4; 30 MB of 1024 x 1024 3.6, 3.6 and 5.0, 5.2; 100 MB of 4096 x 1024 6.2, 6.3 and 8.1, 9.7.
-// From widths of 2048 on a layer has 120 MB; below, the matrices are smaller than this.
+// Whether W's rows are loaded with the streaming hint (nt): where the caller says that the weights of its step are too large to
+// stay in the last-level cache (256 MB) until the next one, or the matrix is by itself. Without the hint such weights push out of
+// it, and of the L2, what the step reads again (x, sums, keys of shared prompts) and hit nothing themselves. us without and with:
+//   SILU  16384 x 2048   1 row 14.3, 12.8 with 335 MB of weights in turn   13.8, 12.5 with 870   128 rows 19.1, 18.6   18.6, 18.2
+//   PART  2048 x 8192   1 row 8.5, 8.1 with 301 MB   8.4, 7.8 with 870   128 rows 12.7, 12.8   12.5, 12.3
+//     4096 x 4096   1 row 8.1, 7.9   8.0, 7.6   128 rows 13.2, 13.2   13.0, 12.8     4096 x 14336   5 rows 23.8, 20.9 with 900 MB
+//   SILU  28672 x 4096   5 rows 41.6, 37.6 (6.2 TB/s)   120 49.6, 46.9   256 64.3, 63.5 with 900 MB     F32   32000 x 4096   5 rows
+//     46.6, 41.3   120 54.9, 51.7
+// Weights that do fit lose by it: with 200 MB 16384 x 2048 1 row 12.5, 12.3   128 rows 14.3, 18.9; 2048 x 8192 8.0, 8.5   10.3, 12.9;
+// 8192 x 1024 6.0, 6.9   8.1, 10.7; between 268 and 290 MB it depends on the rows. Matrices of less than LR_ONCE are plain
+// always: nobody waits for them.
 #define LR_ONCE (8 << 20)
+#define LR_ONCE_ALONE ((int64_t)320 << 20)
 
 template <int NI, int MJ, int FORM, int KB, bool ONCE>
 static int linear_rows_go(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* more, int M, int N, int K, int x_stride,
@@ -206,9 +208,9 @@ static int linear_rows_go(void* out, const bf16_t* x, const bf16_t* w, const bf1
 
 template <int FORM>
 static int linear_rows_form(const LinearPlan& p, void* out, const bf16_t* x, const bf16_t* w, const bf16_t* more, int M, int N,
-                            int K, int x_stride, int splits, float limit, float alpha, hipStream_t stream) {
-  // of two matrices K is both's
-  const bool once = (int64_t)N * K * (int64_t)sizeof(bf16_t) >= LR_ONCE;
+                            int K, int x_stride, int splits, float limit, float alpha, bool once, hipStream_t stream) {
+  const int64_t bytes = (int64_t)N * K * (int64_t)sizeof(bf16_t);     // of two matrices K is both's
+  once = once ? bytes >= LR_ONCE : bytes >= LR_ONCE_ALONE;
 #define LR_CASE(NI, MJ)                                                                                              \
   if (p.ni == NI && p.mj == MJ)                                                                                      \
     return once ? linear_rows_go<NI, MJ, FORM, (NI == 2 || MJ <= 2 ? 80 : 160), true>(out, x, w, more, M, N, K, x_stride, p.m_tiles, \
@@ -241,12 +243,13 @@ extern "C" int linear_rows_most(int form) { return form == LR_PART ? 384 : form 
 // x_stride from which on 64 rows' offsets would leave 32 bits
 extern "C" int64_t linear_rows_strides() { return 1 << 25; }
 
-// 0, or -1 where the LDS cannot be had. x_stride: any below linear_rows_strides(), 0 and less than K too
+// 0, or -1 where the LDS cannot be had. x_stride: any below linear_rows_strides(), 0 and less than K too; once: the weights of
+// the caller's step pass the caches by (LR_ONCE)
 extern "C" int launch_linear_rows(void* out, const bf16_t* x, const bf16_t* w, const bf16_t* bias, int M, int N, int K,
-                                  int x_stride, int form, int splits, float limit, float alpha, hipStream_t stream) {
+                                  int x_stride, int form, int splits, float limit, float alpha, bool once, hipStream_t stream) {
   const LinearPlan p = linear_plan(M, N, K, form);
 #define LR_FORM(F) \
-  case F: return linear_rows_form<F>(p, out, x, w, bias, M, N, K, x_stride, splits, limit, alpha, stream)
+  case F: return linear_rows_form<F>(p, out, x, w, bias, M, N, K, x_stride, splits, limit, alpha, once, stream)
   switch (form) {
     LR_FORM(LR_PART);
     LR_FORM(LR_BF16);
@@ -268,6 +271,6 @@ extern "C" int linear_rows_splits(int M, int N, int K) {
 
 // PART sums of two products of one size, x [2, M, K] with w and w2 [N, K]: [S, M, N], the first half of the (even) S the one's
 extern "C" int launch_linear_rows_two(float* out, const bf16_t* x, const bf16_t* w, const bf16_t* w2, int M, int N, int K,
-                                      int splits, hipStream_t stream) {
-  return linear_rows_form<LR_PART>(linear_plan(M, N, K, LR_PART), out, x, w, w2, M, N, 2 * K, K, splits, 0.0f, 0.0f, stream);
+                                      int splits, bool once, hipStream_t stream) {
+  return linear_rows_form<LR_PART>(linear_plan(M, N, K, LR_PART), out, x, w, w2, M, N, 2 * K, K, splits, 0.0f, 0.0f, once, stream);
 }

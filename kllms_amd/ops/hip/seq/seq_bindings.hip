@@ -1200,18 +1200,19 @@ std::optional<torch::Tensor> hybrid_parallel_rows(torch::Tensor, torch::Tensor, 
                                    torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                                    torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                                    torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
-                                   torch::Tensor, int64_t, double, int64_t, double);
+                                   torch::Tensor, int64_t, double, int64_t, double, bool);
 std::optional<torch::Tensor> hybrid_delta_rows(torch::Tensor, torch::Tensor, torch::Tensor, std::vector<int64_t>, torch::Tensor,
                                 torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                                 torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
-                                torch::Tensor, torch::Tensor, int64_t, double);
+                                torch::Tensor, torch::Tensor, int64_t, double, bool);
 std::optional<torch::Tensor> hybrid_glu_rows(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
-                              double, double, double);
+                              double, double, double, bool);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("hybrid_parallel_rows", &hybrid_parallel_rows);
   m.def("hybrid_delta_rows", &hybrid_delta_rows);
-  m.def("hybrid_glu_rows", &hybrid_glu_rows);
+  m.def("hybrid_glu_rows", &hybrid_glu_rows, py::arg("x"), py::arg("h"), py::arg("w_in"), py::arg("w_down"), py::arg("w_post"),
+        py::arg("w_next"), py::arg("limit"), py::arg("alpha"), py::arg("eps"), py::arg("once") = false);
   m.def("embed_rmsnorm", &embed_rmsnorm);
   m.def("rmsnorm_cast", &rmsnorm_cast);
   m.def("sandwich_residual", &sandwich_residual);

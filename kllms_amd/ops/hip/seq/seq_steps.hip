@@ -31,9 +31,9 @@ void seq_launch_delta_rows(const float*, int, const int64_t*, const float*, void
 void seq_launch_gated_act(void*, const void*, const void*, int64_t, int, int, float, float, float, int, hipStream_t);
 // few-row products and paged decode attention (ops/hip/linear_rows.hip, attn_decode.hip, also part of kllms_amd._C)
 int launch_linear_rows(void*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
-                        int, int, float, float, hipStream_t);
+                        int, int, float, float, bool, hipStream_t);
 int launch_linear_rows_two(float*, const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, int, int, int, int,
-                           hipStream_t);
+                           bool, hipStream_t);
 int linear_rows_splits(int, int, int);
 int attn_decode_splits(int, int, int, int, int, int, int);
 void launch_attn_decode(__hip_bfloat16*, float*, int*, int, const __hip_bfloat16*, const void*, const void*, const float*,
@@ -73,10 +73,10 @@ void check_weight(const Tensor& w, int64_t K, const char* name) {
 }
 
 // x [T, K] (contiguous) by w: fp32 sums [S, T, N]
-Tensor part(const Tensor& x, const Tensor& w, int T, hipStream_t st) {
+Tensor part(const Tensor& x, const Tensor& w, int T, bool once, hipStream_t st) {
   const int K = w.size(1), N = w.size(0), S = linear_rows_splits(T, N, K);
   auto out = torch::empty({S, T, N}, x.options().dtype(torch::kFloat));
-  TORCH_CHECK(launch_linear_rows(out.data_ptr(), bf(x), bf(w), nullptr, T, N, K, K, ROWS_PART, S, 0.0f, 0.0f, st) == 0, NO_LDS);
+  TORCH_CHECK(launch_linear_rows(out.data_ptr(), bf(x), bf(w), nullptr, T, N, K, K, ROWS_PART, S, 0.0f, 0.0f, once, st) == 0, NO_LDS);
   return out;
 }
 
@@ -101,7 +101,7 @@ std::optional<Tensor> hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tens
                             Tensor k_cache, Tensor v_cache, Tensor o_left, Tensor decay, Tensor state, Tensor norm_right,
                             Tensor o_right, Tensor wa, Tensor wb, Tensor w_post, Tensor w_next, Tensor positions,
                             Tensor slots, Tensor tables, Tensor lens, Tensor state_slots, Tensor cu, Tensor seg_start,
-                            int64_t heads, double scale, int64_t mask_size, double eps) {
+                            int64_t heads, double scale, int64_t mask_size, double eps, bool once) {
   if (!lie_whole({w_in, o_left, o_right, state, wa, wb, w_post, w_next})) return std::nullopt;
   const Rows r(x, h);
   const int T = r.T, W = r.W;
@@ -144,7 +144,7 @@ std::optional<Tensor> hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tens
 
   auto st = cur_stream();
   const auto f32 = x.options();
-  const Tensor y = part(h, w_in, T, st);
+  const Tensor y = part(h, w_in, T, once, st);
   const int KL = H * D, KR = RH * RV;
   auto q = torch::empty({T, (int64_t)KL}, h.options()), head_gate = torch::empty({T, H}, h.options());
   auto both = torch::empty({(int64_t)T * (KL + KR)}, h.options());     // the left branch's rows, then the right one's
@@ -166,12 +166,12 @@ std::optional<Tensor> hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tens
   if (KL == KR) {    // one launch, half as many sums of each: 40 rows, 2048 x 2048 each, 6.2 us, two launches 5.3 each
     const int S = std::max(linear_rows_splits(T, W, 2 * KL) & ~1, 2);
     const Tensor sums = torch::empty({S, T, (int64_t)W}, f32);
-    TORCH_CHECK(launch_linear_rows_two(sums.data_ptr<float>(), bf(both), bf(o_left), bf(o_right), T, W, KL, S, st) == 0, NO_LDS);
+    TORCH_CHECK(launch_linear_rows_two(sums.data_ptr<float>(), bf(both), bf(o_left), bf(o_right), T, W, KL, S, once, st) == 0, NO_LDS);
     left = sums.narrow(0, 0, S / 2);
     right = sums.narrow(0, S / 2, S / 2);
   } else {
-    left = part(both, o_left, T, st);
-    right = part(both.narrow(0, (int64_t)T * KL, (int64_t)T * KR), o_right, T, st);
+    left = part(both, o_left, T, once, st);
+    right = part(both.narrow(0, (int64_t)T * KL, (int64_t)T * KR), o_right, T, once, st);
   }
   auto out = torch::empty_like(h);
   seq_launch_sandwich_rows(x.data_ptr<float>(), left.data_ptr<float>(), left.size(0), right.data_ptr<float>(),
@@ -185,7 +185,7 @@ std::optional<Tensor> hybrid_parallel_rows(Tensor x, Tensor h, Tensor w_in, Tens
 std::optional<Tensor> hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::vector<int64_t> at, Tensor conv, Tensor conv_state, Tensor a2,
                          Tensor g2, Tensor dt_bias, Tensor a_log, Tensor state, Tensor norm, Tensor w_out, Tensor w_post,
                          Tensor w_next, Tensor state_slots, Tensor cu, Tensor seg_start, Tensor token_seg,
-                         int64_t kv_heads, double eps) {
+                         int64_t kv_heads, double eps, bool once) {
   if (!lie_whole({w_in, w_out, w_post, w_next})) return std::nullopt;
   const Rows r(x, h);
   const int T = r.T, W = r.W;
@@ -220,7 +220,7 @@ std::optional<Tensor> hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::ve
   auto yr = torch::empty({T, (int64_t)H * V}, h.options());
   if (lie_whole({a2, g2, state}) && a2.scalar_type() == at::kBFloat16 && g2.scalar_type() == at::kBFloat16 &&
       seq_delta_rows_takes(H, G, D, V, K, a2.size(1), g2.size(1))) {
-    const Tensor y = part(h, w_in, T, st);
+    const Tensor y = part(h, w_in, T, once, st);
     seq_launch_delta_rows(y.data_ptr<float>(), y.size(0), at.data(), conv.data_ptr<float>(), conv_state.data_ptr(), K, C,
                           a2.data_ptr(), a2.size(1), g2.data_ptr(), g2.size(1), dt_bias.data_ptr<float>(),
                           a_log.data_ptr<float>(), state.data_ptr<float>(), norm.data_ptr<float>(), yr.data_ptr(),
@@ -231,7 +231,7 @@ std::optional<Tensor> hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::ve
     // with them from Python, 499 so
     const auto f32 = x.options();
     auto y = torch::empty({T, (int64_t)N}, h.options());
-    TORCH_CHECK(launch_linear_rows(y.data_ptr(), bf(h), bf(w_in), nullptr, T, N, W, W, ROWS_BF16, 1, 0.0f, 0.0f, st) == 0, NO_LDS);
+    TORCH_CHECK(launch_linear_rows(y.data_ptr(), bf(h), bf(w_in), nullptr, T, N, W, W, ROWS_BF16, 1, 0.0f, 0.0f, once, st) == 0, NO_LDS);
     auto c = torch::empty({T, C}, h.options());
     seq_launch_causal_conv_silu(c.data_ptr(), y.data_ptr(), conv.data_ptr<float>(), conv_state.data_ptr(),
                                 state_slots.data_ptr<int>(), cu.data_ptr<int>(), seg_start.data_ptr<int>(),
@@ -248,7 +248,7 @@ std::optional<Tensor> hybrid_delta_rows(Tensor x, Tensor h, Tensor w_in, std::ve
     seq_launch_gated_rmsnorm(yr.data_ptr(), o.data_ptr<float>(), norm.data_ptr<float>(), gate.data_ptr(), T, H, V, H * V,
                              (float)eps, 0, 0, st);
   }
-  const Tensor p = part(yr, w_out, T, st);
+  const Tensor p = part(yr, w_out, T, once, st);
   auto out = torch::empty_like(h);
   seq_launch_sandwich_rows(x.data_ptr<float>(), p.data_ptr<float>(), p.size(0), nullptr, 0, nullptr, nullptr,
                            w_post.data_ptr<float>(), w_next.data_ptr<float>(), out.data_ptr(), T, W, (float)eps, nullptr, 0, 0.0f, st);
@@ -263,7 +263,7 @@ static bool glu_on_rows(int T, int K) { return T <= 64 || (K & (K - 1)) == 0; }
 
 // The same of a clamped gated-linear-unit sublayer, w_in = [gate; up]
 std::optional<Tensor> hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_down, Tensor w_post, Tensor w_next, double limit,
-                       double alpha, double eps) {
+                       double alpha, double eps, bool once) {
   if (!lie_whole({w_in, w_down, w_post, w_next})) return std::nullopt;
   const Rows r(x, h);
   check_weight(w_in, r.W, "w_in");
@@ -276,12 +276,12 @@ std::optional<Tensor> hybrid_glu_rows(Tensor x, Tensor h, Tensor w_in, Tensor w_
   auto act = torch::empty({r.T, N / 2}, h.options());
   if (glu_on_rows(r.T, r.W)) {
     TORCH_CHECK(launch_linear_rows(act.data_ptr(), bf(h), bf(w_in), nullptr, r.T, N, r.W, r.W, ROWS_CLAMPED, 1, (float)limit,
-                                   (float)alpha, st) == 0, NO_LDS);
+                                   (float)alpha, once, st) == 0, NO_LDS);
   } else {
     const Tensor y = at::linear(h, w_in);
     seq_launch_gated_act(act.data_ptr(), y.data_ptr(), bf(y, N / 2), r.T, N / 2, N, (float)limit, (float)alpha, 1.0f, 0, st);
   }
-  const Tensor p = part(act, w_down, r.T, st);
+  const Tensor p = part(act, w_down, r.T, once, st);
   auto out = torch::empty_like(h);
   seq_launch_sandwich_rows(x.data_ptr<float>(), p.data_ptr<float>(), p.size(0), nullptr, 0, nullptr, nullptr,
                            w_post.data_ptr<float>(), w_next.data_ptr<float>(), out.data_ptr(), r.T, r.W, (float)eps, nullptr, 0, 0.0f, st);

@@ -89,3 +89,26 @@ def test_gate_up_product(shape, most):
 
     w = torch.empty(shape, dtype=torch.bfloat16, device="meta")
     assert [LlamaForCausalLM._silu_rows(r, w) for r in (1, 16, 17, 64, 65)] == [r <= most for r in (1, 16, 17, 64, 65)]
+
+
+def test_models_whose_steps_find_no_weights_in_the_cache():
+    """Matrices count, tables and stacks of experts do not; the model says it to the parts that ask."""
+    import torch
+
+    from kllms_amd.engine.config import ModelArchConfig
+    from kllms_amd.models.llama import LlamaForCausalLM
+    from kllms_amd.models.mixtral import MixtralForCausalLM
+
+    m = torch.nn.Module()
+    with torch.device("meta"):
+        m.table = torch.nn.Embedding(1 << 20, 256, dtype=torch.bfloat16)
+        m.experts = torch.nn.Parameter(torch.empty(64, 4096, 4096, dtype=torch.bfloat16), requires_grad=False)
+        m.a = torch.nn.Linear(4096, 20480, bias=False, dtype=torch.bfloat16)
+        m.b = torch.nn.Linear(4096, 20479, bias=False, dtype=torch.bfloat16)
+        assert not ops.weights_once(m)              # 8 KB less than 320 MB
+        m.b = torch.nn.Linear(4096, 20480, bias=False, dtype=torch.bfloat16)
+        assert ops.weights_once(m)
+        sizes = dict(vocab_size=32000, hidden_size=2048, intermediate_size=8192, num_heads=16, num_kv_heads=4, head_dim=128)
+        assert not LlamaForCausalLM(ModelArchConfig(num_layers=1, **sizes))._once      # 249 MB with the head
+        assert LlamaForCausalLM(ModelArchConfig(num_layers=2, **sizes))._once          # 370 MB
+        assert not MixtralForCausalLM(ModelArchConfig(num_layers=2, num_experts=8, **sizes))._once

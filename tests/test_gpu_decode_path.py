@@ -571,12 +571,17 @@ def test_linear_rows_at_the_lines_of_their_tiles(M, N, K):
 @pytest.mark.parametrize("N,K", [(2032, 2048), (2064, 2048), (1984, 2048), (2112, 2048), (32768, 128), (32704, 128)])
 @pytest.mark.parametrize("M", [1, 33, 128, 160])
 def test_linear_rows_around_the_streaming_line(M, N, K):
-    """A little below 8 MB of weights, and from there on, where they pass the caches by: each form, with ragged tiles."""
+    """A little below 8 MB of weights, and from there on, where they pass the caches by if the caller says so: each form, with
+    ragged tiles, and the same bits either way."""
     g = torch.Generator(device=DEV).manual_seed(M + N)
     x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
     w = (torch.randn(N, K, generator=g, device=DEV) * 0.05).bfloat16()
     xd, wt = x.double(), w.double().t().contiguous()
     ref, tol = xd @ wt, K * 2 ** -24 * (xd.abs() @ wt.abs())     # fp32 sums of K products
+    C, none = ops._hip_or_raise(), ops._none(x)
+    for form in range(4):
+        if M <= (384, 128, 128, 256)[form] and (form != 3 or N % 64 == 0):
+            assert torch.equal(C.linear_rows(x, w, none, form, 0, True), C.linear_rows(x, w, none, form, 0))
     assert ((ops.linear_part(x, w).double().sum(0) - ref).abs() <= tol).all()
     if M <= 128:
         got = ops._hip_or_raise().linear_rows(x, w, ops._none(x), 1, 1).double()
@@ -695,6 +700,34 @@ def test_linear_rows_of_repeated_and_overlapping_rows(M, stride, N, K):
         assert ops.linear_rows_ok(x, w)
         assert ((ops.linear_f32(x, w).double() - ref).abs() <= tol).all()
         assert ((C.linear_rows(x, w, none, 1, 1).double() - ref).abs() <= tol + 2 ** -8 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("preset", ["mid-llama", "mid-zutalix"])
+def test_steps_of_weights_that_pass_the_caches_by(preset):
+    """The word of a model of many weights reaches each product of a step and changes none of its bits."""
+    from kllms_amd.engine.config import EngineConfig
+    from kllms_amd.engine.engine import LLMEngine
+
+    out, said = [], []
+    for once in (False, True):
+        eng = LLMEngine(EngineConfig(model=preset, max_kv_blocks=64, use_hip_graphs=False, seed=3))
+        m = eng.model
+        assert not m._once
+        for part in m.modules():
+            for name in ("_once", "once"):
+                if name in part.__dict__:
+                    setattr(part, name, once)
+        saved, rows = ops.linear_part, []
+        ops.linear_part = lambda x, w, o=False: rows.append(o) or saved(x, w, o)
+        try:
+            s = eng.open_sequence()
+            eng.step_segments([(s, list(range(5, 40)), [34])])
+            out.append([eng.step_segments([(s, [7 + i], [0])]) for i in range(2)])
+        finally:
+            ops.linear_part = saved
+        said.append(set(rows))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+    assert said == ([set(), set()] if preset == "mid-zutalix" else [{False}, {True}])
 
 
 @pytest.mark.parametrize("preset", ["mid-llama", "mid-zutalix"])
