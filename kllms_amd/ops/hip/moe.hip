@@ -420,19 +420,22 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(bf16_t* __restrict__ o
   reinterpret_cast<bf16x8_vec*>(out)[(int64_t)t * nvec + i] = o;
 }
 
-// Whether the products load W with the streaming hint, which leaves the caches to x: where the weights of all experts are
-// themselves too large for the 256 MB last-level cache, so that no call finds anything of the one before, and few enough
-// rows go to an expert that its W is read by one row tile, or two. Smaller ones stay in the cache from layer to layer or
-// from call to call in part, and the hint gives that up. us without and with, 8 experts, width and size of an expert:
+// Whether the products load W with the streaming hint, which leaves the caches to x and to act: where the weights of all experts
+// are themselves too large for the 256 MB last-level cache, so that no call finds anything of the one before, and few enough
+// rows go to an expert that its W is read by one or two row tiles. Smaller ones stay in the cache in part from call to call, and
+// the hint gives that up; of many rows act is as large as the cache itself. us plain and with it, 8 experts, width and size of
+// an expert:
 //   gate/up  1024x4096 (134 MB), 1024 tokens, 2 choices 58, 61   2048x4096 (268 MB) alone 4 tokens 36, 37; 600 56, 58
 //            2048x6144 (402 MB) 32 tokens 84, 80; 800 113, 112   2048x8192 (537 MB) 4 tokens 85, 81; 300 117, 107; 800 131, 127
-//            4096x14336 (1879 MB) 32 tokens 341, 316; 800 422, 417
-//     but with 256 rows an expert and more 2048x8192 168, 171; 4096x14336 532, 539; 2048x6144, 512 rows 213, 217
+//              but 1024 168, 171; 2048 270, 273      4096x14336 (1879 MB) 32 tokens 341, 316; 800 422, 417
 //   down     2048x4096 (134 MB) alone 32 tokens 32, 54; 1024 73, 93   2048x6144 (201 MB) 2048 tokens 141, 157
-//            4096x7168 (470 MB) 4 tokens 96, 93; 300 124, 120; 1024 175, 172   4096x14336 (940 MB) 2048 tokens 564, 558
+//            4096x7168 (470 MB) 4 tokens 96, 93; 300 124, 120; 1024 175, 172
+//   both     4096x7168 600 tokens 317, 301; 1600 549, 542; 2048 699, 694; 3000 922, 938
+//            4096x14336 150 523, 507; 1024 884, 867; 2048 1321, 1309; 3000 1766, 1796; 6000 3212, 3271
 #define MOE_ONCE_BYTES ((int64_t)320 << 20)
 static bool moe_once(bool gateup, int64_t S, int64_t E, int64_t N, int64_t K) {
-  return E * (gateup ? 2 : 1) * N * K * 2 >= MOE_ONCE_BYTES && S <= E * (gateup ? 224 : 512);
+  const int64_t bytes = E * (gateup ? 2 : 1) * N * K * 2;
+  return bytes >= MOE_ONCE_BYTES && S <= E * (gateup && bytes < 2 * MOE_ONCE_BYTES ? 224 : 512);
 }
 
 // rows S in sorted space; the grid holds the most tiles that S rows of E experts can make
