@@ -108,7 +108,7 @@ class LlamaAttention(nn.Module):
         if paged is not None and k_scale is None:
             plan, short = paged
             return ops.attn_segments_paged(q, k_cache, v_cache, batch.block_tables, batch.context_lens, self.scale,
-                                           plan, short, batch.seg_tables, batch.seg_start, batch.plans.get("few", False))
+                                           plan, short, batch.seg_tables, batch.seg_start)
         return ops.attn_decode_paged(
             q, k_cache, v_cache, batch.block_tables, batch.context_lens, self.scale,
             k_scale, v_scale, arrived,
@@ -419,10 +419,10 @@ class LlamaForCausalLM(nn.Module):
                 and self.layers and self.layers[0].self_attn.head_dim == 128
                 and ops.paged_prefill_pays(batch.host_segs, self.layers[0].self_attn.num_kv_heads)):
             at = self.layers[0].self_attn
-            few = hasattr(at, "num_heads") and ops.paged_prefill_few(batch.host_segs, at.num_heads)
-            plan, short = ops.paged_prefill_plan(batch.host_segs, input_ids.device, *([64] if few else []))
+            rows = 64 if ops.paged_prefill_few(batch.host_segs, at.num_heads) else 256
+            plan, short = ops.paged_prefill_plan(batch.host_segs, input_ids.device, rows)
             if plan is not None:
-                return replace(batch, plans={**(batch.plans or {}), "paged": (plan, short), "few": few})
+                return replace(batch, plans={**(batch.plans or {}), "paged": (plan, short)})
         return batch
 
     def forward_hidden(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:

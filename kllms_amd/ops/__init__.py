@@ -15,7 +15,7 @@ from __future__ import annotations
 
 import heapq
 import os
-from typing import Optional, Sequence, Tuple
+from typing import NamedTuple, Optional, Sequence, Tuple
 
 import torch
 
@@ -206,9 +206,15 @@ def paged_prefill_few(segs, heads: int) -> bool:
     return cost(64) < cost(256)
 
 
+class PagedGroups(NamedTuple):
+    """Groups of up to ``rows`` (64 or 256) rows of segments, [4, G] on the device: the kernel is the one of that size."""
+    groups: torch.Tensor
+    rows: int
+
+
 def paged_prefill_plan(segs, device, rows: int = 256) -> tuple:
-    """(groups [4, G] of up to ``rows`` rows on the device, [(first row, rows)] left to row-by-row attention) for segments
-    [(start position, rows)] packed in that order; groups None when every segment is short."""
+    """(PagedGroups, [(first row, rows)] left to row-by-row attention) for segments [(start position, rows)] packed in that
+    order; None for the groups when every segment is short."""
     groups, short, row = [], [], 0
     for i, (_, n) in enumerate(segs):
         if n >= PAGED_PREFILL_ROWS:
@@ -220,15 +226,15 @@ def paged_prefill_plan(segs, device, rows: int = 256) -> tuple:
         row += n
     # the groups that see most first
     groups.sort(key=lambda g: -(segs[g[3]][0] + g[2]))
-    plan = upload(torch.tensor(groups, dtype=torch.int32).t().contiguous(), device) if groups else None
-    return plan, short
+    if not groups:
+        return None, short
+    return PagedGroups(upload(torch.tensor(groups, dtype=torch.int32).t().contiguous(), device), rows), short
 
 
-def attn_segments_paged(q, k_cache, v_cache, block_tables, context_lens, scale, plan, short, seg_tables, seg_start, few=False):
-    """Rows of long segments on the matrix cores against the paged bf16 cache, the others row by row (GPU only). ``few``: the
-    plan's groups are of 64 rows."""
+def attn_segments_paged(q, k_cache, v_cache, block_tables, context_lens, scale, plan, short, seg_tables, seg_start):
+    """Rows of long segments on the matrix cores against the paged bf16 cache, the others row by row (GPU only)."""
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    _hip_or_raise().attn_prefill_paged(out, q, k_cache, v_cache, plan, seg_tables, seg_start, scale, few)
+    _hip_or_raise().attn_prefill_paged(out, q, k_cache, v_cache, plan.groups, seg_tables, seg_start, scale, plan.rows)
     f = _none(q, torch.float32)
     for r, n in short:
         _hip_or_raise().attn_decode_paged(out[r:r + n], q[r:r + n], k_cache, v_cache, block_tables[r:r + n],

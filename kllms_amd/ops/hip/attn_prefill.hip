@@ -401,13 +401,13 @@ extern "C" int launch_attn_prefill(bf16_t* out, const bf16_t* q, const bf16_t* k
   return 0;
 }
 
-// few: groups of 64 rows
+// rows: of a group, 64 or 256
 extern "C" int launch_attn_prefill_paged(bf16_t* out, const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache,
                                          const int* grp_start, const int* grp_len, const int* grp_q0,
                                          const int* grp_seg, const int* block_tables, const int* seg_pos, int ngroups,
                                          float scale, int num_q_heads, int num_kv_heads, int q_tstride,
-                                         int block_size, int max_blocks, int few, hipStream_t stream) {
-  const auto kernel = few ? attn_prefill_kernel<true, true> : attn_prefill_kernel<true, false>;
+                                         int block_size, int max_blocks, int rows, hipStream_t stream) {
+  const auto kernel = rows == 64 ? attn_prefill_kernel<true, true> : attn_prefill_kernel<true, false>;
   if (!prefill_lds_ready(reinterpret_cast<const void*>(kernel))) return -1;
   const uint32_t inverse = block_size > 1 ? (uint32_t)(((1ull << 32) + block_size - 1) / block_size) : ~0u;
   for (int g = 0; g < ngroups; g += MAX_GROUPS)

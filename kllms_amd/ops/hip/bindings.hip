@@ -235,9 +235,9 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k, torch::Te
 
 // rows of segments against the paged cache (bf16): plan [4, G] int32 (first row, rows, first row within the
 // segment, segment), tables [n, MAXB], pos [n] = position of each segment's first row. The segments' own keys and
-// values are in the cache already. few: the plan's groups are of 64 rows.
+// values are in the cache already. rows: of the plan's groups, 64 or 256.
 void attn_prefill_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache, torch::Tensor v_cache,
-                        torch::Tensor plan, torch::Tensor tables, torch::Tensor pos, double scale, bool few) {
+                        torch::Tensor plan, torch::Tensor tables, torch::Tensor pos, double scale, int64_t rows) {
   CHECK_BF16_CONTIG(out); CHECK_BF16_ROWS(q); CHECK_BF16_CONTIG(k_cache); CHECK_BF16_CONTIG(v_cache);
   const int H = q.size(1), KVH = k_cache.size(1), BS = k_cache.size(2);
   TORCH_CHECK(q.size(2) == 128 && k_cache.size(3) == 128 && v_cache.sizes() == k_cache.sizes() && H % KVH == 0,
@@ -246,13 +246,14 @@ void attn_prefill_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cach
                   plan.size(0) == 4 && tables.is_cuda() && tables.is_contiguous() && tables.scalar_type() == at::kInt &&
                   tables.dim() == 2 && pos.is_cuda() && pos.is_contiguous() && pos.scalar_type() == at::kInt &&
                   pos.numel() == tables.size(0), "attn_prefill_paged: plan, tables or positions");
+  TORCH_CHECK(rows == 64 || rows == 256, "attn_prefill_paged: groups of 64 or 256 rows");
   const int G = plan.size(1);
   if (G == 0) return;
   if (!rows_aligned(q)) q = q.contiguous();
   const int* p = plan.data_ptr<int>();
   TORCH_CHECK(launch_attn_prefill_paged(bf(out), cbf(q), cbf(k_cache), cbf(v_cache), p, p + G, p + 2 * G, p + 3 * G,
                                         tables.data_ptr<int>(), pos.data_ptr<int>(), G, (float)scale, H, KVH, (int)q.stride(0),
-                                        BS, (int)tables.size(1), few, cur_stream()) == 0,
+                                        BS, (int)tables.size(1), (int)rows, cur_stream()) == 0,
               "attn_prefill_paged: 128 KB of LDS are not available");
 }
 
@@ -755,7 +756,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill", &attn_prefill);
   m.def("attn_prefill_plan", &attn_prefill_plan);
   m.def("attn_prefill_paged", &attn_prefill_paged, py::arg("out"), py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
-        py::arg("plan"), py::arg("tables"), py::arg("pos"), py::arg("scale"), py::arg("few") = false);
+        py::arg("plan"), py::arg("tables"), py::arg("pos"), py::arg("scale"), py::arg("rows") = 256);
   m.def("sample", &sample);
   m.def("mfma_selftest", &mfma_selftest);
   m.def("one_shot_allreduce", &one_shot_allreduce);

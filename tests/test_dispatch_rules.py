@@ -50,7 +50,8 @@ def test_shares_of_a_context(rows, kv_heads, group, keys, fp8, most):
 
 
 def test_one_short_portion_behind_a_long_cache_goes_row_by_row(monkeypatch):
-    """The model asks the rule: a step of one 32-row portion has no plan, one of eight has."""
+    """The model asks the rules: a step of one 32-row portion has no plan, one of eight has, and its groups are as large as the
+    other rule says."""
     import torch
 
     from kllms_amd.models.llama import ForwardBatch, LlamaForCausalLM
@@ -60,14 +61,14 @@ def test_one_short_portion_behind_a_long_cache_goes_row_by_row(monkeypatch):
     model.dtype = torch.bfloat16
 
     class Attn:
-        head_dim, num_kv_heads = 128, 8
+        head_dim, num_heads, num_kv_heads = 128, 32, 8
 
     class Layer(torch.nn.Module):
         self_attn = Attn
 
     model.layers = torch.nn.ModuleList([Layer()])
     monkeypatch.setattr(ops, "_force_torch", lambda: False)
-    monkeypatch.setattr(ops, "paged_prefill_plan", lambda segs, device: ("plan", []))
+    monkeypatch.setattr(ops, "paged_prefill_plan", lambda segs, device, rows=256: (("plan", rows), []))
 
     class Ids:
         is_cuda, device = True, "cpu"
@@ -78,7 +79,8 @@ def test_one_short_portion_behind_a_long_cache_goes_row_by_row(monkeypatch):
         return (LlamaForCausalLM._planned(model, Ids, batch).plans or {}).get("paged")
 
     assert planned([(6000, 32)]) is None
-    assert planned([(1536, 150)] * 8) == ("plan", [])
+    assert planned([(1536, 150)] * 8) == (("plan", 256), [])
+    assert planned([(1536, 150)] * 2) == (("plan", 64), [])
 
 
 @pytest.mark.parametrize("shape,most", [((1024, 512), 64), ((28672, 4096), 64), ((27648, 5120), 16), ((57344, 8192), 0)])

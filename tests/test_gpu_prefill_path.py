@@ -87,8 +87,7 @@ def test_segments_against_cache(H, G, BS, segs, few):
     if plan is None:
         return
     out = ops.attn_segments_paged(q, kc.to(DEV), vc.to(DEV), bt[row_seg].to(DEV), ctx.to(DEV), D ** -0.5, plan, short,
-                                  bt.to(DEV), torch.tensor([s for s, _ in segs], dtype=torch.int32).to(DEV),
-                                  few)
+                                  bt.to(DEV), torch.tensor([s for s, _ in segs], dtype=torch.int32).to(DEV))
     r = 0
     for i, (s, n) in enumerate(segs):
         at = torch.arange(s + n)
@@ -98,7 +97,7 @@ def test_segments_against_cache(H, G, BS, segs, few):
 
 
 @pytest.mark.parametrize("rows", [[40, 20], [150, 1, 33], [300]])
-def test_step_segments_matches_row_by_row(rows):
+def test_step_segments_matches_row_by_row(rows, cached=37):
     """Portions behind a cached head through LLMEngine.step_segments, every row's logits, against the same step with
     each row attending alone."""
     from kllms_amd.engine.config import EngineConfig
@@ -110,7 +109,7 @@ def test_step_segments_matches_row_by_row(rows):
     def step(alone):
         eng.model._planned = (lambda ids, batch: batch) if alone else type(eng.model)._planned.__get__(eng.model)
         seqs = [eng.open_sequence() for _ in rows]
-        heads = [torch.randint(0, 2000, (37 + 11 * i,), generator=torch.Generator().manual_seed(i)).tolist()
+        heads = [torch.randint(0, 2000, (cached + 11 * i,), generator=torch.Generator().manual_seed(i)).tolist()
                  for i in range(len(rows))]
         eng.step_segments([(s, h, []) for s, h in zip(seqs, heads)])
         out = eng.step_segments([(s, t, list(range(len(t)))) for s, t in zip(seqs, toks)])
@@ -306,7 +305,7 @@ def test_more_segments_than_a_grid_has_in_y():
     pos = torch.zeros(n, dtype=torch.int32, device=DEV)
     q = torch.randn(n * rows, 1, D, generator=g, device=DEV).bfloat16()
     plan, short = ops.paged_prefill_plan([(0, rows)] * n, DEV)
-    assert plan.shape[1] == n and not short
+    assert plan.groups.shape[1] == n and not short
     out = ops.attn_segments_paged(q, kc, vc, None, None, 0.1, plan, short, tables, pos)
     for lo, hi in ((0, 200), (n - 200, n)):
         part, _ = ops.paged_prefill_plan([(0, rows)] * (hi - lo), DEV)
@@ -317,7 +316,8 @@ def test_more_segments_than_a_grid_has_in_y():
 
 @pytest.mark.parametrize("rows", [32, 65, 300])
 @pytest.mark.parametrize("at", [1, 40, 100])          # the second key beside the first, in the other half, in another tile
-def test_segments_against_cache_keep_32_bit_probabilities(at, rows):
+@pytest.mark.parametrize("group", [64, 256])
+def test_segments_against_cache_keep_32_bit_probabilities(at, rows, group):
     """Two keys of nearly the same score and V of opposite sign: the result is the difference of their probabilities,
     2^-14 to 2^-8 of them, and an error of P shows in it at full size."""
     start, G, rep, BS = 128, 2, 4, 16
@@ -334,7 +334,7 @@ def test_segments_against_cache_keep_32_bit_probabilities(at, rows):
     q[..., 1] = torch.randint(1, 65, (rows, G * rep), generator=g) * 2.0 ** -10
     cache = [t.view(NB, BS, G, D).transpose(1, 2).contiguous().bfloat16().to(DEV) for t in (k, v)]
     bt = torch.arange(NB, dtype=torch.int32, device=DEV).view(1, NB)
-    plan, short = ops.paged_prefill_plan([(start, rows)], DEV)
+    plan, short = ops.paged_prefill_plan([(start, rows)], DEV, group)
     assert plan is not None and not short
     out = ops.attn_segments_paged(q.bfloat16().to(DEV), *cache, None, None, 1.0, plan, [], bt,
                                   torch.tensor([start], dtype=torch.int32, device=DEV))
@@ -413,6 +413,23 @@ def test_step_segments_together_matches_row_by_row(rows, monkeypatch):
     monkeypatch.setattr(LlamaForCausalLM, "_planned", planned)
     test_step_segments_matches_row_by_row(rows)
     assert plans[-1] is not None and plans[-1][0] is not None
+
+
+# group: the size that the rules choose
+@pytest.mark.parametrize("rows,cached,group", [([400], 37, 256), ([150] * 3, 300, 256), ([400], 600, 64), ([129, 1, 300, 20], 1000, 64)])
+def test_step_segments_of_either_group_size_match_row_by_row(rows, cached, group, monkeypatch):
+    from kllms_amd.models.llama import LlamaForCausalLM
+
+    plans, make = [], LlamaForCausalLM._planned
+
+    def planned(self, ids, batch):
+        batch = make(self, ids, batch)
+        plans.append((batch.plans or {}).get("paged"))
+        return batch
+
+    monkeypatch.setattr(LlamaForCausalLM, "_planned", planned)
+    test_step_segments_matches_row_by_row(rows, cached)
+    assert plans[-1][0].rows == group
 
 
 @pytest.mark.parametrize("T", [1, 15, 16, 17, 255, 256, 257, 4113])
