@@ -204,6 +204,9 @@ static bool rows_aligned(const torch::Tensor& t) {  // 16-byte row loads
   return t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 
+// rows of their own: also of a contiguous tensor that begins off 16 bytes, which contiguous() gives as it is
+static torch::Tensor own_rows(const torch::Tensor& t) { return t.clone(at::MemoryFormat::Contiguous); }
+
 // groups of 256 rows of the packed sequences cu [n + 1] over T rows: [3, G] (start, length, first row)
 torch::Tensor attn_prefill_plan(torch::Tensor cu, int64_t T) {
   TORCH_CHECK(cu.is_cuda() && cu.is_contiguous() && cu.scalar_type() == at::kInt && cu.numel() >= 1);
@@ -225,8 +228,8 @@ void attn_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k, torch::Te
                   plan.size(0) == 3, "plan must come from attn_prefill_plan");
   const int G = plan.size(1);
   if (G == 0) return;
-  if (!rows_aligned(q)) q = q.contiguous();
-  if (!rows_aligned(k) || !rows_aligned(v)) { k = k.contiguous(); v = v.contiguous(); }
+  if (!rows_aligned(q)) q = own_rows(q);
+  if (!rows_aligned(k) || !rows_aligned(v)) { k = own_rows(k); v = own_rows(v); }
   const int* p = plan.data_ptr<int>();
   TORCH_CHECK(launch_attn_prefill(bf(out), cbf(q), cbf(k), cbf(v), p, p + G, p + 2 * G, 1, G, (float)scale, H, KVH,
                                   (int)q.stride(0), (int)k.stride(0), cur_stream()) == 0,
@@ -249,7 +252,9 @@ void attn_prefill_paged(torch::Tensor out, torch::Tensor q, torch::Tensor k_cach
   TORCH_CHECK(rows == 64 || rows == 256, "attn_prefill_paged: groups of 64 or 256 rows");
   const int G = plan.size(1);
   if (G == 0) return;
-  if (!rows_aligned(q)) q = q.contiguous();
+  if (!rows_aligned(q)) q = own_rows(q);
+  if (!rows_aligned(k_cache)) k_cache = own_rows(k_cache);
+  if (!rows_aligned(v_cache)) v_cache = own_rows(v_cache);
   const int* p = plan.data_ptr<int>();
   TORCH_CHECK(launch_attn_prefill_paged(bf(out), cbf(q), cbf(k_cache), cbf(v_cache), p, p + G, p + 2 * G, p + 3 * G,
                                         tables.data_ptr<int>(), pos.data_ptr<int>(), G, (float)scale, H, KVH, (int)q.stride(0),

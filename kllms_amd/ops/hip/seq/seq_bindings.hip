@@ -509,6 +509,13 @@ void attn_varlen_mfma(torch::Tensor out, torch::Tensor q, torch::Tensor k, torch
   const int ngroups = grp_start.numel();
   TORCH_CHECK(grp_qpos0.numel() == (int64_t)ngroups * 8 && grp_len.numel() == ngroups);
   if (ngroups == 0) return;
+  // keys and values go to LDS 16 bytes at a time
+  const auto off_16 = [](const torch::Tensor& t) { return t.stride(0) % 8 || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16; };
+  if (off_16(q)) q = q.clone(at::MemoryFormat::Contiguous);
+  if (off_16(k) || off_16(v)) {
+    k = k.clone(at::MemoryFormat::Contiguous);
+    v = v.clone(at::MemoryFormat::Contiguous);
+  }
   TORCH_CHECK(launch_attn_prefill((__hip_bfloat16*)out.data_ptr(), (const __hip_bfloat16*)q.data_ptr(),
                                   (const __hip_bfloat16*)k.data_ptr(), (const __hip_bfloat16*)v.data_ptr(),
                                   grp_start.data_ptr<int>(), grp_len.data_ptr<int>(), grp_qpos0.data_ptr<int>(), 8, ngroups,

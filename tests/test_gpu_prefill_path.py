@@ -265,6 +265,39 @@ def test_mixture_products_of_views_off_16_bytes():
     assert torch.equal(act, act2) and torch.equal(y, y2)
 
 
+@pytest.mark.parametrize("which", ["q", "kv", "all"])
+@pytest.mark.parametrize("stride,at", [(0, 1), (0, 4), (4, 0), (12, 8), (2, 3)])      # elements between rows' ends, and before the first
+def test_prompt_attention_of_rows_off_16_bytes(which, stride, at):
+    """Contiguous rows that begin off 16 bytes, and rows whose stride takes them off: the copies' results, bit by bit, in whole
+    prompts, in tables of pieces and against a paged cache."""
+    T, H, G, BS = 300, 4, 2, 16
+    g = torch.Generator(device=DEV).manual_seed(stride + at)
+    q, k, v = (torch.randn(T, h, D, generator=g, device=DEV).bfloat16() for h in (H, G, G))
+
+    def off(t):
+        row = t[0].numel() + stride
+        flat = torch.zeros(T * row + at, device=DEV, dtype=t.dtype)[at:]
+        return flat.as_strided((T, t.shape[1], D), (row, D, 1)).copy_(t)
+
+    moved = [off(t) if which == "all" or (which == "q") == (t is q) else t for t in (q, k, v)]
+    cu = torch.tensor([0, 41, T], dtype=torch.int32, device=DEV)
+    pieces = ops.dense_tile_groups([(0, 41), (41, T - 41)], torch.device(DEV))
+    got = []
+    for a, b, c in ((q, k, v), moved):
+        out = torch.zeros_like(q)
+        ops.attn_varlen_mfma(out, a, b, c, *pieces, 0.1)
+        got.append((ops.attn_prefill_varlen(a, b, c, cu, 0.1), out))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and torch.isfinite(got[0][1]).all()
+    NB = (T + BS - 1) // BS
+    cache = [torch.randn(NB, G, BS, D, generator=g, device=DEV).bfloat16() for _ in range(2)]
+    other = [torch.zeros(t.numel() + at, device=DEV, dtype=t.dtype)[at:].view_as(t).copy_(t) for t in cache]
+    plan, _ = ops.paged_prefill_plan([(0, T)], DEV)
+    tables, pos = torch.arange(NB, dtype=torch.int32, device=DEV).view(1, NB), torch.zeros(1, dtype=torch.int32, device=DEV)
+    a = ops.attn_segments_paged(q, *cache, None, None, 0.1, plan, [], tables, pos)
+    b = ops.attn_segments_paged(moved[0], *(cache if which == "q" else other), None, None, 0.1, plan, [], tables, pos)
+    assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("T,H", [(65535, 8), (65536, 64), (70001, 2056)])
 def test_mixture_of_more_rows_than_a_grid_has_in_y(T, H):
     g = torch.Generator(device=DEV).manual_seed(T)
