@@ -316,8 +316,8 @@ __global__ void __launch_bounds__(64 * NWAVES) attn_prefill_kernel(
   ask_blocks(STAGE);
   int buf = 0;
   for (int ks = 0; ks < kv_end_grp; ks += STAGE, buf ^= 1) {
-    // this stage is there, and the last one's buffer is free
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    // this stage is there, and the last one's buffer, whose reads have come back, is free
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (ks + STAGE < kv_end_grp) {
       stage(ks + STAGE, buf ^ 1);
       ask_blocks(ks + 2 * STAGE);
