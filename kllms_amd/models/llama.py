@@ -375,7 +375,8 @@ class LlamaForCausalLM(nn.Module):
 
     def _forward_rows(self, input_ids: torch.Tensor, batch: ForwardBatch) -> torch.Tensor:
         """A decode step or a short prompt: weights streamed by the few-row kernel, whose split sums go straight into the
-        next row-wise kernel: 8 launches a layer, one more where gate/up is the library's. A prompt's fused projection stays whole: its attention reads the keys and values as rows."""
+        next row-wise kernel: 8 launches a layer, one more where gate/up is the library's. A prompt's fused projection stays
+        whole: its attention reads the keys and values as rows."""
         layers, norm, once = self.layers, self.layers[0].input_layernorm, self._once
         T = input_ids.shape[0]
         if batch.mode == "decode":

@@ -31,8 +31,9 @@
 //
 // Measured in graphs, 32 heads / 8 kv heads, against rows read as fragments, P V on the vector unit and merges in a launch of
 // their own, us, without the streaming hint (DECODE_ONCE): 120 streams, five to a prompt, of 560 keys 33.5, 25.1; 40, eight to
-// a prompt, of 2000 41, 28; prompts of their own: 128 streams of 700 77, 71 (5.5 TB/s), 24 of 2500 48.6, 42.4; 16 fp8 streams of 6000 45.5, 40; 5 streams of 560 8.4, 7.4;
-// 16 / 4 heads, one of 150 7.5, 5.6; block-local, 100 rows of 600, 16 / 4 heads 15.5, 11.5.
+// a prompt, of 2000 41, 28; prompts of their own: 128 streams of 700 77, 71 (5.5 TB/s), 24 of 2500 48.6, 42.4; 16 fp8 streams of
+// 6000 45.5, 40; 5 streams of 560 8.4, 7.4; 16 / 4 heads, one of 150 7.5, 5.6; block-local, 100 rows of 600, 16 / 4 heads 15.5,
+// 11.5.
 //
 // Without groups of heads P V is a quarter of the vector work, and stays on the vector unit: a lane loads the V rows of the keys
 // whose scores it has, P is where it is needed, and V needs no strip. 8 / 8 heads, us with the fragments' own loads, by way of the
