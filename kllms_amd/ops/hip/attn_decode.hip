@@ -82,22 +82,23 @@ __device__ __forceinline__ int first_key(int L, int mask_size) {
 
 // How many workgroups share a context of so many rounds of four tiles, a tile for each wave (attn_decode_shares): one up to
 // ``few`` rounds. Above, the last of ``most`` from whose ``from`` on it is, no more than ``lo`` or one for every ``per`` rounds,
-// and of those as many as are all equally long.
+// and of those as many as are all equally long. ``near``: the least of ``most`` for a context whose prompt a neighbour shares.
 struct DecodeShares {
-  int few, lo, per, most[3], from[3];
+  int few, lo, per, most[3], from[3], near;
   int grid;                  // of no context more
   bool joined;               // merged in the same launch
 };
-__host__ __device__ __forceinline__ int most_of(int rounds, const DecodeShares& s) {
+__host__ __device__ __forceinline__ int most_of(int rounds, const DecodeShares& s, bool shared) {
   int z = (rounds + s.per - 1) / s.per, most = rounds >= s.from[1] ? s.most[1] : s.most[0];
   most = rounds >= s.from[2] ? s.most[2] : most;
   z = z < s.lo ? s.lo : z;
-  return z < most ? z : most;
+  z = z < most ? z : most;
+  return shared && z < s.near ? s.near : z;
 }
-__host__ __device__ __forceinline__ int shares_of(int tiles, const DecodeShares& s) {
+__host__ __device__ __forceinline__ int shares_of(int tiles, const DecodeShares& s, bool shared) {
   const int rounds = (tiles + 3) / 4;
   if (rounds <= s.few) return 1;
-  const int z = most_of(rounds, s), each = (rounds + z - 1) / z;
+  const int z = most_of(rounds, s, shared), each = (rounds + z - 1) / z;
   return (rounds + each - 1) / each;
 }
 
@@ -591,17 +592,17 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : GQA == 1 && KV != KV_FP8_A
   __shared__ float m_lds[4][GQA], l_lds[4][GQA];
   const int b = blockIdx.y;
   const bool after = b > 0, ahead = b + 1 < rows;
-  int L = context_lens[b], own = 0, prev = 0, next = 0;
+  int L = context_lens[b];
+  bool shared = false;                     // the neighbours' first blocks are this context's: so are more, and lie in the L2
   if constexpr (!LOCAL) {                  // beside the length, not behind it
     const int* bt = block_tables + (int64_t)b * max_blocks;
-    own = bt[0];
-    prev = bt[after ? -max_blocks : 0];
-    next = bt[ahead ? max_blocks : 0];
+    int own = bt[0], prev = bt[after ? -max_blocks : 0], next = bt[ahead ? max_blocks : 0];
     asm volatile("" : "+s"(L), "+s"(own), "+s"(prev), "+s"(next));
+    shared = (after && prev == own) || (ahead && next == own);
   }
   const int first = first_key(L, mask_size);
   const int tiles = (L - first + TKEYS - 1) / TKEYS;
-  const int Z = shares_of(tiles, shares);
+  const int Z = shares_of(tiles, shares, GQA == 1 && shared);
   if ((int)blockIdx.z >= Z) return;
 #define DECODE_SHARE(ONCE)                                                                                                    \
   decode_share<GQA, KV, LOCAL, ONCE>(partials, out, q, k_cache, v_cache, k_scale, v_scale, block_tables, context_lens, gate,   \
@@ -609,7 +610,6 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : GQA == 1 && KV != KV_FP8_A
                                      shares, L, first, tiles, Z, strips, m_lds, l_lds)
   // both sides whole: with the loops alone twice in one body it spilled registers
   if constexpr (!LOCAL) {
-    const bool shared = (after && prev == own) || (ahead && next == own);
     if (!shared && (int64_t)L * rows * gridDim.x * (KV == KV_BF16 ? 512 : 256) >= DECODE_ONCE) {
       DECODE_SHARE(true);
       return;
@@ -634,6 +634,9 @@ __global__ __launch_bounds__(NTHREADS, GQA == 8 ? 2 : GQA == 1 && KV != KV_FP8_A
 //   fp8   5 of 7800 240 22.4   320 22.9   440 20.9   640 23.4      16 / 4, 40 of 1500 160 21.1   320 20.3   480 17.8   640 19.6
 //     7 of 7000 392 25.3   728 27.2      30 of 600 240 12.2   480 13.5
 //   8 / 8   5 of 700 to 7800 240 23.0   440 24.8   fp8 240 19.5   440 16.0 (the lengths of one launch differ: 16.1 with 640 of all)
+// Without groups of heads a context whose prompt a neighbour shares is read from the L2, and bound by its rounds: it has two to
+// three workgroups a unit at any length (near). 8 / 8 and 16 / 16 heads, us by the rule for the others and so: 11 streams of 1097 12.9,
+// 10.2; 7 of 1814 17.5, 13.9; fp8, 15 of 1064 12.0, 10.6; over 65 sizes 4 % less. With groups it gains nothing (4) or little (2).
 // Counted over the launch's lengths by each workgroup, so that all are equally long, they took 0.6 us more and gained nothing.
 // A merge in its own launch takes 1 us more, but many partials of eight heads take a single workgroup longer. 8 / 1 heads, one
 // of 500 7.8, in a launch of its own 8.4; of 7800 12.1, 11.0; of 32768 19.0, 14.5; of 131072 32.1, 22.5: so where tables are long.
@@ -642,6 +645,14 @@ static DecodeShares attn_decode_shares(int B, int num_kv_heads, int gqa, int max
   if (gqa == 8 && pairs <= 2 && max_ctx > 16384) joined = false;
   DecodeShares s;
   s.joined = joined;
+  s.near = 0;
+  if (joined && !local && gqa == 1 && pairs <= 256) {        // of two to three workgroups a unit what fills the units best
+    double best = 0.0;
+    for (int64_t z = 512 / pairs; z <= 768 / pairs; ++z) {
+      const double fill = (double)(pairs * z) / ((pairs * z + 255) / 256 * 256);
+      if (fill >= best) best = fill, s.near = (int)z;
+    }
+  }
   s.few = joined ? 3 : local ? 1 : 2;
   if (pairs <= 256) {
     s.lo = joined ? 32 : 48;
@@ -667,7 +678,7 @@ static DecodeShares attn_decode_shares(int B, int num_kv_heads, int gqa, int max
     }
   }
   const int rounds = (int)(((int64_t)max_ctx + 4 * TKEYS - 1) / (4 * TKEYS));
-  s.grid = rounds <= s.few ? 1 : std::min(most_of(rounds, s), rounds);
+  s.grid = rounds <= s.few ? 1 : std::min(most_of(rounds, s, true), rounds);
   return s;
 }
 
@@ -689,7 +700,7 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int L = context_lens[b];
   const int tiles = (L - first_key(L, mask_size) + TKEYS - 1) / TKEYS;
-  const int n = shares_of(tiles, shares);
+  const int n = shares_of(tiles, shares, false);     // not joined: near is 0
   if (n == 1) return;                    // its one workgroup has written the result
   const float* base = partials + (((int64_t)b * (num_q_heads / gqa) + g_kv) * Z * gqa + g) * PART_STRIDE;
   const int64_t step = (int64_t)gqa * PART_STRIDE;

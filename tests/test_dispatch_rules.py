@@ -38,6 +38,7 @@ def test_groups_of_portions(segs, heads, few):
     (1, 8, 4, 384, 0, 1), (1, 8, 4, 512, 0, 4), (1, 8, 4, 2048, 0, 16), (2, 8, 4, 8192, 0, 16), (5, 8, 4, 8192, 0, 12),
     (1, 8, 4, 32768, 0, 32), (1, 4, 4, 131072, 0, 64), (1, 1, 4, 131072, 0, 64), (1, 1, 8, 131072, 0, 128),    # few long contexts
     (20, 8, 4, 8192, 0, 3), (20, 8, 4, 1000, 0, 1), (20, 8, 4, 1000, 1, 3), (40, 8, 4, 8192, 0, 3), (128, 8, 4, 8192, 0, 1),
+    (11, 8, 1, 1024, 0, 8), (21, 8, 1, 1024, 1, 3), (21, 8, 2, 1024, 1, 3), (11, 8, 2, 1024, 0, 2),     # room for contexts that share a prompt
 ])
 def test_shares_of_a_context(rows, kv_heads, group, keys, fp8, most):
     """Few contexts fill the chip also where they are long; no more partials than fit 1024 workgroups' room."""

@@ -75,7 +75,7 @@ def test_paged_decode_tiles(gqa, KVH, BS, ctx, width, fp8):
 @pytest.mark.parametrize("joined", [True, False])
 # and, with 8 kv heads and 8 streams, the line from which the cache is streamed (512 keys, in fp8 1024), unless blocks are shared
 @pytest.mark.parametrize("gqa,KVH,BS,fp8", [(1, 3, 16, False), (2, 2, 1, True), (4, 4, 16, False), (4, 8, 4, True), (4, 2, 6, True),
-                                            (8, 1, 16, False), (8, 2, 32, True), (4, 8, 16, False)])
+                                            (8, 1, 16, False), (8, 2, 32, True), (4, 8, 16, False), (1, 8, 16, True), (1, 16, 8, False)])
 @pytest.mark.parametrize("ctx", [[384], [385, 1, 33], [1024, 1025, 31, 32], [2048, 2049, 640, 641, 5], [4200, 90],
                                  [513 + 17 * i for i in range(70)], [600, 512, 511, 512, 1024, 1023, 513, 1200]])
 def test_shared_contexts(ctx, gqa, KVH, BS, fp8, joined):
