@@ -38,8 +38,13 @@
 // Without groups of heads P V is a quarter of the vector work, and stays on the vector unit: a lane loads the V rows of the keys
 // whose scores it has, P is where it is needed, and V needs no strip. 8 / 8 heads, us with the fragments' own loads, by way of the
 // matrix cores and so: one stream of 2000 8.0, 8.8, 7.2; 16 of 2000 31.9, 25.3, 24.8; 40 of 500 22.1, 19.9, 18.2; fp8: one of 2000
-// 7.2, 8.4, 7.0; 40 of 500 14.0, 14.1, 12.6; 120 of 20, which is four waves to a SIMD or three 5.4, 8.0, 5.4. Where two heads have
-// a kv head it is one as the other.
+// 7.2, 8.4, 7.0; 40 of 500 14.0, 14.1, 12.6; 120 of 20, which is four waves to a SIMD or three 5.4, 8.0, 5.4.
+//
+// Where two heads have a kv head the vector unit's form needs 160 registers, three waves to a SIMD as well, and is 1 % faster in
+// bf16 and 3 % slower in fp8 (290 sizes). Against the fragments' own loads, us over sizes drawn up to 3000 keys and 260 streams: 311
+// without groups 11 % less, 289 of two heads 11 %, 226 of four 17 %, 74 of eight 27 %. Slower by more than 3 % are a tenth of those
+// without groups, by 6 % on average, and an eighth of those of two heads, by 12 %: most of them fp8 caches, or contexts of less than
+// 128 keys with more than the 768 workgroups that are there at once. 64 / 32 heads, 57 of 17 9.1, 10.6; fp8, 97 of 41 16.7, 19.5.
 
 #include <algorithm>
 #include <type_traits>
